@@ -1,0 +1,451 @@
+// FullyConnected for few rows, few outputs or element types the large tiles do not take: int8 / uint8, float16 and
+// float32 with constant weights, any K - vxFullyConnectedLayer as ovxlib reaches it for such layers (reference:
+// src/tim/vx/internal/src/ops/vsi_nn_op_fullconnect2.c:118-126).
+//
+// A workgroup owns a small tile of outputs (16 x 16 up to 64 x 64), its wavefronts split the reduction: each streams a
+// contiguous run of the weights - packed in fragment order at creation, one kilobyte of consecutive memory per load -
+// and the matching sixteen bytes per lane of the activation rows straight into registers, R steps in flight, with no LDS and
+// no barrier on the way; the partial sums meet in LDS once, and every wavefront finishes its share of the outputs.
+// Weights are the A operand, so a lane ends up with one activation row and four consecutive features.
+//
+// What bounds it: at the few rows of a classifier or a small batch every weight is used once per row tile, so the launch is
+// the time to read them; what a CU has in flight (wavefronts x R x 1 KiB) has to cover the memory's latency, which is why a
+// tile's reduction is cut over up to four wavefronts before tiles grow.
+#include <algorithm>
+#include <cstdlib>
+#include <cstring>
+
+#include "variants.h"
+
+namespace tvx {
+namespace {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+
+constexpr int kI8 = 0, kF16 = 1, kF32 = 2;  // element kinds (uint8 runs as int8 with its sign bit flipped)
+
+struct RowsArgs {
+  const uint8_t* x;
+  uint8_t* y;
+  const v4i* wpk;        // [feature tile][step][64 lanes]
+  const int32_t* bias;   // per padded feature: int32 with the zero-point terms folded in, or float bits
+  const tvx_v4i* rq;
+  int M, N, row_bytes;   // bytes of an activation row
+  int64_t x_bytes;
+  int steps;
+  int tiles_m, total, per_xcd;
+  uint32_t m_tiles_m;    // reciprocal of tiles_m
+  uint32_t xor_mask;
+  int zws;               // weight zero point in the signed domain
+  int out_zp, lo, hi, rq_mode, act;
+};
+
+template <int DT, int TS> struct Mfma;
+template <> struct Mfma<kI8, 32> {
+  using acc = v16i;
+  static __device__ __forceinline__ void Step(acc& c, const v4i& w, const v4i& x) { c = __builtin_amdgcn_mfma_i32_32x32x32_i8(w, x, c, 0, 0, 0); }
+};
+template <> struct Mfma<kI8, 16> {
+  using acc = v4i;
+  static __device__ __forceinline__ void Step(acc& c, const v4i& w, const v4i& x) { c = __builtin_amdgcn_mfma_i32_16x16x64_i8(w, x, c, 0, 0, 0); }
+};
+template <> struct Mfma<kF16, 32> {
+  using acc = v16f;
+  static __device__ __forceinline__ void Step(acc& c, const v4i& w, const v4i& x) {
+    c = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, w), __builtin_bit_cast(v8h, x), c, 0, 0, 0);
+  }
+};
+template <> struct Mfma<kF16, 16> {
+  using acc = v4f;
+  static __device__ __forceinline__ void Step(acc& c, const v4i& w, const v4i& x) {
+    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, w), __builtin_bit_cast(v8h, x), c, 0, 0, 0);
+  }
+};
+// (four float32 products per step: lane part p's j-th element is reduction index 4 p + j on both sides)
+template <> struct Mfma<kF32, 32> {
+  using acc = v16f;
+  static __device__ __forceinline__ void Step(acc& c, const v4i& w, const v4i& x) {
+    const v4f a = __builtin_bit_cast(v4f, w), b = __builtin_bit_cast(v4f, x);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j], b[j], c, 0, 0, 0);
+  }
+};
+template <> struct Mfma<kF32, 16> {
+  using acc = v4f;
+  static __device__ __forceinline__ void Step(acc& c, const v4i& w, const v4i& x) {
+    const v4f a = __builtin_bit_cast(v4f, w), b = __builtin_bit_cast(v4f, x);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], c, 0, 0, 0);
+  }
+};
+
+__device__ __forceinline__ int DivM(int u, uint32_t m) { return m ? static_cast<int>(__umulhi(static_cast<uint32_t>(u), m)) : u; }
+
+// TS: extent of an MFMA tile (16 or 32); WM x WN wavefronts share the rows and features (MT x NT tiles each), KS a tile's
+// reduction; R: steps in flight
+template <int DT, int TS, int WM, int WN, int KS, int MT, int NT, int R>
+__global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(4))) FcRowsKernel(RowsArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  using mfma = Mfma<DT, TS>;
+  constexpr int E = DT == kI8 ? 1 : DT == kF16 ? 2 : 4;
+  constexpr int kParts = 64 / TS, kStep = 16 * kParts;  // lane parts of a step, bytes of a row a step covers
+  constexpr int kQuads = TS * TS / 256;                 // accumulator quads of a lane
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // consecutive workgroups of an XCD: the row tiles of a feature tile, which share its weights
+  const int id = static_cast<int>(blockIdx.x & 7) * a.per_xcd + static_cast<int>(blockIdx.x >> 3);
+  if (id >= a.total) return;
+  const int tn = DivM(id, a.m_tiles_m), tm = id - tn * a.tiles_m;
+  const int ks = wave % KS, wn = wave / KS % WN, wm = wave / KS / WN;
+  const int row = lane & (TS - 1), part = lane / TS;
+  const int per = (a.steps + KS - 1) / KS;
+  const int s0 = min(ks * per, a.steps), s1 = min(s0 + per, a.steps);
+
+  const v4i* wp = a.wpk + static_cast<size_t>((tn * WN + wn) * NT) * a.steps * 64 + lane;
+  const uint8_t* xp[MT];
+  int m[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    m[t] = ((tm * WM + wm) * MT + t) * TS + row;
+    xp[t] = a.x + static_cast<int64_t>(min(m[t], a.M - 1)) * a.row_bytes + part * 16;  // (rows past the end repeat the last and are not stored)
+  }
+  v4i fw[R][NT], fx[R][MT];
+  auto fetch = [&](int s, v4i (&w)[NT], v4i (&x)[MT]) {
+    s = max(min(s, s1 - 1), 0);  // (past the end: the last step once more, not multiplied)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) w[t] = wp[static_cast<uint32_t>(t * a.steps + s) * 64];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      // a step that ends behind the row: from where sixteen bytes of the tensor can be read, put right in `multiply`
+      const uint8_t* p = xp[t] + static_cast<size_t>(s) * kStep;
+      const uint8_t* last = a.x + (a.x_bytes - 16);
+      __builtin_memcpy(&x[t], p < last ? p : last, 16);
+    }
+  };
+  typename mfma::acc acc[MT][NT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int i = 0; i < 4 * kQuads; ++i) acc[t][n][i] = 0;
+  int rs[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) rs[t] = 0;
+  const bool ragged = a.row_bytes % kStep != 0;
+  auto multiply = [&](int s, const v4i (&w)[NT], v4i (&x)[MT]) {
+    if (DT == kI8)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) x[t] ^= static_cast<int>(a.xor_mask);
+    if (ragged && s == a.steps - 1) {  // uniform: the row ends inside this step
+      const int valid = a.row_bytes - (s * kStep + part * 16);  // bytes of this lane's granule inside the row
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const int64_t over = (xp[t] + static_cast<size_t>(s) * kStep) - (a.x + (a.x_bytes - 16));  // bytes the load was moved to the front
+        unsigned __int128 v = __builtin_bit_cast(unsigned __int128, x[t]);
+        if (over > 0) v = over < 16 ? v >> (8 * static_cast<int>(over)) : 0;
+        if (valid < 16) v = valid > 0 ? v & ((static_cast<unsigned __int128>(1) << (8 * valid)) - 1) : 0;
+        x[t] = __builtin_bit_cast(v4i, v);
+      }
+    }
+    if (DT == kI8 && a.zws)  // uniform
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) rs[t] = __builtin_amdgcn_sdot4(x[t][q], 0x01010101, rs[t], false);
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int n = 0; n < NT; ++n) mfma::Step(acc[t][n], w[n], x[t]);
+  };
+#pragma unroll
+  for (int u = 0; u < R; ++u) fetch(s0 + u, fw[u], fx[u]);
+  int s = s0;
+#pragma unroll 1
+  for (; s + R < s1; s += R) {
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      multiply(s + u, fw[u], fx[u]);
+      fetch(s + u + R, fw[u], fx[u]);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < R; ++u)
+    if (s + u < s1) multiply(s + u, fw[u], fx[u]);  // uniform
+
+  // ---- the wavefronts of a tile meet: partial sums by quads, [wave][tile][quad][lane]; quad i is finished by wavefront i % KS ----
+  v4i* red = reinterpret_cast<v4i*>(lds);
+  int* red_rs = reinterpret_cast<int*>(lds + WM * WN * KS * MT * NT * kQuads * 1024);
+  if (KS > 1) {
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int k = 0; k < kQuads; ++k) {
+          v4i q;
+          if constexpr (DT == kI8) q = v4i{acc[t][n][4 * k], acc[t][n][4 * k + 1], acc[t][n][4 * k + 2], acc[t][n][4 * k + 3]};
+          else q = __builtin_bit_cast(v4i, v4f{acc[t][n][4 * k], acc[t][n][4 * k + 1], acc[t][n][4 * k + 2], acc[t][n][4 * k + 3]});
+          red[((wave * MT + t) * NT + n) * kQuads * 64 + k * 64 + lane] = q;
+        }
+  }
+  if (DT == kI8 && a.zws) {
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+#pragma unroll
+      for (int o = TS; o < 64; o <<= 1) rs[t] += __shfl_xor(rs[t], o);
+      if (KS > 1 && part == 0) red_rs[(wave * MT + t) * TS + row] = rs[t];
+    }
+  }
+  if (KS > 1) __syncthreads();
+  const int wave0 = wave - ks;  // the tile's first wavefront
+  if (KS > 1 && DT == kI8 && a.zws)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      rs[t] = 0;
+#pragma unroll
+      for (int k = 0; k < KS; ++k) rs[t] += red_rs[((wave0 + k) * MT + t) * TS + row];
+    }
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int k = 0; k < kQuads; ++k) {
+        if (KS > 1 && ((t * NT + n) * kQuads + k) % KS != ks) continue;  // uniform
+        const int f = ((tn * WN + wn) * NT + n) * TS + (TS == 32 ? 8 * k : 0) + 4 * part;  // first of four features
+        const v4i b = *reinterpret_cast<const v4i*>(a.bias + f);
+        if constexpr (DT == kI8) {
+          v4i v = {acc[t][n][4 * k], acc[t][n][4 * k + 1], acc[t][n][4 * k + 2], acc[t][n][4 * k + 3]};
+          if (KS > 1) {
+            v = red[((wave0 * MT + t) * NT + n) * kQuads * 64 + k * 64 + lane];
+#pragma unroll
+            for (int w = 1; w < KS; ++w) v += red[(((wave0 + w) * MT + t) * NT + n) * kQuads * 64 + k * 64 + lane];
+          }
+          v += b - a.zws * rs[t];
+          uint32_t r = 0;
+          if (a.rq_mode == kRqFastNoTie) {  // uniform
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r |= (static_cast<uint32_t>(Requant8<kRqFastNoTie>(v[e], a.rq[f + e], a.out_zp, a.lo, a.hi)) & 0xff) << (8 * e);
+          } else {  // (rare: a loop keeps the 64-bit form out of the common path's instruction stream)
+#pragma unroll 1
+            for (int e = 0; e < 4; ++e) {
+              const int c = a.rq_mode == kRqFast ? Requant8<kRqFast>(v[e], a.rq[f + e], a.out_zp, a.lo, a.hi)
+                                                 : Requant8<kRqGeneric>(v[e], a.rq[f + e], a.out_zp, a.lo, a.hi);
+              r |= (static_cast<uint32_t>(c) & 0xff) << (8 * e);
+            }
+          }
+          if (m[t] >= a.M) continue;
+          uint8_t* yp = a.y + static_cast<int64_t>(m[t]) * a.N + f;
+          if (f + 3 < a.N) __builtin_memcpy(yp, &r, 4);
+          else
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+              if (f + e < a.N) yp[e] = static_cast<uint8_t>(r >> (8 * e));
+        } else {
+          v4f v = {acc[t][n][4 * k], acc[t][n][4 * k + 1], acc[t][n][4 * k + 2], acc[t][n][4 * k + 3]};
+          if (KS > 1) {
+            v = __builtin_bit_cast(v4f, red[((wave0 * MT + t) * NT + n) * kQuads * 64 + k * 64 + lane]);
+#pragma unroll
+            for (int w = 1; w < KS; ++w) v += __builtin_bit_cast(v4f, red[(((wave0 + w) * MT + t) * NT + n) * kQuads * 64 + k * 64 + lane]);
+          }
+          v += __builtin_bit_cast(v4f, b);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if (a.act != TVX_ACT_NONE) v[e] = v[e] < 0.f ? 0.f : v[e];
+            if (a.act == TVX_ACT_RELU6) v[e] = v[e] > 6.f ? 6.f : v[e];
+          }
+          if (m[t] >= a.M) continue;
+          uint8_t* yp = a.y + (static_cast<int64_t>(m[t]) * a.N + f) * E;
+          if constexpr (DT == kF16) {
+            _Float16 h[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) h[e] = static_cast<_Float16>(v[e]);
+            if (f + 3 < a.N) __builtin_memcpy(yp, h, 8);
+            else
+#pragma unroll
+              for (int e = 0; e < 3; ++e)
+                if (f + e < a.N) reinterpret_cast<_Float16*>(yp)[e] = h[e];
+          } else {
+            if (f + 3 < a.N) __builtin_memcpy(yp, &v, 16);
+            else
+#pragma unroll
+              for (int e = 0; e < 3; ++e)
+                if (f + e < a.N) reinterpret_cast<float*>(yp)[e] = v[e];
+          }
+        }
+      }
+}
+
+typedef void (*RowsFn)(RowsArgs);
+struct Shape { int ts, rows, features, waves, ks, lds; RowsFn fn[3]; };
+#define TVX_ROWS(TS, WM, WN, KS, MT, NT, R)                                                                                          \
+  { TS, WM * MT * TS, WN * NT * TS, WM * WN * KS, KS, KS > 1 ? WM * WN * KS * MT * (NT * TS * TS * 4 + TS * 4) : 0,                    \
+    { FcRowsKernel<kI8, TS, WM, WN, KS, MT, NT, R>, FcRowsKernel<kF16, TS, WM, WN, KS, MT, NT, R>, FcRowsKernel<kF32, TS, WM, WN, KS, MT, NT, R> } }
+const Shape kShapes[] = {
+    TVX_ROWS(16, 1, 1, 4, 1, 1, 8),  // 0: 16 x 16, reduction on four wavefronts
+    TVX_ROWS(32, 1, 1, 4, 1, 1, 7),  // 1: 32 x 32, on four
+    TVX_ROWS(32, 2, 2, 1, 1, 1, 8),  // 2: 64 x 64, not split
+};
+#undef TVX_ROWS
+constexpr int kShapeCount = sizeof(kShapes) / sizeof(kShapes[0]);
+
+uint32_t Magic(int d) { return d <= 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + d - 1) / d); }
+
+// The smallest tile that still gives every CU work of its own: 16 x 16 until there is one for each (f16 16 x 4096 -> 4096:
+// 7.5 us against 9.1 on 32 x 32 tiles), 32 x 32 from there on (f32 256 x 1024 -> 1024: 8.8 against 11.9), and 64 x 64 -
+// fragments used twice, no exchange at the end - where there are more than one of those per CU, or half as many with a
+// reduction too short to split (int8 7104 x 128 -> 112: 4.3 against 7.0). Sixteen wavefronts per tile and 128 x 64 tiles
+// were measured on the same 220 drawn layers and won nowhere by more than a tenth.
+int ChooseShape(const tvx_fc_desc& d, int elem_bytes) {
+  const uint64_t t16 = static_cast<uint64_t>((d.m + 15) / 16) * ((d.n + 15) / 16), t64 = static_cast<uint64_t>((d.m + 63) / 64) * ((d.n + 63) / 64);
+  if (t16 <= 256) return 0;
+  if (t64 >= 384 || (t64 >= 128 && static_cast<uint64_t>(d.k) * elem_bytes <= 384)) return 2;
+  return 1;
+}
+
+// Microseconds of both ways, from measured layers: these tiles multiply at about 330 (int8) and 235 (float16) TFLOP/s
+// whatever the shape; a round of 256 x 256 tiles on all CUs costs its start and end whether full or not.
+bool LargeTilesWin(const tvx_fc_desc& d, int dt) {
+  const double flop = 2.0 * d.m * d.n * d.k;
+  const double rows = 3.5 + flop / (dt == kI8 ? 330e6 : 235e6);
+  const uint64_t tiles = static_cast<uint64_t>((d.m + 255) / 256) * ((d.n + 255) / 256);
+  const double large = static_cast<double>((tiles + 255) / 256) * (dt == kI8 ? 17.0 + 0.009 * d.k : 25.0 + 0.0118 * d.k);
+  return large < rows;
+}
+
+struct Plan {
+  RowsArgs a;
+  RowsFn fn;
+  unsigned grid, threads, lds_bytes;
+  int elem;
+};
+
+int FcRowsRun(tvx_op* op, const void* in0, const void*, void* out, hipStream_t st) {
+  const Plan* plan = reinterpret_cast<const Plan*>(op->host_blob.data());
+  if ((reinterpret_cast<uintptr_t>(in0) | reinterpret_cast<uintptr_t>(out)) & (plan->elem - 1))
+    return SetError(TVX_E_INVALID, "%s: tensors must be aligned to their elements", op->kernel_name);
+  RowsArgs a = plan->a;
+  a.x = static_cast<const uint8_t*>(in0);
+  a.y = static_cast<uint8_t*>(out);
+  hipLaunchKernelGGL(plan->fn, dim3(plan->grid), dim3(plan->threads), plan->lds_bytes, st, a);
+  TVX_HIP_CHECK(hipGetLastError());
+  return TVX_OK;
+}
+
+}  // namespace
+
+int FcRowsSetup(tvx_op* op, const tvx_fc_desc* d, const void* w_host, const void* bias_host) {
+  if (!w_host) return TVX_E_UNSUPPORTED;
+  bool forced = false;
+  if (const char* f = getenv("TVX_FC_ROWS")) {  // test lever: 0 declines, 1 claims also where the large tiles are the better choice
+    if (atoi(f) == 0) return TVX_E_UNSUPPORTED;
+    forced = true;
+  } else if (getenv("TVX_FC_TILE_M")) {
+    return TVX_E_UNSUPPORTED;  // (a lever of the large tiles)
+  }
+  int dt;
+  if (op->quantized) dt = kI8;
+  else if (d->in_dtype == TVX_F16 && d->w_dtype == TVX_F16 && d->out_dtype == TVX_F16) dt = kF16;
+  else if (d->in_dtype == TVX_F32 && d->w_dtype == TVX_F32 && d->out_dtype == TVX_F32) dt = kF32;
+  else return TVX_E_UNSUPPORTED;
+  const int E = dt == kI8 ? 1 : dt == kF16 ? 2 : 4;
+  const uint64_t x_bytes = static_cast<uint64_t>(d->m) * d->k * E;
+  if (x_bytes < 16 || x_bytes >= (1ull << 40) || static_cast<uint64_t>(d->k) * E >= (1ull << 30) || static_cast<uint64_t>(d->n) * d->k * E >= (1ull << 32) ||
+      static_cast<uint64_t>(d->m) >= (1ull << 30) || d->n >= (1u << 30))
+    return TVX_E_UNSUPPORTED;
+  const bool tiles_take_it = dt == kI8 ? d->k % 16 == 0 : dt == kF16 && d->k % 8 == 0;
+  if (tiles_take_it && !forced && LargeTilesWin(*d, dt)) return TVX_E_UNSUPPORTED;
+  // a few hundred quantized outputs: a wavefront per output (fc_generic) is one round trip with nothing to exchange - the same
+  // 3.5 us alone, 0.3 us less behind another layer (LeNet's 800 -> 500 at batch 1)
+  if (dt == kI8 && !forced && static_cast<uint64_t>(d->m) * d->n <= 1024 && d->k >= 128) return TVX_E_UNSUPPORTED;
+  int shape = ChooseShape(*d, E);
+  if (const char* f = getenv("TVX_FC_ROWS_SHAPE")) shape = std::max(0, std::min(kShapeCount - 1, atoi(f)));  // test lever
+  const Shape& sp = kShapes[shape];
+  const int kstep = 16 * (64 / sp.ts);
+  RowsArgs a{};
+  a.M = static_cast<int>(d->m); a.N = static_cast<int>(d->n); a.row_bytes = static_cast<int>(d->k) * E;
+  a.x_bytes = static_cast<int64_t>(x_bytes);
+  a.steps = (a.row_bytes + kstep - 1) / kstep;
+  a.tiles_m = (a.M + sp.rows - 1) / sp.rows;
+  const int tiles_n = (a.N + sp.features - 1) / sp.features;
+  const uint64_t total = static_cast<uint64_t>(a.tiles_m) * tiles_n;
+  if (total >= (1ull << 30) || total * a.tiles_m >= (1ull << 32)) return TVX_E_UNSUPPORTED;
+  a.total = static_cast<int>(total);
+  a.per_xcd = (a.total + 7) / 8;
+  a.m_tiles_m = Magic(a.tiles_m);
+  const bool x_u8 = d->in_dtype == TVX_U8, w_u8 = d->w_dtype == TVX_U8;
+  const int zxs = dt == kI8 ? d->in_zp - (x_u8 ? 128 : 0) : 0, zws = dt == kI8 ? op->w_zp - (w_u8 ? 128 : 0) : 0;
+  a.xor_mask = dt == kI8 && x_u8 ? 0x80808080u : 0u;
+  a.zws = zws;
+  a.out_zp = d->out_zp; a.lo = op->act_lo; a.hi = op->act_hi; a.act = d->activation;
+
+  // ---- weights [n][k] -> [feature tile][step][lane = (part, feature)], zero-padded ----
+  const size_t n_alloc = static_cast<size_t>(tiles_n) * sp.features;
+  std::vector<uint8_t> packed(n_alloc / sp.ts * a.steps * 1024, 0);
+  std::vector<int32_t> bias(n_alloc, 0);
+  const uint8_t* src = static_cast<const uint8_t*>(w_host);
+  const uint8_t flip = w_u8 ? 0x80 : 0;
+  for (int n = 0; n < a.N; ++n) {
+    uint8_t* tile = packed.data() + static_cast<size_t>(n / sp.ts) * a.steps * 1024 + static_cast<size_t>(n % sp.ts) * 16;
+    const uint8_t* row = src + static_cast<size_t>(n) * a.row_bytes;
+    int64_t sw = 0;
+    for (int b = 0; b < a.row_bytes; b += 16) {
+      uint8_t* to = tile + static_cast<size_t>(b / kstep) * 1024 + static_cast<size_t>(b % kstep / 16) * sp.ts * 16;
+      const int len = std::min(16, a.row_bytes - b);
+      if (dt != kI8) {
+        std::memcpy(to, row + b, len);
+      } else {
+        int part = 0;
+        for (int j = 0; j < len; ++j) {
+          const uint8_t v = row[b + j] ^ flip;
+          to[j] = v;
+          part += static_cast<int8_t>(v);
+        }
+        sw += part;
+      }
+    }
+    if (dt == kI8) {
+      const int64_t v = (bias_host ? static_cast<const int32_t*>(bias_host)[n] : 0) - static_cast<int64_t>(zxs) * sw + static_cast<int64_t>(d->k) * zxs * zws;
+      bias[n] = static_cast<int32_t>(static_cast<uint32_t>(v));
+    } else if (bias_host) {
+      std::memcpy(&bias[n], static_cast<const float*>(bias_host) + n, 4);
+    }
+  }
+  if (dt == kI8) {
+    std::vector<int32_t> rqt;
+    a.rq_mode = BuildRequantRecords(op->h_mult, op->h_shift, a.N, static_cast<int>(n_alloc), d->out_zp, &rqt, AccumulatorBound(d->k, bias_host, d->n));
+    const int s = op->aux2.Upload(rqt.data(), rqt.size() * 4);
+    if (s != TVX_OK) return s;
+    a.rq = op->aux2.as<tvx_v4i>();
+  }
+  int s = op->packed.Upload(packed.data(), packed.size());
+  if (s == TVX_OK) s = op->aux.Upload(bias.data(), bias.size() * 4);
+  if (s != TVX_OK) return s;
+  a.wpk = op->packed.as<v4i>();
+  a.bias = op->aux.as<int32_t>();
+  Plan plan{};
+  plan.a = a;
+  plan.fn = sp.fn[dt];
+  plan.grid = static_cast<unsigned>(a.per_xcd) * 8;
+  plan.threads = 64u * sp.waves;
+  plan.lds_bytes = static_cast<unsigned>(sp.lds);
+  plan.elem = E;
+  if (plan.lds_bytes > 48 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(plan.fn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(plan.lds_bytes));
+    if (e != hipSuccess) return SetError(TVX_E_DEVICE, "hipFuncSetAttribute(dynamic LDS %u): %s", plan.lds_bytes, hipGetErrorString(e));
+  }
+  op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
+  op->run = FcRowsRun;
+  // (the names such layers have always been reported under, by size: callers compare them)
+  const uint64_t outputs = static_cast<uint64_t>(d->m) * d->n;
+  op->kernel_name = dt == kF32 ? "fc_rows_f32" : dt == kF16 ? (tiles_take_it ? "fc_mfma_f16_256x256x64" : "fc_rows_f16")
+                    : outputs <= 8192 ? "fc_generic" : !tiles_take_it ? "fc_rows_i8" : outputs <= (1u << 18) ? "fc_mfma_i8_16x16_splitk" : "fc_mfma_i8_256x256x128";
+  return TVX_OK;
+}
+
+}  // namespace tvx

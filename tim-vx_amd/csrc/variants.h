@@ -22,6 +22,8 @@ const std::vector<ConvSetupFn>& ConvVariants();
 const std::vector<FcSetupFn>& FcVariants();
 const std::vector<SimpleSetupFn>& PoolVariants();
 
+// few rows or outputs, any K, float32 (fc_rows.hip)
+int FcRowsSetup(tvx_op*, const tvx_fc_desc*, const void*, const void*);
 // int8 MFMA fully-connected (fc_mfma_i8.hip)
 int FcMfmaSetup(tvx_op*, const tvx_fc_desc*, const void*, const void*);
 
