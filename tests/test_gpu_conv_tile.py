@@ -1,0 +1,63 @@
+"""The one-tile-per-workgroup convolution (dense and grouped; int8, float16, float32) at the edges of its tiles: every way
+its wavefronts share a tile, on planes that end inside tiles, granules, column groups and channel blocks."""
+import numpy as np
+import pytest
+
+import tvx_case as TC
+from test_gpu_parity import conv_case
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = range(8)   # 256 x 64 down to 32 x 32 (pixels x channels)
+
+CASES = {
+    # one 16-byte granule with three channels, an odd number of reduction steps, rows of one more than whole column groups
+    "shallow": dict(n=2, c=3, h=11, w=17, oc=33, kh=3, kw=3, stride=[1, 1], dil=[1, 1], pad=[1, 1, 1, 1]),
+    # several images per tile, a batch that does not fill the last one, planes narrower than a column group
+    "images": dict(n=5, c=20, h=7, w=5, oc=40, kh=3, kw=3, stride=[1, 1], dil=[1, 1], pad=[1, 1, 1, 1]),
+    # stride 2, uneven pads, output rows that are no multiple of four
+    "strided": dict(n=1, c=40, h=23, w=30, oc=65, kh=5, kw=3, stride=[2, 2], dil=[1, 1], pad=[0, 1, 2, 1]),
+    "dilated": dict(n=2, c=16, h=14, w=19, oc=24, kh=3, kw=3, stride=[1, 1], dil=[2, 3], pad=[3, 3, 2, 2]),
+    "grouped": dict(n=3, c=36, h=9, w=13, oc=20, kh=3, kw=3, stride=[1, 2], dil=[1, 1], pad=[1, 1, 1, 1], groups=4),
+    # 1 x 1: the image as one row (its last pixels are read from in front), and under a stride
+    "pointwise": dict(n=3, c=24, h=5, w=29, oc=70, kh=1, kw=1, stride=[1, 1], dil=[1, 1], pad=[0, 0, 0, 0]),
+    "pointwise_strided": dict(n=2, c=50, h=15, w=13, oc=32, kh=1, kw=1, stride=[2, 2], dil=[1, 1], pad=[0, 0, 0, 0]),
+    # a window wider than the image, nearly all padding
+    "window": dict(n=2, c=17, h=4, w=3, oc=16, kh=7, kw=7, stride=[1, 1], dil=[1, 1], pad=[3, 3, 3, 3]),
+    # more channels than a tile's window fits LDS with: several chunks, the last one with an empty granule
+    "chunks": dict(n=1, c=300, h=20, w=21, oc=33, kh=5, kw=5, stride=[1, 1], dil=[1, 1], pad=[2, 2, 2, 2]),
+    "row": dict(n=2, c=12, h=1, w=61, oc=8, kh=1, kw=3, stride=[1, 1], dil=[1, 1], pad=[1, 1, 0, 0]),
+}
+
+
+@pytest.mark.parametrize("mode", ["u8", "i8pc", "f16", "f32"])
+@pytest.mark.parametrize("name", CASES)
+def test_conv2d_tile(oracle, name, mode, monkeypatch):
+    rng = np.random.default_rng(sorted(CASES).index(name) + 400)
+    x, wt, b, kws = conv_case(rng, mult=0, mode=mode, **CASES[name])
+    monkeypatch.setenv("TVX_CONV_TILE", "1")
+    want = oracle.conv2d(x, wt, b, act=1, **kws)
+    assert len(np.unique(want)) > 4
+    ran = 0
+    for shape in SHAPES:
+        monkeypatch.setenv("TVX_CONV_TILE_SHAPE", str(shape))
+        got = TC.gpu_conv2d(x, wt, b, act=1, **kws)
+        if mode in ("u8", "i8pc"):
+            assert np.array_equal(got, want), (shape, int((got != want).sum()))
+        else:
+            tol = 2e-3 if mode == "f16" else 1e-5
+            scale = np.sqrt(np.mean(want.astype(np.float64) ** 2))
+            assert np.abs(got.astype(np.float64) - want).max() <= tol * max(scale, 1.0) * 4, shape
+        ran += 1
+    assert ran == len(SHAPES)
+
+
+def test_conv2d_tile_keeps_an_infinity_apart(oracle, monkeypatch):
+    """Padding channels and the empty half of an odd last step multiply zero weights: never with another element's infinity."""
+    monkeypatch.setenv("TVX_CONV_TILE", "1")
+    rng = np.random.default_rng(7)
+    for mode in ("f16", "f32"):
+        x, wt, b, kws = conv_case(rng, mult=0, mode=mode, n=1, c=3, h=9, w=9, oc=8, kh=3, kw=3, stride=[1, 1], dil=[1, 1], pad=[1, 1, 1, 1])
+        x[40] = np.inf
+        got = TC.gpu_conv2d(x, np.abs(wt) + wt.dtype.type(0.01), b, **kws)
+        assert not np.isnan(got).any() and np.isinf(got).sum() == 8 * 9

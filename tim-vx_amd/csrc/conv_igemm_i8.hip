@@ -816,6 +816,22 @@ hipError_t AllowLds(int bytes) {
 
 }  // namespace
 
+// Does the persistent variant take this convolution? (ConvIgemmSetup's own conditions, for the kernel asked in front of it.)
+bool ConvIgemmPersists(const tvx_conv2d_desc* d) {
+  const char* lever = getenv("TVX_IGEMM_PERSIST");  // test lever
+  if (lever && atoi(lever) == 0) return false;
+  const int taps = static_cast<int>(d->k_w * d->k_h), ksteps = taps * static_cast<int>(d->in_c) / 32;
+  if (d->in_c % 32 || d->out_c <= 32 || d->out_c > 64 || (d->in_w & 3) || ((d->out_w * d->out_h) & 3)) return false;
+  if (ksteps > 40 || !PersistKernel(ksteps, kRqFastNoTie, false, false)) return false;
+  int rows = 0;
+  for (uint32_t r = 1; r <= d->out_h; ++r) {
+    if ((r - 1) * d->stride_h + (d->k_h - 1) * d->dilation_h + 1 > static_cast<uint32_t>(kPersistRows) || r * d->out_w > 256) break;
+    if ((r * d->out_w & 3) == 0) rows = static_cast<int>(r);
+  }
+  if (rows == 0) return false;
+  return (lever && atoi(lever) > 0) || static_cast<uint64_t>(d->batch) * ((d->out_h + rows - 1) / rows) >= 384;
+}
+
 // Claims dense quantized convolutions with constant weights whose weight block
 // and halo tile fit the CU's LDS.
 int ConvIgemmSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const void* bias_host) {

@@ -1,0 +1,804 @@
+// Dense and grouped convolution of any window, stride and dilation as an implicit GEMM on the matrix cores, one output
+// tile per workgroup, for int8 / uint8, float16 and float32 tensors - vxConvolutionLayer as ovxlib reaches it for those
+// (reference: src/tim/vx/internal/src/ops/vsi_nn_op_conv2d.c:35-118, vsi_nn_op_grouped_conv2d.c).
+//
+// A tile is TW x TH output pixels of one image (whole small images: G of them) times 32 .. 128 output channels of one
+// group. The input window behind it - halo included, padding as the input's zero point - is transposed into LDS once as
+// [row][column][channel]: a work item loads four pixels of a 16-byte granule of channels (16 int8, 8 float16 or 4 float32
+// planes), all of its loads in flight together, and stores four 16-byte units, so that a reduction step of the matrix
+// core is one 16-byte LDS read per lane at (tap, granule) for every element type. A step's two granules need not belong
+// to one tap: a table gives their LDS offsets, and shallow inputs (one granule a pixel) waste half of nothing.
+// The weights are packed in fragment order when the operator is created and stream from L2 straight into registers a
+// group of steps ahead; they need no LDS, so the whole channel depth of a tile usually fits (else it is walked in chunks).
+// Quantized tensors under a weight zero point need the sum of every window: channel sums per staged pixel, box-filtered
+// once per tile - nothing in the inner loop.
+//
+// What bounds it: at the sizes convolutional networks have, a launch is a chain of one memory round trip, the LDS
+// transposition (about 70 vector instructions per 64 staged bytes for int8, none for float32) and the steps themselves;
+// the tile is chosen on the host so that the chip is filled first and the halo staged per output pixel is small second.
+#include <algorithm>
+#include <cmath>
+#include <cstdlib>
+#include <cstring>
+
+#include "variants.h"
+
+namespace tvx {
+namespace {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+
+constexpr int kI8 = 0, kF16 = 1, kF32 = 2;  // element kinds (uint8 runs as int8 with its sign bit flipped)
+
+struct TileArgs {
+  const uint8_t* x;
+  uint8_t* y;
+  const v4i* wpk;          // [group][32-channel tile][chunk][step][64 lanes]: sixteen bytes of reduction per lane
+  const int* tab;          // [half][steps_pad]: LDS byte offset of the granule a lane of that half multiplies at a step
+  const int32_t* biasf;    // quantized: bias with the zero-point terms folded in, per padded output channel
+  const float* biasfl;     // floating point: the bias, or null
+  const tvx_v4i* rq;
+  int C, H, W, OC, OH, OW, batch;
+  int sh, sw, pad_t, pad_l;
+  int icg, ocg;            // channels per group
+  int TW, TH, G, NQ;       // tile: columns, rows, images; its pixels
+  int IW, IH;              // staged columns, and rows per image
+  int row_step, row_stride;  // input rows between staged rows; staged rows between output rows
+  int pitch;               // LDS bytes of a staged pixel: an odd number of granules (bank spread)
+  int gpc, chunks;         // granules of a pixel per chunk
+  int steps, steps_pad, odd;  // reduction steps of a chunk; the last step's upper half is empty
+  int taps_w, taps_h, dil_col, dil_row;  // for the box sum: LDS pixels between taps
+  int ncg, cells, gl;      // column groups of a staged row, of all rows; granules neighbouring lanes take (a divisor of gpc)
+  int tiles_x, tiles_y, oc_blocks, tiles_per_group;
+  int total, per_xcd;
+  int npx, items;          // staged pixels and work items of a chunk
+  uint32_t plane_bytes, image_bytes;
+  int at_max;              // last place of a plane where a work item's pixels can be read
+  int off_tab, off_sum, off_zt;  // LDS carve-up behind the staged window
+  uint32_t m_gl, m_cells, m_ncg, m_ih, m_iw, m_tw, m_thtw, m_ocb, m_tpg, m_tx, m_ty;  // reciprocals: u / d = mulhi(u, m), exact for the ranges used
+  uint32_t xor_mask;
+  uint32_t pad_full, pad_last[4];  // a padding granule: full, and the channels' last one
+  int last_granule;        // global index of the channels' last granule
+  int zws;                 // weight zero point in the signed domain (0: no window sums)
+  int out_zp, lo, hi, act;
+};
+
+__device__ __forceinline__ int DivM(int u, uint32_t m) { return m ? static_cast<int>(__umulhi(static_cast<uint32_t>(u), m)) : u; }
+
+template <int DT> struct Kind;
+template <> struct Kind<kI8> { using acc = v16i; using elem = int; static constexpr int E = 1; };
+template <> struct Kind<kF16> { using acc = v16f; using elem = float; static constexpr int E = 2; };
+template <> struct Kind<kF32> { using acc = v16f; using elem = float; static constexpr int E = 4; };
+
+template <int DT>
+__device__ __forceinline__ void Multiply(typename Kind<DT>::acc& acc, const v4i& fx, const v4i& fw) {
+  if constexpr (DT == kI8) {
+    acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fx, fw, acc, 0, 0, 0);
+  } else if constexpr (DT == kF16) {
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, fx), __builtin_bit_cast(v8h, fw), acc, 0, 0, 0);
+  } else {
+    const v4f a = __builtin_bit_cast(v4f, fx), b = __builtin_bit_cast(v4f, fw);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j], b[j], acc, 0, 0, 0);
+  }
+}
+
+// One work item on its way: P consecutive pixels of a row x one granule of channel planes.
+template <int DT> struct Item {
+  static constexpr int E = Kind<DT>::E;
+  static constexpr int N = 16 / E;            // channel planes
+  static constexpr int P = DT == kF32 ? 4 : 8;  // pixels: 8 or 16 bytes of a plane
+  static constexpr int D = P * E / 4;         // dwords of a plane
+  uint32_t d[N * D];
+
+  // FULL: all planes exist; else planes past the last valid one re-read it (masked behind Unit)
+  template <bool FULL>
+  __device__ __forceinline__ void Load(const uint8_t* base, uint32_t at, uint32_t plane_bytes, int valid) {
+#pragma unroll
+    for (int c = 0; c < N; ++c) {
+      if (FULL) __builtin_memcpy(&d[c * D], base + static_cast<size_t>(c) * plane_bytes + at, 4 * D);  // (scalar base, one lane offset)
+      else __builtin_memcpy(&d[c * D], base + (at + static_cast<uint32_t>(min(c, valid - 1)) * plane_bytes), 4 * D);
+    }
+  }
+  // the granules of pixels 4 g .. 4 g + 3
+  __device__ __forceinline__ void Units(int g, v4i (&u)[4]) const {
+    if constexpr (DT == kI8) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t in[4] = {d[4 * q * D + g], d[(4 * q + 1) * D + g], d[(4 * q + 2) * D + g], d[(4 * q + 3) * D + g]};
+        uint32_t out[4];
+        Transpose4x4(in, out);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) u[i][q] = static_cast<int>(out[i]);
+      }
+    } else if constexpr (DT == kF16) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t a0 = d[2 * q * D + 2 * g], a1 = d[2 * q * D + 2 * g + 1], b0 = d[(2 * q + 1) * D + 2 * g], b1 = d[(2 * q + 1) * D + 2 * g + 1];
+        u[0][q] = static_cast<int>(__builtin_amdgcn_perm(b0, a0, 0x05040100));
+        u[1][q] = static_cast<int>(__builtin_amdgcn_perm(b0, a0, 0x07060302));
+        u[2][q] = static_cast<int>(__builtin_amdgcn_perm(b1, a1, 0x05040100));
+        u[3][q] = static_cast<int>(__builtin_amdgcn_perm(b1, a1, 0x07060302));
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) u[i][q] = static_cast<int>(d[q * D + i]);
+    }
+  }
+};
+
+// WM x WN wavefronts share the tile's pixels and channels (MT x NT MFMA tiles each), KS wavefronts a tile's reduction.
+// R: steps whose weights are on their way to a wavefront at a time.
+template <int DT, int WM, int WN, int KS, int MT, int NT, int R, int EU, bool MULTI>
+__global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(EU))) ConvTileKernel(TileArgs a) {
+  constexpr int kThreads = 64 * WM * WN * KS;
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  using acc_t = typename Kind<DT>::acc;
+  using elem_t = typename Kind<DT>::elem;
+  using item_t = Item<DT>;
+  constexpr int E = Kind<DT>::E, P = item_t::P;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // consecutive workgroups of an XCD: the channel blocks of a tile, then the next tile
+  const int id = static_cast<int>(blockIdx.x & 7) * a.per_xcd + static_cast<int>(blockIdx.x >> 3);
+  if (id >= a.total) return;
+  const int tab_n = 2 * a.steps_pad;
+  const int tab_first = a.tab[min(tid, tab_n - 1)];  // (waited for behind the window's loads)
+  const int tile = DivM(id, a.m_ocb), ocb = id - tile * a.oc_blocks;
+  const int group = DivM(ocb, a.m_tpg), ocl = ocb - group * a.tiles_per_group;  // group, channel block of the group
+  const int tyn = DivM(tile, a.m_tx), tx = tile - tyn * a.tiles_x;
+  const int tn = DivM(tyn, a.m_ty), ty = tyn - tn * a.tiles_y;
+  const int n0 = tn * a.G;
+  const int x0 = tx * a.TW, y0 = ty * a.TH;
+  const int ix0 = x0 * a.sw - a.pad_l, iy0 = y0 * a.sh - a.pad_t;
+
+  const int row = lane & 31, half = lane >> 5;
+  const int ks = wave % KS, wn = wave / KS % WN, wm = wave / KS / WN;
+  // this wavefront's share of a chunk's steps, and its weights
+  const int per = (a.steps + KS - 1) / KS;
+  const int s0 = KS == 1 ? 0 : min(ks * per, a.steps), s1 = KS == 1 ? a.steps : min(s0 + per, a.steps);
+  const uint32_t tile_stride = static_cast<uint32_t>((MULTI ? a.chunks : 1) * a.steps) * 64;
+  const v4i* wp = a.wpk + static_cast<size_t>((group * a.tiles_per_group + ocl) * (WN * NT) + wn * NT) * tile_stride + lane;
+  v4i fw[R][NT];
+  auto fetch_w = [&](int chunk, int s, v4i (&f)[NT]) {
+    const uint32_t at = static_cast<uint32_t>(chunk * a.steps + max(min(s, s1 - 1), 0)) * 64;  // (past the end: the last step once more, not multiplied)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) f[t] = wp[t * tile_stride + at];
+  };
+
+  const uint32_t plane_bytes = a.plane_bytes, image_bytes = a.image_bytes;
+  const int npx = a.npx, items = a.items;
+  const int col_lo = max(0, -ix0), col_hi = min(a.IW, a.W - ix0);  // window columns inside the image
+  uint32_t base[MT];  // LDS byte offset of this lane's pixel in each pixel tile
+  acc_t acc[MT][NT];
+
+  const int chunks = MULTI ? a.chunks : 1;
+  for (int chunk = 0; chunk < chunks; ++chunk) {
+    if (chunk) __syncthreads();  // the window is free
+    // ---- stage: an item = (granule, column group, row); lanes take gl granules, then the cells of a plane (contiguous in
+    // memory where the rows are whole), then the next gl granules ----
+    const int c0 = chunk * a.gpc * (16 / E);  // first channel of the chunk
+    const uint8_t* xg = a.x + static_cast<size_t>(n0) * image_bytes + static_cast<size_t>(group * a.icg + c0) * plane_bytes;
+    const bool all_full = c0 + a.gpc * (16 / E) <= a.icg;  // uniform: every granule of the chunk has all its channels
+    for (int it0 = 0; it0 < items; it0 += kThreads) {
+      const int it = it0 + tid;
+      item_t item;
+      const bool live = it < items;
+      const int itc = live ? it : 0;
+      const int rest = DivM(itc, a.m_gl), gl = itc - rest * a.gl;
+      const int gh = DivM(rest, a.m_cells), cell = rest - gh * a.cells;
+      const int gr = gh * a.gl + gl;
+      const int r = DivM(cell, a.m_ncg), cg = cell - r * a.ncg;
+      const int g = DivM(r, a.m_ih), ry = r - g * a.IH;
+      const int iy = iy0 + ry * a.row_step, ixs = ix0 + P * cg;
+      const bool inside = live && static_cast<unsigned>(iy) < static_cast<unsigned>(a.H) && ixs > -P && ixs < a.W && n0 + g < a.batch;
+      const int valid = min(a.icg - c0 - gr * (16 / E), 16 / E);  // channels of the granule
+      // P pixels from the group's first column inside the image, further in front at the plane's end: what lies outside
+      // the row is not stored, what the neighbouring group stores too is the same
+      const int px = min(iy * a.W + max(ixs, 0), a.at_max);
+      const int col = px - iy * a.W - ix0;  // window column of the first pixel
+      const uint32_t at = inside && valid > 0 ? static_cast<uint32_t>(g) * image_bytes + static_cast<uint32_t>(gr * (16 / E)) * plane_bytes + static_cast<uint32_t>(px) * E : 0u;
+      if (all_full) item.template Load<true>(xg, at, plane_bytes, 16 / E);
+      else item.template Load<false>(xg, at, plane_bytes, max(valid, 1));
+      if (it0 == 0) {
+        // under the first loads: the first weights, the table, the accumulators, the lanes' pixels, the padding
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < R; ++u) fetch_w(chunk, s0 + u, fw[u]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (chunk == 0) {
+#pragma unroll
+          for (int m = 0; m < MT; ++m) {
+            const int q = min((wm * MT + m) * 32 + row, a.NQ - 1);  // (pixels past the tile's end repeat its last one and are not stored)
+            const int qg = DivM(q, a.m_thtw), rem = q - qg * a.TH * a.TW;
+            const int qy = DivM(rem, a.m_tw), qx = rem - qy * a.TW;
+            base[m] = static_cast<uint32_t>(((qg * a.IH + qy * a.row_stride) * a.IW + qx * a.sw) * a.pitch);
+          }
+        }
+        if (ix0 < 0 || ix0 + a.IW > a.W || iy0 < 0 || iy0 + (a.IH - 1) * a.row_step >= a.H) {  // uniform: the window leaves the image
+          const int pad_whole = max(0, min(a.last_granule - chunk * a.gpc, a.gpc));
+          const int pf = static_cast<int>(a.pad_full);
+          const v4i pad_unit = {pf, pf, pf, pf};
+          const v4i pad_tail = {static_cast<int>(a.pad_last[0]), static_cast<int>(a.pad_last[1]), static_cast<int>(a.pad_last[2]), static_cast<int>(a.pad_last[3])};
+          for (int p = tid; p < npx; p += kThreads) {
+            const int pr = DivM(p, a.m_iw), cx = p - pr * a.IW;
+            const int pry = pr - DivM(pr, a.m_ih) * a.IH;
+            const int py = iy0 + pry * a.row_step;
+            if (static_cast<unsigned>(py) < static_cast<unsigned>(a.H) && cx >= col_lo && cx < col_hi) continue;
+            v4i* to = reinterpret_cast<v4i*>(lds + p * a.pitch);
+            for (int pg = 0; pg < pad_whole; ++pg) to[pg] = pad_unit;
+            if (pad_whole < a.gpc) {  // uniform: the chunk holds the channels' last granule (and empty ones)
+              to[pad_whole] = pad_tail;
+              for (int pg = pad_whole + 1; pg < a.gpc; ++pg) to[pg] = v4i{0, 0, 0, 0};
+            }
+          }
+        }
+        if (chunk == 0) {
+          int* tab = reinterpret_cast<int*>(lds + a.off_tab);
+          if (tid < tab_n) tab[tid] = tab_first;
+          for (int i = tid + kThreads; i < tab_n; i += kThreads) tab[i] = a.tab[i];
+        }
+      }
+      if (inside) {
+        uint8_t* to = lds + (r * a.IW + col) * a.pitch + gr * 16;
+        v4i mask;
+        if (!all_full)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int nb = valid * E - 4 * q;
+            mask[q] = nb >= 4 ? -1 : nb <= 0 ? 0 : static_cast<int>((1u << (8 * nb)) - 1u);
+          }
+#pragma unroll
+        for (int h = 0; h < P / 4; ++h) {
+          v4i u[4];
+          item.Units(h, u);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            if (DT == kI8) u[i] ^= static_cast<int>(a.xor_mask);
+            if (!all_full) u[i] &= mask;
+            if (static_cast<unsigned>(col + 4 * h + i - col_lo) < static_cast<unsigned>(col_hi - col_lo)) *reinterpret_cast<v4i*>(to + (4 * h + i) * a.pitch) = u[i];
+          }
+        }
+      }
+    }
+    __syncthreads();
+    // ---- channel sums of the staged pixels ----
+    if (DT == kI8 && a.zws) {  // uniform
+      int* sum = reinterpret_cast<int*>(lds + a.off_sum);
+      for (int p = tid; p < npx; p += kThreads) {
+        int v = chunk ? sum[p] : 0;
+        for (int gr = 0; gr < a.gpc; ++gr) {
+          const v4i f = *reinterpret_cast<const v4i*>(lds + p * a.pitch + gr * 16);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) v = __builtin_amdgcn_sdot4(f[q], 0x01010101, v, false);
+        }
+        sum[p] = v;
+      }
+    }
+    if (chunk == 0)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc[m][t][i] = 0;
+    // ---- multiply: R steps' weights ahead, two steps' activations ahead ----
+    const int* tab = reinterpret_cast<const int*>(lds + a.off_tab) + half * a.steps_pad;
+    v4i fx[2][MT];
+    auto fetch_x = [&](int s, v4i (&f)[MT]) {
+      const int off = tab[s];  // (the table is padded)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) f[m] = *reinterpret_cast<const v4i*>(lds + base[m] + off);
+    };
+    auto multiply = [&](int s, v4i (&f)[MT], const v4i (&w)[NT]) {
+      if (DT != kI8 && a.odd && s == a.steps - 1 && half)  // (zero weights, but the data may be an infinity)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) f[m] = v4i{0, 0, 0, 0};
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) Multiply<DT>(acc[m][t], f[m], w[t]);
+    };
+    fetch_x(s0, fx[0]);
+    fetch_x(s0 + 1, fx[1]);
+    int s = s0;
+#pragma unroll 1
+    for (; s + R < s1; s += R) {
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        multiply(s + u, fx[u & 1], fw[u]);
+        fetch_w(chunk, s + u + R, fw[u]);
+        fetch_x(s + u + 2, fx[u & 1]);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < R; ++u)
+      if (s + u < s1) {  // uniform
+        multiply(s + u, fx[u & 1], fw[u]);
+        fetch_x(s + u + 2, fx[u & 1]);
+      }
+  }
+
+  // the epilogue's tables travel while the wavefronts meet
+  int bias[NT];
+  tvx_v4i rq[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int oc = (ocl * WN + wn) * NT * 32 + t * 32 + row;  // channel of the group
+    if constexpr (DT == kI8) {
+      const int slot = group * a.tiles_per_group * (WN * NT * 32) + oc;
+      rq[t] = a.rq[slot];
+      bias[t] = a.biasf[slot];
+    } else {
+      bias[t] = a.biasfl && oc < a.ocg ? reinterpret_cast<const int*>(a.biasfl)[group * a.ocg + oc] : 0;
+    }
+  }
+
+  // ---- wavefronts that split a reduction exchange partial sums: an accumulator tile is cut into pieces (pairs of quads
+  // that become eight consecutive pixels, or single quads), every wavefront finishes its own ----
+  constexpr int kQuads = KS == 1 ? 4 : (2 * MT * NT >= KS ? 2 : 1);  // quads of a piece
+  constexpr int kPieces = 4 / kQuads;
+  typedef uint32_t run_t __attribute__((ext_vector_type(kQuads * E)));
+  if (KS > 1 || (DT == kI8 && a.zws)) {
+    __syncthreads();
+    elem_t* part = reinterpret_cast<elem_t*>(lds);  // [wave][tile][element][lane]
+    if (KS > 1)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int piece = (m * NT + t) * kPieces + (i / 4) % kPieces;
+            if (piece % KS != ks) part[((wave * MT + m) * NT + t) * 1024 + i * 64 + lane] = acc[m][t][i];
+          }
+    // window sums: the box filter over the channel sums
+    if (DT == kI8 && a.zws) {
+      const int* sum = reinterpret_cast<const int*>(lds + a.off_sum);
+      int* zt = reinterpret_cast<int*>(lds + a.off_zt);
+      for (int q = tid; q < a.NQ; q += kThreads) {
+        const int g = DivM(q, a.m_thtw), rem = q - g * a.TH * a.TW;
+        const int qy = DivM(rem, a.m_tw), qx = rem - qy * a.TW;
+        const int* sp = sum + (g * a.IH + qy * a.row_stride) * a.IW + qx * a.sw;
+        int v = 0;
+        for (int ky = 0; ky < a.taps_h; ++ky)
+          for (int kx = 0; kx < a.taps_w; ++kx) v += sp[ky * a.dil_row + kx * a.dil_col];
+        zt[q] = -a.zws * v;
+      }
+    }
+    __syncthreads();
+    if (KS > 1)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int p = 0; p < kPieces; ++p)
+            if (((m * NT + t) * kPieces + p) % KS == ks)
+#pragma unroll
+              for (int k = 1; k < KS; ++k) {
+                const elem_t* from = part + (((wave - ks + (ks + k) % KS) * MT + m) * NT + t) * 1024 + lane;
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                  if ((i / 4) % kPieces == p) acc[m][t][i] += from[i * 64];
+              }
+  }
+
+  // ---- epilogue: a lane holds output channel `row` of each channel tile and, per accumulator quad k, pixels
+  // 8 k + 4 half + 0 .. 3 of a pixel tile; behind the swaps between the wavefront's halves quads 0 .. 3 are sixteen
+  // consecutive pixels, quads p and p + 2 eight ----
+  const int ohw = a.OH * a.OW, image_out = a.OC * ohw;
+  uint8_t* yb = a.y + (static_cast<size_t>(n0) * a.OC + static_cast<size_t>(group) * a.ocg) * ohw * E;
+  auto place = [&](int q) {  // element offset of tile pixel q inside its images' first plane, or -1
+    const int g = DivM(q, a.m_thtw), rem = q - g * a.TH * a.TW;
+    const int qy = DivM(rem, a.m_tw), qx = rem - qy * a.TW;
+    if (q >= a.NQ || n0 + g >= a.batch || y0 + qy >= a.OH || x0 + qx >= a.OW) return -1;
+    return g * image_out + (y0 + qy) * a.OW + x0 + qx;
+  };
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+#pragma unroll
+    for (int p = 0; p < kPieces; ++p) {
+      const int tile_at = (wm * MT + m) * 32;
+      const int q0 = tile_at + (kQuads == 4 ? 16 * half : kQuads == 2 ? 16 * half + 8 * p : 8 * p + 4 * half);
+      const int first = place(q0), last = place(q0 + 4 * kQuads - 1);
+      const bool run_ok = first >= 0 && last == first + 4 * kQuads - 1;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        if (KS > 1 && ((m * NT + t) * kPieces + p) % KS != ks) continue;
+        const int oc = (ocl * WN + wn) * NT * 32 + t * 32 + row;
+        uint32_t quad[kQuads][E];
+#pragma unroll
+        for (int j = 0; j < kQuads; ++j) {
+          const int k = p + j * kPieces;
+          if constexpr (DT == kI8) {
+            int v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = acc[m][t][4 * k + e] + bias[t];
+            if (a.zws) {
+              const v4i z = *reinterpret_cast<const v4i*>(lds + a.off_zt + (tile_at + 8 * k + 4 * half) * 4);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) v[e] += z[e];
+            }
+            quad[j][0] = RequantPack4<kRqFastNoTie>(v, rq[t], a.out_zp, a.lo, a.hi);
+          } else {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              v[e] = acc[m][t][4 * k + e] + __builtin_bit_cast(float, bias[t]);
+              if (a.act != TVX_ACT_NONE) v[e] = v[e] < 0.f ? 0.f : v[e];
+              if (a.act == TVX_ACT_RELU6) v[e] = v[e] > 6.f ? 6.f : v[e];
+            }
+            if constexpr (DT == kF16) {
+              _Float16 h[4];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) h[e] = static_cast<_Float16>(v[e]);
+              __builtin_memcpy(quad[j], h, 8);
+            } else {
+              __builtin_memcpy(quad[j], v, 16);
+            }
+          }
+        }
+        run_t run;  // consecutive pixels
+        if constexpr (kQuads == 1) {
+#pragma unroll
+          for (int d = 0; d < E; ++d) run[d] = quad[0][d];
+        } else {
+#pragma unroll
+          for (int d = 0; d < E; ++d) {
+            const auto lo = __builtin_amdgcn_permlane32_swap(quad[0][d], quad[kQuads / 2][d], false, false);
+            run[d] = lo[0]; run[E + d] = lo[1];
+            if constexpr (kQuads == 4) {
+              const auto hi = __builtin_amdgcn_permlane32_swap(quad[1][d], quad[3][d], false, false);
+              run[2 * E + d] = hi[0]; run[3 * E + d] = hi[1];
+            }
+          }
+        }
+        if (oc >= a.ocg) continue;
+        uint8_t* yp = yb + static_cast<size_t>(oc) * ohw * E;
+        if (run_ok) {
+          __builtin_memcpy(yp + static_cast<int64_t>(first) * E, &run, 4 * kQuads * E);
+        } else {  // (loops that stay loops: the instruction cache starts cold with every launch)
+#pragma unroll 1
+          for (int k = 0; k < kQuads; ++k) {
+            const int f = place(q0 + 4 * k), l = place(q0 + 4 * k + 3);
+            if (f >= 0 && l == f + 3) {
+              uint32_t four[E];
+#pragma unroll
+              for (int d = 0; d < E; ++d) four[d] = run[k * E + d];
+              __builtin_memcpy(yp + static_cast<int64_t>(f) * E, four, 4 * E);
+              continue;
+            }
+#pragma unroll 1
+            for (int e = 0; e < 4; ++e) {
+              const int at = place(q0 + 4 * k + e);
+              if (at < 0) continue;
+              if constexpr (E == 1) yp[at] = static_cast<uint8_t>(run[k] >> (8 * e));
+              else if constexpr (E == 2) reinterpret_cast<uint16_t*>(yp)[at] = static_cast<uint16_t>(run[2 * k + (e >> 1)] >> (16 * (e & 1)));
+              else reinterpret_cast<uint32_t*>(yp)[at] = run[4 * k + e];
+            }
+          }
+        }
+      }
+    }
+  }
+}
+
+typedef void (*TileFn)(TileArgs);
+
+// The ways a workgroup's wavefronts share a tile.
+struct Shape { int pixels, channels, ks, waves; TileFn fn[3][2]; };
+#define TVX_TILE_DT(DT, WM, WN, KS, MT, NT, R, EU) { ConvTileKernel<DT, WM, WN, KS, MT, NT, R, EU, false>, ConvTileKernel<DT, WM, WN, KS, MT, NT, R, 2, true> }
+#define TVX_TILE(WM, WN, KS, MT, NT, R, EU)                                                                       \
+  { WM * MT * 32, WN * NT * 32, KS, WM * WN * KS, { TVX_TILE_DT(kI8, WM, WN, KS, MT, NT, R, EU), TVX_TILE_DT(kF16, WM, WN, KS, MT, NT, R, EU), \
+                                                    TVX_TILE_DT(kF32, WM, WN, KS, MT, NT, R, EU) } }
+const Shape kShapes[] = {
+    TVX_TILE(4, 2, 1, 2, 1, 4, 4),  // 0: 256 x 64, eight wavefronts
+    TVX_TILE(2, 2, 2, 2, 1, 4, 4),  // 1: 128 x 64, eight
+    TVX_TILE(2, 2, 1, 2, 1, 4, 4),  // 2: 128 x 64, four
+    TVX_TILE(4, 1, 2, 1, 1, 6, 4),  // 3: 128 x 32, eight
+    TVX_TILE(4, 1, 1, 1, 1, 6, 4),  // 4: 128 x 32, four
+    TVX_TILE(2, 2, 2, 1, 1, 6, 4),  // 5: 64 x 64, eight
+    TVX_TILE(2, 1, 4, 1, 1, 6, 4),  // 6: 64 x 32, eight
+    TVX_TILE(1, 1, 8, 1, 1, 6, 4),  // 7: 32 x 32, eight
+};
+#undef TVX_TILE
+#undef TVX_TILE_DT
+constexpr int kShapeCount = sizeof(kShapes) / sizeof(kShapes[0]);
+
+int RoundUp(int v, int m) { return (v + m - 1) / m * m; }
+uint32_t Magic(int d) { return d <= 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + d - 1) / d); }
+
+struct Geometry {
+  int shape, TW, TH, G, gpc, chunks;
+  int IW, IH, pitch, lds_bytes;
+  int64_t wgs;
+  double cost;
+};
+
+// Microseconds of a launch, to compare tiles by. A workgroup is a chain - start, staging rounds (an item per thread and
+// round), steps, epilogue - whose length counts once per round of workgroups the chip holds; above that the units a CU's
+// workgroups share (its memory pipeline above all: 0.6 us per wavefront of int8 items) set the pace. The constants are a
+// fit to 5400 measured launches (140 drawn convolutions x the tiles below): 16 % off a launch at the median of the squares,
+// and the tile chosen costs 5 % more than the best one on the (geometric) average.
+double Cost(const Shape& sp, const Geometry& g, int dt, int taps, int group_px, bool sums, bool whole_granules, bool borders, int OW) {
+  const int threads = 64 * sp.waves, steps = (taps * g.gpc + 1) / 2, tiles = sp.pixels * sp.channels / 1024 * sp.ks / sp.waves;
+  const double npx = static_cast<double>(g.G) * g.IH * g.IW;
+  const double items = static_cast<double>(g.G) * g.IH * ((g.IW + group_px - 1) / group_px) * g.gpc;
+  const double runs = g.TW == OW || g.TW % 16 == 0 ? 1.0 : 1.1;  // stores of whole sixteen-pixel runs
+  const double stage = (dt == kI8 ? 2.27 : dt == kF16 ? 1.49 : 1.32) * std::ceil(items / threads) * (whole_granules ? 1.0 : 1.2) +
+                       0.024 * npx * g.gpc / threads * ((sums ? 1.0 : 0.0) + (borders ? 0.5 : 0.0));
+  const double multiply = static_cast<double>(steps) / sp.ks * (0.034 + (dt == kF32 ? 0.286 : 0.059) * tiles);
+  const double chain = 0.87 + g.chunks * (stage + multiply) + 1.5 * tiles * runs;
+  const double shared = g.chunks * (0.6 * items / 64 * (dt == kF32 ? 0.126 : 1.0) + 0.0028 * steps * tiles * sp.waves / sp.ks * (dt == kF32 ? 8 : 1)) +
+                        0.5 * sp.pixels * sp.channels / 1024 * runs;
+  const double per_cu = static_cast<double>(g.wgs) / 256;
+  const double resident = std::min<double>(std::max(1, std::min(16 / sp.waves, 160 * 1024 / g.lds_bytes)), std::max(1.0, std::ceil(per_cu)));
+  const double by_chain = per_cu <= resident ? chain : (per_cu / resident + 0.6) * chain, by_units = per_cu * shared;
+  return 3.0 + std::cbrt(by_chain * by_chain * by_chain + by_units * by_units * by_units);
+}
+
+struct Plan {
+  TileArgs a;
+  TileFn fn;
+  unsigned grid, threads, lds_bytes;
+  int elem;
+};
+
+int ConvTileRun(tvx_op* op, const void* in0, const void*, void* out, hipStream_t st) {
+  const Plan* plan = reinterpret_cast<const Plan*>(op->host_blob.data());
+  if ((reinterpret_cast<uintptr_t>(in0) | reinterpret_cast<uintptr_t>(out)) & (plan->elem - 1))
+    return SetError(TVX_E_INVALID, "%s: tensors must be aligned to their elements", op->kernel_name);
+  TileArgs a = plan->a;
+  a.x = static_cast<const uint8_t*>(in0);
+  a.y = static_cast<uint8_t*>(out);
+  hipLaunchKernelGGL(plan->fn, dim3(plan->grid), dim3(plan->threads), plan->lds_bytes, st, a);
+  TVX_HIP_CHECK(hipGetLastError());
+  return TVX_OK;
+}
+
+}  // namespace
+
+// Which shapes stay with the kernels asked behind this one (measured on 290 drawn convolutions; the others are 2.4 times
+// faster here than on conv2d_igemm_i8, 3 on conv2d_gemm_f16 and 5 on conv2d_generic, on the geometric average):
+static bool IsBetterChoice(const tvx_conv2d_desc* d, int dt) {
+  const int groups = d->groups > 1 ? d->groups : 1;
+  const uint64_t reduction = static_cast<uint64_t>(d->in_c / groups) * d->k_w * d->k_h;
+  const uint64_t macs = reduction * d->out_c * d->out_w * d->out_h * d->batch;
+  // a group of three output channels and fewer fills less than a tenth of a tile's 32 channels
+  if (groups > 1 && d->out_c / groups < 4) return false;
+  // a handful of products per output: one thread per output is quicker than staging a window (4.3 against 5.7 us)
+  if (dt != kI8 && reduction <= 9 && macs <= 4000000) return false;
+  if (dt == kI8 && groups == 1) {
+    if (ConvIgemmPersists(d)) return false;
+    // shallow inputs whose rows are whole dwords at stride 1: conv2d_igemm_i8 stages all channels of a tile in one aligned
+    // pass and its weights fit LDS beside it (6.9 against 8.9 us at 32 -> 80 on 16 x 16, batch 27); with more work than
+    // this its tiles queue up (43 against 28 us at 8 -> 416 on 40 x 40, batch 24)
+    if (d->in_c <= 32 && d->stride_w == 1 && d->stride_h == 1 && d->in_w % 4 == 0 && macs <= 400000000 && reduction <= 512) return false;
+  }
+  return true;
+}
+
+// Claims dense and grouped convolutions with constant weights on quantized (no accumulator on a rounding tie), float16 or
+// float32 tensors whose staged window fits LDS a granule of channels at a time.
+int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const void* bias_host) {
+  if (!w_host || op->fused_add || op->kind != OP_CONV2D || d->multiplier != 0) return TVX_E_UNSUPPORTED;
+  int dt;
+  if (op->quantized) dt = kI8;
+  else if (d->in_dtype == TVX_F16 && d->w_dtype == TVX_F16 && d->out_dtype == TVX_F16) dt = kF16;
+  else if (d->in_dtype == TVX_F32 && d->w_dtype == TVX_F32 && d->out_dtype == TVX_F32) dt = kF32;
+  else return TVX_E_UNSUPPORTED;
+  const int E = dt == kI8 ? 1 : dt == kF16 ? 2 : 4;
+  bool forced = false;
+  if (const char* f = getenv("TVX_CONV_TILE")) {  // test lever: 0 declines, 1 claims also where another kernel is the better choice
+    if (atoi(f) == 0) return TVX_E_UNSUPPORTED;
+    forced = true;
+  }
+  if (!forced && !IsBetterChoice(d, dt)) return TVX_E_UNSUPPORTED;
+
+  TileArgs a{};
+  int W = d->in_w, H = d->in_h, OW = d->out_w, OH = d->out_h;
+  const int kh = d->k_h, kw = d->k_w, dh = d->dilation_h, dw = d->dilation_w;
+  const bool flat = kh == 1 && kw == 1 && d->stride_w == 1 && d->stride_h == 1 && d->pad_left == 0 && d->pad_top == 0 && OW == W && OH == H;
+  if (flat) { W = OW = W * H; H = OH = 1; }  // a 1 x 1 window needs no rows: an image is one
+  const int group_px = dt == kF32 ? 4 : 8;
+  if (W * H < group_px) return TVX_E_UNSUPPORTED;
+  const int groups = d->groups > 1 ? d->groups : 1;
+  a.C = d->in_c; a.H = H; a.W = W; a.OC = d->out_c; a.OH = OH; a.OW = OW; a.batch = d->batch;
+  a.sh = d->stride_h; a.sw = d->stride_w; a.pad_t = d->pad_top; a.pad_l = d->pad_left;
+  a.icg = a.C / groups; a.ocg = a.OC / groups;
+  const int granules = (a.icg * E + 15) / 16, taps = kh * kw;
+  if (taps > 1024) return TVX_E_UNSUPPORTED;
+  const uint64_t image = static_cast<uint64_t>(a.C) * H * W * E, out_image = static_cast<uint64_t>(a.OC) * OH * OW;
+  a.row_step = kh == 1 ? a.sh : 1;
+  a.row_stride = kh == 1 ? 1 : a.sh;
+
+  const int x_u8 = d->in_dtype == TVX_U8, w_u8 = d->w_dtype == TVX_U8;
+  const int zxs = dt == kI8 ? d->in_zp - (x_u8 ? 128 : 0) : 0;
+  const int zws = dt == kI8 ? op->w_zp - (w_u8 ? 128 : 0) : 0;
+
+  // ---- the tile ----
+  int want = -1, want_tw = 0;
+  if (const char* f = getenv("TVX_CONV_TILE_SHAPE")) want = atoi(f);  // test lever
+  if (const char* f = getenv("TVX_CONV_TILE_COLS")) want_tw = atoi(f);  // test lever
+  Geometry best{};
+  best.shape = -1;
+  for (int sidx = 0; sidx < kShapeCount; ++sidx) {
+    if (want >= 0 && sidx != want) continue;
+    const Shape& sp = kShapes[sidx];
+    const int oc_blocks = (a.ocg + sp.channels - 1) / sp.channels;
+    const int cand[] = {OW, (OW + 1) / 2, (OW + 2) / 3, 8, 16, 32, 64, 128};
+    for (int tw : cand) {
+      if (want_tw && tw != want_tw) continue;
+      if (tw < 1 || tw > OW || tw > sp.pixels) continue;
+      Geometry g{};
+      g.shape = sidx;
+      g.TW = tw;
+      g.TH = std::min(OH, sp.pixels / tw);
+      // rows spread evenly over the tiles of a column
+      g.TH = (OH + (OH + g.TH - 1) / g.TH - 1) / ((OH + g.TH - 1) / g.TH);
+      g.G = g.TW == OW && g.TH == OH ? std::min<int>(d->batch, sp.pixels / (g.TW * g.TH)) : 1;
+      g.IW = (g.TW - 1) * a.sw + (kw - 1) * dw + 1;
+      g.IH = (g.TH - 1) * a.row_stride + (kh - 1) * dh + 1;
+      const int64_t npx = static_cast<int64_t>(g.G) * g.IH * g.IW;
+      if (npx > 40000) continue;
+      for (g.chunks = 1; g.chunks <= granules; ++g.chunks) {
+        g.gpc = (granules + g.chunks - 1) / g.chunks;
+        if (g.chunks > 1 && (granules + g.gpc - 1) / g.gpc != g.chunks) continue;
+        g.pitch = (g.gpc | 1) * 16;
+        const int steps = (taps * g.gpc + 1) / 2;
+        int64_t bytes = RoundUp(std::max<int64_t>(npx * g.pitch, sp.ks > 1 ? sp.ks * sp.pixels * sp.channels * 4 : 0), 16);
+        bytes += 2 * RoundUp(steps + 12, 4) * 4;
+        if (zws) bytes += npx * 4 + sp.pixels * 4;
+        g.lds_bytes = static_cast<int>(std::min<int64_t>(bytes, 1 << 30));
+        if (g.lds_bytes <= 78 * 1024) break;
+      }
+      if (g.chunks > granules) continue;
+      const int64_t tiles = static_cast<int64_t>((OW + g.TW - 1) / g.TW) * ((OH + g.TH - 1) / g.TH) * ((d->batch + g.G - 1) / g.G);
+      g.wgs = tiles * oc_blocks * groups;
+      if (g.wgs > 0x3fffffff) continue;
+      g.cost = Cost(sp, g, dt, taps, group_px, zws != 0, (a.icg * E) % 16 == 0, (a.pad_l || a.pad_t) && taps > 1, OW);
+      if (best.shape < 0 || g.cost < best.cost) best = g;
+    }
+  }
+  if (best.shape < 0) return TVX_E_UNSUPPORTED;
+  const Geometry& g = best;
+  const Shape& sp = kShapes[g.shape];
+  if (image * g.G >= (1ull << 32) || out_image * g.G >= (1ull << 31)) return TVX_E_UNSUPPORTED;
+
+  a.TW = g.TW; a.TH = g.TH; a.G = g.G; a.NQ = g.TW * g.TH * g.G;
+  a.IW = g.IW; a.IH = g.IH; a.pitch = g.pitch; a.gpc = g.gpc; a.chunks = g.chunks;
+  a.steps = (taps * g.gpc + 1) / 2;
+  a.odd = (taps * g.gpc) & 1;
+  a.steps_pad = RoundUp(a.steps + 12, 4);
+  a.taps_w = kw; a.taps_h = kh; a.dil_col = dw; a.dil_row = dh * g.IW;
+  a.ncg = (g.IW + group_px - 1) / group_px;
+  a.cells = g.G * g.IH * a.ncg;
+  a.gl = 1;
+  for (int v = 2; v <= 6; ++v) if (a.gpc % v == 0) a.gl = v;
+  if (a.gl == 1) a.gl = a.gpc;
+  a.tiles_x = (OW + g.TW - 1) / g.TW;
+  a.tiles_y = (OH + g.TH - 1) / g.TH;
+  a.tiles_per_group = (a.ocg + sp.channels - 1) / sp.channels;
+  a.oc_blocks = a.tiles_per_group * groups;
+  a.total = static_cast<int>(g.wgs);
+  a.per_xcd = (a.total + 7) / 8;
+  a.npx = g.G * g.IH * g.IW;
+  a.items = a.cells * a.gpc;
+  a.plane_bytes = static_cast<uint32_t>(H) * W * E;
+  a.image_bytes = a.plane_bytes * a.C;
+  a.at_max = H * W - group_px;
+  const int64_t npx = static_cast<int64_t>(g.G) * g.IH * g.IW;
+  const int64_t window = RoundUp(std::max<int64_t>(npx * g.pitch, sp.ks > 1 ? sp.ks * sp.pixels * sp.channels * 4 : 0), 16);
+  a.off_tab = static_cast<int>(window);
+  a.off_sum = a.off_tab + 2 * a.steps_pad * 4;
+  a.off_zt = a.off_sum + (zws ? static_cast<int>(npx) * 4 : 0);
+  a.m_gl = Magic(a.gl); a.m_cells = Magic(a.cells); a.m_ncg = Magic(a.ncg); a.m_ih = Magic(a.IH); a.m_iw = Magic(a.IW); a.m_tw = Magic(a.TW); a.m_thtw = Magic(a.TH * a.TW);
+  a.m_ocb = Magic(a.oc_blocks); a.m_tpg = Magic(a.tiles_per_group); a.m_tx = Magic(a.tiles_x); a.m_ty = Magic(a.tiles_y);
+  // a reciprocal is exact while dividend * divisor < 2^32
+  if (static_cast<uint64_t>(a.total) * std::max({a.oc_blocks, a.tiles_x, a.tiles_y}) >= (1ull << 32)) return TVX_E_UNSUPPORTED;
+  if (static_cast<uint64_t>(npx) * a.gpc * std::max({a.gpc, a.cells, a.IH, a.IW}) >= (1ull << 32)) return TVX_E_UNSUPPORTED;
+  a.xor_mask = dt == kI8 && x_u8 ? 0x80808080u : 0u;
+  a.pad_full = static_cast<uint32_t>(zxs & 0xff) * 0x01010101u;
+  a.last_granule = granules - 1;
+  for (int q = 0; q < 4; ++q) {
+    const int nb = a.icg * E - (granules - 1) * 16 - 4 * q;
+    a.pad_last[q] = nb >= 4 ? a.pad_full : nb <= 0 ? 0u : a.pad_full & ((1u << (8 * nb)) - 1u);
+  }
+  a.zws = zws;
+  a.out_zp = d->out_zp; a.lo = op->act_lo; a.hi = op->act_hi; a.act = d->activation;
+
+  // ---- the step table ----
+  std::vector<int32_t> tab(2 * static_cast<size_t>(a.steps_pad), 0);
+  for (int q = 0; q < taps * a.gpc; ++q) {
+    const int t = q / a.gpc, gr = q % a.gpc, ky = t / kw, kx = t % kw;
+    tab[static_cast<size_t>(q & 1) * a.steps_pad + q / 2] = (ky * dh * g.IW + kx * dw) * g.pitch + gr * 16;
+  }
+
+  // ---- weights [oc][c][ky][kx] -> fragment order; the bias takes the zero points' constants ----
+  const size_t alloc_oc = static_cast<size_t>(a.oc_blocks) * sp.channels;
+  const size_t tile_bytes = static_cast<size_t>(a.chunks) * a.steps * 1024;
+  std::vector<uint8_t> packed(alloc_oc / 32 * tile_bytes, 0);
+  std::vector<int32_t> biasf(dt == kI8 ? alloc_oc : 0, 0);
+  std::vector<int32_t> mult, shift;
+  if (dt == kI8) {
+    // (slots past a group's channels: a real channel's record, so that they do not decide the requantization flavour)
+    mult.assign(alloc_oc, op->h_mult[0]);
+    shift.assign(alloc_oc, op->h_shift[0]);
+  }
+  const uint8_t* src = static_cast<const uint8_t*>(w_host);
+  const int32_t* bi = static_cast<const int32_t*>(bias_host);
+  const uint8_t flip = w_u8 ? 0x80 : 0;
+  const int epg = 16 / E;  // elements of a granule
+  for (int oc = 0; oc < a.OC; ++oc) {
+    const int grp = oc / a.ocg, ol = oc % a.ocg;
+    const size_t slot = static_cast<size_t>(grp) * a.tiles_per_group * sp.channels + ol;
+    uint8_t* tile = packed.data() + slot / 32 * tile_bytes + (slot % 32) * 16;
+    const uint8_t* ws = src + static_cast<size_t>(oc) * a.icg * taps * E;
+    int64_t sw = 0;
+    for (int c = 0; c < a.icg; ++c) {
+      const int gg = c / epg, chunk = gg / a.gpc, gr = gg % a.gpc;
+      uint8_t* cp = tile + static_cast<size_t>(chunk) * a.steps * 1024 + (c % epg) * E;
+      for (int t = 0; t < taps; ++t, ws += E) {
+        const int q = t * a.gpc + gr;
+        uint8_t* to = cp + static_cast<size_t>(q >> 1) * 1024 + (q & 1) * 512;
+        if (E == 1) {
+          const uint8_t v = *ws ^ flip;
+          *to = v;
+          sw += static_cast<int8_t>(v);
+        } else {
+          std::memcpy(to, ws, E);
+        }
+      }
+    }
+    if (dt == kI8) {
+      const int64_t v = (bi ? bi[oc] : 0) - static_cast<int64_t>(zxs) * sw + static_cast<int64_t>(taps) * a.icg * zxs * zws;
+      biasf[slot] = static_cast<int32_t>(static_cast<uint32_t>(v));
+      mult[slot] = op->h_mult[oc];
+      shift[slot] = op->h_shift[oc];
+    }
+  }
+  int s = op->packed.Upload(packed.data(), packed.size());
+  if (s == TVX_OK) s = op->aux3.Upload(tab.data(), tab.size() * 4);
+  if (s == TVX_OK && dt == kI8) {
+    std::vector<int32_t> rqt;
+    const int rq_mode = BuildRequantRecords(mult, shift, static_cast<int>(alloc_oc), static_cast<int>(alloc_oc), d->out_zp, &rqt,
+                                    AccumulatorBound(static_cast<uint64_t>(taps) * a.icg, bias_host, d->out_c));
+    if (rq_mode != kRqFastNoTie) return TVX_E_UNSUPPORTED;
+    s = op->aux.Upload(biasf.data(), biasf.size() * 4);
+    if (s == TVX_OK) s = op->aux2.Upload(rqt.data(), rqt.size() * 4);
+    a.biasf = op->aux.as<int32_t>();
+    a.rq = op->aux2.as<tvx_v4i>();
+  } else if (s == TVX_OK && bias_host) {
+    s = op->bias.Upload(bias_host, static_cast<size_t>(a.OC) * 4);
+    a.biasfl = op->bias.as<float>();
+  }
+  if (s != TVX_OK) return s;
+  a.wpk = op->packed.as<v4i>();
+  a.tab = op->aux3.as<int>();
+
+  Plan plan{};
+  plan.a = a;
+  plan.fn = sp.fn[dt][a.chunks > 1];
+  plan.lds_bytes = static_cast<unsigned>(g.lds_bytes);
+  plan.grid = static_cast<unsigned>(a.per_xcd) * 8;
+  plan.threads = 64u * sp.waves;
+  plan.elem = E;
+  if (plan.lds_bytes > 48 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(plan.fn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(plan.lds_bytes));
+    if (e != hipSuccess) return SetError(TVX_E_DEVICE, "hipFuncSetAttribute(dynamic LDS %u): %s", plan.lds_bytes, hipGetErrorString(e));
+  }
+  op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
+  op->run = ConvTileRun;
+  // (the names these shapes have always been reported under: implicit GEMM for dense int8, GEMM over windows for the rest)
+  op->kernel_name = dt == kF32 ? "conv2d_igemm_f32" : dt == kF16 ? "conv2d_gemm_f16" : groups > 1 ? "conv2d_gemm_i8" : "conv2d_igemm_i8";
+  return TVX_OK;
+}
+
+}  // namespace tvx

@@ -29,6 +29,9 @@ int FcMfmaSetup(tvx_op*, const tvx_fc_desc*, const void*, const void*);
 
 // int8 MFMA implicit-GEMM convolution (conv_igemm_i8.hip)
 int ConvIgemmSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
+bool ConvIgemmPersists(const tvx_conv2d_desc*);
+// one output tile per workgroup: dense or grouped, int8 / float16 / float32 (conv_tile.hip)
+int ConvTileSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 // the same for layers whose weights and two halo tiles fit LDS: one sixteen-wavefront workgroup per CU (conv_band_i8.hip)
 int ConvBandSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 // Dense quantized conv whose whole window (C * Kh * Kw) is at most 64 bytes: im2col rows in LDS + MFMA.
