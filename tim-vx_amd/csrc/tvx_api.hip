@@ -123,6 +123,29 @@ int BuildRequantRecords(const std::vector<int32_t>& mult, const std::vector<int3
   return rq;
 }
 
+bool BuildTieRecords(const std::vector<int32_t>& mult, const std::vector<int32_t>& shift, int channels, int alloc, int out_zp, int64_t acc_bound,
+                     std::vector<int32_t>* records, int* pre, bool* ties) {
+  *pre = 0;
+  *ties = false;
+  for (int c = 0; c < channels; ++c)
+    if (mult[c]) *pre = std::max(*pre, 33 - shift[c]);
+  if (*pre > 16 || (acc_bound << *pre) >= (int64_t{1} << 31)) return false;
+  records->assign(static_cast<size_t>(alloc) * 4, 0);
+  for (int c = 0; c < alloc; ++c) {
+    const int32_t m = c < channels ? mult[c] : 0, s = m ? shift[c] + *pre : 33;
+    if (s - 32 > 20) return false;
+    // a tie needs v * m = 2^(s-1) (mod 2^s): v's lowest set bit is bit s - 1 - ctz(m); out of reach: bit 31 (|v| < 2^31)
+    int bit = m ? s - 1 - __builtin_ctz(static_cast<uint32_t>(m)) : 31;
+    if (bit > 31 || (int64_t{1} << bit) > (acc_bound << *pre)) bit = 31;
+    else *ties = true;
+    int32_t* q = &(*records)[static_cast<size_t>(c) * 4];
+    q[0] = m;
+    q[1] = (s - 32) | bit << 8;
+    q[2] = (1 << (s - 33)) + (out_zp << (s - 32));
+  }
+  return true;
+}
+
 void ActRange(int out_dtype, float out_scale, int32_t out_zp, int act, int32_t* lo, int32_t* hi) {
   *lo = out_dtype == TVX_U8 ? 0 : -128;
   *hi = out_dtype == TVX_U8 ? 255 : 127;
@@ -452,7 +475,8 @@ int tvx_conv2d_add_create(const tvx_conv2d_desc* d, const tvx_eltwise_desc* add,
   op->w_zp = d->w_scales ? 0 : d->w_zp;
   s = BuildRequantTables(d->out_c, d->in_scale, d->w_scale, d->w_scales, d->out_scale, &op->h_mult, &op->h_shift);
   ActRange(d->out_dtype, d->out_scale, d->out_zp, d->activation, &op->act_lo, &op->act_hi);
-  if (s == TVX_OK) s = PwConvSetup(op, &norm, weights_host, bias_host);  // the kernel that has the fused form
+  if (s == TVX_OK) s = PwRegSetup(op, &norm, weights_host, bias_host);  // the kernels that have the fused form
+  if (s == TVX_E_UNSUPPORTED) s = PwConvSetup(op, &norm, weights_host, bias_host);
   if (s != TVX_OK) {
     delete op;
     return s == TVX_E_UNSUPPORTED ? SetError(TVX_E_UNSUPPORTED, "tvx_conv2d_add_create: no fused kernel for this convolution") : s;

@@ -183,6 +183,54 @@ __device__ __forceinline__ uint32_t RequantPack4(const int (&v)[4], const tvx_v4
   return PackBytes(r[0], r[1], r[2], r[3]);
 }
 
+// Exact ties in front of RequantPack4's no-tie form: an accumulator v lies on k + .5 exactly when its lowest set bit is the
+// channel's tie bit (bits 8 and up of q[1], see BuildTieRecords). Those for which rounding half up would give an odd number are
+// lowered by one, which rounds them down (the multiplier is below 1). Two instructions an accumulator where there are none.
+template <int N>
+__device__ __forceinline__ void LowerOddTies(int (&v)[N], const tvx_v4i& q) {
+  const uint32_t bit = 1u << (q[1] >> 8), mask = 2 * bit - 1;
+  uint32_t least = ~0u;
+#pragma unroll
+  for (int e = 0; e < N; ++e) least = min(least, (static_cast<uint32_t>(v[e]) ^ bit) & mask);
+  if (least == 0) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      const uint32_t off = (static_cast<uint32_t>(v[e]) ^ bit) & mask;
+      v[e] -= ((__mulhi(v[e], q[0]) + (1 << ((q[1] & 31) - 1))) >> (q[1] & 31)) & 1 & (off == 0);
+    }
+  }
+}
+
+// Four accumulators of one channel -> four codes in a dword by instructions of the gfx950: the high half of a 64-bit
+// multiply-add is product and rounding constant in one (`round`: the constant in the high half), a shift that saturates to signed
+// bytes takes two. 12 cycles a code and SIMD against 19 for RequantPack4 and its like (high multiply, add, clamp, shift into a byte).
+// Codes of uint8 tensors come out moved to the signed domain: records built with the zero point less 128, the caller flips the
+// sign bits. NARROW: the clamp may be narrower than a byte - lo_t, hi_t, shifted up by t.
+__device__ __forceinline__ int64_t RoundHigh(int rounding) {
+  int64_t r = static_cast<int64_t>(static_cast<uint64_t>(static_cast<uint32_t>(rounding)) << 32);
+  asm("" : "+v"(r));  // (were its low half known to be zero, the multiply-add would be split into a high multiply and an add)
+  return r;
+}
+__device__ __forceinline__ int MulHiAdd(int v, int mult, int64_t round) {  // no inline asm: v may be a matrix instruction's result,
+  return static_cast<int>((static_cast<int64_t>(v) * mult + round) >> 32);  // whose wait states the compiler has to see to
+}
+__device__ __forceinline__ uint32_t ShiftSaturate2(int a, int b, int t) {  // (the upper half of the result is left over)
+  uint32_t d;
+  asm("v_ashr_pk_i8_i32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(t));
+  return d;
+}
+template <bool NARROW>
+__device__ __forceinline__ uint32_t RequantSaturate4(const int (&v)[4], int mult, int t, int64_t round, int lo_t, int hi_t) {
+  int h[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) h[e] = MulHiAdd(v[e], mult, round);
+  if (NARROW) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) h[e] = Med3(h[e], lo_t, hi_t);
+  }
+  return __builtin_amdgcn_perm(ShiftSaturate2(h[2], h[3], t), ShiftSaturate2(h[0], h[1], t), 0x05040100);
+}
+
 // Four accumulators of one channel requantized together (the 32-bit record forms). `ties` (wave-uniform: a kernel
 // argument) tells whether any accumulator of the operator can land on an exact .5: only then is the round-half-even
 // fix-up executed.
@@ -266,6 +314,11 @@ __device__ __forceinline__ int Window(const int (&arr)[N]) {
 int BuildRequantRecords(const std::vector<int32_t>& mult, const std::vector<int32_t>& shift,
                         int channels, int alloc, int out_zp, std::vector<int32_t>* records,
                         int64_t acc_bound = -1);
+// The records for LowerOddTies + RequantPack4<kRqFastNoTie>: {mult, t | tie bit << 8, rounding constant, 0}. A kernel shifts its
+// accumulators left by *pre first (multipliers of .25 and more: their shift alone is below 33; usually 0) and looks for ties
+// if *ties. False where a channel has no such form: a multiplier below 2^-20, or accumulators too large for *pre.
+bool BuildTieRecords(const std::vector<int32_t>& mult, const std::vector<int32_t>& shift, int channels, int alloc, int out_zp, int64_t acc_bound,
+                     std::vector<int32_t>* records, int* pre, bool* ties);
 // reduction length * 255 * 255 + max |bias|: bound of sum (x - zx)(w - zw) + bias for 8-bit operands
 int64_t AccumulatorBound(uint64_t reduction, const void* bias_host, uint32_t channels);
 // Per-output-channel requantization tables (mult/shift) for a conv / FC.

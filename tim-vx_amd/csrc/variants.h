@@ -40,6 +40,9 @@ int ConvIm2colSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 // pointwise (1x1) convolution with the whole channel depth of a pixel tile in LDS (pwconv_i8.hip)
 int PwConvSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 
+// ... with a wavefront's pixels in registers (pwconv_reg_i8.hip)
+int PwRegSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
+
 // depthwise 3x3 stencil (dwconv3x3_i8.hip)
 int DwConv3x3Setup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 
