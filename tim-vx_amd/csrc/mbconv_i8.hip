@@ -4,10 +4,10 @@
 // chains when it verifies the graph (reference: src/tim/vx/internal/src/vsi_nn_graph.c:1591-1603); the
 // operators it fuses are the Conv2d nodes of src/tim/vx/internal/src/ops/vsi_nn_op_conv2d.c:35-118.
 //
-// The expanded tensor never leaves the CU. A workgroup (four wavefronts) owns a band of output rows of one
+// The expanded tensor never leaves the CU. A workgroup (four or eight wavefronts) owns a band of output rows of one
 // image (at most 32 or 64 output pixels) and first transposes the band's input rows - with the halo the 3x3
 // window needs - into LDS as the MFMA operand [pixel][channel]. The expanded channels are then walked in
-// chunks of 32, wavefront w taking chunks w, w + 4, ...: expansion of all halo pixels for the chunk
+// chunks of 32, wavefront w taking chunks w, w + 4 (8), ...: expansion of all halo pixels for the chunk
 // (v_mfma_i32_32x32x32_i8, requantized into a wavefront-private [channel][pixel] image), depthwise stencil on
 // that image (signed dot4 over byte windows, requantized and transposed into the projection's operand), and
 // the chunk's contribution to every output channel accumulated in registers. No barrier inside the walk: a
@@ -25,8 +25,9 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
-constexpr int kThreads = 256;
-constexpr int kWaves = kThreads / 64;
+constexpr int kMinWaves = 4;
+// (two wavefronts a SIMD within 256 registers)
+constexpr int MaxWaves(int acc_tiles) { return acc_tiles <= 5 ? 8 : kMinWaves; }
 constexpr int kMStride = 48;      // bytes per pixel row of the projection operand (32 channels + 16: bank spread)
 constexpr int kMaxCinSteps = 5;   // 32-channel steps of the expansion's reduction (160 input channels)
 
@@ -120,13 +121,13 @@ struct DwRow {
 // (the register budget follows the accumulators: two wavefronts per SIMD up to five output tiles - three with two
 // tiles, 168 registers, spill 36 bytes per lane and measure slower -, one beyond)
 template <int W, int S, int MO, int NTMAX, bool ADD>
-__global__ void __launch_bounds__(kThreads, (MO * NTMAX <= 5 ? 2 : 1)) MbConvKernel(MbArgs a) {
+__global__ void __launch_bounds__(MaxWaves(MO * NTMAX) * 64) MbConvKernel(MbArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   constexpr int PL = S == 1 ? 1 : 0;               // left (and top) padding of the depthwise convolution
   constexpr int OW = (W + S - 1) / S;
   constexpr int NW = (W + 5) / 4;                  // dwords of a normalized input row: bytes 0 .. W + PL
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), threads = blockDim.x, waves = threads >> 6;
   const int n = blockIdx.x / a.bands, band = blockIdx.x - n * a.bands;
   const int or0 = band * a.R;
   const int rows_out = min(a.R, a.OH - or0);
@@ -166,7 +167,7 @@ __global__ void __launch_bounds__(kThreads, (MO * NTMAX <= 5 ? 2 : 1)) MbConvKer
     const uint8_t* xn = a.x + static_cast<size_t>(n) * a.Cin * plane;
     const int live_lo = max(0, -ir0) * W, live_hi = min(a.IR, a.H - ir0) * W;  // the live bytes of a channel's halo rows
     const uint32_t xor4 = static_cast<uint32_t>(a.x_xor) * 0x01010101u;
-    for (int unit = tid; unit < units; unit += kThreads) {
+    for (int unit = tid; unit < units; unit += threads) {
       const int c4 = unit / quads, p0 = (unit - c4 * quads) * 4;
       const int c = c4 * 4;
       const int at = ir0 * W + p0;                     // byte offset in the plane (negative above the image)
@@ -194,7 +195,7 @@ __global__ void __launch_bounds__(kThreads, (MO * NTMAX <= 5 ? 2 : 1)) MbConvKer
       for (int i = 0; i < 4; ++i) *reinterpret_cast<uint32_t*>(xin + (p0 + i) * a.xs + c) = px[i];
     }
   }
-  for (int i = tid; i < a.nt * MO * 256; i += kThreads) reinterpret_cast<v4i*>(lds + a.off_red)[i] = v4i{0, 0, 0, 0};
+  for (int i = tid; i < a.nt * MO * 256; i += threads) reinterpret_cast<v4i*>(lds + a.off_red)[i] = v4i{0, 0, 0, 0};
   __syncthreads();
 
   v16i acc_out[MO][NTMAX];
@@ -216,10 +217,10 @@ __global__ void __launch_bounds__(kThreads, (MO * NTMAX <= 5 ? 2 : 1)) MbConvKer
           Requant8x4Pack(av, rq1, a.e_zp, a.e_lo, a.e_hi, a.ties1) ^ static_cast<uint32_t>(a.e_xor4);
     }
   };
-  for (int chunk = wave; chunk < a.chunks; chunk += kWaves) {
+  for (int chunk = wave; chunk < a.chunks; chunk += waves) {
     const int ch = chunk * 32 + frow;  // this lane's expanded channel, in all three phases
     const ExpandOperands cur = next;
-    fetch(chunk + kWaves, next);
+    fetch(chunk + waves, next);
     const v4i dk = a.dwk[ch];
     const v4i rq2 = a.q2[ch];
     v4i w2f[NTMAX];
@@ -301,7 +302,7 @@ __global__ void __launch_bounds__(kThreads, (MO * NTMAX <= 5 ? 2 : 1)) MbConvKer
   int* red = reinterpret_cast<int*>(lds + a.off_red);
   const size_t out_plane = static_cast<size_t>(a.OH) * OW;
   const int units = a.nt * MO * 4;
-  constexpr int kMaxUnits = (NTMAX * MO * 4 + kWaves - 1) / kWaves;
+  constexpr int kMaxUnits = (NTMAX * MO * 4 + kMinWaves - 1) / kMinWaves;
   // what the units need from memory is requested first: the sums then form under these loads
   int bias3[kMaxUnits];
   v4i rq3[kMaxUnits];
@@ -310,7 +311,8 @@ __global__ void __launch_bounds__(kThreads, (MO * NTMAX <= 5 ? 2 : 1)) MbConvKer
   int px0[kMaxUnits];
 #pragma unroll
   for (int i = 0; i < kMaxUnits; ++i) {
-    const int u = min(wave + i * kWaves, units - 1);
+    const int u = wave + i * waves;
+    if (u >= units) break;
     const int t = u / (MO * 4), mo = (u >> 2) % MO, gq = u & 3;
     const int oc = t * 32 + frow;
     bias3[i] = a.b3[oc];
@@ -342,7 +344,7 @@ __global__ void __launch_bounds__(kThreads, (MO * NTMAX <= 5 ? 2 : 1)) MbConvKer
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < kMaxUnits; ++i) {
-    const int u = wave + i * kWaves;
+    const int u = wave + i * waves;
     if (u >= units) break;
     const int t = u / (MO * 4), gq = u & 3;
     const int oc = t * 32 + frow;
@@ -392,7 +394,7 @@ MbFn KernelOf(int w, int s, int nt) {
 struct Plan {
   MbArgs a;
   int w, s, lds_bytes;
-  unsigned grid;
+  unsigned grid, block;
 };
 
 MbFn Kernel(const Plan& p) {
@@ -408,7 +410,7 @@ int MbConvRun(tvx_op* op, const void* in0, const void* in1, void* out, hipStream
   if (a.add_mode && !in1) return SetError(TVX_E_INVALID, "pwconv_dwconv3x3_pwconv_i8: the fused Add needs its second operand as in1");
   if (a.aligned4 && ((reinterpret_cast<uintptr_t>(out) | (a.add_mode ? reinterpret_cast<uintptr_t>(in1) : 0)) & 3))
     a.aligned4 = 0;
-  hipLaunchKernelGGL(Kernel(*plan), dim3(plan->grid), dim3(kThreads), plan->lds_bytes, st, a);
+  hipLaunchKernelGGL(Kernel(*plan), dim3(plan->grid), dim3(plan->block), plan->lds_bytes, st, a);
   TVX_HIP_CHECK(hipGetLastError());
   return TVX_OK;
 }
@@ -494,12 +496,20 @@ int MbConvSetup(tvx_op* op, const MbStage& ex, const MbStage& dw, const tvx_conv
   a.ep = mh * 32 + 4;
   a.off_wave = RoundUp(mh * 32 * a.xs, 16);
   a.wave_bytes = RoundUp(16 + 32 * a.ep + MO * 32 * kMStride, 16);
-  a.off_red = a.off_wave + kWaves * a.wave_bytes;
+  const uint64_t wgs = static_cast<uint64_t>(e->batch) * a.bands;
+  // With at most one workgroup a CU eight wavefronts walk the chunks in half the rounds; with more, four and a second workgroup
+  // are better. 64 -> 384 -> 64 and 96 -> 576 -> 96 channels on 14 x 14: batch 1 11.9 -> 9.1 and 20.1 -> 13.1 us, batch 64 14.3 and 23.7
+  // against 19.1 and 24.9 with eight.
+  int waves = wgs <= 256 ? MaxWaves(MO * (nt <= 2 ? 2 : nt <= 5 ? 5 : 10)) : kMinWaves;
+  if (const char* f = getenv("TVX_MBCONV_WAVES")) waves = std::max(kMinWaves, atoi(f));  // tuning aid
+  waves = std::min(waves, MaxWaves(MO * (nt <= 2 ? 2 : nt <= 5 ? 5 : 10)));
+  while (waves > kMinWaves && a.off_wave + waves * a.wave_bytes + nt * MO * 4096 > 160 * 1024) --waves;
+  plan.block = 64 * waves;
+  a.off_red = a.off_wave + waves * a.wave_bytes;
   plan.lds_bytes = a.off_red + nt * MO * 4096;
   if (plan.lds_bytes > 160 * 1024) return TVX_E_UNSUPPORTED;
-  const uint64_t grid = static_cast<uint64_t>(e->batch) * a.bands;
-  if (grid > 0x7fffffffull) return TVX_E_UNSUPPORTED;
-  plan.grid = static_cast<unsigned>(grid);
+  if (wgs > 0x7fffffffull) return TVX_E_UNSUPPORTED;
+  plan.grid = static_cast<unsigned>(wgs);
 
   // ---- expansion ----
   const bool x_u8 = e->in_dtype == TVX_U8, w1_u8 = e->w_dtype == TVX_U8;
