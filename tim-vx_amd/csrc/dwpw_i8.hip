@@ -28,7 +28,7 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
-constexpr int kThreads = 256;
+constexpr int kWaves = 4, kMaxWaves = 8;  // of a workgroup
 constexpr int kMaxSlots = 512;      // most pixel slots of a tile (32-pixel MFMA tiles, a multiple of four of them)
 constexpr int kStageStride = 40;    // bytes per staged output row of 32 pixels (8-byte aligned rows)
 constexpr int kStageBytes = 32 * kStageStride;
@@ -171,11 +171,11 @@ __device__ __forceinline__ void PatchCompute(const DwPwArgs& a, const ChannelCon
 // (two wavefronts per SIMD at least: within 256 registers the compiler keeps MFMA accumulators in ordinary vector
 // registers, where the epilogue reads them, instead of moving every value out of the accumulation registers first)
 template <int S, int RPT, bool ADD>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) DwPwKernel(DwPwArgs a) {
+__global__ void __launch_bounds__(kMaxWaves * 64) __attribute__((amdgpu_waves_per_eu(2))) DwPwKernel(DwPwArgs a) {
   extern __shared__ __attribute__((aligned(16))) int8_t lds[];
   constexpr int PL = S == 1 ? 1 : 0;
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), threads = blockDim.x, waves = threads >> 6;
   // an XCD gets a contiguous run of tiles: vertically neighbouring tiles share input rows in its L2
   int wg = blockIdx.x;
   {
@@ -190,7 +190,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   int8_t* mid = lds;                               // [channel][slots + 4]: the depthwise result of the tile
   int8_t* xl = lds + a.cp * mid_stride;            // [pixel slot][pix_stride]: the MFMA operand tile
   int8_t* stage = xl + a.slots * a.pix_stride + wave * kStageBytes;
-  int8_t* w_lds = xl + a.slots * a.pix_stride + 4 * kStageBytes;  // the pointwise weights, in fragment order
+  int8_t* w_lds = xl + a.slots * a.pix_stride + waves * kStageBytes;  // the pointwise weights, in fragment order
   const int oc_alloc = a.oc_tiles * 32;
   v4i* rq_lds = reinterpret_cast<v4i*>(w_lds + oc_alloc * a.cp);
   int* bias_lds = reinterpret_cast<int*>(rq_lds + oc_alloc);
@@ -200,10 +200,10 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     typedef const __attribute__((address_space(1))) void* gptr;
     typedef __attribute__((address_space(3))) void* lptr;
     const int chunks = oc_alloc * a.cp >> 4;
-    for (int i = wave * 64; i < chunks; i += kThreads)
+    for (int i = wave * 64; i < chunks; i += threads)
       if (i + lane < chunks)
         __builtin_amdgcn_global_load_lds((gptr)(a.wpk + i + lane), (lptr)(w_lds + i * 16), 16, 0, 0);
-    for (int i = wave * 64; i < oc_alloc; i += kThreads)
+    for (int i = wave * 64; i < oc_alloc; i += threads)
       if (i + lane < oc_alloc) {
         __builtin_amdgcn_global_load_lds((gptr)(a.rq + i + lane), (lptr)(rq_lds + i), 16, 0, 0);
         __builtin_amdgcn_global_load_lds((gptr)(a.biasf + i + lane), (lptr)(bias_lds + i), 4, 0, 0);
@@ -216,7 +216,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     constexpr int kRows = PatchShape<S, RPT>::kRows, kOwn = PatchShape<S, RPT>::kOwn;
     constexpr int kBatch = (24 / (kRows * kOwn)) > 8 ? 8 : ((24 / (kRows * kOwn)) < 1 ? 1 : (24 / (kRows * kOwn)));
     const int w4 = tid & ((1 << a.lpr_shift) - 1);
-    const int per_pass = kThreads >> a.lpr_shift;
+    const int per_pass = threads >> a.lpr_shift;
     const size_t plane = static_cast<size_t>(a.H) * a.W;
     const uint32_t plane32 = static_cast<uint32_t>(plane);
     const uint8_t* xn = a.x + static_cast<size_t>(n) * a.C * plane;
@@ -250,7 +250,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   {
     const int c4n = a.cp >> 2;                 // (a multiple of 8)
     const int items = (a.slots >> 2) * c4n;
-    for (int it = tid; it < items; it += kThreads) {
+    for (int it = tid; it < items; it += threads) {
       const int pq = __umulhi(it, a.c4n_magic), c4 = it - pq * c4n;
       const bool live = pq * 4 < a.P;
       uint32_t raw[4], t[4];
@@ -271,13 +271,18 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   // ---- 3. pointwise: a wavefront takes 32 pixel slots at a time and walks every output tile ----
   const int frag_row = lane & 31, frag_half = lane >> 5;
   const v4i fz = {a.neg_zws4, a.neg_zws4, a.neg_zws4, a.neg_zws4};
-  for (int part0 = wave * 32; part0 < a.P; part0 += 128) {
+  const int parts = (a.P + 31) >> 5;
+  int part = wave, tile = 0;  // (more wavefronts than 32-pixel parts: they share the output tiles)
+  for (;; part += waves) {
+    while (part >= parts) { part -= parts; ++tile; }
+    if (tile >= a.oc_tiles) break;
+    const int part0 = part * 32;
     // copy-out mapping of a staged 32 x 32 patch: lane -> 16-pixel chunk lane & 1 of output-channel row lane >> 1
     const int px_in_row = part0 + (lane & 1) * 16;
     const bool out_live = px_in_row < a.P;
     const size_t out_off = static_cast<size_t>(n) * a.OC * hw + static_cast<size_t>(g) * a.P + px_in_row;
     const int8_t* xa = xl + (part0 + frag_row) * a.pix_stride + frag_half * 16;
-    for (int tile = 0; tile < a.oc_tiles; ++tile) {
+    {
       const v4i q = rq_lds[tile * 32 + frag_row];
       const int nb = bias_lds[tile * 32 + frag_row];
       v16i acc;
@@ -325,7 +330,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
 
 struct Plan {
   DwPwArgs a;
-  int lds_bytes, stride, rpt;
+  int lds_bytes, stride, rpt, block;
   dim3 grid;
 };
 
@@ -349,7 +354,7 @@ int DwPwRun(tvx_op* op, const void* in0, const void* in1, void* out, hipStream_t
   if (a.add_mode && !in1) return SetError(TVX_E_INVALID, "dwpw_i8: the fused Add needs its second operand as in1");
   if ((reinterpret_cast<uintptr_t>(in0) & 3) | ((reinterpret_cast<uintptr_t>(out) | (a.add_mode ? reinterpret_cast<uintptr_t>(in1) : 0)) & 15))
     return SetError(TVX_E_INVALID, "dwpw_i8: the input must be 4-byte, the output (and the Add's operand) 16-byte aligned");
-  hipLaunchKernelGGL(Kernel(plan->stride, plan->rpt, a.add_mode != 0), plan->grid, dim3(kThreads), plan->lds_bytes, st, a);
+  hipLaunchKernelGGL(Kernel(plan->stride, plan->rpt, a.add_mode != 0), plan->grid, dim3(plan->block), plan->lds_bytes, st, a);
   TVX_HIP_CHECK(hipGetLastError());
   return TVX_OK;
 }
@@ -468,8 +473,19 @@ int DwPwSetup(tvx_op* op, const tvx_conv2d_desc* dw, const void* dw_w, const voi
     a.add_za = e.a_zp; a.add_zb = e.b_zp; a.add_zo = e.out_zp;
     ActRange(pw->out_dtype, e.out_scale, e.out_zp, TVX_ACT_NONE, &a.add_lo, &a.add_hi);
   }
-  const int lds_bytes = lds_of(rpt);
+  int lds_bytes = lds_of(rpt);
   if (lds_bytes > 160 * 1024) return TVX_E_UNSUPPORTED;
+  // Eight wavefronts where four would walk the channels in several rounds of loads (kBatch passes each) and the grid or LDS
+  // leaves a CU fewer than sixteen of them; with one round the second four only wait. MobileNetV2's blocks, 4 -> 8: batch 1
+  // 10.1 -> 8.2 us (144 channels, 56 x 56) and 11.1 -> 9.3 (192, 28 x 28), batch 64 41.0 -> 34.5 and 15.1 -> 14.0; 64 x 128 x 56 x 56
+  // -> 128 45.5 -> 36.1. One round: 32 x 32 x 112 x 112 -> 64 20.7 -> 24.7 us; sixteen in flight: 96, 112 -> 56, batch 64 26.5 -> 27.7.
+  const int kRows = S * (rpt - 1) + 3, batch = std::max(1, std::min(8, 24 / (kRows * S)));
+  const int passes = (C + (64 * kWaves >> lpr_shift) - 1) / (64 * kWaves >> lpr_shift);
+  const uint64_t resident = std::min<uint64_t>(std::min(4, 160 * 1024 / lds_bytes), (tiles + 255) / 256);
+  int waves = passes > batch && resident < 4 ? kMaxWaves : kWaves;
+  if (const char* f = getenv("TVX_DWPW_WAVES")) waves = std::min(kMaxWaves, std::max(kWaves, atoi(f)));  // tuning aid
+  if (lds_bytes + (waves - kWaves) * kStageBytes > 160 * 1024) waves = kWaves;
+  lds_bytes += (waves - kWaves) * kStageBytes;
   // pointwise weights in fragment order, constants folded into the bias (as PwConvSetup packs them)
   const int oc_alloc = a.oc_tiles * 32;
   std::vector<int8_t> packed(static_cast<size_t>(a.oc_tiles) * a.ksteps * 1024, 0);
@@ -515,6 +531,7 @@ int DwPwSetup(tvx_op* op, const tvx_conv2d_desc* dw, const void* dw_w, const voi
   plan.lds_bytes = lds_bytes;
   plan.stride = S;
   plan.rpt = rpt;
+  plan.block = 64 * waves;
   plan.grid = dim3(static_cast<unsigned>(tiles));
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
   op->run = DwPwRun;
