@@ -41,3 +41,14 @@ def test_pointwise_in_registers(oracle, n, c, h, w, oc, mode, monkeypatch):
                 assert np.array_equal(got, want[act]), (form, waves, act, int((got != want[act]).sum()))
             ran += 1
     assert ran
+
+
+@pytest.mark.parametrize("mode", ["u8", "i8pc"])
+@pytest.mark.parametrize("n,side", [(64, 7), (9, 13), (3, 10)])
+def test_add_written_over_its_operand(oracle, n, side, mode, monkeypatch):
+    """The fused Add with its result in the buffer of its other operand: planes whose last pixel group overlaps the one before."""
+    import test_gpu_parity as P
+    made, to_device = [], TC.to_device
+    monkeypatch.setattr(TC, "to_device", lambda a: made.append(to_device(a)) or made[-1])
+    monkeypatch.setattr(TC, "device_out", lambda count, dtype: made[-1])   # the operand, uploaded last
+    P.test_pointwise_conv_with_fused_add(oracle, side, n, mode, 2)

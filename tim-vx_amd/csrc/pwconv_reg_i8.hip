@@ -6,7 +6,7 @@
 // in fragment order (L1 / L2), so the input is read once and there is no barrier. Results come out as PW neighbouring pixels of
 // four channels a lane and are stored as they are, again runs of 16 * PW bytes.
 //  - Pixel groups never straddle images: the last group of an image begins at HW - PW and computes some pixels a second time
-//    (the same values to the same addresses), so that there are no partial groups at any HW >= PW.
+//    (the same values to the same addresses; with an Add, stored once), so that there are no partial groups at any HW >= PW.
 //  - KS = 4: inputs that are deep (or whose pixels are few) share the reduction between the four wavefronts of a workgroup, which
 //    exchange partial sums through LDS.
 //  - Zero points: sum (x - zx)(w - zw) = sum xs ws - zws Sx - zxs Sw + C zxs zws with xs, ws moved to the signed domain; Sx is one
@@ -89,6 +89,7 @@ __global__ void __launch_bounds__(256, 2) PwRegKernel(PwrArgs a, ADD add) {
   const uint32_t grp = min(pix_tile * 16 + n, a.groups - 1);
   const uint32_t image = DivM(grp, a.m_per_image), gi = grp - image * a.per_image;
   const uint32_t p = min(gi * PW, a.HW - PW);
+  const uint32_t twice = gi * PW - p;  // pixels that the group before it computes too
   uint32_t raw[KR][16][kDw];
   {
     const uint32_t at = (image * a.C + g * 16) * a.HW + p;
@@ -181,6 +182,12 @@ __global__ void __launch_bounds__(256, 2) PwRegKernel(PwrArgs a, ADD add) {
         __builtin_memcpy(res, add.res + at, PW);
 #pragma unroll
         for (int d = 0; d < kDw; ++d) o[d] = AddResidual4(add, o[d], res[d]);
+      }
+      if constexpr (!std::is_same<ADD, PwrNoAdd>::value) {
+        if (twice) {  // (the result may be written over the Add's other operand: a pixel is stored once)
+          for (int e = static_cast<int>(twice); e < PW; ++e) a.y[at + e] = static_cast<uint8_t>(o[e / 4] >> (8 * (e & 3)));
+          return;
+        }
       }
       __builtin_memcpy(a.y + at, o, PW);
     };
