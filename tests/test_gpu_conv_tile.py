@@ -61,3 +61,30 @@ def test_conv2d_tile_keeps_an_infinity_apart(oracle, monkeypatch):
         x[40] = np.inf
         got = TC.gpu_conv2d(x, np.abs(wt) + wt.dtype.type(0.01), b, **kws)
         assert not np.isnan(got).any() and np.isinf(got).sum() == 8 * 9
+
+
+@pytest.mark.parametrize("mode", ["u8", "i8pc", "f16", "f32"])
+@pytest.mark.parametrize("cols", [0, 7, 9])
+@pytest.mark.parametrize("groups", [1, 2])
+def test_conv2d_tile_blocks_over_one_window(oracle, groups, cols, mode, monkeypatch):
+    """Several blocks of output channels over one staged window: an even split, a short last pass, a last block of few channels;
+    runs of a whole tile (cols 0: whatever the cost decides, else rows of 7 or 9: no whole quads)."""
+    rng = np.random.default_rng(500 + groups + cols)
+    x, wt, b, kws = conv_case(rng, mult=0, mode=mode, n=2, c=20 * groups, h=13, w=17, oc=230 if groups == 1 else 140, kh=3, kw=3, stride=[1, 1],
+                              dil=[1, 1], pad=[1, 1, 1, 1], **(dict(groups=groups) if groups > 1 else {}))
+    monkeypatch.setenv("TVX_CONV_TILE", "1")
+    if cols:
+        monkeypatch.setenv("TVX_CONV_TILE_COLS", str(cols))
+    want = oracle.conv2d(x, wt, b, act=1, **kws)
+    for shape, channels in ((0, 64), (2, 64), (4, 32)):
+        for loop in (1, 2, 3, 4):
+            if loop > -(-kws["out_shape"][2] // groups // channels):
+                continue
+            monkeypatch.setenv("TVX_CONV_TILE_SHAPE", str(shape))
+            monkeypatch.setenv("TVX_CONV_TILE_LOOP", str(loop))
+            got = TC.gpu_conv2d(x, wt, b, act=1, **kws)
+            if mode in ("u8", "i8pc"):
+                assert np.array_equal(got, want), (shape, loop, int((got != want).sum()))
+            else:   # 32-bit sums in another order, rounded to the type (as above)
+                scale = max(np.sqrt(np.mean(want.astype(np.float64) ** 2)), 1.0)
+                assert np.abs(got.astype(np.float64) - want).max() <= (2e-3 if mode == "f16" else 1e-5) * scale * 4, (shape, loop)

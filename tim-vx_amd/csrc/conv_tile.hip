@@ -13,6 +13,9 @@
 // Results leave through LDS in runs of a whole tile or row per channel: sixteen bytes a lane straight from the accumulators, each in
 // a cache line of its own, wrote 0.5 TB/s (int8 62 -> 144 channels, 3x3 on 73 x 73, batch 48: 100 -> 82 us; float16 29 -> 304 on
 // 141 x 141, batch 3: 48 -> 41; float32 3 -> 16 on 132 x 132, batch 10: 15.9 -> 12.5).
+// Where several blocks of output channels follow from one window and there are workgroups enough without them, a workgroup takes
+// them one after the other over the window it has staged: 8 -> 240 channels 3x3 on 157 x 157, batch 11, 69 -> 49 us; 80 -> 352 on
+// 66 x 66, batch 23, 76 -> 62.
 // Quantized tensors under a weight zero point need the sum of every window: channel sums per staged pixel, box-filtered
 // once per tile - nothing in the inner loop.
 //
@@ -56,20 +59,22 @@ struct TileArgs {
   int steps, steps_pad, odd;  // reduction steps of a chunk; the last step's upper half is empty
   int taps_w, taps_h, dil_col, dil_row;  // for the box sum: LDS pixels between taps
   int ncg, cells, gl;      // column groups of a staged row, of all rows; granules neighbouring lanes take (a divisor of gpc)
-  int tiles_x, tiles_y, oc_blocks, tiles_per_group;
+  int tiles_x, tiles_y, tiles_per_group;
+  int loop, wgs_per_group, oc_wgs;  // channel blocks that a workgroup takes one after the other; workgroups a group's blocks take; of all groups
   int total, per_xcd;
   int npx, items;          // staged pixels and work items of a chunk
   uint32_t plane_bytes, image_bytes;
   int at_max;              // last place of a plane where a work item's pixels can be read
-  int off_tab, off_sum, off_zt;  // LDS carve-up behind the staged window
+  int off_tab, off_sum, off_zt, off_out;  // LDS carve-up behind the staged window; the results (over the window where it is used once)
   int runs, run_px, run_out, out_pitch;  // copy-out: runs of consecutive outputs of a channel, their pixels and distance; LDS bytes of a channel
-  uint32_t m_run4, m_runs4;  // reciprocals of a run's groups of four pixels, and of all runs'
+  uint32_t m_run4;         // reciprocal of a run's groups of four pixels
+  int runs_shift;          // log2 of the threads that a channel's runs take
   uint32_t m_gl, m_cells, m_ncg, m_ih, m_iw, m_tw, m_thtw, m_ocb, m_tpg, m_tx, m_ty;  // reciprocals: u / d = mulhi(u, m), exact for the ranges used
   uint32_t xor_mask;
   uint32_t pad_full, pad_last[4];  // a padding granule: full, and the channels' last one
   int last_granule;        // global index of the channels' last granule
   int zws;                 // weight zero point in the signed domain (0: no window sums)
-  int out_zp, lo, hi, act;
+  int lo, hi, narrow, out_xor, act;  // quantized: clamp in the signed domain, whether it is narrower than a byte; 0x80808080 for uint8 results
 };
 
 __device__ __forceinline__ int DivM(int u, uint32_t m) { return m ? static_cast<int>(__umulhi(static_cast<uint32_t>(u), m)) : u; }
@@ -155,8 +160,9 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
   if (id >= a.total) return;
   const int tab_n = 2 * a.steps_pad;
   const int tab_first = a.tab[min(tid, tab_n - 1)];  // (waited for behind the window's loads)
-  const int tile = DivM(id, a.m_ocb), ocb = id - tile * a.oc_blocks;
-  const int group = DivM(ocb, a.m_tpg), ocl = ocb - group * a.tiles_per_group;  // group, channel block of the group
+  const int tile = DivM(id, a.m_ocb), ocb = id - tile * a.oc_wgs;
+  const int group = DivM(ocb, a.m_tpg);
+  int ocl = (ocb - group * a.wgs_per_group) * a.loop;  // channel block of the group
   const int tyn = DivM(tile, a.m_tx), tx = tile - tyn * a.tiles_x;
   const int tn = DivM(tyn, a.m_ty), ty = tyn - tn * a.tiles_y;
   const int n0 = tn * a.G;
@@ -169,6 +175,7 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
   const int per = (a.steps + KS - 1) / KS;
   const int s0 = KS == 1 ? 0 : min(ks * per, a.steps), s1 = KS == 1 ? a.steps : min(s0 + per, a.steps);
   const uint32_t tile_stride = static_cast<uint32_t>((MULTI ? a.chunks : 1) * a.steps) * 64;
+  const int passes = MULTI ? a.chunks : min(a.loop, a.tiles_per_group - ocl);
   const v4i* wp = a.wpk + static_cast<size_t>((group * a.tiles_per_group + ocl) * (WN * NT) + wn * NT) * tile_stride + lane;
   v4i fw[R][NT];
   auto fetch_w = [&](int chunk, int s, v4i (&f)[NT]) {
@@ -183,8 +190,11 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
   uint32_t base[MT];  // LDS byte offset of this lane's pixel in each pixel tile
   acc_t acc[MT][NT];
 
-  const int chunks = MULTI ? a.chunks : 1;
-  for (int chunk = 0; chunk < chunks; ++chunk) {
+  // MULTI: a pass is a chunk of the channels, the results follow the last. Else: a pass is a block of output channels over the
+  // same staged window.
+  for (int pass = 0; pass < passes; ++pass) {
+    const int chunk = MULTI ? pass : 0;
+    if (MULTI || pass == 0) {
     if (chunk) __syncthreads();  // the window is free
     // ---- stage: an item = (granule, column group, row); lanes take gl granules, then the cells of a plane (contiguous in
     // memory where the rows are whole), then the next gl granules ----
@@ -286,7 +296,8 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
         sum[p] = v;
       }
     }
-    if (chunk == 0)
+    }
+    if (!MULTI || chunk == 0)
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -328,7 +339,12 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
         multiply(s + u, fx[u & 1], fw[u]);
         fetch_x(s + u + 2, fx[u & 1]);
       }
-  }
+    if (MULTI && pass + 1 < passes) continue;
+    if (!MULTI && pass + 1 < passes) {  // the next block's first weights travel under the results
+      wp += static_cast<size_t>(WN * NT) * tile_stride;
+#pragma unroll
+      for (int u = 0; u < R; ++u) fetch_w(0, s0 + u, fw[u]);
+    }
 
   // the epilogue's tables travel while the wavefronts meet
   int bias[NT];
@@ -349,7 +365,8 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
   // that become eight consecutive pixels, or single quads), every wavefront finishes its own ----
   constexpr int kQuads = KS == 1 ? 4 : (2 * MT * NT >= KS ? 2 : 1);  // quads of a piece
   constexpr int kPieces = 4 / kQuads;
-  if (KS > 1 || (DT == kI8 && a.zws)) {
+  const bool box = DT == kI8 && a.zws && (MULTI || pass == 0);  // the window sums are to be made
+  if (KS > 1 || box) {
     __syncthreads();
     elem_t* part = reinterpret_cast<elem_t*>(lds);  // [wave][tile][element][lane]
     if (KS > 1)
@@ -363,7 +380,7 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
             if (piece % KS != ks) part[((wave * MT + m) * NT + t) * 1024 + i * 64 + lane] = acc[m][t][i];
           }
     // window sums: the box filter over the channel sums
-    if (DT == kI8 && a.zws) {
+    if (box) {
       const int* sum = reinterpret_cast<const int*>(lds + a.off_sum);
       int* zt = reinterpret_cast<int*>(lds + a.off_zt);
       for (int q = tid; q < a.NQ; q += kThreads) {
@@ -397,7 +414,7 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
   // ---- epilogue: a lane holds output channel `row` of each channel tile and, per accumulator quad k, pixels
   // 8 k + 4 half + 0 .. 3 of a pixel tile. The results meet in LDS as [channel][pixel] and leave from there in runs: a tile of
   // whole rows is one run of a channel's plane (per image), else every row is one ----
-  if (KS > 1 || !(DT == kI8 && a.zws)) __syncthreads();  // the window (the partial sums) are read
+  if (KS > 1 || !box) __syncthreads();  // the window, the partial sums or the block before are read
 #pragma unroll
   for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -406,7 +423,7 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
       for (int k = 0; k < 4; ++k) {
         if (KS > 1 && ((m * NT + t) * kPieces + k % kPieces) % KS != ks) continue;
         const int q0 = (wm * MT + m) * 32 + 8 * k + 4 * half;
-        uint8_t* to = lds + (wn * NT * 32 + t * 32 + row) * a.out_pitch + q0 * E;
+        uint8_t* to = lds + a.off_out + (wn * NT * 32 + t * 32 + row) * a.out_pitch + q0 * E;
         if constexpr (DT == kI8) {
           int v[4];
 #pragma unroll
@@ -416,7 +433,10 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] += z[e];
           }
-          *reinterpret_cast<uint32_t*>(to) = RequantPack4<kRqFastNoTie>(v, rq[t], a.out_zp, a.lo, a.hi);
+          const int sh = rq[t][1] & 31;
+          const int64_t round = RoundHigh(rq[t][2]);
+          *reinterpret_cast<uint32_t*>(to) = (a.narrow ? RequantSaturate4<true>(v, rq[t][0], sh, round, a.lo << sh, ((a.hi + 1) << sh) - 1)
+                                                       : RequantSaturate4<false>(v, rq[t][0], sh, round, 0, 0)) ^ a.out_xor;
         } else {
           float v[4];
 #pragma unroll
@@ -441,14 +461,15 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
   const int runs_live = whole ? min(a.G, a.batch - n0) : rows_live, run_live = whole ? rows_live * a.OW : min(a.TW, a.OW - x0);
   const int ocb0 = ocl * (WN * NT * 32), channels = min(WN * NT * 32, a.ocg - ocb0);
   uint8_t* yb = a.y + ((static_cast<size_t>(n0) * a.OC + static_cast<size_t>(group) * a.ocg + ocb0) * ohw + y0 * a.OW + x0) * E;
-  const int run4 = (a.run_px + 3) >> 2, runs4 = a.runs * run4;
-  for (int it = tid; it < channels * runs4; it += kThreads) {
-    const int ch = DivM(it, a.m_runs4), rest = it - ch * runs4;
-    const int run = DivM(rest, a.m_run4), px = (rest - run * run4) * 4;
-    const int left = run < runs_live ? run_live - px : 0;
-    if (left <= 0) continue;
-    const uint8_t* from = lds + ch * a.out_pitch + (run * a.run_px + px) * E;
-    uint8_t* to = yb + (static_cast<size_t>(ch) * ohw + static_cast<size_t>(run) * a.run_out + px) * E;
+  // a thread keeps its place in the channels' runs and walks the channels
+  const int place = tid & ((1 << a.runs_shift) - 1), run = DivM(place, a.m_run4), px = (place - run * ((a.run_px + 3) >> 2)) * 4;
+  const int left = run < runs_live ? run_live - px : 0;
+  const int ch0 = tid >> a.runs_shift, ch_step = kThreads >> a.runs_shift;
+  const uint8_t* from = lds + a.off_out + ch0 * a.out_pitch + (run * a.run_px + px) * E;
+  uint8_t* to = yb + (static_cast<size_t>(ch0) * ohw + static_cast<size_t>(run) * a.run_out + px) * E;
+  const size_t to_step = static_cast<size_t>(ch_step) * ohw * E;
+  if (left > 0)
+  for (int ch = ch0; ch < channels; ch += ch_step, from += ch_step * a.out_pitch, to += to_step) {
     uint32_t four[E];
     if (left >= 4) {
       if constexpr (E == 1) {  // (a run begins at any byte: the dword out of two)
@@ -474,6 +495,8 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
         else reinterpret_cast<uint32_t*>(to)[e] = reinterpret_cast<const uint32_t*>(from)[e];
       }
     }
+  }
+    ++ocl;
   }
 }
 
@@ -502,15 +525,17 @@ constexpr int kShapeCount = sizeof(kShapes) / sizeof(kShapes[0]);
 int RoundUp(int v, int m) { return (v + m - 1) / m * m; }
 uint32_t Magic(int d) { return d <= 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + d - 1) / d); }
 
-// LDS of a workgroup in front of its tables: the staged window, then the partial sums, then the results
+// LDS of a workgroup in front of its tables: the staged window, then the partial sums, then the results - those behind it where
+// several blocks of channels read the window
 int OutPitch(const Shape& sp, int E) { return (sp.pixels + 4) * E; }  // (four pixels more against bank conflicts)
-int64_t WindowBytes(const Shape& sp, int64_t staged, int E) {
+int64_t OutBytes(const Shape& sp, int E) { return static_cast<int64_t>(sp.channels) * OutPitch(sp, E); }
+int64_t WindowBytes(const Shape& sp, int64_t staged, int E, int loop) {
   const int64_t sums = sp.ks > 1 ? static_cast<int64_t>(sp.ks) * sp.pixels * sp.channels * 4 : 0;
-  return (std::max({staged, sums, static_cast<int64_t>(sp.channels) * OutPitch(sp, E)}) + 15) / 16 * 16;
+  return (std::max({staged, sums, loop > 1 ? 0 : OutBytes(sp, E)}) + 15) / 16 * 16;
 }
 
 struct Geometry {
-  int shape, TW, TH, G, gpc, chunks;
+  int shape, TW, TH, G, gpc, chunks, loop;
   int IW, IH, pitch, lds_bytes;
   int64_t wgs;
   double cost;
@@ -518,24 +543,24 @@ struct Geometry {
 
 // Microseconds of a launch, to compare tiles by. A workgroup is a chain - start, staging rounds (an item per thread and
 // round), steps, epilogue - whose length counts once per round of workgroups the chip holds; above that the units a CU's
-// workgroups share (its memory pipeline above all: 0.6 us per wavefront of int8 items) set the pace. The constants are a
-// fit to 5400 measured launches (140 drawn convolutions x the tiles below): 16 % off a launch at the median of the squares,
-// and the tile chosen costs 5 % more than the best one on the (geometric) average.
+// workgroups share (its memory pipeline above all: 0.7 us per wavefront of int8 items) set the pace. The constants are a
+// fit to 8800 measured launches (180 drawn convolutions x the tiles below): the tile chosen costs 9 % more than the best
+// measured one on the (geometric) average, noise included, and 46 % at the worst.
 double Cost(const Shape& sp, const Geometry& g, int dt, int taps, int group_px, bool sums, bool whole_granules, bool borders, int OW) {
   const int threads = 64 * sp.waves, steps = (taps * g.gpc + 1) / 2, tiles = sp.pixels * sp.channels / 1024 * sp.ks / sp.waves;
   const double npx = static_cast<double>(g.G) * g.IH * g.IW;
   const double items = static_cast<double>(g.G) * g.IH * ((g.IW + group_px - 1) / group_px) * g.gpc;
-  const double runs = g.TW == OW || g.TW % 16 == 0 ? 1.0 : 1.1;  // stores of whole sixteen-pixel runs
-  const double stage = (dt == kI8 ? 2.27 : dt == kF16 ? 1.49 : 1.32) * std::ceil(items / threads) * (whole_granules ? 1.0 : 1.2) +
-                       0.024 * npx * g.gpc / threads * ((sums ? 1.0 : 0.0) + (borders ? 0.5 : 0.0));
-  const double multiply = static_cast<double>(steps) / sp.ks * (0.034 + (dt == kF32 ? 0.286 : 0.059) * tiles);
-  const double chain = 0.87 + g.chunks * (stage + multiply) + 1.5 * tiles * runs;
-  const double shared = g.chunks * (0.6 * items / 64 * (dt == kF32 ? 0.126 : 1.0) + 0.0028 * steps * tiles * sp.waves / sp.ks * (dt == kF32 ? 8 : 1)) +
-                        0.5 * sp.pixels * sp.channels / 1024 * runs;
+  const double runs = g.TW == OW || g.TW % 4 == 0 ? 1.0 : 1.1;  // stores of whole quads
+  const double stage = (dt == kI8 ? 2.0 : 0.98) * std::ceil(items / threads) * (whole_granules ? 1.0 : 0.94) +
+                       0.3 * npx * g.gpc / threads * ((sums ? 1.0 : 0.0) + (borders ? 0.5 : 0.0));
+  const double multiply = static_cast<double>(steps) / sp.ks * (0.05 + (dt == kF32 ? 0.127 : 0.016) * tiles);
+  const double chain = 2.5 + g.chunks * (stage + g.loop * multiply) + g.loop * 0.32 * tiles / sp.ks * runs;
+  const double shared = g.chunks * ((dt == kF32 ? 0.096 : 0.69) * items / 64 + (dt == kF32 ? 0.045 : 0.0072) * g.loop * steps * tiles * sp.waves / sp.ks) +
+                        g.loop * 0.157 * sp.pixels * sp.channels / 1024 * runs;
   const double per_cu = static_cast<double>(g.wgs) / 256;
   const double resident = std::min<double>(std::max(1, std::min(16 / sp.waves, 160 * 1024 / g.lds_bytes)), std::max(1.0, std::ceil(per_cu)));
-  const double by_chain = per_cu <= resident ? chain : (per_cu / resident + 0.6) * chain, by_units = per_cu * shared;
-  return 3.0 + std::cbrt(by_chain * by_chain * by_chain + by_units * by_units * by_units);
+  const double by_chain = per_cu <= resident ? chain : (per_cu / resident + 0.97) * chain, by_units = per_cu * shared;
+  return 2.7 + std::cbrt(by_chain * by_chain * by_chain + by_units * by_units * by_units);
 }
 
 struct Plan {
@@ -618,15 +643,15 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   const int zws = dt == kI8 ? op->w_zp - (w_u8 ? 128 : 0) : 0;
 
   // ---- the tile ----
-  int want = -1, want_tw = 0;
+  int want = -1, want_tw = 0, want_loop = 0;
   if (const char* f = getenv("TVX_CONV_TILE_SHAPE")) want = atoi(f);  // test lever
   if (const char* f = getenv("TVX_CONV_TILE_COLS")) want_tw = atoi(f);  // test lever
+  if (const char* f = getenv("TVX_CONV_TILE_LOOP")) want_loop = atoi(f);  // test lever
   Geometry best{};
   best.shape = -1;
   for (int sidx = 0; sidx < kShapeCount; ++sidx) {
     if (want >= 0 && sidx != want) continue;
     const Shape& sp = kShapes[sidx];
-    const int oc_blocks = (a.ocg + sp.channels - 1) / sp.channels;
     const int cand[] = {OW, (OW + 1) / 2, (OW + 2) / 3, 8, 16, 32, 64, 128};
     for (int tw : cand) {
       if (want_tw && tw != want_tw) continue;
@@ -642,23 +667,30 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
       g.IH = (g.TH - 1) * a.row_stride + (kh - 1) * dh + 1;
       const int64_t npx = static_cast<int64_t>(g.G) * g.IH * g.IW;
       if (npx > 40000) continue;
+      const int blocks = (a.ocg + sp.channels - 1) / sp.channels;
+      for (int loop : {1, 2, 3, 4, 6, 8, 16}) {
+      g.loop = loop;
+      if (loop > 1 && (loop > blocks || sp.ks > 1)) break;
+      if (want_loop && loop != want_loop) continue;
       for (g.chunks = 1; g.chunks <= granules; ++g.chunks) {
         g.gpc = (granules + g.chunks - 1) / g.chunks;
         if (g.chunks > 1 && (granules + g.gpc - 1) / g.gpc != g.chunks) continue;
         g.pitch = (g.gpc | 1) * 16;
         const int steps = (taps * g.gpc + 1) / 2;
-        int64_t bytes = WindowBytes(sp, npx * g.pitch, E);
+        int64_t bytes = WindowBytes(sp, npx * g.pitch, E, loop);
         bytes += 2 * RoundUp(steps + 12, 4) * 4;
         if (zws) bytes += npx * 4 + sp.pixels * 4;
+        if (loop > 1) bytes = RoundUp(bytes, 16) + OutBytes(sp, E);
         g.lds_bytes = static_cast<int>(std::min<int64_t>(bytes, 1 << 30));
         if (g.lds_bytes <= 78 * 1024) break;
       }
-      if (g.chunks > granules) continue;
+      if (g.chunks > granules || (loop > 1 && g.chunks > 1)) continue;
       const int64_t tiles = static_cast<int64_t>((OW + g.TW - 1) / g.TW) * ((OH + g.TH - 1) / g.TH) * ((d->batch + g.G - 1) / g.G);
-      g.wgs = tiles * oc_blocks * groups;
+      g.wgs = tiles * ((blocks + loop - 1) / loop) * groups;
       if (g.wgs > 0x3fffffff) continue;
       g.cost = Cost(sp, g, dt, taps, group_px, zws != 0, (a.icg * E) % 16 == 0, (a.pad_l || a.pad_t) && taps > 1, OW);
       if (best.shape < 0 || g.cost < best.cost) best = g;
+      }
     }
   }
   if (best.shape < 0) return TVX_E_UNSUPPORTED;
@@ -680,7 +712,9 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   a.tiles_x = (OW + g.TW - 1) / g.TW;
   a.tiles_y = (OH + g.TH - 1) / g.TH;
   a.tiles_per_group = (a.ocg + sp.channels - 1) / sp.channels;
-  a.oc_blocks = a.tiles_per_group * groups;
+  a.loop = g.loop;
+  a.wgs_per_group = (a.tiles_per_group + g.loop - 1) / g.loop;
+  a.oc_wgs = a.wgs_per_group * groups;
   a.total = static_cast<int>(g.wgs);
   a.per_xcd = (a.total + 7) / 8;
   a.npx = g.G * g.IH * g.IW;
@@ -689,19 +723,21 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   a.image_bytes = a.plane_bytes * a.C;
   a.at_max = H * W - group_px;
   const int64_t npx = static_cast<int64_t>(g.G) * g.IH * g.IW;
-  a.off_tab = static_cast<int>(WindowBytes(sp, npx * g.pitch, E));
+  a.off_tab = static_cast<int>(WindowBytes(sp, npx * g.pitch, E, g.loop));
   a.off_sum = a.off_tab + 2 * a.steps_pad * 4;
   a.off_zt = a.off_sum + (zws ? static_cast<int>(npx) * 4 : 0);
+  a.off_out = g.loop > 1 ? g.lds_bytes - static_cast<int>(OutBytes(sp, E)) : 0;
   const bool whole = g.TW == OW;
   a.runs = whole ? g.G : g.TH;
   a.run_px = whole ? g.TH * OW : g.TW;
   a.run_out = whole ? a.OC * OH * OW : OW;
   a.out_pitch = OutPitch(sp, E);
-  a.m_run4 = Magic((a.run_px + 3) / 4); a.m_runs4 = Magic(a.runs * ((a.run_px + 3) / 4));
+  a.m_run4 = Magic((a.run_px + 3) / 4);
+  while ((1 << a.runs_shift) < a.runs * ((a.run_px + 3) / 4)) ++a.runs_shift;
   a.m_gl = Magic(a.gl); a.m_cells = Magic(a.cells); a.m_ncg = Magic(a.ncg); a.m_ih = Magic(a.IH); a.m_iw = Magic(a.IW); a.m_tw = Magic(a.TW); a.m_thtw = Magic(a.TH * a.TW);
-  a.m_ocb = Magic(a.oc_blocks); a.m_tpg = Magic(a.tiles_per_group); a.m_tx = Magic(a.tiles_x); a.m_ty = Magic(a.tiles_y);
+  a.m_ocb = Magic(a.oc_wgs); a.m_tpg = Magic(a.wgs_per_group); a.m_tx = Magic(a.tiles_x); a.m_ty = Magic(a.tiles_y);
   // a reciprocal is exact while dividend * divisor < 2^32
-  if (static_cast<uint64_t>(a.total) * std::max({a.oc_blocks, a.tiles_x, a.tiles_y}) >= (1ull << 32)) return TVX_E_UNSUPPORTED;
+  if (static_cast<uint64_t>(a.total) * std::max({a.oc_wgs, a.tiles_x, a.tiles_y}) >= (1ull << 32)) return TVX_E_UNSUPPORTED;
   if (static_cast<uint64_t>(npx) * a.gpc * std::max({a.gpc, a.cells, a.IH, a.IW}) >= (1ull << 32)) return TVX_E_UNSUPPORTED;
   a.xor_mask = dt == kI8 && x_u8 ? 0x80808080u : 0u;
   a.pad_full = static_cast<uint32_t>(zxs & 0xff) * 0x01010101u;
@@ -711,7 +747,10 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
     a.pad_last[q] = nb >= 4 ? a.pad_full : nb <= 0 ? 0u : a.pad_full & ((1u << (8 * nb)) - 1u);
   }
   a.zws = zws;
-  a.out_zp = d->out_zp; a.lo = op->act_lo; a.hi = op->act_hi; a.act = d->activation;
+  const int out_flip = dt == kI8 && d->out_dtype == TVX_U8 ? 128 : 0;
+  a.lo = op->act_lo - out_flip; a.hi = op->act_hi - out_flip; a.narrow = a.lo > -128 || a.hi < 127;
+  a.out_xor = out_flip ? static_cast<int>(0x80808080u) : 0;
+  a.act = d->activation;
 
   // ---- the step table ----
   std::vector<int32_t> tab(2 * static_cast<size_t>(a.steps_pad), 0);
@@ -721,7 +760,7 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   }
 
   // ---- weights [oc][c][ky][kx] -> fragment order; the bias takes the zero points' constants ----
-  const size_t alloc_oc = static_cast<size_t>(a.oc_blocks) * sp.channels;
+  const size_t alloc_oc = static_cast<size_t>(a.tiles_per_group) * groups * sp.channels;
   const size_t tile_bytes = static_cast<size_t>(a.chunks) * a.steps * 1024;
   std::vector<uint8_t> packed(alloc_oc / 32 * tile_bytes, 0);
   std::vector<int32_t> biasf(dt == kI8 ? alloc_oc : 0, 0);
@@ -767,9 +806,12 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   if (s == TVX_OK) s = op->aux3.Upload(tab.data(), tab.size() * 4);
   if (s == TVX_OK && dt == kI8) {
     std::vector<int32_t> rqt;
-    const int rq_mode = BuildRequantRecords(mult, shift, static_cast<int>(alloc_oc), static_cast<int>(alloc_oc), d->out_zp, &rqt,
-                                    AccumulatorBound(static_cast<uint64_t>(taps) * a.icg, bias_host, d->out_c));
-    if (rq_mode != kRqFastNoTie) return TVX_E_UNSUPPORTED;
+    const int64_t bound = AccumulatorBound(static_cast<uint64_t>(taps) * a.icg, bias_host, d->out_c);
+    const int slots = static_cast<int>(alloc_oc);
+    if (BuildRequantRecords(mult, shift, slots, slots, d->out_zp, &rqt, bound) != kRqFastNoTie) return TVX_E_UNSUPPORTED;
+    int up;
+    bool ties;
+    if (!BuildTieRecords(mult, shift, slots, slots, d->out_zp - out_flip, bound, &rqt, &up, &ties) || up || ties) return TVX_E_UNSUPPORTED;
     s = op->aux.Upload(biasf.data(), biasf.size() * 4);
     if (s == TVX_OK) s = op->aux2.Upload(rqt.data(), rqt.size() * 4);
     a.biasf = op->aux.as<int32_t>();
