@@ -88,3 +88,23 @@ def test_conv2d_tile_blocks_over_one_window(oracle, groups, cols, mode, monkeypa
             else:   # 32-bit sums in another order, rounded to the type (as above)
                 scale = max(np.sqrt(np.mean(want.astype(np.float64) ** 2)), 1.0)
                 assert np.abs(got.astype(np.float64) - want).max() <= (2e-3 if mode == "f16" else 1e-5) * scale * 4, (shape, loop)
+
+
+@pytest.mark.parametrize("groups", [1, 3])
+@pytest.mark.parametrize("act", [0, 1])
+def test_conv2d_tile_rounds_ties_to_even(oracle, act, groups, monkeypatch):
+    """Multipliers of .25 to 2 (powers of two among them) on small codes: accumulators shifted up, ties everywhere, exact."""
+    rng = np.random.default_rng(600 + groups)
+    n, c, h, w, oc = 2, 21, 11, 13, 66
+    x, wt = rng.integers(-4, 4, n * c * h * w).astype(np.int8), rng.integers(-4, 4, oc * (c // groups) * 9).astype(np.int8)
+    b = rng.integers(-30, 31, oc).astype(np.int32)
+    scales = np.array([0.25, 0.5, 0.31, 1.0, 1.7, 0.75])[np.arange(oc) % 6].astype(np.float32)
+    kws = dict(in_shape=[w, h, c, n], w_shape=[3, 3, c // groups, oc], out_shape=[w, h, oc, n], stride=[1, 1], dilation=[1, 1], pad_left=1, pad_top=1,
+               multiplier=0, in_dtype=1, w_dtype=1, out_dtype=1, in_q=(1.0, -2), w_q=(1.0, 0, scales), out_q=(1.0, 3), **(dict(groups=groups) if groups > 1 else {}))
+    monkeypatch.setenv("TVX_CONV_TILE", "1")
+    want = oracle.conv2d(x, wt, b, act=act, **kws)
+    assert len(np.unique(want)) > 20
+    for shape in SHAPES:
+        monkeypatch.setenv("TVX_CONV_TILE_SHAPE", str(shape))
+        got = TC.gpu_conv2d(x, wt, b, act=act, **kws)
+        assert np.array_equal(got, want), (shape, int((got != want).sum()))

@@ -74,6 +74,7 @@ struct TileArgs {
   uint32_t pad_full, pad_last[4];  // a padding granule: full, and the channels' last one
   int last_granule;        // global index of the channels' last granule
   int zws;                 // weight zero point in the signed domain (0: no window sums)
+  int pre_ties;            // accumulators' left shift (BuildTieRecords) * 2 + whether ties are possible
   int lo, hi, narrow, out_xor, act;  // quantized: clamp in the signed domain, whether it is narrower than a byte; 0x80808080 for uint8 results
 };
 
@@ -433,6 +434,11 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] += z[e];
           }
+          if (a.pre_ties) {  // (uniform)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] <<= a.pre_ties >> 1;
+            if (a.pre_ties & 1) LowerOddTies(v, rq[t]);
+          }
           const int sh = rq[t][1] & 31;
           const int64_t round = RoundHigh(rq[t][2]);
           *reinterpret_cast<uint32_t*>(to) = (a.narrow ? RequantSaturate4<true>(v, rq[t][0], sh, round, a.lo << sh, ((a.hi + 1) << sh) - 1)
@@ -604,8 +610,8 @@ static bool IsBetterChoice(const tvx_conv2d_desc* d, int dt) {
   return true;
 }
 
-// Claims dense and grouped convolutions with constant weights on quantized (no accumulator on a rounding tie), float16 or
-// float32 tensors whose staged window fits LDS a granule of channels at a time.
+// Claims dense and grouped convolutions with constant weights on quantized (multipliers of 2^-20 and more), float16 or float32
+// tensors whose staged window fits LDS a granule of channels at a time.
 int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const void* bias_host) {
   if (!w_host || op->fused_add || op->kind != OP_CONV2D || d->multiplier != 0) return TVX_E_UNSUPPORTED;
   int dt;
@@ -808,10 +814,10 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
     std::vector<int32_t> rqt;
     const int64_t bound = AccumulatorBound(static_cast<uint64_t>(taps) * a.icg, bias_host, d->out_c);
     const int slots = static_cast<int>(alloc_oc);
-    if (BuildRequantRecords(mult, shift, slots, slots, d->out_zp, &rqt, bound) != kRqFastNoTie) return TVX_E_UNSUPPORTED;
     int up;
     bool ties;
-    if (!BuildTieRecords(mult, shift, slots, slots, d->out_zp - out_flip, bound, &rqt, &up, &ties) || up || ties) return TVX_E_UNSUPPORTED;
+    if (!BuildTieRecords(mult, shift, slots, slots, d->out_zp - out_flip, bound, &rqt, &up, &ties)) return TVX_E_UNSUPPORTED;
+    a.pre_ties = up * 2 + ties;
     s = op->aux.Upload(biasf.data(), biasf.size() * 4);
     if (s == TVX_OK) s = op->aux2.Upload(rqt.data(), rqt.size() * 4);
     a.biasf = op->aux.as<int32_t>();
