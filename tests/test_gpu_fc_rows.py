@@ -44,3 +44,13 @@ def test_fully_connected_rows_keep_an_infinity_apart(monkeypatch):
     x[2, 0] = np.inf
     got = TC.gpu_fully_connected(x.ravel(), w.ravel(), None, m=4, k=37, n=20, in_dtype=3, w_dtype=3, out_dtype=3).reshape(4, 20)
     assert np.isinf(got[2]).all() and np.array_equal(got[[0, 1, 3]], np.full((3, 20), 37, np.float32))
+
+
+@pytest.mark.parametrize("offset", [1, 2, 3])
+@pytest.mark.parametrize("mode", ["u8", "f16"])
+def test_fully_connected_rows_of_a_view(oracle, mode, offset, monkeypatch):
+    """Rows of whole dwords in a tensor that does not begin on one: the input is a view some elements into a buffer."""
+    import torch
+    to_device = TC.to_device
+    monkeypatch.setattr(TC, "to_device", lambda a: torch.cat([to_device(np.zeros(offset, a.dtype)), to_device(a)])[offset:])
+    test_fully_connected_rows(oracle, 33, 96, 70, mode, monkeypatch)

@@ -83,11 +83,15 @@ template <> struct Mfma<kF32, 16> {
   }
 };
 
+typedef int Dwords4 __attribute__((ext_vector_type(4), aligned(4)));
+
 __device__ __forceinline__ int DivM(int u, uint32_t m) { return m ? static_cast<int>(__umulhi(static_cast<uint32_t>(u), m)) : u; }
 
 // TS: extent of an MFMA tile (16 or 32); WM x WN wavefronts share the rows and features (MT x NT tiles each), KS a tile's
-// reduction; R: steps in flight
-template <int DT, int TS, int WM, int WN, int KS, int MT, int NT, int R>
+// reduction; R: steps in flight. SPLIT: rows that do not begin on whole dwords: sixteen bytes out of five dwords - a load at any
+// byte takes several times as long (int8 29 x 2501 -> 46: 6.7 -> 5.3 us,
+// 512 x 2501 -> 512 9.0 -> 7.0; at 2500 bytes 4.0 and 5.3)
+template <int DT, int TS, int WM, int WN, int KS, int MT, int NT, int R, bool SPLIT>
 __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(4))) FcRowsKernel(RowsArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   using mfma = Mfma<DT, TS>;
@@ -114,7 +118,8 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
     xp[t] = a.x + static_cast<int64_t>(min(m[t], a.M - 1)) * a.row_bytes + part * 16;  // (rows past the end repeat the last and are not stored)
   }
   v4i fw[R][NT], fx[R][MT];
-  auto fetch = [&](int s, v4i (&w)[NT], v4i (&x)[MT]) {
+  int fifth[R][MT];
+  auto fetch = [&](int s, v4i (&w)[NT], v4i (&x)[MT], int (&x5)[MT]) {
     s = max(min(s, s1 - 1), 0);  // (past the end: the last step once more, not multiplied)
 #pragma unroll
     for (int t = 0; t < NT; ++t) w[t] = wp[static_cast<uint32_t>(t * a.steps + s) * 64];
@@ -123,7 +128,14 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
       // a step that ends behind the row: from where sixteen bytes of the tensor can be read, put right in `multiply`
       const uint8_t* p = xp[t] + static_cast<size_t>(s) * kStep;
       const uint8_t* last = a.x + (a.x_bytes - 16);
-      __builtin_memcpy(&x[t], p < last ? p : last, 16);
+      p = p < last ? p : last;
+      if (SPLIT) {  // the dwords with the first and the last of the sixteen bytes, and what lies between
+        const uintptr_t at = reinterpret_cast<uintptr_t>(p);
+        x[t] = *reinterpret_cast<const Dwords4*>(at & ~uintptr_t{3});
+        x5[t] = *reinterpret_cast<const int*>((at + 15) & ~uintptr_t{3});
+      } else {
+        __builtin_memcpy(&x[t], p, 16);
+      }
     }
   };
   typename mfma::acc acc[MT][NT];
@@ -137,7 +149,22 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
 #pragma unroll
   for (int t = 0; t < MT; ++t) rs[t] = 0;
   const bool ragged = a.row_bytes % kStep != 0;
-  auto multiply = [&](int s, const v4i (&w)[NT], v4i (&x)[MT]) {
+  uint32_t by_row[MT], by_last[MT];  // SPLIT: bytes behind a dword; of the last step, whose load may have been moved
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    const uint8_t *p = xp[t] + static_cast<size_t>(a.steps - 1) * kStep, *last = a.x + (a.x_bytes - 16);
+    by_row[t] = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(xp[t])) & 3;
+    by_last[t] = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p < last ? p : last)) & 3;
+  }
+  auto multiply = [&](int s, const v4i (&w)[NT], v4i (&x)[MT], const int (&x5)[MT]) {
+    if (SPLIT)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const uint32_t by = s == a.steps - 1 ? by_last[t] : by_row[t];  // (the condition is uniform)
+        const v4i v = x[t];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[t][q] = static_cast<int>(__builtin_amdgcn_alignbyte(q < 3 ? v[q + 1] : x5[t], v[q], by));
+      }
     if (DT == kI8)
 #pragma unroll
       for (int t = 0; t < MT; ++t) x[t] ^= static_cast<int>(a.xor_mask);
@@ -163,19 +190,19 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
       for (int n = 0; n < NT; ++n) mfma::Step(acc[t][n], w[n], x[t]);
   };
 #pragma unroll
-  for (int u = 0; u < R; ++u) fetch(s0 + u, fw[u], fx[u]);
+  for (int u = 0; u < R; ++u) fetch(s0 + u, fw[u], fx[u], fifth[u]);
   int s = s0;
 #pragma unroll 1
   for (; s + R < s1; s += R) {
 #pragma unroll
     for (int u = 0; u < R; ++u) {
-      multiply(s + u, fw[u], fx[u]);
-      fetch(s + u + R, fw[u], fx[u]);
+      multiply(s + u, fw[u], fx[u], fifth[u]);
+      fetch(s + u + R, fw[u], fx[u], fifth[u]);
     }
   }
 #pragma unroll
   for (int u = 0; u < R; ++u)
-    if (s + u < s1) multiply(s + u, fw[u], fx[u]);  // uniform
+    if (s + u < s1) multiply(s + u, fw[u], fx[u], fifth[u]);  // uniform
 
   // ---- the wavefronts of a tile meet: partial sums by quads, [wave][tile][quad][lane]; quad i is finished by wavefront i % KS ----
   v4i* red = reinterpret_cast<v4i*>(lds);
@@ -282,10 +309,12 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
 }
 
 typedef void (*RowsFn)(RowsArgs);
-struct Shape { int ts, rows, features, waves, ks, lds; RowsFn fn[3]; };
+struct Shape { int ts, rows, features, waves, ks, lds; RowsFn fn[3][2]; };
 #define TVX_ROWS(TS, WM, WN, KS, MT, NT, R)                                                                                          \
   { TS, WM * MT * TS, WN * NT * TS, WM * WN * KS, KS, KS > 1 ? WM * WN * KS * MT * (NT * TS * TS * 4 + TS * 4) : 0,                    \
-    { FcRowsKernel<kI8, TS, WM, WN, KS, MT, NT, R>, FcRowsKernel<kF16, TS, WM, WN, KS, MT, NT, R>, FcRowsKernel<kF32, TS, WM, WN, KS, MT, NT, R> } }
+    { { FcRowsKernel<kI8, TS, WM, WN, KS, MT, NT, R, false>, FcRowsKernel<kI8, TS, WM, WN, KS, MT, NT, R, true> },                        \
+      { FcRowsKernel<kF16, TS, WM, WN, KS, MT, NT, R, false>, FcRowsKernel<kF16, TS, WM, WN, KS, MT, NT, R, true> },                      \
+      { FcRowsKernel<kF32, TS, WM, WN, KS, MT, NT, R, false>, nullptr } } }
 const Shape kShapes[] = {
     TVX_ROWS(16, 1, 1, 4, 1, 1, 8),  // 0: 16 x 16, reduction on four wavefronts
     TVX_ROWS(32, 1, 1, 4, 1, 1, 7),  // 1: 32 x 32, on four
@@ -320,7 +349,7 @@ bool LargeTilesWin(const tvx_fc_desc& d, int dt) {
 
 struct Plan {
   RowsArgs a;
-  RowsFn fn;
+  RowsFn fn[2];  // rows on whole dwords; at any element
   unsigned grid, threads, lds_bytes;
   int elem;
 };
@@ -332,7 +361,7 @@ int FcRowsRun(tvx_op* op, const void* in0, const void*, void* out, hipStream_t s
   RowsArgs a = plan->a;
   a.x = static_cast<const uint8_t*>(in0);
   a.y = static_cast<uint8_t*>(out);
-  hipLaunchKernelGGL(plan->fn, dim3(plan->grid), dim3(plan->threads), plan->lds_bytes, st, a);
+  hipLaunchKernelGGL(plan->fn[((reinterpret_cast<uintptr_t>(in0) | static_cast<unsigned>(a.row_bytes)) & 3) != 0], dim3(plan->grid), dim3(plan->threads), plan->lds_bytes, st, a);
   TVX_HIP_CHECK(hipGetLastError());
   return TVX_OK;
 }
@@ -430,14 +459,16 @@ int FcRowsSetup(tvx_op* op, const tvx_fc_desc* d, const void* w_host, const void
   a.bias = op->aux.as<int32_t>();
   Plan plan{};
   plan.a = a;
-  plan.fn = sp.fn[dt];
+  for (int i = 0; i < 2; ++i) plan.fn[i] = sp.fn[dt][i];
   plan.grid = static_cast<unsigned>(a.per_xcd) * 8;
   plan.threads = 64u * sp.waves;
   plan.lds_bytes = static_cast<unsigned>(sp.lds);
   plan.elem = E;
   if (plan.lds_bytes > 48 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(plan.fn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(plan.lds_bytes));
-    if (e != hipSuccess) return SetError(TVX_E_DEVICE, "hipFuncSetAttribute(dynamic LDS %u): %s", plan.lds_bytes, hipGetErrorString(e));
+    for (RowsFn fn : plan.fn) {
+      const hipError_t e = fn ? hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(plan.lds_bytes)) : hipSuccess;
+      if (e != hipSuccess) return SetError(TVX_E_DEVICE, "hipFuncSetAttribute(dynamic LDS %u): %s", plan.lds_bytes, hipGetErrorString(e));
+    }
   }
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
   op->run = FcRowsRun;
