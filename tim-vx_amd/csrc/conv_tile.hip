@@ -606,6 +606,9 @@ static bool IsBetterChoice(const tvx_conv2d_desc* d, int dt) {
     // pass and its weights fit LDS beside it (6.9 against 8.9 us at 32 -> 80 on 16 x 16, batch 27); with more work than
     // this its tiles queue up (43 against 28 us at 8 -> 416 on 40 x 40, batch 24)
     if (d->in_c <= 32 && d->stride_w == 1 && d->stride_h == 1 && d->in_w % 4 == 0 && macs <= 400000000 && reduction <= 512) return false;
+    // one granule of channels on planes of at most 16 x 16: its shorter chain (5.2 against 7.0 us at 12 -> 8 on 7 x 7, batch 29; 6.9
+    // against 8.9 at 16 -> 240 on 7 x 13, batch 7); on larger planes the tiles win as often as not, and then by more (12.8 against 7.0)
+    if (d->in_c <= 16 && d->in_w * d->in_h <= 256 && macs <= 60000000 && reduction <= 512) return false;
   }
   return true;
 }
