@@ -596,19 +596,32 @@ static bool IsBetterChoice(const tvx_conv2d_desc* d, int dt) {
   const int groups = d->groups > 1 ? d->groups : 1;
   const uint64_t reduction = static_cast<uint64_t>(d->in_c / groups) * d->k_w * d->k_h;
   const uint64_t macs = reduction * d->out_c * d->out_w * d->out_h * d->batch;
-  // a group of three output channels and fewer fills less than a tenth of a tile's 32 channels
-  if (groups > 1 && d->out_c / groups < 4) return false;
+  // a group of three output channels and fewer fills less than a tenth of a tile's 32 channels: only where each has little to add up
+  // (float16 432 -> 12 in four groups, 7x7 on 42 x 42, batch 28: 2495 us with one thread per output, 140 here)
+  if (groups > 1 && d->out_c / groups < 4 && reduction <= 128) return false;
   // a handful of products per output: one thread per output is quicker than staging a window (4.3 against 5.7 us)
   if (dt != kI8 && reduction <= 9 && macs <= 4000000) return false;
+  // float16 1 x 1: conv2d_gemm_f16 gathers four pixels a load where planes are whole quads and has less to set up. Few channels (4.2
+  // against 6.9 us at 24 -> 16 on 50 x 50, batch 4; 8.9 against 11.5 at 40 -> 192 on 44 x 44, batch 13; above 64 the tiles: 8.0 against 33.4
+  // at 448 -> 320 on 26 x 26), tiny layers (4.4 against 6.0), and few results of many pixels (21.7 against 41.5 at 368 -> 8 on
+  // 112 x 112, batch 10; 59.9 against 47.9 at 256 -> 273 on 54 x 54).
+  if (dt == kF16 && groups == 1 && d->k_w == 1 && d->k_h == 1 && d->in_c >= 16) {
+    const uint64_t plane = static_cast<uint64_t>(d->in_w) * d->in_h;
+    if (d->in_c <= 32 && macs <= 20000000) return false;
+    if (d->stride_w == 1 && d->stride_h == 1 && plane % 4 == 0) {
+      if (d->in_c <= 64 && d->out_c <= 256 && macs <= 200000000) return false;
+      if (d->out_c <= 96 && plane * d->batch >= 32768) return false;
+    }
+  }
   if (dt == kI8 && groups == 1) {
     if (ConvIgemmPersists(d)) return false;
     // shallow inputs whose rows are whole dwords at stride 1: conv2d_igemm_i8 stages all channels of a tile in one aligned
     // pass and its weights fit LDS beside it (6.9 against 8.9 us at 32 -> 80 on 16 x 16, batch 27); with more work than
     // this its tiles queue up (43 against 28 us at 8 -> 416 on 40 x 40, batch 24)
     if (d->in_c <= 32 && d->stride_w == 1 && d->stride_h == 1 && d->in_w % 4 == 0 && macs <= 400000000 && reduction <= 512) return false;
-    // one granule of channels on planes of at most 16 x 16: its shorter chain (5.2 against 7.0 us at 12 -> 8 on 7 x 7, batch 29; 6.9
+    // a granule of channels or two on planes of at most 16 x 16: its shorter chain (5.2 against 7.0 us at 12 -> 8 on 7 x 7, batch 29; 6.9
     // against 8.9 at 16 -> 240 on 7 x 13, batch 7); on larger planes the tiles win as often as not, and then by more (12.8 against 7.0)
-    if (d->in_c <= 16 && d->in_w * d->in_h <= 256 && macs <= 60000000 && reduction <= 512) return false;
+    if (d->in_c <= 24 && d->in_w * d->in_h <= 256 && macs <= 250000000 && reduction <= 512) return false;
   }
   return true;
 }
