@@ -8,7 +8,7 @@ import test_gpu_mbconv as MB
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("waves", [4, 5, 8])
+@pytest.mark.parametrize("waves", [4, 8])
 @pytest.mark.parametrize("ci", range(len(DP.CASES)))
 def test_depthwise_pointwise(oracle, monkeypatch, ci, waves):
     monkeypatch.setenv("TVX_DWPW_WAVES", str(waves))

@@ -271,18 +271,13 @@ __global__ void __launch_bounds__(kMaxWaves * 64) __attribute__((amdgpu_waves_pe
   // ---- 3. pointwise: a wavefront takes 32 pixel slots at a time and walks every output tile ----
   const int frag_row = lane & 31, frag_half = lane >> 5;
   const v4i fz = {a.neg_zws4, a.neg_zws4, a.neg_zws4, a.neg_zws4};
-  const int parts = (a.P + 31) >> 5;
-  int part = wave, tile = 0;  // (more wavefronts than 32-pixel parts: they share the output tiles)
-  for (;; part += waves) {
-    while (part >= parts) { part -= parts; ++tile; }
-    if (tile >= a.oc_tiles) break;
-    const int part0 = part * 32;
+  for (int part0 = (wave & 3) * 32; part0 < a.P; part0 += 128) {
     // copy-out mapping of a staged 32 x 32 patch: lane -> 16-pixel chunk lane & 1 of output-channel row lane >> 1
     const int px_in_row = part0 + (lane & 1) * 16;
     const bool out_live = px_in_row < a.P;
     const size_t out_off = static_cast<size_t>(n) * a.OC * hw + static_cast<size_t>(g) * a.P + px_in_row;
     const int8_t* xa = xl + (part0 + frag_row) * a.pix_stride + frag_half * 16;
-    {
+    for (int tile = wave >> 2; tile < a.oc_tiles; tile += waves >> 2) {  // (the second four wavefronts take every other tile)
       const v4i q = rq_lds[tile * 32 + frag_row];
       const int nb = bias_lds[tile * 32 + frag_row];
       v16i acc;
@@ -483,7 +478,7 @@ int DwPwSetup(tvx_op* op, const tvx_conv2d_desc* dw, const void* dw_w, const voi
   const int passes = (C + (64 * kWaves >> lpr_shift) - 1) / (64 * kWaves >> lpr_shift);
   const uint64_t resident = std::min<uint64_t>(std::min(4, 160 * 1024 / lds_bytes), (tiles + 255) / 256);
   int waves = passes > batch && resident < 4 ? kMaxWaves : kWaves;
-  if (const char* f = getenv("TVX_DWPW_WAVES")) waves = std::min(kMaxWaves, std::max(kWaves, atoi(f)));  // tuning aid
+  if (const char* f = getenv("TVX_DWPW_WAVES")) waves = atoi(f) >= kMaxWaves ? kMaxWaves : kWaves;  // tuning aid
   if (lds_bytes + (waves - kWaves) * kStageBytes > 160 * 1024) waves = kWaves;
   lds_bytes += (waves - kWaves) * kStageBytes;
   // pointwise weights in fragment order, constants folded into the bias (as PwConvSetup packs them)
