@@ -108,3 +108,39 @@ def test_conv2d_tile_rounds_ties_to_even(oracle, act, groups, monkeypatch):
         monkeypatch.setenv("TVX_CONV_TILE_SHAPE", str(shape))
         got = TC.gpu_conv2d(x, wt, b, act=act, **kws)
         assert np.array_equal(got, want), (shape, int((got != want).sum()))
+
+
+def _check(got, want, mode, what):
+    if mode in ("u8", "i8pc"):
+        assert np.array_equal(got, want), (what, int((got != want).sum()))
+    else:   # 32-bit sums in another order, rounded to the type (as above)
+        scale = max(np.sqrt(np.mean(want.astype(np.float64) ** 2)), 1.0)
+        assert np.abs(got.astype(np.float64) - want).max() <= (2e-3 if mode == "f16" else 1e-5) * scale * 4, what
+
+
+@pytest.mark.parametrize("mode", ["u8", "i8pc", "f16", "f32"])
+@pytest.mark.parametrize("k,stride,dil,h,w", [(2, 2, 1, 7, 4), (3, 1, 1, 6, 6), (3, 1, 2, 5, 9), (1, 1, 1, 4, 13), (5, 3, 1, 7, 7)])
+def test_conv2d_tile_pads_wider_than_the_window(oracle, k, stride, dil, h, w, mode, monkeypatch):
+    """Padding one to four columns (rows) wider than the window: tiles whose window lies left of (above) the image hold nothing but
+    padding, whichever way the output columns are cut into tiles."""
+    monkeypatch.setenv("TVX_CONV_TILE", "1")
+    reach = (k - 1) * dil + 1
+    for more in (1, 2, 3, 4):
+        rng = np.random.default_rng(700 + 10 * k + more)
+        x, wt, b, kws = conv_case(rng, mult=0, mode=mode, n=3, c=20, h=h, w=w, oc=40, kh=k, kw=k, stride=[stride, stride], dil=[dil, dil],
+                                  pad=[reach + more, reach - 1, reach + more if more % 2 else 0, reach - 1])
+        want = oracle.conv2d(x, wt, b, act=1, **kws)
+        ow = kws["out_shape"][0]
+        for cols in sorted({0, ow, (ow + 1) // 2, (ow + 2) // 3} | ({8} if ow >= 8 else set())):
+            if cols:
+                monkeypatch.setenv("TVX_CONV_TILE_COLS", str(cols))
+            else:
+                monkeypatch.delenv("TVX_CONV_TILE_COLS", raising=False)
+            _check(TC.gpu_conv2d(x, wt, b, act=1, **kws), want, mode, (more, cols))
+
+
+@pytest.mark.parametrize("mode,case", [("f32", dict(n=4, c=32, h=7, w=4, oc=128, kh=2, kw=2, stride=[2, 2], dil=[1, 1], pad=[3, 0, 0, 0])),
+                                       ("i8pc", dict(n=1, c=64, h=6, w=6, oc=128, kh=3, kw=3, stride=[1, 1], dil=[1, 1], pad=[7, 0, 0, 0]))])
+def test_conv2d_pads_wider_than_the_window_by_default(oracle, mode, case):
+    x, wt, b, kws = conv_case(np.random.default_rng(710), mult=0, mode=mode, **case)
+    _check(TC.gpu_conv2d(x, wt, b, act=1, **kws), oracle.conv2d(x, wt, b, act=1, **kws), mode, "default")

@@ -187,7 +187,8 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
 
   const uint32_t plane_bytes = a.plane_bytes, image_bytes = a.image_bytes;
   const int npx = a.npx, items = a.items;
-  const int col_lo = max(0, -ix0), col_hi = min(a.IW, a.W - ix0);  // window columns inside the image
+  // window columns inside the image (none where the window lies in padding altogether: the stores' unsigned range needs hi >= lo)
+  const int col_lo = max(0, -ix0), col_hi = max(col_lo, min(a.IW, a.W - ix0));
   uint32_t base[MT];  // LDS byte offset of this lane's pixel in each pixel tile
   acc_t acc[MT][NT];
 
