@@ -10,7 +10,9 @@ pytestmark = pytest.mark.gpu
 
 # n, c, h, w, oc
 SIZES = [(1, 1, 1, 4, 1), (1, 5, 2, 4, 3), (3, 64, 3, 3, 16), (2, 65, 7, 7, 33), (5, 130, 5, 13, 17), (1, 192, 16, 16, 48), (2, 256, 9, 11, 70),
-         (3, 300, 7, 7, 20), (1, 512, 4, 4, 100), (2, 577, 3, 5, 40), (40, 24, 13, 13, 144), (1, 2048, 2, 3, 18)]
+         (3, 300, 7, 7, 20), (1, 512, 4, 4, 100), (2, 577, 3, 5, 40), (40, 24, 13, 13, 144), (1, 2048, 2, 3, 18),
+         # channels at the edges of steps of 32 and of 64 and of a lane's 8 and 16; the last images' rows end with the tensor
+         (2, 8, 5, 11, 20), (3, 16, 4, 9, 33), (2, 31, 9, 9, 17), (5, 32, 3, 5, 16), (2, 33, 7, 5, 40), (3, 48, 6, 6, 16), (2, 129, 5, 5, 20)]
 
 
 @pytest.mark.parametrize("mode", ["u8", "i8pc", "u8pc", "i8big"])

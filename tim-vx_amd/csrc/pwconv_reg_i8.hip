@@ -9,6 +9,9 @@
 //    (the same values to the same addresses; with an Add, stored once), so that there are no partial groups at any HW >= PW.
 //  - KS = 4: inputs that are deep (or whose pixels are few) share the reduction between the four wavefronts of a workgroup, which
 //    exchange partial sums through LDS.
+//  - Lanes load the channels that exist and no others; inputs of at most 32 take steps of 32 channels instead of 64. All lanes
+//    loading 64 channels fetched the next image's rows with these: 32 x 32 x 112 x 112 -> 64 channels 15.5 -> 13.5 us, 64 x 32 x 112 x
+//    112 -> 16 12.8 -> 10.9, 64 x 32 x 28 x 28 -> 192 7.5 -> 6.6, 12 x 12 x 150 x 150 -> 12 5.7 -> 4.6 (buffers in rotation).
 //  - Zero points: sum (x - zx)(w - zw) = sum xs ws - zws Sx - zxs Sw + C zxs zws with xs, ws moved to the signed domain; Sx is one
 //    more MFMA against a constant fragment per pixel tile, the per-channel constants are folded into the bias.
 // Bound by memory; what is left above it is the launch, whose wavefronts load, compute and store at about the same time. Against
@@ -25,16 +28,16 @@ namespace tvx {
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v2i __attribute__((ext_vector_type(2)));
 
 struct PwrArgs {
   const uint8_t* x;
   uint8_t* y;
-  const v4i* wpk;        // [16-channel tile][64-channel step][lane]: 16 reduction bytes of channel tile * 16 + lane % 16
+  const uint8_t* wpk;    // [16-channel tile][step of 4 KL channels][lane]: KL reduction bytes of channel tile * 16 + lane % 16
   const v4i* rec;        // per channel {multiplier, shift, rounding constant, folded bias}
   uint32_t C, OC, HW;
   uint32_t groups;       // batch * groups per image
   uint32_t per_image, m_per_image;  // pixel groups of an image, and their reciprocal
-  uint32_t limit;        // last byte offset of the input at which PW bytes may be read
   int ksteps;
   int tiles, tiles_per_wave;  // 16-channel output tiles
   uint32_t tile_groups, m_tile_groups, units;  // pixel tiles x tile groups
@@ -54,11 +57,18 @@ struct PwrNoAdd {};
 
 __device__ __forceinline__ uint32_t DivM(uint32_t u, uint32_t m) { return m ? __umulhi(u, m) : u; }
 
-// PW: pixels of a lane (8: 128 pixels a wavefront; 4: 64, for deep inputs and few pixels). KR: 64-channel steps of a wavefront.
+__device__ __forceinline__ v4i Multiply(const v4i& w, const v4i& x, const v4i& acc) { return __builtin_amdgcn_mfma_i32_16x16x64_i8(w, x, acc, 0, 0, 0); }
+__device__ __forceinline__ v4i Multiply(const v2i& w, const v2i& x, const v4i& acc) {
+  return __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, w), __builtin_bit_cast(long, x), acc, 0, 0, 0);
+}
+
+// PW: pixels of a lane (8: 128 pixels a wavefront; 4: 64, for deep inputs and few pixels). KL: channels of a lane and step (16; 8 for
+// inputs of at most 32 channels, half the bytes and half the transposition). KR: steps of a wavefront (4 KL channels each).
 // KS: wavefronts that share a reduction (4), or 1.
-template <int PW, int KR, int KS, class ADD>
+template <int PW, int KL, int KR, int KS, class ADD>
 __global__ void __launch_bounds__(256, 2) PwRegKernel(PwrArgs a, ADD add) {
   constexpr int kDw = PW / 4;  // dwords of a lane's pixels
+  using frag_t = std::conditional_t<KL == 16, v4i, v2i>;
   __shared__ v4i part[KS > 1 ? 4 * 4 * 64 : 1];
   const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -76,8 +86,9 @@ __global__ void __launch_bounds__(256, 2) PwRegKernel(PwrArgs a, ADD add) {
   const int k0 = KS > 1 ? wave * KR : 0;
 
   // ---- weights and tables of the first output tile; pixels ----
-  auto frag = [&](int t, int k) { return a.wpk[(static_cast<uint32_t>(t) * a.ksteps + (k0 + k)) * 64 + lane]; };
-  v4i w[KR], q[4];
+  auto frag = [&](int t, int k) { return reinterpret_cast<const frag_t*>(a.wpk)[(static_cast<uint32_t>(t) * a.ksteps + (k0 + k)) * 64 + lane]; };
+  frag_t w[KR];
+  v4i q[4];
 #pragma unroll
   for (int k = 0; k < KR; ++k) w[k] = frag(t0, k);
   auto records = [&](int t) {
@@ -90,23 +101,33 @@ __global__ void __launch_bounds__(256, 2) PwRegKernel(PwrArgs a, ADD add) {
   const uint32_t image = DivM(grp, a.m_per_image), gi = grp - image * a.per_image;
   const uint32_t p = min(gi * PW, a.HW - PW);
   const uint32_t twice = gi * PW - p;  // pixels that the group before it computes too
-  uint32_t raw[KR][16][kDw];
+  uint32_t raw[KR][KL][kDw];
+  const int channel0 = k0 * 4 * KL + g * KL;  // this lane's first channel; its steps are 4 KL apart
   {
-    const uint32_t at = (image * a.C + g * 16) * a.HW + p;
+    // lanes whose channels do not exist load nothing; past the input's last channel it is read again. Both meet zero weights.
+    const uint32_t at = (image * a.C + channel0) * a.HW + p;
 #pragma unroll
-    for (int k = 0; k < KR; ++k)
+    for (int k = 0; k < KR; ++k) {
+      const int left = static_cast<int>(a.C) - (channel0 + k * 4 * KL);
 #pragma unroll
-      for (int j = 0; j < 16; ++j)  // (channels that do not exist read something else: their weights are zero)
-        __builtin_memcpy(raw[k][j], a.x + min(at + static_cast<uint32_t>((k0 + k) * 64 + j) * a.HW, a.limit), PW);
+      for (int j = 0; j < KL; ++j)
+#pragma unroll
+        for (int d = 0; d < kDw; ++d) raw[k][j][d] = 0;
+      if (left > 0) {
+        const uint32_t first = at + static_cast<uint32_t>(k * 4 * KL) * a.HW, last = first + static_cast<uint32_t>(left - 1) * a.HW;
+#pragma unroll
+        for (int j = 0; j < KL; ++j) __builtin_memcpy(raw[k][j], a.x + min(first + static_cast<uint32_t>(j) * a.HW, last), PW);
+      }
+    }
   }
   __builtin_amdgcn_sched_barrier(0);  // all of them in flight before the first is used
-  v4i b[KR][PW];
+  frag_t b[KR][PW];
 #pragma unroll
   for (int k = 0; k < KR; ++k)
 #pragma unroll
     for (int d = 0; d < kDw; ++d)
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
+      for (int c = 0; c < KL / 4; ++c) {
         uint32_t in[4], t[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) in[j] = raw[k][c * 4 + j][d] ^ a.xor_mask;
@@ -124,14 +145,14 @@ __global__ void __launch_bounds__(256, 2) PwRegKernel(PwrArgs a, ADD add) {
       v4i acc = {0, 0, 0, 0};
 #pragma unroll
       for (int k = 0; k < KR; ++k) {
-        const int left = static_cast<int>(a.C) - ((k0 + k) * 64 + g * 16);  // channels of this lane that exist
-        v4i f;
+        const int left = static_cast<int>(a.C) - (channel0 + k * 4 * KL);  // channels of this lane that exist
+        frag_t f;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < KL / 4; ++c) {
           const int bytes = min(max(left - c * 4, 0), 4);
           f[c] = bytes == 4 ? a.neg_zws4 : a.neg_zws4 & ((1 << (8 * bytes)) - 1);
         }
-        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(f, b[k][j], acc, 0, 0, 0);
+        acc = Multiply(f, b[k][j], acc);
       }
       z[j] = acc[0];
     }
@@ -150,7 +171,7 @@ __global__ void __launch_bounds__(256, 2) PwRegKernel(PwrArgs a, ADD add) {
 #pragma unroll
     for (int k = 0; k < KR; ++k)
 #pragma unroll
-      for (int j = 0; j < PW; ++j) acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[k], b[k][j], acc[j], 0, 0, 0);
+      for (int j = 0; j < PW; ++j) acc[j] = Multiply(w[k], b[k][j], acc[j]);
     // the next tile's weights and records travel during this one's requantization
     const int tn = min(t + 1, t1 - 1);
     v4i r[4] = {q[0], q[1], q[2], q[3]};
@@ -223,18 +244,18 @@ __global__ void __launch_bounds__(256, 2) PwRegKernel(PwrArgs a, ADD add) {
 struct Plan {
   PwrArgs a;
   PwrAdd add;
-  int kr, ks;
+  int kl, kr, ks;
   unsigned grid, block;
 };
 
-template <int PW, int KR, int KS>
+template <int PW, int KL, int KR, int KS>
 void Launch(const Plan& p, const PwrArgs& a, const void* res, hipStream_t st) {
   if (p.add.add_mode) {
     PwrAdd add = p.add;
     add.res = static_cast<const uint8_t*>(res);
-    hipLaunchKernelGGL((PwRegKernel<PW, KR, KS, PwrAdd>), dim3(p.grid), dim3(p.block), 0, st, a, add);
+    hipLaunchKernelGGL((PwRegKernel<PW, KL, KR, KS, PwrAdd>), dim3(p.grid), dim3(p.block), 0, st, a, add);
   } else {
-    hipLaunchKernelGGL((PwRegKernel<PW, KR, KS, PwrNoAdd>), dim3(p.grid), dim3(p.block), 0, st, a, PwrNoAdd{});
+    hipLaunchKernelGGL((PwRegKernel<PW, KL, KR, KS, PwrNoAdd>), dim3(p.grid), dim3(p.block), 0, st, a, PwrNoAdd{});
   }
 }
 
@@ -244,17 +265,18 @@ int PwRegRun(tvx_op* op, const void* in0, const void* in1, void* out, hipStream_
   PwrArgs a = p.a;
   a.x = static_cast<const uint8_t*>(in0);
   a.y = static_cast<uint8_t*>(out);
-  switch (p.ks * 10 + p.kr) {
-    case 11: Launch<8, 1, 1>(p, a, in1, st); break;
-    case 12: Launch<8, 2, 1>(p, a, in1, st); break;
-    case 13: Launch<8, 3, 1>(p, a, in1, st); break;
-    case 14: Launch<8, 4, 1>(p, a, in1, st); break;
-    case 41: Launch<4, 1, 4>(p, a, in1, st); break;
-    case 42: Launch<4, 2, 4>(p, a, in1, st); break;
-    case 43: Launch<4, 3, 4>(p, a, in1, st); break;
-    case 44: Launch<4, 4, 4>(p, a, in1, st); break;
-    case 46: Launch<4, 6, 4>(p, a, in1, st); break;
-    default: Launch<4, 8, 4>(p, a, in1, st);
+  switch (p.kl == 8 ? 0 : p.ks * 10 + p.kr) {
+    case 0: Launch<8, 8, 1, 1>(p, a, in1, st); break;
+    case 11: Launch<8, 16, 1, 1>(p, a, in1, st); break;
+    case 12: Launch<8, 16, 2, 1>(p, a, in1, st); break;
+    case 13: Launch<8, 16, 3, 1>(p, a, in1, st); break;
+    case 14: Launch<8, 16, 4, 1>(p, a, in1, st); break;
+    case 41: Launch<4, 16, 1, 4>(p, a, in1, st); break;
+    case 42: Launch<4, 16, 2, 4>(p, a, in1, st); break;
+    case 43: Launch<4, 16, 3, 4>(p, a, in1, st); break;
+    case 44: Launch<4, 16, 4, 4>(p, a, in1, st); break;
+    case 46: Launch<4, 16, 6, 4>(p, a, in1, st); break;
+    default: Launch<4, 16, 8, 4>(p, a, in1, st);
   }
   TVX_HIP_CHECK(hipGetLastError());
   return TVX_OK;
@@ -299,6 +321,8 @@ int PwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   int kr = (ksteps + ks - 1) / ks;
   if (kr > 8) return TVX_E_UNSUPPORTED;
   if (kr > 4) kr = kr <= 6 ? 6 : 8;
+  const int kl = ks == 1 && C <= 32 ? 8 : 16;
+  plan.kl = kl;
   plan.ks = ks;
   plan.kr = kr;
   a.C = C;
@@ -309,14 +333,14 @@ int PwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   a.per_image = static_cast<uint32_t>(per_image);
   a.m_per_image = Magic(per_image);
   a.groups = static_cast<uint32_t>(groups);
-  a.limit = static_cast<uint32_t>(in_bytes - pw);
   const int ksteps_alloc = kr * ks;  // (steps past the last channel: zero weights)
   a.ksteps = ksteps_alloc;
   a.tiles = tiles;
   // pixel tiles fill the chip, or the output tiles of each are spread over wavefronts: two wavefronts a SIMD, or one where every
-  // further one reads more than 64 channels again (64 x 7 x 7 pixels, 960 -> 320 channels: 512 workgroups 9.2 us, 256 7.2 us)
+  // further one reads more than 64 channels again (64 x 7 x 7 pixels, 960 -> 320 channels: 512 workgroups 9.2 us, 256 7.2 us), four
+  // where that is at most 32 (64 x 56 x 56 pixels, 32 -> 128 channels: 2048 wavefronts 13.7 us, 4096 12.8, 8192 14.2)
   const uint64_t pix_tiles = (groups + 15) / 16;
-  uint64_t want = ks > 1 ? (ksteps > 8 ? 256 : 512) : (ksteps > 1 ? 1024 : 2048);
+  uint64_t want = ks > 1 ? (ksteps > 8 ? 256 : 512) : (ksteps > 1 ? 1024 : kl == 16 ? 2048 : 4096);
   if (const char* f = getenv("TVX_PWCONV_REG_WAVES")) want = std::max(1, atoi(f));  // tuning aid
   const uint64_t split = std::min<uint64_t>(tiles, std::max<uint64_t>(1, want / pix_tiles));
   a.tiles_per_wave = static_cast<int>((tiles + split - 1) / split);
@@ -346,7 +370,7 @@ int PwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   }
 
   // ---- weights in fragment order, constants folded into the bias ----
-  std::vector<int8_t> packed(static_cast<size_t>(tiles) * ksteps_alloc * 1024, 0);
+  std::vector<int8_t> packed(static_cast<size_t>(tiles) * ksteps_alloc * 64 * kl, 0);
   const uint8_t* src = static_cast<const uint8_t*>(w_host);
   const int32_t* bias = static_cast<const int32_t*>(bias_host);
   for (uint32_t oc = 0; oc < OC; ++oc) {
@@ -354,7 +378,8 @@ int PwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
     for (uint32_t c = 0; c < C; ++c) {
       const uint8_t r = src[static_cast<size_t>(oc) * C + c];
       const int8_t v = static_cast<int8_t>(w_u8 ? r ^ 0x80 : r);
-      packed[((static_cast<size_t>(oc / 16) * ksteps_alloc + c / 64) * 64 + c % 64 / 16 * 16 + oc % 16) * 16 + c % 16] = v;
+      const uint32_t step = c / (4 * kl), lane = c / kl % 4 * 16 + oc % 16;
+      packed[((static_cast<size_t>(oc / 16) * ksteps_alloc + step) * 64 + lane) * kl + c % kl] = v;
       sw += v;
     }
     const int64_t v = (bias ? bias[oc] : 0) - static_cast<int64_t>(zxs) * sw + static_cast<int64_t>(C) * zxs * zws;
@@ -363,7 +388,7 @@ int PwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   int s = op->packed.Upload(packed.data(), packed.size());
   if (s == TVX_OK) s = op->aux.Upload(rqt.data(), rqt.size() * 4);
   if (s != TVX_OK) return s;
-  a.wpk = op->packed.as<v4i>();
+  a.wpk = op->packed.as<uint8_t>();
   a.rec = op->aux.as<v4i>();
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
   op->run = PwRegRun;
