@@ -313,6 +313,13 @@ int PwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   // up to 256 channels (128 registers) in one wavefront; deeper inputs would leave too few wavefronts in flight: 16 x 14 x 14 pixels,
   // 512 -> 512 channels, 9.4 us with the reduction in one, 6.0 us shared by four (old form 6.8)
   int ks = hw >= 8 && ksteps <= 4 ? 1 : 4;
+  // ... and so do inputs of 65 to 256 channels where the results are few: a wavefront's loads, one step after the other, are most of such
+  // a launch. 7 x 19 x 19 pixels, 224 -> 256 channels: 5.6 us in one wavefront, 4.2 shared (5.2 staged in LDS); 4 x 18 x 18, 246 -> 24: 4.3,
+  // 3.0 (4.1); 64 x 7 x 7, 160 -> 960: 7.8, 7.3 (7.4). With more, the four wavefronts' exchange costs more than the shorter chain gives: over
+  // 200 drawn layers the two cross at about 1600 pieces of 64 pixels x 16 results for two steps and as many again for every further one
+  // (17 x 29 x 29, 65 -> 186, 2700 pieces: 3 % slower shared; 13 x 52 x 52, 208 -> 80, 2750 pieces: 10 % faster).
+  const uint64_t pieces = (((hw + 3) / 4) * d->batch + 15) / 16 * tiles;
+  if (ksteps > 1 && ksteps <= 4 && pieces <= 1600ull * (ksteps - 1)) ks = 4;
   if (const char* f = getenv("TVX_PWCONV_REG")) {  // tuning / test aid: wavefronts that share a reduction; 0 = off
     ks = atoi(f);
     if ((ks != 1 && ks != 4) || (ks == 1 && (hw < 8 || ksteps > 4))) return TVX_E_UNSUPPORTED;
@@ -340,7 +347,7 @@ int PwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   // further one reads more than 64 channels again (64 x 7 x 7 pixels, 960 -> 320 channels: 512 workgroups 9.2 us, 256 7.2 us), four
   // where that is at most 32 (64 x 56 x 56 pixels, 32 -> 128 channels: 2048 wavefronts 13.7 us, 4096 12.8, 8192 14.2)
   const uint64_t pix_tiles = (groups + 15) / 16;
-  uint64_t want = ks > 1 ? (ksteps > 8 ? 256 : 512) : (ksteps > 1 ? 1024 : kl == 16 ? 2048 : 4096);
+  uint64_t want = ks > 1 ? (ksteps > 8 ? 256 : ksteps > 4 ? 512 : 1024) : (ksteps > 1 ? 1024 : kl == 16 ? 2048 : 4096);
   if (const char* f = getenv("TVX_PWCONV_REG_WAVES")) want = std::max(1, atoi(f));  // tuning aid
   const uint64_t split = std::min<uint64_t>(tiles, std::max<uint64_t>(1, want / pix_tiles));
   a.tiles_per_wave = static_cast<int>((tiles + split - 1) / split);
