@@ -61,7 +61,7 @@ def test_conv2d_sweep(oracle, tvx):
         seen[d_kernel[0]] += 1
         assert np.array_equal(got, want), (i, cfg, mode, act, d_kernel[0], int((got != want).sum()))
     # the sweep is only worth its name if it reaches every convolution kernel
-    for k in ("conv2d_igemm_i8", "pwconv_i8", "dwconv3x3_i8", "dwconv_planes_i8", "conv2d_generic"):
+    for k in ("conv2d_tile_i8", "conv2d_igemm_i8", "pwconv_i8", "dwconv3x3_i8", "dwconv_planes_i8", "conv2d_generic"):
         assert seen[k] >= 5, seen
 
 

@@ -520,15 +520,19 @@ IGEMM_GRID = [
 
 @pytest.mark.parametrize("mode", ["u8", "i8pc", "u8pc"])
 @pytest.mark.parametrize("gi", range(len(IGEMM_GRID)))
-def test_conv2d_igemm_shapes(oracle, gi, mode):
+def test_conv2d_igemm_shapes(oracle, gi, mode, monkeypatch):
+    """The kernel each shape gets by default, and the dense int8 kernels it gets where the tiles decline."""
     n, c, h, w, oc, kh, kw, stride, dil, pad = IGEMM_GRID[gi]
     rng = np.random.default_rng(2000 + gi)
     x, wt, b, kws = conv_case(rng, n=n, c=c, h=h, w=w, oc=oc, kh=kh, kw=kw, stride=stride, dil=dil,
                               pad=pad, mult=0, mode=mode)
     want = oracle.conv2d(x, wt, b, act=1, **kws)
     pointwise = kh == 1 and kw == 1 and stride == [1, 1] and pad == [0, 0, 0, 0]
-    got = TC.gpu_conv2d(x, wt, b, act=1, want_kernel="pwconv_i8" if pointwise else IGEMM_KERNELS, **kws)
+    got = TC.gpu_conv2d(x, wt, b, act=1, want_kernel="pwconv_i8" if pointwise else IGEMM_KERNELS + ("conv2d_tile_i8",), **kws)
     assert np.array_equal(got, want)
+    if not pointwise:
+        monkeypatch.setenv("TVX_CONV_TILE", "0")
+        assert np.array_equal(TC.gpu_conv2d(x, wt, b, act=1, want_kernel=IGEMM_KERNELS, **kws), want)
     assert len(np.unique(want)) > 4
 
 
@@ -810,8 +814,9 @@ GEMM_GRID = [
 
 @pytest.mark.parametrize("mode", ["u8", "i8pc", "u8pc", "f16"])
 @pytest.mark.parametrize("gi", range(len(GEMM_GRID)))
-def test_conv2d_gemm(oracle, gi, mode):
-    """conv2d_gemm_i8 / conv2d_gemm_f16: windows gathered into LDS, MFMA over 64-byte chunks of the reduction."""
+def test_conv2d_gemm(oracle, gi, mode, monkeypatch):
+    """conv2d_gemm_i8 / conv2d_gemm_f16: windows gathered into LDS, MFMA over 64-byte chunks of the reduction. The tiles are
+    asked before them: the same shapes on whichever of the two they get by default."""
     n, c, oc, groups, h, w, kh, kw, stride, dil, pad = GEMM_GRID[gi]
     rng = np.random.default_rng(7300 + gi)
     x, wt, b, kws = conv_case(rng, n=n, c=c, h=h, w=w, oc=oc, kh=kh, kw=kw, stride=stride, dil=dil,
@@ -821,22 +826,29 @@ def test_conv2d_gemm(oracle, gi, mode):
         pytest.skip("the pointwise kernel takes the quantized 1x1 case")
     for act in (0, 2):
         want = oracle.conv2d(x, wt, b, act=act, **kws)
-        got = TC.gpu_conv2d(x, wt, b, act=act, want_kernel="conv2d_gemm_i8" if quant else "conv2d_gemm_f16", **kws)
-        if quant:
-            assert np.array_equal(got, want), int((got != want).sum())
-        else:
-            assert np.allclose(got.astype(np.float32), want.astype(np.float32), rtol=FLOAT_RTOL, atol=2e-2)
+        suffix = "i8" if quant else "f16"
+        for lever, kernels in (("0", "conv2d_gemm_" + suffix), (None, ("conv2d_gemm_" + suffix, "conv2d_tile_" + suffix))):
+            if lever:
+                monkeypatch.setenv("TVX_CONV_TILE", lever)
+            else:
+                monkeypatch.delenv("TVX_CONV_TILE")
+            got = TC.gpu_conv2d(x, wt, b, act=act, want_kernel=kernels, **kws)
+            if quant:
+                assert np.array_equal(got, want), int((got != want).sum())
+            else:
+                assert np.allclose(got.astype(np.float32), want.astype(np.float32), rtol=FLOAT_RTOL, atol=2e-2)
     assert len(np.unique(want)) > 4
 
 
-@pytest.mark.parametrize("kernel", ["conv2d_gemm_f16", "conv2d_igemm_f16"])
+@pytest.mark.parametrize("kernel", ["conv2d_gemm_f16", "conv2d_igemm_f16", "conv2d_tile_f16"])
 def test_conv2d_f16_kernels_match_float32_arithmetic(oracle, kernel, monkeypatch):
     """The float16 kernels accumulate in float32 and round once: against a float64 convolution of the same
     float16 operands the error stays within one float16 rounding of the result (plus the accumulation's)."""
     import torch
     import torch.nn.functional as F
-    if kernel == "conv2d_gemm_f16":
+    if kernel != "conv2d_igemm_f16":
         monkeypatch.setenv("TVX_NO_CONV_IGEMM_F16", "1")
+    monkeypatch.setenv("TVX_CONV_TILE", "1" if kernel == "conv2d_tile_f16" else "0")
     rng = np.random.default_rng(7400)
     n, c, oc, h, w = 2, 48, 64, 20, 20
     x, wt, b, kws = conv_case(rng, n=n, c=c, h=h, w=w, oc=oc, kh=3, kw=3, stride=[1, 1], dil=[1, 1],
@@ -873,6 +885,7 @@ def test_conv2d_igemm_f16(oracle, gi, pixel_tiles, monkeypatch):
     import os
     n, c, oc, h, w, kh, kw, stride, pad = IGEMM_F16_GRID[gi]
     monkeypatch.setenv("TVX_CONV_F16_PIXEL_TILES", str(pixel_tiles))   # 128- and 256-pixel workgroups
+    monkeypatch.setenv("TVX_CONV_TILE", "0")   # (asked between the two kernels compared)
     rng = np.random.default_rng(7600 + gi)
     x, wt, b, kws = conv_case(rng, n=n, c=c, h=h, w=w, oc=oc, kh=kh, kw=kw, stride=[stride, stride], dil=[1, 1],
                               pad=pad, mult=0, mode="f16")

@@ -59,6 +59,10 @@ CONV_TIE_CASES = [
     ("dwconv3x3_i8", dict(n=10, c=16, h=32, w=48, oc=16, k=3, stride=2, pad=1, mult=1), None),
     ("dwconv_planes_i8", dict(n=4, c=24, h=14, w=14, oc=24, k=3, stride=1, pad=1, mult=1), (15, 7)),
     ("dwconv_planes_i8", dict(n=32, c=40, h=9, w=11, oc=40, k=5, stride=1, pad=2, mult=1), None),
+    ("conv2d_tile_i8", dict(n=2, c=48, h=28, w=28, oc=96, k=3, stride=1, pad=1, mult=0), (15, 7)),
+    ("conv2d_tile_i8", dict(n=8, c=64, h=28, w=28, oc=80, k=3, stride=1, pad=1, mult=0), None),
+    ("conv2d_tile_i8", dict(n=2, c=40, h=16, w=16, oc=40, k=3, stride=1, pad=1, mult=0, groups=2), (15, 7)),
+    ("conv2d_tile_i8", dict(n=16, c=48, h=48, w=48, oc=48, k=3, stride=2, pad=1, mult=0, groups=2), None),
 ]
 
 
@@ -71,6 +75,8 @@ def test_conv_epilogues_round_ties_to_even(oracle, ci, mode, monkeypatch):
     if kernel.endswith("_persistent"):
         monkeypatch.setenv("TVX_IGEMM_PERSIST", "1")
         monkeypatch.setenv("TVX_CONV_BAND", "0")
+    if kernel in ("conv2d_igemm_i8", "conv2d_gemm_i8", "conv2d_tile_i8"):
+        monkeypatch.setenv("TVX_CONV_TILE", str(int(kernel == "conv2d_tile_i8")))
     if kernel == "conv2d_band_i8":
         monkeypatch.setenv("TVX_CONV_BAND", "1")
     if kernel.endswith("_stream"):  # (the form is chosen from 1024 pixel tiles up)

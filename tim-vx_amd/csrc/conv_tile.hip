@@ -677,7 +677,7 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
     const Shape& sp = kShapes[sidx];
     const int cand[] = {OW, (OW + 1) / 2, (OW + 2) / 3, 8, 16, 32, 64, 128};
     for (int tw : cand) {
-      if (want_tw && tw != want_tw) continue;
+      if (want_tw) tw = want_tw;
       if (tw < 1 || tw > OW || tw > sp.pixels) continue;
       Geometry g{};
       g.shape = sidx;
@@ -860,8 +860,7 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   }
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
   op->run = ConvTileRun;
-  // (the names these shapes have always been reported under: implicit GEMM for dense int8, GEMM over windows for the rest)
-  op->kernel_name = dt == kF32 ? "conv2d_igemm_f32" : dt == kF16 ? "conv2d_gemm_f16" : groups > 1 ? "conv2d_gemm_i8" : "conv2d_igemm_i8";
+  op->kernel_name = dt == kF32 ? "conv2d_tile_f32" : dt == kF16 ? "conv2d_tile_f16" : "conv2d_tile_i8";
   return TVX_OK;
 }
 
