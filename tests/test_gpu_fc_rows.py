@@ -30,7 +30,7 @@ def test_fully_connected_rows(oracle, m, k, n, mode, monkeypatch):
     want = oracle.fully_connected(x, w, b, act=1, **kws)
     for shape in range(3):   # 16 x 16, 32 x 32, 64 x 64
         monkeypatch.setenv("TVX_FC_ROWS_SHAPE", str(shape))
-        got = TC.gpu_fully_connected(x, w, b, act=1, **kws)
+        got = TC.gpu_fully_connected(x, w, b, act=1, want_kernel="fc_rows_" + {"f16": "f16", "f32": "f32"}.get(mode, "i8"), **kws)
         if mode in ("f16", "f32"):
             assert np.allclose(got.astype(np.float64), want.astype(np.float64), rtol=2e-3 if mode == "f16" else 1e-5, atol=2e-3 if mode == "f16" else 1e-5), shape
         else:
@@ -42,7 +42,7 @@ def test_fully_connected_rows_keep_an_infinity_apart(monkeypatch):
     monkeypatch.setenv("TVX_FC_ROWS", "1")
     x, w = np.ones((4, 37), np.float32), np.ones((20, 37), np.float32)
     x[2, 0] = np.inf
-    got = TC.gpu_fully_connected(x.ravel(), w.ravel(), None, m=4, k=37, n=20, in_dtype=3, w_dtype=3, out_dtype=3).reshape(4, 20)
+    got = TC.gpu_fully_connected(x.ravel(), w.ravel(), None, m=4, k=37, n=20, in_dtype=3, w_dtype=3, out_dtype=3, want_kernel="fc_rows_f32").reshape(4, 20)
     assert np.isinf(got[2]).all() and np.array_equal(got[[0, 1, 3]], np.full((3, 20), 37, np.float32))
 
 

@@ -342,21 +342,23 @@ def test_eltwise_float(oracle):
 FC_EDGE_SHAPES = [
     # 256 x 256 tiles: M, N not multiples of the tile, K not of the 128-byte step
     ((600, 512, 528), "fc_mfma_i8_256x256x128"), ((513, 144, 769), "fc_mfma_i8_256x256x128"),
-    # few outputs -> 16 x 16 tiles with the reduction split over four wavefronts: ragged M / N, N not a
+    # few outputs -> small tiles with the reduction split over wavefronts: ragged M / N, N not a
     # multiple of 4 (byte stores), K with a 16 / 32 / 48-byte tail and shorter than one 64-byte step,
     # more k-steps than one batch of loads, the MobileNetV2 and LeNet classifier shapes
-    ((300, 512, 272), "fc_mfma_i8_16x16_splitk"), ((257, 144, 513), "fc_mfma_i8_16x16_splitk"),
-    ((12, 1280, 1000), "fc_mfma_i8_16x16_splitk"), ((64, 1280, 1000), "fc_mfma_i8_16x16_splitk"),
-    ((256, 800, 500), "fc_mfma_i8_16x16_splitk"), ((17, 48, 1001), "fc_mfma_i8_16x16_splitk"),
-    ((1000, 16, 9), "fc_mfma_i8_16x16_splitk"), ((33, 4112, 250), "fc_mfma_i8_16x16_splitk"),
+    ((300, 512, 272), "fc_rows_i8"), ((257, 144, 513), "fc_rows_i8"),
+    ((12, 1280, 1000), "fc_rows_i8"), ((64, 1280, 1000), "fc_rows_i8"),
+    ((256, 800, 500), "fc_rows_i8"), ((17, 48, 1001), "fc_rows_i8"),
+    ((1000, 16, 9), "fc_rows_i8"), ((33, 4112, 250), "fc_rows_i8"),
 ]
 
 
 @pytest.mark.parametrize("mode", ["u8", "i8pc", "u8pc"])
 @pytest.mark.parametrize("shape,kernel", FC_EDGE_SHAPES)
-def test_fully_connected_mfma_edges(oracle, mode, shape, kernel):
+def test_fully_connected_mfma_edges(oracle, mode, shape, kernel, monkeypatch):
     """Tile and reduction edges of the two MFMA variants."""
     m, k, n = shape
+    if kernel != "fc_rows_i8":
+        monkeypatch.setenv("TVX_FC_ROWS", "0")   # (of its own accord the large form takes thousands of rows)
     rng = np.random.default_rng(m + k + n)
     in_dt = 0 if mode.startswith("u8") else 1
     w_dt = 0 if mode == "u8" else 1
@@ -449,7 +451,7 @@ def test_fully_connected_full_size_int8_per_channel(oracle):
 
 @pytest.mark.parametrize("shape", [(300, 200, 260), (256, 64, 256), (1, 8, 3), (517, 1032, 40)])
 @pytest.mark.parametrize("act", [0, 1, 2])
-def test_fully_connected_float16_mfma_edges(oracle, shape, act):
+def test_fully_connected_float16_mfma_edges(oracle, shape, act, monkeypatch):
     """float16 FC on the matrix cores: ragged M / N tiles, K tails (K % 64 != 0), fused
     ReLU / ReLU6. fp32 accumulation on both sides; tolerance 1e-2 relative."""
     m, k, n = shape
@@ -459,6 +461,8 @@ def test_fully_connected_float16_mfma_edges(oracle, shape, act):
     b = rng.standard_normal(n).astype(np.float32)
     kws = dict(m=m, k=k, n=n, in_dtype=2, w_dtype=2, out_dtype=2)
     want = oracle.fully_connected(x, w, b, act=act, **kws)
+    assert np.allclose(TC.gpu_fully_connected(x, w, b, act=act, want_kernel="fc_rows_f16", **kws).astype(np.float32), want.astype(np.float32), rtol=1e-2, atol=1e-2)
+    monkeypatch.setenv("TVX_FC_ROWS", "0")
     got = TC.gpu_fully_connected(x, w, b, act=act, want_kernel="fc_mfma_f16_256x256x64", **kws)
     assert np.allclose(got.astype(np.float32), want.astype(np.float32), rtol=1e-2, atol=1e-2)
     if act == 2:

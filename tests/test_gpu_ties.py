@@ -118,15 +118,17 @@ def test_conv_epilogues_round_ties_to_even(oracle, ci, mode, monkeypatch):
 FC_TIE_CASES = [
     ("fc_mfma_i8_256x256x128", (600, 512, 528), (15, 7)),
     ("fc_mfma_i8_256x256x128", (1025, 144, 769), None),
-    ("fc_mfma_i8_16x16_splitk", (300, 512, 272), (15, 7)),
-    ("fc_mfma_i8_16x16_splitk", (64, 1280, 1000), (None, 7)),
+    ("fc_rows_i8", (300, 512, 272), (15, 7)),
+    ("fc_rows_i8", (64, 1280, 1000), (None, 7)),
 ]
 
 
 @pytest.mark.parametrize("mode", ["u8", "i8pc"])
 @pytest.mark.parametrize("ci", range(len(FC_TIE_CASES)))
-def test_fully_connected_epilogues_round_ties_to_even(oracle, ci, mode):
+def test_fully_connected_epilogues_round_ties_to_even(oracle, ci, mode, monkeypatch):
     kernel, (mm, k, n), amp = FC_TIE_CASES[ci]
+    if kernel != "fc_rows_i8":
+        monkeypatch.setenv("TVX_FC_ROWS", "0")
     rng = np.random.default_rng(9100 + ci)
     u8 = mode == "u8"
     zx, zw, zo = (131, 117, 99) if u8 else (-2, 0, -9)

@@ -129,7 +129,8 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
       const uint8_t* p = xp[t] + static_cast<size_t>(s) * kStep;
       const uint8_t* last = a.x + (a.x_bytes - 16);
       p = p < last ? p : last;
-      if (SPLIT) {  // the dwords with the first and the last of the sixteen bytes, and what lies between
+      if (SPLIT) {  // the dwords with the first and the last of the sixteen bytes, and what lies between (at the tensor's ends up to three
+                    // bytes beside it, in a dword that holds bytes of it; they are shifted out)
         const uintptr_t at = reinterpret_cast<uintptr_t>(p);
         x[t] = *reinterpret_cast<const Dwords4*>(at & ~uintptr_t{3});
         x5[t] = *reinterpret_cast<const int*>((at + 15) & ~uintptr_t{3});
@@ -472,10 +473,7 @@ int FcRowsSetup(tvx_op* op, const tvx_fc_desc* d, const void* w_host, const void
   }
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
   op->run = FcRowsRun;
-  // (the names such layers have always been reported under, by size: callers compare them)
-  const uint64_t outputs = static_cast<uint64_t>(d->m) * d->n;
-  op->kernel_name = dt == kF32 ? "fc_rows_f32" : dt == kF16 ? (tiles_take_it ? "fc_mfma_f16_256x256x64" : "fc_rows_f16")
-                    : outputs <= 8192 ? "fc_generic" : !tiles_take_it ? "fc_rows_i8" : outputs <= (1u << 18) ? "fc_mfma_i8_16x16_splitk" : "fc_mfma_i8_256x256x128";
+  op->kernel_name = dt == kF32 ? "fc_rows_f32" : dt == kF16 ? "fc_rows_f16" : "fc_rows_i8";
   return TVX_OK;
 }
 
