@@ -345,9 +345,10 @@ int PwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   a.tiles = tiles;
   // pixel tiles fill the chip, or the output tiles of each are spread over wavefronts: two wavefronts a SIMD, or one where every
   // further one reads more than 64 channels again (64 x 7 x 7 pixels, 960 -> 320 channels: 512 workgroups 9.2 us, 256 7.2 us), four
-  // where that is at most 32 (64 x 56 x 56 pixels, 32 -> 128 channels: 2048 wavefronts 13.7 us, 4096 12.8, 8192 14.2)
+  // where that is at most 32 (64 x 56 x 56 pixels, 32 -> 128 channels: 1568 wavefronts 13.7 us, 3136 12.8, 6272 14.2) - short of four, since
+  // pixel tiles that make two wavefronts a SIMD as they are stay whole (19 x 116 x 116, 14 -> 80: 1998 wavefronts 10.8 us, 3996 11.5)
   const uint64_t pix_tiles = (groups + 15) / 16;
-  uint64_t want = ks > 1 ? (ksteps > 8 ? 256 : ksteps > 4 ? 512 : 1024) : (ksteps > 1 ? 1024 : kl == 16 ? 2048 : 4096);
+  uint64_t want = ks > 1 ? (ksteps > 8 ? 256 : ksteps > 4 ? 512 : 1024) : (ksteps > 1 ? 1024 : kl == 16 ? 2048 : 3584);
   if (const char* f = getenv("TVX_PWCONV_REG_WAVES")) want = std::max(1, atoi(f));  // tuning aid
   const uint64_t split = std::min<uint64_t>(tiles, std::max<uint64_t>(1, want / pix_tiles));
   a.tiles_per_wave = static_cast<int>((tiles + split - 1) / split);
