@@ -345,7 +345,7 @@ def test_mobilenet_v2_graph_bit_exact(tmp_path, oracle, batch, res):
     assert np.array_equal(out[0], ref), int((out[0] != ref).sum())
     # the ten residual Adds ride on the projection convolutions in front of them: no Add kernel in the plan
     plan = [l for l in log.splitlines() if "uid" in l and "->" in l]
-    assert sum("pwconv_add_i8" in l or "pwconv_add_blocked_i8" in l for l in plan) == 10 and not any("ADD" in l for l in plan), plan
+    assert sum("pwconv_add_i8" in l or "pwconv_reg_add_i8" in l or "pwconv_add_blocked_i8" in l for l in plan) == 10 and not any("ADD" in l for l in plan), plan
 
 
 @pytest.mark.gpu

@@ -29,7 +29,7 @@ def test_mobilenet_v2_batch64_224_bit_exact(tmp_path, oracle):
     assert len(np.unique(values[g["output"]])) > 100
     log = _check([g], tmp_path / "full", values, env={"VSI_NN_LOG_LEVEL": "3"})
     plan = [l for l in log.splitlines() if "uid" in l and "->" in l]
-    assert sum("pwconv_add_i8" in l or "pwconv_add_blocked_i8" in l for l in plan) == 10, plan
+    assert sum("pwconv_add_i8" in l or "pwconv_reg_add_i8" in l or "pwconv_add_blocked_i8" in l for l in plan) == 10, plan
     # the 7 x 7 stage runs between channel-blocked tensors: the stride-2 depthwise convolution in front writes the
     # first of them (no copy), the whole-plane average leaves the stage
     assert not any("layout_to_blocked" in l for l in plan) and sum("dwconv_planes_to_blocked_i8" in l for l in plan) == 1, plan

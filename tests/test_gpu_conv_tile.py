@@ -34,7 +34,7 @@ CASES = {
     "row_deep": dict(n=2, c=44, h=1, w=61, oc=8, kh=1, kw=3, stride=[1, 1], dil=[1, 1], pad=[1, 1, 0, 0]),
 }
 # quantized windows of at most 64 bytes and quantized 1 x 1 layers are taken by kernels that are asked before the tiles
-EARLIER = {"shallow": "conv2d_im2col_i8", "row": "conv2d_im2col_i8", "pointwise_strided": "conv2d_im2col_i8", "pointwise": "pwconv_i8"}
+EARLIER = {"shallow": "conv2d_im2col_i8", "row": "conv2d_im2col_i8", "pointwise_strided": "conv2d_im2col_i8", "pointwise": "pwconv_reg_i8"}
 
 
 @pytest.mark.parametrize("mode", ["u8", "i8pc", "f16", "f32"])

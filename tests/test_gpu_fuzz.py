@@ -61,7 +61,7 @@ def test_conv2d_sweep(oracle, tvx):
         seen[d_kernel[0]] += 1
         assert np.array_equal(got, want), (i, cfg, mode, act, d_kernel[0], int((got != want).sum()))
     # the sweep is only worth its name if it reaches every convolution kernel
-    for k in ("conv2d_tile_i8", "conv2d_igemm_i8", "pwconv_i8", "dwconv3x3_i8", "dwconv_planes_i8", "conv2d_generic"):
+    for k in ("conv2d_tile_i8", "conv2d_igemm_i8", "pwconv_reg_i8", "dwconv3x3_i8", "dwconv_planes_i8", "conv2d_generic"):
         assert seen[k] >= 5, seen
 
 
@@ -228,24 +228,22 @@ def test_depthwise_eight_column_form_sweep(oracle):
         assert np.array_equal(got, want), (i, n, c, h, w, pl, pt, mode, act, mis, int((got != want).sum()))
 
 
-def test_pointwise_streaming_form_sweep(oracle, monkeypatch):
-    """The streaming pointwise form forced onto random small cases: 1 to 32 input channels, pixel counts that are
-    multiples of 16 in several ways, partial output tiles, 1 to 5 pixel tiles per wavefront."""
-    monkeypatch.setenv("TVX_PWCONV_STREAM_MIN_TILES", "1")
-    monkeypatch.setenv("TVX_PWCONV_SHAPE", "128,1")
+def test_pointwise_shallow_inputs_sweep(oracle, monkeypatch):
+    """Random small cases of shallow inputs: 1 to 32 input channels, pixel counts that are multiples of 16 in several
+    ways, partial output tiles, output tiles shared by 1 to 5 times 16 wavefronts."""
     rng = np.random.default_rng(78)
     for i in range(60):
         n, c, oc = int(rng.integers(1, 6)), int(rng.integers(1, 33)), int(rng.integers(1, 200))
         w, h = 16, int(rng.integers(1, 40))
         if rng.integers(0, 2):
             w, h = 4 * int(rng.integers(1, 9)), 4 * int(rng.integers(1, 9))
-        monkeypatch.setenv("TVX_PWCONV_STREAM", str(int(rng.integers(1, 6))))
+        monkeypatch.setenv("TVX_PWCONV_REG_WAVES", str(16 * int(rng.integers(1, 6))))
         mode = str(rng.choice(["u8", "i8pc", "u8pc"]))
         x, wt, b, kws = conv_case(rng, n=n, c=c, h=h, w=w, oc=oc, kh=1, kw=1, stride=[1, 1], dil=[1, 1],
                                   pad=[0, 0, 0, 0], mult=0, mode=mode)
         act = int(rng.integers(0, 3))
         want = oracle.conv2d(x, wt, b, act=act, **kws)
-        got = TC.gpu_conv2d(x, wt, b, act=act, want_kernel="pwconv_i8_stream", **kws)
+        got = TC.gpu_conv2d(x, wt, b, act=act, want_kernel="pwconv_reg_i8", **kws)
         assert np.array_equal(got, want), (i, n, c, h, w, oc, mode, act, int((got != want).sum()))
 
 

@@ -532,7 +532,7 @@ def test_conv2d_igemm_shapes(oracle, gi, mode, monkeypatch):
                               pad=pad, mult=0, mode=mode)
     want = oracle.conv2d(x, wt, b, act=1, **kws)
     pointwise = kh == 1 and kw == 1 and stride == [1, 1] and pad == [0, 0, 0, 0]
-    got = TC.gpu_conv2d(x, wt, b, act=1, want_kernel="pwconv_i8" if pointwise else IGEMM_KERNELS + ("conv2d_tile_i8",), **kws)
+    got = TC.gpu_conv2d(x, wt, b, act=1, want_kernel="pwconv_reg_i8" if pointwise else IGEMM_KERNELS + ("conv2d_tile_i8",), **kws)
     assert np.array_equal(got, want)
     if not pointwise:
         monkeypatch.setenv("TVX_CONV_TILE", "0")
@@ -637,17 +637,19 @@ PW_GRID = [
 @pytest.mark.parametrize("mode", ["u8", "i8pc", "u8pc"])
 @pytest.mark.parametrize("gi", range(len(PW_GRID)))
 def test_pointwise_conv_shapes(oracle, gi, mode, shape, monkeypatch):
-    """Every workgroup shape of the kernel (pixels per workgroup, wavefronts) on every case,
-    not only the one the heuristic would pick."""
+    """Every workgroup shape of the LDS form (pixels per workgroup, wavefronts) on every case, not only the one the
+    heuristic would pick; None: the kernel that each case gets by default."""
     n, c, h, w, oc = PW_GRID[gi]
+    kernel = "pwconv_i8" if shape is not None or h * w < 4 else "pwconv_reg_i8"   # (asked first; images of four pixels and more)
     if shape is not None:
+        monkeypatch.setenv("TVX_PWCONV_REG", "0")
         monkeypatch.setenv("TVX_PWCONV_SHAPE", shape)
     rng = np.random.default_rng(4000 + gi)
     x, wt, b, kws = conv_case(rng, n=n, c=c, h=h, w=w, oc=oc, kh=1, kw=1, stride=[1, 1], dil=[1, 1],
                               pad=[0, 0, 0, 0], mult=0, mode=mode)
     for act in (0, 2):
         want = oracle.conv2d(x, wt, b, act=act, **kws)
-        got = TC.gpu_conv2d(x, wt, b, act=act, want_kernel="pwconv_i8", **kws)
+        got = TC.gpu_conv2d(x, wt, b, act=act, want_kernel=kernel, **kws)
         assert np.array_equal(got, want), int((got != want).sum())
     assert len(np.unique(want)) > 4
 
@@ -660,6 +662,7 @@ def test_pointwise_conv_walks_several_output_tiles_per_wavefront(oracle, gi, mod
     a batch-64 network): every wavefront then walks several output tiles in sequence, re-using its input tile
     and - with per-tensor uint8 weights whose zero point is not 128 - the zero-point sums it computed once."""
     n, c, h, w, oc = PW_GRID[gi]
+    monkeypatch.setenv("TVX_PWCONV_REG", "0")
     monkeypatch.setenv("TVX_PWCONV_SHAPE", shape)
     monkeypatch.setenv("TVX_PWCONV_WGS", "1")
     rng = np.random.default_rng(4100 + gi)
@@ -673,7 +676,7 @@ def test_pointwise_conv_walks_several_output_tiles_per_wavefront(oracle, gi, mod
     assert len(np.unique(want)) > 4
 
 
-STREAM_GRID = [
+SHALLOW_GRID = [
     # (n, c, h, w, oc): shallow inputs, pixel groups of sixteen inside one image
     (3, 32, 16, 48, 64),    # 18 pixel tiles, whole output tiles
     (2, 24, 20, 36, 40),    # padded input channels, a partial output tile, a ragged last pixel tile (1440 pixels)
@@ -682,22 +685,20 @@ STREAM_GRID = [
 ]
 
 
-@pytest.mark.parametrize("tiles", [1, 2, 5])
+@pytest.mark.parametrize("waves", ["1", "12", "100000"])
 @pytest.mark.parametrize("mode", ["u8", "i8pc", "u8pc"])
-@pytest.mark.parametrize("gi", range(len(STREAM_GRID)))
-def test_pointwise_conv_streaming_form(oracle, gi, mode, tiles, monkeypatch):
-    """The form for shallow inputs in which a wavefront walks several pixel tiles with the next tile's rows in
-    flight: forced onto small cases (it is chosen from 1024 pixel tiles up), 1, 2 and 5 tiles per wavefront."""
-    n, c, h, w, oc = STREAM_GRID[gi]
-    monkeypatch.setenv("TVX_PWCONV_STREAM_MIN_TILES", "1")
-    monkeypatch.setenv("TVX_PWCONV_STREAM", str(tiles))
-    monkeypatch.setenv("TVX_PWCONV_SHAPE", "128,1")
+@pytest.mark.parametrize("gi", range(len(SHALLOW_GRID)))
+def test_pointwise_conv_shallow_inputs(oracle, gi, mode, waves, monkeypatch):
+    """Inputs of at most 32 channels (steps of 32 channels): a pixel tile's output tiles in one wavefront, shared by a few, each
+    in its own."""
+    n, c, h, w, oc = SHALLOW_GRID[gi]
+    monkeypatch.setenv("TVX_PWCONV_REG_WAVES", waves)
     rng = np.random.default_rng(4300 + gi)
     x, wt, b, kws = conv_case(rng, n=n, c=c, h=h, w=w, oc=oc, kh=1, kw=1, stride=[1, 1], dil=[1, 1],
                               pad=[0, 0, 0, 0], mult=0, mode=mode)
     for act in (0, 2):
         want = oracle.conv2d(x, wt, b, act=act, **kws)
-        got = TC.gpu_conv2d(x, wt, b, act=act, want_kernel="pwconv_i8_stream", **kws)
+        got = TC.gpu_conv2d(x, wt, b, act=act, want_kernel="pwconv_reg_i8", **kws)
         assert np.array_equal(got, want), int((got != want).sum())
     assert len(np.unique(want)) > 4
 
@@ -966,7 +967,7 @@ def test_depthwise_then_pointwise_full_size(oracle):
               dilation=[1, 1], pad_left=0, pad_top=0, multiplier=0, in_dtype=1, w_dtype=1, out_dtype=1,
               in_q=(0.08, 0), w_q=(1.0, 0, sp), out_q=(0.05, 0), act=2)
     out_want = oracle.conv2d(mid, wp, bp, **kp)
-    out = TC.gpu_conv2d(mid, wp, bp, want_kernel=("pwconv_i8", "pwconv_i8_stream"), **kp)
+    out = TC.gpu_conv2d(mid, wp, bp, want_kernel="pwconv_reg_i8", **kp)
     assert np.array_equal(out, out_want)
     assert out.min() == 0 and out.max() == 120  # ReLU6 at scale 0.05
 
@@ -1119,7 +1120,7 @@ def test_pointwise_conv_with_fused_add(oracle, side, n, mode, conv_operand):
     e.b_scale, e.b_zp = bq
     e.out_scale, e.out_zp = sum_q
     op = T.conv2d_add_create(d, e, conv_operand, w, b)
-    assert op.kernel_name == "pwconv_add_i8"
+    assert op.kernel_name == ("pwconv_reg_add_i8" if side * side >= 4 else "pwconv_add_i8")
     import torch
     xd, od = TC.to_device(x), TC.to_device(other)
     yd = TC.device_out(want.size, TC.NP_OF[dt])

@@ -39,7 +39,7 @@ def test_pointwise_in_registers(oracle, n, c, h, w, oc, mode, monkeypatch):
             monkeypatch.setenv("TVX_PWCONV_REG", form)
             monkeypatch.setenv("TVX_PWCONV_REG_WAVES", waves)
             for act in (0, 1):
-                got = TC.gpu_conv2d(x, wt, b, act=act, want_kernel="pwconv_i8", **kws)
+                got = TC.gpu_conv2d(x, wt, b, act=act, want_kernel="pwconv_reg_i8", **kws)
                 assert np.array_equal(got, want[act]), (form, waves, act, int((got != want[act]).sum()))
             ran += 1
     assert ran

@@ -43,8 +43,8 @@ CONV_TIE_CASES = [
     # need accumulators of 2^10 .. 2^14 and are rare: those cases are sized for a few dozen of them)
     ("pwconv_i8", dict(n=2, c=32, h=16, w=16, oc=64, k=1, stride=1, pad=0, mult=0), (15, 7)),
     ("pwconv_i8", dict(n=8, c=96, h=14, w=14, oc=160, k=1, stride=1, pad=0, mult=0), None),
-    ("pwconv_i8_stream", dict(n=2, c=32, h=16, w=16, oc=64, k=1, stride=1, pad=0, mult=0), (15, 7)),
-    ("pwconv_i8_stream", dict(n=24, c=24, h=16, w=32, oc=72, k=1, stride=1, pad=0, mult=0), None),
+    ("pwconv_reg_i8", dict(n=2, c=32, h=16, w=16, oc=64, k=1, stride=1, pad=0, mult=0), (15, 7)),
+    ("pwconv_reg_i8", dict(n=24, c=24, h=16, w=32, oc=72, k=1, stride=1, pad=0, mult=0), None),
     ("conv2d_igemm_i8_persistent", dict(n=2, c=32, h=28, w=28, oc=64, k=3, stride=1, pad=1, mult=0), (15, 7)),
     ("conv2d_band_i8", dict(n=2, c=32, h=24, w=24, oc=64, k=3, stride=1, pad=1, mult=0), (15, 7)),
     ("conv2d_band_i8", dict(n=10, c=64, h=28, w=24, oc=64, k=3, stride=1, pad=1, mult=0), None),
@@ -59,6 +59,7 @@ CONV_TIE_CASES = [
     ("dwconv3x3_i8", dict(n=10, c=16, h=32, w=48, oc=16, k=3, stride=2, pad=1, mult=1), None),
     ("dwconv_planes_i8", dict(n=4, c=24, h=14, w=14, oc=24, k=3, stride=1, pad=1, mult=1), (15, 7)),
     ("dwconv_planes_i8", dict(n=32, c=40, h=9, w=11, oc=40, k=5, stride=1, pad=2, mult=1), None),
+    ("pwconv_reg_i8", dict(n=8, c=96, h=14, w=14, oc=160, k=1, stride=1, pad=0, mult=0), None),
     ("conv2d_tile_i8", dict(n=2, c=48, h=28, w=28, oc=96, k=3, stride=1, pad=1, mult=0), (15, 7)),
     ("conv2d_tile_i8", dict(n=8, c=64, h=28, w=28, oc=80, k=3, stride=1, pad=1, mult=0), None),
     ("conv2d_tile_i8", dict(n=2, c=40, h=16, w=16, oc=40, k=3, stride=1, pad=1, mult=0, groups=2), (15, 7)),
@@ -79,9 +80,8 @@ def test_conv_epilogues_round_ties_to_even(oracle, ci, mode, monkeypatch):
         monkeypatch.setenv("TVX_CONV_TILE", str(int(kernel == "conv2d_tile_i8")))
     if kernel == "conv2d_band_i8":
         monkeypatch.setenv("TVX_CONV_BAND", "1")
-    if kernel.endswith("_stream"):  # (the form is chosen from 1024 pixel tiles up)
-        monkeypatch.setenv("TVX_PWCONV_STREAM_MIN_TILES", "1")
-        monkeypatch.setenv("TVX_PWCONV_SHAPE", "128,1")
+    if kernel == "pwconv_i8":  # (asked behind the form that keeps pixels in registers)
+        monkeypatch.setenv("TVX_PWCONV_REG", "0")
     rng = np.random.default_rng(9000 + ci)
     u8 = mode == "u8"
     n, c, h, w, oc, k, stride, pad, dm = (g[key] for key in ("n", "c", "h", "w", "oc", "k", "stride", "pad", "mult"))

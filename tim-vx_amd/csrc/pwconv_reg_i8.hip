@@ -261,7 +261,7 @@ void Launch(const Plan& p, const PwrArgs& a, const void* res, hipStream_t st) {
 
 int PwRegRun(tvx_op* op, const void* in0, const void* in1, void* out, hipStream_t st) {
   const Plan& p = *reinterpret_cast<const Plan*>(op->host_blob.data());
-  if (p.add.add_mode && !in1) return SetError(TVX_E_INVALID, "pwconv_i8: the fused Add needs its second operand as in1");
+  if (p.add.add_mode && !in1) return SetError(TVX_E_INVALID, "pwconv_reg_add_i8: the fused Add needs its second operand as in1");
   PwrArgs a = p.a;
   a.x = static_cast<const uint8_t*>(in0);
   a.y = static_cast<uint8_t*>(out);
@@ -292,8 +292,6 @@ int PwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   if (d->k_w != 1 || d->k_h != 1 || d->stride_w != 1 || d->stride_h != 1 || d->pad_left != 0 || d->pad_top != 0 || d->out_w != d->in_w ||
       d->out_h != d->in_h)
     return TVX_E_UNSUPPORTED;
-  for (const char* lever : {"TVX_PWCONV_SHAPE", "TVX_PWCONV_WGS", "TVX_PWCONV_STREAM", "TVX_PWCONV_STREAM_MIN_TILES", "TVX_PWCONV_XCD_RUNS"})
-    if (getenv(lever)) return TVX_E_UNSUPPORTED;  // (tuning aids of the form that stages pixels in LDS)
   const uint64_t hw = static_cast<uint64_t>(d->in_w) * d->in_h;
   const uint64_t in_bytes = hw * d->in_c * d->batch, out_bytes = hw * d->out_c * d->batch;
   if (hw < 4 || in_bytes + (hw << 11) >= (1ull << 32) || out_bytes + (hw << 6) >= (1ull << 32)) return TVX_E_UNSUPPORTED;  // 32-bit offsets
@@ -400,7 +398,7 @@ int PwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   a.rec = op->aux.as<v4i>();
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
   op->run = PwRegRun;
-  op->kernel_name = op->fused_add ? "pwconv_add_i8" : "pwconv_i8";
+  op->kernel_name = op->fused_add ? "pwconv_reg_add_i8" : "pwconv_reg_i8";
   return TVX_OK;
 }
 
