@@ -149,6 +149,7 @@ template <int DT> struct Item {
 template <int DT, int WM, int WN, int KS, int MT, int NT, int R, int EU, bool MULTI>
 __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(EU))) ConvTileKernel(TileArgs a) {
   constexpr int kThreads = 64 * WM * WN * KS;
+  static_assert(R % 2 == 0, "the activations' two buffers alternate with the steps");
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   using acc_t = typename Kind<DT>::acc;
   using elem_t = typename Kind<DT>::elem;
@@ -522,7 +523,7 @@ const Shape kShapes[] = {
     TVX_TILE(4, 1, 2, 1, 1, 6, 4),  // 3: 128 x 32, eight
     TVX_TILE(4, 1, 1, 1, 1, 6, 4),  // 4: 128 x 32, four
     TVX_TILE(2, 2, 2, 1, 1, 6, 4),  // 5: 64 x 64, eight
-    TVX_TILE(2, 1, 4, 1, 1, 6, 4),  // 6: 64 x 32, eight
+    TVX_TILE(2, 1, 4, 1, 1, 4, 4),  // 6: 64 x 32, eight
     TVX_TILE(1, 1, 8, 1, 1, 6, 4),  // 7: 32 x 32, eight
 };
 #undef TVX_TILE
