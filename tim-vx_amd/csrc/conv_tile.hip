@@ -511,20 +511,20 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
 typedef void (*TileFn)(TileArgs);
 
 // The ways a workgroup's wavefronts share a tile.
-struct Shape { int pixels, channels, ks, waves; TileFn fn[3][2]; };
+struct Shape { int pixels, channels, ks, waves; double length; TileFn fn[3][2]; };  // length: of its chain, fitted (Cost)
 #define TVX_TILE_DT(DT, WM, WN, KS, MT, NT, R, EU) { ConvTileKernel<DT, WM, WN, KS, MT, NT, R, EU, false>, ConvTileKernel<DT, WM, WN, KS, MT, NT, R, 2, true> }
-#define TVX_TILE(WM, WN, KS, MT, NT, R, EU)                                                                       \
-  { WM * MT * 32, WN * NT * 32, KS, WM * WN * KS, { TVX_TILE_DT(kI8, WM, WN, KS, MT, NT, R, EU), TVX_TILE_DT(kF16, WM, WN, KS, MT, NT, R, EU), \
+#define TVX_TILE(WM, WN, KS, MT, NT, R, EU, LENGTH)                                                               \
+  { WM * MT * 32, WN * NT * 32, KS, WM * WN * KS, LENGTH, { TVX_TILE_DT(kI8, WM, WN, KS, MT, NT, R, EU), TVX_TILE_DT(kF16, WM, WN, KS, MT, NT, R, EU), \
                                                     TVX_TILE_DT(kF32, WM, WN, KS, MT, NT, R, EU) } }
 const Shape kShapes[] = {
-    TVX_TILE(4, 2, 1, 2, 1, 4, 4),  // 0: 256 x 64, eight wavefronts
-    TVX_TILE(2, 2, 2, 2, 1, 4, 4),  // 1: 128 x 64, eight
-    TVX_TILE(2, 2, 1, 2, 1, 4, 4),  // 2: 128 x 64, four
-    TVX_TILE(4, 1, 2, 1, 1, 6, 4),  // 3: 128 x 32, eight
-    TVX_TILE(4, 1, 1, 1, 1, 6, 4),  // 4: 128 x 32, four
-    TVX_TILE(2, 2, 2, 1, 1, 6, 4),  // 5: 64 x 64, eight
-    TVX_TILE(2, 1, 4, 1, 1, 4, 4),  // 6: 64 x 32, eight
-    TVX_TILE(1, 1, 8, 1, 1, 6, 4),  // 7: 32 x 32, eight
+    TVX_TILE(4, 2, 1, 2, 1, 4, 4, 1.0),   // 0: 256 x 64, eight wavefronts
+    TVX_TILE(2, 2, 2, 2, 1, 4, 4, 1.27),  // 1: 128 x 64, eight
+    TVX_TILE(2, 2, 1, 2, 1, 4, 4, 0.8),   // 2: 128 x 64, four
+    TVX_TILE(4, 1, 2, 1, 1, 6, 4, 1.43),  // 3: 128 x 32, eight
+    TVX_TILE(4, 1, 1, 1, 1, 6, 4, 1.0),   // 4: 128 x 32, four
+    TVX_TILE(2, 2, 2, 1, 1, 6, 4, 1.4),   // 5: 64 x 64, eight
+    TVX_TILE(2, 1, 4, 1, 1, 4, 4, 1.7),   // 6: 64 x 32, eight
+    TVX_TILE(1, 1, 8, 1, 1, 6, 4, 1.75),  // 7: 32 x 32, eight
 };
 #undef TVX_TILE
 #undef TVX_TILE_DT
@@ -549,26 +549,30 @@ struct Geometry {
   double cost;
 };
 
-// Microseconds of a launch, to compare tiles by. A workgroup is a chain - start, staging rounds (an item per thread and
-// round), steps, epilogue - whose length counts once per round of workgroups the chip holds; above that the units a CU's
-// workgroups share (its memory pipeline above all: 0.7 us per wavefront of int8 items) set the pace. The constants are a
-// fit to 8800 measured launches (180 drawn convolutions x the tiles below): the tile chosen costs 9 % more than the best
-// measured one on the (geometric) average, noise included, and 46 % at the worst.
-double Cost(const Shape& sp, const Geometry& g, int dt, int taps, int group_px, bool sums, bool whole_granules, bool borders, int OW) {
+// Microseconds of a launch, to compare tiles by. A workgroup is a chain - staging rounds (an item per thread and round), steps,
+// results - which grows longer with every workgroup that shares its CU and counts once per round of workgroups the chip holds; to that
+// come the units all of a CU's workgroups share (its memory pipeline, its matrix cores). The constants are a fit to 46000 launches
+// measured back to back in a captured graph (900 drawn convolutions x the tiles below). On 900 others the tile chosen takes 3 %
+// more than the best measured one on the (geometric) average, a quarter more in one of a hundred, half more at the worst. (Constants
+// fitted to launches from a host loop lost 11 % on the same ones, and up to 1.7 times on layers of a few microseconds: int8 14 -> 9
+// channels, 3x3 on 43 x 43, batch 14, 11.0 us where a tile of 6.3 was to be had. The host's own time had hidden what those take.)
+double Cost(const Shape& sp, const Geometry& g, int dt, int taps, int group_px, bool sums, bool borders, int OW, int cus) {
   const int threads = 64 * sp.waves, steps = (taps * g.gpc + 1) / 2, tiles = sp.pixels * sp.channels / 1024 * sp.ks / sp.waves;
   const double npx = static_cast<double>(g.G) * g.IH * g.IW;
   const double items = static_cast<double>(g.G) * g.IH * ((g.IW + group_px - 1) / group_px) * g.gpc;
   const double runs = g.TW == OW || g.TW % 4 == 0 ? 1.0 : 1.1;  // stores of whole quads
-  const double stage = (dt == kI8 ? 2.0 : 0.98) * std::ceil(items / threads) * (whole_granules ? 1.0 : 0.94) +
-                       0.3 * npx * g.gpc / threads * ((sums ? 1.0 : 0.0) + (borders ? 0.5 : 0.0));
-  const double multiply = static_cast<double>(steps) / sp.ks * (0.05 + (dt == kF32 ? 0.127 : 0.016) * tiles);
-  const double chain = 2.5 + g.chunks * (stage + g.loop * multiply) + g.loop * 0.32 * tiles / sp.ks * runs;
-  const double shared = g.chunks * ((dt == kF32 ? 0.096 : 0.69) * items / 64 + (dt == kF32 ? 0.045 : 0.0072) * g.loop * steps * tiles * sp.waves / sp.ks) +
-                        g.loop * 0.157 * sp.pixels * sp.channels / 1024 * runs;
-  const double per_cu = static_cast<double>(g.wgs) / 256;
-  const double resident = std::min<double>(std::max(1, std::min(16 / sp.waves, 160 * 1024 / g.lds_bytes)), std::max(1.0, std::ceil(per_cu)));
-  const double by_chain = per_cu <= resident ? chain : (per_cu / resident + 0.97) * chain, by_units = per_cu * shared;
-  return 2.7 + std::cbrt(by_chain * by_chain * by_chain + by_units * by_units * by_units);
+  const double stage = (dt == kI8 ? 1.4 : dt == kF16 ? 0.6 : 0.35) * std::ceil(items / threads) +
+                       0.25 * npx * g.gpc / threads * ((sums ? 1.0 : 0.0) + (borders ? 0.5 : 0.0));
+  const double multiply = static_cast<double>(steps) / sp.ks * (0.015 + (dt == kF32 ? 0.13 : 0.036) * tiles);
+  const double chain = 0.6 + g.chunks * (stage + g.loop * multiply) + g.loop * 1.2 * tiles / sp.ks * runs;
+  const double shared = g.chunks * ((dt == kI8 ? 0.12 : dt == kF16 ? 0.24 : 0.033) * items / 64 +
+                                    (dt == kF32 ? 0.016 : 0.0025) * g.loop * steps * tiles * sp.waves / sp.ks);
+  const double per_cu = static_cast<double>(g.wgs) / cus;
+  // (the kernels that walk chunks hold more than 128 registers, but for float32)
+  const int waves_cu = g.chunks > 1 && dt != kF32 ? 12 : 16;
+  const double resident = std::min<double>(std::max(1, std::min(waves_cu / sp.waves, 160 * 1024 / g.lds_bytes)), std::max(1.0, std::ceil(per_cu)));
+  const double by_chain = chain * sp.length * (1.0 + 0.48 * (resident - 1.0) * sp.waves / 8);
+  return 3.1 + by_chain * (per_cu <= resident ? 1.0 : per_cu / resident + 0.35) + per_cu * shared;
 }
 
 struct Plan {
@@ -667,6 +671,7 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   const int zws = dt == kI8 ? op->w_zp - (w_u8 ? 128 : 0) : 0;
 
   // ---- the tile ----
+  const int cus = ComputeUnits();
   int want = -1, want_tw = 0, want_loop = 0;
   if (const char* f = getenv("TVX_CONV_TILE_SHAPE")) want = atoi(f);  // test lever
   if (const char* f = getenv("TVX_CONV_TILE_COLS")) want_tw = atoi(f);  // test lever
@@ -712,7 +717,7 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
       const int64_t tiles = static_cast<int64_t>((OW + g.TW - 1) / g.TW) * ((OH + g.TH - 1) / g.TH) * ((d->batch + g.G - 1) / g.G);
       g.wgs = tiles * ((blocks + loop - 1) / loop) * groups;
       if (g.wgs > 0x3fffffff) continue;
-      g.cost = Cost(sp, g, dt, taps, group_px, zws != 0, (a.icg * E) % 16 == 0, (a.pad_l || a.pad_t) && taps > 1, OW);
+      g.cost = Cost(sp, g, dt, taps, group_px, zws != 0, (a.pad_l || a.pad_t) && taps > 1, OW, cus);
       if (best.shape < 0 || g.cost < best.cost) best = g;
       }
     }

@@ -146,6 +146,12 @@ bool BuildTieRecords(const std::vector<int32_t>& mult, const std::vector<int32_t
   return true;
 }
 
+int ComputeUnits() {
+  int device = 0, n = 0;
+  if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0) return 256;
+  return n;
+}
+
 void ActRange(int out_dtype, float out_scale, int32_t out_zp, int act, int32_t* lo, int32_t* hi) {
   *lo = out_dtype == TVX_U8 ? 0 : -128;
   *hi = out_dtype == TVX_U8 ? 255 : 127;

@@ -325,6 +325,9 @@ int64_t AccumulatorBound(uint64_t reduction, const void* bias_host, uint32_t cha
 int BuildRequantTables(uint32_t channels, float in_scale, float w_scale,
                        const float* w_scales, float out_scale,
                        std::vector<int32_t>* mult, std::vector<int32_t>* shift);
+// compute units of the current device
+int ComputeUnits();
+
 void ActRange(int out_dtype, float out_scale, int32_t out_zp, int act, int32_t* lo, int32_t* hi);
 inline bool IsQuant(int dtype) { return dtype == TVX_U8 || dtype == TVX_I8; }
 inline size_t DtypeBytes(int dtype) {
