@@ -152,3 +152,31 @@ def test_conv2d_tile_pads_wider_than_the_window(oracle, k, stride, dil, h, w, mo
 def test_conv2d_pads_wider_than_the_window_by_default(oracle, mode, case):
     x, wt, b, kws = conv_case(np.random.default_rng(710), mult=0, mode=mode, **case)
     _check(TC.gpu_conv2d(x, wt, b, act=1, want_kernel=KERNEL[mode], **kws), oracle.conv2d(x, wt, b, act=1, **kws), mode, "default")
+
+
+ROUTES = [
+    # mode, layer, kernel: both sides of the lines between the tiles and the kernels asked behind them
+    ("u8", dict(c=16, h=8, w=8, oc=16, kh=3, kw=3, pad=[1, 1, 1, 1]), "conv2d_igemm_i8"),            # one granule, weights with a zero point
+    ("u8", dict(c=17, h=8, w=8, oc=16, kh=3, kw=3, pad=[1, 1, 1, 1]), "conv2d_tile_i8"),
+    ("i8pc", dict(c=16, h=8, w=8, oc=16, kh=3, kw=3, pad=[1, 1, 1, 1]), "conv2d_tile_i8"),           # without one
+    ("u8", dict(c=16, h=17, w=17, oc=16, kh=3, kw=3, pad=[1, 1, 1, 1]), "conv2d_tile_i8"),           # rows of no whole dwords, a larger plane
+    ("u8", dict(c=16, h=17, w=20, oc=16, kh=3, kw=3, pad=[1, 1, 1, 1]), "conv2d_igemm_i8"),
+    ("i8pc", dict(c=80, h=9, w=9, oc=64, kh=1, kw=1, pad=[0] * 4, groups=2), "conv2d_gemm_i8"),      # 32 results of a group
+    ("i8pc", dict(c=80, h=9, w=9, oc=66, kh=1, kw=1, pad=[0] * 4, groups=2), "conv2d_tile_i8"),
+    ("i8pc", dict(c=8, h=9, w=9, oc=64, kh=1, kw=1, pad=[0] * 4, groups=2), "conv2d_generic"),       # four products a result
+    ("i8pc", dict(c=18, h=9, w=9, oc=64, kh=1, kw=1, pad=[0] * 4, groups=2), "conv2d_tile_i8"),
+    ("f16", dict(c=64, h=10, w=10, oc=512, kh=1, kw=1, pad=[0] * 4), "conv2d_gemm_f16"),
+    ("f16", dict(c=64, h=10, w=10, oc=513, kh=1, kw=1, pad=[0] * 4), "conv2d_tile_f16"),
+    ("f16", dict(c=32, h=9, w=9, oc=8, kh=1, kw=1, pad=[0] * 4), "conv2d_gemm_f16"),
+    ("f16", dict(c=144, h=64, w=128, oc=24, kh=1, kw=1, pad=[0] * 4), "conv2d_gemm_f16"),            # 16384 pixels of whole cache lines
+    ("f16", dict(c=144, h=63, w=127, oc=24, kh=1, kw=1, pad=[0] * 4), "conv2d_tile_f16"),
+]
+
+
+@pytest.mark.parametrize("mode,layer,kernel", ROUTES)
+def test_conv2d_tile_or_an_older_kernel(oracle, mode, layer, kernel, monkeypatch):
+    if mode == "f16":
+        monkeypatch.setenv("TVX_NO_CONV_IGEMM_F16", "1")   # (asked before both)
+    x, wt, b, kws = conv_case(np.random.default_rng(720), mult=0, mode=mode, n=2, stride=[1, 1], dil=[1, 1], **layer)
+    got = TC.gpu_conv2d(x, wt, b, act=1, want_kernel=kernel, **kws)
+    _check(got, oracle.conv2d(x, wt, b, act=1, **kws), mode, kernel)

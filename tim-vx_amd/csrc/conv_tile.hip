@@ -596,38 +596,46 @@ int ConvTileRun(tvx_op* op, const void* in0, const void*, void* out, hipStream_t
 
 }  // namespace
 
-// Which shapes stay with the kernels asked behind this one (measured on 290 drawn convolutions; the others are 2.4 times
-// faster here than on conv2d_igemm_i8, 3 on conv2d_gemm_f16 and 5 on conv2d_generic, on the geometric average):
-static bool IsBetterChoice(const tvx_conv2d_desc* d, int dt) {
-  const int groups = d->groups > 1 ? d->groups : 1;
+// Which shapes stay with the kernels asked behind this one (measured back to back in a captured graph on 3900 drawn convolutions;
+// what is left slower here than there by more than 3 % is one in twenty-five, at most 1.4 times):
+static bool IsBetterChoice(const tvx_conv2d_desc* d, int dt, bool sums) {
+  const int groups = d->groups > 1 ? d->groups : 1, ocg = d->out_c / groups;
   const uint64_t reduction = static_cast<uint64_t>(d->in_c / groups) * d->k_w * d->k_h;
   const uint64_t macs = reduction * d->out_c * d->out_w * d->out_h * d->batch;
+  const bool pointwise = d->k_w == 1 && d->k_h == 1;
   // a group of three output channels and fewer fills less than a tenth of a tile's 32 channels: only where each has little to add up
   // (float16 432 -> 12 in four groups, 7x7 on 42 x 42, batch 28: 2495 us with one thread per output, 140 here)
-  if (groups > 1 && d->out_c / groups < 4 && reduction <= 128) return false;
-  // a handful of products per output: one thread per output is quicker than staging a window (4.3 against 5.7 us)
+  if (groups > 1 && ocg < 4 && reduction <= 128) return false;
+  // a handful of products per output: one thread per output is quicker than staging a window (4.3 against 5.7 us; int8 in groups, which
+  // has no other kernel for so few: 4 -> 64 in two, 1x1 on 25 x 25, 3.9 against 6.5, but 64 -> 240 in eight on 22 x 22 7.7 against 6.0)
   if (dt != kI8 && reduction <= 9 && macs <= 4000000) return false;
+  if (dt == kI8 && groups > 1 && reduction <= 8 && macs <= (reduction <= 4 ? 4000000 : 1000000)) return false;
+  // int8 1 x 1 in groups that fill less than a tile's channels: conv2d_gemm_i8 (188 -> 60 in four groups on 108 x 108, batch 6: 9.9 against
+  // 17.4 us, 240 -> 96 on 74 x 74, batch 49: 36.8 against 52.3); with more than 32 channels in a group the tiles (144 -> 128 in two on
+  // 29889 pixels: 9.5 against 16.8)
+  if (dt == kI8 && groups > 1 && pointwise && reduction >= 32 && reduction <= 128 && ocg >= 8 && ocg <= 32) return false;
   // float16 1 x 1: conv2d_gemm_f16 gathers four pixels a load where planes are whole quads and has less to set up. Few channels (4.2
-  // against 6.9 us at 24 -> 16 on 50 x 50, batch 4; 8.9 against 11.5 at 40 -> 192 on 44 x 44, batch 13; above 64 the tiles: 8.0 against 33.4
-  // at 448 -> 320 on 26 x 26), tiny layers (4.4 against 6.0), and few results of many pixels (21.7 against 41.5 at 368 -> 8 on
-  // 112 x 112, batch 10; 59.9 against 47.9 at 256 -> 273 on 54 x 54).
-  if (dt == kF16 && groups == 1 && d->k_w == 1 && d->k_h == 1 && d->in_c >= 16) {
-    const uint64_t plane = static_cast<uint64_t>(d->in_w) * d->in_h;
-    if (d->in_c <= 32 && macs <= 20000000) return false;
-    if (d->stride_w == 1 && d->stride_h == 1 && plane % 4 == 0) {
-      if (d->in_c <= 64 && d->out_c <= 256 && macs <= 200000000) return false;
-      if (d->out_c <= 96 && plane * d->batch >= 32768) return false;
+  // against 6.9 us at 24 -> 16 on 50 x 50, batch 4; 7.4 against 9.5 at 40 -> 384 on 28 x 28, batch 12), few results (10.2 against 13.4 at
+  // 32 -> 8 on 105 x 105, batch 18). Its rows are cache lines where a plane is a multiple of sixteen pixels: there also few results of
+  // many pixels (22.0 against 28.6 at 480 -> 16 on 146 x 160, batch 4) and many pixels of deep inputs (38.5 against 53.7 at 240 -> 240 on
+  // 60 x 60, batch 19; 74.3 against 100.5 at 465 -> 224 on 44 x 44, batch 48); on other planes the tiles (117 against 61.5 at 496 -> 160 on
+  // 58 x 58, batch 22).
+  if (dt == kF16 && groups == 1 && pointwise && d->in_c >= 16) {
+    const uint64_t plane = static_cast<uint64_t>(d->in_w) * d->in_h, pixels = plane * d->batch;
+    if (d->in_c <= 32 && (macs <= 20000000 || d->out_c <= 8)) return false;
+    if (d->stride_w == 1 && d->stride_h == 1) {
+      if (plane % 4 == 0 && d->in_c <= 64 && d->out_c <= 512 && macs <= 200000000) return false;
+      if (plane % 16 == 0 && ((d->out_c <= 16 && pixels >= 32768) || (d->in_c >= 144 && pixels >= 16384))) return false;
     }
   }
   if (dt == kI8 && groups == 1) {
     if (ConvIgemmPersists(d)) return false;
-    // shallow inputs whose rows are whole dwords at stride 1: conv2d_igemm_i8 stages all channels of a tile in one aligned
-    // pass and its weights fit LDS beside it (6.9 against 8.9 us at 32 -> 80 on 16 x 16, batch 27); with more work than
-    // this its tiles queue up (43 against 28 us at 8 -> 416 on 40 x 40, batch 24)
-    if (d->in_c <= 32 && d->stride_w == 1 && d->stride_h == 1 && d->in_w % 4 == 0 && macs <= 400000000 && reduction <= 512) return false;
-    // a granule of channels or two on planes of at most 16 x 16: its shorter chain (5.2 against 7.0 us at 12 -> 8 on 7 x 7, batch 29; 6.9
-    // against 8.9 at 16 -> 240 on 7 x 13, batch 7); on larger planes the tiles win as often as not, and then by more (12.8 against 7.0)
-    if (d->in_c <= 24 && d->in_w * d->in_h <= 256 && macs <= 250000000 && reduction <= 512) return false;
+    // a granule of channels under weights with a zero point: conv2d_igemm_i8 takes the window sums from a second multiplication instead of a
+    // pass over the window, stages rows of whole dwords in one aligned pass, and its chain is short on planes of at most 16 x 16 (16 ->
+    // 16, 3x3 on 7 x 7, batch 20, 5.4 against 6.6 us; even on the average). With more work than this its tiles queue up
+    // (8 -> 416 on 40 x 40, batch 24, 43 against 28); without the sums, and from two granules on, the tiles are ahead by a sixth.
+    const bool aligned = d->stride_w == 1 && d->stride_h == 1 && d->in_w % 4 == 0 && macs <= 400000000;
+    if (sums && d->in_c <= 16 && reduction <= 512 && (aligned || (d->in_w * d->in_h <= 256 && macs <= 250000000))) return false;
   }
   return true;
 }
@@ -647,7 +655,7 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
     if (atoi(f) == 0) return TVX_E_UNSUPPORTED;
     forced = true;
   }
-  if (!forced && !IsBetterChoice(d, dt)) return TVX_E_UNSUPPORTED;
+  if (!forced && !IsBetterChoice(d, dt, dt == kI8 && op->w_zp != (d->w_dtype == TVX_U8 ? 128 : 0))) return TVX_E_UNSUPPORTED;
 
   TileArgs a{};
   int W = d->in_w, H = d->in_h, OW = d->out_w, OH = d->out_h;
