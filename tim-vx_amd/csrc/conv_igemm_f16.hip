@@ -267,12 +267,7 @@ int ConvIgemmF16Setup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, 
   a.aligned4 = hw % 4 == 0;
   // 256-pixel workgroups (two pixel tiles a wavefront: every weight fragment multiplies twice) where that still leaves
   // two workgroups per CU and the rows behind them fit LDS
-  int cus = 256;
-  {
-    hipDeviceProp_t prop;
-    int dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess) cus = prop.multiProcessorCount;
-  }
+  const int cus = ComputeUnits();
   auto lds_of = [&](int pt) {
     const int rows = static_cast<int>(std::min<int64_t>(a.OH, (kPixels * pt + a.OW - 2) / a.OW + 1));  // most output rows the pixels of a tile touch
     return (static_cast<int64_t>(rows - 1) * a.s + a.kh) * a.halo_w * a.pix_stride;

@@ -858,10 +858,7 @@ int ConvIgemmSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, con
   // tiles) plus two blocks' worth of loads and barriers, the launch as that times the rounds the workgroups
   // need on two slots per CU; ties go to the larger tiles (fewer halo copies).
   {
-    int cus = 256;
-    hipDeviceProp_t prop;
-    int dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess) cus = prop.multiProcessorCount;
+    const int cus = ComputeUnits();
     const long long slots = 2ll * cus;
     auto workgroups = [&](int ot_, int p_) {
       return static_cast<long long>(d->batch) * ((hw + p_ - 1) / p_) * ((oc_pad + 32 * ot_ - 1) / (32 * ot_));

@@ -397,12 +397,8 @@ int DwPwSetup(tvx_op* op, const tvx_conv2d_desc* dw, const void* dw_w, const voi
   // Among the tiles that fit: the one with the least work on the busiest CU. A CU handles a whole number of
   // tiles; a tile's cost grows with its pixels, shorter tiles re-read more input rows per output row.
   int rpt = 0;
+  const int cus = ComputeUnits();
   {
-    int cus = 256;
-    hipDeviceProp_t prop;
-    int dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0)
-      cus = prop.multiProcessorCount;
     double best = 0;
     for (int r : {4, 2, 1}) {
       if (!fits(r) || lds_of(r) > 52 * 1024) continue;
@@ -476,7 +472,7 @@ int DwPwSetup(tvx_op* op, const tvx_conv2d_desc* dw, const void* dw_w, const voi
   // -> 128 45.5 -> 36.1. One round: 32 x 32 x 112 x 112 -> 64 20.7 -> 24.7 us; sixteen in flight: 96, 112 -> 56, batch 64 26.5 -> 27.7.
   const int kRows = S * (rpt - 1) + 3, batch = std::max(1, std::min(8, 24 / (kRows * S)));
   const int passes = (C + (64 * kWaves >> lpr_shift) - 1) / (64 * kWaves >> lpr_shift);
-  const uint64_t resident = std::min<uint64_t>(std::min(4, 160 * 1024 / lds_bytes), (tiles + 255) / 256);
+  const uint64_t resident = std::min<uint64_t>(std::min(4, 160 * 1024 / lds_bytes), (tiles + cus - 1) / cus);
   int waves = passes > batch && resident < 4 ? kMaxWaves : kWaves;
   if (const char* f = getenv("TVX_DWPW_WAVES")) waves = atoi(f) >= kMaxWaves ? kMaxWaves : kWaves;  // tuning aid
   if (lds_bytes + (waves - kWaves) * kStageBytes > 160 * 1024) waves = kWaves;

@@ -333,8 +333,9 @@ uint32_t Magic(int d) { return d <= 1 ? 0u : static_cast<uint32_t>(((uint64_t{1}
 // were measured on the same 220 drawn layers and won nowhere by more than a tenth.
 int ChooseShape(const tvx_fc_desc& d, int elem_bytes) {
   const uint64_t t16 = static_cast<uint64_t>((d.m + 15) / 16) * ((d.n + 15) / 16), t64 = static_cast<uint64_t>((d.m + 63) / 64) * ((d.n + 63) / 64);
-  if (t16 <= 256) return 0;
-  if (t64 >= 384 || (t64 >= 128 && static_cast<uint64_t>(d.k) * elem_bytes <= 384)) return 2;
+  const uint64_t cus = ComputeUnits();
+  if (t16 <= cus) return 0;
+  if (2 * t64 >= 3 * cus || (2 * t64 >= cus && static_cast<uint64_t>(d.k) * elem_bytes <= 384)) return 2;
   return 1;
 }
 
@@ -344,7 +345,8 @@ bool LargeTilesWin(const tvx_fc_desc& d, int dt) {
   const double flop = 2.0 * d.m * d.n * d.k;
   const double rows = 3.5 + flop / (dt == kI8 ? 330e6 : 235e6);
   const uint64_t tiles = static_cast<uint64_t>((d.m + 255) / 256) * ((d.n + 255) / 256);
-  const double large = static_cast<double>((tiles + 255) / 256) * (dt == kI8 ? 17.0 + 0.009 * d.k : 25.0 + 0.0118 * d.k);
+  const uint64_t cus = ComputeUnits();
+  const double large = static_cast<double>((tiles + cus - 1) / cus) * (dt == kI8 ? 17.0 + 0.009 * d.k : 25.0 + 0.0118 * d.k);
   return large < rows;
 }
 

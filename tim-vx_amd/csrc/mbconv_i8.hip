@@ -500,7 +500,7 @@ int MbConvSetup(tvx_op* op, const MbStage& ex, const MbStage& dw, const tvx_conv
   // With at most one workgroup a CU eight wavefronts walk the chunks in half the rounds; with more, four and a second workgroup
   // are better. 64 -> 384 -> 64 and 96 -> 576 -> 96 channels on 14 x 14: batch 1 11.9 -> 9.1 and 20.1 -> 13.1 us, batch 64 14.3 and 23.7
   // against 19.1 and 24.9 with eight.
-  int waves = wgs <= 256 ? MaxWaves(MO * (nt <= 2 ? 2 : nt <= 5 ? 5 : 10)) : kMinWaves;
+  int waves = wgs <= static_cast<uint64_t>(ComputeUnits()) ? MaxWaves(MO * (nt <= 2 ? 2 : nt <= 5 ? 5 : 10)) : kMinWaves;
   if (const char* f = getenv("TVX_MBCONV_WAVES")) waves = std::max(kMinWaves, atoi(f));  // tuning aid
   waves = std::min(waves, MaxWaves(MO * (nt <= 2 ? 2 : nt <= 5 ? 5 : 10)));
   while (waves > kMinWaves && a.off_wave + waves * a.wave_bytes + nt * MO * 4096 > 160 * 1024) --waves;

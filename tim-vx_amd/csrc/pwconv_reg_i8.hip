@@ -316,8 +316,8 @@ int PwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   // 3.0 (4.1); 64 x 7 x 7, 160 -> 960: 7.8, 7.3 (7.4). With more, the four wavefronts' exchange costs more than the shorter chain gives: over
   // 200 drawn layers the two cross at about 1600 pieces of 64 pixels x 16 results for two steps and as many again for every further one
   // (17 x 29 x 29, 65 -> 186, 2700 pieces: 3 % slower shared; 13 x 52 x 52, 208 -> 80, 2750 pieces: 10 % faster).
-  const uint64_t pieces = (((hw + 3) / 4) * d->batch + 15) / 16 * tiles;
-  if (ksteps > 1 && ksteps <= 4 && pieces <= 1600ull * (ksteps - 1)) ks = 4;
+  const uint64_t cus = ComputeUnits(), pieces = (((hw + 3) / 4) * d->batch + 15) / 16 * tiles;
+  if (ksteps > 1 && ksteps <= 4 && 4 * pieces <= 25 * cus * (ksteps - 1)) ks = 4;
   if (const char* f = getenv("TVX_PWCONV_REG")) {  // tuning / test aid: wavefronts that share a reduction; 0 = off
     ks = atoi(f);
     if ((ks != 1 && ks != 4) || (ks == 1 && (hw < 8 || ksteps > 4))) return TVX_E_UNSUPPORTED;
@@ -346,7 +346,7 @@ int PwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   // where that is at most 32 (64 x 56 x 56 pixels, 32 -> 128 channels: 1568 wavefronts 13.7 us, 3136 12.8, 6272 14.2) - short of four, since
   // pixel tiles that make two wavefronts a SIMD as they are stay whole (19 x 116 x 116, 14 -> 80: 1998 wavefronts 10.8 us, 3996 11.5)
   const uint64_t pix_tiles = (groups + 15) / 16;
-  uint64_t want = ks > 1 ? (ksteps > 8 ? 256 : ksteps > 4 ? 512 : 1024) : (ksteps > 1 ? 1024 : kl == 16 ? 2048 : 3584);
+  uint64_t want = cus * (ks > 1 ? (ksteps > 8 ? 1 : ksteps > 4 ? 2 : 4) : (ksteps > 1 ? 4 : kl == 16 ? 8 : 14));
   if (const char* f = getenv("TVX_PWCONV_REG_WAVES")) want = std::max(1, atoi(f));  // tuning aid
   const uint64_t split = std::min<uint64_t>(tiles, std::max<uint64_t>(1, want / pix_tiles));
   a.tiles_per_wave = static_cast<int>((tiles + split - 1) / split);
