@@ -573,7 +573,9 @@ double Cost(const Shape& sp, const Geometry& g, int dt, int taps, int group_px, 
   // (the kernels that walk chunks hold more than 128 registers, but for float32)
   const int waves_cu = g.chunks > 1 && dt != kF32 ? 12 : 16;
   const double resident = std::min<double>(std::max(1, std::min(waves_cu / sp.waves, 160 * 1024 / g.lds_bytes)), std::max(1.0, std::ceil(per_cu)));
-  const double by_chain = chain * sp.length * (1.0 + 0.48 * (resident - 1.0) * sp.waves / 8);
+  // (eight wavefronts without shares of a sum walk chunks alone on their CU, 1.06 to 1.25 times as long as their length says)
+  const double alone = sp.ks == 1 && sp.waves == 8 && waves_cu == 12 ? 1.12 : 1.0;
+  const double by_chain = chain * sp.length * alone * (1.0 + 0.48 * (resident - 1.0) * sp.waves / 8);
   return 3.1 + by_chain * (per_cu <= resident ? 1.0 : per_cu / resident + 0.35) + per_cu * shared;
 }
 
