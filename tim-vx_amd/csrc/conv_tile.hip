@@ -21,9 +21,9 @@
 //
 // What bounds it: at the sizes convolutional networks have, a launch is a chain of one memory round trip, the LDS
 // transposition (about 70 vector instructions per 64 staged bytes for int8, none for float32) and the steps themselves, and no unit
-// is busy for long: int8 3x3 256 -> 256 on 14 x 14, batch 32 (13.6 us under the tracer): vector units 26 %, LDS 22 % and a third of that
-// in bank conflicts, matrix cores 16 %, wavefronts waiting 45 % of their cycles; float16 5x5 96 -> 256 on 27 x 27, batch 16 (32.3 us):
-// 37, 37, 30 and 35 %. The tile is chosen on the host so that the chip is filled first and the halo staged per output pixel is small second.
+// is busy for long: int8 3x3 256 -> 256 on 14 x 14, batch 32 (13.3 us under the tracer): vector units 26 %, LDS 22 % and a third of that
+// in bank conflicts, matrix cores 16 %, wavefronts waiting 45 % of their cycles; float16 5x5 96 -> 256 on 27 x 27, batch 16 (31.8 us):
+// 40, 51 (half of it conflicts), 28 and 38 %. The tile is chosen on the host so that the chip is filled first and the halo staged per output pixel is small second.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
