@@ -1,0 +1,497 @@
+// Depthwise convolution (multiplier 1) as a register stencil on planes of any width: float16 and float32 windows of 3x3 and
+// 5x5, int8 / uint8 windows of 5x5 (and of 3x3 on rows that are not whole dwords), at stride 1 or 2 (vxConvolutionLayer's depthwise form; reference:
+// src/tim/vx/internal/src/ops/vsi_nn_op_conv2d.c:35-118).
+//
+// A thread computes R output rows x PX neighbouring outputs of one plane. Each input row behind them is one unaligned run of
+// the plane's memory (10 to 22 bytes of elements, loaded as whole dwords): a run that leaves its row reads the neighbouring
+// row's elements, which are masked - by the column pattern, the same for all of a thread's rows - so that no load depends on
+// the position. Only runs that would leave the tensor, at its first and last elements, are read from inside it and shifted. All
+// of a thread's loads are issued before the first use. Column and row groups at a plane's end are moved back inside it: they
+// compute some outputs twice, and every store but those of planes smaller than a group is a whole vector.
+// A plane's channel is uniform where its threads fill whole wavefronts (weights then are scalar operands); small planes share
+// wavefronts and keep their weights in vector registers.
+//
+// What bounds it: vector instructions and bytes, about even. One thread per output took (us, back to back; here) 125 (15.5: 49 MB at 3.2
+// TB/s) for float16 3x3 on 92 channels of 105 x 160, batch 8; 186 (34: 131 MB at 3.9 TB/s) for float32 3x3 on 400 of 39 x 39, batch 27;
+// 166 (27.8) for float16 5x5 at stride 2 on 352 of 46 x 46, batch 42. Planes in LDS with a byte load a tap took 34 (4.4) for int8 5x5 on
+// 48 of 114 x 114, batch 2, and 43 (15.5) for uint8 on 208 of 38 x 38, batch 26.
+#include <algorithm>
+#include <cmath>
+#include <cstdlib>
+#include <cstring>
+
+#include "variants.h"
+
+namespace tvx {
+namespace {
+
+struct DwrArgs {
+  const uint8_t* x;
+  uint8_t* y;
+  const float* wf;        // floating point: [channel][K * K, padded to whole fours], then the bias at place K * K
+  const int* wi;          // quantized: [channel][K rows of two dwords, folded bias, pad]
+  const tvx_v4i* rq;
+  int C, H, W, OH, OW, pad_t, pad_l;
+  int ncg, tpp, bpp;      // column groups of a row, threads and (whole wavefronts per plane) workgroups of a plane
+  int planes;
+  uint32_t m_tpp, m_ncg, m_c;
+  int total;              // elements of the input
+  int act;
+  int fill, xor_in, zws, lo, hi, narrow, out_xor, pre_ties;
+};
+
+__device__ __forceinline__ int DivM(int u, uint32_t m) { return m ? static_cast<int>(__umulhi(static_cast<uint32_t>(u), m)) : u; }
+
+// DT: TVX_I8 (uint8 too), TVX_F16 or TVX_F32
+template <int DT, int K, int S> struct Tile {
+  static constexpr int E = DT == TVX_F32 ? 4 : DT == TVX_F16 ? 2 : 1;
+  static constexpr int PX = S == 1 && DT != TVX_F32 ? 8 : 4;
+  static constexpr int L = (PX - 1) * S + K;          // elements of a row behind PX outputs
+  static constexpr int LD = (L * E + 3) / 4;          // ... in dwords
+  static constexpr int LE = LD * 4 / E;               // ... and the elements these load
+  static constexpr int WS = DT == TVX_I8 ? 2 * K + 2 : (K * K + 4) / 4 * 4;  // words of a channel's table: weights, bias
+};
+
+// Place of a thread: its plane, channel and first output.
+struct Place { int plane, c, oy, ox; bool live; };
+template <bool UNIFORM, int R, int PX>
+__device__ __forceinline__ Place Find(const DwrArgs& a) {
+  Place p;
+  int t;
+  if (UNIFORM) {  // a grid of (channel, part of the plane, image)
+    p.c = blockIdx.x;
+    p.plane = static_cast<int>(blockIdx.z) * a.C + p.c;
+    t = static_cast<int>(blockIdx.y * blockDim.x + threadIdx.x);
+    p.live = t < a.tpp;
+    t = min(t, a.tpp - 1);
+  } else {
+    const uint32_t first = blockIdx.x * blockDim.x;
+    const int plane0 = __builtin_amdgcn_readfirstlane(static_cast<int>(first / static_cast<uint32_t>(a.tpp)));
+    const int c0 = __builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<uint32_t>(plane0) % static_cast<uint32_t>(a.C)));
+    const int local = static_cast<int>(first - static_cast<uint32_t>(plane0) * a.tpp + threadIdx.x);
+    const int more = DivM(local, a.m_tpp);
+    t = local - more * a.tpp;
+    p.live = plane0 + more < a.planes;
+    p.plane = min(plane0 + more, a.planes - 1);
+    const int c = c0 + p.plane - plane0;
+    p.c = c - DivM(c, a.m_c) * a.C;
+  }
+  const int rg = DivM(t, a.m_ncg), cg = t - rg * a.ncg;
+  p.oy = min(rg * R, max(a.OH - R, 0));
+  p.ox = min(cg * PX, max(a.OW - PX, 0));
+  return p;
+}
+
+// The rows behind a thread's outputs; what lies outside the image is `fill`.
+template <int DT, int K, int S, int R>
+struct Rows {
+  using T = Tile<DT, K, S>;
+  static constexpr int NR = (R - 1) * S + K;
+  uint32_t d[NR][T::LD];
+
+  // the row's elements by n places up (towards higher columns) or down; where n is a row or more, nothing of it counts
+  template <bool UP, int STEP = 1>
+  static __device__ __forceinline__ void ShiftDwords(uint32_t (&v)[T::LD], int dwords) {
+    const uint32_t on = dwords & STEP ? ~0u : 0u;
+#pragma unroll
+    for (int k = 0; k < T::LD; ++k) {
+      const int j = UP ? T::LD - 1 - k : k;
+      const uint32_t from = UP ? (j >= STEP ? v[j >= STEP ? j - STEP : 0] : 0u) : (j + STEP < T::LD ? v[j + STEP < T::LD ? j + STEP : 0] : 0u);
+      v[j] = (from & on) | (v[j] & ~on);
+    }
+    if constexpr (2 * STEP <= T::LD) ShiftDwords<UP, 2 * STEP>(v, dwords);
+  }
+  template <bool UP>
+  static __device__ __forceinline__ void Shift(uint32_t (&v)[T::LD], int n) {
+    const int bytes = min(n, T::LE) * T::E;
+    ShiftDwords<UP>(v, bytes / 4);
+    if constexpr (T::E < 4) {
+      const uint32_t rest = 8 * (bytes & 3);
+#pragma unroll
+      for (int k = 0; k < T::LD; ++k) {
+        const int j = UP ? T::LD - 1 - k : k;
+        const uint64_t lo = UP ? (j > 0 ? v[j > 0 ? j - 1 : 0] : 0u) : v[j], hi = UP ? v[j] : (j + 1 < T::LD ? v[j + 1 < T::LD ? j + 1 : 0] : 0u);
+        v[j] = static_cast<uint32_t>((hi << 32 | lo) >> (UP ? 32 - rest : rest));
+      }
+    }
+  }
+
+  __device__ __forceinline__ void Load(const DwrArgs& a, const Place& p) {
+    const int ix = p.ox * S - a.pad_l, iy = p.oy * S - a.pad_t;
+    const int first = p.plane * (a.H * a.W);
+    int moved[NR];  // elements by which a run was moved to lie inside the tensor
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int at = first + min(max(iy + i, 0), a.H - 1) * a.W + ix, in = min(max(at, 0), a.total - T::LE);
+      __builtin_memcpy(d[i], a.x + static_cast<size_t>(static_cast<uint32_t>(in)) * T::E, T::LD * 4);
+      moved[i] = in - at;
+    }
+    // the tensor's first and last elements: back to their places (what is shifted in lies outside the image)
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+      if (__ballot(moved[i] != 0)) {
+        Shift<true>(d[i], max(moved[i], 0));
+        Shift<false>(d[i], max(-moved[i], 0));
+      }
+    if (DT == TVX_I8) {
+#pragma unroll
+      for (int i = 0; i < NR; ++i)
+#pragma unroll
+        for (int j = 0; j < T::LD; ++j) d[i][j] ^= static_cast<uint32_t>(a.xor_in);
+    }
+    const uint32_t fill = DT == TVX_I8 ? static_cast<uint32_t>(a.fill) : 0u;
+    // columns: the same pattern in every row; a wavefront without an edge skips it
+    if (__ballot(ix < 0 || ix + T::L > a.W)) {
+#pragma unroll
+      for (int j = 0; j < T::LD; ++j) {
+        uint32_t keep = 0;
+#pragma unroll
+        for (int e = 0; e < 4 / T::E; ++e)
+          if (static_cast<unsigned>(ix + j * (4 / T::E) + e) < static_cast<unsigned>(a.W)) keep |= (T::E == 4 ? ~0u : (1u << (8 * T::E & 31)) - 1u) << (8 * T::E * e);
+#pragma unroll
+        for (int i = 0; i < NR; ++i) d[i][j] = (d[i][j] & keep) | (fill & ~keep);
+      }
+    }
+    if (__ballot(iy < 0 || iy + NR > a.H)) {
+#pragma unroll
+      for (int i = 0; i < NR; ++i) {
+        const bool in = static_cast<unsigned>(iy + i) < static_cast<unsigned>(a.H);
+#pragma unroll
+        for (int j = 0; j < T::LD; ++j) d[i][j] = in ? d[i][j] : fill;
+      }
+    }
+  }
+};
+
+// PX results of a row; where the row has fewer than that, but four: its first four and its last four.
+template <int E, int N>
+__device__ __forceinline__ void StoreRow(uint8_t* to, const uint32_t (&out)[N], int OW) {
+  constexpr int PX = N * 4 / E;
+  if (OW >= PX) {  // (uniform)
+    __builtin_memcpy(to, out, N * 4);
+  } else if (PX == 8 && OW >= 4) {
+    const int back = (OW - 4) * E;  // bytes in front of the last four
+    uint32_t last[E];
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      const uint32_t a = back < 4 ? out[j] : out[j + 1], b = back < 4 ? out[j + 1] : j + 2 < N ? out[j + 2 < N ? j + 2 : 0] : 0u;
+      last[j] = __builtin_amdgcn_alignbyte(b, a, static_cast<uint32_t>(back & 3));
+    }
+    __builtin_memcpy(to, out, 4 * E);
+    __builtin_memcpy(to + back, last, 4 * E);
+  } else {
+#pragma unroll
+    for (int q = 0; q < PX; ++q)
+      if (q < OW) {
+        if constexpr (E == 1) to[q] = static_cast<uint8_t>(out[q / 4] >> (8 * (q & 3)));
+        else if constexpr (E == 2) reinterpret_cast<uint16_t*>(to)[q] = static_cast<uint16_t>(out[q / 2] >> (16 * (q & 1)));
+        else reinterpret_cast<uint32_t*>(to)[q] = out[q];
+      }
+  }
+}
+
+template <int DT, int K, int S, int R, bool UNIFORM>
+__global__ void __launch_bounds__(256) DwRegFloatKernel(DwrArgs a) {
+  using T = Tile<DT, K, S>;
+  constexpr int PX = T::PX;
+  const Place p = Find<UNIFORM, R, PX>(a);
+  const float* w = a.wf + p.c * T::WS;
+  Rows<DT, K, S, R> rows;
+  rows.Load(a, p);
+  float acc[R][PX];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int q = 0; q < PX; ++q) acc[r][q] = 0.f;
+#pragma unroll
+  for (int i = 0; i < Rows<DT, K, S, R>::NR; ++i) {
+    float v[T::L];
+#pragma unroll
+    for (int j = 0; j < T::L; ++j) {
+      if constexpr (DT == TVX_F16) v[j] = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(rows.d[i][j / 2] >> (16 * (j & 1)))));
+      else v[j] = __builtin_bit_cast(float, rows.d[i][j]);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int ky = i - r * S;
+      if (ky < 0 || ky >= K) continue;
+#pragma unroll
+      for (int kx = 0; kx < K; ++kx)
+#pragma unroll
+        for (int q = 0; q < PX; ++q) acc[r][q] = __builtin_fmaf(v[q * S + kx], w[ky * K + kx], acc[r][q]);
+    }
+  }
+  if (!p.live) return;
+  const float bias = w[K * K];
+  const size_t to0 = static_cast<size_t>(p.plane) * (a.OH * a.OW) + p.oy * a.OW + p.ox;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (p.oy + r >= a.OH) continue;
+    uint32_t out[PX * T::E / 4];
+#pragma unroll
+    for (int q = 0; q < PX; ++q) {
+      float v = acc[r][q] + bias;
+      if (a.act != TVX_ACT_NONE) v = v < 0.f ? 0.f : v;
+      if (a.act == TVX_ACT_RELU6) v = v > 6.f ? 6.f : v;
+      if constexpr (DT == TVX_F16) {
+        const uint32_t h = __builtin_bit_cast(uint16_t, static_cast<_Float16>(v));
+        out[q / 2] = q & 1 ? out[q / 2] | h << 16 : h;
+      } else {
+        out[q] = __builtin_bit_cast(uint32_t, v);
+      }
+    }
+    StoreRow<T::E>(a.y + (to0 + static_cast<size_t>(r) * a.OW) * T::E, out, a.OW);
+  }
+}
+
+// bytes o .. o + 3 of a row; what lies behind its last dword meets zero weights
+template <int N>
+__device__ __forceinline__ int Cut(const uint32_t (&d)[N], int o) {
+  const uint32_t lo = d[o / 4], hi = o / 4 + 1 < N ? d[o / 4 + 1] : 0u;
+  return static_cast<int>(o % 4 ? __builtin_amdgcn_alignbyte(hi, lo, o % 4) : lo);
+}
+
+// The first product of an accumulator takes the bias as its third operand (the builtin's instruction adds to a copy of it).
+template <bool UNIFORM>
+__device__ __forceinline__ int FirstDot(int x, int w, int bias) {
+  if constexpr (!UNIFORM) return Dot4Add(x, w, bias);
+  int r;
+  asm("v_dot4_i32_i8 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(w), "v"(bias));
+  return r;
+}
+
+// Accumulators start from the folded bias. A row's window is two dot products (weights 0 .. 3, and the fifth alone); under a weight
+// zero point (SUMS) the rows' window sums are made once per input row and added to the output rows they belong to.
+template <int K, int S, int R, bool UNIFORM, bool SUMS>
+__global__ void __launch_bounds__(256) DwRegI8Kernel(DwrArgs a) {
+  using T = Tile<TVX_I8, K, S>;
+  constexpr int PX = T::PX;
+  const Place p = Find<UNIFORM, R, PX>(a);
+  const int* w = a.wi + p.c * T::WS;
+  const tvx_v4i rq = a.rq[p.c];
+  Rows<TVX_I8, K, S, R> rows;
+  rows.Load(a, p);
+  const int bias = w[2 * K];
+  int acc[R][PX], sum[R][PX];
+#pragma unroll
+  for (int i = 0; i < Rows<TVX_I8, K, S, R>::NR; ++i) {
+#pragma unroll
+    for (int q = 0; q < PX; ++q) {
+      const int w0 = Cut(rows.d[i], q * S), w1 = K > 4 ? Cut(rows.d[i], q * S + 4) : 0;
+      int box = 0;
+      if (SUMS) {
+        box = __builtin_amdgcn_sdot4(w0, K > 3 ? 0x01010101 : 0x00010101, 0, false);
+        if (K > 4) box = __builtin_amdgcn_sdot4(w1, 0x00000001, box, false);
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int ky = i - r * S;
+        if (ky < 0 || ky >= K) continue;
+        acc[r][q] = ky == 0 ? FirstDot<UNIFORM>(w0, w[0], bias) : __builtin_amdgcn_sdot4(w0, w[2 * ky], acc[r][q], false);
+        if (K > 4) acc[r][q] = __builtin_amdgcn_sdot4(w1, w[2 * ky + 1], acc[r][q], false);
+        if (SUMS) sum[r][q] = ky == 0 ? box : sum[r][q] + box;
+      }
+    }
+  }
+  if (!p.live) return;
+  const int sh = rq[1] & 31;
+  const int64_t round = RoundHigh(rq[2]);
+  const size_t to0 = static_cast<size_t>(p.plane) * (a.OH * a.OW) + p.oy * a.OW + p.ox;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (p.oy + r >= a.OH) continue;
+    uint32_t out[PX / 4];
+#pragma unroll
+    for (int h = 0; h < PX / 4; ++h) {
+      int v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = SUMS ? __mul24(-a.zws, sum[r][4 * h + e]) + acc[r][4 * h + e] : acc[r][4 * h + e];
+      if (a.pre_ties) {  // (uniform)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] <<= a.pre_ties >> 1;
+        if (a.pre_ties & 1) LowerOddTies(v, rq);
+      }
+      out[h] = (a.narrow ? RequantSaturate4<true>(v, rq[0], sh, round, a.lo << sh, ((a.hi + 1) << sh) - 1) : RequantSaturate4<false>(v, rq[0], sh, round, 0, 0)) ^ static_cast<uint32_t>(a.out_xor);
+    }
+    StoreRow<1>(a.y + to0 + static_cast<size_t>(r) * a.OW, out, a.OW);
+  }
+}
+
+typedef void (*DwRegFn)(DwrArgs);
+template <int DT, int K, int S, int R>
+DwRegFn Pick(bool uniform, bool sums) {
+  if constexpr (DT == TVX_I8) {
+    if (sums) return uniform ? DwRegI8Kernel<K, S, R, true, true> : DwRegI8Kernel<K, S, R, false, true>;
+    return uniform ? DwRegI8Kernel<K, S, R, true, false> : DwRegI8Kernel<K, S, R, false, false>;
+  } else {
+    return uniform ? DwRegFloatKernel<DT, K, S, R, true> : DwRegFloatKernel<DT, K, S, R, false>;
+  }
+}
+template <int DT>
+DwRegFn PickKernel(int k, int s, int r, bool uniform, bool sums) {
+  if (k == 3) {
+    if (s == 1) return r == 4 ? Pick<DT, 3, 1, 4>(uniform, sums) : Pick<DT, 3, 1, 2>(uniform, sums);
+    return r == 4 ? Pick<DT, 3, 2, 4>(uniform, sums) : Pick<DT, 3, 2, 2>(uniform, sums);
+  }
+  if (s == 1) return r == 4 ? Pick<DT, 5, 1, 4>(uniform, sums) : Pick<DT, 5, 1, 2>(uniform, sums);
+  return r == 4 ? Pick<DT, 5, 2, 4>(uniform, sums) : Pick<DT, 5, 2, 2>(uniform, sums);
+}
+
+uint32_t Magic(int d) { return d <= 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + d - 1) / d); }
+
+struct Plan {
+  DwrArgs a;
+  DwRegFn fn;
+  dim3 grid;
+  unsigned threads, align;  // align: address bits of the tensors that must not be set (as the stencils for these layers have it)
+};
+
+int DwRegRun(tvx_op* op, const void* in0, const void*, void* out, hipStream_t st) {
+  const Plan* p = reinterpret_cast<const Plan*>(op->host_blob.data());
+  if ((reinterpret_cast<uintptr_t>(in0) | reinterpret_cast<uintptr_t>(out)) & p->align)
+    return SetError(TVX_E_INVALID, "%s: tensors must be %u-byte aligned", op->kernel_name, p->align + 1);
+  DwrArgs a = p->a;
+  a.x = static_cast<const uint8_t*>(in0);
+  a.y = static_cast<uint8_t*>(out);
+  hipLaunchKernelGGL(p->fn, p->grid, dim3(p->threads), 0, st, a);
+  TVX_HIP_CHECK(hipGetLastError());
+  return TVX_OK;
+}
+
+// dwconv3x3_i8's layers: rows of whole dwords, shared between lanes
+bool WholeDwordRows(const tvx_conv2d_desc* d) { return d->in_w % 4 == 0 && d->out_w % 4 == 0 && d->pad_left <= 1 && d->out_w <= 256; }
+
+// Which quantized 3x3 layers come here. The stencil for rows of whole dwords gives a row a power of two of lanes: where its outputs fill
+// less than 0.6 of them (132 columns: 33 of 64) it takes 41.8 us against 33.0 (80 channels, 117 x 132, batch 36), else it is ahead (52
+// columns: 12.6 against 14.3). The one that stages planes in LDS: at stride 2 it is never ahead by more than the runs differ (57 x 57, 240
+// channels, batch 44: 26.1 against 13.7 us here), at stride 1 in launches of a few workgroups (25 channels of 14 x 14, batch 2: 3.1 against 3.4;
+// 16 of 69 x 69, batch 2: 4.6 against 3.2; 64 of 93 x 93, batch 43: 29.8 against 21.2).
+bool BetterAt3x3(const tvx_conv2d_desc* d) {
+  if (WholeDwordRows(d)) {
+    if (d->stride_w == 1 && d->in_w % 8 == 0 && d->out_w % 8 == 0) return false;  // (eight columns a lane there)
+    const int patches = d->out_w / 4;
+    int lanes = 1;
+    while (lanes < patches) lanes *= 2;
+    return patches * 10 < lanes * 6;
+  }
+  return d->stride_w == 2 || static_cast<uint64_t>(d->batch) * d->in_c * d->out_h * d->out_w >= 32768;
+}
+
+float HalfToFloat(uint16_t h) {
+  _Float16 v;
+  std::memcpy(&v, &h, 2);
+  return static_cast<float>(v);
+}
+
+}  // namespace
+
+// Claims depthwise 3x3 and 5x5 convolutions of stride 1 or 2 with constant weights: float16, float32, and int8 / uint8.
+int DwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const void* bias_host) {
+  if (!w_host || op->kind != OP_CONV2D || d->multiplier != 1 || op->fused_add || op->out_blocked) return TVX_E_UNSUPPORTED;
+  const int K = d->k_w, S = d->stride_w;
+  if (d->k_h != d->k_w || (K != 3 && K != 5) || d->stride_h != d->stride_w || (S != 1 && S != 2) || d->dilation_w != 1 || d->dilation_h != 1)
+    return TVX_E_UNSUPPORTED;
+  const bool q = op->quantized;
+  if (!q && (d->in_dtype != d->w_dtype || d->in_dtype != d->out_dtype || (d->in_dtype != TVX_F16 && d->in_dtype != TVX_F32))) return TVX_E_UNSUPPORTED;
+  const int dt = q ? TVX_I8 : d->in_dtype;
+  const char* lever = getenv("TVX_DWCONV_REG");  // test lever: 0 declines, 1 claims quantized 3x3 windows too
+  if (lever && atoi(lever) == 0) return TVX_E_UNSUPPORTED;
+  if (q && K == 3 && !lever && !BetterAt3x3(d)) return TVX_E_UNSUPPORTED;
+
+  DwrArgs a{};
+  a.C = d->in_c; a.H = d->in_h; a.W = d->in_w; a.OH = d->out_h; a.OW = d->out_w;
+  a.pad_t = d->pad_top; a.pad_l = d->pad_left;
+  const int64_t planes = static_cast<int64_t>(d->batch) * d->in_c;
+  const int64_t in = planes * d->in_h * d->in_w, out = planes * d->out_h * d->out_w;
+  if (in >= (1 << 30) || out >= (1 << 30) || d->in_c > 60000 || d->pad_left > 1024 || d->pad_top > 1024) return TVX_E_UNSUPPORTED;
+  // (a window's first column and row lie within the padded input: no place below overflows)
+  a.planes = static_cast<int>(planes);
+  a.total = static_cast<int>(in);
+  a.act = d->activation;
+
+  // Rows of a thread: four, so that a row is loaded 1.5 times (3x3) or twice (5x5, stride 1) instead of twice or three times - two
+  // where four leave the chip short of wavefronts.
+  const int px = S == 1 && dt != TVX_F32 ? 8 : 4;
+  a.ncg = (a.OW + px - 1) / px;
+  int R = 4;
+  auto threads = [&](int r) { return planes * a.ncg * ((a.OH + r - 1) / r); };
+  if (threads(4) < 256 * 4 * 64) R = 2;
+  if (const char* f = getenv("TVX_DWCONV_REG_ROWS")) R = atoi(f) == 2 ? 2 : 4;  // test lever
+  a.tpp = a.ncg * ((a.OH + R - 1) / R);
+  // whole wavefronts per plane where at most a quarter of their lanes is idle
+  const int waves = (a.tpp + 63) / 64;
+  const bool uniform = a.tpp * 4 >= waves * 64 * 3;
+  unsigned block = 256;
+  if (uniform) {
+    a.bpp = (waves + 3) / 4;
+    block = static_cast<unsigned>((waves + a.bpp - 1) / a.bpp) * 64;
+  }
+  const int64_t grid = uniform ? planes * a.bpp : (planes * a.tpp + 255) / 256;
+  if (uniform && (d->batch > 65535 || a.bpp > 65535)) return TVX_E_UNSUPPORTED;
+  if (grid * block >= (int64_t{1} << 31) || in < 12) return TVX_E_UNSUPPORTED;  // (a run of at most twelve elements fits the tensor)
+  if (static_cast<uint64_t>(a.tpp + 256) * std::max(a.tpp, a.ncg) >= (1ull << 32)) return TVX_E_UNSUPPORTED;  // reciprocals are exact below
+  a.m_tpp = Magic(a.tpp);
+  a.m_ncg = Magic(a.ncg);
+  a.m_c = Magic(a.C);
+
+  int s = TVX_OK;
+  if (q) {
+    const bool w_u8 = d->w_dtype == TVX_U8, x_u8 = d->in_dtype == TVX_U8;
+    const int zxs = d->in_zp - (x_u8 ? 128 : 0), zws = op->w_zp - (w_u8 ? 128 : 0);
+    const int words = 2 * K + 2;
+    std::vector<int32_t> tab(static_cast<size_t>(a.C) * words, 0);
+    const uint8_t* src = static_cast<const uint8_t*>(w_host);
+    const int32_t* bi = static_cast<const int32_t*>(bias_host);
+    for (int c = 0; c < a.C; ++c) {
+      int64_t sw = 0;
+      int32_t* t = &tab[static_cast<size_t>(c) * words];
+      for (int i = 0; i < K * K; ++i) {
+        const uint8_t v = src[static_cast<size_t>(c) * K * K + i] ^ (w_u8 ? 0x80 : 0);
+        sw += static_cast<int8_t>(v);
+        const int ky = i / K, kx = i % K;
+        t[2 * ky + kx / 4] |= static_cast<int32_t>(static_cast<uint32_t>(v) << (8 * (kx & 3)));
+      }
+      const int64_t v = (bi ? bi[c] : 0) - static_cast<int64_t>(zxs) * sw + static_cast<int64_t>(K) * K * zxs * zws;
+      t[2 * K] = static_cast<int32_t>(static_cast<uint32_t>(v));
+    }
+    const int out_flip = d->out_dtype == TVX_U8 ? 128 : 0;
+    std::vector<int32_t> rqt;
+    int up;
+    bool ties;
+    if (!BuildTieRecords(op->h_mult, op->h_shift, a.C, a.C, d->out_zp - out_flip, AccumulatorBound(K * K, bias_host, a.C), &rqt, &up, &ties)) return TVX_E_UNSUPPORTED;
+    a.pre_ties = up * 2 + ties;
+    a.fill = static_cast<int>(static_cast<uint32_t>(zxs & 0xff) * 0x01010101u);
+    a.xor_in = x_u8 ? static_cast<int>(0x80808080u) : 0;
+    a.zws = zws;
+    a.lo = op->act_lo - out_flip; a.hi = op->act_hi - out_flip; a.narrow = a.lo > -128 || a.hi < 127;
+    a.out_xor = out_flip ? static_cast<int>(0x80808080u) : 0;
+    s = op->packed.Upload(tab.data(), tab.size() * 4);
+    if (s == TVX_OK) s = op->aux2.Upload(rqt.data(), rqt.size() * 4);
+    a.wi = op->packed.as<int>();
+    a.rq = op->aux2.as<tvx_v4i>();
+  } else {
+    const int words = (K * K + 4) / 4 * 4;
+    std::vector<float> tab(static_cast<size_t>(a.C) * words, 0.f);
+    for (int c = 0; c < a.C; ++c) {
+      float* t = &tab[static_cast<size_t>(c) * words];
+      for (int i = 0; i < K * K; ++i) {
+        const size_t at = static_cast<size_t>(c) * K * K + i;
+        t[i] = dt == TVX_F16 ? HalfToFloat(static_cast<const uint16_t*>(w_host)[at]) : static_cast<const float*>(w_host)[at];
+        if (!std::isfinite(t[i])) return TVX_E_UNSUPPORTED;  // (padding multiplies its zeros by the weights)
+      }
+      t[K * K] = bias_host ? static_cast<const float*>(bias_host)[c] : 0.f;
+    }
+    s = op->packed.Upload(tab.data(), tab.size() * 4);
+    a.wf = op->packed.as<float>();
+  }
+  if (s != TVX_OK) return s;
+  Plan plan{a, nullptr, dim3(1), block, !q || (K == 3 && WholeDwordRows(d)) ? 0u : 15u};
+  plan.fn = dt == TVX_I8 ? PickKernel<TVX_I8>(K, S, R, uniform, a.zws != 0) : dt == TVX_F16 ? PickKernel<TVX_F16>(K, S, R, uniform, false) : PickKernel<TVX_F32>(K, S, R, uniform, false);
+  plan.grid = uniform ? dim3(a.C, a.bpp, d->batch) : dim3(static_cast<unsigned>(grid));
+  op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
+  op->run = DwRegRun;
+  op->kernel_name = dt == TVX_I8 ? "dwconv_planes_i8" : dt == TVX_F16 ? "dwconv_reg_f16" : "dwconv_reg_f32";
+  return TVX_OK;
+}
+
+}  // namespace tvx

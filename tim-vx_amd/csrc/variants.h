@@ -54,6 +54,8 @@ int LayoutSetup(tvx_op*, uint32_t w, uint32_t h, uint32_t c, uint32_t n, int to_
 
 // depthwise, any kernel / width, planes staged through LDS (dwconv_planes_i8.hip)
 int DwPlanesSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
+// depthwise 3x3 / 5x5 as a register stencil on planes of any width: float16, float32, int8 (dwconv_reg.hip)
+int DwRegSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 // shared by the two depthwise 3x3 stencils (defined in dwconv3x3_i8.hip)
 bool PackDepthwise3x3(int C, const void* w_host, bool w_u8, const void* bias_host, int zxs, int zws,
                       bool all_or_none, std::vector<int32_t>* wpk, std::vector<int32_t>* biasf);
