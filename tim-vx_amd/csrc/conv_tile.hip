@@ -21,9 +21,11 @@
 //
 // What bounds it: at the sizes convolutional networks have, a launch is a chain of one memory round trip, the LDS
 // transposition (about 70 vector instructions per 64 staged bytes for int8, none for float32) and the steps themselves, and no unit
-// is busy for long: int8 3x3 256 -> 256 on 14 x 14, batch 32 (13.3 us under the tracer): vector units 26 %, LDS 22 % and a third of that
-// in bank conflicts, matrix cores 16 %, wavefronts waiting 45 % of their cycles; float16 5x5 96 -> 256 on 27 x 27, batch 16 (31.8 us):
-// 40, 51 (half of it conflicts), 28 and 38 %. The tile is chosen on the host so that the chip is filled first and the halo staged per output pixel is small second.
+// is busy for long: int8 3x3 256 -> 256 on 14 x 14, batch 32: first addresses .6 us, loads 3, transposition and barrier 1.4, steps 4.2,
+// exchange, requantization and stores 3. What a phase needs of the arguments is read when it begins (LateArgs), its first loads' addresses
+// come first, and a chunk's odd last step is looked for behind the main loop: int8 80 -> 9 channels, 3x3 on 21 x 21, batch 15, 8.1 -> 6.4 us;
+// 288 -> 40, 3x3 at stride 2 on 98 x 65, batch 22, 54 -> 43; float16 3 -> 48, 7x7 on 142 x 142, batch 16, 33 -> 28. The tile is chosen on the
+// host so that the chip is filled first and the halo staged per output pixel is small second.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -42,45 +44,55 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 constexpr int kI8 = 0, kF16 = 1, kF32 = 2;  // element kinds (uint8 runs as int8 with its sign bit flipped)
 
+// In the order of their use: what comes before a launch's first loads is fetched together (LateArgs).
 struct TileArgs {
   const uint8_t* x;
-  uint8_t* y;
+  int total, per_xcd;
+  int oc_wgs, wgs_per_group, loop;  // workgroups that the channel blocks take, of all groups and of one; channel blocks that a workgroup takes one after the other
+  int tiles_x, tiles_y;
+  uint32_t m_ocb, m_tpg, m_tx, m_ty;  // reciprocals: u / d = mulhi(u, m), exact for the ranges used
+  int TW, TH, G;           // tile: columns, rows, images
+  int sh, sw, pad_t, pad_l;
+  int icg;                 // input channels of a group
+  int gpc;                 // granules of a pixel per chunk
+  int items;               // work items of a chunk
+  int gl, cells, ncg, IH;  // granules neighbouring lanes take (a divisor of gpc); column groups of all staged rows, of a row; staged rows per image
+  uint32_t m_gl, m_cells, m_ncg, m_ih;
+  int row_step, H, W, batch;  // row_step: input rows between staged rows
+  int at_max;              // last place of a plane where a work item's pixels can be read
+  uint32_t plane_bytes, image_bytes;
+  int IW, pitch;           // staged columns; LDS bytes of a staged pixel: an odd number of granules (bank spread)
+  uint32_t xor_mask;
+  // ---- under the first loads
   const v4i* wpk;          // [group][32-channel tile][chunk][step][64 lanes]: sixteen bytes of reduction per lane
   const int* tab;          // [half][steps_pad]: LDS byte offset of the granule a lane of that half multiplies at a step
+  int steps, steps_pad, odd;  // reduction steps of a chunk; the last step's upper half is empty
+  int chunks, tiles_per_group;
+  int row_stride, NQ, npx;  // staged rows between output rows; pixels of the tile; staged pixels
+  uint32_t m_iw, m_tw, m_thtw;
+  uint32_t pad_full, pad_last[4];  // a padding granule: full, and the channels' last one
+  int last_granule;        // global index of the channels' last granule
+  int off_tab, off_sum, off_zt, off_out;  // LDS carve-up behind the staged window; the results (over the window where it is used once)
+  int zws;                 // weight zero point in the signed domain (0: no window sums)
+  // ---- behind the multiplications
+  uint8_t* y;
   const int32_t* biasf;    // quantized: bias with the zero-point terms folded in, per padded output channel
   const float* biasfl;     // floating point: the bias, or null
   const tvx_v4i* rq;
-  int C, H, W, OC, OH, OW, batch;
-  int sh, sw, pad_t, pad_l;
-  int icg, ocg;            // channels per group
-  int TW, TH, G, NQ;       // tile: columns, rows, images; its pixels
-  int IW, IH;              // staged columns, and rows per image
-  int row_step, row_stride;  // input rows between staged rows; staged rows between output rows
-  int pitch;               // LDS bytes of a staged pixel: an odd number of granules (bank spread)
-  int gpc, chunks;         // granules of a pixel per chunk
-  int steps, steps_pad, odd;  // reduction steps of a chunk; the last step's upper half is empty
+  int OC, OH, OW, ocg;     // ocg: output channels of a group
   int taps_w, taps_h, dil_col, dil_row;  // for the box sum: LDS pixels between taps
-  int ncg, cells, gl;      // column groups of a staged row, of all rows; granules neighbouring lanes take (a divisor of gpc)
-  int tiles_x, tiles_y, tiles_per_group;
-  int loop, wgs_per_group, oc_wgs;  // channel blocks that a workgroup takes one after the other; workgroups a group's blocks take; of all groups
-  int total, per_xcd;
-  int npx, items;          // staged pixels and work items of a chunk
-  uint32_t plane_bytes, image_bytes;
-  int at_max;              // last place of a plane where a work item's pixels can be read
-  int off_tab, off_sum, off_zt, off_out;  // LDS carve-up behind the staged window; the results (over the window where it is used once)
   int runs, run_px, run_out, out_pitch;  // copy-out: runs of consecutive outputs of a channel, their pixels and distance; LDS bytes of a channel
   uint32_t m_run4;         // reciprocal of a run's groups of four pixels
   int runs_shift;          // log2 of the threads that a channel's runs take
-  uint32_t m_gl, m_cells, m_ncg, m_ih, m_iw, m_tw, m_thtw, m_ocb, m_tpg, m_tx, m_ty;  // reciprocals: u / d = mulhi(u, m), exact for the ranges used
-  uint32_t xor_mask;
-  uint32_t pad_full, pad_last[4];  // a padding granule: full, and the channels' last one
-  int last_granule;        // global index of the channels' last granule
-  int zws;                 // weight zero point in the signed domain (0: no window sums)
   int pre_ties;            // accumulators' left shift (BuildTieRecords) * 2 + whether ties are possible
   int lo, hi, narrow, out_xor, act;  // quantized: clamp in the signed domain, whether it is narrower than a byte; 0x80808080 for uint8 results
 };
 
-__device__ __forceinline__ int DivM(int u, uint32_t m) { return m ? static_cast<int>(__umulhi(static_cast<uint32_t>(u), m)) : u; }
+// (a sum and not a choice of two: that became a branch per division)
+__device__ __forceinline__ int DivM(int u, uint32_t m) {
+  const uint32_t one = m ? 0u : ~0u;
+  return static_cast<int>(__umulhi(static_cast<uint32_t>(u), m) + (static_cast<uint32_t>(u) & one));
+}
 
 template <int DT> struct Kind;
 template <> struct Kind<kI8> { using acc = v16i; using elem = int; static constexpr int E = 1; };
@@ -113,8 +125,27 @@ template <int DT> struct Item {
   __device__ __forceinline__ void Load(const uint8_t* base, uint32_t at, uint32_t plane_bytes, int valid) {
 #pragma unroll
     for (int c = 0; c < N; ++c) {
-      if (FULL) __builtin_memcpy(&d[c * D], base + static_cast<size_t>(c) * plane_bytes + at, 4 * D);  // (scalar base, one lane offset)
-      else __builtin_memcpy(&d[c * D], base + (at + static_cast<uint32_t>(min(c, valid - 1)) * plane_bytes), 4 * D);
+      if (FULL) {
+        const uint8_t* plane = base + static_cast<size_t>(c) * plane_bytes;
+        asm("" : "+s"(plane));  // (a scalar base and one lane offset for all planes, not sixteen lane addresses)
+        __builtin_memcpy(&d[c * D], plane + at, 4 * D);
+      } else {
+        __builtin_memcpy(&d[c * D], base + (at + static_cast<uint32_t>(min(c, valid - 1)) * plane_bytes), 4 * D);
+      }
+    }
+  }
+  // a granule that holds all the channels there are (uniform): the planes behind them are not loaded but zero
+  __device__ __forceinline__ void LoadFew(const uint8_t* base, uint32_t at, uint32_t plane_bytes, int valid) {
+#pragma unroll
+    for (int c = 0; c < N; ++c) {
+      if (c < valid) {
+        const uint8_t* plane = base + static_cast<size_t>(c) * plane_bytes;
+        asm("" : "+s"(plane));
+        __builtin_memcpy(&d[c * D], plane + at, 4 * D);
+      } else {
+#pragma unroll
+        for (int i = 0; i < D; ++i) d[c * D + i] = 0;
+      }
     }
   }
   // the granules of pixels 4 g .. 4 g + 3
@@ -162,8 +193,6 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
   // consecutive workgroups of an XCD: the channel blocks of a tile, then the next tile
   const int id = static_cast<int>(blockIdx.x & 7) * a.per_xcd + static_cast<int>(blockIdx.x >> 3);
   if (id >= a.total) return;
-  const int tab_n = 2 * a.steps_pad;
-  const int tab_first = a.tab[min(tid, tab_n - 1)];  // (waited for behind the window's loads)
   const int tile = DivM(id, a.m_ocb), ocb = id - tile * a.oc_wgs;
   const int group = DivM(ocb, a.m_tpg);
   int ocl = (ocb - group * a.wgs_per_group) * a.loop;  // channel block of the group
@@ -172,136 +201,167 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
   const int n0 = tn * a.G;
   const int x0 = tx * a.TW, y0 = ty * a.TH;
   const int ix0 = x0 * a.sw - a.pad_l, iy0 = y0 * a.sh - a.pad_t;
+  // window columns inside the image (none where the window lies in padding altogether: the stores' unsigned range needs hi >= lo)
+  const int col_lo = max(0, -ix0), col_hi = max(col_lo, min(a.IW, a.W - ix0));
 
   const int row = lane & 31, half = lane >> 5;
   const int ks = wave % KS, wn = wave / KS % WN, wm = wave / KS / WN;
-  // this wavefront's share of a chunk's steps, and its weights
-  const int per = (a.steps + KS - 1) / KS;
-  const int s0 = KS == 1 ? 0 : min(ks * per, a.steps), s1 = KS == 1 ? a.steps : min(s0 + per, a.steps);
-  const uint32_t tile_stride = static_cast<uint32_t>((MULTI ? a.chunks : 1) * a.steps) * 64;
-  const int passes = MULTI ? a.chunks : min(a.loop, a.tiles_per_group - ocl);
-  const v4i* wp = a.wpk + static_cast<size_t>((group * a.tiles_per_group + ocl) * (WN * NT) + wn * NT) * tile_stride + lane;
-  v4i fw[R][NT];
-  auto fetch_w = [&](int chunk, int s, v4i (&f)[NT]) {
-    const uint32_t at = static_cast<uint32_t>(chunk * a.steps + max(min(s, s1 - 1), 0)) * 64;  // (past the end: the last step once more, not multiplied)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) f[t] = wp[t * tile_stride + at];
-  };
-
-  const uint32_t plane_bytes = a.plane_bytes, image_bytes = a.image_bytes;
-  const int npx = a.npx, items = a.items;
-  // window columns inside the image (none where the window lies in padding altogether: the stores' unsigned range needs hi >= lo)
-  const int col_lo = max(0, -ix0), col_hi = max(col_lo, min(a.IW, a.W - ix0));
   uint32_t base[MT];  // LDS byte offset of this lane's pixel in each pixel tile
   acc_t acc[MT][NT];
+  v4i fw[R][NT];
 
-  // MULTI: a pass is a chunk of the channels, the results follow the last. Else: a pass is a block of output channels over the
-  // same staged window.
-  for (int pass = 0; pass < passes; ++pass) {
-    const int chunk = MULTI ? pass : 0;
-    if (MULTI || pass == 0) {
-    if (chunk) __syncthreads();  // the window is free
-    // ---- stage: an item = (granule, column group, row); lanes take gl granules, then the cells of a plane (contiguous in
-    // memory where the rows are whole), then the next gl granules ----
-    const int c0 = chunk * a.gpc * (16 / E);  // first channel of the chunk
-    const uint8_t* xg = a.x + static_cast<size_t>(n0) * image_bytes + static_cast<size_t>(group * a.icg + c0) * plane_bytes;
-    const bool all_full = c0 + a.gpc * (16 / E) <= a.icg;  // uniform: every granule of the chunk has all its channels
-    for (int it0 = 0; it0 < items; it0 += kThreads) {
-      const int it = it0 + tid;
-      item_t item;
-      const bool live = it < items;
-      const int itc = live ? it : 0;
-      const int rest = DivM(itc, a.m_gl), gl = itc - rest * a.gl;
-      const int gh = DivM(rest, a.m_cells), cell = rest - gh * a.cells;
-      const int gr = gh * a.gl + gl;
-      const int r = DivM(cell, a.m_ncg), cg = cell - r * a.ncg;
-      const int g = DivM(r, a.m_ih), ry = r - g * a.IH;
-      const int iy = iy0 + ry * a.row_step, ixs = ix0 + P * cg;
-      const bool inside = live && static_cast<unsigned>(iy) < static_cast<unsigned>(a.H) && ixs > -P && ixs < a.W && n0 + g < a.batch;
-      const int valid = min(a.icg - c0 - gr * (16 / E), 16 / E);  // channels of the granule
-      // P pixels from the group's first column inside the image, further in front at the plane's end: what lies outside
-      // the row is not stored, what the neighbouring group stores too is the same
-      const int px = min(iy * a.W + max(ixs, 0), a.at_max);
-      const int col = px - iy * a.W - ix0;  // window column of the first pixel
-      const uint32_t at = inside && valid > 0 ? static_cast<uint32_t>(g) * image_bytes + static_cast<uint32_t>(gr * (16 / E)) * plane_bytes + static_cast<uint32_t>(px) * E : 0u;
-      if (all_full) item.template Load<true>(xg, at, plane_bytes, 16 / E);
-      else item.template Load<false>(xg, at, plane_bytes, max(valid, 1));
-      if (it0 == 0) {
-        // under the first loads: the first weights, the table, the accumulators, the lanes' pixels, the padding
-        __builtin_amdgcn_sched_barrier(0);
+  // A work item's place: an item = (granule, column group, row); lanes take gl granules, then the cells of a plane (contiguous in
+  // memory where the rows are whole), then the next gl granules.
+  struct Where { uint32_t at; int to, col, valid; bool inside; };
+  auto find = [&](const TileArgs& a, int it, int c0) {
+    Where w;
+    const bool live = it < a.items;
+    const int itc = live ? it : 0;
+    const int rest = DivM(itc, a.m_gl), gl = itc - __mul24(rest, a.gl);
+    const int gh = DivM(rest, a.m_cells), cell = rest - __mul24(gh, a.cells);
+    const int gr = __mul24(gh, a.gl) + gl;
+    const int r = DivM(cell, a.m_ncg), cg = cell - __mul24(r, a.ncg);
+    const int g = DivM(r, a.m_ih), ry = r - __mul24(g, a.IH);
+    const int iy = iy0 + __mul24(ry, a.row_step), ixs = ix0 + P * cg;
+    w.inside = live && static_cast<unsigned>(iy) < static_cast<unsigned>(a.H) && ixs > -P && ixs < a.W && n0 + g < a.batch;
+    w.valid = min(a.icg - c0 - gr * (16 / E), 16 / E);  // channels of the granule
+    // P pixels from the group's first column inside the image, further in front at the plane's end: what lies outside
+    // the row is not stored, what the neighbouring group stores too is the same
+    const int px = min(iy * a.W + max(ixs, 0), a.at_max);
+    w.col = px - iy * a.W - ix0;  // window column of the first pixel
+    w.at = w.inside && w.valid > 0 ? static_cast<uint32_t>(g) * a.image_bytes + static_cast<uint32_t>(gr * (16 / E)) * a.plane_bytes + static_cast<uint32_t>(px) * E : 0u;
+    w.to = __mul24(__mul24(r, a.IW) + w.col, a.pitch) + gr * 16;
+    return w;
+  };
+  auto store = [&](const TileArgs& a, const item_t& item, const Where& w, bool all_full) {
+    if (!w.inside) return;
+    uint8_t* to = lds + w.to;
+    v4i mask;
+    if (!all_full)
 #pragma unroll
-        for (int u = 0; u < R; ++u) fetch_w(chunk, s0 + u, fw[u]);
-        __builtin_amdgcn_sched_barrier(0);
-        if (chunk == 0) {
-#pragma unroll
-          for (int m = 0; m < MT; ++m) {
-            const int q = min((wm * MT + m) * 32 + row, a.NQ - 1);  // (pixels past the tile's end repeat its last one and are not stored)
-            const int qg = DivM(q, a.m_thtw), rem = q - qg * a.TH * a.TW;
-            const int qy = DivM(rem, a.m_tw), qx = rem - qy * a.TW;
-            base[m] = static_cast<uint32_t>(((qg * a.IH + qy * a.row_stride) * a.IW + qx * a.sw) * a.pitch);
-          }
-        }
-        if (ix0 < 0 || ix0 + a.IW > a.W || iy0 < 0 || iy0 + (a.IH - 1) * a.row_step >= a.H) {  // uniform: the window leaves the image
-          const int pad_whole = max(0, min(a.last_granule - chunk * a.gpc, a.gpc));
-          const int pf = static_cast<int>(a.pad_full);
-          const v4i pad_unit = {pf, pf, pf, pf};
-          const v4i pad_tail = {static_cast<int>(a.pad_last[0]), static_cast<int>(a.pad_last[1]), static_cast<int>(a.pad_last[2]), static_cast<int>(a.pad_last[3])};
-          for (int p = tid; p < npx; p += kThreads) {
-            const int pr = DivM(p, a.m_iw), cx = p - pr * a.IW;
-            const int pry = pr - DivM(pr, a.m_ih) * a.IH;
-            const int py = iy0 + pry * a.row_step;
-            if (static_cast<unsigned>(py) < static_cast<unsigned>(a.H) && cx >= col_lo && cx < col_hi) continue;
-            v4i* to = reinterpret_cast<v4i*>(lds + p * a.pitch);
-            for (int pg = 0; pg < pad_whole; ++pg) to[pg] = pad_unit;
-            if (pad_whole < a.gpc) {  // uniform: the chunk holds the channels' last granule (and empty ones)
-              to[pad_whole] = pad_tail;
-              for (int pg = pad_whole + 1; pg < a.gpc; ++pg) to[pg] = v4i{0, 0, 0, 0};
-            }
-          }
-        }
-        if (chunk == 0) {
-          int* tab = reinterpret_cast<int*>(lds + a.off_tab);
-          if (tid < tab_n) tab[tid] = tab_first;
-          for (int i = tid + kThreads; i < tab_n; i += kThreads) tab[i] = a.tab[i];
-        }
+      for (int q = 0; q < 4; ++q) {
+        const int nb = w.valid * E - 4 * q;
+        mask[q] = nb >= 4 ? -1 : nb <= 0 ? 0 : static_cast<int>((1u << (8 * nb)) - 1u);
       }
-      if (inside) {
-        uint8_t* to = lds + (r * a.IW + col) * a.pitch + gr * 16;
-        v4i mask;
-        if (!all_full)
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int nb = valid * E - 4 * q;
-            mask[q] = nb >= 4 ? -1 : nb <= 0 ? 0 : static_cast<int>((1u << (8 * nb)) - 1u);
-          }
+    for (int h = 0; h < P / 4; ++h) {
+      v4i u[4];
+      item.Units(h, u);
 #pragma unroll
-        for (int h = 0; h < P / 4; ++h) {
-          v4i u[4];
-          item.Units(h, u);
+      for (int i = 0; i < 4; ++i) {
+        if (DT == kI8) u[i] ^= static_cast<int>(a.xor_mask);
+        if (!all_full) u[i] &= mask;
+        if (static_cast<unsigned>(w.col + 4 * h + i - col_lo) < static_cast<unsigned>(col_hi - col_lo)) *reinterpret_cast<v4i*>(to + (4 * h + i) * a.pitch) = u[i];
+      }
+    }
+  };
+
+  // a wavefront's share of a chunk's steps, and its weights for a block of channels
+  struct Steps { int s0, s1; const v4i* wp; uint32_t tile_stride; };
+  auto share = [&](const TileArgs& a) {
+    Steps w;
+    const int per = (a.steps + KS - 1) / KS;
+    w.s0 = KS == 1 ? 0 : min(ks * per, a.steps);
+    w.s1 = KS == 1 ? a.steps : min(w.s0 + per, a.steps);
+    w.tile_stride = static_cast<uint32_t>((MULTI ? a.chunks : 1) * a.steps) * 64;
+    w.wp = a.wpk + static_cast<size_t>((group * a.tiles_per_group + ocl) * (WN * NT) + wn * NT) * w.tile_stride + lane;
+    return w;
+  };
+  auto fetch_w = [&](const Steps& w, int first, int s, v4i (&f)[NT]) {
+    const uint32_t at = static_cast<uint32_t>(first + max(min(s, w.s1 - 1), 0)) * 64;  // (past the end: the last step once more, not multiplied)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            if (DT == kI8) u[i] ^= static_cast<int>(a.xor_mask);
-            if (!all_full) u[i] &= mask;
-            if (static_cast<unsigned>(col + 4 * h + i - col_lo) < static_cast<unsigned>(col_hi - col_lo)) *reinterpret_cast<v4i*>(to + (4 * h + i) * a.pitch) = u[i];
-          }
+    for (int t = 0; t < NT; ++t) f[t] = w.wp[t * w.tile_stride + at];
+  };
+  // ---- stage a chunk's window. `a`: what the first loads need; `late()`: the rest ----
+  auto load = [&](const TileArgs& a, const uint8_t* xg, bool all_full, item_t& item, const Where& w) {
+    if (all_full) item.template Load<true>(xg, w.at, a.plane_bytes, 16 / E);
+    else if (a.icg < 16 / E) item.LoadFew(xg, w.at, a.plane_bytes, a.icg);
+    else item.template Load<false>(xg, w.at, a.plane_bytes, max(w.valid, 1));
+  };
+  auto stage = [&](const TileArgs& a, auto late, int chunk) {
+    const int c0 = chunk * a.gpc * (16 / E);  // first channel of the chunk
+    const uint8_t* xg = a.x + static_cast<size_t>(n0) * a.image_bytes + static_cast<size_t>(group * a.icg + c0) * a.plane_bytes;
+    const bool all_full = c0 + a.gpc * (16 / E) <= a.icg;  // uniform: every granule of the chunk has all its channels
+    item_t item;
+    Where where = find(a, tid, c0);
+    load(a, xg, all_full, item, where);
+    // under the first loads: the first weights, the table, the lanes' pixels, the padding
+    const TileArgs& b = late();
+    const int tab_n = 2 * b.steps_pad;
+    const int tab_first = b.tab[min(tid, tab_n - 1)];
+    const Steps w = share(b);
+#pragma unroll
+    for (int u = 0; u < R; ++u) fetch_w(w, chunk * b.steps, w.s0 + u, fw[u]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (chunk == 0) {
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const int q = min((wm * MT + m) * 32 + row, b.NQ - 1);  // (pixels past the tile's end repeat its last one and are not stored)
+        const int qg = DivM(q, b.m_thtw), rem = q - __mul24(qg, b.TH * b.TW);
+        const int qy = DivM(rem, b.m_tw), qx = rem - __mul24(qy, b.TW);
+        base[m] = static_cast<uint32_t>(__mul24(__mul24(__mul24(qg, b.IH) + __mul24(qy, b.row_stride), b.IW) + __mul24(qx, b.sw), b.pitch));
+      }
+    }
+    if (ix0 < 0 || ix0 + b.IW > b.W || iy0 < 0 || iy0 + (b.IH - 1) * b.row_step >= b.H) {  // uniform: the window leaves the image
+      const int pad_whole = max(0, min(b.last_granule - chunk * b.gpc, b.gpc));
+      const int pf = static_cast<int>(b.pad_full);
+      const v4i pad_unit = {pf, pf, pf, pf};
+      const v4i pad_tail = {static_cast<int>(b.pad_last[0]), static_cast<int>(b.pad_last[1]), static_cast<int>(b.pad_last[2]), static_cast<int>(b.pad_last[3])};
+      for (int p = tid; p < b.npx; p += kThreads) {
+        const int pr = DivM(p, b.m_iw), cx = p - __mul24(pr, b.IW);
+        const int pry = pr - __mul24(DivM(pr, b.m_ih), b.IH);
+        const int py = iy0 + __mul24(pry, b.row_step);
+        if (static_cast<unsigned>(py) < static_cast<unsigned>(b.H) && cx >= col_lo && cx < col_hi) continue;
+        v4i* to = reinterpret_cast<v4i*>(lds + __mul24(p, b.pitch));
+        for (int pg = 0; pg < pad_whole; ++pg) to[pg] = pad_unit;
+        if (pad_whole < b.gpc) {  // uniform: the chunk holds the channels' last granule (and empty ones)
+          to[pad_whole] = pad_tail;
+          for (int pg = pad_whole + 1; pg < b.gpc; ++pg) to[pg] = v4i{0, 0, 0, 0};
         }
       }
     }
+    if (chunk == 0) {
+      int* tab = reinterpret_cast<int*>(lds + b.off_tab);
+      if (tid < tab_n) tab[tid] = tab_first;
+      for (int i = tid + kThreads; i < tab_n; i += kThreads) tab[i] = b.tab[i];
+    }
+    store(b, item, where, all_full);
+#pragma unroll 1
+    for (int it0 = kThreads; it0 < b.items; it0 += kThreads) {
+      where = find(b, it0 + tid, c0);
+      load(b, xg, all_full, item, where);
+      store(b, item, where, all_full);
+    }
     __syncthreads();
     // ---- channel sums of the staged pixels ----
-    if (DT == kI8 && a.zws) {  // uniform
-      int* sum = reinterpret_cast<int*>(lds + a.off_sum);
-      for (int p = tid; p < npx; p += kThreads) {
+    if (DT == kI8 && b.zws) {  // uniform
+      int* sum = reinterpret_cast<int*>(lds + b.off_sum);
+      for (int p = tid; p < b.npx; p += kThreads) {
         int v = chunk ? sum[p] : 0;
-        for (int gr = 0; gr < a.gpc; ++gr) {
-          const v4i f = *reinterpret_cast<const v4i*>(lds + p * a.pitch + gr * 16);
+        for (int gr = 0; gr < b.gpc; ++gr) {
+          const v4i f = *reinterpret_cast<const v4i*>(lds + __mul24(p, b.pitch) + gr * 16);
 #pragma unroll
           for (int q = 0; q < 4; ++q) v = __builtin_amdgcn_sdot4(f[q], 0x01010101, v, false);
         }
         sum[p] = v;
       }
     }
+  };
+
+  // MULTI: a pass is a chunk of the channels, the results follow the last. Else: a pass is a block of output channels over the
+  // same staged window.
+  const int loop = a.loop;
+  stage(a, []() -> const TileArgs& { return LateArgs<TileArgs>(); }, 0);
+  const TileArgs& b = LateArgs<TileArgs>();
+  for (int pass = 0;; ++pass) {
+    const int chunk = MULTI ? pass : 0;
+    if (MULTI && chunk) {
+      __syncthreads();  // the window is free
+      stage(b, [&]() -> const TileArgs& { return b; }, chunk);
     }
+    const int passes = MULTI ? b.chunks : min(loop, b.tiles_per_group - ocl + pass);
+    const Steps w = share(b);
+    const int s0 = w.s0, s1 = w.s1;
     if (!MULTI || chunk == 0)
 #pragma unroll
       for (int m = 0; m < MT; ++m)
@@ -310,15 +370,15 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
 #pragma unroll
           for (int i = 0; i < 16; ++i) acc[m][t][i] = 0;
     // ---- multiply: R steps' weights ahead, two steps' activations ahead ----
-    const int* tab = reinterpret_cast<const int*>(lds + a.off_tab) + half * a.steps_pad;
+    const int* tab = reinterpret_cast<const int*>(lds + b.off_tab) + half * b.steps_pad;
     v4i fx[2][MT];
     auto fetch_x = [&](int s, v4i (&f)[MT]) {
       const int off = tab[s];  // (the table is padded)
 #pragma unroll
       for (int m = 0; m < MT; ++m) f[m] = *reinterpret_cast<const v4i*>(lds + base[m] + off);
     };
-    auto multiply = [&](int s, v4i (&f)[MT], const v4i (&w)[NT]) {
-      if (DT != kI8 && a.odd && s == a.steps - 1 && half)  // (zero weights, but the data may be an infinity)
+    auto multiply = [&](int s, bool last, v4i (&f)[MT], const v4i (&w)[NT]) {
+      if (DT != kI8 && last && b.odd && s == b.steps - 1 && half)  // (zero weights, but the data may be an infinity)
 #pragma unroll
         for (int m = 0; m < MT; ++m) f[m] = v4i{0, 0, 0, 0};
 #pragma unroll
@@ -333,24 +393,26 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
     for (; s + R < s1; s += R) {
 #pragma unroll
       for (int u = 0; u < R; ++u) {
-        multiply(s + u, fx[u & 1], fw[u]);
-        fetch_w(chunk, s + u + R, fw[u]);
+        multiply(s + u, false, fx[u & 1], fw[u]);  // (a chunk's last step is below)
+        fetch_w(w, chunk * b.steps, s + u + R, fw[u]);
         fetch_x(s + u + 2, fx[u & 1]);
       }
     }
 #pragma unroll
     for (int u = 0; u < R; ++u)
       if (s + u < s1) {  // uniform
-        multiply(s + u, fx[u & 1], fw[u]);
+        multiply(s + u, true, fx[u & 1], fw[u]);
         fetch_x(s + u + 2, fx[u & 1]);
       }
     if (MULTI && pass + 1 < passes) continue;
     if (!MULTI && pass + 1 < passes) {  // the next block's first weights travel under the results
-      wp += static_cast<size_t>(WN * NT) * tile_stride;
+      Steps next = w;
+      next.wp += static_cast<uint32_t>(WN * NT) * w.tile_stride;
 #pragma unroll
-      for (int u = 0; u < R; ++u) fetch_w(0, s0 + u, fw[u]);
+      for (int u = 0; u < R; ++u) fetch_w(next, 0, s0 + u, fw[u]);
     }
 
+  const TileArgs& c = LateArgs<TileArgs>();
   // the epilogue's tables travel while the wavefronts meet
   int bias[NT];
   tvx_v4i rq[NT];
@@ -358,11 +420,11 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
   for (int t = 0; t < NT; ++t) {
     const int oc = (ocl * WN + wn) * NT * 32 + t * 32 + row;  // channel of the group
     if constexpr (DT == kI8) {
-      const int slot = group * a.tiles_per_group * (WN * NT * 32) + oc;
-      rq[t] = a.rq[slot];
-      bias[t] = a.biasf[slot];
+      const int slot = group * c.tiles_per_group * (WN * NT * 32) + oc;
+      rq[t] = c.rq[slot];
+      bias[t] = c.biasf[slot];
     } else {
-      bias[t] = a.biasfl && oc < a.ocg ? reinterpret_cast<const int*>(a.biasfl)[group * a.ocg + oc] : 0;
+      bias[t] = c.biasfl && oc < c.ocg ? reinterpret_cast<const int*>(c.biasfl)[group * c.ocg + oc] : 0;
     }
   }
 
@@ -370,7 +432,7 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
   // that become eight consecutive pixels, or single quads), every wavefront finishes its own ----
   constexpr int kQuads = KS == 1 ? 4 : (2 * MT * NT >= KS ? 2 : 1);  // quads of a piece
   constexpr int kPieces = 4 / kQuads;
-  const bool box = DT == kI8 && a.zws && (MULTI || pass == 0);  // the window sums are to be made
+  const bool box = DT == kI8 && c.zws && (MULTI || pass == 0);  // the window sums are to be made
   if (KS > 1 || box) {
     __syncthreads();
     elem_t* part = reinterpret_cast<elem_t*>(lds);  // [wave][tile][element][lane]
@@ -386,16 +448,16 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
           }
     // window sums: the box filter over the channel sums
     if (box) {
-      const int* sum = reinterpret_cast<const int*>(lds + a.off_sum);
-      int* zt = reinterpret_cast<int*>(lds + a.off_zt);
-      for (int q = tid; q < a.NQ; q += kThreads) {
-        const int g = DivM(q, a.m_thtw), rem = q - g * a.TH * a.TW;
-        const int qy = DivM(rem, a.m_tw), qx = rem - qy * a.TW;
-        const int* sp = sum + (g * a.IH + qy * a.row_stride) * a.IW + qx * a.sw;
+      const int* sum = reinterpret_cast<const int*>(lds + c.off_sum);
+      int* zt = reinterpret_cast<int*>(lds + c.off_zt);
+      for (int q = tid; q < c.NQ; q += kThreads) {
+        const int g = DivM(q, c.m_thtw), rem = q - g * c.TH * c.TW;
+        const int qy = DivM(rem, c.m_tw), qx = rem - qy * c.TW;
+        const int* sp = sum + (g * c.IH + qy * c.row_stride) * c.IW + qx * c.sw;
         int v = 0;
-        for (int ky = 0; ky < a.taps_h; ++ky)
-          for (int kx = 0; kx < a.taps_w; ++kx) v += sp[ky * a.dil_row + kx * a.dil_col];
-        zt[q] = -a.zws * v;
+        for (int ky = 0; ky < c.taps_h; ++ky)
+          for (int kx = 0; kx < c.taps_w; ++kx) v += sp[ky * c.dil_row + kx * c.dil_col];
+        zt[q] = -c.zws * v;
       }
     }
     __syncthreads();
@@ -428,32 +490,32 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
       for (int k = 0; k < 4; ++k) {
         if (KS > 1 && ((m * NT + t) * kPieces + k % kPieces) % KS != ks) continue;
         const int q0 = (wm * MT + m) * 32 + 8 * k + 4 * half;
-        uint8_t* to = lds + a.off_out + (wn * NT * 32 + t * 32 + row) * a.out_pitch + q0 * E;
+        uint8_t* to = lds + c.off_out + (wn * NT * 32 + t * 32 + row) * c.out_pitch + q0 * E;
         if constexpr (DT == kI8) {
           int v[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = acc[m][t][4 * k + e] + bias[t];
-          if (a.zws) {
-            const v4i z = *reinterpret_cast<const v4i*>(lds + a.off_zt + q0 * 4);
+          if (c.zws) {
+            const v4i z = *reinterpret_cast<const v4i*>(lds + c.off_zt + q0 * 4);
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] += z[e];
           }
-          if (a.pre_ties) {  // (uniform)
+          if (c.pre_ties) {  // (uniform)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] <<= a.pre_ties >> 1;
-            if (a.pre_ties & 1) LowerOddTies(v, rq[t]);
+            for (int e = 0; e < 4; ++e) v[e] <<= c.pre_ties >> 1;
+            if (c.pre_ties & 1) LowerOddTies(v, rq[t]);
           }
           const int sh = rq[t][1] & 31;
           const int64_t round = RoundHigh(rq[t][2]);
-          *reinterpret_cast<uint32_t*>(to) = (a.narrow ? RequantSaturate4<true>(v, rq[t][0], sh, round, a.lo << sh, ((a.hi + 1) << sh) - 1)
-                                                       : RequantSaturate4<false>(v, rq[t][0], sh, round, 0, 0)) ^ a.out_xor;
+          *reinterpret_cast<uint32_t*>(to) = (c.narrow ? RequantSaturate4<true>(v, rq[t][0], sh, round, c.lo << sh, ((c.hi + 1) << sh) - 1)
+                                                       : RequantSaturate4<false>(v, rq[t][0], sh, round, 0, 0)) ^ c.out_xor;
         } else {
           float v[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             v[e] = acc[m][t][4 * k + e] + __builtin_bit_cast(float, bias[t]);
-            if (a.act != TVX_ACT_NONE) v[e] = v[e] < 0.f ? 0.f : v[e];
-            if (a.act == TVX_ACT_RELU6) v[e] = v[e] > 6.f ? 6.f : v[e];
+            if (c.act != TVX_ACT_NONE) v[e] = v[e] < 0.f ? 0.f : v[e];
+            if (c.act == TVX_ACT_RELU6) v[e] = v[e] > 6.f ? 6.f : v[e];
           }
           if constexpr (DT == kF16) {
             _Float16 h[4];
@@ -466,24 +528,24 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
         }
       }
   __syncthreads();
-  const int ohw = a.OH * a.OW, whole = a.TW == a.OW;  // (uniform)
-  const int rows_live = min(a.TH, a.OH - y0);
-  const int runs_live = whole ? min(a.G, a.batch - n0) : rows_live, run_live = whole ? rows_live * a.OW : min(a.TW, a.OW - x0);
-  const int ocb0 = ocl * (WN * NT * 32), channels = min(WN * NT * 32, a.ocg - ocb0);
-  uint8_t* yb = a.y + ((static_cast<size_t>(n0) * a.OC + static_cast<size_t>(group) * a.ocg + ocb0) * ohw + y0 * a.OW + x0) * E;
+  const int ohw = c.OH * c.OW, whole = c.TW == c.OW;  // (uniform)
+  const int rows_live = min(c.TH, c.OH - y0);
+  const int runs_live = whole ? min(c.G, c.batch - n0) : rows_live, run_live = whole ? rows_live * c.OW : min(c.TW, c.OW - x0);
+  const int ocb0 = ocl * (WN * NT * 32), channels = min(WN * NT * 32, c.ocg - ocb0);
+  uint8_t* yb = c.y + ((static_cast<size_t>(n0) * c.OC + static_cast<size_t>(group) * c.ocg + ocb0) * ohw + y0 * c.OW + x0) * E;
   // a thread keeps its place in the channels' runs and walks the channels
-  const int place = tid & ((1 << a.runs_shift) - 1), run = DivM(place, a.m_run4), px = (place - run * ((a.run_px + 3) >> 2)) * 4;
+  const int place = tid & ((1 << c.runs_shift) - 1), run = DivM(place, c.m_run4), px = (place - run * ((c.run_px + 3) >> 2)) * 4;
   const int left = run < runs_live ? run_live - px : 0;
-  const int ch0 = tid >> a.runs_shift, ch_step = kThreads >> a.runs_shift;
-  const uint8_t* from = lds + a.off_out + ch0 * a.out_pitch + (run * a.run_px + px) * E;
-  uint8_t* to = yb + (static_cast<size_t>(ch0) * ohw + static_cast<size_t>(run) * a.run_out + px) * E;
+  const int ch0 = tid >> c.runs_shift, ch_step = kThreads >> c.runs_shift;
+  const uint8_t* from = lds + c.off_out + ch0 * c.out_pitch + (run * c.run_px + px) * E;
+  uint8_t* to = yb + (static_cast<size_t>(ch0) * ohw + static_cast<size_t>(run) * c.run_out + px) * E;
   const size_t to_step = static_cast<size_t>(ch_step) * ohw * E;
   if (left > 0)
-  for (int ch = ch0; ch < channels; ch += ch_step, from += ch_step * a.out_pitch, to += to_step) {
+  for (int ch = ch0; ch < channels; ch += ch_step, from += ch_step * c.out_pitch, to += to_step) {
     uint32_t four[E];
     if (left >= 4) {
       if constexpr (E == 1) {  // (a run begins at any byte: the dword out of two)
-        const uint32_t at = static_cast<uint32_t>(run * a.run_px), *w = reinterpret_cast<const uint32_t*>(from - (at & 3));
+        const uint32_t at = static_cast<uint32_t>(run * c.run_px), *w = reinterpret_cast<const uint32_t*>(from - (at & 3));
         four[0] = __builtin_amdgcn_alignbyte(w[1], w[0], at & 3);
       } else {
 #pragma unroll
@@ -506,6 +568,7 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
       }
     }
   }
+    if (pass + 1 >= passes) break;
     ++ocl;
   }
 }
@@ -669,12 +732,13 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   const int group_px = dt == kF32 ? 4 : 8;
   if (W * H < group_px) return TVX_E_UNSUPPORTED;
   const int groups = d->groups > 1 ? d->groups : 1;
-  a.C = d->in_c; a.H = H; a.W = W; a.OC = d->out_c; a.OH = OH; a.OW = OW; a.batch = d->batch;
+  const int C = d->in_c;
+  a.H = H; a.W = W; a.OC = d->out_c; a.OH = OH; a.OW = OW; a.batch = d->batch;
   a.sh = d->stride_h; a.sw = d->stride_w; a.pad_t = d->pad_top; a.pad_l = d->pad_left;
-  a.icg = a.C / groups; a.ocg = a.OC / groups;
+  a.icg = C / groups; a.ocg = a.OC / groups;
   const int granules = (a.icg * E + 15) / 16, taps = kh * kw;
   if (taps > 1024) return TVX_E_UNSUPPORTED;
-  const uint64_t image = static_cast<uint64_t>(a.C) * H * W * E, out_image = static_cast<uint64_t>(a.OC) * OH * OW;
+  const uint64_t image = static_cast<uint64_t>(C) * H * W * E, out_image = static_cast<uint64_t>(a.OC) * OH * OW;
   a.row_step = kh == 1 ? a.sh : 1;
   a.row_stride = kh == 1 ? 1 : a.sh;
 
@@ -761,7 +825,7 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   a.npx = g.G * g.IH * g.IW;
   a.items = a.cells * a.gpc;
   a.plane_bytes = static_cast<uint32_t>(H) * W * E;
-  a.image_bytes = a.plane_bytes * a.C;
+  a.image_bytes = a.plane_bytes * C;
   a.at_max = H * W - group_px;
   const int64_t npx = static_cast<int64_t>(g.G) * g.IH * g.IW;
   a.off_tab = static_cast<int>(WindowBytes(sp, npx * g.pitch, E, g.loop));

@@ -114,6 +114,16 @@ constexpr int kRqGeneric = 0;    // any shift: 64-bit product
 constexpr int kRqFast = 1;       // high half of the product + tie fix-up
 constexpr int kRqFastNoTie = 2;  // additionally no accumulator can land on a tie
 
+// A kernel's (first) argument, to be read behind this place. What a kernel computes from its arguments for its later phases - strides,
+// reciprocals, epilogue addresses - the compiler moves in front of its first loads, with one round trip to the argument segment after
+// the other and scalar registers spilled to lanes: 700 instructions and 1.5 us there in conv2d_tile_i8. Fields read through this are not.
+template <class Args>
+__device__ __forceinline__ const Args& LateArgs() {
+  auto p = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *reinterpret_cast<const Args*>((const void*)p);
+}
+
 // clamp(v, lo, hi) for lo <= hi in one instruction
 __device__ __forceinline__ int Med3(int v, int lo, int hi) {
   int r;
