@@ -2,12 +2,8 @@
 // 5x5, int8 / uint8 windows of 5x5 (and of 3x3 on rows that are not whole dwords), at stride 1 or 2 (vxConvolutionLayer's depthwise form; reference:
 // src/tim/vx/internal/src/ops/vsi_nn_op_conv2d.c:35-118).
 //
-// A thread computes R output rows x PX neighbouring outputs of one plane. Each input row behind them is one unaligned run of
-// the plane's memory (10 to 22 bytes of elements, loaded as whole dwords): a run that leaves its row reads the neighbouring
-// row's elements, which are masked - by the column pattern, the same for all of a thread's rows - so that no load depends on
-// the position. Only runs that would leave the tensor, at its first and last elements, are read from inside it and shifted. All
-// of a thread's loads are issued before the first use. Column and row groups at a plane's end are moved back inside it: they
-// compute some outputs twice, and every store but those of planes smaller than a group is a whole vector.
+// A thread computes two or four output rows x four or eight neighbouring outputs of one plane from rows held in registers
+// (plane_rows.h).
 // A plane's channel is uniform where its threads fill whole wavefronts (weights then are scalar operands); small planes share
 // wavefronts and keep their weights in vector registers.
 //
@@ -20,36 +16,30 @@
 #include <cstdlib>
 #include <cstring>
 
+#include "plane_rows.h"
 #include "variants.h"
 
 namespace tvx {
 namespace {
 
-struct DwrArgs {
-  const uint8_t* x;
-  uint8_t* y;
+struct DwrArgs : PlaneArgs {
   const float* wf;        // floating point: [channel][K * K, padded to whole fours], then the bias at place K * K
   const int* wi;          // quantized: [channel][K rows of two dwords, folded bias, pad]
   const tvx_v4i* rq;
-  int C, H, W, OH, OW, pad_t, pad_l;
-  int ncg, tpp, bpp;      // column groups of a row, threads and (whole wavefronts per plane) workgroups of a plane
-  int planes;
-  uint32_t m_tpp, m_ncg, m_c;
-  int total;              // elements of the input
+  int C;
+  uint32_t m_c;
   int act;
-  int fill, xor_in, zws, lo, hi, narrow, out_xor, pre_ties;
+  int zws, lo, hi, narrow, out_xor, pre_ties;
 };
 
-__device__ __forceinline__ int DivM(int u, uint32_t m) { return m ? static_cast<int>(__umulhi(static_cast<uint32_t>(u), m)) : u; }
-
 // DT: TVX_I8 (uint8 too), TVX_F16 or TVX_F32
-template <int DT, int K, int S> struct Tile {
+template <int DT, int K, int S, int R> struct Tile {
   static constexpr int E = DT == TVX_F32 ? 4 : DT == TVX_F16 ? 2 : 1;
   static constexpr int PX = S == 1 && DT != TVX_F32 ? 8 : 4;
   static constexpr int L = (PX - 1) * S + K;          // elements of a row behind PX outputs
-  static constexpr int LD = (L * E + 3) / 4;          // ... in dwords
-  static constexpr int LE = LD * 4 / E;               // ... and the elements these load
+  static constexpr int NR = (R - 1) * S + K;          // rows behind R outputs
   static constexpr int WS = DT == TVX_I8 ? 2 * K + 2 : (K * K + 4) / 4 * 4;  // words of a channel's table: weights, bias
+  using Rows = PlaneRows<E, L, NR>;
 };
 
 // Place of a thread: its plane, channel and first output.
@@ -65,146 +55,31 @@ __device__ __forceinline__ Place Find(const DwrArgs& a) {
     p.live = t < a.tpp;
     t = min(t, a.tpp - 1);
   } else {
-    const uint32_t first = blockIdx.x * blockDim.x;
-    const int plane0 = __builtin_amdgcn_readfirstlane(static_cast<int>(first / static_cast<uint32_t>(a.tpp)));
+    int plane0;
+    p.plane = SharedPlane(a, &plane0, &t, &p.live);
     const int c0 = __builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<uint32_t>(plane0) % static_cast<uint32_t>(a.C)));
-    const int local = static_cast<int>(first - static_cast<uint32_t>(plane0) * a.tpp + threadIdx.x);
-    const int more = DivM(local, a.m_tpp);
-    t = local - more * a.tpp;
-    p.live = plane0 + more < a.planes;
-    p.plane = min(plane0 + more, a.planes - 1);
     const int c = c0 + p.plane - plane0;
-    p.c = c - DivM(c, a.m_c) * a.C;
+    p.c = c - DivReciprocal(c, a.m_c) * a.C;
   }
-  const int rg = DivM(t, a.m_ncg), cg = t - rg * a.ncg;
-  p.oy = min(rg * R, max(a.OH - R, 0));
-  p.ox = min(cg * PX, max(a.OW - PX, 0));
+  FirstOutput<R, PX>(a, t, &p.oy, &p.ox);
   return p;
-}
-
-// The rows behind a thread's outputs; what lies outside the image is `fill`.
-template <int DT, int K, int S, int R>
-struct Rows {
-  using T = Tile<DT, K, S>;
-  static constexpr int NR = (R - 1) * S + K;
-  uint32_t d[NR][T::LD];
-
-  // the row's elements by n places up (towards higher columns) or down; where n is a row or more, nothing of it counts
-  template <bool UP, int STEP = 1>
-  static __device__ __forceinline__ void ShiftDwords(uint32_t (&v)[T::LD], int dwords) {
-    const uint32_t on = dwords & STEP ? ~0u : 0u;
-#pragma unroll
-    for (int k = 0; k < T::LD; ++k) {
-      const int j = UP ? T::LD - 1 - k : k;
-      const uint32_t from = UP ? (j >= STEP ? v[j >= STEP ? j - STEP : 0] : 0u) : (j + STEP < T::LD ? v[j + STEP < T::LD ? j + STEP : 0] : 0u);
-      v[j] = (from & on) | (v[j] & ~on);
-    }
-    if constexpr (2 * STEP <= T::LD) ShiftDwords<UP, 2 * STEP>(v, dwords);
-  }
-  template <bool UP>
-  static __device__ __forceinline__ void Shift(uint32_t (&v)[T::LD], int n) {
-    const int bytes = min(n, T::LE) * T::E;
-    ShiftDwords<UP>(v, bytes / 4);
-    if constexpr (T::E < 4) {
-      const uint32_t rest = 8 * (bytes & 3);
-#pragma unroll
-      for (int k = 0; k < T::LD; ++k) {
-        const int j = UP ? T::LD - 1 - k : k;
-        const uint64_t lo = UP ? (j > 0 ? v[j > 0 ? j - 1 : 0] : 0u) : v[j], hi = UP ? v[j] : (j + 1 < T::LD ? v[j + 1 < T::LD ? j + 1 : 0] : 0u);
-        v[j] = static_cast<uint32_t>((hi << 32 | lo) >> (UP ? 32 - rest : rest));
-      }
-    }
-  }
-
-  __device__ __forceinline__ void Load(const DwrArgs& a, const Place& p) {
-    const int ix = p.ox * S - a.pad_l, iy = p.oy * S - a.pad_t;
-    const int first = p.plane * (a.H * a.W);
-    int moved[NR];  // elements by which a run was moved to lie inside the tensor
-#pragma unroll
-    for (int i = 0; i < NR; ++i) {
-      const int at = first + min(max(iy + i, 0), a.H - 1) * a.W + ix, in = min(max(at, 0), a.total - T::LE);
-      __builtin_memcpy(d[i], a.x + static_cast<size_t>(static_cast<uint32_t>(in)) * T::E, T::LD * 4);
-      moved[i] = in - at;
-    }
-    // the tensor's first and last elements: back to their places (what is shifted in lies outside the image)
-#pragma unroll
-    for (int i = 0; i < NR; ++i)
-      if (__ballot(moved[i] != 0)) {
-        Shift<true>(d[i], max(moved[i], 0));
-        Shift<false>(d[i], max(-moved[i], 0));
-      }
-    if (DT == TVX_I8) {
-#pragma unroll
-      for (int i = 0; i < NR; ++i)
-#pragma unroll
-        for (int j = 0; j < T::LD; ++j) d[i][j] ^= static_cast<uint32_t>(a.xor_in);
-    }
-    const uint32_t fill = DT == TVX_I8 ? static_cast<uint32_t>(a.fill) : 0u;
-    // columns: the same pattern in every row; a wavefront without an edge skips it
-    if (__ballot(ix < 0 || ix + T::L > a.W)) {
-#pragma unroll
-      for (int j = 0; j < T::LD; ++j) {
-        uint32_t keep = 0;
-#pragma unroll
-        for (int e = 0; e < 4 / T::E; ++e)
-          if (static_cast<unsigned>(ix + j * (4 / T::E) + e) < static_cast<unsigned>(a.W)) keep |= (T::E == 4 ? ~0u : (1u << (8 * T::E & 31)) - 1u) << (8 * T::E * e);
-#pragma unroll
-        for (int i = 0; i < NR; ++i) d[i][j] = (d[i][j] & keep) | (fill & ~keep);
-      }
-    }
-    if (__ballot(iy < 0 || iy + NR > a.H)) {
-#pragma unroll
-      for (int i = 0; i < NR; ++i) {
-        const bool in = static_cast<unsigned>(iy + i) < static_cast<unsigned>(a.H);
-#pragma unroll
-        for (int j = 0; j < T::LD; ++j) d[i][j] = in ? d[i][j] : fill;
-      }
-    }
-  }
-};
-
-// PX results of a row; where the row has fewer than that, but four: its first four and its last four.
-template <int E, int N>
-__device__ __forceinline__ void StoreRow(uint8_t* to, const uint32_t (&out)[N], int OW) {
-  constexpr int PX = N * 4 / E;
-  if (OW >= PX) {  // (uniform)
-    __builtin_memcpy(to, out, N * 4);
-  } else if (PX == 8 && OW >= 4) {
-    const int back = (OW - 4) * E;  // bytes in front of the last four
-    uint32_t last[E];
-#pragma unroll
-    for (int j = 0; j < E; ++j) {
-      const uint32_t a = back < 4 ? out[j] : out[j + 1], b = back < 4 ? out[j + 1] : j + 2 < N ? out[j + 2 < N ? j + 2 : 0] : 0u;
-      last[j] = __builtin_amdgcn_alignbyte(b, a, static_cast<uint32_t>(back & 3));
-    }
-    __builtin_memcpy(to, out, 4 * E);
-    __builtin_memcpy(to + back, last, 4 * E);
-  } else {
-#pragma unroll
-    for (int q = 0; q < PX; ++q)
-      if (q < OW) {
-        if constexpr (E == 1) to[q] = static_cast<uint8_t>(out[q / 4] >> (8 * (q & 3)));
-        else if constexpr (E == 2) reinterpret_cast<uint16_t*>(to)[q] = static_cast<uint16_t>(out[q / 2] >> (16 * (q & 1)));
-        else reinterpret_cast<uint32_t*>(to)[q] = out[q];
-      }
-  }
 }
 
 template <int DT, int K, int S, int R, bool UNIFORM>
 __global__ void __launch_bounds__(256) DwRegFloatKernel(DwrArgs a) {
-  using T = Tile<DT, K, S>;
+  using T = Tile<DT, K, S, R>;
   constexpr int PX = T::PX;
   const Place p = Find<UNIFORM, R, PX>(a);
   const float* w = a.wf + p.c * T::WS;
-  Rows<DT, K, S, R> rows;
-  rows.Load(a, p);
+  typename T::Rows rows;
+  rows.Load(a, p.plane, p.oy * S - a.pad_t, p.ox * S - a.pad_l);
   float acc[R][PX];
 #pragma unroll
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int q = 0; q < PX; ++q) acc[r][q] = 0.f;
 #pragma unroll
-  for (int i = 0; i < Rows<DT, K, S, R>::NR; ++i) {
+  for (int i = 0; i < T::NR; ++i) {
     float v[T::L];
 #pragma unroll
     for (int j = 0; j < T::L; ++j) {
@@ -264,17 +139,17 @@ __device__ __forceinline__ int FirstDot(int x, int w, int bias) {
 // zero point (SUMS) the rows' window sums are made once per input row and added to the output rows they belong to.
 template <int K, int S, int R, bool UNIFORM, bool SUMS>
 __global__ void __launch_bounds__(256) DwRegI8Kernel(DwrArgs a) {
-  using T = Tile<TVX_I8, K, S>;
+  using T = Tile<TVX_I8, K, S, R>;
   constexpr int PX = T::PX;
   const Place p = Find<UNIFORM, R, PX>(a);
   const int* w = a.wi + p.c * T::WS;
   const tvx_v4i rq = a.rq[p.c];
-  Rows<TVX_I8, K, S, R> rows;
-  rows.Load(a, p);
+  typename T::Rows rows;
+  rows.Load(a, p.plane, p.oy * S - a.pad_t, p.ox * S - a.pad_l);
   const int bias = w[2 * K];
   int acc[R][PX], sum[R][PX];
 #pragma unroll
-  for (int i = 0; i < Rows<TVX_I8, K, S, R>::NR; ++i) {
+  for (int i = 0; i < T::NR; ++i) {
 #pragma unroll
     for (int q = 0; q < PX; ++q) {
       const int w0 = Cut(rows.d[i], q * S), w1 = K > 4 ? Cut(rows.d[i], q * S + 4) : 0;
@@ -337,8 +212,6 @@ DwRegFn PickKernel(int k, int s, int r, bool uniform, bool sums) {
   return r == 4 ? Pick<DT, 5, 2, 4>(uniform, sums) : Pick<DT, 5, 2, 2>(uniform, sums);
 }
 
-uint32_t Magic(int d) { return d <= 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + d - 1) / d); }
-
 struct Plan {
   DwrArgs a;
   DwRegFn fn;
@@ -399,40 +272,28 @@ int DwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   if (q && K == 3 && !lever && !BetterAt3x3(d)) return TVX_E_UNSUPPORTED;
 
   DwrArgs a{};
-  a.C = d->in_c; a.H = d->in_h; a.W = d->in_w; a.OH = d->out_h; a.OW = d->out_w;
-  a.pad_t = d->pad_top; a.pad_l = d->pad_left;
-  const int64_t planes = static_cast<int64_t>(d->batch) * d->in_c;
-  const int64_t in = planes * d->in_h * d->in_w, out = planes * d->out_h * d->out_w;
-  if (in >= (1 << 30) || out >= (1 << 30) || d->in_c > 60000 || d->pad_left > 1024 || d->pad_top > 1024) return TVX_E_UNSUPPORTED;
-  // (a window's first column and row lie within the padded input: no place below overflows)
-  a.planes = static_cast<int>(planes);
-  a.total = static_cast<int>(in);
+  a.C = d->in_c;
   a.act = d->activation;
+  const uint64_t planes = static_cast<uint64_t>(d->batch) * d->in_c;
+  if (d->in_c > 60000) return TVX_E_UNSUPPORTED;
 
   // Rows of a thread: four, so that a row is loaded 1.5 times (3x3) or twice (5x5, stride 1) instead of twice or three times - two
   // where four leave the chip short of wavefronts.
   const int px = S == 1 && dt != TVX_F32 ? 8 : 4;
-  a.ncg = (a.OW + px - 1) / px;
-  int R = 4;
-  auto threads = [&](int r) { return planes * a.ncg * ((a.OH + r - 1) / r); };
-  if (threads(4) < 256 * 4 * 64) R = 2;
+  int R = planes * ((d->out_w + px - 1) / px) * ((d->out_h + 3) / 4) < 256 * 4 * 64 ? 2 : 4;
   if (const char* f = getenv("TVX_DWCONV_REG_ROWS")) R = atoi(f) == 2 ? 2 : 4;  // test lever
-  a.tpp = a.ncg * ((a.OH + R - 1) / R);
+  if (!PlanPlaneRows(&a, planes, d->in_h, d->in_w, d->out_h, d->out_w, d->pad_top, d->pad_left, px, R)) return TVX_E_UNSUPPORTED;
+  if (a.total < 12) return TVX_E_UNSUPPORTED;  // (a run of at most twelve elements fits the tensor)
   // whole wavefronts per plane where at most a quarter of their lanes is idle
   const int waves = (a.tpp + 63) / 64;
   const bool uniform = a.tpp * 4 >= waves * 64 * 3;
-  unsigned block = 256;
+  unsigned block = 256, parts = 1;
   if (uniform) {
-    a.bpp = (waves + 3) / 4;
-    block = static_cast<unsigned>((waves + a.bpp - 1) / a.bpp) * 64;
+    parts = static_cast<unsigned>((waves + 3) / 4);
+    block = static_cast<unsigned>((waves + parts - 1) / parts) * 64;
+    if (d->batch > 65535 || parts > 65535) return TVX_E_UNSUPPORTED;
   }
-  const int64_t grid = uniform ? planes * a.bpp : (planes * a.tpp + 255) / 256;
-  if (uniform && (d->batch > 65535 || a.bpp > 65535)) return TVX_E_UNSUPPORTED;
-  if (grid * block >= (int64_t{1} << 31) || in < 12) return TVX_E_UNSUPPORTED;  // (a run of at most twelve elements fits the tensor)
-  if (static_cast<uint64_t>(a.tpp + 256) * std::max(a.tpp, a.ncg) >= (1ull << 32)) return TVX_E_UNSUPPORTED;  // reciprocals are exact below
-  a.m_tpp = Magic(a.tpp);
-  a.m_ncg = Magic(a.ncg);
-  a.m_c = Magic(a.C);
+  a.m_c = Reciprocal(a.C);
 
   int s = TVX_OK;
   if (q) {
@@ -487,7 +348,7 @@ int DwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   if (s != TVX_OK) return s;
   Plan plan{a, nullptr, dim3(1), block, !q || (K == 3 && WholeDwordRows(d)) ? 0u : 15u};
   plan.fn = dt == TVX_I8 ? PickKernel<TVX_I8>(K, S, R, uniform, a.zws != 0) : dt == TVX_F16 ? PickKernel<TVX_F16>(K, S, R, uniform, false) : PickKernel<TVX_F32>(K, S, R, uniform, false);
-  plan.grid = uniform ? dim3(a.C, a.bpp, d->batch) : dim3(static_cast<unsigned>(grid));
+  plan.grid = uniform ? dim3(a.C, parts, d->batch) : dim3(static_cast<unsigned>((planes * a.tpp + 255) / 256));
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
   op->run = DwRegRun;
   op->kernel_name = dt == TVX_I8 ? "dwconv_planes_i8" : dt == TVX_F16 ? "dwconv_reg_f16" : "dwconv_reg_f32";

@@ -509,6 +509,8 @@ int PoolRowsSetup(tvx_op* op) {
   plan.pipelined = pipelined;
   plan.a = a;
   if (!Kernel(&plan)) return TVX_E_UNSUPPORTED;
+  s = PoolRegPlan(op, pipelined ? 15 : 0, a.OW & 3 ? 0 : 3, "pool2d_rows_i8");
+  if (s != TVX_E_UNSUPPORTED) return s;
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
   op->run = PoolRowsRun;
   op->kernel_name = "pool2d_rows_i8";

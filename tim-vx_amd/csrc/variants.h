@@ -93,6 +93,9 @@ int PoolGenericSetup(tvx_op*);
 int PoolRowsSetup(tvx_op*);
 // quantized MAX pooling at stride 2, windows of 2 or 3 taps, rows of whole 8-byte units: register stencil (pool2d_stencil_i8.hip)
 int PoolStencilSetup(tvx_op*);
+// square windows of 2, 3 or side by side 7 taps on planes of any width, every type: register stencil (pool2d_reg.hip)
+int PoolRegSetup(tvx_op*);
+int PoolRegPlan(tvx_op*, unsigned align_in, unsigned align_out, const char* name);
 int TransposeSetup(tvx_op*);
 int ConvertSetup(tvx_op*);
 
