@@ -2,7 +2,7 @@
 // 5x5, int8 / uint8 windows of 5x5 (and of 3x3 on rows that are not whole dwords), at stride 1 or 2 (vxConvolutionLayer's depthwise form; reference:
 // src/tim/vx/internal/src/ops/vsi_nn_op_conv2d.c:35-118).
 //
-// A thread computes two or four output rows x four or eight neighbouring outputs of one plane from rows held in registers
+// A thread computes one, two or four output rows x four or eight neighbouring outputs of one plane from rows held in registers
 // (plane_rows.h).
 // A plane's channel is uniform where its threads fill whole wavefronts (weights then are scalar operands); small planes share
 // wavefronts and keep their weights in vector registers.
@@ -202,14 +202,14 @@ DwRegFn Pick(bool uniform, bool sums) {
     return uniform ? DwRegFloatKernel<DT, K, S, R, true> : DwRegFloatKernel<DT, K, S, R, false>;
   }
 }
+template <int DT, int K, int S>
+DwRegFn PickRows(int r, bool uniform, bool sums) {
+  return r == 4 ? Pick<DT, K, S, 4>(uniform, sums) : r == 2 ? Pick<DT, K, S, 2>(uniform, sums) : Pick<DT, K, S, 1>(uniform, sums);
+}
 template <int DT>
 DwRegFn PickKernel(int k, int s, int r, bool uniform, bool sums) {
-  if (k == 3) {
-    if (s == 1) return r == 4 ? Pick<DT, 3, 1, 4>(uniform, sums) : Pick<DT, 3, 1, 2>(uniform, sums);
-    return r == 4 ? Pick<DT, 3, 2, 4>(uniform, sums) : Pick<DT, 3, 2, 2>(uniform, sums);
-  }
-  if (s == 1) return r == 4 ? Pick<DT, 5, 1, 4>(uniform, sums) : Pick<DT, 5, 1, 2>(uniform, sums);
-  return r == 4 ? Pick<DT, 5, 2, 4>(uniform, sums) : Pick<DT, 5, 2, 2>(uniform, sums);
+  if (k == 3) return s == 1 ? PickRows<DT, 3, 1>(r, uniform, sums) : PickRows<DT, 3, 2>(r, uniform, sums);
+  return s == 1 ? PickRows<DT, 5, 1>(r, uniform, sums) : PickRows<DT, 5, 2>(r, uniform, sums);
 }
 
 struct Plan {
@@ -236,9 +236,8 @@ bool WholeDwordRows(const tvx_conv2d_desc* d) { return d->in_w % 4 == 0 && d->ou
 
 // Which quantized 3x3 layers come here. The stencil for rows of whole dwords gives a row a power of two of lanes: where its outputs fill
 // less than 0.6 of them (132 columns: 33 of 64) it takes 41.8 us against 33.0 (80 channels, 117 x 132, batch 36), else it is ahead (52
-// columns: 12.6 against 14.3). The one that stages planes in LDS: at stride 2 it is never ahead by more than the runs differ (57 x 57, 240
-// channels, batch 44: 26.1 against 13.7 us here), at stride 1 in launches of a few workgroups (25 channels of 14 x 14, batch 2: 3.1 against 3.4;
-// 16 of 69 x 69, batch 2: 4.6 against 3.2; 64 of 93 x 93, batch 43: 29.8 against 21.2).
+// columns: 12.6 against 14.3). The one that stages planes in LDS is behind on all others (25 channels of 14 x 14, batch 2: 3.1 against
+// 2.8 here; 240 of 57 x 57 at stride 2, batch 44, 26.1 against 13.7; 64 of 93 x 93, batch 43, 29.8 against 21.2).
 bool BetterAt3x3(const tvx_conv2d_desc* d) {
   if (WholeDwordRows(d)) {
     if (d->stride_w == 1 && d->in_w % 8 == 0 && d->out_w % 8 == 0) return false;  // (eight columns a lane there)
@@ -247,7 +246,7 @@ bool BetterAt3x3(const tvx_conv2d_desc* d) {
     while (lanes < patches) lanes *= 2;
     return patches * 10 < lanes * 6;
   }
-  return d->stride_w == 2 || static_cast<uint64_t>(d->batch) * d->in_c * d->out_h * d->out_w >= 32768;
+  return true;
 }
 
 float HalfToFloat(uint16_t h) {
@@ -277,11 +276,14 @@ int DwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   const uint64_t planes = static_cast<uint64_t>(d->batch) * d->in_c;
   if (d->in_c > 60000) return TVX_E_UNSUPPORTED;
 
-  // Rows of a thread: four, so that a row is loaded 1.5 times (3x3) or twice (5x5, stride 1) instead of twice or three times - two
-  // where four leave the chip short of wavefronts.
+  // Output rows of a thread: four in registers read a row 1.5 times (3x3) or twice (5x5, stride 1) instead of three or five times, but are a
+  // long chain for few wavefronts. One up to 300000 threads (16 channels of 23 x 25, 3x3: 2.8 us, 3.5 with two, 4.4 with four; 20 x 24 of 48 x
+  // 32 in float32 3.4, 3.9, 4.6), two up to 1.2 million (60 K planes of 7 x 7: 6.4, 6.0, 6.2), four from there on (5 x 288 of 125 x 125 23.1,
+  // 19.3, 17.9; 5x5 on 37 x 341 of 34 x 34 32.6, 29.3, 25.6).
   const int px = S == 1 && dt != TVX_F32 ? 8 : 4;
-  int R = planes * ((d->out_w + px - 1) / px) * ((d->out_h + 3) / 4) < 256 * 4 * 64 ? 2 : 4;
-  if (const char* f = getenv("TVX_DWCONV_REG_ROWS")) R = atoi(f) == 2 ? 2 : 4;  // test lever
+  const uint64_t row_threads = planes * ((d->out_w + px - 1) / px) * d->out_h;
+  int R = row_threads < 300000 ? 1 : row_threads < 1200000 ? 2 : 4;
+  if (const char* f = getenv("TVX_DWCONV_REG_ROWS")) R = atoi(f) == 4 ? 4 : atoi(f) == 2 ? 2 : 1;  // test lever
   if (!PlanPlaneRows(&a, planes, d->in_h, d->in_w, d->out_h, d->out_w, d->pad_top, d->pad_left, px, R)) return TVX_E_UNSUPPORTED;
   if (a.total < 12) return TVX_E_UNSUPPORTED;  // (a run of at most twelve elements fits the tensor)
   // whole wavefronts per plane where at most a quarter of their lanes is idle
