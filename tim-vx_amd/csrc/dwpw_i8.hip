@@ -6,17 +6,22 @@
 // depthwise result is requantized to its own tensor's scale and zero point (and clamped by its fused
 // ReLU / ReLU6) before the pointwise convolution reads it.
 //
-// A workgroup owns RPT whole output rows of one image (at most 128 pixels) for every channel:
-//   1. depthwise phase - the stencil of dwconv3x3_i8: a thread holds four columns x RPT rows of one
-//      channel plane, loads only the dwords under its own columns (the neighbours' come by wavefront
-//      shifts), cuts the windows with v_alignbyte and multiplies with v_dot4; the requantized dwords
-//      (four pixels of one channel) go to an LDS tile in the tensor's own order [channel][pixel];
-//   2. from there the pixel-major operand tile of the matrix cores is built exactly as pwconv_i8 builds
-//      it from global memory (4 x 4 byte transposes in registers, 16-byte LDS stores);
-//   3. pointwise phase - as in pwconv_i8's 32-pixel form: a wavefront owns 32 pixels and walks the 32-channel
-//      output tiles, weights stream from L2 in MFMA-fragment order, results are staged per wavefront and
-//      leave as 16-byte chunks of contiguous WHCN rows; the zero-point term of uint8 weights is a second MFMA
-//      against a constant fragment; a residual Add behind the pointwise convolution rides on the copy-out.
+// A workgroup owns RPT whole output rows of one image for every channel:
+//   1. depthwise phase - a thread holds four columns x RPT rows of four channel planes. A row behind four outputs is loaded as it
+//      lies, from the column in front of them on; windows are cut with v_alignbyte and multiplied with v_dot4. Four requantized
+//      dwords (four pixels of a channel each) are transposed in registers and go straight to the operand tile of the matrix cores,
+//      [pixel slot][channel]; no copy of the tensor in its own order, one barrier;
+//   2. pointwise phase - a wavefront takes 32 pixels x 32 output channels at a time. A tile's pixels are permuted: pixel 4 i + e lies in
+//      slot 8 e + i. The depthwise stores of neighbouring lanes then spread over four times the banks, and a lane finds the sixteen
+//      consecutive pixels of a channel in its accumulators: results are stored from there, sixteen bytes a lane. The zero-point term of
+//      uint8 weights is a second MFMA against a constant fragment; a residual Add behind the pointwise convolution rides on the
+//      results. A last channel tile of at most 16 takes two pixel tiles at once: the second one's weights stand in the
+//      columns that hold no channel, so that no lane requantizes nothing.
+// Bound by the vector ALU in large batches (about 15 instructions a depthwise result, 11 a pointwise one) and by the chain load -
+// windows - barrier - MFMA - store in small ones. uint8, before (codes staged in the tensor's order, the operand tile built from them
+// behind a second barrier, results staged per wavefront) and now, microseconds: 112 x 112, 32 to 16: batch 1 5.0 / 4.6, batch 64 32.9 / 24.6;
+// 56 x 56, 144 to 24: 8.1 / 6.9, 36.1 / 30.3; 28 x 28, 144 to 32, stride 2: 9.2 / 5.0, 15.2 / 13.5; 28 x 28, 192 to 32: 9.3 / 6.4, 15.6 / 14.6;
+// int8 112 x 112, 32 to 64, batch 32: 22.5 / 20.0. (Two pixel tiles at once: 25.7 -> 24.6 in the first of these.)
 #include <algorithm>
 #include <cstdlib>
 
@@ -28,35 +33,33 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
-constexpr int kWaves = 4, kMaxWaves = 8;  // of a workgroup
-constexpr int kMaxSlots = 512;      // most pixel slots of a tile (32-pixel MFMA tiles, a multiple of four of them)
-constexpr int kStageStride = 40;    // bytes per staged output row of 32 pixels (8-byte aligned rows)
-constexpr int kStageBytes = 32 * kStageStride;
+constexpr int kWaves = 4, kMaxWaves = 8;  // of a workgroup: many tiles, few tiles
+constexpr int kMaxSlots = 512;            // most pixels of a tile
+constexpr int kWeightBytes = 64 * 1024;   // most weights that are copied to LDS
 
 struct DwPwArgs {
   const uint8_t* x;      // depthwise input {W, H, C, N}
-  uint8_t* y;            // pointwise output {OW, OH, OC, N}
-  // ---- depthwise part (tables as in dwconv3x3_i8)
-  const int32_t* dw_wpk;
-  const int32_t* dw_biasf;
-  const tvx_v4i* dw_rq;
-  int C, H, W, OH, OW;
-  int pad_t;
-  int ow4, lpr_shift;
-  int dw_xor_mask, dw_pad_fill, dw_zws, dw_out_zp, dw_lo, dw_hi;
-  int dw_box;            // the depthwise weights are packed unshifted: the window sum carries their zero point
-  int dw_ties, pw_ties;  // whether an accumulator of the depthwise / pointwise convolution can land on an exact .5
-  uint32_t c4n_magic;    // ceil(2^32 / (cp / 4)): a division by multiply-high
-  // ---- pointwise part (tables as in pwconv_i8)
-  const v4i* wpk;
+  // ---- depthwise part
+  const v4i* dw;         // per channel: {three rows of taps, folded bias}, {multiplier, shift and tie bit, rounding constant, -}
+  int C, H, W, OW, batch;
+  int pad_t, ow4, lpr_shift, quads;  // quads: channels in fours
+  int tiles_per_image;
+  uint32_t m_tiles;      // reciprocal
+  int dw_xor_mask, dw_pad_fill;
+  int dw_nzws, dw_nzws3;  // minus the weights' zero point where they are packed unshifted (the window sum carries it), else 0; in three bytes
+  int dw_pre_ties, dw_lo, dw_hi, dw_narrow;
+  // ---- pointwise part
+  const v4i* wpk;        // [32-channel tile][step][64 lanes]
   const int32_t* biasf;
   const v4i* rq;
-  int OC, cp, ksteps, pix_stride, oc_tiles;
-  int xor_mask, neg_zws4, zp;
-  int out_zp, lo, hi;
+  int cp, ksteps, pix_stride, oc_tiles, ptiles;
+  int paired;            // the last 32-channel tile holds at most 16 channels: it takes two pixel tiles at a time
+  int off_w, off_rq, off_bias;  // LDS behind the operand tile
+  int neg_zws4, zp, last_channels;  // last_channels: of the last reduction step
   int P;                 // pixels of a tile: RPT * OW
-  int slots;             // P rounded up to a multiple of 128
-  int tiles_per_image;
+  uint8_t* y;            // pointwise output {OW, OH, OC, N}
+  int OC, hw;
+  int pre_ties, lo, hi, narrow, out_xor;
   // ---- fused residual Add behind the pointwise convolution (0 = off), as in pwconv_i8
   const uint8_t* res;
   double add_ra, add_rb;
@@ -64,116 +67,27 @@ struct DwPwArgs {
   int add_za, add_zb, add_zo, add_lo, add_hi;
 };
 
-// Four columns x RPT output rows of one depthwise channel plane, in two steps so that the loads of several
-// channels can be in flight together; S = stride, PL = left padding.
-template <int S, int RPT>
-struct PatchShape {
-  static constexpr int kOwn = S;                    // input dwords under a thread's four outputs
-  static constexpr int kRows = S * (RPT - 1) + 3;   // input rows behind its output rows
-};
-
-template <int S, int RPT>
-__device__ __forceinline__ void PatchLoad(const DwPwArgs& a, const uint8_t* xn, uint32_t plane_off, int w4, int oh0,
-                                          int (&raw)[PatchShape<S, RPT>::kRows][PatchShape<S, RPT>::kOwn + 2]) {
-  constexpr int kOwn = PatchShape<S, RPT>::kOwn, kRows = PatchShape<S, RPT>::kRows;
-  const int in_dwords = a.W / 4;
-  const int d0 = S * w4;
-  const int ih0 = oh0 * S - a.pad_t;
-  // xn: the image (uniform), plane_off: the channel plane inside it; offsets inside an image fit 32 bits (checked at
-  // creation): one scalar base + one vector offset per load. Rows outside the image read the nearest row inside.
+// Four codes of one channel, in the signed domain. PLAIN: no accumulator on a tie or to be shifted, and a clamp no narrower than a byte.
+template <bool PLAIN>
+__device__ __forceinline__ uint32_t Codes(int (&v)[4], const v4i& q, int64_t round, int pre_ties, int narrow, int lo, int hi) {
+  const int sh = q[1] & 31;
+  if constexpr (PLAIN) return RequantSaturate4<false>(v, q[0], sh, round, 0, 0);
+  if (pre_ties) {  // (uniform)
 #pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    const int ihc = min(max(ih0 + r, 0), a.H - 1);
-    const uint32_t row_off = plane_off + __umul24(static_cast<uint32_t>(ihc), static_cast<uint32_t>(a.W));
-#pragma unroll
-    for (int i = 0; i < kOwn; ++i)  // unconditional: masked later
-      raw[r][1 + i] = *reinterpret_cast<const int*>(xn + (row_off + static_cast<uint32_t>(min(d0 + i, in_dwords - 1)) * 4u));
+    for (int e = 0; e < 4; ++e) v[e] <<= pre_ties >> 1;
+    if (pre_ties & 1) LowerOddTies(v, q);
   }
+  return narrow ? RequantSaturate4<true>(v, q[0], sh, round, lo << sh, ((hi + 1) << sh) - 1) : RequantSaturate4<false>(v, q[0], sh, round, 0, 0);
 }
 
-// A depthwise channel's constants: three rows of taps (a dword each), the folded bias, the requantization record.
-struct ChannelConsts {
-  v4i taps;  // (the fourth dword is not used here)
-  int bias;
-  v4i q;
-};
+constexpr int kPlain = 0, kPlainBox = 1, kAny = 2;  // requantizations without ties and narrow clamps; ... and window sums; decided at run time
 
-__device__ __forceinline__ ChannelConsts LoadChannelConsts(const DwPwArgs& a, int c) {
-  ChannelConsts k;
-  k.taps = *reinterpret_cast<const v4i*>(a.dw_wpk + c * 4);
-  k.bias = a.dw_biasf[c];
-  k.q = a.dw_rq[c];
-  return k;
-}
-
-template <int S, int PL, int RPT>
-__device__ __forceinline__ void PatchCompute(const DwPwArgs& a, const ChannelConsts& k, int w4, int oh0,
-                                             int (&raw)[PatchShape<S, RPT>::kRows][PatchShape<S, RPT>::kOwn + 2],
-                                             uint32_t (&packed)[RPT]) {
-  constexpr int kOwn = PatchShape<S, RPT>::kOwn, kRows = PatchShape<S, RPT>::kRows;
-  const int wk0 = k.taps[0], wk1 = k.taps[1], wk2 = k.taps[2];
-  const bool box = a.dw_box != 0;  // (wave-uniform: a branch, not a mask)
-  const int bias = k.bias;
-  const v4i q = k.q;
-  const int in_dwords = a.W / 4;
-  const int d0 = S * w4;
-  const int ih0 = oh0 * S - a.pad_t;
-  const bool has_left = w4 > 0;
-  const bool has_right = d0 + kOwn < in_dwords;
-#pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    const int ih = ih0 + r;
-    const int keep_row = (ih >= 0 && ih < a.H) ? -1 : 0;
-#pragma unroll
-    for (int i = 0; i < kOwn; ++i) {
-      const int keep = d0 + i < in_dwords ? keep_row : 0;
-      raw[r][1 + i] = ((raw[r][1 + i] ^ a.dw_xor_mask) & keep) | (a.dw_pad_fill & ~keep);
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    // (the wavefront's first / last lane has no such neighbour; it is the first / last lane of an image row and takes the padding)
-    const int l = __builtin_amdgcn_mov_dpp(raw[r][kOwn], 0x138, 0xf, 0xf, true);
-    const int rr = __builtin_amdgcn_mov_dpp(raw[r][1], 0x130, 0xf, 0xf, true);
-    raw[r][0] = has_left ? l : a.dw_pad_fill;
-    raw[r][kOwn + 1] = has_right ? rr : a.dw_pad_fill;
-  }
-#pragma unroll
-  for (int o = 0; o < RPT; ++o) {
-    int win[3][4];
-#pragma unroll
-    for (int r = 0; r < 3; ++r) {
-      win[r][0] = Window<4 + S * 0 - PL>(raw[S * o + r]);
-      win[r][1] = Window<4 + S * 1 - PL>(raw[S * o + r]);
-      win[r][2] = Window<4 + S * 2 - PL>(raw[S * o + r]);
-      win[r][3] = Window<4 + S * 3 - PL>(raw[S * o + r]);
-    }
-    int accs[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      int acc = Dot4Add(win[0][i], wk0, bias);
-      acc = __builtin_amdgcn_sdot4(win[1][i], wk1, acc, false);
-      acc = __builtin_amdgcn_sdot4(win[2][i], wk2, acc, false);
-      if (box) {
-        int sx = __builtin_amdgcn_sdot4(win[0][i], 0x00010101, 0, false);
-        sx = __builtin_amdgcn_sdot4(win[1][i], 0x00010101, sx, false);
-        sx = __builtin_amdgcn_sdot4(win[2][i], 0x00010101, sx, false);
-        acc -= a.dw_zws * sx;
-      }
-      accs[i] = acc;
-    }
-    packed[o] = Requant8x4Pack(accs, q, a.dw_out_zp, a.dw_lo, a.dw_hi, a.dw_ties);
-  }
-}
-
-// S: stride of the depthwise convolution (left padding 1 at stride 1, 0 at stride 2: SAME);
-// RPT: output rows of a tile.
-// (two wavefronts per SIMD at least: within 256 registers the compiler keeps MFMA accumulators in ordinary vector
-// registers, where the epilogue reads them, instead of moving every value out of the accumulation registers first)
-template <int S, int RPT, bool ADD>
-__global__ void __launch_bounds__(kMaxWaves * 64) __attribute__((amdgpu_waves_per_eu(2))) DwPwKernel(DwPwArgs a) {
+// S: stride of the depthwise convolution (left padding 1 at stride 1, 0 at stride 2: SAME); RPT: output rows of a tile;
+// WLDS: the pointwise weights are copied to LDS; FLAVOUR: above.
+template <int S, int RPT, bool ADD, bool WLDS, int FLAVOUR>
+__global__ void __launch_bounds__(kMaxWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) DwPwKernel(DwPwArgs a) {
   extern __shared__ __attribute__((aligned(16))) int8_t lds[];
-  constexpr int PL = S == 1 ? 1 : 0;
+  constexpr int kRows = S * (RPT - 1) + 3;  // input rows behind a thread's output rows; its dwords of each: S
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), threads = blockDim.x, waves = threads >> 6;
   // an XCD gets a contiguous run of tiles: vertically neighbouring tiles share input rows in its L2
@@ -182,162 +96,242 @@ __global__ void __launch_bounds__(kMaxWaves * 64) __attribute__((amdgpu_waves_pe
     const int per = gridDim.x >> 3, rem = gridDim.x & 7, xcd = wg & 7;
     wg = xcd * per + min(xcd, rem) + (wg >> 3);
   }
-  const int n = wg / a.tiles_per_image;
+  const uint32_t one = a.m_tiles ? 0u : ~0u;
+  const int n = static_cast<int>(__umulhi(static_cast<uint32_t>(wg), a.m_tiles) + (static_cast<uint32_t>(wg) & one));
   const int g = wg - n * a.tiles_per_image;
-  const int oh0 = g * RPT;
-  const int hw = a.OH * a.OW;
-  const int mid_stride = a.slots + 4;              // bytes per channel row of the depthwise tile (+ 4: bank spread)
-  int8_t* mid = lds;                               // [channel][slots + 4]: the depthwise result of the tile
-  int8_t* xl = lds + a.cp * mid_stride;            // [pixel slot][pix_stride]: the MFMA operand tile
-  int8_t* stage = xl + a.slots * a.pix_stride + wave * kStageBytes;
-  int8_t* w_lds = xl + a.slots * a.pix_stride + waves * kStageBytes;  // the pointwise weights, in fragment order
-  const int oc_alloc = a.oc_tiles * 32;
-  v4i* rq_lds = reinterpret_cast<v4i*>(w_lds + oc_alloc * a.cp);
-  int* bias_lds = reinterpret_cast<int*>(rq_lds + oc_alloc);
+  const int oh0 = g * RPT, ih0 = oh0 * S - a.pad_t;
 
   // ---- the pointwise weights and the epilogue's tables: global -> LDS by DMA, under the depthwise phase ----
   {
     typedef const __attribute__((address_space(1))) void* gptr;
     typedef __attribute__((address_space(3))) void* lptr;
-    const int chunks = oc_alloc * a.cp >> 4;
-    for (int i = wave * 64; i < chunks; i += threads)
-      if (i + lane < chunks)
-        __builtin_amdgcn_global_load_lds((gptr)(a.wpk + i + lane), (lptr)(w_lds + i * 16), 16, 0, 0);
+    const int oc_alloc = a.oc_tiles * 32, chunks = oc_alloc * a.cp >> 4;
+    if (WLDS)
+      for (int i = wave * 64; i < chunks; i += threads)
+        if (i + lane < chunks) __builtin_amdgcn_global_load_lds((gptr)(a.wpk + i + lane), (lptr)(lds + a.off_w + i * 16), 16, 0, 0);
     for (int i = wave * 64; i < oc_alloc; i += threads)
       if (i + lane < oc_alloc) {
-        __builtin_amdgcn_global_load_lds((gptr)(a.rq + i + lane), (lptr)(rq_lds + i), 16, 0, 0);
-        __builtin_amdgcn_global_load_lds((gptr)(a.biasf + i + lane), (lptr)(bias_lds + i), 4, 0, 0);
+        __builtin_amdgcn_global_load_lds((gptr)(a.rq + i + lane), (lptr)(lds + a.off_rq + i * 16), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((gptr)(a.biasf + i + lane), (lptr)(lds + a.off_bias + i * 4), 4, 0, 0);
       }
   }
 
-  // ---- 1. depthwise: (channel, four columns) per thread and pass, RPT rows; the loads of several passes
-  // are issued together (a pass on its own would be one memory round trip each) ----
+  // ---- 1. depthwise: (four channels, four columns) per thread and pass, RPT rows. A row behind four outputs is the bytes from the
+  // column in front of them on (stride 1: eight; stride 2 needs none in front: twelve), loaded as they lie: what is no column of the row is
+  // masked. (x & keep) ^ flip is that and the move to the signed domain in one instruction. ----
   {
-    constexpr int kRows = PatchShape<S, RPT>::kRows, kOwn = PatchShape<S, RPT>::kOwn;
-    constexpr int kBatch = (24 / (kRows * kOwn)) > 8 ? 8 : ((24 / (kRows * kOwn)) < 1 ? 1 : (24 / (kRows * kOwn)));
+    constexpr int kDw = S + 1;
     const int w4 = tid & ((1 << a.lpr_shift) - 1);
-    const int per_pass = threads >> a.lpr_shift;
-    const size_t plane = static_cast<size_t>(a.H) * a.W;
-    const uint32_t plane32 = static_cast<uint32_t>(plane);
-    const uint8_t* xn = a.x + static_cast<size_t>(n) * a.C * plane;
-    for (int c0 = tid >> a.lpr_shift; c0 < a.C; c0 += per_pass * kBatch) {
-      int raw[kBatch][kRows][kOwn + 2];
-      ChannelConsts consts[kBatch];
+    const uint32_t plane = static_cast<uint32_t>(a.H) * static_cast<uint32_t>(a.W);
+    const uint8_t* xn = a.x + static_cast<size_t>(n) * a.C * plane - 4;  // (offsets inside an image fit 32 bits)
+    const uint32_t image = static_cast<uint32_t>(a.C) * plane;
+    const int col = 4 * S * min(w4, a.ow4 - 1) - (S == 1 ? 1 : 0);
+    int keep[kDw], flip[kDw];
 #pragma unroll
-      for (int b = 0; b < kBatch; ++b) {
-        const int c = min(c0 + b * per_pass, a.C - 1);
-        PatchLoad<S, RPT>(a, xn, static_cast<uint32_t>(c) * plane32, w4, oh0, raw[b]);
-        consts[b] = LoadChannelConsts(a, c);
+    for (int i = 0; i < kDw; ++i) {
+      uint32_t k = ~0u;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (static_cast<unsigned>(col + 4 * i + e) >= static_cast<unsigned>(a.W)) k &= ~(0xffu << (8 * e));
+      keep[i] = static_cast<int>(k);
+      flip[i] = (a.dw_xor_mask & keep[i]) | (a.dw_pad_fill & ~keep[i]);
+    }
+    // a run that would leave the tensor, at its first and its last bytes, is read from inside it
+    const uint32_t lowest = n == 0 ? 4u : 0u, highest = n == a.batch - 1 ? image + 4u - 4u * kDw : ~0u;
+    for (int c4 = tid >> a.lpr_shift; c4 < a.quads; c4 += threads >> a.lpr_shift) {
+      int raw[4][kRows][kDw];
+      int moved = 0;
+      v4i taps[4], q[4];
+#pragma unroll
+      for (int r = 0; r < kRows; ++r) {
+        const int ih = ih0 + r;
+        if (ih >= 0 && ih < a.H) {  // (uniform)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const uint32_t at = static_cast<uint32_t>(min(4 * c4 + j, a.C - 1)) * plane + static_cast<uint32_t>(ih) * static_cast<uint32_t>(a.W) + static_cast<uint32_t>(col + 4);
+            const uint32_t in = min(max(at, lowest), highest);
+            moved |= static_cast<int>(in - at);
+            __builtin_memcpy(raw[j][r], xn + in, 4 * kDw);
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < kDw; ++i) raw[j][r][i] = a.dw_pad_fill ^ a.dw_xor_mask;
+        }
       }
 #pragma unroll
-      for (int b = 0; b < kBatch; ++b) {
-        const int c = c0 + b * per_pass;
-        if (c < a.C) {  // whole image rows of lanes take this branch together
-          uint32_t packed[RPT];
-          PatchCompute<S, PL, RPT>(a, consts[b], w4, oh0, raw[b], packed);
-          if (w4 < a.ow4) {
+      for (int j = 0; j < 4; ++j) {
+        const int c = min(4 * c4 + j, a.C - 1);
+        taps[j] = a.dw[2 * c];
+        q[j] = a.dw[2 * c + 1];
+      }
+      if (__ballot(moved)) {  // (the first and the last workgroup)
 #pragma unroll
-            for (int o = 0; o < RPT; ++o)
-              *reinterpret_cast<uint32_t*>(mid + c * mid_stride + o * a.OW + w4 * 4) = packed[o];
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int r = 0; r < kRows; ++r) {
+            const int ih = ih0 + r;
+            if (ih < 0 || ih >= a.H) continue;
+            const uint32_t at = static_cast<uint32_t>(min(4 * c4 + j, a.C - 1)) * plane + static_cast<uint32_t>(ih) * static_cast<uint32_t>(a.W) + static_cast<uint32_t>(col + 4);
+            const int by = static_cast<int>(min(max(at, lowest), highest) - at);
+            if constexpr (S == 1) {  // one byte up or three down
+              const uint64_t v = static_cast<uint64_t>(static_cast<uint32_t>(raw[j][r][1])) << 32 | static_cast<uint32_t>(raw[j][r][0]);
+              const uint64_t w = by > 0 ? v << 8 : by < 0 ? v >> 24 : v;
+              raw[j][r][0] = static_cast<int>(w);
+              raw[j][r][1] = static_cast<int>(w >> 32);
+            } else {  // a dword down
+              const int down = by ? ~0 : 0;
+              raw[j][r][0] = (raw[j][r][1] & down) | (raw[j][r][0] & ~down);
+              raw[j][r][1] = (raw[j][r][2] & down) | (raw[j][r][1] & ~down);
+            }
           }
+      }
+      uint32_t codes[RPT][4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        int acc[RPT][4], sum[RPT][4];
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) {
+          int d[kDw + 1];
+          d[kDw] = 0;
+#pragma unroll
+          for (int i = 0; i < kDw; ++i) d[i] = S == 2 && i < 2 ? raw[j][r][i] ^ a.dw_xor_mask : (raw[j][r][i] & keep[i]) ^ flip[i];
+          int win[4];
+          win[0] = Window<0>(d);
+          win[1] = Window<S>(d);
+          win[2] = Window<2 * S>(d);
+          win[3] = Window<3 * S>(d);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int o = 0; o < RPT; ++o) {
+              const int ky = r - S * o;
+              if (ky < 0 || ky > 2) continue;
+              acc[o][i] = ky == 0 ? Dot4Add(win[i], taps[j][0], taps[j][3]) : __builtin_amdgcn_sdot4(win[i], taps[j][ky], acc[o][i], false);
+              if (FLAVOUR == kPlainBox) acc[o][i] = __builtin_amdgcn_sdot4(win[i], a.dw_nzws3, acc[o][i], false);
+              if (FLAVOUR == kAny) sum[o][i] = __builtin_amdgcn_sdot4(win[i], 0x00010101, ky == 0 ? 0 : sum[o][i], false);
+            }
+          }
+        }
+        const int64_t round = RoundHigh(q[j][2]);
+#pragma unroll
+        for (int o = 0; o < RPT; ++o) {
+          if (FLAVOUR == kAny)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[o][i] += __mul24(a.dw_nzws, sum[o][i]);
+          codes[o][j] = Codes<FLAVOUR != kAny>(acc[o], q[j], round, a.dw_pre_ties, a.dw_narrow, a.dw_lo, a.dw_hi);
+        }
+      }
+      if (w4 < a.ow4) {
+#pragma unroll
+        for (int o = 0; o < RPT; ++o) {
+          uint32_t t[4];
+          Transpose4x4(codes[o], t);
+          const int p4 = o * a.ow4 + w4;
+          int8_t* to = lds + __mul24((p4 >> 3) * 32 + (p4 & 7), a.pix_stride) + 4 * c4;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) *reinterpret_cast<uint32_t*>(to + 8 * e * a.pix_stride) = t[e];
         }
       }
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the DMA above)
   __syncthreads();
-  // ---- 2. [channel][pixel] -> [pixel][channel]: a thread turns four channels of four pixels ----
-  {
-    const int c4n = a.cp >> 2;                 // (a multiple of 8)
-    const int items = (a.slots >> 2) * c4n;
-    for (int it = tid; it < items; it += threads) {
-      const int pq = __umulhi(it, a.c4n_magic), c4 = it - pq * c4n;
-      const bool live = pq * 4 < a.P;
-      uint32_t raw[4], t[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int c = c4 * 4 + j;
-        const uint32_t v = *reinterpret_cast<const uint32_t*>(mid + min(c, a.C - 1) * mid_stride + pq * 4);
-        raw[j] = (live && c < a.C) ? v ^ a.xor_mask : 0u;
-      }
-      Transpose4x4(raw, t);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        *reinterpret_cast<uint32_t*>(xl + (pq * 4 + e) * a.pix_stride + c4 * 4) = t[e];
-    }
-  }
-  __syncthreads();
 
-  // ---- 3. pointwise: a wavefront takes 32 pixel slots at a time and walks every output tile ----
-  const int frag_row = lane & 31, frag_half = lane >> 5;
-  const v4i fz = {a.neg_zws4, a.neg_zws4, a.neg_zws4, a.neg_zws4};
-  for (int part0 = (wave & 3) * 32; part0 < a.P; part0 += 128) {
-    // copy-out mapping of a staged 32 x 32 patch: lane -> 16-pixel chunk lane & 1 of output-channel row lane >> 1
-    const int px_in_row = part0 + (lane & 1) * 16;
-    const bool out_live = px_in_row < a.P;
-    const size_t out_off = static_cast<size_t>(n) * a.OC * hw + static_cast<size_t>(g) * a.P + px_in_row;
-    const int8_t* xa = xl + (part0 + frag_row) * a.pix_stride + frag_half * 16;
-    for (int tile = wave >> 2; tile < a.oc_tiles; tile += waves >> 2) {  // (the second four wavefronts take every other tile)
-      const v4i q = rq_lds[tile * 32 + frag_row];
-      const int nb = bias_lds[tile * 32 + frag_row];
-      v16i acc;
+  // ---- 2. pointwise: a wavefront takes 32 pixel slots x 32 output channels at a time ----
+  const DwPwArgs& b = LateArgs<DwPwArgs>();
+  const int row = lane & 31, half = lane >> 5;
+  const v4i fz = {b.neg_zws4, b.neg_zws4, b.neg_zws4, b.neg_zws4};
+  v4i fz_last;  // (what lies behind the channels in their last step counts for no sum)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[r] = nb;
-      const v4i* wf = reinterpret_cast<const v4i*>(w_lds) + tile * a.ksteps * 64 + lane;
-      v4i fw = wf[0], fx = *reinterpret_cast<const v4i*>(xa);
-      for (int k = 0; k < a.ksteps; ++k) {
-        const int kn = min(k + 1, a.ksteps - 1);
-        const v4i fw1 = wf[kn * 64];
-        const v4i fx1 = *reinterpret_cast<const v4i*>(xa + kn * 32);
-        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fx, fw, acc, 0, 0, 0);
-        if (a.zp) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fx, fz, acc, 0, 0, 0);
-        fw = fw1; fx = fx1;
-      }
-      // ---- epilogue: the residual operand first (it travels while the results are requantized) ----
-      const int rows = min(32, a.OC - tile * 32);
-      const int row = lane >> 1;
-      const size_t at = out_off + (static_cast<size_t>(tile) * 32 + row) * hw;
-      uint4 res16 = make_uint4(0, 0, 0, 0);
-      if (ADD && row < rows && out_live) res16 = *reinterpret_cast<const uint4*>(a.res + at);
-#pragma unroll
-      for (int gq = 0; gq < 4; ++gq) {
-        const int pl = 8 * gq + 4 * frag_half;
-        const int av[4] = {acc[gq * 4], acc[gq * 4 + 1], acc[gq * 4 + 2], acc[gq * 4 + 3]};
-        *reinterpret_cast<uint32_t*>(stage + frag_row * kStageStride + pl) = Requant8x4Pack(av, q, a.out_zp, a.lo, a.hi, a.pw_ties);
-      }
-      __builtin_amdgcn_wave_barrier();
-      {
-        const int8_t* sp = stage + row * kStageStride + (lane & 1) * 16;
-        const uint2 lo8 = *reinterpret_cast<const uint2*>(sp);
-        const uint2 hi8 = *reinterpret_cast<const uint2*>(sp + 8);
-        if (row < rows && out_live) {
-          uint4 o = make_uint4(lo8.x, lo8.y, hi8.x, hi8.y);
-          if (ADD)
-            o = make_uint4(AddResidual4(a, o.x, res16.x), AddResidual4(a, o.y, res16.y), AddResidual4(a, o.z, res16.z),
-                           AddResidual4(a, o.w, res16.w));
-          *reinterpret_cast<uint4*>(a.y + at) = o;
-        }
-      }
-      __builtin_amdgcn_wave_barrier();
+  for (int i = 0; i < 4; ++i) {
+    const int left = b.last_channels - 16 * half - 4 * i;
+    fz_last[i] = left >= 4 ? fz[i] : left <= 0 ? 0 : fz[i] & static_cast<int>((1u << (8 * left)) - 1u);
+  }
+  int ot = 0, pair = b.oc_tiles == 1 ? b.paired : 0, tasks = b.ptiles;
+  if (pair) tasks = (b.ptiles + 1) >> 1;
+  for (int task = wave; ; task += waves) {
+    while (task >= tasks) {
+      task -= tasks;
+      if (++ot == b.oc_tiles - 1 && b.paired) { pair = 1; tasks = (b.ptiles + 1) >> 1; }
     }
+    if (ot >= b.oc_tiles) break;
+    const int pt = task << pair, second = pair ? row & 16 : 0;
+    const int oc = ot * 32 + row - second, p0 = (pt + (second >> 4)) * 32 + 16 * half;
+    const bool live = oc < b.OC && p0 < b.P, whole = p0 + 16 <= b.P;
+    const size_t at = (static_cast<size_t>(n) * b.OC + oc) * b.hw + static_cast<size_t>(g) * b.P + p0;
+    uint32_t res[4] = {0, 0, 0, 0};
+    if (ADD && live) {
+      if (whole) __builtin_memcpy(res, b.res + at, 16);
+      else
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+          if (p0 + 4 * e < b.P) __builtin_memcpy(&res[e], b.res + at + 4 * e, 4);
+    }
+    const v4i q = *reinterpret_cast<const v4i*>(lds + b.off_rq + oc * 16);
+    const int bias = *reinterpret_cast<const int*>(lds + b.off_bias + oc * 4);
+    v16i acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = bias;
+    const int8_t* xa = lds + (pt * 32 + row) * b.pix_stride + half * 16;
+    const int8_t* wl = lds + b.off_w + (ot * b.ksteps * 64 + lane) * 16;
+    const v4i* wg4 = b.wpk + static_cast<size_t>(ot) * b.ksteps * 64 + lane;
+    auto weights = [&](int k) { return WLDS ? *reinterpret_cast<const v4i*>(wl + k * 1024) : wg4[k * 64]; };
+    // at most 16 channels: two pixel tiles at once, the second one's results in the columns that hold no channel
+    const int8_t* xb = xa + (pt + 1 < b.ptiles ? 32 * b.pix_stride : 0);
+    auto weights2 = [&](int k) { return WLDS ? *reinterpret_cast<const v4i*>(wl + k * 1024 + (second ? -256 : 256)) : wg4[k * 64 + (second ? -16 : 16)]; };
+    const int upper = second ? ~0 : 0, lower = ~upper;
+    v4i fw = weights(0), fx = *reinterpret_cast<const v4i*>(xa);
+    for (int k = 0; k < b.ksteps; ++k) {
+      const int kn = min(k + 1, b.ksteps - 1);
+      const v4i fw1 = weights(kn);
+      const v4i fx1 = *reinterpret_cast<const v4i*>(xa + kn * 32);
+      acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fx, fw, acc, 0, 0, 0);
+      if (b.zp) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fx, (k + 1 < b.ksteps ? fz : fz_last) & lower, acc, 0, 0, 0);
+      if (pair) {  // (uniform)
+        const v4i fx2 = *reinterpret_cast<const v4i*>(xb + k * 32);
+        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fx2, weights2(k), acc, 0, 0, 0);
+        if (b.zp) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fx2, (k + 1 < b.ksteps ? fz : fz_last) & upper, acc, 0, 0, 0);
+      }
+      fw = fw1; fx = fx1;
+    }
+    // accumulator 4 e + i is slot 8 e + 4 half + i: pixel 16 half + 4 i + e of the tile
+    uint32_t out[4];
+    const int64_t round = RoundHigh(q[2]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      int v[4] = {acc[i], acc[4 + i], acc[8 + i], acc[12 + i]};
+      out[i] = Codes<FLAVOUR != kAny>(v, q, round, b.pre_ties, b.narrow, b.lo, b.hi) ^ static_cast<uint32_t>(b.out_xor);
+      if (ADD) out[i] = AddResidual4(b, out[i], res[i]);
+    }
+    if (!live) continue;
+    if (whole) __builtin_memcpy(b.y + at, out, 16);
+    else
+#pragma unroll
+      for (int e = 0; e < 3; ++e)
+        if (p0 + 4 * e < b.P) __builtin_memcpy(b.y + at + 4 * e, &out[e], 4);
   }
 }
 
 struct Plan {
   DwPwArgs a;
-  int lds_bytes, stride, rpt, block;
+  void (*fn)(DwPwArgs);
+  int lds_bytes, block;
   dim3 grid;
 };
 
 typedef void (*DwPwFn)(DwPwArgs);
 
-template <bool ADD>
+template <bool ADD, bool WLDS, int FLAVOUR>
 DwPwFn KernelOf(int stride, int rpt) {
-  if (stride == 1) return rpt == 4 ? DwPwKernel<1, 4, ADD> : (rpt == 2 ? DwPwKernel<1, 2, ADD> : DwPwKernel<1, 1, ADD>);
-  return rpt == 4 ? DwPwKernel<2, 4, ADD> : (rpt == 2 ? DwPwKernel<2, 2, ADD> : DwPwKernel<2, 1, ADD>);
+  if (stride == 1) return rpt == 4 ? DwPwKernel<1, 4, ADD, WLDS, FLAVOUR> : (rpt == 2 ? DwPwKernel<1, 2, ADD, WLDS, FLAVOUR> : DwPwKernel<1, 1, ADD, WLDS, FLAVOUR>);
+  return rpt == 2 ? DwPwKernel<2, 2, ADD, WLDS, FLAVOUR> : DwPwKernel<2, 1, ADD, WLDS, FLAVOUR>;
 }
-DwPwFn Kernel(int stride, int rpt, bool add) {
-  return add ? KernelOf<true>(stride, rpt) : KernelOf<false>(stride, rpt);
+template <bool ADD>
+DwPwFn KernelOf(int stride, int rpt, bool wlds, int flavour) {
+  if (!wlds) return KernelOf<ADD, false, kAny>(stride, rpt);
+  return flavour == kPlain ? KernelOf<ADD, true, kPlain>(stride, rpt) : flavour == kPlainBox ? KernelOf<ADD, true, kPlainBox>(stride, rpt) : KernelOf<ADD, true, kAny>(stride, rpt);
 }
 
 int DwPwRun(tvx_op* op, const void* in0, const void* in1, void* out, hipStream_t st) {
@@ -349,7 +343,7 @@ int DwPwRun(tvx_op* op, const void* in0, const void* in1, void* out, hipStream_t
   if (a.add_mode && !in1) return SetError(TVX_E_INVALID, "dwpw_i8: the fused Add needs its second operand as in1");
   if ((reinterpret_cast<uintptr_t>(in0) & 3) | ((reinterpret_cast<uintptr_t>(out) | (a.add_mode ? reinterpret_cast<uintptr_t>(in1) : 0)) & 15))
     return SetError(TVX_E_INVALID, "dwpw_i8: the input must be 4-byte, the output (and the Add's operand) 16-byte aligned");
-  hipLaunchKernelGGL(Kernel(plan->stride, plan->rpt, a.add_mode != 0), plan->grid, dim3(plan->block), plan->lds_bytes, st, a);
+  hipLaunchKernelGGL(plan->fn, plan->grid, dim3(plan->block), plan->lds_bytes, st, a);
   TVX_HIP_CHECK(hipGetLastError());
   return TVX_OK;
 }
@@ -383,76 +377,88 @@ int DwPwSetup(tvx_op* op, const tvx_conv2d_desc* dw, const void* dw_w, const voi
       pw->out_w != pw->in_w || pw->out_h != pw->in_h || pw->in_dtype != dw->out_dtype ||
       pw->in_scale != dw->out_scale || pw->in_zp != dw->out_zp)
     return TVX_E_UNSUPPORTED;
-  // ---- tile: whole rows, at most kMaxSlots pixels, 16-byte chunks ----
-  // (as many rows as keep the tile's LDS image - depthwise tile, operand tile, staging - within a third of a CU's)
+  // ---- which pairs: those with whole rows of at most kMaxSlots pixels that make 16-byte chunks, up to this much LDS (larger ones: two
+  // kernels) ----
   const int cp_ = RoundUp(static_cast<int>(dw->in_c), 32);
   const int oc_alloc_ = RoundUp(static_cast<int>(pw->out_c), 32);
-  auto lds_of = [&](int r) {
-    const int slots = RoundUp(r * static_cast<int>(dw->out_w), 128);
-    return cp_ * (slots + 4) + slots * (cp_ + 16) + 4 * kStageBytes + oc_alloc_ * (cp_ + 20);
-  };
-  auto fits = [&](int r) {
-    return r * dw->out_w <= static_cast<uint32_t>(kMaxSlots) && dw->out_h % r == 0 && (r * dw->out_w) % 16 == 0;
-  };
-  // Among the tiles that fit: the one with the least work on the busiest CU. A CU handles a whole number of
-  // tiles; a tile's cost grows with its pixels, shorter tiles re-read more input rows per output row.
-  int rpt = 0;
+  int fewest = 0;
+  for (int r : {4, 2, 1})
+    if (r * dw->out_w <= static_cast<uint32_t>(kMaxSlots) && dw->out_h % r == 0 && (r * dw->out_w) % 16 == 0) fewest = r;
+  const int slots_ = RoundUp(fewest * static_cast<int>(dw->out_w), 128);
+  if (!fewest || cp_ * (slots_ + 4) + slots_ * (cp_ + 16) + 5120 + oc_alloc_ * (cp_ + 20) > 160 * 1024) return TVX_E_UNSUPPORTED;
+  // ---- tile: more rows share more of the loads and the requantization tables, fewer fill more CUs. Microseconds with (rows, wavefronts),
+  // uint8, by output rows in the batch per CU:
+  //   0.9  28 x 28, 144 to 32, stride 2    (1,8) 5.1, (2,8) 6.4      28 x 28, 192 to 32            (1,8) 6.7, (2,8) 7.3, (4,8) 9.3
+  //   1.8  112 x 112, 32 to 16             (1,8) 5.7, (2,8) 5.3      28 x 28, 144 to 32, stride 2  (1,8) 6.0, (2,8) 6.3
+  //   3.5  56 x 56, 144 to 24              (1,4) 15.4, (2,8) 12.2, (4,8) 12.3, (2,4) 13.8      28 x 28, 192 to 32  (2,8) 10.5, (4,8) 9.7
+  //   7    28 x 28, 192 to 32              (1,4) 18.5, (2,4) 15.0, (4,8) 14.4, (4,4) 16.0
+  //   14   56 x 56, 96 to 24, stride 2     (1,4) 27.7, (2,4) 24.4, (2,8) 25.9
+  //   28   112 x 112, 32 to 16             (1,4) 36.6, (2,4) 28.8, (4,4) 25.7, (4,8) 29.2 ----
   const int cus = ComputeUnits();
-  {
-    double best = 0;
-    for (int r : {4, 2, 1}) {
-      if (!fits(r) || lds_of(r) > 52 * 1024) continue;
-      const uint64_t wgs = static_cast<uint64_t>(dw->batch) * (dw->out_h / r);
-      const double per_cu = static_cast<double>((wgs + cus - 1) / cus);
-      const double cost = per_cu * r * (r == 1 ? 1.3 : (r == 2 ? 1.08 : 1.0));
-      if (!rpt || cost < best) { rpt = r; best = cost; }
-    }
-  }
-  if (!rpt)  // (no tile that small: the fewest rows that make 16-byte chunks)
-    for (int r : {1, 2, 4})
-      if (fits(r)) { rpt = r; break; }
-  if (const char* f = getenv("TVX_DWPW_ROWS")) {  // tuning aid
+  const uint64_t rows = static_cast<uint64_t>(dw->batch) * dw->out_h, cu = cus;
+  int rpt = 1;
+  for (int r : {2, 4})
+    if (rows > (r == 4 ? 3 * cu : S * cu) && dw->out_h % r == 0 && (r == 2 || S == 1) && r * dw->out_w <= static_cast<uint32_t>(kMaxSlots)) rpt = r;
+  if (const char* f = getenv("TVX_DWPW_ROWS")) {  // test lever
     const int r = atoi(f);
-    if ((r == 1 || r == 2 || r == 4) && fits(r)) rpt = r;
+    if ((r == 1 || r == 2 || (r == 4 && S == 1)) && r * dw->out_w <= static_cast<uint32_t>(kMaxSlots) && dw->out_h % r == 0) rpt = r;
   }
-  if (!rpt) return TVX_E_UNSUPPORTED;
   const uint64_t tiles = static_cast<uint64_t>(dw->batch) * (dw->out_h / rpt);
   if (tiles > 0x7fffffffull || static_cast<uint64_t>(dw->in_h) * dw->in_w * dw->in_c >= (1ull << 32) - 16 || dw->in_h >= (1u << 24)) return TVX_E_UNSUPPORTED;  // (32-bit offsets inside an image)
 
   DwPwArgs a{};
   const int C = dw->in_c;
-  a.C = C; a.H = dw->in_h; a.W = dw->in_w; a.OH = dw->out_h; a.OW = dw->out_w;
+  a.C = C; a.H = dw->in_h; a.W = dw->in_w; a.OW = dw->out_w; a.batch = dw->batch;
   a.pad_t = dw->pad_top;
-  a.ow4 = ow4; a.lpr_shift = lpr_shift;
+  a.ow4 = ow4; a.lpr_shift = lpr_shift; a.quads = (C + 3) / 4;
   const bool x_u8 = dw->in_dtype == TVX_U8, dww_u8 = dw->w_dtype == TVX_U8;
   const int dzxs = dw->in_zp - (x_u8 ? 128 : 0);
   const int dzws = (dw->w_scales ? 0 : dw->w_zp) - (dww_u8 ? 128 : 0);
   if (dzxs < -128 || dzxs > 127) return TVX_E_UNSUPPORTED;
   std::vector<int32_t> dwpk, dbiasf, drq;
-  a.dw_box = PackDepthwise3x3(C, dw_w, dww_u8, dw_b, dzxs, dzws, true, &dwpk, &dbiasf);
-  const int dw_rq = BuildRequantRecords(dw_mult, dw_shift, C, C, dw->out_zp, &drq, AccumulatorBound(9, dw_b, C));
-  if (dw_rq == kRqGeneric) return TVX_E_UNSUPPORTED;
-  a.dw_ties = dw_rq == kRqFast;
+  const bool box = PackDepthwise3x3(C, dw_w, dww_u8, dw_b, dzxs, dzws, true, &dwpk, &dbiasf);
+  // (the 32-bit record forms decide which pairs are taken; accumulators are 32 bits, whatever the bias would make of their bound)
+  if (BuildRequantRecords(dw_mult, dw_shift, C, C, dw->out_zp, &drq, AccumulatorBound(9, dw_b, C)) == kRqGeneric) return TVX_E_UNSUPPORTED;
+  const bool mid_u8 = pw->in_dtype == TVX_U8;
+  const int mid_flip = mid_u8 ? 128 : 0;
+  int up;
+  bool ties;
+  if (!BuildTieRecords(dw_mult, dw_shift, C, C, dw->out_zp - mid_flip, std::min<int64_t>(AccumulatorBound(9, dw_b, C), INT32_MAX), &drq, &up, &ties)) return TVX_E_UNSUPPORTED;
+  a.dw_pre_ties = up * 2 + ties;
+  a.dw_lo = dw_lo - mid_flip; a.dw_hi = dw_hi - mid_flip; a.dw_narrow = a.dw_lo > -128 || a.dw_hi < 127;
   a.dw_xor_mask = x_u8 ? static_cast<int>(0x80808080u) : 0;
   a.dw_pad_fill = static_cast<int>(static_cast<uint32_t>(dzxs & 0xff) * 0x01010101u);
-  a.dw_zws = dzws; a.dw_out_zp = dw->out_zp; a.dw_lo = dw_lo; a.dw_hi = dw_hi;
+  a.dw_nzws = box ? -dzws : 0;
+  a.dw_nzws3 = (a.dw_nzws & 0xff) * 0x010101;
+  std::vector<int32_t> dw_tab(static_cast<size_t>(C) * 8);
+  for (int c = 0; c < C; ++c) {
+    for (int i = 0; i < 3; ++i) dw_tab[c * 8 + i] = dwpk[c * 4 + i];
+    dw_tab[c * 8 + 3] = dbiasf[c];
+    for (int i = 0; i < 4; ++i) dw_tab[c * 8 + 4 + i] = drq[c * 4 + i];
+  }
 
   a.OC = pw->out_c;
+  a.hw = static_cast<int>(dw->out_w) * static_cast<int>(dw->out_h);
   a.cp = RoundUp(C, 32);
   a.ksteps = a.cp / 32;
+  a.last_channels = C - (a.ksteps - 1) * 32;
   a.pix_stride = a.cp + 16;
   a.oc_tiles = (a.OC + 31) / 32;
+  a.paired = a.oc_tiles * 32 - a.OC >= 16;
   a.P = rpt * dw->out_w;
-  a.slots = RoundUp(a.P, 128);
+  a.ptiles = (a.P + 31) / 32;
   a.tiles_per_image = dw->out_h / rpt;
-  const bool m_u8 = pw->in_dtype == TVX_U8, pww_u8 = pw->w_dtype == TVX_U8;
-  const int zxs = pw->in_zp - (m_u8 ? 128 : 0);
+  a.m_tiles = a.tiles_per_image > 1 ? static_cast<uint32_t>(((1ull << 32) + a.tiles_per_image - 1) / a.tiles_per_image) : 0u;
+  if (tiles * a.tiles_per_image >= (1ull << 32)) return TVX_E_UNSUPPORTED;
+  const bool pww_u8 = pw->w_dtype == TVX_U8;
+  const int zxs = pw->in_zp - mid_flip;
   const int zws = op->w_zp - (pww_u8 ? 128 : 0);
   if (zxs < -128 || zxs > 127 || zws < -127 || zws > 127) return TVX_E_UNSUPPORTED;
-  a.xor_mask = m_u8 ? static_cast<int>(0x80808080u) : 0;
   a.neg_zws4 = static_cast<int>(static_cast<uint32_t>((-zws) & 0xff) * 0x01010101u);
   a.zp = zws != 0;
-  a.out_zp = pw->out_zp; a.lo = op->act_lo; a.hi = op->act_hi;
+  const int out_flip = pw->out_dtype == TVX_U8 ? 128 : 0;
+  a.lo = op->act_lo - out_flip; a.hi = op->act_hi - out_flip; a.narrow = a.lo > -128 || a.hi < 127;
+  a.out_xor = out_flip ? static_cast<int>(0x80808080u) : 0;
   if (op->fused_add) {
     const tvx_eltwise_desc& e = op->elt;
     const double ra = static_cast<double>(e.a_scale) / static_cast<double>(e.out_scale);
@@ -464,19 +470,15 @@ int DwPwSetup(tvx_op* op, const tvx_conv2d_desc* dw, const void* dw_w, const voi
     a.add_za = e.a_zp; a.add_zb = e.b_zp; a.add_zo = e.out_zp;
     ActRange(pw->out_dtype, e.out_scale, e.out_zp, TVX_ACT_NONE, &a.add_lo, &a.add_hi);
   }
-  int lds_bytes = lds_of(rpt);
+  const int oc_bytes = a.oc_tiles * 32 * a.cp;
+  const bool wlds = oc_bytes <= kWeightBytes;
+  a.off_w = a.ptiles * 32 * a.pix_stride;
+  a.off_rq = a.off_w + (wlds ? oc_bytes : 0);
+  a.off_bias = a.off_rq + a.oc_tiles * 32 * 16;
+  const int lds_bytes = a.off_bias + a.oc_tiles * 32 * 4;
   if (lds_bytes > 160 * 1024) return TVX_E_UNSUPPORTED;
-  // Eight wavefronts where four would walk the channels in several rounds of loads (kBatch passes each) and the grid or LDS
-  // leaves a CU fewer than sixteen of them; with one round the second four only wait. MobileNetV2's blocks, 4 -> 8: batch 1
-  // 10.1 -> 8.2 us (144 channels, 56 x 56) and 11.1 -> 9.3 (192, 28 x 28), batch 64 41.0 -> 34.5 and 15.1 -> 14.0; 64 x 128 x 56 x 56
-  // -> 128 45.5 -> 36.1. One round: 32 x 32 x 112 x 112 -> 64 20.7 -> 24.7 us; sixteen in flight: 96, 112 -> 56, batch 64 26.5 -> 27.7.
-  const int kRows = S * (rpt - 1) + 3, batch = std::max(1, std::min(8, 24 / (kRows * S)));
-  const int passes = (C + (64 * kWaves >> lpr_shift) - 1) / (64 * kWaves >> lpr_shift);
-  const uint64_t resident = std::min<uint64_t>(std::min(4, 160 * 1024 / lds_bytes), (tiles + cus - 1) / cus);
-  int waves = passes > batch && resident < 4 ? kMaxWaves : kWaves;
-  if (const char* f = getenv("TVX_DWPW_WAVES")) waves = atoi(f) >= kMaxWaves ? kMaxWaves : kWaves;  // tuning aid
-  if (lds_bytes + (waves - kWaves) * kStageBytes > 160 * 1024) waves = kWaves;
-  lds_bytes += (waves - kWaves) * kStageBytes;
+  int waves = tiles <= 2ull * cus || (rpt == 4 && (a.quads << lpr_shift) > 64 * kWaves) ? kMaxWaves : kWaves;
+  if (const char* f = getenv("TVX_DWPW_WAVES")) waves = std::max(1, std::min(atoi(f), kMaxWaves));  // test lever
   // pointwise weights in fragment order, constants folded into the bias (as PwConvSetup packs them)
   const int oc_alloc = a.oc_tiles * 32;
   std::vector<int8_t> packed(static_cast<size_t>(a.oc_tiles) * a.ksteps * 1024, 0);
@@ -496,32 +498,26 @@ int DwPwSetup(tvx_op* op, const tvx_conv2d_desc* dw, const void* dw_w, const voi
     biasf[oc] = static_cast<int32_t>(static_cast<uint32_t>(v));
   }
   std::vector<int32_t> rqt;
-  const int pw_rq =
-      BuildRequantRecords(op->h_mult, op->h_shift, a.OC, oc_alloc, pw->out_zp, &rqt, AccumulatorBound(C, pw_b, a.OC));
-  if (pw_rq == kRqGeneric) return TVX_E_UNSUPPORTED;
-  a.pw_ties = pw_rq == kRqFast;
-  a.c4n_magic = static_cast<uint32_t>(((1ull << 32) + a.cp / 4 - 1) / (a.cp / 4));
+  const int64_t bound = AccumulatorBound(C, pw_b, a.OC);
+  if (BuildRequantRecords(op->h_mult, op->h_shift, a.OC, oc_alloc, pw->out_zp, &rqt, bound) == kRqGeneric) return TVX_E_UNSUPPORTED;
+  if (!BuildTieRecords(op->h_mult, op->h_shift, a.OC, oc_alloc, pw->out_zp - out_flip, std::min<int64_t>(bound, INT32_MAX), &rqt, &up, &ties)) return TVX_E_UNSUPPORTED;
+  a.pre_ties = up * 2 + ties;
   int s = op->packed.Upload(packed.data(), packed.size());
   if (s == TVX_OK) s = op->aux.Upload(biasf.data(), biasf.size() * 4);
   if (s == TVX_OK) s = op->aux2.Upload(rqt.data(), rqt.size() * 4);
-  if (s == TVX_OK) s = op->weights.Upload(dwpk.data(), dwpk.size() * 4);
-  if (s == TVX_OK) s = op->bias.Upload(dbiasf.data(), dbiasf.size() * 4);
-  if (s == TVX_OK) s = op->aux3.Upload(drq.data(), drq.size() * 4);
+  if (s == TVX_OK) s = op->aux3.Upload(dw_tab.data(), dw_tab.size() * 4);
   if (s != TVX_OK) return s;
   a.wpk = op->packed.as<v4i>();
   a.biasf = op->aux.as<int32_t>();
   a.rq = op->aux2.as<v4i>();
-  a.dw_wpk = op->weights.as<int32_t>();
-  a.dw_biasf = op->bias.as<int32_t>();
-  a.dw_rq = op->aux3.as<tvx_v4i>();
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel(S, rpt, a.add_mode != 0)),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-  if (e != hipSuccess) return SetError(TVX_E_DEVICE, "hipFuncSetAttribute(dynamic LDS %d): %s", lds_bytes, hipGetErrorString(e));
+  a.dw = op->aux3.as<v4i>();
   Plan plan{};
   plan.a = a;
+  const int flavour = a.dw_pre_ties || a.dw_narrow || a.pre_ties || a.narrow || a.dw_nzws > 127 ? kAny : a.dw_nzws ? kPlainBox : kPlain;
+  plan.fn = a.add_mode ? KernelOf<true>(S, rpt, wlds, flavour) : KernelOf<false>(S, rpt, wlds, flavour);
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(plan.fn), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+  if (e != hipSuccess) return SetError(TVX_E_DEVICE, "hipFuncSetAttribute(dynamic LDS %d): %s", lds_bytes, hipGetErrorString(e));
   plan.lds_bytes = lds_bytes;
-  plan.stride = S;
-  plan.rpt = rpt;
   plan.block = 64 * waves;
   plan.grid = dim3(static_cast<unsigned>(tiles));
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
