@@ -67,19 +67,6 @@ struct DwPwArgs {
   int add_za, add_zb, add_zo, add_lo, add_hi;
 };
 
-// Four codes of one channel, in the signed domain. PLAIN: no accumulator on a tie or to be shifted, and a clamp no narrower than a byte.
-template <bool PLAIN>
-__device__ __forceinline__ uint32_t Codes(int (&v)[4], const v4i& q, int64_t round, int pre_ties, int narrow, int lo, int hi) {
-  const int sh = q[1] & 31;
-  if constexpr (PLAIN) return RequantSaturate4<false>(v, q[0], sh, round, 0, 0);
-  if (pre_ties) {  // (uniform)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] <<= pre_ties >> 1;
-    if (pre_ties & 1) LowerOddTies(v, q);
-  }
-  return narrow ? RequantSaturate4<true>(v, q[0], sh, round, lo << sh, ((hi + 1) << sh) - 1) : RequantSaturate4<false>(v, q[0], sh, round, 0, 0);
-}
-
 constexpr int kPlain = 0, kPlainBox = 1, kAny = 2;  // requantizations without ties and narrow clamps; ... and window sums; decided at run time
 
 // S: stride of the depthwise convolution (left padding 1 at stride 1, 0 at stride 2: SAME); RPT: output rows of a tile;
@@ -220,7 +207,7 @@ __global__ void __launch_bounds__(kMaxWaves * 64) __attribute__((amdgpu_waves_pe
           if (FLAVOUR == kAny)
 #pragma unroll
             for (int i = 0; i < 4; ++i) acc[o][i] += __mul24(a.dw_nzws, sum[o][i]);
-          codes[o][j] = Codes<FLAVOUR != kAny>(acc[o], q[j], round, a.dw_pre_ties, a.dw_narrow, a.dw_lo, a.dw_hi);
+          codes[o][j] = RequantCodes4<FLAVOUR != kAny>(acc[o], q[j], round, a.dw_pre_ties, a.dw_narrow, a.dw_lo, a.dw_hi);
         }
       }
       if (w4 < a.ow4) {
@@ -302,7 +289,7 @@ __global__ void __launch_bounds__(kMaxWaves * 64) __attribute__((amdgpu_waves_pe
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       int v[4] = {acc[i], acc[4 + i], acc[8 + i], acc[12 + i]};
-      out[i] = Codes<FLAVOUR != kAny>(v, q, round, b.pre_ties, b.narrow, b.lo, b.hi) ^ static_cast<uint32_t>(b.out_xor);
+      out[i] = RequantCodes4<FLAVOUR != kAny>(v, q, round, b.pre_ties, b.narrow, b.lo, b.hi) ^ static_cast<uint32_t>(b.out_xor);
       if (ADD) out[i] = AddResidual4(b, out[i], res[i]);
     }
     if (!live) continue;

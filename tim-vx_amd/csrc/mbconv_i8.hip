@@ -4,16 +4,18 @@
 // chains when it verifies the graph (reference: src/tim/vx/internal/src/vsi_nn_graph.c:1591-1603); the
 // operators it fuses are the Conv2d nodes of src/tim/vx/internal/src/ops/vsi_nn_op_conv2d.c:35-118.
 //
-// The expanded tensor never leaves the CU. A workgroup (four or eight wavefronts) owns a band of output rows of one
-// image (at most 32 or 64 output pixels) and first transposes the band's input rows - with the halo the 3x3
-// window needs - into LDS as the MFMA operand [pixel][channel]. The expanded channels are then walked in
-// chunks of 32, wavefront w taking chunks w, w + 4 (8), ...: expansion of all halo pixels for the chunk
-// (v_mfma_i32_32x32x32_i8, requantized into a wavefront-private [channel][pixel] image), depthwise stencil on
-// that image (signed dot4 over byte windows, requantized and transposed into the projection's operand), and
-// the chunk's contribution to every output channel accumulated in registers. No barrier inside the walk: a
-// wavefront only reads what it wrote. At the end the partial projections meet in LDS by integer atomics and
-// every wavefront requantizes, adds the residual to and stores its share of the outputs.
+// The expanded tensor never leaves the CU. A workgroup owns a tile of output pixels of one image and first transposes the input
+// pixels behind it - with the halo the 3x3 window needs - into LDS as the MFMA operand [pixel][channel]. The expanded channels are
+// then walked in chunks of 32, the wavefronts taking them in turns: expansion of all halo pixels for the chunk
+// (v_mfma_i32_32x32x32_i8, requantized), depthwise stencil (signed dot4 over byte windows, requantized and
+// transposed into the projection's operand), and the chunk's contribution to every output channel accumulated in
+// registers. No barrier inside the walk: a wavefront only reads what it wrote. At the end the partial projections meet in
+// LDS by integer atomics and every wavefront requantizes, adds the residual to and stores its share of the outputs.
+//
+// At stride 1 (MbTileKernel) the expanded chunk stays in a lane's registers, at stride 2 (MbConvKernel) it is a wavefront-private
+// [channel][pixel] image in LDS.
 #include <algorithm>
+#include <climits>
 #include <cstdlib>
 #include <cstring>
 
@@ -26,7 +28,7 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr int kMinWaves = 4;
-// (two wavefronts a SIMD within 256 registers)
+// (stride 2: two wavefronts a SIMD within 256 registers)
 constexpr int MaxWaves(int acc_tiles) { return acc_tiles <= 5 ? 8 : kMinWaves; }
 constexpr int kMStride = 48;      // bytes per pixel row of the projection operand (32 channels + 16: bank spread)
 constexpr int kMaxCinSteps = 5;   // 32-channel steps of the expansion's reduction (160 input channels)
@@ -371,46 +373,438 @@ __global__ void __launch_bounds__(MaxWaves(MO * NTMAX) * 64) MbConvKernel(MbArgs
   }
 }
 
-typedef void (*MbFn)(MbArgs);
+// ---- stride 1: a lane keeps its halo rows in registers ----
+//
+// Tile rows of the expansion's matrix product come in fours to a lane (rows 8 i + 4 f .. + 3 to lane half f), so four neighbouring
+// halo columns are one requantized dword of a lane, and the halo can be dealt out such that a lane half finds the whole halo of
+// the outputs it computes in its own accumulators: the expanded tensor passes through registers only. Of the two splits
+//   WIDE   64 halo pixels, four rows x eight columns a half, 2 x 7 outputs a half (the ninth halo column is padding): the halves
+//          are the two column halves of 14 columns, or two pairs of rows of 7;
+//   narrow 32 halo pixels, four rows x four columns a half (two of them in both), 2 x 2 outputs a half: 2 x 4 outputs a workgroup,
+// the first computes an output for fewer expanded pixels (2.3 against 4), the second makes four times the workgroups. Bound by
+// the vector ALU (390 instructions and 2200 cycles a chunk in the wide form, a third of them dot products) where a batch fills the
+// chip, by the chain load - expansion - stencil - projection - sum - store in small ones. Before, one kernel served both strides: the
+// expanded image went through LDS, every window was cut from it and every code requantized by itself. uint8, before and
+// now, microseconds: 14 columns, 64 to 384 to 64: batch 1 9.0 / 4.8, batch 64 15.8 / 10.6; 96 to 576 to 96: 12.9 / 6.3, 26.3 / 16.6.
+struct MbTileArgs : MbArgs {
+  int W, batch;
+  int tiles_per_image, col_tiles, tile_rows;
+  uint32_t m_tiles, m_cols;        // reciprocals
+  int half_rows, half_cols, half_halo;  // the second half's outputs: rows and columns behind the first's, and its halo's columns
+  int last1, last3;                // channels of the last reduction step of the expansion and of the projection
+  int dw_nzws3;                    // minus the depthwise weights' zero point in three bytes (0: folded)
+  int pre1, pre2, pre3;            // ties, narrow clamps: as RequantCodes4 takes them (clamps in the signed domain)
+  int narrow1, narrow2, narrow3;
+  int out_xor4;
+};
 
-template <int W, int S, int MO, bool ADD>
+constexpr int TileWaves(bool wide, int steps) { return wide || steps > 3 ? 8 : 12; }  // (two wavefronts a SIMD within 256 registers, three within 168)
+
+template <bool WIDE, int KS, int NT, bool ADD, bool PLAIN>
+__global__ void __launch_bounds__(TileWaves(WIDE, KS) * 64) MbTileKernel(MbTileArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  constexpr int MT = WIDE ? 2 : 1;    // 32-pixel halo tiles = dwords of a lane's halo row
+  constexpr int kWin = WIDE ? 4 : 1;  // window dwords of a halo row: two outputs each
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), threads = blockDim.x, waves = threads >> 6;
+  int wg = blockIdx.x;  // an XCD gets a contiguous run of tiles: neighbours share halo rows in its L2
+  {
+    const int per = gridDim.x >> 3, rem = gridDim.x & 7, xcd = wg & 7;
+    wg = xcd * per + min(xcd, rem) + (wg >> 3);
+  }
+  const auto over = [](int v, uint32_t m) { return static_cast<int>(__umulhi(static_cast<uint32_t>(v), m) + (static_cast<uint32_t>(v) & (m ? 0u : ~0u))); };
+  const int n = over(wg, a.m_tiles), tile = wg - n * a.tiles_per_image;
+  const int band = over(tile, a.m_cols);
+  const int r0 = band * a.tile_rows, c0 = (tile - band * a.col_tiles) * 4;  // (WIDE: one tile of columns)
+
+  // what the first chunk needs is requested before the input
+  struct ExpandOperands {
+    v4i wf[KS];
+    int bias;
+    v4i q;
+  } next;
+  v4i taps4, q2, w2[WIDE ? NT : 2 * NT];
+  const auto fetch = [&](int chunk) {
+#pragma unroll
+    for (int k = 0; k < KS; ++k) next.wf[k] = a.w1[(chunk * a.cin_steps + min(k, a.cin_steps - 1)) * 64 + lane];
+    next.bias = a.b1[chunk * 32 + col];
+    next.q = a.q1[chunk * 32 + col];
+  };
+  const auto fetch_depthwise = [&](int chunk) {
+    taps4 = a.dwk[chunk * 32 + col];
+    q2 = a.q2[chunk * 32 + col];
+  };
+  const auto fetch_projection = [&](int chunk) {
+    if constexpr (WIDE) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) w2[t] = a.w2[(min(t, a.nt - 1) * a.chunks + chunk) * 64 + lane];
+    } else {  // sixteen output channels a product, the upper half of whose reduction meets zeros
+#pragma unroll
+      for (int t = 0; t < 2 * NT; ++t) w2[t] = a.w2[(min(t >> 1, a.nt - 1) * a.chunks + chunk) * 64 + (lane & 16) * 2 + (t & 1) * 16 + (lane & 15)];
+    }
+  };
+  if (wave < a.chunks) {
+    fetch(wave);
+    fetch_depthwise(wave);
+  }
+
+  // ---- the halo as the expansion's operand: xin[slot][channel], signed bytes; slots 4 s .. 4 s + 3 are dword s >> 1 of half s & 1.
+  // What lies outside the image holds anything: its expanded codes are replaced. ----
+  const int items = a.cin_steps * 64 * MT;
+  struct Item {
+    uint32_t d[4];
+    int by[4];
+  };
+  const auto slots = [&](int u) { return u & (8 * MT - 1); };
+  const auto channel = [&](int u) { return u / (8 * MT) * 4; };
+  const auto load = [&](int u) {
+    Item it;
+    const int plane = a.H * a.W, image = a.Cin * plane;
+    const uint8_t* xn = a.x + static_cast<size_t>(n) * image;
+    const int lowest = n == 0 ? 0 : -4, highest = n == a.batch - 1 ? image - 4 : INT_MAX;  // (inside the tensor)
+    const int s = slots(u), c = channel(u), f = s & 1, i = s >> 1;
+    const int row = r0 + f * a.half_rows - 1 + (WIDE ? i >> 1 : i);
+    const int x = WIDE ? f * a.half_halo + 4 * (i & 1) : c0 - 1 + 2 * f;
+    const int at = min(max(row, 0), a.H - 1) * a.W + x;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int o = min(c + j, a.Cin - 1) * plane + at, in = min(max(o, lowest), highest);
+      it.by[j] = in - o;
+      __builtin_memcpy(&it.d[j], xn + in, 4);
+    }
+    return it;
+  };
+  const auto store = [&](int u, const Item& it) {
+    uint32_t d[4], px[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)  // a dword at an end of the tensor was read from inside it
+      d[j] = (it.d[j] << (8 * max(it.by[j], 0)) >> (8 * min(max(-it.by[j], 0), 3))) ^ (a.x_xor * 0x01010101u);
+    Transpose4x4(d, px);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) *reinterpret_cast<uint32_t*>(lds + (4 * slots(u) + e) * a.xs + channel(u)) = px[e];
+  };
+  Item first;
+  if (tid < items) first = load(tid);
+
+  // ---- under these loads: the constants of the later phases ----
+  const MbTileArgs& b = LateArgs<MbTileArgs>();
+  constexpr int kQuads = WIDE ? 4 : 1;  // of output pixels of a lane and 32-channel tile
+  int* red = reinterpret_cast<int*>(lds + b.off_red);
+  for (int i = tid; i < b.nt * kQuads * 64; i += threads) reinterpret_cast<v4i*>(red)[i] = v4i{0, 0, 0, 0};
+  const auto constant = [&](int value4, int live, int group) {  // a fragment of `value` for `live` channels
+    v4i f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int left = live - 16 * group - 4 * i;
+      f[i] = left >= 4 ? value4 : left <= 0 ? 0 : value4 & static_cast<int>((1u << (8 * left)) - 1u);
+    }
+    return f;
+  };
+  const v4i z1_last = constant(b.neg_zws1_4, b.last1, half);
+  const v4i z1 = {b.neg_zws1_4, b.neg_zws1_4, b.neg_zws1_4, b.neg_zws1_4};
+  // bytes of a lane's halo dwords that are columns of the image, and which of its four halo rows are none
+  uint32_t keep[MT], fill[MT];
+  int outside = 0;
+#pragma unroll
+  for (int j = 0; j < MT; ++j) {
+    const int x = WIDE ? half * b.half_halo + 4 * j : c0 - 1 + 2 * half;
+    keep[j] = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (static_cast<unsigned>(x + e) < static_cast<unsigned>(b.W)) keep[j] |= 0xffu << (8 * e);
+    fill[j] = static_cast<uint32_t>(b.e_pad4) & ~keep[j];
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = r0 + half * b.half_rows - 1 + r;
+    if (static_cast<unsigned>(row) >= static_cast<unsigned>(b.H)) outside |= 1 << r;
+  }
+  const bool edge = r0 == 0 || r0 + b.tile_rows >= b.H;
+  const uint32_t order = WIDE && half && b.half_halo ? 0x07060504u : 0x06050403u;  // left padding in front of the halo's columns, or right behind
+  const int cin_steps = b.cin_steps, xs = b.xs, e_pad4 = b.e_pad4, chunks = b.chunks, nt = b.nt, zp1 = b.zp1, zp3 = b.zp3, neg_zws3_4 = b.neg_zws3_4,
+            dw_box = b.dw_box, dw_nzws3 = b.dw_nzws3, last3 = b.last3, H = b.H, W = b.W, Cout = b.Cout, half_rows = b.half_rows, half_cols = b.half_cols;
+  const int32_t* const b3 = b.b3;
+  const v4i* const q3 = b.q3;
+  const uint8_t* const other = b.res;
+  uint8_t* const y = b.y;  // (read through the reference behind a store, each would be loaded again)
+
+  if (tid < items) store(tid, first);
+  for (int u = tid + threads; u < items; u += threads) store(u, load(u));
+  __syncthreads();
+
+  // the zero-point term of uint8 expansion weights depends on the pixel alone
+  const uint8_t* xa = lds + col * xs + half * 16;
+  v16i xsum[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) xsum[mt][r] = 0;
+  if (zp1) {  // (uniform)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+        if (k < cin_steps)
+          xsum[mt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i*>(xa + mt * 32 * xs + k * 32), k + 1 < cin_steps ? z1 : z1_last, xsum[mt], 0, 0, 0);
+  }
+
+  constexpr bool kResident = WIDE ? KS <= 3 : NT <= 5;  // the operand stays in registers (with more steps it would not fit)
+  v4i fx[MT][KS];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int k = 0; k < (kResident ? KS : 0); ++k) fx[mt][k] = *reinterpret_cast<const v4i*>(xa + mt * 32 * xs + min(k, cin_steps - 1) * 32);
+  uint8_t* m_w = lds + b.off_wave + wave * b.wave_bytes;
+  v16i acc_w[WIDE ? NT : 1], zp_w;
+  v4i acc_n[WIDE ? 1 : 2 * NT], zp_n = {0, 0, 0, 0};
+#pragma unroll
+  for (int r = 0; r < 16; ++r) zp_w[r] = 0;
+#pragma unroll
+  for (int t = 0; t < (WIDE ? NT : 1); ++t) acc_w[t] = zp_w;
+#pragma unroll
+  for (int t = 0; t < (WIDE ? 1 : 2 * NT); ++t) acc_n[t] = zp_n;
+
+  // a chunk's contribution to every output tile
+  v4i fm = {0, 0, 0, 0};
+#pragma unroll
+  for (int t = 0; t < (WIDE ? NT : 2 * NT); ++t) w2[t] = fm;
+  const auto project = [&](int live3) {
+    if constexpr (!WIDE) fm = half ? v4i{0, 0, 0, 0} : fm;
+    if constexpr (WIDE) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        if (t < nt) acc_w[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fm, w2[t], acc_w[t], 0, 0, 0);
+      if (zp3) zp_w = __builtin_amdgcn_mfma_i32_32x32x32_i8(fm, constant(neg_zws3_4, live3, half), zp_w, 0, 0, 0);
+    } else {
+#pragma unroll
+      for (int t = 0; t < 2 * NT; ++t)
+        if (t < 2 * nt) acc_n[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fm, w2[t], acc_n[t], 0, 0, 0);
+      if (zp3) zp_n = __builtin_amdgcn_mfma_i32_16x16x64_i8(fm, constant(neg_zws3_4, live3, lane >> 4 & 1), zp_n, 0, 0, 0);
+    }
+  };
+  for (int chunk = wave; chunk < chunks; chunk += waves) {
+    // ---- expansion of the halo for this chunk's 32 channels: a lane's is `col` ----
+    const uint8_t* xc = xa;
+    if (!kResident) asm volatile("" : "+v"(xc));  // (or the compiler takes the reads out of the loop)
+    v16i acc[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[mt][r] = xsum[mt][r] + next.bias;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+        if (k < cin_steps) acc[mt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kResident ? fx[mt][k] : *reinterpret_cast<const v4i*>(xc + mt * 32 * xs + k * 32), next.wf[k], acc[mt], 0, 0, 0);
+    project(32);
+    fetch_projection(chunk);
+    uint32_t e[4][MT];
+    {
+      const int64_t round = RoundHigh(next.q[2]);
+#pragma unroll
+      for (int i = 0; i < 4 * MT; ++i) {
+        int v[4] = {acc[i / 4][4 * (i % 4)], acc[i / 4][4 * (i % 4) + 1], acc[i / 4][4 * (i % 4) + 2], acc[i / 4][4 * (i % 4) + 3]};
+        e[i / MT][i % MT] = (RequantCodes4<PLAIN>(v, next.q, round, b.pre1, b.narrow1, b.e_lo, b.e_hi) & keep[i % MT]) | fill[i % MT];
+      }
+    }
+    if (edge) {  // (uniform)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) e[r][j] = outside >> r & 1 ? static_cast<uint32_t>(e_pad4) : e[r][j];
+    }
+    const bool more = chunk + waves < chunks;
+    if (more) fetch(chunk + waves);
+
+    // ---- depthwise 3x3: two rows of outputs; a window dword serves two outputs, the second by taps a byte further up ----
+    int win[4][kWin];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if constexpr (WIDE) {
+        const uint32_t pad = static_cast<uint32_t>(e_pad4);
+        const uint32_t w0 = __builtin_amdgcn_perm(e[r][0], pad, order), w1 = __builtin_amdgcn_perm(e[r][1], e[r][0], order), w2 = __builtin_amdgcn_perm(pad, e[r][1], order);
+        win[r][0] = static_cast<int>(w0);
+        win[r][1] = static_cast<int>(__builtin_amdgcn_alignbyte(w1, w0, 2));
+        win[r][2] = static_cast<int>(w1);
+        win[r][3] = static_cast<int>(__builtin_amdgcn_alignbyte(w2, w1, 2));
+      } else {
+        win[r][0] = static_cast<int>(e[r][0]);
+      }
+    }
+    int sums[2][2 * kWin];  // [row][column]
+    {
+      int taps[2][3];
+#pragma unroll
+      for (int t = 0; t < 3; ++t) {
+        taps[0][t] = taps4[t];
+        taps[1][t] = taps4[t] << 8;
+      }
+#pragma unroll
+      for (int o = 0; o < 2; ++o)
+#pragma unroll
+        for (int c = 0; c < 2 * kWin; ++c) {
+          int v = Dot4Add(win[o][c / 2], taps[c % 2][0], taps4[3]);
+          v = __builtin_amdgcn_sdot4(win[o + 1][c / 2], taps[c % 2][1], v, false);
+          sums[o][c] = __builtin_amdgcn_sdot4(win[o + 2][c / 2], taps[c % 2][2], v, false);
+        }
+      if (dw_box) {  // (uniform) weights packed unshifted: their zero point times the window sum
+#pragma unroll
+        for (int o = 0; o < 2; ++o)
+#pragma unroll
+          for (int c = 0; c < 2 * kWin; ++c)
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+              if (PLAIN) sums[o][c] = __builtin_amdgcn_sdot4(win[o + t][c / 2], dw_nzws3 << (c % 2 * 8), sums[o][c], false);
+              else sums[o][c] -= b.dw_zws * __builtin_amdgcn_sdot4(win[o + t][c / 2], 0x00010101 << (c % 2 * 8), 0, false);
+            }
+      }
+    }
+    {
+      const int64_t round = RoundHigh(q2[2]);
+      const auto codes = [&](int v0, int v1, int v2, int v3) {
+        int v[4] = {v0, v1, v2, v3};
+        return RequantCodes4<PLAIN>(v, q2, round, b.pre2, b.narrow2, b.m_lo, b.m_hi);
+      };
+      if constexpr (WIDE) {  // the projection's operand [pixel][channel]: pixel 16 half + 8 row + column
+#pragma unroll
+        for (int o = 0; o < 2; ++o)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const uint32_t c = codes(sums[o][4 * h], sums[o][4 * h + 1], sums[o][4 * h + 2], sums[o][4 * h + 3]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (4 * h + i < 7) m_w[(16 * half + 8 * o + 4 * h + i) * kMStride + col] = static_cast<uint8_t>(c >> (8 * i));
+          }
+      } else {  // pixel 4 row + column
+        const uint32_t c = codes(sums[0][0], sums[0][1], sums[1][0], sums[1][1]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m_w[(4 * (i / 2) + 2 * half + i % 2) * kMStride + col] = static_cast<uint8_t>(c >> (8 * i));
+      }
+    }
+    __builtin_amdgcn_wave_barrier();  // (a wavefront reads what it wrote)
+
+    // its contribution to the output tiles is added behind the next chunk's expansion
+    fm = *reinterpret_cast<const v4i*>(m_w + (WIDE ? col * kMStride + half * 16 : (lane & 7) * kMStride + (lane & 16)));
+    if (chunk + waves < chunks) fetch_depthwise(chunk + waves);
+    __builtin_amdgcn_wave_barrier();
+  }
+
+  project((chunks - 1) % waves == wave ? last3 : 32);  // (a wavefront that walked no chunk adds nothing)
+  // ---- the wavefronts' partial projections meet in LDS, laid out [32-channel tile][pixel quad][pixel][lane half = quad of the eight
+  // pixels, channel]; every wavefront finishes its share of the quads. What a unit needs from memory is requested first. ----
+  const int units = nt * kQuads;
+  constexpr int kUnits = (NT * kQuads + kMinWaves - 1) / kMinWaves;
+  const size_t plane = static_cast<size_t>(H) * W, lane_at = col * plane + (WIDE ? 4 : W) * half;
+  int bias[kUnits], live[kUnits];
+  v4i q[kUnits];
+  uint32_t res[kUnits];
+  size_t at[kUnits];
+#pragma unroll
+  for (int i = 0; i < kUnits; ++i) {
+    const int u = wave + i * waves;
+    if (u >= units) break;
+    const int t = u / kQuads, quad = u % kQuads, oc = t * 32 + col;  // (u, t and quad are uniform)
+    const int row = r0 + (WIDE ? (quad >> 1) * half_rows + (quad & 1) : 0), x = c0 + (WIDE ? (quad >> 1) * half_cols : 0);
+    live[i] = row + (WIDE ? 0 : half) < H && oc < Cout ? (WIDE ? 4 - half : min(4, W - x)) : 0;
+    at[i] = (static_cast<size_t>(n) * Cout + t * 32) * plane + static_cast<size_t>(row) * W + x + lane_at;
+    bias[i] = b3[oc];
+    q[i] = q3[oc];
+    res[i] = 0;
+    if (ADD) {
+      if (live[i] == 4) {
+        __builtin_memcpy(&res[i], other + at[i], 4);
+      } else {
+        uint16_t lo = 0;
+        if (live[i] & 2) __builtin_memcpy(&lo, other + at[i], 2);
+        res[i] = lo;
+        if (live[i] & 1) res[i] |= static_cast<uint32_t>(other[at[i] + (live[i] & 2)]) << (8 * (live[i] & 2));
+      }
+    }
+  }
+  if (wave < chunks) {  // (a wavefront that walked no chunk has nothing to add)
+    if constexpr (WIDE) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        if (t < nt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) __hip_atomic_fetch_add(red + (t * 16 + r) * 64 + lane, acc_w[t][r] + zp_w[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    } else if (half == 0) {  // (rows 8 to 15 of a product hold no pixel)
+#pragma unroll
+      for (int t = 0; t < 2 * NT; ++t)
+        if (t < 2 * nt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            __hip_atomic_fetch_add(red + ((t >> 1) * 4 + r) * 64 + (lane & 16) * 2 + (t & 1) * 16 + (lane & 15), acc_n[t][r] + zp_n[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kUnits; ++i) {
+    const int u = wave + i * waves;
+    if (u >= units) break;
+    int v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = red[(u * 4 + e) * 64 + lane] + bias[i];
+    uint32_t codes = RequantCodes4<PLAIN>(v, q[i], RoundHigh(q[i][2]), b.pre3, b.narrow3, b.lo, b.hi) ^ static_cast<uint32_t>(b.out_xor4);
+    if (ADD) codes = AddResidual4(b, codes, res[i]);
+    if (live[i] == 4) {
+      __builtin_memcpy(y + at[i], &codes, 4);
+    } else {
+      if (live[i] & 2) __builtin_memcpy(y + at[i], &codes, 2);
+      if (live[i] & 1) y[at[i] + (live[i] & 2)] = static_cast<uint8_t>(codes >> (8 * (live[i] & 2)));
+    }
+  }
+}
+
+typedef void (*MbFn)(MbArgs);
+typedef void (*MbTileFn)(MbTileArgs);
+
+template <bool WIDE, bool ADD, bool PLAIN>
+MbTileFn TileKernelOf(int widest) {  // (in 32-channel steps: the block's input and output)
+  if (widest <= 2) return MbTileKernel<WIDE, 2, 2, ADD, PLAIN>;
+  if (widest <= 3) return MbTileKernel<WIDE, 3, 3, ADD, PLAIN>;
+  if (widest <= 5) return MbTileKernel<WIDE, 5, 5, ADD, PLAIN>;
+  if constexpr (!WIDE) return MbTileKernel<false, 5, 10, ADD, PLAIN>;
+  return nullptr;
+}
+template <bool WIDE>
+MbTileFn TileKernelOf(int widest, bool add, bool plain) {
+  return add ? (plain ? TileKernelOf<WIDE, true, true>(widest) : TileKernelOf<WIDE, true, false>(widest))
+             : (plain ? TileKernelOf<WIDE, false, true>(widest) : TileKernelOf<WIDE, false, false>(widest));
+}
+
+template <int W, bool ADD>
 MbFn KernelNt(int nt) {
-  if (nt <= 2) return MbConvKernel<W, S, MO, 2, ADD>;
-  if (nt <= 5) return MbConvKernel<W, S, MO, 5, ADD>;
-  if (MO == 1 && nt <= 10) return MbConvKernel<W, S, 1, 10, ADD>;
+  if (nt <= 2) return MbConvKernel<W, 2, 1, 2, ADD>;
+  if (nt <= 5) return MbConvKernel<W, 2, 1, 5, ADD>;
+  if (nt <= 10) return MbConvKernel<W, 2, 1, 10, ADD>;
   return nullptr;
 }
 
 template <bool ADD>
-MbFn KernelOf(int w, int s, int nt) {
-  if (w == 28 && s == 1) return KernelNt<28, 1, 2, ADD>(nt);
-  if (w == 28 && s == 2) return KernelNt<28, 2, 1, ADD>(nt);
-  if (w == 14 && s == 1) return KernelNt<14, 1, 1, ADD>(nt);
-  if (w == 14 && s == 2) return KernelNt<14, 2, 1, ADD>(nt);
-  if (w == 7 && s == 1) return KernelNt<7, 1, 1, ADD>(nt);
-  return nullptr;
+MbFn KernelOf(int w, int nt) {
+  return w == 28 ? KernelNt<28, ADD>(nt) : w == 14 ? KernelNt<14, ADD>(nt) : nullptr;
 }
 
 struct Plan {
-  MbArgs a;
-  int w, s, lds_bytes;
+  MbTileArgs a;
+  MbFn fn;            // stride 2
+  MbTileFn tile_fn;   // stride 1
+  int lds_bytes;
   unsigned grid, block;
 };
 
-MbFn Kernel(const Plan& p) {
-  return p.a.add_mode ? KernelOf<true>(p.w, p.s, p.a.nt) : KernelOf<false>(p.w, p.s, p.a.nt);
-}
-
 int MbConvRun(tvx_op* op, const void* in0, const void* in1, void* out, hipStream_t st) {
   const Plan* plan = reinterpret_cast<const Plan*>(op->host_blob.data());
-  MbArgs a = plan->a;
+  MbTileArgs a = plan->a;
   a.x = static_cast<const uint8_t*>(in0);
   a.y = static_cast<uint8_t*>(out);
   a.res = static_cast<const uint8_t*>(in1);
   if (a.add_mode && !in1) return SetError(TVX_E_INVALID, "pwconv_dwconv3x3_pwconv_i8: the fused Add needs its second operand as in1");
   if (a.aligned4 && ((reinterpret_cast<uintptr_t>(out) | (a.add_mode ? reinterpret_cast<uintptr_t>(in1) : 0)) & 3))
     a.aligned4 = 0;
-  hipLaunchKernelGGL(Kernel(*plan), dim3(plan->grid), dim3(plan->block), plan->lds_bytes, st, a);
+  if (plan->tile_fn) hipLaunchKernelGGL(plan->tile_fn, dim3(plan->grid), dim3(plan->block), plan->lds_bytes, st, a);
+  else hipLaunchKernelGGL(plan->fn, dim3(plan->grid), dim3(plan->block), plan->lds_bytes, st, static_cast<const MbArgs&>(a));
   TVX_HIP_CHECK(hipGetLastError());
   return TVX_OK;
 }
@@ -464,49 +858,82 @@ int MbConvSetup(tvx_op* op, const MbStage& ex, const MbStage& dw, const tvx_conv
   const int Cin = e->in_c, Cexp = e->out_c, Cout = pr->out_c;
   const int cin_steps = (Cin + 31) / 32, chunks = (Cexp + 31) / 32, nt = (Cout + 31) / 32;
   if (cin_steps > kMaxCinSteps) return TVX_E_UNSUPPORTED;
+  if (S == 1 ? (W != 7 && W != 14 && W != 28) || nt > (W == 28 ? 5 : 10) : (W != 14 && W != 28) || nt > 10) return TVX_E_UNSUPPORTED;
   Plan plan{};
-  plan.w = W; plan.s = S;
-  MbArgs& a = plan.a;
+  MbTileArgs& a = plan.a;
   a.nt = nt;
   a.add_mode = op->fused_add;
-  if (!Kernel(plan)) return TVX_E_UNSUPPORTED;
   if (const char* f = getenv("TVX_NO_MBCONV"))  // tuning aid: leaves blocks to the single operators
     if (atoi(f)) return TVX_E_UNSUPPORTED;
-  // Measured on MobileNetV2 at batch 64: the block kernel beats the single operators on the 14-column stride-1
-  // blocks (25 against 32 us); on 28 columns their launches carry enough work, on 7 columns and at stride 2 the
-  // block's work per wavefront is too long a chain. Those shapes are taken on request only.
-  if (W != 14 || S != 1) {
-    const char* f = getenv("TVX_MBCONV_ALL");
-    if (!f || !atoi(f)) return TVX_E_UNSUPPORTED;
-  }
-  const int MO = (W == 28 && S == 1) ? 2 : 1;
-  // rows of a band: what fills the output tiles; on 7-column planes two rows only, which doubles the bands (a batch
-  // of 64 images then fills the chip) and needs a single halo tile
-  int R = W == 7 ? 2 : MO * 32 / OW;
-  R = std::min<int>(R, d->out_h);
-  if (R < 1) return TVX_E_UNSUPPORTED;
-  const int IR = (R - 1) * S + 3;
-  const int mh = (IR * W + 31) / 32;
   if (static_cast<uint64_t>(e->in_c) * H * W >= (1ull << 31)) return TVX_E_UNSUPPORTED;
-
+  const char* const every = getenv("TVX_MBCONV_ALL");  // takes blocks also where the single operators are faster
+  const bool all = every && atoi(every);
+  if (S == 2 && !all) return TVX_E_UNSUPPORTED;  // (28 columns, 32 to 192 to 64: batch 1 8.5 us against 7.5, batch 64 15.0 against 15.7; 14 columns: twice their time)
   a.Cin = Cin; a.H = H; a.Cexp = Cexp; a.Cout = Cout; a.OH = d->out_h;
   a.cin_steps = cin_steps; a.chunks = chunks;
-  a.R = R; a.IR = IR; a.bands = (d->out_h + R - 1) / R; a.mh = mh;
   a.xs = cin_steps * 32 + 16;
-  a.ep = mh * 32 + 4;
-  a.off_wave = RoundUp(mh * 32 * a.xs, 16);
-  a.wave_bytes = RoundUp(16 + 32 * a.ep + MO * 32 * kMStride, 16);
-  const uint64_t wgs = static_cast<uint64_t>(e->batch) * a.bands;
-  // With at most one workgroup a CU eight wavefronts walk the chunks in half the rounds; with more, four and a second workgroup
-  // are better. 64 -> 384 -> 64 and 96 -> 576 -> 96 channels on 14 x 14: batch 1 11.9 -> 9.1 and 20.1 -> 13.1 us, batch 64 14.3 and 23.7
-  // against 19.1 and 24.9 with eight.
-  int waves = wgs <= static_cast<uint64_t>(ComputeUnits()) ? MaxWaves(MO * (nt <= 2 ? 2 : nt <= 5 ? 5 : 10)) : kMinWaves;
-  if (const char* f = getenv("TVX_MBCONV_WAVES")) waves = std::max(kMinWaves, atoi(f));  // tuning aid
-  waves = std::min(waves, MaxWaves(MO * (nt <= 2 ? 2 : nt <= 5 ? 5 : 10)));
-  while (waves > kMinWaves && a.off_wave + waves * a.wave_bytes + nt * MO * 4096 > 160 * 1024) --waves;
+  uint64_t wgs;
+  int waves;
+  bool wide = false;
+  if (S == 1) {
+    // Microseconds, uint8 (a network of single operators: "apart"), by batch:
+    //                                             1    4    8    16    32    64
+    //   14 columns, 64 to 384 to 64    narrow   4.8  5.1  5.4   6.8   9.6  15.3    (the better of four and twelve wavefronts)
+    //                                  wide     6.4  6.5  6.6   6.9   7.4  10.8    (of four and eight)
+    //   14 columns, 96 to 576 to 96    narrow   6.4  6.7  6.9   9.6  15.2  25.9    wide 8.8  8.8  9.1  9.4  10.3  16.7
+    //   28 columns, 32 to 192 to 32    narrow   4.2  5.3  6.7  10.2  16.3  29.5    apart 9.2  9.4  9.7  11.0  13.9  20.5
+    //   7 columns, 160 to 960 to 160   narrow   9.7  9.9  9.9  10.3  11.0  18.0    apart 10.4  11.6  12.2  14.3  16.6  20.2    wide - 16.6
+    //   7 columns, 160 to 960 to 320   narrow  33.6  ...             36.0  61.8    apart 10.3  11.4  12.0  14.3  16.8  20.5
+    // narrow as long as each of its workgroups finds a CU of its own
+    const uint64_t narrow_wgs = static_cast<uint64_t>(e->batch) * ((H + 1) / 2) * ((W + 3) / 4), cus = ComputeUnits();
+    wide = W != 28 && nt <= 5 && narrow_wgs > cus;
+    if (const char* f = getenv("TVX_MBCONV_WIDE")) wide = W != 28 && nt <= 5 && atoi(f);  // test lever
+    if (!all && ((W == 28 && narrow_wgs > 7 * cus) || (W == 7 && nt > 5))) return TVX_E_UNSUPPORTED;
+    a.W = W; a.batch = e->batch;
+    a.half_rows = wide && W == 7 ? 2 : 0;
+    a.half_cols = wide && W == 14 ? 7 : 0;
+    a.half_halo = wide && W == 14 ? 6 : 0;
+    a.tile_rows = 2 + a.half_rows;
+    a.col_tiles = wide ? 1 : (W + 3) / 4;
+    a.tiles_per_image = (H + a.tile_rows - 1) / a.tile_rows * a.col_tiles;
+    const auto reciprocal = [](int v) { return v > 1 ? static_cast<uint32_t>(((1ull << 32) + v - 1) / v) : 0u; };
+    a.m_tiles = reciprocal(a.tiles_per_image);
+    a.m_cols = reciprocal(a.col_tiles);
+    wgs = static_cast<uint64_t>(e->batch) * a.tiles_per_image;
+    if (wgs * a.tiles_per_image >= (1ull << 32)) return TVX_E_UNSUPPORTED;
+    a.last1 = Cin - (cin_steps - 1) * 32;
+    a.last3 = Cexp - (chunks - 1) * 32;
+    a.off_wave = (wide ? 64 : 32) * a.xs;
+    a.wave_bytes = (wide ? 32 : 8) * kMStride;
+    const int most = TileWaves(wide, std::max(cin_steps, nt));
+    // as many wavefronts as share the chunks evenly; four where a CU holds several workgroups (others leave SIMDs empty: 28 columns,
+    // batch 64, 29.5 us with four, 49 with five, 46 with six)
+    const int rounds = (chunks + most - 1) / most;
+    waves = wgs > cus ? kMinWaves : std::max(kMinWaves, wide ? most : (chunks + rounds - 1) / rounds);
+    if (const char* f = getenv("TVX_MBCONV_WAVES")) waves = std::min(std::max(kMinWaves, atoi(f)), most);  // test lever
+    a.off_red = a.off_wave + waves * a.wave_bytes;
+    plan.lds_bytes = a.off_red + nt * (wide ? 4096 : 1024);
+  } else {
+    // rows of a band: what fills the output tile
+    const int R = std::min<int>(32 / OW, d->out_h);
+    if (R < 1) return TVX_E_UNSUPPORTED;
+    const int IR = (R - 1) * S + 3, mh = (IR * W + 31) / 32;
+    a.R = R; a.IR = IR; a.bands = (d->out_h + R - 1) / R; a.mh = mh;
+    a.ep = mh * 32 + 4;
+    a.off_wave = RoundUp(mh * 32 * a.xs, 16);
+    a.wave_bytes = RoundUp(16 + 32 * a.ep + 32 * kMStride, 16);
+    wgs = static_cast<uint64_t>(e->batch) * a.bands;
+    // with at most one workgroup a CU eight wavefronts walk the chunks in half the rounds; with more, four and a second workgroup are better
+    const int most = MaxWaves(nt <= 2 ? 2 : nt <= 5 ? 5 : 10);
+    waves = wgs <= static_cast<uint64_t>(ComputeUnits()) ? most : kMinWaves;
+    if (const char* f = getenv("TVX_MBCONV_WAVES")) waves = std::max(kMinWaves, atoi(f));  // tuning aid
+    waves = std::min(waves, most);
+    while (waves > kMinWaves && a.off_wave + waves * a.wave_bytes + nt * 4096 > 160 * 1024) --waves;
+    a.off_red = a.off_wave + waves * a.wave_bytes;
+    plan.lds_bytes = a.off_red + nt * 4096;
+    a.aligned4 = static_cast<uint64_t>(d->out_h) * OW % 4 == 0 && (R * OW) % 4 == 0 && (static_cast<int>(d->out_h) % R * OW) % 4 == 0;
+  }
   plan.block = 64 * waves;
-  a.off_red = a.off_wave + waves * a.wave_bytes;
-  plan.lds_bytes = a.off_red + nt * MO * 4096;
   if (plan.lds_bytes > 160 * 1024) return TVX_E_UNSUPPORTED;
   if (wgs > 0x7fffffffull) return TVX_E_UNSUPPORTED;
   plan.grid = static_cast<unsigned>(wgs);
@@ -582,8 +1009,30 @@ int MbConvSetup(tvx_op* op, const MbStage& ex, const MbStage& dw, const tvx_conv
     a.add_za = el.a_zp; a.add_zb = el.b_zp; a.add_zo = el.out_zp;
     ActRange(pr->out_dtype, el.out_scale, el.out_zp, TVX_ACT_NONE, &a.add_lo, &a.add_hi);
   }
-  const uint64_t out_plane = static_cast<uint64_t>(d->out_h) * OW;
-  a.aligned4 = out_plane % 4 == 0 && (R * OW) % 4 == 0 && (static_cast<int>(d->out_h) % R * OW) % 4 == 0;
+  if (S == 1) {
+    // codes in the signed domain, records for the packed requantization
+    const int e_flip = e_u8 ? 128 : 0, m_flip = m_u8 ? 128 : 0, out_flip = pr->out_dtype == TVX_U8 ? 128 : 0;
+    int up[3];
+    bool ties[3];
+    const auto capped = [](int64_t bound) { return std::min<int64_t>(bound, INT32_MAX); };
+    if (!BuildTieRecords(*ex.mult, *ex.shift, Cexp, exp_alloc, e->out_zp - e_flip, capped(AccumulatorBound(Cin, ex.b, Cexp)), &rq1, &up[0], &ties[0]) ||
+        !BuildTieRecords(*dw.mult, *dw.shift, Cexp, exp_alloc, d->out_zp - m_flip, capped(AccumulatorBound(9, dw.b, Cexp)), &rq2, &up[1], &ties[1]) ||
+        !BuildTieRecords(op->h_mult, op->h_shift, Cout, out_alloc, pr->out_zp - out_flip, capped(AccumulatorBound(Cexp, pr_b, Cout)), &rq3, &up[2], &ties[2]))
+      return TVX_E_UNSUPPORTED;
+    a.pre1 = up[0] * 2 + ties[0]; a.pre2 = up[1] * 2 + ties[1]; a.pre3 = up[2] * 2 + ties[2];
+    a.e_lo -= e_flip; a.e_hi -= e_flip;
+    a.m_lo -= m_flip; a.m_hi -= m_flip;
+    a.lo -= out_flip; a.hi -= out_flip;
+    const auto narrow = [](int lo, int hi) { return lo > -128 || hi < 127; };
+    a.narrow1 = narrow(a.e_lo, a.e_hi); a.narrow2 = narrow(a.m_lo, a.m_hi); a.narrow3 = narrow(a.lo, a.hi);
+    a.out_xor4 = out_flip ? static_cast<int>(0x80808080u) : 0;
+    a.dw_nzws3 = (-zwd & 0xff) * 0x010101;
+    const bool plain = !(a.pre1 | a.pre2 | a.pre3 | a.narrow1 | a.narrow2 | a.narrow3) && !(a.dw_box && zwd == -128);
+    const int widest = std::max(cin_steps, nt);
+    plan.tile_fn = wide ? TileKernelOf<true>(widest, a.add_mode, plain) : TileKernelOf<false>(widest, a.add_mode, plain);
+  } else {
+    plan.fn = a.add_mode ? KernelOf<true>(W, nt) : KernelOf<false>(W, nt);
+  }
 
   // ---- one device image: [w1 | w2 | b1 | q1 | dwk | q2 | b3 | q3], every part 16-byte aligned ----
   std::vector<uint8_t> blob;
@@ -610,7 +1059,7 @@ int MbConvSetup(tvx_op* op, const MbStage& ex, const MbStage& dw, const tvx_conv
   a.b3 = reinterpret_cast<const int32_t*>(base + o_b3);
   a.q3 = reinterpret_cast<const v4i*>(base + o_q3);
 
-  const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel(plan)),
+  const hipError_t err = hipFuncSetAttribute(plan.tile_fn ? reinterpret_cast<const void*>(plan.tile_fn) : reinterpret_cast<const void*>(plan.fn),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, plan.lds_bytes);
   if (err != hipSuccess) return SetError(TVX_E_DEVICE, "hipFuncSetAttribute(dynamic LDS %d): %s", plan.lds_bytes, hipGetErrorString(err));
   op->host_blob.resize(sizeof(Plan));

@@ -241,6 +241,20 @@ __device__ __forceinline__ uint32_t RequantSaturate4(const int (&v)[4], int mult
   return __builtin_amdgcn_perm(ShiftSaturate2(h[2], h[3], t), ShiftSaturate2(h[0], h[1], t), 0x05040100);
 }
 
+// ... with the accumulators of BuildTieRecords (`pre`: 2 * shift + ties) and a clamp in the signed domain. PLAIN: pre is 0 and the clamp no narrower
+// than a byte.
+template <bool PLAIN>
+__device__ __forceinline__ uint32_t RequantCodes4(int (&v)[4], const tvx_v4i& q, int64_t round, int pre, int narrow, int lo, int hi) {
+  const int sh = q[1] & 31;
+  if constexpr (PLAIN) return RequantSaturate4<false>(v, q[0], sh, round, 0, 0);
+  if (pre) {  // (uniform)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] <<= pre >> 1;
+    if (pre & 1) LowerOddTies(v, q);
+  }
+  return narrow ? RequantSaturate4<true>(v, q[0], sh, round, lo << sh, ((hi + 1) << sh) - 1) : RequantSaturate4<false>(v, q[0], sh, round, 0, 0);
+}
+
 // Four accumulators of one channel requantized together (the 32-bit record forms). `ties` (wave-uniform: a kernel
 // argument) tells whether any accumulator of the operator can land on an exact .5: only then is the round-half-even
 // fix-up executed.
