@@ -3,7 +3,8 @@
 // channels of every tap to 16 and would multiply mostly zeros there; here the whole window of an
 // output pixel - its (c, ky, kx) bytes, padded to 32 or 64 - is one row of the MFMA A operand.
 //
-// Workgroup = 256 output pixels of one image x all output channels (<= 128). Each thread
+// Windows three or five taps wide are gathered into registers (ConvIm2colRegKernel, below), any others through LDS: a
+// workgroup = 256 output pixels of one image x all output channels (<= 128). Each thread
 // gathers the window of one pixel with byte loads (16 in flight, no branches: out-of-image taps
 // read a safe address and are replaced by the input zero point), keeps the window sum for the
 // zero-point expansion
@@ -12,6 +13,7 @@
 // tile) follow; the epilogue is the implicit-GEMM kernel's: requantize, pack four pixels per
 // dword, stage [oc][pixel] in LDS, copy out as contiguous runs of the WHCN output.
 #include <algorithm>
+#include <type_traits>
 
 #include "variants.h"
 
@@ -44,20 +46,15 @@ struct ImArgs {
   // c * H * W + dy * W + dx. They travel in the kernel arguments so that the (wavefront-uniform) reads
   // are scalar loads of memory nothing can write; a table in global memory is read per lane, one round
   // trip a tap.
-  // In row mode (kernels three or five taps wide, unit dilation along the row) entry r stands for a whole
-  // kernel row of a channel: dy | 1 << 16 and c * H * W + dy * W; the taps are one or two dword loads.
   int taps[64];
   int offs[64];
-  int rows;              // row mode: C * Kh
-  int rows_mask;         // row mode: the window rows in use (bit dy), all of them inside the image for most pixels
-  int total_bytes;       // row mode: size of the input tensor (< 2^31)
   int pool;              // 1: a 2 x 2 / stride-2 max pooling rides on the epilogue (the result has OH / 2 x OW / 2 pixels)
 };
 
-// KW: 0 = any window, one byte load per tap; 3 / 5 = row mode for kernels three / five taps wide
+// any window, one byte load per tap
 // (two wavefronts per SIMD at least: within 256 registers the compiler keeps MFMA accumulators in ordinary vector
 // registers, where the epilogue reads them, instead of moving every value out of the accumulation registers first)
-template <int OT, int RQ, int KW>
+template <int OT, int RQ>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) ConvIm2colKernel(ImArgs a) {
   extern __shared__ __attribute__((aligned(16))) int8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -112,119 +109,6 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
       return n <= 0 ? 0u : ((n >= 32 ? 0xffffffffu : ((1u << n) - 1u)) << lo);
     };
     const uint32_t row_ok = span_mask(ih0, a.H), col_ok = span_mask(iw0, a.W);
-    if constexpr (KW == 3 || KW == 5) {
-      // Row mode: byte loads cost the L1 a tag lookup for every few lanes, and those lookups bound the
-      // gather; the taps of a kernel row are adjacent bytes, so one (unaligned) dword fetches three of
-      // them, two dwords five. A dword may begin in front of the tensor (left padding of its first row)
-      // or end behind it: it is moved inside and shifted back. A row with no tap inside the image reads
-      // the tensor's first dword(s) and is not used.
-      constexpr int kMaxRows = 64 / KW;
-      constexpr uint32_t kColMask = (1u << KW) - 1u;
-      const int img_at = n * (a.C * a.H * a.W) + origin;
-      auto place = [&](int r, int which, bool* row_in, int* moved) {  // -> byte index of the row's dword `which` in the tensor
-        const int t = a.taps[r];
-        *row_in = ((row_ok >> (t & 0xff)) & static_cast<uint32_t>(t >> 16) & 1u) != 0;
-        const bool any = *row_in & ((col_ok & kColMask) != 0);
-        const int want = (any ? img_at + a.offs[r] : 0) + 4 * which;
-        const int at = min(max(want, 0), a.total_bytes - 4);
-        *moved = at - want;  // first dword: -3 .. 4; second: -7 .. 0
-        return at;
-      };
-      uint32_t v[kMaxRows], v2[KW == 5 ? kMaxRows : 1];
-      int dw[16];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) dw[i] = 0;
-      // Nearly every wavefront holds only pixels whose window rows all lie inside the image and whose dwords all
-      // lie inside the tensor (the exceptions: an image's first / last output rows under padding, the tensor's
-      // first and last bytes). There a row's dword sits where it is expected, nothing is moved or shifted back,
-      // and what is left of the border - the same one or two window columns outside the image in every row of a
-      // pixel - is one mask and one XOR pattern per thread: (dword & inside) ^ (re-bias where inside, the input
-      // zero point where not).
-      const int first_at = img_at + a.offs[0], last_at = img_at + a.offs[a.rows - 1] + (KW == 5 ? 4 : 0);
-      const bool plain = (row_ok & static_cast<uint32_t>(a.rows_mask)) == static_cast<uint32_t>(a.rows_mask) &&
-                         first_at >= 0 && last_at + 4 <= a.total_bytes;
-      if (__builtin_amdgcn_ballot_w64(!plain) == 0) {
-#pragma unroll
-        for (int r = 0; r < kMaxRows; ++r) {
-          v[r] = 0;
-          if (KW == 5) v2[r] = 0;
-          if (r < a.rows) {  // uniform
-            const uint32_t at = static_cast<uint32_t>(img_at + a.offs[r]);
-            __builtin_memcpy(&v[r], a.x + at, 4);
-            if constexpr (KW == 5) __builtin_memcpy(&v2[r], a.x + at + 4, 4);
-          }
-        }
-        __builtin_amdgcn_sched_barrier(0);  // all loads travel together
-        uint32_t keep = 0, flip = 0, keep2 = 0, flip2 = 0;  // per window column: 0xff where inside; re-bias or zero point
-#pragma unroll
-        for (int e = 0; e < KW; ++e) {
-          const bool inside = ((col_ok >> e) & 1u) != 0;
-          const uint32_t k8 = inside ? 0xffu : 0u, f8 = static_cast<uint32_t>(inside ? a.xor_mask : a.pad_fill) & 0xffu;
-          if (e < 4) keep |= k8 << (8 * e), flip |= f8 << (8 * e);
-          else keep2 = k8, flip2 = f8;
-        }
-#pragma unroll
-        for (int r = 0; r < kMaxRows; ++r) {
-          if (r < a.rows) {
-            const int k = r * KW, i = k >> 2, pos = k & 3;  // (constants once unrolled)
-            const uint32_t row = (v[r] & keep) ^ flip;  // KW == 3: the fourth byte is masked away
-            dw[i] |= static_cast<int>(row << (8 * pos));
-            if (pos + (KW == 3 ? 3 : 4) > 4) dw[i + 1] |= static_cast<int>(row >> (8 * (4 - pos)));
-            if constexpr (KW == 5) {
-              const int k5 = k + 4;
-              dw[k5 >> 2] |= static_cast<int>(((v2[r] & keep2) ^ flip2) << (8 * (k5 & 3)));
-            }
-          }
-        }
-      } else {
-#pragma unroll
-      for (int r = 0; r < kMaxRows; ++r) {
-        v[r] = 0;
-        if (KW == 5) v2[r] = 0;
-        if (r < a.rows) {  // uniform
-          bool row_in;
-          int moved;
-          const int at = place(r, 0, &row_in, &moved);
-          __builtin_memcpy(&v[r], a.x + static_cast<uint32_t>(at), 4);
-          if constexpr (KW == 5) {
-            const int at2 = place(r, 1, &row_in, &moved);
-            __builtin_memcpy(&v2[r], a.x + static_cast<uint32_t>(at2), 4);
-          }
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);  // all loads travel together
-#pragma unroll
-      for (int r = 0; r < kMaxRows; ++r) {
-        if (r < a.rows) {
-          bool row_in;
-          int moved;
-          (void)place(r, 0, &row_in, &moved);
-          // (moved by a whole dword - a five-tap row four columns in front of the tensor: every tap is masked)
-          const uint32_t got = moved >= 4 ? 0u : (moved >= 0 ? v[r] << (8 * moved) : v[r] >> (-8 * moved));
-          uint32_t got2 = 0;  // (fifth tap: the second dword's first byte)
-          if constexpr (KW == 5) {
-            (void)place(r, 1, &row_in, &moved);
-            got2 = moved <= -4 ? 0u : v2[r] >> (-8 * moved);  // (moved by four bytes or more: the tap lies behind the tensor and is masked)
-          }
-#pragma unroll
-          for (int e = 0; e < KW; ++e) {
-            const bool inside = row_in & (((col_ok >> e) & 1u) != 0);
-            const uint32_t raw = e < 4 ? (got >> (8 * e)) & 0xffu : got2 & 0xffu;
-            const int byte = inside ? static_cast<int>(raw ^ static_cast<uint32_t>(a.xor_mask)) : a.pad_fill;
-            const int k = r * KW + e;
-            dw[k >> 2] |= byte << (8 * (k & 3));
-          }
-        }
-      }
-      }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) sx = __builtin_amdgcn_sdot4(dw[i], 0x01010101, sx, false);
-      for (int k0 = 0; k0 < a.kp; k0 += 16) {
-        const int i = k0 >> 2;
-        const v4i out = i == 0 ? v4i{dw[0], dw[1], dw[2], dw[3]} : (i == 4 ? v4i{dw[4], dw[5], dw[6], dw[7]} : (i == 8 ? v4i{dw[8], dw[9], dw[10], dw[11]} : v4i{dw[12], dw[13], dw[14], dw[15]}));
-        *reinterpret_cast<v4i*>(a_lds + tid * a.row_stride + k0) = out;
-      }
-    } else
     for (int k0 = 0; k0 < a.kp; k0 += 16) {
       int b[16];
       bool inside[16];
@@ -330,29 +214,271 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   }
 }
 
+// ---- windows three or five taps wide, undilated along the row: the operand in registers ----
+//
+// A reduction step of the matrix product takes 32 bytes of a window, sixteen from either lane half; a half is given five (three) whole
+// kernel rows of three (five) taps, and the weights are packed in the same order. A lane thus gathers its own fragment - an unaligned
+// load a row - and nothing passes through LDS: no barrier, every wavefront goes its own way through a run of 32-pixel tiles, with
+// the next tile's loads in flight. Pixel 4 i + e of a tile stands in row 8 e + i of the product, so that a lane finds sixteen
+// consecutive pixels of a channel (or the candidates of four consecutive pooled ones) in its accumulators and stores them from there. The
+// window sums of the zero-point expansion are a product with a constant fragment.
+// Bound by the latency of the chain in small layers, by the vector ALU (6.5 of the 14 us below) and by stores of 32 bytes a channel and tile in
+// large ones. Before (every pixel's window through LDS, results staged there, three barriers) and now, microseconds, uint8: 3 x 3 at
+// stride 2 on 224 x 224, 3 to 32: batch 1 6.0 / 2.7, batch 64 18.3 / 14.3; 5 x 5 on 28 x 28, 1 to 20, pooled: batch 1 5.6 / 2.4, batch 207 6.8 / 3.8.
+struct ImRegArgs {
+  const uint8_t* x;
+  const v4i* w;          // [channel tile][step][64 lanes], then the constant fragments [step][64 lanes]
+  const int32_t* biasf;
+  const v4i* rq;
+  int offs[2][16];       // per lane half and kernel row: c * H * W + dy * W
+  int dys[2][16];
+  int image, W, H, OW, hw, sh, sw, pad_t, pad_l;
+  int tiles_per_image, tiles, run;  // run: tiles of a wavefront
+  uint32_t m_tiles, m_ow;           // reciprocals (of the pooled width under a pooling)
+  int last, max_off;     // highest index a load may start at; highest of the offsets
+  int max_dy;            // lowest window row
+  uint32_t flip_in, flip_out;  // a window byte inside the image is moved to the signed domain, one outside is the zero point: all four bytes
+  int ztwice;            // the constant fragment holds half of minus the weights' zero point, 128, and is taken twice
+  uint8_t* y;
+  int OC, pre, narrow, lo, hi, out_xor4, out_zp, generic;
+};
+
+// PLAIN: no ties, narrow clamps, 64-bit products or second constant, and factors below 2^23.
+template <int KW, int KS, int OT, bool PLAIN, bool POOL>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) ConvIm2colRegKernel(ImRegArgs a) {
+  constexpr int kRows = KW == 3 ? 5 : 3, kDw = KW == 3 ? 1 : 2;  // kernel rows of a lane half and step; dwords of each
+  const int lane = threadIdx.x & 63, col = lane & 31, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int wg = blockIdx.x;  // an XCD gets a contiguous run of tiles: neighbours share input rows in its L2
+  {
+    const int per = gridDim.x >> 3, rem = gridDim.x & 7, xcd = wg & 7;
+    wg = xcd * per + min(xcd, rem) + (wg >> 3);
+  }
+  int t = (wg * static_cast<int>(blockDim.x >> 6) + wave) * a.run;
+  const int t_end = min(t + a.run, a.tiles);
+  if (t >= t_end) return;
+  // v / d by the reciprocal rounded up, which is never too small and at most one too large (m = 0: d = 1)
+  const auto times = [](int v, int w) { return PLAIN ? __mul24(v, w) : v * w; };
+  const auto over = [&](int v, uint32_t m, int d) {
+    const int q = static_cast<int>(__umulhi(static_cast<uint32_t>(v), m) + (static_cast<uint32_t>(v) & (m ? 0u : ~0u)));
+    return q - (times(q, d) > v ? 1 : 0);
+  };
+
+  const auto image = [](int tile, uint32_t m, int d) {  // (uniform)
+    const int q = static_cast<int>(__umulhi(static_cast<uint32_t>(tile), m) + (static_cast<uint32_t>(tile) & (m ? 0u : ~0u)));
+    return q - (static_cast<uint32_t>(q) * static_cast<uint32_t>(d) > static_cast<uint32_t>(tile) ? 1 : 0);
+  };
+
+  int off[KS * kRows];
+#pragma unroll
+  for (int j = 0; j < KS * kRows; ++j) off[j] = half ? a.offs[1][j] : a.offs[0][j];
+  struct Raw {
+    uint32_t v[KS * kRows][kDw];
+    int at, iw0;        // of the window's origin
+    int ih0;
+  };
+  const int slot = 4 * (col & 7) + (col >> 3);  // the pixel of this lane's row of a product
+  const auto load = [&](int tile) {
+    Raw r;
+    const int n = image(tile, a.m_tiles, a.tiles_per_image);
+    const int p = min((tile - n * a.tiles_per_image) * 32 + slot, a.hw - 1);  // (past the end the last pixel again: nobody stores it)
+    int oh, ow;
+    if constexpr (POOL) {  // four consecutive pixels are a 2 x 2 window, windows row-major over the pooled image
+      const int pw = a.OW >> 1, qh = over(p >> 2, a.m_ow, pw);
+      oh = 2 * qh + (p >> 1 & 1);
+      ow = 2 * ((p >> 2) - times(qh, pw)) + (p & 1);
+    } else {
+      oh = over(p, a.m_ow, a.OW);
+      ow = p - times(oh, a.OW);
+    }
+    r.ih0 = times(oh, a.sh) - a.pad_t;
+    r.iw0 = times(ow, a.sw) - a.pad_l;
+    r.at = n * a.image + times(r.ih0, a.W) + r.iw0;
+#pragma unroll
+    for (int j = 0; j < KS * kRows; ++j) __builtin_memcpy(r.v[j], a.x + static_cast<uint32_t>(Med3(r.at + off[j], 0, a.last)), 4 * kDw);
+    return r;
+  };
+  Raw cur = load(t);
+
+  // ---- under these loads: weights, tables ----
+  const ImRegArgs& b = LateArgs<ImRegArgs>();
+  v4i fw[OT][KS], fz[KS], q[OT];
+  int bias[OT];
+#pragma unroll
+  for (int j = 0; j < OT; ++j) {
+#pragma unroll
+    for (int k = 0; k < KS; ++k) fw[j][k] = b.w[(j * KS + k) * 64 + lane];
+    q[j] = b.rq[j * 32 + col];
+    bias[j] = b.biasf[j * 32 + col];
+  }
+#pragma unroll
+  for (int k = 0; k < KS; ++k) fz[k] = b.w[(OT * KS + k) * 64 + lane];
+  const int W = b.W, last = b.last, max_off = b.max_off, ztwice = b.ztwice, OC = b.OC, tiles_per_image = b.tiles_per_image, hw = b.hw;
+  const int hw_y = POOL ? hw >> 2 : hw;
+  const int H = b.H, below = H - 1 - b.max_dy;
+  const uint32_t m_tiles = b.m_tiles, flip_in = b.flip_in, flip_out = b.flip_out, out_xor4 = static_cast<uint32_t>(b.out_xor4);
+  uint8_t* const y = b.y;
+  const size_t lane_y = static_cast<size_t>(col) * hw_y;
+  int dy[KS * kRows];
+#pragma unroll
+  for (int j = 0; j < KS * kRows; ++j) dy[j] = half ? b.dys[1][j] : b.dys[0][j];
+
+  // (a plain requantization takes the bias in its rounding constant: mult * (acc + bias) + round)
+  int64_t rounds[OT];
+#pragma unroll
+  for (int j = 0; j < OT; ++j) rounds[j] = static_cast<int64_t>(static_cast<uint64_t>(static_cast<uint32_t>(q[j][2])) << 32) + static_cast<int64_t>(q[j][0]) * bias[j];
+
+  for (;;) {
+    const bool more = t + 1 < t_end;
+    Raw next = cur;
+    if (more) next = load(t + 1);
+    if (__builtin_amdgcn_ballot_w64(cur.at < 0 || cur.at > last - max_off)) {  // a load at the tensor's ends was moved inside
+#pragma unroll
+      for (int j = 0; j < KS * kRows; ++j) {
+        const int at = cur.at + off[j], by = min(max(min(max(at, 0), last) - at, -4 * kDw), 4 * kDw);
+        uint64_t v = cur.v[j][0];
+        if (kDw == 2) v |= static_cast<uint64_t>(cur.v[j][kDw - 1]) << 32;
+        v = by > 4 * kDw - 1 || by < 1 - 4 * kDw ? 0 : by > 0 ? v << (8 * by) : v >> (-8 * by);
+        cur.v[j][0] = static_cast<uint32_t>(v);
+        if (kDw == 2) cur.v[j][kDw - 1] = static_cast<uint32_t>(v >> 32);
+      }
+    }
+    // window columns outside the image, the same in each row: (byte & keep) ^ flip
+    uint32_t keep[kDw], flip[kDw];
+    {
+      typedef std::conditional_t<KW == 3, uint32_t, uint64_t> Bytes;
+      constexpr Bytes kAll = static_cast<Bytes>((1ull << (8 * KW)) - 1);
+      const int left = min(max(-cur.iw0, 0), KW), right = KW - min(max(W - cur.iw0, 0), KW);
+      const Bytes k = (kAll << (8 * left)) & (kAll >> (8 * right));
+#pragma unroll
+      for (int i = 0; i < kDw; ++i) {
+        keep[i] = static_cast<uint32_t>(static_cast<uint64_t>(k) >> (32 * i));
+        flip[i] = ((flip_in ^ flip_out) & keep[i]) ^ (flip_out & static_cast<uint32_t>(static_cast<uint64_t>(kAll) >> (32 * i)));
+      }
+    }
+    if (__builtin_amdgcn_ballot_w64(cur.ih0 < 0 || cur.ih0 > below) == 0) {  // every window row lies inside the image
+#pragma unroll
+      for (int j = 0; j < KS * kRows; ++j)
+#pragma unroll
+        for (int i = 0; i < kDw; ++i) cur.v[j][i] = (cur.v[j][i] & keep[i]) ^ flip[i];
+    } else {
+#pragma unroll
+      for (int j = 0; j < KS * kRows; ++j) {
+        const uint32_t in = static_cast<unsigned>(cur.ih0 + dy[j]) < static_cast<unsigned>(H) ? ~0u : 0u;
+#pragma unroll
+        for (int i = 0; i < kDw; ++i) {
+          const uint32_t all = KW == 3 ? 0xffffffu : i ? 0xffu : ~0u;
+          cur.v[j][i] = (((cur.v[j][i] & keep[i]) ^ flip[i]) & in) | (flip_out & all & ~in);
+        }
+      }
+    }
+    v4i fx[KS];
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      const uint32_t (*v)[kDw] = cur.v + k * kRows;
+      uint32_t d[4];
+      if constexpr (KW == 3) {
+        d[0] = v[0][0] | v[1][0] << 24;
+        d[1] = __builtin_amdgcn_perm(v[2][0], v[1][0], 0x05040201);
+        d[2] = v[2][0] >> 16 | v[3][0] << 8;
+        d[3] = v[4][0];
+      } else {
+        d[0] = v[0][0];
+        d[1] = v[0][kDw - 1] | v[1][0] << 8;
+        d[2] = __builtin_amdgcn_perm(v[1][kDw - 1], v[1][0], 0x0c0c0403) | v[2][0] << 16;
+        d[3] = v[2][0] >> 16 | v[2][kDw - 1] << 16;
+      }
+      fx[k] = v4i{static_cast<int>(d[0]), static_cast<int>(d[1]), static_cast<int>(d[2]), static_cast<int>(d[3])};
+    }
+    const int n = image(t, m_tiles, tiles_per_image), p0 = (t - n * tiles_per_image) * 32;
+    // what of this lane's sixteen pixels (four pooled ones) exists
+    const int first = POOL ? (p0 >> 2) + 4 * half : p0 + 16 * half;
+    const int live = hw_y - first;
+    v16i zsum;  // the window sums' part
+#pragma unroll
+    for (int r = 0; r < 16; ++r) zsum[r] = 0;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) zsum = __builtin_amdgcn_mfma_i32_32x32x32_i8(fx[k], fz[k], zsum, 0, 0, 0);
+    if constexpr (!PLAIN)
+      if (ztwice)  // (uniform)
+#pragma unroll
+        for (int k = 0; k < KS; ++k) zsum = __builtin_amdgcn_mfma_i32_32x32x32_i8(fx[k], fz[k], zsum, 0, 0, 0);
+    uint8_t* const tile_y = y + static_cast<size_t>(n) * OC * hw_y + first;
+#pragma unroll
+    for (int j = 0; j < OT; ++j) {
+      v16i acc = zsum;
+#pragma unroll
+      for (int k = 0; k < KS; ++k) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fx[k], fw[j][k], acc, 0, 0, 0);
+      if constexpr (!PLAIN)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] += bias[j];
+      const int oc = j * 32 + col;
+      const int64_t round = PLAIN ? rounds[j] : RoundHigh(q[j][2]);
+      const auto codes = [&](int (&v)[4]) {
+        if constexpr (!PLAIN)
+          if (b.generic) return RequantPack4<kRqGeneric>(v, q[j], b.out_zp, b.lo, b.hi);
+        return RequantCodes4<PLAIN>(v, q[j], round, b.pre, b.narrow, b.lo, b.hi) ^ out_xor4;
+      };
+      uint8_t* const to = tile_y + lane_y + static_cast<size_t>(j * 32) * hw_y;
+      constexpr int kOut = POOL ? 1 : 4;
+      uint32_t out[kOut];
+      // accumulator 4 e + i is row 8 e + 4 half + i of the product: pixel 16 half + 4 i + e
+      if constexpr (POOL) {  // requantization is monotone: a window's largest accumulator gives its largest code
+        int v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = max(max(acc[i], acc[4 + i]), max(acc[8 + i], acc[12 + i]));
+        out[0] = codes(v);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          int v[4] = {acc[i], acc[4 + i], acc[8 + i], acc[12 + i]};
+          out[i] = codes(v);
+        }
+      }
+      if (oc >= OC || live <= 0) continue;
+      if (live >= 4 * kOut) {
+        __builtin_memcpy(to, out, 4 * kOut);
+      } else {
+#pragma unroll
+        for (int i = 0; i < kOut; ++i) {
+          if (live >= 4 * i + 4) {
+            __builtin_memcpy(to + 4 * i, &out[i], 4);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+              if (live > 4 * i + e) to[4 * i + e] = static_cast<uint8_t>(out[i] >> (8 * e));
+          }
+        }
+      }
+    }
+    if (!more) break;
+    ++t;
+    cur = next;
+  }
+}
+
+struct RegPlan {
+  ImRegArgs a;
+  void (*fn)(ImRegArgs);
+  unsigned grid, block;
+};
+
 struct Plan {
   ImArgs a;
   int lds_bytes;
-  int ot, rq, row_mode;
+  int ot, rq;
   dim3 grid;
 };
 
-template <int OT, int KW>
-void LaunchRq(const Plan* plan, const ImArgs& a, hipStream_t st) {
+template <int OT>
+void Launch(const Plan* plan, const ImArgs& a, hipStream_t st) {
   const dim3 block(kThreads);
   if (plan->rq == kRqFastNoTie)
-    hipLaunchKernelGGL((ConvIm2colKernel<OT, kRqFastNoTie, KW>), plan->grid, block, plan->lds_bytes, st, a);
+    hipLaunchKernelGGL((ConvIm2colKernel<OT, kRqFastNoTie>), plan->grid, block, plan->lds_bytes, st, a);
   else if (plan->rq == kRqFast)
-    hipLaunchKernelGGL((ConvIm2colKernel<OT, kRqFast, KW>), plan->grid, block, plan->lds_bytes, st, a);
+    hipLaunchKernelGGL((ConvIm2colKernel<OT, kRqFast>), plan->grid, block, plan->lds_bytes, st, a);
   else
-    hipLaunchKernelGGL((ConvIm2colKernel<OT, kRqGeneric, KW>), plan->grid, block, plan->lds_bytes, st, a);
-}
-
-template <int KW>
-void LaunchOt(const Plan* plan, const ImArgs& a, hipStream_t st) {
-  if (plan->ot == 1) LaunchRq<1, KW>(plan, a, st);
-  else if (plan->ot == 2) LaunchRq<2, KW>(plan, a, st);
-  else LaunchRq<4, KW>(plan, a, st);
+    hipLaunchKernelGGL((ConvIm2colKernel<OT, kRqGeneric>), plan->grid, block, plan->lds_bytes, st, a);
 }
 
 int ConvIm2colRun(tvx_op* op, const void* in0, const void*, void* out, hipStream_t st) {
@@ -360,10 +486,127 @@ int ConvIm2colRun(tvx_op* op, const void* in0, const void*, void* out, hipStream
   ImArgs a = plan->a;
   a.x = static_cast<const uint8_t*>(in0);
   a.y = static_cast<uint8_t*>(out);
-  if (plan->row_mode == 5) LaunchOt<5>(plan, a, st);
-  else if (plan->row_mode) LaunchOt<3>(plan, a, st);
-  else LaunchOt<0>(plan, a, st);
+  if (plan->ot == 1) Launch<1>(plan, a, st);
+  else if (plan->ot == 2) Launch<2>(plan, a, st);
+  else Launch<4>(plan, a, st);
   TVX_HIP_CHECK(hipGetLastError());
+  return TVX_OK;
+}
+
+typedef void (*RegFn)(ImRegArgs);
+
+template <int KW, int KS, bool PLAIN, bool POOL>
+RegFn RegKernel(int ot) {
+  return ot == 1 ? ConvIm2colRegKernel<KW, KS, 1, PLAIN, POOL> : ot == 2 ? ConvIm2colRegKernel<KW, KS, 2, PLAIN, POOL> : ConvIm2colRegKernel<KW, KS, 4, PLAIN, POOL>;
+}
+template <bool PLAIN, bool POOL>
+RegFn RegKernel(int kw, int ks, int ot) {
+  if (kw == 5) return ks == 1 ? RegKernel<5, 1, PLAIN, POOL>(ot) : RegKernel<5, 2, PLAIN, POOL>(ot);
+  return ks == 1 ? RegKernel<3, 1, PLAIN, POOL>(ot) : ks == 2 ? RegKernel<3, 2, PLAIN, POOL>(ot) : RegKernel<3, 3, PLAIN, POOL>(ot);
+}
+
+int ConvIm2colRegRun(tvx_op* op, const void* in0, const void*, void* out, hipStream_t st) {
+  const RegPlan* plan = reinterpret_cast<const RegPlan*>(op->host_blob.data());
+  ImRegArgs a = plan->a;
+  a.x = static_cast<const uint8_t*>(in0);
+  a.y = static_cast<uint8_t*>(out);
+  hipLaunchKernelGGL(plan->fn, dim3(plan->grid), dim3(plan->block), 0, st, a);
+  TVX_HIP_CHECK(hipGetLastError());
+  return TVX_OK;
+}
+
+// The register form: windows three or five taps wide, undilated along the row.
+int RegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const void* bias_host, int zxs, int zws) {
+  const int kw = static_cast<int>(d->k_w), C = d->in_c, kh = d->k_h, rows = C * kh;
+  const uint64_t total = static_cast<uint64_t>(d->batch) * d->in_c * d->in_h * d->in_w;
+  const uint64_t out_pixels = static_cast<uint64_t>(d->out_h) * d->out_w, tpi = (out_pixels + 31) / 32, tiles = tpi * d->batch;
+  if ((kw != 3 && kw != 5) || d->dilation_w != 1 || total < 8 || total >= (1ull << 31) - 64 || tiles >= (1ull << 31) - 4096) return TVX_E_UNSUPPORTED;
+  if (const char* f = getenv("TVX_IM2COL_ROWS"))  // tuning aid
+    if (!atoi(f)) return TVX_E_UNSUPPORTED;
+  const int per = kw == 3 ? 5 : 3, ks = (rows + 2 * per - 1) / (2 * per), K = rows * kw;
+  if (ks > (kw == 3 ? 3 : 2)) return TVX_E_UNSUPPORTED;
+  const bool x_u8 = d->in_dtype == TVX_U8, w_u8 = d->w_dtype == TVX_U8;
+  RegPlan plan{};
+  ImRegArgs& a = plan.a;
+  const int pool = op->fused_pool;
+  a.image = C * static_cast<int>(d->in_h) * static_cast<int>(d->in_w);
+  a.W = d->in_w; a.H = d->in_h; a.OW = d->out_w; a.hw = static_cast<int>(out_pixels);
+  a.sh = d->stride_h; a.sw = d->stride_w; a.pad_t = d->pad_top; a.pad_l = d->pad_left;
+  const auto reciprocal = [](uint64_t v) { return v > 1 ? static_cast<uint32_t>(((1ull << 32) + v - 1) / v) : 0u; };
+  a.tiles_per_image = static_cast<int>(tpi); a.tiles = static_cast<int>(tiles);
+  a.m_tiles = reciprocal(tpi);
+  a.m_ow = reciprocal(pool ? d->out_w / 2 : d->out_w);
+  a.last = static_cast<int>(total) - (kw == 3 ? 4 : 8);
+  a.flip_in = x_u8 ? 0x80808080u : 0u;
+  a.flip_out = static_cast<uint32_t>(zxs & 0xff) * 0x01010101u;
+  a.OC = d->out_c;
+  for (int r = 0; r < rows; ++r) {
+    const int dy = r % kh * static_cast<int>(d->dilation_h), group = r / per;
+    a.offs[group & 1][group / 2 * per + r % per] = (r / kh * a.H + dy) * a.W;
+    a.dys[group & 1][group / 2 * per + r % per] = dy;
+    a.max_dy = std::max(a.max_dy, dy);
+    a.max_off = std::max(a.max_off, (r / kh * a.H + dy) * a.W);
+  }
+  a.ztwice = zws == -128;
+  const int ot = d->out_c <= 32 ? 1 : d->out_c <= 64 ? 2 : 4, alloc = 32 * ot;
+  std::vector<int8_t> packed(static_cast<size_t>(ot + 1) * ks * 1024, 0);
+  std::vector<int32_t> biasf(alloc, 0);
+  const uint8_t* src = static_cast<const uint8_t*>(w_host);
+  const int32_t* b = static_cast<const int32_t*>(bias_host);
+  // byte k of a window -> [step][half][16 bytes]
+  const auto place = [&](int tile, int column, int k) {
+    const int r = k / kw, group = r / per;
+    return ((static_cast<size_t>(tile) * ks + group / 2) * 64 + (group & 1) * 32 + column) * 16 + r % per * kw + k % kw;
+  };
+  for (int oc = 0; oc < a.OC; ++oc) {
+    int64_t sum = 0;
+    for (int k = 0; k < K; ++k) {
+      const uint8_t raw = src[static_cast<size_t>(oc) * K + k];
+      const int8_t v = static_cast<int8_t>(w_u8 ? raw ^ 0x80 : raw);
+      packed[place(oc / 32, oc % 32, k)] = v;
+      sum += v;
+    }
+    const int64_t v = (b ? b[oc] : 0) - static_cast<int64_t>(zxs) * sum + static_cast<int64_t>(K) * zxs * zws;
+    biasf[oc] = static_cast<int32_t>(static_cast<uint32_t>(v));
+  }
+  for (int column = 0; column < 32; ++column)
+    for (int k = 0; k < K; ++k) packed[place(ot, column, k)] = static_cast<int8_t>(a.ztwice ? 64 : -zws);
+  const int64_t bound = AccumulatorBound(static_cast<uint64_t>(K), bias_host, a.OC);
+  const int flip = d->out_dtype == TVX_U8 ? 128 : 0;
+  std::vector<int32_t> rqt;
+  int up = 0;
+  bool ties = false;
+  a.out_zp = d->out_zp; a.lo = op->act_lo; a.hi = op->act_hi;
+  a.generic = BuildRequantRecords(op->h_mult, op->h_shift, a.OC, alloc, d->out_zp, &rqt, bound) == kRqGeneric;
+  if (!a.generic) {
+    if (!BuildTieRecords(op->h_mult, op->h_shift, a.OC, alloc, d->out_zp - flip, std::min<int64_t>(bound, INT32_MAX), &rqt, &up, &ties)) return TVX_E_UNSUPPORTED;
+    a.lo -= flip; a.hi -= flip;
+    a.narrow = a.lo > -128 || a.hi < 127;
+    a.pre = up * 2 + ties;
+    a.out_xor4 = flip ? static_cast<int>(0x80808080u) : 0;
+  }
+  int s = op->packed.Upload(packed.data(), packed.size());
+  if (s == TVX_OK) s = op->aux.Upload(biasf.data(), biasf.size() * 4);
+  if (s == TVX_OK) s = op->aux2.Upload(rqt.data(), rqt.size() * 4);
+  if (s != TVX_OK) return s;
+  a.w = op->packed.as<v4i>();
+  a.biasf = op->aux.as<int32_t>();
+  a.rq = op->aux2.as<v4i>();
+  const bool small = out_pixels < (1u << 23) && d->in_h < (1u << 23) && d->in_w < (1u << 23) && d->stride_h < (1u << 23) && d->stride_w < (1u << 23) && d->pad_top < (1u << 22);
+  const bool plain = !a.generic && !a.narrow && !a.pre && !a.ztwice && small;
+  plan.fn = pool ? (plain ? RegKernel<true, true>(kw, ks, ot) : RegKernel<false, true>(kw, ks, ot)) : plain ? RegKernel<true, false>(kw, ks, ot) : RegKernel<false, false>(kw, ks, ot);
+  // a wavefront's run: one tile until every SIMD has a few wavefronts (the first of the layers above at batch 64, 98 tiles a CU: 16.1 us with
+  // runs of one, 14.6 two, 14.2 three, 14.8 four, 15.6 six; at batch 1, 1.5 a CU: 2.7, 3.3, 3.8, 4.7, 5.0)
+  const int cus = ComputeUnits();
+  a.run = static_cast<int>(std::min<uint64_t>(8, std::max<uint64_t>(1, tiles / (32ull * cus))));
+  if (const char* f = getenv("TVX_IM2COL_RUN")) a.run = std::max(1, atoi(f));  // test lever
+  const uint64_t waves = (tiles + a.run - 1) / a.run;
+  const int per_wg = waves <= 2ull * cus ? 1 : kThreads / 64;
+  plan.block = 64 * per_wg;
+  plan.grid = static_cast<unsigned>((waves + per_wg - 1) / per_wg);
+  op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
+  op->run = ConvIm2colRegRun;
+  op->kernel_name = pool ? "conv2d_im2col_maxpool_i8" : "conv2d_im2col_i8";
   return TVX_OK;
 }
 
@@ -391,6 +634,9 @@ int ConvIm2colSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, co
   const int zxs = d->in_zp - (x_u8 ? 128 : 0);
   const int zws = op->w_zp - (w_u8 ? 128 : 0);
   if (zxs < -128 || zxs > 127) return TVX_E_UNSUPPORTED;  // zero point outside the tensor's range
+  if ((d->k_h - 1) * d->dilation_h > 31 || (d->k_w - 1) * d->dilation_w > 31) return TVX_E_UNSUPPORTED;  // window offsets index 32-bit masks
+  const int reg = RegSetup(op, d, w_host, bias_host, zxs, zws);
+  if (reg != TVX_E_UNSUPPORTED) return reg;
   a.xor_mask = x_u8 ? 0x80 : 0;
   a.pad_fill = zxs & 0xff;
   a.zws = zws;
@@ -424,28 +670,12 @@ int ConvIm2colSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, co
   std::vector<int32_t> rqt;
   const int rq = BuildRequantRecords(op->h_mult, op->h_shift, a.OC, a.oct, d->out_zp, &rqt,
                                      AccumulatorBound(static_cast<uint64_t>(K), bias_host, a.OC));
-  if ((d->k_h - 1) * d->dilation_h > 31 || (d->k_w - 1) * d->dilation_w > 31) return TVX_E_UNSUPPORTED;  // window offsets index 32-bit masks
-  const uint64_t total_bytes = static_cast<uint64_t>(d->batch) * d->in_c * d->in_h * d->in_w;
-  bool row_mode = (d->k_w == 3 || d->k_w == 5) && d->dilation_w == 1 && total_bytes >= 4 && total_bytes < (1ull << 31);
-  if (const char* f = getenv("TVX_IM2COL_ROWS")) row_mode = row_mode && atoi(f) != 0;  // tuning aid
-  if (row_mode) {
-    a.rows = static_cast<int>(d->in_c * d->k_h);
-    a.total_bytes = static_cast<int>(total_bytes);
-    for (int r = 0; r < a.rows; ++r) {
-      const int c = r / static_cast<int>(d->k_h);
-      const int dy = (r % static_cast<int>(d->k_h)) * static_cast<int>(d->dilation_h);
-      a.taps[r] = dy | 1 << 16;
-      a.offs[r] = c * a.H * a.W + dy * a.W;
-      a.rows_mask |= 1 << dy;
-    }
-  } else {
-    for (int k = 0; k < K; ++k) {
-      const int c = k / taps, t = k % taps;
-      const int dy = (t / static_cast<int>(d->k_w)) * static_cast<int>(d->dilation_h);
-      const int dx = (t % static_cast<int>(d->k_w)) * static_cast<int>(d->dilation_w);
-      a.taps[k] = dy | dx << 8 | 1 << 16;
-      a.offs[k] = c * a.H * a.W + dy * a.W + dx;
-    }
+  for (int k = 0; k < K; ++k) {
+    const int c = k / taps, t = k % taps;
+    const int dy = (t / static_cast<int>(d->k_w)) * static_cast<int>(d->dilation_h);
+    const int dx = (t % static_cast<int>(d->k_w)) * static_cast<int>(d->dilation_w);
+    a.taps[k] = dy | dx << 8 | 1 << 16;
+    a.offs[k] = c * a.H * a.W + dy * a.W + dx;
   }
   int s = op->packed.Upload(packed.data(), packed.size());
   if (s == TVX_OK) s = op->aux.Upload(biasf.data(), biasf.size() * 4);
@@ -460,7 +690,6 @@ int ConvIm2colSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, co
   plan.lds_bytes = lds_bytes;
   plan.ot = ot;
   plan.rq = rq;
-  plan.row_mode = row_mode ? static_cast<int>(d->k_w) : 0;  // 0, or the taps of a kernel row (3 / 5)
   const int hw = a.OH * a.OW;
   plan.grid = dim3(static_cast<unsigned>((hw + kPixels - 1) / kPixels), static_cast<unsigned>(d->batch));
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));

@@ -34,7 +34,7 @@ bool ConvIgemmPersists(const tvx_conv2d_desc*);
 int ConvTileSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 // the same for layers whose weights and two halo tiles fit LDS: one sixteen-wavefront workgroup per CU (conv_band_i8.hip)
 int ConvBandSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
-// Dense quantized conv whose whole window (C * Kh * Kw) is at most 64 bytes: im2col rows in LDS + MFMA.
+// Dense quantized conv whose whole window (C * Kh * Kw) is at most 64 bytes: im2col rows in registers or LDS + MFMA.
 int ConvIm2colSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 
 // pointwise (1x1) convolution with the whole channel depth of a pixel tile in LDS (pwconv_i8.hip)
