@@ -1,0 +1,50 @@
+"""Op.run's native call against the ctypes one: the same status and error for every kind of argument. No GPU: the library checks
+its operands before it launches anything."""
+import ctypes as C
+
+import pytest
+
+import tvx_case as TC
+
+
+class _Tensor:
+    def __init__(self, address):
+        self.address = address
+
+    def data_ptr(self):
+        return self.address
+
+
+@pytest.mark.parametrize("native", [False, True], ids=["ctypes", "native"])
+def test_run_arguments(monkeypatch, native):
+    T = TC.tvx()
+    T.lib()
+    if native:
+        assert T._run is not T._ctypes_run, "lib/tvx_call.so is not built"
+    else:
+        monkeypatch.setattr(T, "_run", T._ctypes_run)
+    t = _Tensor(4096)
+    for handle in (None, C.c_void_p(None)):
+        for stream in (None, 0, C.c_void_p(0), C.POINTER(C.c_int)()):
+            op = T.Op(handle)
+            with pytest.raises(T.TvxError, match="null operator") as err:
+                op.run(t, None, 4096, stream)
+            assert err.value.status == T.E_INVALID
+    with pytest.raises(AttributeError):
+        T.Op(None).run(t, "text", t)
+
+
+def test_native_call_passes_addresses():
+    T = TC.tvx()
+    L = T.lib()
+    seen = []
+    run = C.CFUNCTYPE(C.c_int, *[C.c_void_p] * 5)(lambda *a: seen.append(a) or -3)
+    module = T._run.__self__
+    module.bind(C.cast(run, C.c_void_p).value)
+    try:
+        high = (1 << 47) + 16
+        assert T._run(C.c_void_p(high), _Tensor(high + 1), None, high + 2, C.c_void_p(7)) == -3
+        assert T._run(5, 6, _Tensor(0), _Tensor(8), None) == -3
+    finally:
+        module.bind(C.cast(L.tvx_op_run, C.c_void_p).value)
+    assert seen == [((1 << 47) + 16, (1 << 47) + 17, None, (1 << 47) + 18, 7), (5, 6, None, 8, None)]

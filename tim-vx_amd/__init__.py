@@ -6,6 +6,7 @@ through ctypes so tests and the benchmark can drive it with device memory
 held in torch tensors. There is no CPU path: every compute call needs a GPU.
 """
 import ctypes as C
+import importlib.util
 import os
 
 from . import build as _build
@@ -73,6 +74,26 @@ class TvxError(RuntimeError):
 
 
 _lib = None
+_run = None   # tvx_op_run by the native binding (src/op_call.c), or through ctypes
+
+
+def _ctypes_run(handle, in0, in1, out, stream):
+    def ptr(t):
+        if t is None:
+            return None
+        return t if isinstance(t, int) else t.data_ptr()
+    return lib().tvx_op_run(handle, ptr(in0), ptr(in1), ptr(out), stream)
+
+
+def _native_run(L):
+    path = os.path.join(PKG_DIR, "lib", "tvx_call.so")
+    if not os.path.exists(path):
+        return _ctypes_run
+    spec = importlib.util.spec_from_file_location("tvx_call", path)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    module.bind(C.cast(L.tvx_op_run, C.c_void_p).value)
+    return module.run
 
 
 def build(verbose=False):
@@ -82,7 +103,7 @@ def build(verbose=False):
 
 def lib():
     """The loaded C ABI. Raises if the library has not been built."""
-    global _lib
+    global _lib, _run
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise RuntimeError("%s is missing: run __graft_entry__.build() first" % LIB_PATH)
@@ -135,6 +156,7 @@ def lib():
         L.tvx_op_run.argtypes = [vp, vp, vp, vp, vp]
         L.tvx_op_destroy.argtypes = [vp]
         L.tvx_op_destroy.restype = None
+        _run = _native_run(L)
         _lib = L
     return _lib
 
@@ -156,11 +178,9 @@ class Op:
 
     def run(self, in0, in1, out, stream=None):
         """in0 / in1 / out are device pointers (ints) or torch CUDA tensors."""
-        def ptr(t):
-            if t is None:
-                return None
-            return t if isinstance(t, int) else t.data_ptr()
-        check(lib().tvx_op_run(self.handle, ptr(in0), ptr(in1), ptr(out), stream))
+        status = _run(self.handle, in0, in1, out, stream)
+        if status:
+            check(status if status is not NotImplemented else _ctypes_run(self.handle, in0, in1, out, stream))
 
     def close(self):
         if self.handle:

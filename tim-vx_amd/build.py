@@ -5,6 +5,7 @@ import glob
 import os
 import subprocess
 import sys
+import sysconfig
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 REPO = os.path.dirname(PKG_DIR)
@@ -74,8 +75,17 @@ def build_runtime(verbose=False):
           "-o", os.path.join(PKG_DIR, "lib", "tvx_graph_runner")], verbose)
 
 
+def build_binding(verbose=False):
+    """The Python binding's native call (lib/tvx_call.so); without Python's headers the binding goes through ctypes."""
+    include = sysconfig.get_paths()["include"]
+    if os.path.exists(os.path.join(include, "Python.h")):
+        _run(["gcc", "-O2", "-fPIC", "-shared", "-Wall", "-I", include, os.path.join(PKG_DIR, "src", "op_call.c"),
+              "-o", os.path.join(PKG_DIR, "lib", "tvx_call.so")], verbose)
+
+
 def build_all(verbose=False):
     build_hip(verbose)
+    build_binding(verbose)
     build_runtime(verbose)
 
 
