@@ -403,6 +403,7 @@ static int CreateConv(const tvx_conv2d_desc* d, const void* weights_host, const 
   s = TVX_E_UNSUPPORTED;
   if (fused_pool) {
     s = ConvIm2colSetup(op, d, weights_host, bias_host);
+    if (s == TVX_E_UNSUPPORTED) s = ConvPoolSetup(op, d, weights_host, bias_host);
     if (s == TVX_E_UNSUPPORTED) s = ConvIgemmSetup(op, d, weights_host, bias_host);
   } else {
     for (ConvSetupFn fn : ConvVariants()) {

@@ -37,6 +37,8 @@ int ConvBandSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 // Dense quantized conv whose whole window (C * Kh * Kw) is at most 64 bytes: im2col rows in registers or LDS + MFMA.
 int ConvIm2colSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 
+// with a 2 x 2 MAX pooling behind it, planes that fit LDS (conv_pool_i8.hip)
+int ConvPoolSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 // pointwise (1x1) convolution with the whole channel depth of a pixel tile in LDS (pwconv_i8.hip)
 int PwConvSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 
