@@ -194,18 +194,22 @@ FcQuantKernel(FcArgs a, const XT* __restrict__ x, const WT* __restrict__ w,
   y[idx] = static_cast<XT>(RequantClamp(acc, mult[n], shift[n], a.out_zp, a.lo, a.hi));
 }
 
-// (x - zx) . (w - zw) over the sixteen bytes of two vectors
+// (x - zx) . (w - zw) over the sixteen bytes of two vectors: in the signed domain, xs . ws - zws sum xs - zxs sum ws + 16 zxs zws
+// (modulo 2^32, as the sum of products is)
 template <typename XT, typename WT>
 __device__ __forceinline__ int32_t Dot16(const uint4& xv, const uint4& wv, int in_zp, int w_zp) {
+  constexpr uint32_t kFlipX = std::is_same<XT, uint8_t>::value ? 0x80808080u : 0u, kFlipW = std::is_same<WT, uint8_t>::value ? 0x80808080u : 0u;
   const uint32_t xd[4] = {xv.x, xv.y, xv.z, xv.w}, wd[4] = {wv.x, wv.y, wv.z, wv.w};
-  int32_t acc = 0;
+  int32_t dot = 0, sx = 0, sw = 0;
 #pragma unroll
-  for (int d = 0; d < 4; ++d)
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-      acc += (static_cast<int32_t>(static_cast<XT>(xd[d] >> (8 * b))) - in_zp) *
-             (static_cast<int32_t>(static_cast<WT>(wd[d] >> (8 * b))) - w_zp);
-  return acc;
+  for (int d = 0; d < 4; ++d) {
+    const int xs = static_cast<int>(xd[d] ^ kFlipX), ws = static_cast<int>(wd[d] ^ kFlipW);
+    dot = __builtin_amdgcn_sdot4(xs, ws, dot, false);
+    sx = __builtin_amdgcn_sdot4(xs, 0x01010101, sx, false);
+    sw = __builtin_amdgcn_sdot4(ws, 0x01010101, sw, false);
+  }
+  const uint32_t zx = static_cast<uint32_t>(in_zp - (kFlipX ? 128 : 0)), zw = static_cast<uint32_t>(w_zp - (kFlipW ? 128 : 0));
+  return static_cast<int32_t>(static_cast<uint32_t>(dot) - zw * static_cast<uint32_t>(sx) - zx * static_cast<uint32_t>(sw) + 16u * zx * zw);
 }
 
 // One wavefront per output: the lanes stride over K sixteen bytes at a time (consecutive lanes
@@ -219,10 +223,10 @@ FcQuantWaveKernel(FcArgs a, const XT* __restrict__ x, const WT* __restrict__ w,
                   const int32_t* __restrict__ bias, const int32_t* __restrict__ mult,
                   const int32_t* __restrict__ shift, XT* __restrict__ y, uint64_t total) {
   const int lane = threadIdx.x & 63;
-  const uint64_t idx = static_cast<uint64_t>(blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6);
+  const uint64_t idx = static_cast<uint64_t>(blockIdx.x) * (kBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (idx >= total) return;
-  const int n = idx % a.n;
-  const uint64_t m = idx / a.n;
+  const uint64_t m = total >> 32 ? idx / a.n : static_cast<uint32_t>(idx) / static_cast<uint32_t>(a.n);  // (uniform; a 64-bit division is a long chain)
+  const int n = static_cast<int>(idx - m * a.n);
   const XT* xp = x + m * a.k;
   const WT* wp = w + static_cast<uint64_t>(n) * a.k;
   int32_t acc = 0;
@@ -907,8 +911,20 @@ int SoftmaxRun(tvx_op* op, const void* in0, const void*, void* out, hipStream_t 
 // bytes at a time for every output (the row of x is loaded once), the partial sums meet in a butterfly, lane n
 // requantizes output n as the FullyConnected kernels do, and the Softmax runs across those lanes in the
 // arithmetic - and the order of additions - of SoftmaxRowKernel on the stored codes.
+// (500 to 10: 4.6 us with byte products and a butterfly of all sixteen sums, 3.3 with dot products and sums that meet by halves)
 // ---------------------------------------------------------------------------
 constexpr int kFcSmMaxN = 16;
+
+template <int KEEP>
+__device__ __forceinline__ void HalveSums(int32_t (&acc)[kFcSmMaxN], int lane) {
+  const int32_t upper = lane & (4 * KEEP) ? -1 : 0;
+#pragma unroll
+  for (int n = 0; n < KEEP; ++n) {  // (masks: a select between array elements would put the array in memory)
+    const int32_t differ = (acc[n] ^ acc[n + KEEP]) & upper;
+    acc[n] = (acc[n] ^ differ) + __shfl_xor(acc[n + KEEP] ^ differ, 4 * KEEP);
+  }
+  if constexpr (KEEP > 1) HalveSums<KEEP / 2>(acc, lane);
+}
 
 template <typename XT, typename WT>
 __global__ void __launch_bounds__(kBlock)
@@ -925,10 +941,17 @@ FcSoftmaxKernel(FcArgs a, float beta, float sm_scale, const XT* __restrict__ x, 
   // Sixteen bytes of the row and of every weight row per lane and step; the loads stand under no branch
   // (outputs past the last read the last row again, lanes past the row's end read its start and add nothing),
   // so that all of a step travel together: a row of up to 1024 bytes is one round trip to memory.
+  // The bytes behind the last whole sixteen are requested with the first step's.
   int32_t acc[kFcSmMaxN];
+  const int k16 = a.k & ~15;
+  const bool tail_ok = k16 + lane < a.k;
+  const int tail_at = tail_ok ? k16 + lane : 0;
+  const XT tail_x = xp[tail_at];
+  WT tail_w[kFcSmMaxN];
+#pragma unroll
+  for (int n = 0; n < kFcSmMaxN; ++n) tail_w[n] = w[static_cast<uint64_t>(min(n, a.n - 1)) * a.k + tail_at];
 #pragma unroll
   for (int n = 0; n < kFcSmMaxN; ++n) acc[n] = 0;
-  const int k16 = a.k & ~15;
   for (int k0 = 0; k0 < k16; k0 += 1024) {
     const int k = k0 + lane * 16;
     const bool ok = k < k16;
@@ -945,24 +968,16 @@ FcSoftmaxKernel(FcArgs a, float beta, float sm_scale, const XT* __restrict__ x, 
     }
   }
   {
-    const bool ok = k16 + lane < a.k;
-    const int kk = ok ? k16 + lane : 0;
-    const int32_t xe = static_cast<int32_t>(xp[kk]) - a.in_zp;
-    int32_t we[kFcSmMaxN];
+    const int32_t xe = tail_ok ? static_cast<int32_t>(tail_x) - a.in_zp : 0;
 #pragma unroll
-    for (int n = 0; n < kFcSmMaxN; ++n) we[n] = static_cast<int32_t>(w[static_cast<uint64_t>(min(n, a.n - 1)) * a.k + kk]) - a.w_zp;
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int n = 0; n < kFcSmMaxN; ++n) acc[n] += ok ? xe * we[n] : 0;
+    for (int n = 0; n < kFcSmMaxN; ++n) acc[n] += xe * (static_cast<int32_t>(tail_w[n]) - a.w_zp);
   }
-  int32_t mine = 0;  // output `lane` of the row
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1)
-#pragma unroll
-    for (int n = 0; n < kFcSmMaxN; ++n) acc[n] += __shfl_xor(acc[n], off);
-#pragma unroll
-  for (int n = 0; n < kFcSmMaxN; ++n)
-    if (lane == n) mine = acc[n];
+  // The lanes' sums meet by halves: a lane keeps half of its outputs and adds its partner's sums of them, four times over, which is 15
+  // exchanges where a butterfly of every output takes 96; lane 32 a + 16 b + 8 c + 4 d + e then holds output 8 a + 4 b + 2 c + d.
+  HalveSums<kFcSmMaxN / 2>(acc, lane);
+  acc[0] += __shfl_xor(acc[0], 2);
+  acc[0] += __shfl_xor(acc[0], 1);
+  const int32_t mine = __shfl(acc[0], (lane & 8) * 4 + (lane & 4) * 4 + (lane & 2) * 4 + (lane & 1) * 4);  // output `lane` of the row (lanes 0 to 15)
   const int code = RequantClamp(mine + my_bias, my_mult, my_shift, a.out_zp, a.lo, a.hi);
   // ---- Softmax over lanes 0 .. n-1 ----
   const bool live = lane < a.n;
