@@ -184,20 +184,22 @@ __global__ void __launch_bounds__(kMaxWaves * 64) __attribute__((amdgpu_waves_pe
           d[kDw] = 0;
 #pragma unroll
           for (int i = 0; i < kDw; ++i) d[i] = S == 2 && i < 2 ? raw[j][r][i] ^ a.dw_xor_mask : (raw[j][r][i] & keep[i]) ^ flip[i];
+          // (at stride 1 a window dword serves two outputs, the second by taps a byte further up)
           int win[4];
           win[0] = Window<0>(d);
-          win[1] = Window<S>(d);
+          win[1] = S == 1 ? win[0] : Window<S>(d);
           win[2] = Window<2 * S>(d);
-          win[3] = Window<3 * S>(d);
+          win[3] = S == 1 ? win[2] : Window<3 * S>(d);
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
 #pragma unroll
             for (int o = 0; o < RPT; ++o) {
               const int ky = r - S * o;
               if (ky < 0 || ky > 2) continue;
-              acc[o][i] = ky == 0 ? Dot4Add(win[i], taps[j][0], taps[j][3]) : __builtin_amdgcn_sdot4(win[i], taps[j][ky], acc[o][i], false);
-              if (FLAVOUR == kPlainBox) acc[o][i] = __builtin_amdgcn_sdot4(win[i], a.dw_nzws3, acc[o][i], false);
-              if (FLAVOUR == kAny) sum[o][i] = __builtin_amdgcn_sdot4(win[i], 0x00010101, ky == 0 ? 0 : sum[o][i], false);
+              const int up = S == 1 ? i % 2 * 8 : 0;
+              acc[o][i] = ky == 0 ? Dot4Add(win[i], taps[j][0] << up, taps[j][3]) : __builtin_amdgcn_sdot4(win[i], taps[j][ky] << up, acc[o][i], false);
+              if (FLAVOUR == kPlainBox) acc[o][i] = __builtin_amdgcn_sdot4(win[i], a.dw_nzws3 << up, acc[o][i], false);
+              if (FLAVOUR == kAny) sum[o][i] = __builtin_amdgcn_sdot4(win[i], 0x00010101 << up, ky == 0 ? 0 : sum[o][i], false);
             }
           }
         }
