@@ -8,10 +8,13 @@
 // no barrier on the way; the partial sums meet in LDS once, and every wavefront finishes its share of the outputs.
 // Weights are the A operand, so a lane ends up with one activation row and four consecutive features.
 //
+// Many rows and outputs: tiles of up to 128 x 128 with the rows and weights of a stage in LDS (FcTileKernel).
+//
 // What bounds it: at the few rows of a classifier or a small batch every weight is used once per row tile, so the launch is
 // the time to read them; what a CU has in flight (wavefronts x R x 1 KiB) has to cover the memory's latency, which is why a
 // tile's reduction is cut over up to four wavefronts before tiles grow.
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 
@@ -309,45 +312,269 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
       }
 }
 
+// ---- larger layers: a workgroup's rows and weights through LDS ----
+//
+// The tiles above read each fragment from memory for every 32 x 32 products of a wavefront; with many rows and many outputs the CU's
+// address unit (32 rows of 32 bytes an instruction) is what they wait for, at a tenth of the matrix cores' rate, and rows of
+// outputs leave eight bytes at a time. Here four wavefronts share a tile of 64 MT x 64 NT outputs: 128 bytes of each row and the weights
+// behind them, in fragment order, are brought to LDS once for all of them - rows through registers (they begin anywhere), weights by
+// DMA - while the stage before is multiplied. Weights are packed so that a lane ends up with sixteen consecutive features of a row.
+template <int DT, int MT, int NT, int kStage>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) FcTileKernel(RowsArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  using mfma = Mfma<DT, 32>;
+  constexpr int E = DT == kI8 ? 1 : DT == kF16 ? 2 : 4;
+  constexpr int kRows = 64 * MT, kPitch = kStage + 16, kSteps = kStage / 32, kPer = kStage / 16;
+  constexpr int kX = kRows * kPitch, kBuffer = kX + 2 * NT * kSteps * 1024;  // bytes of one of two buffers: rows, weights
+  constexpr int kChunks = kRows * (kStage / 16) / 256;                       // sixteen-byte chunks of rows a thread brings
+  const int tid = threadIdx.x, lane = tid & 63, row = lane & 31, part = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
+  const int id = static_cast<int>(blockIdx.x & 7) * a.per_xcd + static_cast<int>(blockIdx.x >> 3);
+  if (id >= a.total) return;
+  const int tn = DivM(id, a.m_tiles_m), tm = id - tn * a.tiles_m;
+  const int stages = a.steps / kSteps;  // (packed to whole stages)
+
+  int64_t at[kChunks];  // of a chunk in the first stage
+#pragma unroll
+  for (int i = 0; i < kChunks; ++i) {
+    const int j = tid + i * 256;
+    at[i] = static_cast<int64_t>(min(tm * kRows + (j / kPer), a.M - 1)) * a.row_bytes + (j % kPer) * 16;  // (rows past the end repeat the last and are not stored)
+  }
+  const int64_t last = a.x_bytes - 16;
+  v4i x[kChunks];
+  const auto fetch_x = [&](int stage) {
+#pragma unroll
+    for (int i = 0; i < kChunks; ++i) {
+      const int64_t p = at[i] + stage * kStage;
+      __builtin_memcpy(&x[i], a.x + (p < last ? p : last), 16);
+    }
+  };
+  const bool ragged = a.row_bytes % kStage != 0;
+  const auto store_x = [&](int stage, uint8_t* to) {
+#pragma unroll
+    for (int i = 0; i < kChunks; ++i) {
+      const int j = tid + i * 256;
+      v4i v = x[i];
+      if (ragged && stage == stages - 1) {  // (uniform) the rows end inside this stage; at the tensor's end a load was moved to the front
+        const int64_t over = at[i] + stage * kStage - last;
+        const int valid = a.row_bytes - (stage * kStage + (j % kPer) * 16);
+        unsigned __int128 b = __builtin_bit_cast(unsigned __int128, v);
+        if (over > 0) b = over < 16 ? b >> (8 * static_cast<int>(over)) : 0;
+        if (DT == kI8) b ^= __builtin_bit_cast(unsigned __int128, v4i{static_cast<int>(a.xor_mask), static_cast<int>(a.xor_mask), static_cast<int>(a.xor_mask), static_cast<int>(a.xor_mask)});
+        if (valid < 16) b = valid > 0 ? b & ((static_cast<unsigned __int128>(1) << (8 * valid)) - 1) : 0;
+        v = __builtin_bit_cast(v4i, b);
+      } else if (DT == kI8) {
+        v ^= static_cast<int>(a.xor_mask);
+      }
+      *reinterpret_cast<v4i*>(to + (j / kPer) * kPitch + (j % kPer) * 16) = v;
+    }
+  };
+  const v4i* const wt = a.wpk + static_cast<size_t>(tn) * 2 * NT * a.steps * 64 + lane;
+  const auto fetch_w = [&](int stage, uint8_t* to) {
+    typedef const __attribute__((address_space(1))) void* gptr;
+    typedef __attribute__((address_space(3))) void* lptr;
+#pragma unroll
+    for (int i = 0; i < 2 * NT * kSteps / 4; ++i) {
+      const int j = wave + 4 * i, tile = j / kSteps, step = j % kSteps;
+      __builtin_amdgcn_global_load_lds((gptr)(wt + static_cast<size_t>(tile * a.steps + stage * kSteps + step) * 64), (lptr)(to + kX + j * 1024), 16, 0, 0);
+    }
+  };
+  typename mfma::acc acc[MT][NT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[t][n][i] = 0;
+  int rs[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) rs[t] = 0;
+  fetch_x(0);
+  fetch_w(0, lds);
+  // the features' tables, behind the buffers
+  uint8_t* const tables = lds + 2 * kBuffer;
+  constexpr int kFeatures = 64 * NT;
+  for (int i = tid; i < kFeatures; i += 256) {
+    if (DT == kI8) reinterpret_cast<tvx_v4i*>(tables)[i] = a.rq[tn * kFeatures + i];
+    reinterpret_cast<int*>(tables + kFeatures * 16)[i] = a.bias[tn * kFeatures + i];
+  }
+  store_x(0, lds);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the weights' DMA)
+  __syncthreads();
+  for (int stage = 0; stage < stages; ++stage) {
+    const uint8_t* const now = lds + (stage & 1) * kBuffer;
+    uint8_t* const then = lds + (~stage & 1) * kBuffer;
+    const bool more = stage + 1 < stages;
+    if (more) {
+      fetch_x(stage + 1);
+      fetch_w(stage + 1, then);
+    }
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+      v4i fx[MT], fw[NT];
+#pragma unroll
+      for (int t = 0; t < MT; ++t) fx[t] = *reinterpret_cast<const v4i*>(now + ((wm * MT + t) * 32 + row) * kPitch + s * 32 + part * 16);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) fw[n] = *reinterpret_cast<const v4i*>(now + kX + ((wn * NT + n) * kSteps + s) * 1024 + lane * 16);
+      if (DT == kI8 && a.zws)  // uniform
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) rs[t] = __builtin_amdgcn_sdot4(fx[t][q], 0x01010101, rs[t], false);
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) mfma::Step(acc[t][n], fw[n], fx[t]);
+    }
+    if (more) {
+      store_x(stage + 1, then);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+    }
+  }
+
+  // ---- a lane: sixteen consecutive features of each of its rows ----
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    if (DT == kI8 && a.zws) rs[t] = a.zws * (rs[t] + __shfl_xor(rs[t], 32));
+    const int m = tm * kRows + (wm * MT + t) * 32 + row;
+    if (m >= a.M) continue;
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      const int f = (wn * NT + n) * 32 + 16 * part, live = a.N - (tn * kFeatures + f);
+      if (live <= 0) continue;
+      uint8_t* const yp = a.y + (static_cast<int64_t>(m) * a.N + tn * kFeatures + f) * E;
+      uint32_t out[4 * E];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const v4i b = reinterpret_cast<const v4i*>(tables + kFeatures * 16)[f / 4 + k];
+        if constexpr (DT == kI8) {
+          int v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = acc[t][n][4 * k + e] + (b[e] - rs[t]);
+          const tvx_v4i* const rq = reinterpret_cast<const tvx_v4i*>(tables) + f + 4 * k;
+          if (a.rq_mode == kRqFastNoTie) {  // uniform
+            int c[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) c[e] = Requant8<kRqFastNoTie>(v[e], rq[e], a.out_zp, a.lo, a.hi);
+            out[k] = PackBytes(c[0], c[1], c[2], c[3]);
+          } else {
+            uint32_t r = 0;
+#pragma unroll 1
+            for (int e = 0; e < 4; ++e) {
+              const int c = a.rq_mode == kRqFast ? Requant8<kRqFast>(v[0], rq[e], a.out_zp, a.lo, a.hi) : Requant8<kRqGeneric>(v[0], rq[e], a.out_zp, a.lo, a.hi);
+              r = r >> 8 | static_cast<uint32_t>(c) << 24;
+              v[0] = v[1]; v[1] = v[2]; v[2] = v[3];
+            }
+            out[k] = r;
+          }
+        } else {
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            v[e] = acc[t][n][4 * k + e] + __builtin_bit_cast(v4f, b)[e];
+            if (a.act != TVX_ACT_NONE) v[e] = v[e] < 0.f ? 0.f : v[e];
+            if (a.act == TVX_ACT_RELU6) v[e] = v[e] > 6.f ? 6.f : v[e];
+          }
+          if constexpr (DT == kF16) {
+            _Float16 h[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) h[e] = static_cast<_Float16>(v[e]);
+            __builtin_memcpy(&out[2 * k], h, 8);
+          } else {
+            __builtin_memcpy(&out[4 * k], v, 16);
+          }
+        }
+      }
+      if (live >= 16) {
+        __builtin_memcpy(yp, out, 16 * E);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 15; ++j)
+          if (j < live) {
+            if constexpr (E == 1) yp[j] = static_cast<uint8_t>(out[j / 4] >> (8 * (j % 4)));
+            else if constexpr (E == 2) reinterpret_cast<uint16_t*>(yp)[j] = static_cast<uint16_t>(out[j / 2] >> (16 * (j % 2)));
+            else reinterpret_cast<uint32_t*>(yp)[j] = out[j];
+          }
+      }
+    }
+  }
+}
+
 typedef void (*RowsFn)(RowsArgs);
-struct Shape { int ts, rows, features, waves, ks, lds; RowsFn fn[3][2]; };
+struct Shape { int ts, rows, features, waves, ks, lds, stage; RowsFn fn[3][2]; };  // stage: steps that are brought to LDS together, or 0
 #define TVX_ROWS(TS, WM, WN, KS, MT, NT, R)                                                                                          \
-  { TS, WM * MT * TS, WN * NT * TS, WM * WN * KS, KS, KS > 1 ? WM * WN * KS * MT * (NT * TS * TS * 4 + TS * 4) : 0,                    \
+  { TS, WM * MT * TS, WN * NT * TS, WM * WN * KS, KS, KS > 1 ? WM * WN * KS * MT * (NT * TS * TS * 4 + TS * 4) : 0, 0,                 \
     { { FcRowsKernel<kI8, TS, WM, WN, KS, MT, NT, R, false>, FcRowsKernel<kI8, TS, WM, WN, KS, MT, NT, R, true> },                        \
       { FcRowsKernel<kF16, TS, WM, WN, KS, MT, NT, R, false>, FcRowsKernel<kF16, TS, WM, WN, KS, MT, NT, R, true> },                      \
       { FcRowsKernel<kF32, TS, WM, WN, KS, MT, NT, R, false>, nullptr } } }
+#define TVX_FC_TILE(MT, NT, STAGE)                                                                                                         \
+  { 32, 64 * MT, 64 * NT, 4, 1, 2 * (64 * MT * (STAGE + 16) + 2 * NT * STAGE * 32) + 64 * NT * 20, STAGE / 32,                                               \
+    { { FcTileKernel<kI8, MT, NT, STAGE>, FcTileKernel<kI8, MT, NT, STAGE> }, { FcTileKernel<kF16, MT, NT, STAGE>, FcTileKernel<kF16, MT, NT, STAGE> },            \
+      { nullptr, nullptr } } }
 const Shape kShapes[] = {
     TVX_ROWS(16, 1, 1, 4, 1, 1, 8),  // 0: 16 x 16, reduction on four wavefronts
     TVX_ROWS(32, 1, 1, 4, 1, 1, 7),  // 1: 32 x 32, on four
     TVX_ROWS(32, 2, 2, 1, 1, 1, 8),  // 2: 64 x 64, not split
+    TVX_FC_TILE(1, 1, 128),          // 3: 64 x 64 through LDS, 128 bytes of a row at a time
+    TVX_FC_TILE(1, 2, 128),          // 4: 64 rows x 128
+    TVX_FC_TILE(2, 2, 128),          // 5: 128 x 128
+    TVX_FC_TILE(1, 1, 256),          // 6: 64 x 64, 256 bytes
+    TVX_FC_TILE(2, 2, 64),           // 7: 128 x 128, 64 bytes
 };
 #undef TVX_ROWS
+#undef TVX_FC_TILE
 constexpr int kShapeCount = sizeof(kShapes) / sizeof(kShapes[0]);
 
 uint32_t Magic(int d) { return d <= 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + d - 1) / d); }
 
-// The smallest tile that still gives every CU work of its own: 16 x 16 until there is one for each (f16 16 x 4096 -> 4096:
-// 7.5 us against 9.1 on 32 x 32 tiles), 32 x 32 from there on (f32 256 x 1024 -> 1024: 8.8 against 11.9), and 64 x 64 -
-// fragments used twice, no exchange at the end - where there are more than one of those per CU, or half as many with a
-// reduction too short to split (int8 7104 x 128 -> 112: 4.3 against 7.0). Sixteen wavefronts per tile and 128 x 64 tiles
-// were measured on the same 220 drawn layers and won nowhere by more than a tenth.
-int ChooseShape(const tvx_fc_desc& d, int elem_bytes) {
+// Microseconds of a launch on tiles of a shape: what a launch takes anyway, then per stage of the reduction either its latency, once for
+// every round of workgroups a CU holds, or the time its share of the CU's units takes, whichever is longer, and at the end its results. The
+// constants are a fit to 310 drawn layers (at least 60000 outputs, int8 and float16) measured back to back in a captured graph, 6 to 15 %
+// off each; the shape chosen by them takes 3 % more than the best measured one on the (geometric) average, where the rule before (32 x 32 or
+// 64 x 64 by their number, or the 256 x 256 tiles) took 20 %. u8 4978 x 64 -> 3462: 30.7 -> 15.6 us, i8 3521 x 560 -> 1238:
+// 19.9 -> 13.3, f16 4138 x 3888 -> 603: 82.8 -> 47.9.
+struct Fit { int resident; double base, latency, share, end, unaligned; };  // workgroups of a CU; us, and by how much more at any byte
+const Fit kFits[2][kShapeCount] = {
+    {{}, {4, 1.15, 0.48, 0.80, 0.10, 0.49}, {4, 2.25, 0.11, 0.16, 1.12, 1.33}, {4, 1.53, 0.62, 0.37, 0.55, 0.17}, {2, 2.09, 0.72, 0.56, 1.02, 0.14},
+     {2, 3.69, 0.92, 0.97, 2.01, 0.20}, {2, 1.83, 0.95, 0.80, 0.99, 0.19}, {3, 3.21, 0.60, 0.48, 1.61, 0.14}},
+    {{}, {4, 1.07, 0.43, 0.76, 0.00, 0.66}, {4, 1.97, 0.11, 0.16, 0.29, 0.79}, {4, 0.96, 0.57, 0.32, 0.89, 0.24}, {2, 1.61, 0.64, 0.55, 1.22, 0.18},
+     {2, 3.10, 0.84, 0.94, 3.26, 0.20}, {2, 1.50, 0.80, 0.74, 0.90, 0.22}, {3, 2.40, 0.56, 0.55, 1.93, 0.22}}};
+double Cost(const tvx_fc_desc& d, int dt, int shape) {
+  const Shape& sp = kShapes[shape];
+  const Fit& f = kFits[dt][shape];
+  const double row = static_cast<double>(d.k) * (dt == kI8 ? 1 : 2);
+  const int stage = sp.stage ? 32 * sp.stage : 32 * sp.ks * (sp.ks > 1 ? 4 : 1);
+  const double per_cu = static_cast<double>((d.m + sp.rows - 1) / sp.rows) * ((d.n + sp.features - 1) / sp.features) / ComputeUnits();
+  const double stages = std::ceil(row / stage) * (static_cast<uint64_t>(row) % 4 ? 1 + f.unaligned : 1);
+  const double latency = std::max(per_cu / f.resident, 1.0) * stages * f.latency, share = per_cu * (f.end + stages * f.share);
+  return 2.2 + f.base + std::sqrt(std::sqrt(std::pow(latency, 4) + std::pow(share, 4)));
+}
+
+// 16 x 16 tiles until there is one for each CU (f16 16 x 4096 -> 4096: 7.5 us against 9.1 on 32 x 32 tiles), 32 x 32 from there on (f32
+// 256 x 1024 -> 1024: 8.8 against 11.9), and 64 x 64 - fragments used twice, no exchange at the end - where there are more than one
+// of those per CU, or half as many with a reduction too short to split; int8 and float16 otherwise where Cost sees more than it may be
+// off by. float32, whose products take the longest, gains nothing by rows through LDS (882 x 3984 -> 1070: 95 us, 101 with).
+int ChooseShape(const tvx_fc_desc& d, int dt) {
   const uint64_t t16 = static_cast<uint64_t>((d.m + 15) / 16) * ((d.n + 15) / 16), t64 = static_cast<uint64_t>((d.m + 63) / 64) * ((d.n + 63) / 64);
   const uint64_t cus = ComputeUnits();
   if (t16 <= cus) return 0;
-  if (2 * t64 >= 3 * cus || (2 * t64 >= cus && static_cast<uint64_t>(d.k) * elem_bytes <= 384)) return 2;
-  return 1;
+  const int direct = 2 * t64 >= 3 * cus || (2 * t64 >= cus && static_cast<uint64_t>(d.k) * (dt == kI8 ? 1 : dt == kF16 ? 2 : 4) <= 384) ? 2 : 1;
+  if (dt == kF32) return direct;
+  int best = direct;
+  double least = 0.94 * Cost(d, dt, direct);  // (what the fit is off by; then the shorter program)
+  for (int shape = 1; shape < kShapeCount; ++shape) {
+    const double cost = Cost(d, dt, shape);
+    if (cost < least) { best = shape; least = cost; }
+  }
+  return best;
 }
 
-// Microseconds of both ways, from measured layers: these tiles multiply at about 330 (int8) and 235 (float16) TFLOP/s
-// whatever the shape; a round of 256 x 256 tiles on all CUs costs its start and end whether full or not.
-bool LargeTilesWin(const tvx_fc_desc& d, int dt) {
-  const double flop = 2.0 * d.m * d.n * d.k;
-  const double rows = 3.5 + flop / (dt == kI8 ? 330e6 : 235e6);
-  const uint64_t tiles = static_cast<uint64_t>((d.m + 255) / 256) * ((d.n + 255) / 256);
-  const uint64_t cus = ComputeUnits();
-  const double large = static_cast<double>((tiles + cus - 1) / cus) * (dt == kI8 ? 17.0 + 0.009 * d.k : 25.0 + 0.0118 * d.k);
-  return large < rows;
+// A round of 256 x 256 tiles on all CUs costs its start and end whether full or not (microseconds, from measured layers).
+bool LargeTilesWin(const tvx_fc_desc& d, int dt, int shape) {
+  if (shape == 0) return false;
+  const uint64_t tiles = static_cast<uint64_t>((d.m + 255) / 256) * ((d.n + 255) / 256), cus = ComputeUnits();
+  return static_cast<double>((tiles + cus - 1) / cus) * (dt == kI8 ? 17.0 + 0.009 * d.k : 25.0 + 0.0118 * d.k) < Cost(d, dt, shape);
 }
 
 struct Plan {
@@ -391,18 +618,19 @@ int FcRowsSetup(tvx_op* op, const tvx_fc_desc* d, const void* w_host, const void
       static_cast<uint64_t>(d->m) >= (1ull << 30) || d->n >= (1u << 30))
     return TVX_E_UNSUPPORTED;
   const bool tiles_take_it = dt == kI8 ? d->k % 16 == 0 : dt == kF16 && d->k % 8 == 0;
-  if (tiles_take_it && !forced && LargeTilesWin(*d, dt)) return TVX_E_UNSUPPORTED;
+  int shape = ChooseShape(*d, dt);
+  if (tiles_take_it && !forced && LargeTilesWin(*d, dt, shape)) return TVX_E_UNSUPPORTED;
   // a few hundred quantized outputs: a wavefront per output (fc_generic) is one round trip with nothing to exchange - the same
   // 3.5 us alone, 0.3 us less behind another layer (LeNet's 800 -> 500 at batch 1)
   if (dt == kI8 && !forced && static_cast<uint64_t>(d->m) * d->n <= 1024 && d->k >= 128) return TVX_E_UNSUPPORTED;
-  int shape = ChooseShape(*d, E);
-  if (const char* f = getenv("TVX_FC_ROWS_SHAPE")) shape = std::max(0, std::min(kShapeCount - 1, atoi(f)));  // test lever
+  if (const char* f = getenv("TVX_FC_ROWS_SHAPE")) shape = std::max(0, std::min((dt == kF32 ? 3 : kShapeCount) - 1, atoi(f)));  // test lever
   const Shape& sp = kShapes[shape];
   const int kstep = 16 * (64 / sp.ts);
   RowsArgs a{};
   a.M = static_cast<int>(d->m); a.N = static_cast<int>(d->n); a.row_bytes = static_cast<int>(d->k) * E;
   a.x_bytes = static_cast<int64_t>(x_bytes);
   a.steps = (a.row_bytes + kstep - 1) / kstep;
+  if (sp.stage) a.steps = (a.steps + sp.stage - 1) / sp.stage * sp.stage;
   a.tiles_m = (a.M + sp.rows - 1) / sp.rows;
   const int tiles_n = (a.N + sp.features - 1) / sp.features;
   const uint64_t total = static_cast<uint64_t>(a.tiles_m) * tiles_n;
@@ -423,7 +651,9 @@ int FcRowsSetup(tvx_op* op, const tvx_fc_desc* d, const void* w_host, const void
   const uint8_t* src = static_cast<const uint8_t*>(w_host);
   const uint8_t flip = w_u8 ? 0x80 : 0;
   for (int n = 0; n < a.N; ++n) {
-    uint8_t* tile = packed.data() + static_cast<size_t>(n / sp.ts) * a.steps * 1024 + static_cast<size_t>(n % sp.ts) * 16;
+    // (through LDS: sixteen consecutive features in the accumulators of a lane part)
+    const int j = n % sp.ts, at = sp.stage ? j % 16 / 4 * 8 + j / 16 * 4 + j % 4 : j;
+    uint8_t* tile = packed.data() + static_cast<size_t>(n / sp.ts) * a.steps * 1024 + static_cast<size_t>(at) * 16;
     const uint8_t* row = src + static_cast<size_t>(n) * a.row_bytes;
     int64_t sw = 0;
     for (int b = 0; b < a.row_bytes; b += 16) {
