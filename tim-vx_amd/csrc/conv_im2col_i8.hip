@@ -240,7 +240,7 @@ struct ImRegArgs {
   uint32_t flip_in, flip_out;  // a window byte inside the image is moved to the signed domain, one outside is the zero point: all four bytes
   int ztwice;            // the constant fragment holds half of minus the weights' zero point, 128, and is taken twice
   uint8_t* y;
-  int OC, pre, narrow, lo, hi, out_xor4, out_zp, generic;
+  int OC, pre, lo, hi, out_xor4, out_zp, generic;
 };
 
 // PLAIN: no ties, narrow clamps, 64-bit products or second constant, and factors below 2^23.
@@ -417,7 +417,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
       const auto codes = [&](int (&v)[4]) {
         if constexpr (!PLAIN)
           if (b.generic) return RequantPack4<kRqGeneric>(v, q[j], b.out_zp, b.lo, b.hi);
-        return RequantCodes4<PLAIN>(v, q[j], round, b.pre, b.narrow, b.lo, b.hi) ^ out_xor4;
+        return RequantCodes4<PLAIN>(v, q[j], round, b.pre, b.lo, b.hi) ^ out_xor4;
       };
       uint8_t* const to = tile_y + lane_y + static_cast<size_t>(j * 32) * hw_y;
       constexpr int kOut = POOL ? 1 : 4;
@@ -581,7 +581,6 @@ int RegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const voi
   if (!a.generic) {
     if (!BuildTieRecords(op->h_mult, op->h_shift, a.OC, alloc, d->out_zp - flip, std::min<int64_t>(bound, INT32_MAX), &rqt, &up, &ties)) return TVX_E_UNSUPPORTED;
     a.lo -= flip; a.hi -= flip;
-    a.narrow = a.lo > -128 || a.hi < 127;
     a.pre = up * 2 + ties;
     a.out_xor4 = flip ? static_cast<int>(0x80808080u) : 0;
   }
@@ -593,7 +592,7 @@ int RegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const voi
   a.biasf = op->aux.as<int32_t>();
   a.rq = op->aux2.as<v4i>();
   const bool small = out_pixels < (1u << 23) && d->in_h < (1u << 23) && d->in_w < (1u << 23) && d->stride_h < (1u << 23) && d->stride_w < (1u << 23) && d->pad_top < (1u << 22);
-  const bool plain = !a.generic && !a.narrow && !a.pre && !a.ztwice && small;
+  const bool plain = !a.generic && a.lo == -128 && a.hi == 127 && !a.pre && !a.ztwice && small;
   plan.fn = pool ? (plain ? RegKernel<true, true>(kw, ks, ot) : RegKernel<false, true>(kw, ks, ot)) : plain ? RegKernel<true, false>(kw, ks, ot) : RegKernel<false, false>(kw, ks, ot);
   // a wavefront's run: one tile until every SIMD has a few wavefronts (the first of the layers above at batch 64, 98 tiles a CU: 16.1 us with
   // runs of one, 14.6 two, 14.2 three, 14.8 four, 15.6 six; at batch 1, 1.5 a CU: 2.7, 3.3, 3.8, 4.7, 5.0)

@@ -46,7 +46,7 @@ struct PoolConvArgs {
   int z4, z4_last, ztwice;    // constant fragment: minus the weights' zero point in four bytes
   int last_channels;
   int off_red;
-  int OC, pre, narrow, lo, hi, out_xor4, out_zp, generic;
+  int OC, pre, lo, hi, out_xor4, out_zp, generic;
   uint8_t* y;
 };
 
@@ -117,7 +117,7 @@ __global__ void __launch_bounds__(kMaxWaves * 64) ConvPoolKernel(PoolConvArgs a)
     const int p = tile * 8 + 4 * half, live = pooled - p;
     if (oc >= b.OC || live <= 0) return;
     const uint32_t codes = b.generic ? RequantPack4<kRqGeneric>(v, q, b.out_zp, b.lo, b.hi)
-                                     : RequantCodes4<false>(v, q, RoundHigh(q[2]), b.pre, b.narrow, b.lo, b.hi) ^ static_cast<uint32_t>(b.out_xor4);
+                                     : RequantCodes4<false>(v, q, RoundHigh(q[2]), b.pre, b.lo, b.hi) ^ static_cast<uint32_t>(b.out_xor4);
     uint8_t* const to = b.y + (static_cast<size_t>(n) * b.OC + oc) * pooled + p;
     if (live >= 4) {
       __builtin_memcpy(to, &codes, 4);
@@ -294,7 +294,6 @@ int ConvPoolSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   if (!a.generic) {
     if (!BuildTieRecords(op->h_mult, op->h_shift, a.OC, alloc, d->out_zp - flip, std::min<int64_t>(bound, INT32_MAX), &rqt, &up, &ties)) return TVX_E_UNSUPPORTED;
     a.lo -= flip; a.hi -= flip;
-    a.narrow = a.lo > -128 || a.hi < 127;
     a.pre = up * 2 + ties;
     a.out_xor4 = flip ? static_cast<int>(0x80808080u) : 0;
   }

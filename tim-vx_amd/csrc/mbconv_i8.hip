@@ -393,8 +393,7 @@ struct MbTileArgs : MbArgs {
   int half_rows, half_cols, half_halo;  // the second half's outputs: rows and columns behind the first's, and its halo's columns
   int last1, last3;                // channels of the last reduction step of the expansion and of the projection
   int dw_nzws3;                    // minus the depthwise weights' zero point in three bytes (0: folded)
-  int pre1, pre2, pre3;            // ties, narrow clamps: as RequantCodes4 takes them (clamps in the signed domain)
-  int narrow1, narrow2, narrow3;
+  int pre1, pre2, pre3;            // as RequantCodes4 takes them (clamps in the signed domain)
   int out_xor4;
 };
 
@@ -604,7 +603,7 @@ __global__ void __launch_bounds__(TileWaves(WIDE, KS) * 64) MbTileKernel(MbTileA
 #pragma unroll
       for (int i = 0; i < 4 * MT; ++i) {
         int v[4] = {acc[i / 4][4 * (i % 4)], acc[i / 4][4 * (i % 4) + 1], acc[i / 4][4 * (i % 4) + 2], acc[i / 4][4 * (i % 4) + 3]};
-        e[i / MT][i % MT] = (RequantCodes4<PLAIN>(v, next.q, round, b.pre1, b.narrow1, b.e_lo, b.e_hi) & keep[i % MT]) | fill[i % MT];
+        e[i / MT][i % MT] = (RequantCodes4<PLAIN>(v, next.q, round, b.pre1, b.e_lo, b.e_hi) & keep[i % MT]) | fill[i % MT];
       }
     }
     if (edge) {  // (uniform)
@@ -663,7 +662,7 @@ __global__ void __launch_bounds__(TileWaves(WIDE, KS) * 64) MbTileKernel(MbTileA
       const int64_t round = RoundHigh(q2[2]);
       const auto codes = [&](int v0, int v1, int v2, int v3) {
         int v[4] = {v0, v1, v2, v3};
-        return RequantCodes4<PLAIN>(v, q2, round, b.pre2, b.narrow2, b.m_lo, b.m_hi);
+        return RequantCodes4<PLAIN>(v, q2, round, b.pre2, b.m_lo, b.m_hi);
       };
       if constexpr (WIDE) {  // the projection's operand [pixel][channel]: pixel 16 half + 8 row + column
 #pragma unroll
@@ -745,7 +744,7 @@ __global__ void __launch_bounds__(TileWaves(WIDE, KS) * 64) MbTileKernel(MbTileA
     int v[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = red[(u * 4 + e) * 64 + lane] + bias[i];
-    uint32_t codes = RequantCodes4<PLAIN>(v, q[i], RoundHigh(q[i][2]), b.pre3, b.narrow3, b.lo, b.hi) ^ static_cast<uint32_t>(b.out_xor4);
+    uint32_t codes = RequantCodes4<PLAIN>(v, q[i], RoundHigh(q[i][2]), b.pre3, b.lo, b.hi) ^ static_cast<uint32_t>(b.out_xor4);
     if (ADD) codes = AddResidual4(b, codes, res[i]);
     if (live[i] == 4) {
       __builtin_memcpy(y + at[i], &codes, 4);
@@ -1024,10 +1023,9 @@ int MbConvSetup(tvx_op* op, const MbStage& ex, const MbStage& dw, const tvx_conv
     a.m_lo -= m_flip; a.m_hi -= m_flip;
     a.lo -= out_flip; a.hi -= out_flip;
     const auto narrow = [](int lo, int hi) { return lo > -128 || hi < 127; };
-    a.narrow1 = narrow(a.e_lo, a.e_hi); a.narrow2 = narrow(a.m_lo, a.m_hi); a.narrow3 = narrow(a.lo, a.hi);
     a.out_xor4 = out_flip ? static_cast<int>(0x80808080u) : 0;
     a.dw_nzws3 = (-zwd & 0xff) * 0x010101;
-    const bool plain = !(a.pre1 | a.pre2 | a.pre3 | a.narrow1 | a.narrow2 | a.narrow3) && !(a.dw_box && zwd == -128);
+    const bool plain = !(a.pre1 | a.pre2 | a.pre3 | narrow(a.e_lo, a.e_hi) | narrow(a.m_lo, a.m_hi) | narrow(a.lo, a.hi)) && !(a.dw_box && zwd == -128);
     const int widest = std::max(cin_steps, nt);
     plan.tile_fn = wide ? TileKernelOf<true>(widest, a.add_mode, plain) : TileKernelOf<false>(widest, a.add_mode, plain);
   } else {

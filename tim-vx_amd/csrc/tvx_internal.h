@@ -194,21 +194,16 @@ __device__ __forceinline__ uint32_t RequantPack4(const int (&v)[4], const tvx_v4
 }
 
 // Exact ties in front of RequantPack4's no-tie form: an accumulator v lies on k + .5 exactly when its lowest set bit is the
-// channel's tie bit (bits 8 and up of q[1], see BuildTieRecords). Those for which rounding half up would give an odd number are
-// lowered by one, which rounds them down (the multiplier is below 1). Two instructions an accumulator where there are none.
+// channel's tie bit b (bits 8 and up of q[1], see BuildTieRecords). Those for which rounding half up would give an odd number are
+// lowered by one, which rounds them down (the multiplier is below 1): with v = u 2^b and the multiplier m 2^z (u, m odd) half up gives
+// (u m + 1) / 2, odd where u m = 1, that is u = m, modulo four. Three instructions an accumulator and no branch: where multipliers are powers
+// of two every wavefront has such ties.
 template <int N>
 __device__ __forceinline__ void LowerOddTies(int (&v)[N], const tvx_v4i& q) {
-  const uint32_t bit = 1u << (q[1] >> 8), mask = 2 * bit - 1;
-  uint32_t least = ~0u;
+  const int b = q[1] >> 8;
+  const uint32_t mask = (4u << b) - 1, lower = (((static_cast<uint32_t>(q[0]) >> (31 + (q[1] & 31) - b)) & 2u) | 1u) << b;  // (b 31: no accumulator)
 #pragma unroll
-  for (int e = 0; e < N; ++e) least = min(least, (static_cast<uint32_t>(v[e]) ^ bit) & mask);
-  if (least == 0) {
-#pragma unroll
-    for (int e = 0; e < N; ++e) {
-      const uint32_t off = (static_cast<uint32_t>(v[e]) ^ bit) & mask;
-      v[e] -= ((__mulhi(v[e], q[0]) + (1 << ((q[1] & 31) - 1))) >> (q[1] & 31)) & 1 & (off == 0);
-    }
-  }
+  for (int e = 0; e < N; ++e) v[e] -= (static_cast<uint32_t>(v[e]) & mask) == lower;
 }
 
 // Four accumulators of one channel -> four codes in a dword by instructions of the gfx950: the high half of a 64-bit
@@ -242,17 +237,15 @@ __device__ __forceinline__ uint32_t RequantSaturate4(const int (&v)[4], int mult
 }
 
 // ... with the accumulators of BuildTieRecords (`pre`: 2 * shift + ties) and a clamp in the signed domain. PLAIN: pre is 0 and the clamp no narrower
-// than a byte.
+// than a byte. (A branch around the shift or the clamp costs more than they do: accumulators to scratch in kernels near their registers' end.)
 template <bool PLAIN>
-__device__ __forceinline__ uint32_t RequantCodes4(int (&v)[4], const tvx_v4i& q, int64_t round, int pre, int narrow, int lo, int hi) {
+__device__ __forceinline__ uint32_t RequantCodes4(int (&v)[4], const tvx_v4i& q, int64_t round, int pre, int lo, int hi) {
   const int sh = q[1] & 31;
   if constexpr (PLAIN) return RequantSaturate4<false>(v, q[0], sh, round, 0, 0);
-  if (pre) {  // (uniform)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] <<= pre >> 1;
-    if (pre & 1) LowerOddTies(v, q);
-  }
-  return narrow ? RequantSaturate4<true>(v, q[0], sh, round, lo << sh, ((hi + 1) << sh) - 1) : RequantSaturate4<false>(v, q[0], sh, round, 0, 0);
+  for (int e = 0; e < 4; ++e) v[e] <<= pre >> 1;
+  if (pre & 1) LowerOddTies(v, q);  // (uniform)
+  return RequantSaturate4<true>(v, q[0], sh, round, lo << sh, ((hi + 1) << sh) - 1);
 }
 
 // Four accumulators of one channel requantized together (the 32-bit record forms). `ties` (wave-uniform: a kernel
