@@ -243,7 +243,7 @@ struct ImRegArgs {
   int OC, pre, lo, hi, out_xor4, out_zp, generic;
 };
 
-// PLAIN: no ties, narrow clamps, 64-bit products or second constant, and factors below 2^23.
+// PLAIN: no ties, narrow clamps, 64-bit products or second constant, factors below 2^23, and biases that leave sums within 32 bits.
 template <int KW, int KS, int OT, bool PLAIN, bool POOL>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) ConvIm2colRegKernel(ImRegArgs a) {
   constexpr int kRows = KW == 3 ? 5 : 3, kDw = KW == 3 ? 1 : 2;  // kernel rows of a lane half and step; dwords of each
@@ -592,7 +592,8 @@ int RegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const voi
   a.biasf = op->aux.as<int32_t>();
   a.rq = op->aux2.as<v4i>();
   const bool small = out_pixels < (1u << 23) && d->in_h < (1u << 23) && d->in_w < (1u << 23) && d->stride_h < (1u << 23) && d->stride_w < (1u << 23) && d->pad_top < (1u << 22);
-  const bool plain = !a.generic && a.lo == -128 && a.hi == 127 && !a.pre && !a.ztwice && small;
+  // (the plain form multiplies sum and bias apart, in 64 bits: a bias whose folded constants wrap around has to meet the sum in 32)
+  const bool plain = !a.generic && a.lo == -128 && a.hi == 127 && !a.pre && !a.ztwice && small && bound <= INT32_MAX;
   plan.fn = pool ? (plain ? RegKernel<true, true>(kw, ks, ot) : RegKernel<false, true>(kw, ks, ot)) : plain ? RegKernel<true, false>(kw, ks, ot) : RegKernel<false, false>(kw, ks, ot);
   // a wavefront's run: one tile until every SIMD has a few wavefronts (the first of the layers above at batch 64, 98 tiles a CU: 16.1 us with
   // runs of one, 14.6 two, 14.2 three, 14.8 four, 15.6 six; at batch 1, 1.5 a CU: 2.7, 3.3, 3.8, 4.7, 5.0)
