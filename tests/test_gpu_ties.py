@@ -167,3 +167,21 @@ def test_zero_points_outside_the_type_are_rejected():
         assert err.value.status == T.E_INVALID and "zero point" in str(err.value)
         setattr(d, field, 0)
     T.conv2d_create(d, w, None).close()
+
+
+def test_lowest_accumulator_is_no_tie(oracle):
+    """Where some channels can tie, the others' lowest accumulator, -2^31, stays what it is."""
+    rng = np.random.default_rng(77)
+    n, c, oc, side = 2, 3, 24, 9
+    x = rng.integers(-128, 128, n * c * side * side).astype(np.int8)
+    w = rng.integers(-128, 128, (oc, c * 9)).astype(np.int8)
+    b = rng.integers(-4096, 4097, oc).astype(np.int32)
+    m = np.where(np.arange(oc) % 2, 0.0016, 2.0 ** -6)     # odd channels: no product with 24 bits of multiplier ends in .5
+    b[1::4] = -2 ** 31
+    w[1::4] = 0
+    kws = dict(in_shape=[side, side, c, n], w_shape=[3, 3, c, oc], out_shape=[side, side, oc, n], stride=[1, 1], dilation=[1, 1], pad_left=1, pad_top=1,
+               multiplier=0, in_dtype=1, w_dtype=1, out_dtype=1, in_q=(0.5, 3), w_q=(1.0, 0, (2 * m).astype(np.float32)), out_q=(1.0, -5))
+    want = oracle.conv2d(x, w.reshape(-1), b, act=0, **kws)
+    assert (want.reshape(n, oc, -1)[:, 1::4] == -128).all()
+    got = TC.gpu_conv2d(x, w.reshape(-1), b, act=0, want_kernel="conv2d_im2col_i8", **kws)
+    assert np.array_equal(got, want), int((got != want).sum())

@@ -134,9 +134,9 @@ bool BuildTieRecords(const std::vector<int32_t>& mult, const std::vector<int32_t
   for (int c = 0; c < alloc; ++c) {
     const int32_t m = c < channels ? mult[c] : 0, s = m ? shift[c] + *pre : 33;
     if (s - 32 > 20) return false;
-    // a tie needs v * m = 2^(s-1) (mod 2^s): v's lowest set bit is bit s - 1 - ctz(m); out of reach: bit 31 (|v| < 2^31)
+    // a tie needs v * m = 2^(s-1) (mod 2^s): v's lowest set bit is bit s - 1 - ctz(m); bit 31 stands for out of reach
     int bit = m ? s - 1 - __builtin_ctz(static_cast<uint32_t>(m)) : 31;
-    if (bit > 31 || (int64_t{1} << bit) > (acc_bound << *pre)) bit = 31;
+    if (bit >= 31 || (int64_t{1} << bit) > (acc_bound << *pre)) bit = 31;
     else *ties = true;
     int32_t* q = &(*records)[static_cast<size_t>(c) * 4];
     q[0] = m;

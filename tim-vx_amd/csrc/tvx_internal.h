@@ -201,7 +201,8 @@ __device__ __forceinline__ uint32_t RequantPack4(const int (&v)[4], const tvx_v4
 template <int N>
 __device__ __forceinline__ void LowerOddTies(int (&v)[N], const tvx_v4i& q) {
   const int b = q[1] >> 8;
-  const uint32_t mask = (4u << b) - 1, lower = (((static_cast<uint32_t>(q[0]) >> (31 + (q[1] & 31) - b)) & 2u) | 1u) << b;  // (b 31: no accumulator)
+  const uint32_t mask = (2u << ((b + 1) & 31)) - 1;  // (b 31, no ties: one bit, which is none of the bits below)
+  const uint32_t lower = (((static_cast<uint32_t>(q[0]) >> (31 + (q[1] & 31) - b)) & 2u) | 1u) << b;
 #pragma unroll
   for (int e = 0; e < N; ++e) v[e] -= (static_cast<uint32_t>(v[e]) & mask) == lower;
 }
