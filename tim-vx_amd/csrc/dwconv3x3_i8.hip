@@ -156,7 +156,7 @@ __global__ void __launch_bounds__(kThreads) DwConv3x3Kernel(DwArgs a) {
     raw[r][kOwn + 1] = has_right ? rr : a.pad_fill;
   }
   if (w4 >= a.ow4) return;  // lanes that only fed their neighbour
-  // Uniform operands that the instructions below take from vector registers (the three-address dot product, the
+  // Uniform operands that the instructions below take from vector registers (the first dot product, the
   // clamp) get one copy for all output rows: each row is a block of its own behind the bounds test, and the
   // compiler would copy them again in every block.
   int bias_v = bias, wk0_v = wk0, lo_v = a.lo, hi_v = a.hi, t_v = q[1];
@@ -180,7 +180,7 @@ __global__ void __launch_bounds__(kThreads) DwConv3x3Kernel(DwArgs a) {
                   : i == 3 ? Window<4 + 3 - PL>(rw) : i == 4 ? Window<4 + 4 - PL>(rw) : i == 5 ? Window<4 + 5 - PL>(rw)
                   : i == 6 ? Window<4 + 6 - PL>(rw) : Window<4 + 7 - PL>(rw);
         }
-        int acc = Dot4Add(win3[0], wk0_v, bias_v);
+        int acc = __builtin_amdgcn_sdot4(win3[0], wk0_v, bias_v, false);
         acc = __builtin_amdgcn_sdot4(win3[1], wk1, acc, false);
         acc = __builtin_amdgcn_sdot4(win3[2], wk2, acc, false);
         if (BOXSUM && box) {
@@ -211,7 +211,7 @@ __global__ void __launch_bounds__(kThreads) DwConv3x3Kernel(DwArgs a) {
     int res[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      int acc = Dot4Add(win[S * o][i], wk0_v, bias_v);
+      int acc = __builtin_amdgcn_sdot4(win[S * o][i], wk0_v, bias_v, false);
       acc = __builtin_amdgcn_sdot4(win[S * o + 1][i], wk1, acc, false);
       acc = __builtin_amdgcn_sdot4(win[S * o + 2][i], wk2, acc, false);
       if (BOXSUM && box) {

@@ -126,15 +126,6 @@ __device__ __forceinline__ int Cut(const uint32_t (&d)[N], int o) {
   return static_cast<int>(o % 4 ? __builtin_amdgcn_alignbyte(hi, lo, o % 4) : lo);
 }
 
-// The first product of an accumulator takes the bias as its third operand (the builtin's instruction adds to a copy of it).
-template <bool UNIFORM>
-__device__ __forceinline__ int FirstDot(int x, int w, int bias) {
-  if constexpr (!UNIFORM) return Dot4Add(x, w, bias);
-  int r;
-  asm("v_dot4_i32_i8 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(w), "v"(bias));
-  return r;
-}
-
 // Accumulators start from the folded bias. A row's window is two dot products (weights 0 .. 3, and the fifth alone); under a weight
 // zero point (SUMS) the rows' window sums are made once per input row and added to the output rows they belong to.
 template <int K, int S, int R, bool UNIFORM, bool SUMS>
@@ -162,7 +153,7 @@ __global__ void __launch_bounds__(256) DwRegI8Kernel(DwrArgs a) {
       for (int r = 0; r < R; ++r) {
         const int ky = i - r * S;
         if (ky < 0 || ky >= K) continue;
-        acc[r][q] = ky == 0 ? FirstDot<UNIFORM>(w0, w[0], bias) : __builtin_amdgcn_sdot4(w0, w[2 * ky], acc[r][q], false);
+        acc[r][q] = __builtin_amdgcn_sdot4(w0, w[2 * ky], ky == 0 ? bias : acc[r][q], false);
         if (K > 4) acc[r][q] = __builtin_amdgcn_sdot4(w1, w[2 * ky + 1], acc[r][q], false);
         if (SUMS) sum[r][q] = ky == 0 ? box : sum[r][q] + box;
       }

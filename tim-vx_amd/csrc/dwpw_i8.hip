@@ -217,7 +217,7 @@ __global__ void __launch_bounds__(kMaxWaves * 64) __attribute__((amdgpu_waves_pe
               const int ky = r - S * o;
               if (ky < 0 || ky > 2) continue;
               const int up = S == 1 ? i % 2 * 8 : 0;
-              acc[o][i] = ky == 0 ? Dot4Add(win[i], taps[j][0] << up, taps[j][3]) : __builtin_amdgcn_sdot4(win[i], taps[j][ky] << up, acc[o][i], false);
+              acc[o][i] = __builtin_amdgcn_sdot4(win[i], taps[j][ky] << up, ky == 0 ? taps[j][3] : acc[o][i], false);
               if (FLAVOUR & kBox) acc[o][i] = __builtin_amdgcn_sdot4(win[i], a.dw_nzws3 << up, acc[o][i], false);
               if (FLAVOUR & kTwice) acc[o][i] = __builtin_amdgcn_sdot4(win[i], a.dw_rest3 << up, acc[o][i], false);
             }

@@ -81,7 +81,7 @@ __device__ __forceinline__ int WindowOf(const int (&row)[(W + 5) / 4 + 1]) {
 template <int W, int S, int J>
 __device__ __forceinline__ int DwOne(const MbArgs& a, const int (&rows)[3][(W + 5) / 4 + 1], const v4i& k) {
   const int w0 = WindowOf<W, S, J>(rows[0]), w1 = WindowOf<W, S, J>(rows[1]), w2 = WindowOf<W, S, J>(rows[2]);
-  int v = Dot4Add(w0, k[0], k[3]);
+  int v = __builtin_amdgcn_sdot4(w0, k[0], k[3], false);
   v = __builtin_amdgcn_sdot4(w1, k[1], v, false);
   v = __builtin_amdgcn_sdot4(w2, k[2], v, false);
   if (a.dw_box) {  // (wave-uniform) weights packed unshifted: their zero point times the window sum
@@ -642,7 +642,7 @@ __global__ void __launch_bounds__(TileWaves(WIDE, KS) * 64) MbTileKernel(MbTileA
       for (int o = 0; o < 2; ++o)
 #pragma unroll
         for (int c = 0; c < 2 * kWin; ++c) {
-          int v = Dot4Add(win[o][c / 2], taps[c % 2][0], taps4[3]);
+          int v = __builtin_amdgcn_sdot4(win[o][c / 2], taps[c % 2][0], taps4[3], false);
           v = __builtin_amdgcn_sdot4(win[o + 1][c / 2], taps[c % 2][1], v, false);
           sums[o][c] = __builtin_amdgcn_sdot4(win[o + 2][c / 2], taps[c % 2][2], v, false);
         }
