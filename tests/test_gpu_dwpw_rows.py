@@ -37,3 +37,27 @@ def test_rows(oracle, monkeypatch, ci, rows, mode):
             return x, wd, bd, kd, wp, bp, kp
         monkeypatch.setattr(DP, "_pair", shifted)
     DP.test_depthwise_pointwise_fused(oracle, ci, "u8" if mode == "u8zp0" else mode, 1 if ci % 2 else 0)
+
+
+@pytest.mark.parametrize("n,c,h,w,oc", [(8, 288, 128, 128, 64), (8, 224, 112, 112, 256), (8, 256, 128, 128, 96), (16, 352, 80, 80, 128)])
+def test_as_many_rows_as_fit(oracle, n, c, h, w, oc):
+    """Pairs whose four rows a tile do not fit LDS, though fewer do: taken with those."""
+    import numpy as np
+    import torch
+    import tvx_case as TC
+    rng = np.random.default_rng(8100 + c)
+    x, wd, bd, kd, wp, bp, kp = DP._pair(rng, n, c, h, w, oc, 1, "i8pc")
+    T, keep = TC.tvx(), []
+    op = T.conv2d_dw_pw_create(DP._desc(T, kd, 0, keep), wd, bd, DP._desc(T, kp, 2, keep), wp, bp)
+    assert op.kernel_name == "dwconv3x3_pwconv_i8"
+    xd, yd = TC.to_device(x), TC.device_out(n * oc * h * w, np.int8)
+    op.run(xd, None, yd)
+    torch.cuda.synchronize()
+    got = yd.cpu().numpy().reshape(n, -1)
+    op.close()
+    for image in (0, n - 1):   # (the oracle takes seconds for one)
+        for k in (kd, kp):
+            k["in_shape"][3] = k["out_shape"][3] = 1
+        mid = oracle.conv2d(x.reshape(n, -1)[image].copy(), wd, bd, act=0, **kd)
+        want = oracle.conv2d(mid, wp, bp, act=2, **kp)
+        assert np.array_equal(got[image], want), (image, int((got[image] != want).sum()))

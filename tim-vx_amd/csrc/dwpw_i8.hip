@@ -403,15 +403,23 @@ int DwPwSetup(tvx_op* op, const tvx_conv2d_desc* dw, const void* dw_w, const voi
   //   3.5  56 x 56, 144 to 24              (1,4) 15.4, (2,8) 12.2, (4,8) 12.3, (2,4) 13.8      28 x 28, 192 to 32  (2,8) 10.5, (4,8) 9.7
   //   7    28 x 28, 192 to 32              (1,4) 18.5, (2,4) 15.0, (4,8) 14.4, (4,4) 16.0
   //   14   56 x 56, 96 to 24, stride 2     (1,4) 27.7, (2,4) 24.4, (2,8) 25.9
-  //   28   112 x 112, 32 to 16             (1,4) 36.6, (2,4) 28.8, (4,4) 25.7, (4,8) 29.2 ----
+  //   28   112 x 112, 32 to 16             (1,4) 36.6, (2,4) 28.8, (4,4) 25.7, (4,8) 29.2
+  // Never more than fit LDS: of the pairs taken at all one row always does (int8, batch 8, four rows too many: 128 x 128, 288 to 64 (1,8) 40.6, (2,8)
+  // 34.8; 112 x 112, 224 to 256 58.2, 41.0; 128 x 128, 256 to 96 39.1, 36.1. As two kernels these are 28.3, 34.3 and 28.5: callers who need the
+  // fused operator get it, callers who have the choice lose by it.) ----
   const int cus = ComputeUnits();
   const uint64_t rows = static_cast<uint64_t>(dw->batch) * dw->out_h, cu = cus;
+  const int oc_bytes = oc_alloc_ * cp_;
+  const bool wlds = oc_bytes <= kWeightBytes;
+  const auto weights_at = [&](int r) { return RoundUp(r * static_cast<int>(dw->out_w), 32) * (cp_ + 16); };  // behind the operand tile
+  const auto lds_of = [&](int r) { return weights_at(r) + (wlds ? oc_bytes : 0) + oc_alloc_ * 20; };
+  const auto fits = [&](int r) { return dw->out_h % r == 0 && (r < 4 || S == 1) && r * dw->out_w <= static_cast<uint32_t>(kMaxSlots) && lds_of(r) <= 160 * 1024; };
   int rpt = 1;
   for (int r : {2, 4})
-    if (rows > (r == 4 ? 3 * cu : S * cu) && dw->out_h % r == 0 && (r == 2 || S == 1) && r * dw->out_w <= static_cast<uint32_t>(kMaxSlots)) rpt = r;
+    if (rows > (r == 4 ? 3 * cu : S * cu) && fits(r)) rpt = r;
   if (const char* f = getenv("TVX_DWPW_ROWS")) {  // test lever
     const int r = atoi(f);
-    if ((r == 1 || r == 2 || (r == 4 && S == 1)) && r * dw->out_w <= static_cast<uint32_t>(kMaxSlots) && dw->out_h % r == 0) rpt = r;
+    if ((r == 1 || r == 2 || r == 4) && fits(r)) rpt = r;
   }
   const uint64_t tiles = static_cast<uint64_t>(dw->batch) * (dw->out_h / rpt);
   if (tiles > 0x7fffffffull || static_cast<uint64_t>(dw->in_h) * dw->in_w * dw->in_c >= (1ull << 32) - 16 || dw->in_h >= (1u << 24)) return TVX_E_UNSUPPORTED;  // (32-bit offsets inside an image)
@@ -481,14 +489,13 @@ int DwPwSetup(tvx_op* op, const tvx_conv2d_desc* dw, const void* dw_w, const voi
     a.add_za = e.a_zp; a.add_zb = e.b_zp; a.add_zo = e.out_zp;
     ActRange(pw->out_dtype, e.out_scale, e.out_zp, TVX_ACT_NONE, &a.add_lo, &a.add_hi);
   }
-  const int oc_bytes = a.oc_tiles * 32 * a.cp;
-  const bool wlds = oc_bytes <= kWeightBytes;
-  a.off_w = a.ptiles * 32 * a.pix_stride;
+  a.off_w = weights_at(rpt);
   a.off_rq = a.off_w + (wlds ? oc_bytes : 0);
-  a.off_bias = a.off_rq + a.oc_tiles * 32 * 16;
-  const int lds_bytes = a.off_bias + a.oc_tiles * 32 * 4;
+  a.off_bias = a.off_rq + oc_alloc_ * 16;
+  const int lds_bytes = lds_of(rpt);
   if (lds_bytes > 160 * 1024) return TVX_E_UNSUPPORTED;
-  int waves = tiles <= 2ull * cus || (rpt == 4 && (a.quads << lpr_shift) > 64 * kWaves) ? kMaxWaves : kWaves;
+  // (where a CU holds one workgroup, eight: 80 x 80, 352 to 128, batch 16 63.7 us, 95.4 with four)
+  int waves = tiles <= 2ull * cus || lds_bytes > 80 * 1024 || (rpt == 4 && (a.quads << lpr_shift) > 64 * kWaves) ? kMaxWaves : kWaves;
   // stride 2, a depthwise pass of at most 128 threads: half of four wavefronts would only wait for the other half (batch 64: 112 x 112, 32 to 16
   // 11.6 -> 9.9 us, 16 to 32 10.7 -> 8.9, 56 x 56, 32 to 64 6.3 -> 6.2; at stride 1 four are ahead: 28 x 28, 32 to 64 6.4 against 7.7)
   if (S == 2 && tiles > 2ull * cus && (a.quads << lpr_shift) <= 128) waves = 2;
