@@ -65,3 +65,14 @@ def test_infinite_weights_stay_with_the_kernel_that_skips_padding(oracle):
     wt[0] = np.inf
     got = TC.gpu_conv2d(np.abs(x), wt, b, want_kernel="conv2d_generic", **kws).reshape(2, 6, 6)
     assert np.isfinite(got[0, 0]).all() and np.isinf(got[0, 1:, 1:]).all()
+
+
+@pytest.mark.parametrize("offset", [1, 6, 8])
+@pytest.mark.parametrize("mode", ["u8", "i8pc"])
+@pytest.mark.parametrize("c,h,w,k,stride", [(3, 160, 160, 5, 1), (5, 14, 14, 3, 1), (4, 7, 9, 3, 2), (2, 20, 21, 5, 2)])
+def test_tensors_at_any_address(oracle, c, h, w, k, stride, mode, offset):
+    rng = np.random.default_rng(7300)
+    x, wt, b, kws = conv_case(rng, n=2, c=c, h=h, w=w, oc=0, kh=k, kw=k, stride=[stride, stride], dil=[1, 1], pad=[k // 2] * 4, mult=1, mode=mode)
+    want = oracle.conv2d(x, wt, b, act=2, **kws)
+    got = TC.gpu_conv2d(x, wt, b, act=2, want_kernel="dwconv_planes_i8", misalign=offset, **kws)
+    assert np.array_equal(got, want), int((got != want).sum())

@@ -207,13 +207,11 @@ struct Plan {
   DwrArgs a;
   DwRegFn fn;
   dim3 grid;
-  unsigned threads, align;  // align: address bits of the tensors that must not be set (as the stencils for these layers have it)
+  unsigned threads;
 };
 
 int DwRegRun(tvx_op* op, const void* in0, const void*, void* out, hipStream_t st) {
   const Plan* p = reinterpret_cast<const Plan*>(op->host_blob.data());
-  if ((reinterpret_cast<uintptr_t>(in0) | reinterpret_cast<uintptr_t>(out)) & p->align)
-    return SetError(TVX_E_INVALID, "%s: tensors must be %u-byte aligned", op->kernel_name, p->align + 1);
   DwrArgs a = p->a;
   a.x = static_cast<const uint8_t*>(in0);
   a.y = static_cast<uint8_t*>(out);
@@ -339,7 +337,7 @@ int DwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
     a.wf = op->packed.as<float>();
   }
   if (s != TVX_OK) return s;
-  Plan plan{a, nullptr, dim3(1), block, !q || (K == 3 && WholeDwordRows(d)) ? 0u : 15u};
+  Plan plan{a, nullptr, dim3(1), block};
   plan.fn = dt == TVX_I8 ? PickKernel<TVX_I8>(K, S, R, uniform, a.zws != 0) : dt == TVX_F16 ? PickKernel<TVX_F16>(K, S, R, uniform, false) : PickKernel<TVX_F32>(K, S, R, uniform, false);
   plan.grid = uniform ? dim3(a.C, parts, d->batch) : dim3(static_cast<unsigned>((planes * a.tpp + 255) / 256));
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
