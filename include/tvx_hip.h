@@ -352,6 +352,9 @@ int tvx_op_run(tvx_op* op, const void* in0, const void* in1, void* out, void* st
 int tvx_op_run3(tvx_op* op, const void* in0, const void* in1, const void* in2, void* out, void* stream);
 /* Name of the kernel variant chosen at creation, e.g. "conv2d_generic". */
 const char* tvx_op_kernel_name(const tvx_op* op);
+/* Several kernels report one name, where a newer one took over some of a name's layers. This tells them apart, e.g.
+ * "dwconv_reg_i8" for an operator named "dwconv_planes_i8"; the name itself where it says enough. */
+const char* tvx_op_variant(const tvx_op* op);
 void tvx_op_destroy(tvx_op* op);
 
 #ifdef __cplusplus

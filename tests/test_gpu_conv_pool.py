@@ -4,6 +4,7 @@ end inside a tile, a weight zero point at the end of its range. Exact against th
 import pytest
 
 import test_gpu_fused_small_nets as SN
+import tvx_case as TC
 
 pytestmark = pytest.mark.gpu
 
@@ -33,4 +34,5 @@ def test_split_reductions(oracle, monkeypatch, ci, parts, mode):
         kws["in_q"] = (kws["in_q"][0] / 8, kws["in_q"][1])   # (the largest of four results would mostly lie on the clamp)
         return x, w, b, kws
     monkeypatch.setattr(SN, "conv_case", fitted)
+    TC.expect_variant(monkeypatch, "conv2d_pool_i8")
     SN.test_conv2d_with_fused_max_pool(oracle, ci, "u8" if mode == "u8zp0" else mode, 0, monkeypatch)

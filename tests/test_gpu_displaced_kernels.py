@@ -1,0 +1,59 @@
+"""Kernels whose layers newer ones mostly take, on the layers that are still theirs and, by the newer ones' levers, on their old ones; and
+which kernel takes a layer of its own accord. Exact against the oracle."""
+import numpy as np
+import pytest
+
+import test_gpu_fused_small_nets as SN
+import test_gpu_parity as PT
+import tvx_case as TC
+from test_gpu_parity import conv_case
+
+pytestmark = pytest.mark.gpu
+
+IGEMM_POOL = [c for c in SN.CONV_POOL if c["kernel"] == "conv2d_igemm_maxpool_i8"]
+# an image too large for LDS; rows of fewer than four columns
+OWN_POOL = [dict(n=2, c=64, h=40, w=40, oc=24, kh=3, kw=3, stride=[1, 1], dil=[1, 1], pad=[1, 1, 1, 1], kernel="conv2d_igemm_maxpool_i8"),
+            dict(n=1, c=40, h=10, w=2, oc=20, kh=3, kw=3, stride=[1, 1], dil=[1, 1], pad=[1, 1, 1, 1], kernel="conv2d_igemm_maxpool_i8")]
+
+
+@pytest.mark.parametrize("tile", [0, 32])
+@pytest.mark.parametrize("mode", ["u8", "i8pc"])
+@pytest.mark.parametrize("gi", range(len(IGEMM_POOL) + len(OWN_POOL)))
+def test_pooled_implicit_gemm(oracle, gi, mode, tile, monkeypatch):
+    if gi < len(IGEMM_POOL):
+        monkeypatch.setenv("TVX_CONV_POOL", "0")
+    else:
+        case = SN.conv_case
+
+        def fitted(*args, **kws):  # (the largest of four sums of 576 products would mostly lie on the clamp)
+            x, w, b, kws = case(*args, **kws)
+            kws["in_q"] = (kws["in_q"][0] / 8, kws["in_q"][1])
+            return x, w, b, kws
+        monkeypatch.setattr(SN, "conv_case", fitted)
+    monkeypatch.setattr(SN, "CONV_POOL", IGEMM_POOL + OWN_POOL)
+    TC.expect_variant(monkeypatch, "conv2d_igemm_maxpool_i8")
+    SN.test_conv2d_with_fused_max_pool(oracle, gi, mode, tile, monkeypatch)
+
+
+@pytest.mark.parametrize("mode", ["u8", "i8pc", "u8pc"])
+@pytest.mark.parametrize("gi", range(len(PT.DWP_GRID)))
+def test_depthwise_planes(oracle, gi, mode, monkeypatch):
+    n, c, h, w, kh, kw, stride, dil, pad = PT.DWP_GRID[gi]
+    monkeypatch.setenv("TVX_DWCONV_REG", "0")
+    dwords = kh == kw == 3 and stride[0] == stride[1] and dil == [1, 1]
+    TC.expect_variant(monkeypatch, "dwconv_rows_i8" if dwords else "dwconv_planes_i8")
+    PT.test_depthwise_planes_shapes(oracle, gi, mode)
+
+
+@pytest.mark.parametrize("c,h,w,stride,kernel", [
+    (4, 9, 132, 1, "dwconv_reg_i8"), (3, 9, 52, 1, "dwconv3x3_i8"),      # outputs of a row in 33 of 64 lanes, in 13 of 16
+    (3, 9, 136, 1, "dwconv3x3_i8"), (2, 9, 264, 1, "dwconv_reg_i8"),     # rows of whole 8-byte units; rows over 256 columns
+    (5, 14, 14, 1, "dwconv_reg_i8"), (5, 7, 7, 1, "dwconv_reg_i8"),      # no whole dwords
+    (3, 20, 24, 2, "dwconv3x3_i8"), (3, 20, 27, 2, "dwconv_reg_i8")])
+def test_which_kernel_takes_a_quantized_3x3_layer(oracle, c, h, w, stride, kernel):
+    pad = [1, 1, 1, 1] if stride == 1 else [0, 1, 0, 1]
+    rng = np.random.default_rng(7400 + w)
+    for mode in ("u8", "i8pc"):
+        x, wt, b, kws = conv_case(rng, n=2, c=c, h=h, w=w, oc=0, kh=3, kw=3, stride=[stride, stride], dil=[1, 1], pad=pad, mult=1, mode=mode)
+        got = TC.gpu_conv2d(x, wt, b, act=2, want_variant=kernel, **kws)
+        assert np.array_equal(got, oracle.conv2d(x, wt, b, act=2, **kws))

@@ -30,7 +30,8 @@ def test_depthwise_register_stencil(oracle, gi, k, stride, mode, monkeypatch):
     pads = [[k // 2] * 4, [0, k // 2, 0, k // 2], [k - 1, 0, 1, k - 1]] if same else [[0, 0, 0, 0]]
     rng = np.random.default_rng(7000 + gi)
     if mode not in ("f16", "f32"):
-        monkeypatch.setenv("TVX_DWCONV_REG", "1")  # (of their own accord quantized 3x3 windows go to other stencils)
+        monkeypatch.setenv("TVX_DWCONV_REG", "1")  # (of their own accord some quantized 3x3 windows go to another stencil)
+        TC.expect_variant(monkeypatch, "dwconv_reg_i8")
     for pad in pads:
         if h + pad[2] + pad[3] < k or w + pad[0] + pad[1] < k:
             continue
@@ -74,5 +75,5 @@ def test_tensors_at_any_address(oracle, c, h, w, k, stride, mode, offset):
     rng = np.random.default_rng(7300)
     x, wt, b, kws = conv_case(rng, n=2, c=c, h=h, w=w, oc=0, kh=k, kw=k, stride=[stride, stride], dil=[1, 1], pad=[k // 2] * 4, mult=1, mode=mode)
     want = oracle.conv2d(x, wt, b, act=2, **kws)
-    got = TC.gpu_conv2d(x, wt, b, act=2, want_kernel="dwconv_planes_i8", misalign=offset, **kws)
+    got = TC.gpu_conv2d(x, wt, b, act=2, want_kernel="dwconv_planes_i8", want_variant="dwconv_reg_i8", misalign=offset, **kws)
     assert np.array_equal(got, want), int((got != want).sum())

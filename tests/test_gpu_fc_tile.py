@@ -35,6 +35,7 @@ def test_tiles_through_lds(oracle, m, k, n, mode, offset, monkeypatch):
         to_device = TC.to_device
         monkeypatch.setattr(TC, "to_device", lambda a: torch.cat([to_device(np.zeros(offset, a.dtype)), to_device(a)])[offset:])
     want = oracle.fully_connected(x, w, b, act=1, **kws)
+    TC.expect_variant(monkeypatch, "fc_tile_f16" if mode == "f16" else "fc_tile_i8")
     for shape in range(3, 8):
         monkeypatch.setenv("TVX_FC_ROWS_SHAPE", str(shape))
         got = TC.gpu_fully_connected(x, w, b, act=1, want_kernel="fc_rows_f16" if mode == "f16" else "fc_rows_i8", **kws)
@@ -49,6 +50,7 @@ def test_rows_keep_an_infinity_apart(monkeypatch, shape):
     """What lies behind a row that ends inside a stage is not multiplied."""
     monkeypatch.setenv("TVX_FC_ROWS", "1")
     monkeypatch.setenv("TVX_FC_ROWS_SHAPE", str(shape))
+    TC.expect_variant(monkeypatch, "fc_tile_f16")
     x, w = np.ones((4, 37), np.float16), np.ones((20, 37), np.float16)
     x[2, 0] = np.inf
     got = TC.gpu_fully_connected(x.ravel(), w.ravel(), None, m=4, k=37, n=20, in_dtype=2, w_dtype=2, out_dtype=2, want_kernel="fc_rows_f16").reshape(4, 20)

@@ -31,7 +31,7 @@ def test_register_gather(oracle, monkeypatch, ci, mode, run):
         kws["w_q"] = (kws["w_q"][0], 0, None)
         kws["out_q"] = (kws["out_q"][0] * 2, kws["out_q"][1])
     want = oracle.conv2d(x, w, b, act=2, **kws)
-    got = TC.gpu_conv2d(x, w, b, act=2, want_kernel="conv2d_im2col_i8", **kws)
+    got = TC.gpu_conv2d(x, w, b, act=2, want_kernel="conv2d_im2col_i8", want_variant="conv2d_im2col_reg_i8", **kws)
     assert np.array_equal(got, want), (int((got != want).sum()), np.flatnonzero(got != want)[:8])
 
 
@@ -54,7 +54,7 @@ def test_biases_at_the_ends_of_their_range(oracle, in_zp, pool):
     want = oracle.conv2d(x, w, b.astype(np.int32), act=0, **kws)
     assert (want.reshape(n, oc, -1)[:, ::2] == (127 if sign > 0 else -128)).all() and len(np.unique(want)) > 50
     if not pool:
-        got = TC.gpu_conv2d(x, w, b.astype(np.int32), act=0, want_kernel="conv2d_im2col_i8", **kws)
+        got = TC.gpu_conv2d(x, w, b.astype(np.int32), act=0, want_variant="conv2d_im2col_reg_i8", **kws)
         assert np.array_equal(got, want), int((got != want).sum())
         return
     import torch
@@ -62,7 +62,7 @@ def test_biases_at_the_ends_of_their_range(oracle, in_zp, pool):
     want = want.reshape(n * oc, side // 2, 2, side // 2, 2).max(axis=(2, 4)).reshape(-1)
     keep = []
     op = TC.tvx().conv2d_pool_create(*SN._descs(TC.tvx(), kws, 0, keep), w, b.astype(np.int32))
-    assert op.kernel_name == "conv2d_im2col_maxpool_i8"
+    assert op.variant == "conv2d_im2col_reg_maxpool_i8"
     xd, yd = TC.to_device(x), TC.device_out(want.size, np.int8)
     op.run(xd, None, yd)
     torch.cuda.synchronize()

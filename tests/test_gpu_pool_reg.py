@@ -25,6 +25,8 @@ def test_pool2d_register_stencil(oracle, si, k, s, ptype, dtype, monkeypatch):
     w, h, c, n = SHAPES[si]
     rng = np.random.default_rng(8000 + si * 100 + k * 10 + s)
     zi = 7 if dtype == 1 else 120
+    if dtype < 2:
+        TC.expect_variant(monkeypatch, "pool2d_reg_i8")
     scales = (((0.1, zi), (0.1, zi)), ((0.1, zi), (0.1, zi - 9)), ((0.1, zi), (0.07, 3))) if dtype < 2 else (((1.0, 0), (1.0, 0)),)
     for pad in ([0, 0, 0, 0], [0, 1, 0, 1], [1, 1, 1, 1], [k - 1, 0, k - 1, k - 1]):
         ow, oh = (w + pad[0] + pad[1] - k) // s + 1, (h + pad[2] + pad[3] - k) // s + 1
@@ -62,7 +64,7 @@ def test_max_pool_of_lowest_values_and_infinities(oracle, dtype):
 
 @pytest.mark.parametrize("dtype", [0, 1, 2, 3])
 @pytest.mark.parametrize("w,h", [(64, 32), (45, 46), (127, 129), (159, 160), (16, 1061)])
-def test_average_of_large_planes(oracle, w, h, dtype):
+def test_average_of_large_planes(oracle, w, h, dtype, monkeypatch):
     """A workgroup per plane: whole units of sixteen bytes and what is left of them, planes that begin at any element."""
     rng = np.random.default_rng(8100 + w)
     c, n = 3, 2
@@ -71,6 +73,7 @@ def test_average_of_large_planes(oracle, w, h, dtype):
         x = x + x.dtype.type(1)
     kws = dict(in_shape=[w, h, c, n], out_shape=[1, 1, c, n], ksize=[w, h], stride=[1, 1], pad_left=0, pad_top=0, pool_type=1, dtype=dtype)
     q = dict(in_q=(0.1, 3), out_q=(0.002, 5)) if dtype < 2 else {}
+    TC.expect_variant(monkeypatch, "pool2d_plane_sum")
     want = oracle.pool2d(x, **q, **kws)
     got = TC.gpu_pool2d(x, **q, **kws)
     if dtype < 2:

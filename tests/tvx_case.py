@@ -70,6 +70,17 @@ def device_out(n, np_dtype):
 NP_OF = {0: np.uint8, 1: np.int8, 2: np.float16, 3: np.float32}
 
 
+def expect_variant(monkeypatch, name):
+    """Every operator that runs from here on is the kernel `name` (several report one kernel_name)."""
+    T = tvx()
+    run = T.Op.run
+
+    def checked(op, *args):
+        assert op.variant == name, op.variant
+        return run(op, *args)
+    monkeypatch.setattr(T.Op, "run", checked)
+
+
 def _wq(desc, w_q, keep):
     desc.w_scale, desc.w_zp = w_q[0], w_q[1]
     if w_q[2] is not None:
@@ -80,7 +91,8 @@ def _wq(desc, w_q, keep):
 
 def gpu_conv2d(x, w, bias, *, in_shape, w_shape, out_shape, stride, dilation, pad_left, pad_top,
                multiplier, in_dtype, w_dtype, out_dtype, in_q=(1.0, 0), w_q=(1.0, 0, None),
-               out_q=(1.0, 0), act=0, const_weights=True, want_kernel=None, groups=0, transposed=False, misalign=0):
+               out_q=(1.0, 0), act=0, const_weights=True, want_kernel=None, groups=0, transposed=False, misalign=0,
+               want_variant=None):
     """misalign: byte offset of the activation and result tensors from their (256-byte aligned) allocations."""
     T = tvx()
     d = T.Conv2dDesc()
@@ -100,6 +112,7 @@ def gpu_conv2d(x, w, bias, *, in_shape, w_shape, out_shape, stride, dilation, pa
     op = (T.deconv2d_create if transposed else T.conv2d_create)(d, w if const_weights else None, bias)
     if want_kernel is not None:
         assert op.kernel_name in ((want_kernel,) if isinstance(want_kernel, str) else want_kernel), op.kernel_name
+    assert want_variant is None or op.variant == want_variant, op.variant
     import torch
     xd = to_device(x)
     wd = None if const_weights else to_device(w)

@@ -122,6 +122,8 @@ def lib():
         L.tvx_status_string.argtypes = [C.c_int]
         L.tvx_op_kernel_name.restype = C.c_char_p
         L.tvx_op_kernel_name.argtypes = [vp]
+        L.tvx_op_variant.restype = C.c_char_p
+        L.tvx_op_variant.argtypes = [vp]
         L.tvx_malloc.argtypes = [C.POINTER(vp), C.c_size_t]
         L.tvx_free.argtypes = [vp]
         for f in (L.tvx_memcpy_h2d, L.tvx_memcpy_d2h, L.tvx_memcpy_d2d):
@@ -175,6 +177,10 @@ class Op:
     @property
     def kernel_name(self):
         return lib().tvx_op_kernel_name(self.handle).decode()
+
+    @property
+    def variant(self):
+        return lib().tvx_op_variant(self.handle).decode()
 
     def run(self, in0, in1, out, stream=None):
         """in0 / in1 / out are device pointers (ints) or torch CUDA tensors."""

@@ -607,6 +607,7 @@ int RegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const voi
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
   op->run = ConvIm2colRegRun;
   op->kernel_name = pool ? "conv2d_im2col_maxpool_i8" : "conv2d_im2col_i8";
+  op->variant = pool ? "conv2d_im2col_reg_maxpool_i8" : "conv2d_im2col_reg_i8";
   return TVX_OK;
 }
 

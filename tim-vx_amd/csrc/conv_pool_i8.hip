@@ -314,6 +314,7 @@ int ConvPoolSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
   op->run = ConvPoolRun;
   op->kernel_name = "conv2d_igemm_maxpool_i8";
+  op->variant = "conv2d_pool_i8";
   return TVX_OK;
 }
 

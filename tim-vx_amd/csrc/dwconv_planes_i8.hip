@@ -491,6 +491,7 @@ int DwRowsSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const 
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&p), reinterpret_cast<const uint8_t*>(&p) + sizeof(p));
   op->run = DwRowsRun;
   op->kernel_name = op->out_blocked ? "dwconv_planes_to_blocked_i8" : "dwconv_planes_i8";
+  if (!op->out_blocked) op->variant = "dwconv_rows_i8";
   return TVX_OK;
 }
 

@@ -343,6 +343,7 @@ int DwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
   op->run = DwRegRun;
   op->kernel_name = dt == TVX_I8 ? "dwconv_planes_i8" : dt == TVX_F16 ? "dwconv_reg_f16" : "dwconv_reg_f32";
+  if (dt == TVX_I8) op->variant = "dwconv_reg_i8";
   return TVX_OK;
 }
 

@@ -706,6 +706,7 @@ int FcRowsSetup(tvx_op* op, const tvx_fc_desc* d, const void* w_host, const void
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
   op->run = FcRowsRun;
   op->kernel_name = dt == kF32 ? "fc_rows_f32" : dt == kF16 ? "fc_rows_f16" : "fc_rows_i8";
+  if (sp.stage) op->variant = dt == kF16 ? "fc_tile_f16" : "fc_tile_i8";
   return TVX_OK;
 }
 

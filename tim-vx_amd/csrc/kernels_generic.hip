@@ -501,12 +501,12 @@ __global__ void __launch_bounds__(kBlock) PoolPlaneSumKernel(PoolArgs a, const T
 }
 
 template <typename T>
-static void LaunchPoolPlaneAvg(const PoolArgs& a, const void* in0, void* out, uint64_t planes, hipStream_t st) {
+static void LaunchPoolPlaneAvg(const PoolArgs& a, const void* in0, void* out, uint64_t planes, bool by_workgroup, hipStream_t st) {
   const int n_dw = (a.in_w * a.in_h + 3) / 4;
   const T* x = static_cast<const T*>(in0);
   T* y = static_cast<T*>(out);
   const dim3 block(kBlock);
-  if (a.in_w * a.in_h >= kPlaneBytes && planes < (1u << 31)) {
+  if (by_workgroup) {
     hipLaunchKernelGGL((PoolPlaneSumKernel<T>), dim3(static_cast<unsigned>(planes)), block, 0, st, a, x, y);
     return;
   }
@@ -552,6 +552,12 @@ static bool IsPlaneAverageFloat(const tvx_op* op) {
   const uint64_t hw = static_cast<uint64_t>(op->pool.in_w) * op->pool.in_h;
   return !op->quantized && CoversPlane(op) && hw >= 32 && hw <= (1u << 30);
 }
+// ... by a workgroup of PoolPlaneSumKernel each?
+static bool SumsByWorkgroup(const tvx_op* op) {
+  const tvx_pool2d_desc& d = op->pool;
+  const uint64_t planes = static_cast<uint64_t>(d.channels) * d.batch;
+  return (IsPlaneAverage(op) || IsPlaneAverageFloat(op)) && static_cast<uint64_t>(d.in_w) * d.in_h * DtypeBytes(d.dtype) >= kPlaneBytes && planes < (1u << 31);
+}
 
 int PoolGenericRun(tvx_op* op, const void* in0, const void*, void* out, hipStream_t st) {
   const tvx_pool2d_desc& d = op->pool;
@@ -564,15 +570,15 @@ int PoolGenericRun(tvx_op* op, const void* in0, const void*, void* out, hipStrea
              op->quantized ? static_cast<double>(d.in_scale) / static_cast<double>(d.out_scale) : 1.0};
   const uint64_t total = static_cast<uint64_t>(d.out_w) * d.out_h * d.channels * d.batch;
   if (IsPlaneAverage(op)) {
-    if (d.dtype == TVX_U8) LaunchPoolPlaneAvg<uint8_t>(a, in0, out, total, st);
-    else LaunchPoolPlaneAvg<int8_t>(a, in0, out, total, st);
+    if (d.dtype == TVX_U8) LaunchPoolPlaneAvg<uint8_t>(a, in0, out, total, SumsByWorkgroup(op), st);
+    else LaunchPoolPlaneAvg<int8_t>(a, in0, out, total, SumsByWorkgroup(op), st);
     TVX_HIP_CHECK(hipGetLastError());
     return TVX_OK;
   }
   if (IsPlaneAverageFloat(op)) {
     const int hw = a.in_w * a.in_h;
     const dim3 blocks(Blocks(total * 64)), threads(kBlock);
-    if (static_cast<uint64_t>(hw) * DtypeBytes(d.dtype) >= kPlaneBytes && total < (1u << 31)) {
+    if (SumsByWorkgroup(op)) {
       const dim3 grid(static_cast<unsigned>(total));
       if (d.dtype == TVX_F32) hipLaunchKernelGGL((PoolPlaneSumKernel<float>), grid, threads, 0, st, a, static_cast<const float*>(in0), static_cast<float*>(out));
       else hipLaunchKernelGGL((PoolPlaneSumKernel<__half>), grid, threads, 0, st, a, static_cast<const __half*>(in0), static_cast<__half*>(out));
@@ -1187,6 +1193,7 @@ int PoolGenericSetup(tvx_op* op) {
   }
   op->run = PoolGenericRun;
   op->kernel_name = IsPlaneAverage(op) ? "avgpool_plane_i8" : "pool2d_generic";
+  if (SumsByWorkgroup(op)) op->variant = "pool2d_plane_sum";
   return TVX_OK;
 }
 

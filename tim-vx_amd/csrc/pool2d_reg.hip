@@ -357,6 +357,7 @@ int PoolRegPlan(tvx_op* op, unsigned align_in, unsigned align_out, const char* n
   plan.align_out = align_out;
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
   op->run = PoolRegRun;
+  op->variant = op->quantized ? "pool2d_reg_i8" : nullptr;
   op->kernel_name = name ? name : op->quantized ? "pool2d_reg_i8" : d.dtype == TVX_F16 ? "pool2d_reg_f16" : "pool2d_reg_f32";
   return TVX_OK;
 }

@@ -1030,6 +1030,7 @@ int tvx_op_run3(tvx_op* op, const void* in0, const void* in1, const void* in2, v
 }
 
 const char* tvx_op_kernel_name(const tvx_op* op) { return op ? op->kernel_name : ""; }
+const char* tvx_op_variant(const tvx_op* op) { return op && op->variant ? op->variant : tvx_op_kernel_name(op); }
 
 void tvx_op_destroy(tvx_op* op) { delete op; }
 
