@@ -57,3 +57,24 @@ def test_which_kernel_takes_a_quantized_3x3_layer(oracle, c, h, w, stride, kerne
         x, wt, b, kws = conv_case(rng, n=2, c=c, h=h, w=w, oc=0, kh=3, kw=3, stride=[stride, stride], dil=[1, 1], pad=pad, mult=1, mode=mode)
         got = TC.gpu_conv2d(x, wt, b, act=2, want_variant=kernel, **kws)
         assert np.array_equal(got, oracle.conv2d(x, wt, b, act=2, **kws))
+
+
+def test_launches_of_no_more_threads_than_there_can_be():
+    """2^32 threads: kernels that take more of them than the ones before decline from there on. (Nothing runs: these tensors have gigabytes.)"""
+    T = TC.tvx()
+    p = T.Pool2dDesc()
+    p.in_w, p.in_h, p.channels, p.out_w, p.out_h, p.k_w, p.k_h, p.stride_w, p.stride_h = 64, 32, 64, 1, 1, 64, 32, 1, 1
+    p.pool_type = T.POOL_AVG
+    for dtype, kernel in ((T.U8, "avgpool_plane_i8"), (T.F16, "pool2d_generic"), (T.F32, "pool2d_generic")):
+        p.dtype, p.in_scale, p.out_scale = dtype, 0.5, 0.5
+        for p.batch, want in ((2 ** 18 - 1, "pool2d_plane_sum"), (2 ** 18, kernel)):
+            op = T.pool2d_create(p)
+            assert op.variant == want, (dtype, p.batch, op.variant)
+            op.close()
+    rng = np.random.default_rng(5)
+    x, w, b, kws = conv_case(rng, n=1, c=17, h=8, w=8, oc=128, kh=3, kw=3, stride=[1, 1], dil=[1, 1], pad=[1, 1, 1, 1], mult=0, mode="u8")
+    for n, want in ((2 ** 22 - 1, "conv2d_pool_i8"), (2 ** 22, "conv2d_igemm_maxpool_i8")):
+        kws["in_shape"][3] = kws["out_shape"][3] = n
+        op = T.conv2d_pool_create(*SN._descs(T, kws, 0, []), w, b)
+        assert op.variant == want, (n, op.variant)
+        op.close()

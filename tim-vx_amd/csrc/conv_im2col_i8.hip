@@ -520,7 +520,7 @@ int RegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const voi
   const int kw = static_cast<int>(d->k_w), C = d->in_c, kh = d->k_h, rows = C * kh;
   const uint64_t total = static_cast<uint64_t>(d->batch) * d->in_c * d->in_h * d->in_w;
   const uint64_t out_pixels = static_cast<uint64_t>(d->out_h) * d->out_w, tpi = (out_pixels + 31) / 32, tiles = tpi * d->batch;
-  if ((kw != 3 && kw != 5) || d->dilation_w != 1 || total < 8 || total >= (1ull << 31) - 64 || tiles >= (1ull << 31) - 4096) return TVX_E_UNSUPPORTED;
+  if ((kw != 3 && kw != 5) || d->dilation_w != 1 || total < 8 || total >= (1ull << 31) - 64 || !LaunchFits((tiles + 7) / 8, 64)) return TVX_E_UNSUPPORTED;
   if (const char* f = getenv("TVX_IM2COL_ROWS"))  // tuning aid
     if (!atoi(f)) return TVX_E_UNSUPPORTED;
   const int per = kw == 3 ? 5 : 3, ks = (rows + 2 * per - 1) / (2 * per), K = rows * kw;

@@ -261,6 +261,7 @@ int ConvPoolSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   a.parts = (a.steps + a.per_part - 1) / a.per_part;
   a.m_parts = reciprocal(a.parts);
   const int waves = a.parts > 1 ? a.parts * a.tiles : std::min(kMaxWaves, a.tiles);
+  if (!LaunchFits(wgs, 64 * waves)) return TVX_E_UNSUPPORTED;
   a.z4 = static_cast<int>(static_cast<uint32_t>((zws == -128 ? 64 : -zws) & 0xff) * 0x01010101u);
   a.ztwice = zws == -128;
   a.last_channels = a.C - (a.per_tap - 1) * 32;

@@ -499,6 +499,7 @@ int DwPwSetup(tvx_op* op, const tvx_conv2d_desc* dw, const void* dw_w, const voi
   // stride 2, a depthwise pass of at most 128 threads: half of four wavefronts would only wait for the other half (batch 64: 112 x 112, 32 to 16
   // 11.6 -> 9.9 us, 16 to 32 10.7 -> 8.9, 56 x 56, 32 to 64 6.3 -> 6.2; at stride 1 four are ahead: 28 x 28, 32 to 64 6.4 against 7.7)
   if (S == 2 && tiles > 2ull * cus && (a.quads << lpr_shift) <= 128) waves = 2;
+  if (!LaunchFits(tiles, 64 * waves)) waves = kWaves;
   if (const char* f = getenv("TVX_DWPW_WAVES")) waves = std::max(1, std::min(atoi(f), kMaxWaves));  // test lever
   // pointwise weights in fragment order, constants folded into the bias (as PwConvSetup packs them)
   const int oc_alloc = a.oc_tiles * 32;

@@ -556,7 +556,7 @@ static bool IsPlaneAverageFloat(const tvx_op* op) {
 static bool SumsByWorkgroup(const tvx_op* op) {
   const tvx_pool2d_desc& d = op->pool;
   const uint64_t planes = static_cast<uint64_t>(d.channels) * d.batch;
-  return (IsPlaneAverage(op) || IsPlaneAverageFloat(op)) && static_cast<uint64_t>(d.in_w) * d.in_h * DtypeBytes(d.dtype) >= kPlaneBytes && planes < (1u << 31);
+  return (IsPlaneAverage(op) || IsPlaneAverageFloat(op)) && static_cast<uint64_t>(d.in_w) * d.in_h * DtypeBytes(d.dtype) >= kPlaneBytes && LaunchFits(planes, kBlock);
 }
 
 int PoolGenericRun(tvx_op* op, const void* in0, const void*, void* out, hipStream_t st) {

@@ -934,7 +934,7 @@ int MbConvSetup(tvx_op* op, const MbStage& ex, const MbStage& dw, const tvx_conv
   }
   plan.block = 64 * waves;
   if (plan.lds_bytes > 160 * 1024) return TVX_E_UNSUPPORTED;
-  if (wgs > 0x7fffffffull) return TVX_E_UNSUPPORTED;
+  if (!LaunchFits(wgs, plan.block)) return TVX_E_UNSUPPORTED;
   plan.grid = static_cast<unsigned>(wgs);
 
   // ---- expansion ----

@@ -336,6 +336,8 @@ int64_t AccumulatorBound(uint64_t reduction, const void* bias_host, uint32_t cha
 int BuildRequantTables(uint32_t channels, float in_scale, float w_scale,
                        const float* w_scales, float out_scale,
                        std::vector<int32_t>* mult, std::vector<int32_t>* shift);
+// A launch has fewer than 2^32 threads.
+inline bool LaunchFits(uint64_t workgroups, unsigned threads) { return workgroups < (uint64_t{1} << 32) / threads; }
 // compute units of the current device
 int ComputeUnits();
 
