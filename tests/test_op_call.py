@@ -1,6 +1,9 @@
 """Op.run's native call against the ctypes one: the same status and error for every kind of argument. No GPU: the library checks
 its operands before it launches anything."""
 import ctypes as C
+import importlib.util
+import sys
+import warnings
 
 import pytest
 
@@ -48,3 +51,26 @@ def test_native_call_passes_addresses():
     finally:
         module.bind(C.cast(L.tvx_op_run, C.c_void_p).value)
     assert seen == [((1 << 47) + 16, (1 << 47) + 17, None, (1 << 47) + 18, 7), (5, 6, None, 8, None)]
+
+
+@pytest.mark.parametrize("native", [False, True], ids=["ctypes", "native"])
+def test_no_truth_of_not_implemented(monkeypatch, native):
+    """A pointer type that only ctypes knows gives NotImplemented, whose truth warns and in later versions raises."""
+    T = TC.tvx()
+    T.lib()
+    if not native:
+        monkeypatch.setattr(T, "_run", T._ctypes_run)
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        with pytest.raises(T.TvxError, match="null operator"):
+            T.Op(None).run(_Tensor(4096), None, 4096, C.POINTER(C.c_int)())
+
+
+def test_run_loads_the_library(monkeypatch):
+    T = TC.tvx()
+    spec = importlib.util.spec_from_file_location("tvx_unloaded", T.__file__, submodule_search_locations=T.__path__)
+    unloaded = importlib.util.module_from_spec(spec)
+    monkeypatch.setitem(sys.modules, "tvx_unloaded", unloaded)
+    spec.loader.exec_module(unloaded)
+    with pytest.raises(unloaded.TvxError, match="null operator"):
+        unloaded.Op(None).run(4096, None, 4096)

@@ -74,7 +74,14 @@ class TvxError(RuntimeError):
 
 
 _lib = None
-_run = None   # tvx_op_run by the native binding (src/op_call.c), or through ctypes
+
+
+def _first_run(*args):
+    lib()
+    return _run(*args)
+
+
+_run = _first_run   # from lib() on tvx_op_run by the native binding (src/op_call.c), or through ctypes
 
 
 def _ctypes_run(handle, in0, in1, out, stream):
@@ -185,7 +192,7 @@ class Op:
     def run(self, in0, in1, out, stream=None):
         """in0 / in1 / out are device pointers (ints) or torch CUDA tensors."""
         status = _run(self.handle, in0, in1, out, stream)
-        if status:
+        if status != OK:
             check(status if status is not NotImplemented else _ctypes_run(self.handle, in0, in1, out, stream))
 
     def close(self):
