@@ -1,6 +1,7 @@
 """Op.run's native call against the ctypes one: the same status and error for every kind of argument. No GPU: the library checks
 its operands before it launches anything."""
 import ctypes as C
+import enum
 import importlib.util
 import sys
 import warnings
@@ -43,13 +44,13 @@ def test_native_call_passes_addresses():
     seen = []
     run = C.CFUNCTYPE(C.c_int, *[C.c_void_p] * 5)(lambda *a: seen.append(a) or -3)
     module = T._run.__self__
-    module.bind(C.cast(run, C.c_void_p).value)
+    module.bind(C.cast(run, C.c_void_p).value, C.c_void_p)
     try:
         high = (1 << 47) + 16
         assert T._run(C.c_void_p(high), _Tensor(high + 1), None, high + 2, C.c_void_p(7)) == -3
         assert T._run(5, 6, _Tensor(0), _Tensor(8), None) == -3
     finally:
-        module.bind(C.cast(L.tvx_op_run, C.c_void_p).value)
+        module.bind(C.cast(L.tvx_op_run, C.c_void_p).value, C.c_void_p)
     assert seen == [((1 << 47) + 16, (1 << 47) + 17, None, (1 << 47) + 18, 7), (5, 6, None, 8, None)]
 
 
@@ -74,3 +75,33 @@ def test_run_loads_the_library(monkeypatch):
     spec.loader.exec_module(unloaded)
     with pytest.raises(unloaded.TvxError, match="null operator"):
         unloaded.Op(None).run(4096, None, 4096)
+
+
+class _Code(enum.Enum):
+    OTHER = 4096
+
+
+@pytest.mark.parametrize("native", [False, True], ids=["ctypes", "native"])
+def test_what_is_no_pointer_is_refused(monkeypatch, native):
+    T = TC.tvx()
+    T.lib()
+    if not native:
+        monkeypatch.setattr(T, "_run", T._ctypes_run)
+    for wrong in (C.c_int(4096), C.c_uint64(4096), _Code.OTHER):
+        with pytest.raises(C.ArgumentError):
+            T.Op(None).run(4096, None, 4096, wrong)
+        with pytest.raises(C.ArgumentError):
+            T.Op(wrong).run(4096, None, 4096)
+
+
+@pytest.mark.parametrize("native", [False, True], ids=["ctypes", "native"])
+def test_addresses_of_every_kind(monkeypatch, native):
+    T = TC.tvx()
+    T.lib()
+    if not native:
+        monkeypatch.setattr(T, "_run", T._ctypes_run)
+    for address in (None, 4096, C.c_void_p(4096), C.POINTER(C.c_int)()):
+        with pytest.raises(T.TvxError, match="null operator"):
+            T.Op(None).run(_Tensor(address), None, _Tensor(4096))
+    with pytest.raises(C.ArgumentError):
+        T.Op(None).run(_Tensor(1.5), None, _Tensor(4096))

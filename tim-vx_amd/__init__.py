@@ -99,7 +99,7 @@ def _native_run(L):
     spec = importlib.util.spec_from_file_location("tvx_call", path)
     module = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(module)
-    module.bind(C.cast(L.tvx_op_run, C.c_void_p).value)
+    module.bind(C.cast(L.tvx_op_run, C.c_void_p).value, C.c_void_p)
     return module.run
 
 
