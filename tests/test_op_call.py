@@ -2,8 +2,11 @@
 its operands before it launches anything."""
 import ctypes as C
 import enum
+import importlib.machinery
 import importlib.util
+import os
 import sys
+import sysconfig
 import warnings
 
 import pytest
@@ -19,12 +22,18 @@ class _Tensor:
         return self.address
 
 
+def _needs_binding(T):
+    if not os.path.exists(os.path.join(sysconfig.get_paths()["include"], "Python.h")):
+        pytest.skip("no headers of Python: the call goes through ctypes")
+    assert T._run is not T._ctypes_run, "the native call is not built"
+
+
 @pytest.mark.parametrize("native", [False, True], ids=["ctypes", "native"])
 def test_run_arguments(monkeypatch, native):
     T = TC.tvx()
     T.lib()
     if native:
-        assert T._run is not T._ctypes_run, "lib/tvx_call.so is not built"
+        _needs_binding(T)
     else:
         monkeypatch.setattr(T, "_run", T._ctypes_run)
     t = _Tensor(4096)
@@ -41,6 +50,7 @@ def test_run_arguments(monkeypatch, native):
 def test_native_call_passes_addresses():
     T = TC.tvx()
     L = T.lib()
+    _needs_binding(T)
     seen = []
     run = C.CFUNCTYPE(C.c_int, *[C.c_void_p] * 5)(lambda *a: seen.append(a) or -3)
     module = T._run.__self__
@@ -105,3 +115,25 @@ def test_addresses_of_every_kind(monkeypatch, native):
             T.Op(None).run(_Tensor(address), None, _Tensor(4096))
     with pytest.raises(C.ArgumentError):
         T.Op(None).run(_Tensor(1.5), None, _Tensor(4096))
+
+
+def test_a_binding_that_does_not_load_leaves_the_call_to_ctypes(monkeypatch, tmp_path):
+    """A file of another interpreter's ABI, or a broken one."""
+    T = TC.tvx()
+    L = T.lib()
+    (tmp_path / "lib").mkdir()
+    (tmp_path / "lib" / ("tvx_call" + importlib.machinery.EXTENSION_SUFFIXES[0])).write_bytes(b"no library")
+    (tmp_path / "lib" / "tvx_call.so").write_bytes(b"no library")
+    monkeypatch.setattr(T, "PKG_DIR", str(tmp_path))
+    assert T._native_run(L) is T._ctypes_run
+
+
+def test_a_build_without_headers_leaves_no_binding_behind(monkeypatch, tmp_path):
+    build = importlib.import_module("tim-vx_amd.build")
+    (tmp_path / "lib").mkdir()
+    for name in ("tvx_call" + importlib.machinery.EXTENSION_SUFFIXES[0], "tvx_call.so"):
+        (tmp_path / "lib" / name).write_bytes(b"")
+    monkeypatch.setattr(build, "PKG_DIR", str(tmp_path))
+    monkeypatch.setattr(sysconfig, "get_paths", lambda: {"include": str(tmp_path)})
+    build.build_binding()
+    assert os.listdir(str(tmp_path / "lib")) == []

@@ -6,6 +6,7 @@ through ctypes so tests and the benchmark can drive it with device memory
 held in torch tensors. There is no CPU path: every compute call needs a GPU.
 """
 import ctypes as C
+import importlib.machinery
 import importlib.util
 import os
 
@@ -93,12 +94,13 @@ def _ctypes_run(handle, in0, in1, out, stream):
 
 
 def _native_run(L):
-    path = os.path.join(PKG_DIR, "lib", "tvx_call.so")
-    if not os.path.exists(path):
-        return _ctypes_run
+    path = os.path.join(PKG_DIR, "lib", "tvx_call" + importlib.machinery.EXTENSION_SUFFIXES[0])   # (this interpreter's)
     spec = importlib.util.spec_from_file_location("tvx_call", path)
-    module = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(module)
+    try:
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+    except ImportError:   # not built, or no library
+        return _ctypes_run
     module.bind(C.cast(L.tvx_op_run, C.c_void_p).value, C.c_void_p)
     return module.run
 

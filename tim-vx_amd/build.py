@@ -2,6 +2,7 @@
 runtime on top of it (lib/libtim-vx.so). hipcc cross-compiles gfx950 without a
 GPU, so this runs in the build container; the results travel to the GPU box."""
 import glob
+import importlib.machinery
 import os
 import subprocess
 import sys
@@ -76,11 +77,13 @@ def build_runtime(verbose=False):
 
 
 def build_binding(verbose=False):
-    """The Python binding's native call (lib/tvx_call.so); without Python's headers the binding goes through ctypes."""
+    """The Python binding's native call, for this interpreter alone; without Python's headers the binding goes through ctypes."""
     include = sysconfig.get_paths()["include"]
+    for old in glob.glob(os.path.join(PKG_DIR, "lib", "tvx_call*.so")):
+        os.remove(old)
     if os.path.exists(os.path.join(include, "Python.h")):
         _run(["gcc", "-O2", "-fPIC", "-shared", "-Wall", "-I", include, os.path.join(PKG_DIR, "src", "op_call.c"),
-              "-o", os.path.join(PKG_DIR, "lib", "tvx_call.so")], verbose)
+              "-o", os.path.join(PKG_DIR, "lib", "tvx_call" + importlib.machinery.EXTENSION_SUFFIXES[0])], verbose)
 
 
 def build_all(verbose=False):
