@@ -35,3 +35,26 @@ def test_tilings(oracle, monkeypatch, ci, wide, mode):
             return x, first, (wd, bd, kd), last
         monkeypatch.setattr(MB, "_block", shifted)
     MB.test_inverted_residual_block(oracle, ci, "u8" if mode == "u8zp0" else mode, ci % 3, monkeypatch)
+
+
+@pytest.mark.parametrize("n,cin,cexp,cout,w,taken", [
+    (13, 32, 64, 96, 28, True), (14, 32, 64, 96, 28, False), (5, 128, 160, 32, 28, True), (6, 128, 160, 32, 28, False), (6, 32, 64, 100, 28, False),
+    (64, 64, 96, 160, 14, True), (1, 64, 96, 161, 14, False), (64, 64, 96, 160, 7, True), (1, 64, 96, 161, 7, False)])
+def test_blocks_taken_of_its_own_accord(n, cin, cexp, cout, w, taken):
+    """Both sides of each line of the rule, at 256 compute units."""
+    import numpy as np
+    import torch
+    import tvx_case as TC
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the lines are drawn in workgroups a compute unit")
+    T, keep = TC.tvx(), []
+    x, (w1, b1, k1), (wd, bd, kd), (w3, b3, k3) = MB._block(np.random.default_rng(3), 1, cin, cexp, cout, w, w, 1, "u8")
+    for k in (k1, kd, k3):
+        k["in_shape"][3] = k["out_shape"][3] = n
+    descs = [MB._desc(T, k, 0, keep) for k in (k1, kd, k3)]
+    try:
+        T.mbconv_create(descs[0], w1, b1, descs[1], wd, bd, descs[2], w3, b3).close()
+    except T.TvxError as e:
+        assert e.status == T.E_UNSUPPORTED and not taken
+    else:
+        assert taken

@@ -883,11 +883,14 @@ int MbConvSetup(tvx_op* op, const MbStage& ex, const MbStage& dw, const tvx_conv
     //   28 columns, 32 to 192 to 32    narrow   4.2  5.3  6.7  10.2  16.3  29.5    apart 9.2  9.4  9.7  11.0  13.9  20.5
     //   7 columns, 160 to 960 to 160   narrow   9.7  9.9  9.9  10.3  11.0  18.0    apart 10.4  11.6  12.2  14.3  16.6  20.2    wide - 16.6
     //   7 columns, 160 to 960 to 320   narrow  33.6  ...             36.0  61.8    apart 10.3  11.4  12.0  14.3  16.8  20.5
-    // narrow as long as each of its workgroups finds a CU of its own
+    //  14 columns, 160 to 960 to 320   narrow  19.3  20.1       35.1       108.6   apart 10.1  13.6       20.5        46.6
+    // Taken: up to 160 results; of 28 columns only while workgroups are few (batch 13, here and as two or three launches: 32 to 192 to 32 9.2 and 9.9,
+    // 64 to 384 to 64 13.1 and 14.2, 96 to 576 to 96 20.9 and 22.8; batch 14 10.1 and 10.2, 14.7 and 14.8; 160 to 160 to 160 batch 5 8.2 and 10.1, 6
+    // 13.0 and 10.1; 128 to 768 to 128 14.5 and 16.6, 21.3 and 18.2). Narrow as long as each of its workgroups finds a CU of its own.
     const uint64_t narrow_wgs = static_cast<uint64_t>(e->batch) * ((H + 1) / 2) * ((W + 3) / 4), cus = ComputeUnits();
     wide = W != 28 && nt <= 5 && narrow_wgs > cus;
     if (const char* f = getenv("TVX_MBCONV_WIDE")) wide = W != 28 && nt <= 5 && atoi(f);  // test lever
-    if (!all && ((W == 28 && narrow_wgs > 7 * cus) || (W == 7 && nt > 5))) return TVX_E_UNSUPPORTED;
+    if (!all && (nt > 5 || (W == 28 && narrow_wgs > (std::max(cin_steps, nt) <= 3 ? 5 : 2) * cus))) return TVX_E_UNSUPPORTED;
     a.W = W; a.batch = e->batch;
     a.half_rows = wide && W == 7 ? 2 : 0;
     a.half_cols = wide && W == 14 ? 7 : 0;
