@@ -866,6 +866,7 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   while ((1 << a.wide_shift) < a.runs * wide_groups) ++a.wide_shift;
   a.m_gl = Magic(a.gl); a.m_cells = Magic(a.cells); a.m_ncg = Magic(a.ncg); a.m_ih = Magic(a.IH); a.m_iw = Magic(a.IW); a.m_tw = Magic(a.TW); a.m_thtw = Magic(a.TH * a.TW);
   a.m_ocb = Magic(a.oc_wgs); a.m_tpg = Magic(a.wgs_per_group); a.m_tx = Magic(a.tiles_x); a.m_ty = Magic(a.tiles_y);
+  if (static_cast<int64_t>(a.IH - 1) * a.row_step >= 1 << 23) return TVX_E_UNSUPPORTED;  // (24-bit products of rows and columns; the others lie within LDS)
   // a reciprocal is exact while dividend * divisor < 2^32
   if (static_cast<uint64_t>(a.total) * std::max({a.oc_wgs, a.tiles_x, a.tiles_y}) >= (1ull << 32)) return TVX_E_UNSUPPORTED;
   if (static_cast<uint64_t>(npx) * a.gpc * std::max({a.gpc, a.cells, a.IH, a.IW}) >= (1ull << 32)) return TVX_E_UNSUPPORTED;
