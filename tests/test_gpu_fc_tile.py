@@ -55,3 +55,16 @@ def test_rows_keep_an_infinity_apart(monkeypatch, shape):
     x[2, 0] = np.inf
     got = TC.gpu_fully_connected(x.ravel(), w.ravel(), None, m=4, k=37, n=20, in_dtype=2, w_dtype=2, out_dtype=2, want_kernel="fc_rows_f16").reshape(4, 20)
     assert np.isinf(got[2]).all() and np.array_equal(got[[0, 1, 3]], np.full((3, 20), 37, np.float16))
+
+
+@pytest.mark.parametrize("m,k,n,mode,kernel", [
+    (332, 672, 1965, "i8pc", "fc_rows_i8"), (578, 685, 832, "i8pc", "fc_rows_i8"), (617, 358, 921, "f16", "fc_rows_f16"),   # reductions that end early in their last stage
+    (393, 704, 1908, "u8", "fc_tile_i8"), (900, 512, 1100, "f16", "fc_tile_f16"), (3521, 560, 1238, "i8pc", "fc_tile_i8")])
+def test_which_tiles_a_layer_gets(oracle, m, k, n, mode, kernel, monkeypatch):
+    x, w, b, kws = _case(m, k, n, mode)
+    TC.expect_variant(monkeypatch, kernel)
+    got, want = TC.gpu_fully_connected(x, w, b, act=1, **kws), oracle.fully_connected(x, w, b, act=1, **kws)
+    if mode == "f16":   # (as above)
+        assert np.allclose(got.astype(np.float64), want.astype(np.float64), rtol=2e-3, atol=2e-3)
+    else:
+        assert np.array_equal(got, want)

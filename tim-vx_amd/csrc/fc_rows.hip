@@ -531,9 +531,10 @@ uint32_t Magic(int d) { return d <= 1 ? 0u : static_cast<uint32_t>(((uint64_t{1}
 // Microseconds of a launch on tiles of a shape: what a launch takes anyway, then per stage of the reduction either its latency, once for
 // every round of workgroups a CU holds, or the time its share of the CU's units takes, whichever is longer, and at the end its results. The
 // constants are a fit to 310 drawn layers (at least 60000 outputs, int8 and float16) measured back to back in a captured graph, 6 to 15 %
-// off each; the shape chosen by them takes 3 % more than the best measured one on the (geometric) average, where the rule before (32 x 32 or
-// 64 x 64 by their number, or the 256 x 256 tiles) took 20 %. u8 4978 x 64 -> 3462: 30.7 -> 15.6 us, i8 3521 x 560 -> 1238:
-// 19.9 -> 13.3, f16 4138 x 3888 -> 603: 82.8 -> 47.9.
+// off each. On 1961 other drawn layers (m 1 to 8192, k 64 to 4096, n 10 to 4096, more 16 x 16 tiles than CUs) the shape chosen takes 0.86
+// of the time of 32 x 32 or 64 x 64 tiles by their number (geometric mean) and 1.4 % more than the best of the seven; 18 of them are slower
+// than those tiles by more than 3 %, 30 where a cut reduction was charged whole stages (i8 332 x 672 -> 1965: 5.2 us, 6.5 on the tiles that were
+// chosen then). u8 4978 x 64 -> 3462: 30.7 -> 15.6 us, i8 3521 x 560 -> 1238: 19.9 -> 13.3, f16 4138 x 3888 -> 603: 82.8 -> 47.9.
 struct Fit { int resident; double base, latency, share, end, unaligned; };  // workgroups of a CU; us, and by how much more at any byte
 const Fit kFits[2][kShapeCount] = {
     {{}, {4, 1.15, 0.48, 0.80, 0.10, 0.49}, {4, 2.25, 0.11, 0.16, 1.12, 1.33}, {4, 1.53, 0.62, 0.37, 0.55, 0.17}, {2, 2.09, 0.72, 0.56, 1.02, 0.14},
@@ -546,7 +547,10 @@ double Cost(const tvx_fc_desc& d, int dt, int shape) {
   const double row = static_cast<double>(d.k) * (dt == kI8 ? 1 : 2);
   const int stage = sp.stage ? 32 * sp.stage : 32 * sp.ks * (sp.ks > 1 ? 4 : 1);
   const double per_cu = static_cast<double>((d.m + sp.rows - 1) / sp.rows) * ((d.n + sp.features - 1) / sp.features) / ComputeUnits();
-  const double stages = std::ceil(row / stage) * (static_cast<uint64_t>(row) % 4 ? 1 + f.unaligned : 1);
+  double stages = std::ceil(row / stage);
+  // (a reduction cut over wavefronts may end early in its last stage, which saves half of what is missing; behind one stage alone, nothing)
+  if (sp.ks > 1 && stages > 1) stages = 0.5 * (stages + 0.25 * std::ceil(std::ceil(row / 32) / sp.ks));
+  if (static_cast<uint64_t>(row) % 4) stages *= 1 + f.unaligned;
   const double latency = std::max(per_cu / f.resident, 1.0) * stages * f.latency, share = per_cu * (f.end + stages * f.share);
   return 2.2 + f.base + std::sqrt(std::sqrt(std::pow(latency, 4) + std::pow(share, 4)));
 }
