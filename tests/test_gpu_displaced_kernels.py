@@ -59,11 +59,34 @@ def test_which_kernel_takes_a_quantized_3x3_layer(oracle, c, h, w, stride, kerne
         assert np.array_equal(got, oracle.conv2d(x, wt, b, act=2, **kws))
 
 
+@pytest.mark.parametrize("dtype,w,h", [(0, 40, 70), (1, 61, 46), (2, 60, 76), (3, 42, 42)])
+def test_averages_of_many_planes_by_wavefronts(oracle, dtype, w, h):
+    """Up to eight planes a compute unit, a workgroup each; of more, planes just below their type's line take a wavefront, those beyond a workgroup."""
+    import torch
+    planes, base = 8 * torch.cuda.get_device_properties(0).multi_processor_count, {0: "avgpool_plane_i8", 1: "avgpool_plane_i8", 2: "pool2d_generic", 3: "pool2d_generic"}[dtype]
+    rng = np.random.default_rng(7500 + dtype)
+    T, p = TC.tvx(), TC.tvx().Pool2dDesc()
+    seen = []
+    for n, cols in ((planes - 1, w), (planes, w), (planes, w + 2)):
+        p.in_w, p.in_h, p.channels, p.batch, p.out_w, p.out_h, p.k_w, p.k_h, p.stride_w, p.stride_h = cols, h, n, 1, 1, 1, cols, h, 1, 1
+        p.pool_type, p.dtype, p.in_scale, p.out_scale = T.POOL_AVG, dtype, 0.5, 0.5
+        op = T.pool2d_create(p)
+        seen.append(op.variant)
+        x = rng.integers(0, 100, n * cols * h).astype(TC.NP_OF[dtype])
+        y = TC.device_out(n, TC.NP_OF[dtype])
+        op.run(TC.to_device(x), None, y)
+        got, want = y.cpu().numpy().astype(np.float64), x.astype(np.float64).reshape(n, -1).mean(1)
+        # (whole codes, ties to even; float32 sums of under 5000 values to 2^-19 of them, then a rounding to float16: 2^-11)
+        assert np.array_equal(got, np.rint(want)) if dtype < 2 else np.abs(got / want - 1).max() <= (2.0 ** -10 if dtype == 2 else 2.0 ** -18)
+        op.close()
+    assert seen == ["pool2d_plane_sum", base, "pool2d_plane_sum"]
+
+
 def test_launches_of_no_more_threads_than_there_can_be():
     """2^32 threads: kernels that take more of them than the ones before decline from there on. (Nothing runs: these tensors have gigabytes.)"""
     T = TC.tvx()
     p = T.Pool2dDesc()
-    p.in_w, p.in_h, p.channels, p.out_w, p.out_h, p.k_w, p.k_h, p.stride_w, p.stride_h = 64, 32, 64, 1, 1, 64, 32, 1, 1
+    p.in_w, p.in_h, p.channels, p.out_w, p.out_h, p.k_w, p.k_h, p.stride_w, p.stride_h = 64, 256, 64, 1, 1, 64, 256, 1, 1
     p.pool_type = T.POOL_AVG
     for dtype, kernel in ((T.U8, "avgpool_plane_i8"), (T.F16, "pool2d_generic"), (T.F32, "pool2d_generic")):
         p.dtype, p.in_scale, p.out_scale = dtype, 0.5, 0.5

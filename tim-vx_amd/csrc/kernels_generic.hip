@@ -430,7 +430,7 @@ PoolPlaneAvgKernel(PoolArgs a, const T* __restrict__ x, T* __restrict__ y, uint6
   y[plane] = static_cast<T>(r);
 }
 
-// A workgroup per plane, sixteen bytes a thread and load, four loads in flight: planes of 2 KiB and more (uint8, 240 planes of 120 x 160:
+// A workgroup per plane, sixteen bytes a thread and load, four loads in flight: planes of 2 KiB and more, of some more where there are many (uint8, 240 planes of 120 x 160:
 // 10.2 us with a wavefront a plane and a dword a lane, 2.5 here; int8, 672 of 132 x 132, 20.6 and 3.7).
 constexpr int kPlaneBytes = 2048;
 template <typename T>
@@ -552,11 +552,15 @@ static bool IsPlaneAverageFloat(const tvx_op* op) {
   const uint64_t hw = static_cast<uint64_t>(op->pool.in_w) * op->pool.in_h;
   return !op->quantized && CoversPlane(op) && hw >= 32 && hw <= (1u << 30);
 }
-// ... by a workgroup of PoolPlaneSumKernel each?
+// ... by a workgroup of PoolPlaneSumKernel each? Where there are eight planes a CU, a wavefront each keeps the chip busy, and a
+// workgroup's start and exchange are paid for larger planes alone (400 drawn averages: float32 1530 elements, 5115 planes, 4.7 us by
+// wavefronts, 7.6 by workgroups, 4096 of 3025 8.3 and 9.2, 5014 of 10240 31.7 and 29.8; float16 1463 of 6936 4.8 and 6.8, 4489 of 5696
+// 10.2 and 11.4; 8 bits, which a wavefront loads a dword a lane, 2460 of 6303 4.7 and 5.5, 3249 of 4770 5.7 and 5.4).
 static bool SumsByWorkgroup(const tvx_op* op) {
   const tvx_pool2d_desc& d = op->pool;
-  const uint64_t planes = static_cast<uint64_t>(d.channels) * d.batch;
-  return (IsPlaneAverage(op) || IsPlaneAverageFloat(op)) && static_cast<uint64_t>(d.in_w) * d.in_h * DtypeBytes(d.dtype) >= kPlaneBytes && LaunchFits(planes, kBlock);
+  const uint64_t planes = static_cast<uint64_t>(d.channels) * d.batch, bytes = static_cast<uint64_t>(d.in_w) * d.in_h * DtypeBytes(d.dtype);
+  const uint64_t least = planes < 8ull * ComputeUnits() ? kPlaneBytes : d.dtype == TVX_F32 ? 7168 : d.dtype == TVX_F16 ? 9216 : 2816;
+  return (IsPlaneAverage(op) || IsPlaneAverageFloat(op)) && bytes >= least && LaunchFits(planes, kBlock);
 }
 
 int PoolGenericRun(tvx_op* op, const void* in0, const void*, void* out, hipStream_t st) {
