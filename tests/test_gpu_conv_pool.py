@@ -1,4 +1,4 @@
-"""The convolution + 2 x 2 MAX pooling kernel for planes that fit LDS, with its reduction whole and split: channel counts around a
+"""The convolution + 2 x 2 MAX pooling kernel for planes that fit LDS, with its reduction whole and split, its tiles in one workgroup and in several: channel counts around a
 step, padding on every side, strides and dilation, rows of four to nine columns, more pixel tiles than wavefronts, pooled planes that
 end inside a tile, a weight zero point at the end of its range. Exact against the oracle's two operators."""
 import pytest
@@ -18,11 +18,24 @@ CASES = [
 ]
 
 
+@pytest.mark.parametrize("mode", ["u8", "u8zp0"])
+@pytest.mark.parametrize("groups", [1, 2, 7, 99])
+@pytest.mark.parametrize("ci", range(len(CASES)))
+def test_tiles_dealt_out_to_workgroups(oracle, monkeypatch, ci, groups, mode):
+    """Each loads the rows behind its own tiles."""
+    monkeypatch.setenv("TVX_CONV_POOL_GROUPS", str(groups))
+    _run(oracle, monkeypatch, ci, mode)
+
+
 @pytest.mark.parametrize("mode", ["u8", "i8pc", "u8zp0"])
 @pytest.mark.parametrize("parts", [1, 3, 8])
 @pytest.mark.parametrize("ci", range(len(CASES)))
 def test_split_reductions(oracle, monkeypatch, ci, parts, mode):
     monkeypatch.setenv("TVX_CONV_POOL_PARTS", str(parts))
+    _run(oracle, monkeypatch, ci, mode)
+
+
+def _run(oracle, monkeypatch, ci, mode):
     monkeypatch.setattr(SN, "CONV_POOL", [dict(c, kernel="conv2d_igemm_maxpool_i8") for c in CASES])
     case = SN.conv_case
 

@@ -2,9 +2,9 @@
 // channels), the whole input image in LDS. What bounds such a layer is not its arithmetic but the chain a workgroup walks - load,
 // transpose, multiply, sum, store - and how many wavefronts share it.
 //
-// Workgroup = (image, 32 output channels). Its wavefronts are (32-pixel tile, part of the reduction) pairs, eight where the layer has
-// that many: weights come straight from L2 into registers, the first ones requested before the input; the input is transposed into
-// LDS as [pixel][channel], each tap's operand is read from there; partial sums meet in LDS by integer atomics where the reduction is
+// Workgroup = (image, 32 output channels, all or some of the 32-pixel tiles). Its wavefronts are (tile, part of the reduction) pairs, eight
+// where the layer has that many: weights come straight from L2 into registers, the first ones requested before the input; the rows behind its
+// tiles are transposed into LDS as [pixel][channel], each tap's operand is read from there; partial sums meet in LDS by integer atomics where the reduction is
 // split. Pixels run in pooling order, and pixel 4 i + e of a tile stands in row 8 e + i of the product: a lane finds the four candidates
 // of four consecutive pooled pixels in its accumulators. Requantization is monotone, so a window's largest accumulator is
 // requantized once. The zero-point term of uint8 weights is a second product with a constant fragment.
@@ -12,6 +12,7 @@
 // 12 x 12, 20 to 50, 5 x 5, before (conv2d_igemm_i8's tile, weights through LDS, results staged there) and now,
 // microseconds: batch 1 7.9 / 4.8, batch 90 9.4 / 5.2, batch 207 9.6 / 6.7.
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 
 #include "variants.h"
@@ -30,18 +31,22 @@ struct PoolConvArgs {
   const v4i* w;          // [32-channel tile][step][64 lanes]; steps run over (ky, kx, 32 channels)
   const int32_t* biasf;
   const v4i* rq;
-  int C, H, W, oc_tiles;
-  uint32_t m_octiles;    // reciprocals
+  int C, H, W, oc_tiles, groups;  // groups: workgroups that share an image's tiles
+  uint32_t m_octiles, m_groups;   // reciprocals
   int chan_quads, col_quads;  // of the input in fours
   uint32_t m_units, m_cols;
   int pix_stride, row_stride, pad_t, pad_l;
   uint32_t xor4;
+  int tiles, per_group;       // 32-pixel tiles, of a workgroup
+  int pooled, pw, tile_rows;  // input rows behind two rows of outputs
+  uint32_t m_pw;
+  int sh;
   // ---- later
   int steps, per_tap, kw;     // reduction steps; of a tap; taps of a kernel row
   int tap_x, tap_y;           // bytes from a tap to the next one, from a kernel row's start to the next's
-  int tiles, parts, per_part; // 32-pixel tiles, parts of the reduction, steps of a part
-  uint32_t m_parts, m_pw;
-  int pooled, pw, sh, sw, OH, OW;
+  int parts, per_part;        // parts of the reduction, steps of a part
+  uint32_t m_parts;
+  int sw, OH, OW;
   int halo_rows, halo_cols, pad_fill4, padded;
   int z4, z4_last, ztwice;    // constant fragment: minus the weights' zero point in four bytes
   int last_channels;
@@ -55,7 +60,9 @@ __global__ void __launch_bounds__(kMaxWaves * 64) ConvPoolKernel(PoolConvArgs a)
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, half = lane >> 5, threads = blockDim.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = threads >> 6;
   const auto over = [](int v, uint32_t m) { return static_cast<int>(__umulhi(static_cast<uint32_t>(v), m) + (static_cast<uint32_t>(v) & (m ? 0u : ~0u))); };
-  const int n = over(blockIdx.x, a.m_octiles), ot = blockIdx.x - n * a.oc_tiles;
+  const int pair = over(blockIdx.x, a.m_groups), group = blockIdx.x - pair * a.groups;
+  const int n = over(pair, a.m_octiles), ot = pair - n * a.oc_tiles;
+  const int tile0 = group * a.per_group, tiles = min(a.per_group, a.tiles - tile0);
 
   // ---- the first weights, then the input: [row][column][channel] ----
   const int first_tile = over(wave, a.m_parts), part = wave - first_tile * a.parts;
@@ -71,11 +78,14 @@ __global__ void __launch_bounds__(kMaxWaves * 64) ConvPoolKernel(PoolConvArgs a)
   const v4i q = a.rq[oc];
   const int bias = a.biasf[oc];
   {
+    // the rows behind the workgroup's tiles
+    const int top = 2 * a.sh * over(8 * tile0, a.m_pw) - a.pad_t, bottom = 2 * a.sh * over(min(8 * (tile0 + tiles), a.pooled) - 1, a.m_pw) - a.pad_t + a.tile_rows;
     const int plane = a.H * a.W, units = a.H * a.col_quads * a.chan_quads;
     const uint8_t* const xn = a.x + static_cast<size_t>(n) * a.C * plane;
     for (int u = tid; u < units; u += threads) {
       const int c4 = over(u, a.m_units), at = u - c4 * (a.H * a.col_quads);
       const int r = over(at, a.m_cols), x = min((at - r * a.col_quads) * 4, a.W - 4);  // (the last four columns of a row may overlap the ones before)
+      if (r < top || r >= bottom) continue;
       uint32_t d[4], px[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) __builtin_memcpy(&d[j], xn + static_cast<uint32_t>(min(4 * c4 + j, a.C - 1) * plane + r * a.W + x), 4);
@@ -88,7 +98,7 @@ __global__ void __launch_bounds__(kMaxWaves * 64) ConvPoolKernel(PoolConvArgs a)
     }
   }
   const PoolConvArgs& b = LateArgs<PoolConvArgs>();
-  const int parts = b.parts, steps = b.steps, tiles = b.tiles;
+  const int parts = b.parts, steps = b.steps;
   if (b.padded) {  // (uniform) the cells around the image
     const int quads = b.chan_quads, cells = b.halo_rows * b.halo_cols;
     for (int u = tid; u < cells; u += threads) {
@@ -114,7 +124,7 @@ __global__ void __launch_bounds__(kMaxWaves * 64) ConvPoolKernel(PoolConvArgs a)
     int v[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = max(max(acc[i], acc[4 + i]), max(acc[8 + i], acc[12 + i])) + bias;
-    const int p = tile * 8 + 4 * half, live = pooled - p;
+    const int p = (tile0 + tile) * 8 + 4 * half, live = pooled - p;
     if (oc >= b.OC || live <= 0) return;
     const uint32_t codes = b.generic ? RequantPack4<kRqGeneric>(v, q, b.out_zp, b.lo, b.hi)
                                      : RequantCodes4<false>(v, q, RoundHigh(q[2]), b.pre, b.lo, b.hi) ^ static_cast<uint32_t>(b.out_xor4);
@@ -128,7 +138,7 @@ __global__ void __launch_bounds__(kMaxWaves * 64) ConvPoolKernel(PoolConvArgs a)
     }
   };
   for (int tile = first_tile; tile < tiles; tile += parts > 1 ? tiles : waves) {  // (a split reduction: one tile a wavefront)
-    const int slot = min(tile * 32 + 4 * (col & 7) + (col >> 3), 4 * pooled - 1);
+    const int slot = min((tile0 + tile) * 32 + 4 * (col & 7) + (col >> 3), 4 * pooled - 1);
     const int qh = over(slot >> 2, b.m_pw), oh = 2 * qh + (slot >> 1 & 1), ow = 2 * ((slot >> 2) - qh * b.pw) + (slot & 1);
     const int8_t* const window = lds + oh * b.sh * b.row_stride + ow * b.sw * b.pix_stride + 16 * half;
     // the step k0 stands at: channels, column and row of its tap
@@ -232,8 +242,8 @@ int ConvPoolSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   a.padded = a.halo_rows != a.H || a.halo_cols != a.W;
   const auto reciprocal = [](uint64_t v) { return v > 1 ? static_cast<uint32_t>(((1ull << 32) + v - 1) / v) : 0u; };
   a.oc_tiles = (a.OC + 31) / 32;
-  const uint64_t wgs = static_cast<uint64_t>(d->batch) * a.oc_tiles;
-  if (wgs * a.oc_tiles >= (1ull << 32)) return TVX_E_UNSUPPORTED;
+  const uint64_t pairs = static_cast<uint64_t>(d->batch) * a.oc_tiles;  // of an image and 32 channels
+  if (pairs * a.oc_tiles >= (1ull << 32)) return TVX_E_UNSUPPORTED;
   a.m_octiles = reciprocal(a.oc_tiles);
   a.chan_quads = (a.C + 3) / 4; a.col_quads = (a.W + 3) / 4;
   const uint64_t row_units = static_cast<uint64_t>(a.H) * a.col_quads;
@@ -252,21 +262,53 @@ int ConvPoolSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   a.m_pw = reciprocal(a.pw);
   if (static_cast<uint64_t>(a.pooled) * a.pw >= (1ull << 32)) return TVX_E_UNSUPPORTED;
   a.tiles = (4 * a.pooled + 31) / 32;
+  a.tile_rows = a.sh + (static_cast<int>(d->k_h) - 1) * static_cast<int>(d->dilation_h) + 1;
+  // While there are CUs without one, more workgroups share an image: a wavefront's chain is then shorter. Microseconds, from 3254 launches on
+  // 865 drawn layers: per reduction step of a wavefront, per pass over the input's units and per unit loaded. int8, 5 x 5, 32 x 32, before
+  // this kernel, with a workgroup an image and here: 3 to 16, batch 2 6.6, 18.9 and 7.3; 16 to 64, batch 31 10.2, 20.4 and 12.4. Of those layers
+  // 24 are slower than the implicit GEMM's by more than 3 %, 163 with a workgroup an image; the mean is 0.57 of its time (0.71). What is left are
+  // long chains on about as many workgroups as CUs (12 to 21, 32 x 32, batch 150: 11.4 and 19.6), among which more gain, up to six times.
+  a.per_group = a.tiles; a.groups = 1;
+  {
+    const int cus = ComputeUnits();
+    double least = 0;
+    for (int groups = 1; groups <= a.tiles && (groups == 1 || pairs * groups <= static_cast<uint64_t>(cus)); ++groups) {
+      const int per_group = (a.tiles + groups - 1) / groups;
+      if (groups > 1 && per_group == (a.tiles + groups - 2) / (groups - 1)) continue;
+      const int share = pairs * groups <= static_cast<uint64_t>(cus) ? kMaxWaves : kMaxWaves / 2;
+      const int parts = std::max(1, std::min(share / per_group, a.steps)), waves = parts > 1 ? parts * per_group : std::min(kMaxWaves, per_group);
+      const double chain = static_cast<double>((a.steps + parts - 1) / parts) * (parts > 1 ? 1 : (per_group + waves - 1) / waves);
+      const double units = static_cast<double>(row_units) * a.chan_quads / (64 * waves);
+      const double loaded = std::min(1.0, (2.0 * a.sh * (8 * per_group / a.pw + 2) + a.tile_rows) / a.H);
+      const double cost = 4.0 + 0.13 * chain + 0.2 * std::ceil(units) + 0.14 * units * loaded;
+      if (groups > 1 && cost >= least) continue;
+      least = groups > 1 ? cost : 0.95 * cost;
+      a.per_group = per_group;
+      a.groups = (a.tiles + per_group - 1) / per_group;
+    }
+  }
+  if (const char* f = getenv("TVX_CONV_POOL_GROUPS")) {  // test lever
+    a.per_group = (a.tiles + std::max(1, atoi(f)) - 1) / std::max(1, atoi(f));
+    a.groups = (a.tiles + a.per_group - 1) / a.per_group;
+  }
+  const uint64_t wgs = pairs * a.groups;
+  if (wgs * a.groups >= (1ull << 32)) return TVX_E_UNSUPPORTED;  // (exact reciprocals)
+  a.m_groups = reciprocal(a.groups);
   // few tiles: the reduction is split, so that eight wavefronts share the chain, four where a CU gets more than one workgroup
   // (the layer above: batch 1 6.3 us with one part, 5.3 with two, 4.8 with four; batch 207 8.3, 6.7, 8.4)
   const int share = wgs <= static_cast<uint64_t>(ComputeUnits()) ? kMaxWaves : kMaxWaves / 2;
-  a.parts = std::max(1, std::min(share / a.tiles, a.steps));
-  if (const char* f = getenv("TVX_CONV_POOL_PARTS")) a.parts = std::max(1, std::min(std::min(atoi(f), kMaxWaves / a.tiles), a.steps));  // test lever
+  a.parts = std::max(1, std::min(share / a.per_group, a.steps));
+  if (const char* f = getenv("TVX_CONV_POOL_PARTS")) a.parts = std::max(1, std::min(std::min(atoi(f), kMaxWaves / a.per_group), a.steps));  // test lever
   a.per_part = (a.steps + a.parts - 1) / a.parts;
   a.parts = (a.steps + a.per_part - 1) / a.per_part;
   a.m_parts = reciprocal(a.parts);
-  const int waves = a.parts > 1 ? a.parts * a.tiles : std::min(kMaxWaves, a.tiles);
+  const int waves = a.parts > 1 ? a.parts * a.per_group : std::min(kMaxWaves, a.per_group);
   if (!LaunchFits(wgs, 64 * waves)) return TVX_E_UNSUPPORTED;
   a.z4 = static_cast<int>(static_cast<uint32_t>((zws == -128 ? 64 : -zws) & 0xff) * 0x01010101u);
   a.ztwice = zws == -128;
   a.last_channels = a.C - (a.per_tap - 1) * 32;
   a.off_red = (static_cast<int>(image) + 15) / 16 * 16;
-  const int lds_bytes = a.off_red + (a.parts > 1 ? a.tiles * 4096 : 0);
+  const int lds_bytes = a.off_red + (a.parts > 1 ? a.per_group * 4096 : 0);
   // ---- weights in fragment order, constants folded into the bias ----
   const int alloc = a.oc_tiles * 32;
   std::vector<int8_t> packed(static_cast<size_t>(a.oc_tiles) * a.steps * 1024, 0);
