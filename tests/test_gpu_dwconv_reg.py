@@ -1,4 +1,4 @@
-"""The depthwise register stencil (float16 and float32 3x3 / 5x5, int8 5x5; strides 1 and 2) at the edges of its column and row
+"""The depthwise register stencil (float16, float32 and int8 windows of 3x3 and 5x5; strides 1 and 2) at the edges of its column and row
 groups: planes narrower and lower than a group, ragged ends, padding on every side and on none, the tensor's first and last
 elements, planes that share wavefronts and planes that fill them, every row count."""
 import numpy as np

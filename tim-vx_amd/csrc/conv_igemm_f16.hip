@@ -261,10 +261,10 @@ int ConvIgemmF16Setup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, 
   // against 16.1) and many rows of at least 56 pixels under 3x3 taps and 32 to 64 channels with few results (batch 32, 56 x 56: 32 -> 16 10.6 against
   // 12.9, 64 -> 32 16.5 against 21.1, 64 -> 64 22.8 against 24.3; on the other side of that line 16 -> 16 at batch 64 13.6 against 12.9, 96 -> 16
   // 46.8 against 41.7, 64 -> 128 at batch 32 38.9 against 38.5, 64 -> 64 at batch 22 21.3 against 19.2, 64 -> 16 on 28 x 28, batch 96, 14.9 against 14.6).
-  const uint64_t pixels = static_cast<uint64_t>(d->batch) * d->out_w * d->out_h;
-  const bool few = d->k_w == 1 && d->k_h == 1 && d->in_c >= 48 && d->out_c <= 16 && pixels < 32768;
+  const uint64_t pixels = static_cast<uint64_t>(d->batch) * d->out_w * d->out_h, cu = ComputeUnits();  // (the lines were drawn on 256 of them)
+  const bool few = d->k_w == 1 && d->k_h == 1 && d->in_c >= 48 && d->out_c <= 16 && pixels < 128 * cu;
   const bool rows = d->k_w == 3 && d->k_h == 3 && d->stride_w == 1 && d->in_c >= 32 && d->in_c <= 64 && d->out_w >= 56 && d->out_c <= 64 &&
-                    pixels >= (d->out_c <= 32 ? 65536u : 98304u);
+                    pixels >= (d->out_c <= 32 ? 256 : 384) * cu;
   const char* const tiles = getenv("TVX_CONV_TILE");  // (its lever 0 leaves the tiles' layers to the kernels before them)
   if (!few && !rows && !(tiles && atoi(tiles) == 0)) return TVX_E_UNSUPPORTED;
   Plan plan{};

@@ -1,9 +1,9 @@
 // Depthwise convolution (multiplier 1) as a register stencil on planes of any width: float16 and float32 windows of 3x3 and
-// 5x5, int8 / uint8 windows of 5x5 (and of 3x3 on rows that are not whole dwords), at stride 1 or 2 (vxConvolutionLayer's depthwise form; reference:
-// src/tim/vx/internal/src/ops/vsi_nn_op_conv2d.c:35-118).
+// 5x5, int8 / uint8 windows of 5x5 and, where BetterAt3x3 finds this ahead, of 3x3, at stride 1 or 2 (vxConvolutionLayer's depthwise form;
+// reference: src/tim/vx/internal/src/ops/vsi_nn_op_conv2d.c:35-118).
 //
-// A thread computes one, two or four output rows x four or eight neighbouring outputs of one plane from rows held in registers
-// (plane_rows.h).
+// A thread computes one, two or four output rows x eight neighbouring outputs (four of float32, and at stride 2) of one plane from rows held in
+// registers (plane_rows.h).
 // A plane's channel is uniform where its threads fill whole wavefronts (weights then are scalar operands); small planes share
 // wavefronts and keep their weights in vector registers.
 //
@@ -266,12 +266,13 @@ int DwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   if (d->in_c > 60000) return TVX_E_UNSUPPORTED;
 
   // Output rows of a thread: four in registers read a row 1.5 times (3x3) or twice (5x5, stride 1) instead of three or five times, but are a
-  // long chain for few wavefronts. One up to 300000 threads (16 channels of 23 x 25, 3x3: 2.8 us, 3.5 with two, 4.4 with four; 20 x 24 of 48 x
-  // 32 in float32 3.4, 3.9, 4.6), two up to 1.2 million (60 K planes of 7 x 7: 6.4, 6.0, 6.2), four from there on (5 x 288 of 125 x 125 23.1,
+  // long chain for few wavefronts. One up to 300000 threads, 1172 a CU (16 channels of 23 x 25, 3x3: 2.8 us, 3.5 with two, 4.4 with four; 20 x 24 of 48 x
+  // 32 in float32 3.4, 3.9, 4.6), two up to four times as many (60 K planes of 7 x 7: 6.4, 6.0, 6.2), four from there on (5 x 288 of 125 x 125 23.1,
   // 19.3, 17.9; 5x5 on 37 x 341 of 34 x 34 32.6, 29.3, 25.6).
   const int px = S == 1 && dt != TVX_F32 ? 8 : 4;
   const uint64_t row_threads = planes * ((d->out_w + px - 1) / px) * d->out_h;
-  int R = row_threads < 300000 ? 1 : row_threads < 1200000 ? 2 : 4;
+  const uint64_t few = 1172ull * ComputeUnits();
+  int R = row_threads < few ? 1 : row_threads < 4 * few ? 2 : 4;
   if (const char* f = getenv("TVX_DWCONV_REG_ROWS")) R = atoi(f) == 4 ? 4 : atoi(f) == 2 ? 2 : 1;  // test lever
   if (!PlanPlaneRows(&a, planes, d->in_h, d->in_w, d->out_h, d->out_w, d->pad_top, d->pad_left, px, R)) return TVX_E_UNSUPPORTED;
   if (a.total < 12) return TVX_E_UNSUPPORTED;  // (a run of at most twelve elements fits the tensor)

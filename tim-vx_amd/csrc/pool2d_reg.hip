@@ -166,7 +166,7 @@ __global__ void __launch_bounds__(256) PoolRegI8Kernel(PoolRegArgs a) {
         int c;
         if constexpr (SAME) {
           const int u = 2 * sum[r][p] + __mul24(513, div);
-          // (u + .5, at most 50000, lies half a step or more from a multiple of 2 div, and the factor is good to 2^-21)
+          // (u + .5, at most 50128, lies half a step or more from a multiple of 2 div, and the factor is good to 2^-21)
           int w = static_cast<int>((static_cast<float>(u) + .5f) * (rx[p] * ry[r]));
           if (u == 2 * __mul24(w, div)) w -= w & 1;
           c = Med3(w - 256 + a.out_zp, 0, 255);
@@ -329,7 +329,7 @@ int PoolRegPlan(tvx_op* op, unsigned align_in, unsigned align_out, const char* n
   // Output rows of a thread: one - four in registers read a row 1.5 times instead of three times, but are a long chain for few wavefronts (int8
   // average 3x3 on 480 channels of 15 x 15: 2.6 against 4.9 us) - until there are two wavefronts a SIMD at four (336 of 32 x 32, batch 18: 6.8
   // against 5.2), and at stride 2, where rows are read 1.5 times at the most, always.
-  int rows = S == 1 && planes * ((d.out_w + px - 1) / px) * ((d.out_h + 3) / 4) >= 131072 ? 4 : 1;
+  int rows = S == 1 && planes * ((d.out_w + px - 1) / px) * ((d.out_h + 3) / 4) >= 512ull * ComputeUnits() ? 4 : 1;
   if (const char* f = getenv("TVX_POOL_REG_ROWS")) rows = S == 1 && atoi(f) == 4 ? 4 : 1;  // test lever
   Plan plan{};
   PoolRegArgs& a = plan.a;
