@@ -59,6 +59,24 @@ def test_which_kernel_takes_a_quantized_3x3_layer(oracle, c, h, w, stride, kerne
         assert np.array_equal(got, oracle.conv2d(x, wt, b, act=2, **kws))
 
 
+@pytest.mark.parametrize("room,kernel", [(9 * 128 * 128, "dwconv3x3_i8"), (9 * 128 * 128 - 1, "dwconv_rows_i8")])
+@pytest.mark.parametrize("sign", [1, -1])
+def test_depthwise_biases_at_the_ends_of_their_range(oracle, sign, room, kernel):
+    """The sums of the register stencil saturate: a bias that leaves them no room goes to the kernel whose sums wrap around."""
+    n, c, h, w = 2, 6, 16, 16
+    rng = np.random.default_rng(7600)
+    x, wt = rng.integers(-128, 128, n * c * h * w).astype(np.int8), rng.integers(-128, 128, c * 9).astype(np.int8)
+    b = rng.integers(-4096, 4097, c).astype(np.int32)
+    b[1] = sign * (2 ** 31 - 1 - room)
+    scales = np.full(c, 0.02, np.float32)
+    kws = dict(in_shape=[w, h, c, n], w_shape=[3, 3, 1, c], out_shape=[w, h, c, n], stride=[1, 1], dilation=[1, 1], pad_left=1, pad_top=1, multiplier=1,
+               in_dtype=1, w_dtype=1, out_dtype=1, in_q=(0.05, 0), w_q=(1.0, 0, scales), out_q=(0.6, 3))
+    want = oracle.conv2d(x, wt, b, act=0, **kws)
+    assert (want.reshape(n, c, -1)[:, 1] == (127 if sign > 0 else -128)).all() and len(np.unique(want)) > 100
+    got = TC.gpu_conv2d(x, wt, b, act=0, want_variant=kernel, **kws)
+    assert np.array_equal(got, want), int((got != want).sum())
+
+
 @pytest.mark.parametrize("dtype,w,h", [(0, 40, 70), (1, 61, 46), (2, 60, 76), (3, 42, 42)])
 def test_averages_of_many_planes_by_wavefronts(oracle, dtype, w, h):
     """Up to eight planes a compute unit, a workgroup each; of more, planes just below their type's line take a wavefront, those beyond a workgroup."""
