@@ -911,19 +911,20 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
     uint8_t* tile = packed.data() + slot / 32 * tile_bytes + (slot % 32) * 16;
     const uint8_t* ws = src + static_cast<size_t>(oc) * a.icg * taps * E;
     int64_t sw = 0;
-    for (int c = 0; c < a.icg; ++c) {
-      const int gg = c / epg, chunk = gg / a.gpc, gr = gg % a.gpc;
-      uint8_t* cp = tile + static_cast<size_t>(chunk) * a.steps * 1024 + (c % epg) * E;
-      for (int t = 0; t < taps; ++t, ws += E) {
-        const int q = t * a.gpc + gr;
-        uint8_t* to = cp + static_cast<size_t>(q >> 1) * 1024 + (q & 1) * 512;
-        if (E == 1) {
-          const uint8_t v = *ws ^ flip;
-          *to = v;
+    // (copies: a byte stored may be any of the fields')
+    const int icg = a.icg, gpc = a.gpc;
+    const size_t chunk_bytes = static_cast<size_t>(a.steps) * 1024;
+    for (int c = 0; c < icg; ++c) {
+      const int gg = c / epg, chunk = gg / gpc, gr = gg % gpc;
+      uint8_t* cp = tile + static_cast<size_t>(chunk) * chunk_bytes + (c % epg) * E;
+      if (E == 1) {
+        for (int t = 0, q = gr; t < taps; ++t, q += gpc) {
+          const uint8_t v = *ws++ ^ flip;
+          cp[static_cast<size_t>(q >> 1) * 1024 + (q & 1) * 512] = v;
           sw += static_cast<int8_t>(v);
-        } else {
-          std::memcpy(to, ws, E);
         }
+      } else {
+        for (int t = 0, q = gr; t < taps; ++t, q += gpc, ws += E) std::memcpy(cp + static_cast<size_t>(q >> 1) * 1024 + (q & 1) * 512, ws, E);
       }
     }
     if (dt == kI8) {
