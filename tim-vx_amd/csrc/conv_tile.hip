@@ -56,8 +56,8 @@ struct TileArgs {
   int icg;                 // input channels of a group
   int gpc;                 // granules of a pixel per chunk
   int items;               // work items of a chunk
-  int gl, cells, ncg, IH;  // granules neighbouring lanes take (a divisor of gpc); column groups of all staged rows, of a row; staged rows per image
-  uint32_t m_gl, m_cells, m_ncg, m_ih;
+  int gl, cells, cells4, ncg, IH;  // granules neighbouring lanes take (a divisor of gpc); column groups of all staged rows, fours of them, groups of a row; staged rows per image
+  uint32_t m_gl, m_cells4, m_ncg, m_ih;
   int row_step, H, W, batch;  // row_step: input rows between staged rows
   int at_max;              // last place of a plane where a work item's pixels can be read
   uint32_t plane_bytes, image_bytes;
@@ -114,6 +114,16 @@ __device__ __forceinline__ void Multiply(typename Kind<DT>::acc& acc, const v4i&
   }
 }
 
+// N bytes at a scalar base and a lane's offset. The base is made anew for every load (sixteen of them kept over a loop are spilled, a lane
+// address for each is three instructions) and named global memory: behind the empty assembly the compiler knows no address space and takes
+// flat loads, which wait for LDS as well.
+typedef const __attribute__((address_space(1))) uint8_t* GlobalBytes;
+template <int N>
+__device__ __forceinline__ void Fetch(uint32_t* d, const uint8_t*& base, uint32_t at) {
+  asm volatile("" : "+s"(base));
+  __builtin_memcpy(d, (const void*)((GlobalBytes)base + at), N);
+}
+
 // One work item on its way: P consecutive pixels of a row x one granule of channel planes.
 template <int DT> struct Item {
   static constexpr int E = Kind<DT>::E;
@@ -125,12 +135,12 @@ template <int DT> struct Item {
   // FULL: all planes exist; else planes past the last valid one re-read it (masked behind Unit)
   template <bool FULL>
   __device__ __forceinline__ void Load(const uint8_t* base, uint32_t at, uint32_t plane_bytes, int valid) {
+    const uint8_t* plane = base;
 #pragma unroll
     for (int c = 0; c < N; ++c) {
       if (FULL) {
-        const uint8_t* plane = base + static_cast<size_t>(c) * plane_bytes;
-        asm("" : "+s"(plane));  // (a scalar base and one lane offset for all planes, not sixteen lane addresses)
-        __builtin_memcpy(&d[c * D], plane + at, 4 * D);
+        Fetch<4 * D>(&d[c * D], plane, at);
+        plane += plane_bytes;
       } else {
         __builtin_memcpy(&d[c * D], base + (at + static_cast<uint32_t>(min(c, valid - 1)) * plane_bytes), 4 * D);
       }
@@ -138,12 +148,12 @@ template <int DT> struct Item {
   }
   // a granule that holds all the channels there are (uniform): the planes behind them are not loaded but zero
   __device__ __forceinline__ void LoadFew(const uint8_t* base, uint32_t at, uint32_t plane_bytes, int valid) {
+    const uint8_t* plane = base;
 #pragma unroll
     for (int c = 0; c < N; ++c) {
       if (c < valid) {
-        const uint8_t* plane = base + static_cast<size_t>(c) * plane_bytes;
-        asm("" : "+s"(plane));
-        __builtin_memcpy(&d[c * D], plane + at, 4 * D);
+        Fetch<4 * D>(&d[c * D], plane, at);
+        plane += plane_bytes;
       } else {
 #pragma unroll
         for (int i = 0; i < D; ++i) d[c * D + i] = 0;
@@ -212,20 +222,22 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
   acc_t acc[MT][NT];
   v4i fw[R][NT];
 
-  // A work item's place: an item = (granule, column group, row); lanes take gl granules, then the cells of a plane (contiguous in
-  // memory where the rows are whole), then the next gl granules.
+  // A work item's place: an item = (granule, column group, row); lanes take four cells of a plane (contiguous in memory where the rows are
+  // whole), then these of gl granules, then the next four cells, then the next gl granules. Four neighbouring lanes are what the L1 looks up
+  // at once: with the granules innermost each of the four was a line of its own, and a wavefront's load took 64 clocks of the L1 instead of
+  // 16 (int8 3x3 272 -> 64 on 55 x 70, batch 13: 25.0 -> 22.9 us); with cells alone innermost the LDS stores, 128 bytes apart, meet in two banks.
   struct Where { uint32_t at; int to, col, valid; bool inside; };
   auto find = [&](const TileArgs& a, int it, int c0) {
     Where w;
     const bool live = it < a.items;
-    const int itc = live ? it : 0;
-    const int rest = DivM(itc, a.m_gl), gl = itc - __mul24(rest, a.gl);
-    const int gh = DivM(rest, a.m_cells), cell = rest - __mul24(gh, a.cells);
+    const int itc = live ? it : 0, four = itc >> 2;
+    const int rest = DivM(four, a.m_gl), gl = four - __mul24(rest, a.gl);
+    const int gh = DivM(rest, a.m_cells4), cell = (rest - __mul24(gh, a.cells4)) * 4 + (itc & 3);
     const int gr = __mul24(gh, a.gl) + gl;
     const int r = DivM(cell, a.m_ncg), cg = cell - __mul24(r, a.ncg);
     const int g = DivM(r, a.m_ih), ry = r - __mul24(g, a.IH);
     const int iy = iy0 + __mul24(ry, a.row_step), ixs = ix0 + P * cg;
-    w.inside = live && static_cast<unsigned>(iy) < static_cast<unsigned>(a.H) && ixs > -P && ixs < a.W && n0 + g < a.batch;
+    w.inside = live && cell < a.cells && static_cast<unsigned>(iy) < static_cast<unsigned>(a.H) && ixs > -P && ixs < a.W && n0 + g < a.batch;
     w.valid = min(a.icg - c0 - gr * (16 / E), 16 / E);  // channels of the granule
     // P pixels from the group's first column inside the image, further in front at the plane's end: what lies outside
     // the row is not stored, what the neighbouring group stores too is the same
@@ -845,7 +857,8 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   a.total = static_cast<int>(g.wgs);
   a.per_xcd = (a.total + 7) / 8;
   a.npx = g.G * g.IH * g.IW;
-  a.items = a.cells * a.gpc;
+  a.cells4 = (a.cells + 3) / 4;
+  a.items = a.cells4 * 4 * a.gpc;
   a.plane_bytes = static_cast<uint32_t>(H) * W * E;
   a.image_bytes = a.plane_bytes * C;
   a.at_max = H * W - group_px;
@@ -864,7 +877,7 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   const int wide_groups = (a.run_px + 16 / E - 1) / (16 / E);
   a.m_run_wide = Magic(wide_groups);
   while ((1 << a.wide_shift) < a.runs * wide_groups) ++a.wide_shift;
-  a.m_gl = Magic(a.gl); a.m_cells = Magic(a.cells); a.m_ncg = Magic(a.ncg); a.m_ih = Magic(a.IH); a.m_iw = Magic(a.IW); a.m_tw = Magic(a.TW); a.m_thtw = Magic(a.TH * a.TW);
+  a.m_gl = Magic(a.gl); a.m_cells4 = Magic(a.cells4); a.m_ncg = Magic(a.ncg); a.m_ih = Magic(a.IH); a.m_iw = Magic(a.IW); a.m_tw = Magic(a.TW); a.m_thtw = Magic(a.TH * a.TW);
   a.m_ocb = Magic(a.oc_wgs); a.m_tpg = Magic(a.wgs_per_group); a.m_tx = Magic(a.tiles_x); a.m_ty = Magic(a.tiles_y);
   if (static_cast<int64_t>(a.IH - 1) * a.row_step >= 1 << 23) return TVX_E_UNSUPPORTED;  // (24-bit products of rows and columns; the others lie within LDS)
   // a reciprocal is exact while dividend * divisor < 2^32
