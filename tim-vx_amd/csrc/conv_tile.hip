@@ -43,6 +43,7 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 constexpr int kI8 = 0, kF16 = 1, kF32 = 2;  // element kinds (uint8 runs as int8 with its sign bit flipped)
+constexpr int kMostAhead = 8;  // steps whose weights are on their way to a wavefront at a time, at most (R)
 
 // In the order of their use: what comes before a launch's first loads is fetched together (LateArgs).
 struct TileArgs {
@@ -66,7 +67,7 @@ struct TileArgs {
   // ---- under the first loads
   const v4i* wpk;          // [group][32-channel tile][chunk][step][64 lanes]: sixteen bytes of reduction per lane
   const int* tab;          // [half][steps_pad]: LDS byte offset of the granule a lane of that half multiplies at a step
-  int steps, steps_pad, odd;  // reduction steps of a chunk; the last step's upper half is empty
+  int steps, steps_pad, odd;  // reduction steps of a chunk, and padded for what is read ahead; the last step's upper half is empty
   int chunks, tiles_per_group;
   int row_stride, NQ, npx;  // staged rows between output rows; pixels of the tile; staged pixels
   uint32_t m_iw, m_tw, m_thtw;
@@ -194,7 +195,7 @@ template <int DT> struct Item {
 template <int DT, int WM, int WN, int KS, int MT, int NT, int R, int EU, bool MULTI>
 __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(EU))) ConvTileKernel(TileArgs a) {
   constexpr int kThreads = 64 * WM * WN * KS;
-  static_assert(R % 2 == 0, "the activations' two buffers alternate with the steps");
+  static_assert(R % 2 == 0 && R <= kMostAhead, "the activations' two buffers alternate with the steps");
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   using acc_t = typename Kind<DT>::acc;
   using elem_t = typename Kind<DT>::elem;
@@ -383,40 +384,53 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
         for (int t = 0; t < NT; ++t)
 #pragma unroll
           for (int i = 0; i < 16; ++i) acc[m][t][i] = 0;
-    // ---- multiply: R steps' weights ahead, two steps' activations ahead ----
-    const int* tab = reinterpret_cast<const int*>(lds + b.off_tab) + half * b.steps_pad;
+    // ---- multiply: R steps' weights ahead, two steps' activations, R steps' offsets of those. The order inside a step is kept by hand: left
+    // to itself the compiler put an offset and the activations behind it in front of the multiplication that waits for them ----
+    const int* tab = reinterpret_cast<const int*>(lds + b.off_tab) + half * b.steps_pad + s0;
     v4i fx[2][MT];
-    auto fetch_x = [&](int s, v4i (&f)[MT]) {
-      const int off = tab[s];  // (the table is padded)
+    int off[R];
+    auto fetch_x = [&](int o, v4i (&f)[MT]) {
 #pragma unroll
-      for (int m = 0; m < MT; ++m) f[m] = *reinterpret_cast<const v4i*>(lds + base[m] + off);
+      for (int m = 0; m < MT; ++m) f[m] = *reinterpret_cast<const v4i*>(lds + base[m] + o);
     };
-    auto multiply = [&](int s, bool last, v4i (&f)[MT], const v4i (&w)[NT]) {
-      if (DT != kI8 && last && b.odd && s == b.steps - 1 && half)  // (zero weights, but the data may be an infinity)
-#pragma unroll
-        for (int m = 0; m < MT; ++m) f[m] = v4i{0, 0, 0, 0};
+    auto multiply = [&](const v4i (&f)[MT], const v4i (&w)[NT]) {
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int t = 0; t < NT; ++t) Multiply<DT>(acc[m][t], f[m], w[t]);
     };
-    fetch_x(s0, fx[0]);
-    fetch_x(s0 + 1, fx[1]);
+    const v4i* wp = w.wp + static_cast<uint32_t>(chunk * b.steps + s0) * 64;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) fetch_x(tab[u], fx[u]);
+#pragma unroll
+    for (int u = 0; u < R; ++u) off[u] = tab[2 + u];  // (the table is padded)
     int s = s0;
 #pragma unroll 1
     for (; s + R < s1; s += R) {
+      wp += R * 64;
+      tab += R;
 #pragma unroll
       for (int u = 0; u < R; ++u) {
-        multiply(s + u, false, fx[u & 1], fw[u]);  // (a chunk's last step is below)
-        fetch_w(w, chunk * b.steps, s + u + R, fw[u]);
-        fetch_x(s + u + 2, fx[u & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(fx[u & 1], fw[u]);  // (a chunk's last step is below)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) fw[u][t] = wp[t * w.tile_stride + u * 64];  // (past the share's end: not multiplied; the array is padded)
+        fetch_x(off[u], fx[u & 1]);
+        if (u & 1) {
+          off[u - 1] = tab[2 + u - 1];
+          off[u] = tab[2 + u];
+        }
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int u = 0; u < R; ++u)
       if (s + u < s1) {  // uniform
-        multiply(s + u, true, fx[u & 1], fw[u]);
-        fetch_x(s + u + 2, fx[u & 1]);
+        if (DT != kI8 && b.odd && s + u == b.steps - 1 && half)  // (zero weights, but the data may be an infinity)
+#pragma unroll
+          for (int m = 0; m < MT; ++m) fx[u & 1][m] = v4i{0, 0, 0, 0};
+        multiply(fx[u & 1], fw[u]);
+        fetch_x(off[u], fx[u & 1]);
       }
     if (MULTI && pass + 1 < passes) continue;
     if (!MULTI && pass + 1 < passes) {  // the next block's first weights travel under the results
@@ -817,7 +831,7 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
         g.pitch = (g.gpc | 1) * 16;
         const int steps = (taps * g.gpc + 1) / 2;
         int64_t bytes = WindowBytes(sp, npx * g.pitch, E, loop);
-        bytes += 2 * RoundUp(steps + 12, 4) * 4;
+        bytes += 2 * RoundUp(steps + kMostAhead + 4, 4) * 4;
         if (zws) bytes += npx * 4 + sp.pixels * 4;
         if (loop > 1) bytes = RoundUp(bytes, 16) + OutBytes(sp, E);
         g.lds_bytes = static_cast<int>(std::min<int64_t>(bytes, 1 << 30));
@@ -841,7 +855,7 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   a.IW = g.IW; a.IH = g.IH; a.pitch = g.pitch; a.gpc = g.gpc; a.chunks = g.chunks;
   a.steps = (taps * g.gpc + 1) / 2;
   a.odd = (taps * g.gpc) & 1;
-  a.steps_pad = RoundUp(a.steps + 12, 4);
+  a.steps_pad = RoundUp(a.steps + kMostAhead + 4, 4);
   a.taps_w = kw; a.taps_h = kh; a.dil_col = dw; a.dil_row = dh * g.IW;
   a.ncg = (g.IW + group_px - 1) / group_px;
   a.cells = g.G * g.IH * a.ncg;
@@ -906,7 +920,7 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   // ---- weights [oc][c][ky][kx] -> fragment order; the bias takes the zero points' constants ----
   const size_t alloc_oc = static_cast<size_t>(a.tiles_per_group) * groups * sp.channels;
   const size_t tile_bytes = static_cast<size_t>(a.chunks) * a.steps * 1024;
-  std::vector<uint8_t> packed(alloc_oc / 32 * tile_bytes, 0);
+  std::vector<uint8_t> packed(alloc_oc / 32 * tile_bytes + kMostAhead * 1024, 0);  // (the last steps read ahead)
   std::vector<int32_t> biasf(dt == kI8 ? alloc_oc : 0, 0);
   std::vector<int32_t> mult, shift;
   if (dt == kI8) {
