@@ -16,8 +16,9 @@
 // Where several blocks of output channels follow from one window and there are workgroups enough without them, a workgroup takes
 // them one after the other over the window it has staged: 8 -> 240 channels 3x3 on 157 x 157, batch 11, 69 -> 49 us; 80 -> 352 on
 // 66 x 66, batch 23, 76 -> 62.
-// Quantized tensors under a weight zero point need the sum of every window: channel sums per staged pixel, box-filtered
-// once per tile - nothing in the inner loop.
+// Quantized tensors under a weight zero point need the sum of every window. Where a wavefront has few steps a lane adds up the bytes of the
+// fragments it multiplies, four dot products each (kSumsInLoop), and the lanes, halves and shares of a pixel meet in LDS; where it has many
+// the staged pixels' channels are summed once and box-filtered per tile (kSumsBox), nothing in the loop.
 //
 // What bounds it: at the sizes convolutional networks have, a launch is a chain of one memory round trip, the LDS
 // transposition (about 70 vector instructions per 64 staged bytes for int8, none for float32) and the steps themselves, and no unit
@@ -43,6 +44,7 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 constexpr int kI8 = 0, kF16 = 1, kF32 = 2;  // element kinds (uint8 runs as int8 with its sign bit flipped)
+constexpr int kNoSums = 0, kSumsInLoop = 1, kSumsBox = 2;
 constexpr int kMostAhead = 8;  // steps whose weights are on their way to a wavefront at a time, at most (R)
 
 // In the order of their use: what comes before a launch's first loads is fetched together (LateArgs).
@@ -192,7 +194,7 @@ template <int DT> struct Item {
 
 // WM x WN wavefronts share the tile's pixels and channels (MT x NT MFMA tiles each), KS wavefronts a tile's reduction.
 // R: steps whose weights are on their way to a wavefront at a time.
-template <int DT, int WM, int WN, int KS, int MT, int NT, int R, int EU, bool MULTI>
+template <int DT, int SUMS, int WM, int WN, int KS, int MT, int NT, int R, int EU, bool MULTI>
 __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(EU))) ConvTileKernel(TileArgs a) {
   constexpr int kThreads = 64 * WM * WN * KS;
   static_assert(R % 2 == 0 && R <= kMostAhead, "the activations' two buffers alternate with the steps");
@@ -221,6 +223,7 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
   const int ks = wave % KS, wn = wave / KS % WN, wm = wave / KS / WN;
   uint32_t base[MT];  // LDS byte offset of this lane's pixel in each pixel tile
   acc_t acc[MT][NT];
+  int xs[MT];  // kSumsInLoop: sums of the bytes multiplied
   v4i fw[R][NT];
 
   // A work item's place: an item = (granule, column group, row); lanes take four cells of a plane (contiguous in memory where the rows are
@@ -304,10 +307,12 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
     const TileArgs& b = late();
     const int tab_n = 2 * b.steps_pad;
     const int tab_first = b.tab[min(tid, tab_n - 1)];
-    const Steps w = share(b);
+    if (!MULTI) {
+      const Steps w = share(b);
 #pragma unroll
-    for (int u = 0; u < R; ++u) fetch_w(w, chunk * b.steps, w.s0 + u, fw[u]);
-    __builtin_amdgcn_sched_barrier(0);
+      for (int u = 0; u < R; ++u) fetch_w(w, 0, w.s0 + u, fw[u]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     if (chunk == 0) {
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
@@ -339,6 +344,7 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
       int* tab = reinterpret_cast<int*>(lds + b.off_tab);
       if (tid < tab_n) tab[tid] = tab_first;
       for (int i = tid + kThreads; i < tab_n; i += kThreads) tab[i] = b.tab[i];
+      if (SUMS == kSumsInLoop && tid < WM * MT * 32) reinterpret_cast<int*>(lds + b.off_zt)[tid] = 0;
     }
     store(b, item, where, all_full);
 #pragma unroll 1
@@ -347,9 +353,14 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
       load(b, xg, all_full, item, where);
       store(b, item, where, all_full);
     }
+    if (MULTI) {  // (beside accumulators, an item's planes and its results the weights would need more registers than two workgroups a CU leave)
+      const Steps w = share(b);
+#pragma unroll
+      for (int u = 0; u < R; ++u) fetch_w(w, chunk * b.steps, w.s0 + u, fw[u]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     __syncthreads();
-    // ---- channel sums of the staged pixels ----
-    if (DT == kI8 && b.zws) {  // uniform
+    if (SUMS == kSumsBox) {  // channel sums of the staged pixels
       int* sum = reinterpret_cast<int*>(lds + b.off_sum);
       for (int p = tid; p < b.npx; p += kThreads) {
         int v = chunk ? sum[p] : 0;
@@ -379,11 +390,13 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
     const int s0 = w.s0, s1 = w.s1;
     if (!MULTI || chunk == 0)
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
+      for (int m = 0; m < MT; ++m) {
+        xs[m] = 0;
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
           for (int i = 0; i < 16; ++i) acc[m][t][i] = 0;
+      }
     // ---- multiply: R steps' weights ahead, two steps' activations, R steps' offsets of those. The order inside a step is kept by hand: left
     // to itself the compiler put an offset and the activations behind it in front of the multiplication that waits for them ----
     const int* tab = reinterpret_cast<const int*>(lds + b.off_tab) + half * b.steps_pad + s0;
@@ -398,6 +411,11 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
       for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int t = 0; t < NT; ++t) Multiply<DT>(acc[m][t], f[m], w[t]);
+      if (SUMS == kSumsInLoop)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) xs[m] = __builtin_amdgcn_sdot4(f[m][q], 0x01010101, xs[m], false);
     };
     const v4i* wp = w.wp + static_cast<uint32_t>(chunk * b.steps + s0) * 64;
 #pragma unroll
@@ -426,7 +444,7 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
 #pragma unroll
     for (int u = 0; u < R; ++u)
       if (s + u < s1) {  // uniform
-        if (DT != kI8 && b.odd && s + u == b.steps - 1 && half)  // (zero weights, but the data may be an infinity)
+        if ((DT != kI8 || SUMS == kSumsInLoop) && b.odd && s + u == b.steps - 1 && half)  // (zero weights, but the data may be an infinity, or is summed up)
 #pragma unroll
           for (int m = 0; m < MT; ++m) fx[u & 1][m] = v4i{0, 0, 0, 0};
         multiply(fx[u & 1], fw[u]);
@@ -460,22 +478,26 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
   // that become eight consecutive pixels, or single quads), every wavefront finishes its own ----
   constexpr int kQuads = KS == 1 ? 4 : (2 * MT * NT >= KS ? 2 : 1);  // quads of a piece
   constexpr int kPieces = 4 / kQuads;
-  const bool box = DT == kI8 && c.zws && (MULTI || pass == 0);  // the window sums are to be made
+  if (SUMS == kSumsInLoop && (MULTI || pass == 0) && wn == 0) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) atomicAdd(reinterpret_cast<int*>(lds + c.off_zt) + (wm * MT + m) * 32 + row, -c.zws * xs[m]);
+  }
+  const bool box = SUMS == kSumsBox && (MULTI || pass == 0);  // the window sums are to be made
   if (KS > 1 || box) {
     __syncthreads();
-    elem_t* part = reinterpret_cast<elem_t*>(lds);  // [wave][tile][element][lane]
+    v4i* part = reinterpret_cast<v4i*>(lds);  // [wave][tile][quad][lane]
     if (KS > 1)
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int piece = (m * NT + t) * kPieces + (i / 4) % kPieces;
-            if (piece % KS != ks) part[((wave * MT + m) * NT + t) * 1024 + i * 64 + lane] = acc[m][t][i];
-          }
-    // window sums: the box filter over the channel sums
-    if (box) {
+          for (int k = 0; k < 4; ++k)
+            if (((m * NT + t) * kPieces + k % kPieces) % KS != ks) {
+              const elem_t q[4] = {acc[m][t][4 * k], acc[m][t][4 * k + 1], acc[m][t][4 * k + 2], acc[m][t][4 * k + 3]};
+              part[((wave * MT + m) * NT + t) * 256 + k * 64 + lane] = __builtin_bit_cast(v4i, q);
+            }
+    if (box) {  // the box filter over the channel sums
       const int* sum = reinterpret_cast<const int*>(lds + c.off_sum);
       int* zt = reinterpret_cast<int*>(lds + c.off_zt);
       for (int q = tid; q < c.NQ; q += kThreads) {
@@ -499,17 +521,21 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
             if (((m * NT + t) * kPieces + p) % KS == ks)
 #pragma unroll
               for (int k = 1; k < KS; ++k) {
-                const elem_t* from = part + (((wave - ks + (ks + k) % KS) * MT + m) * NT + t) * 1024 + lane;
+                const v4i* from = part + (((wave - ks + (ks + k) % KS) * MT + m) * NT + t) * 256 + lane;
 #pragma unroll
-                for (int i = 0; i < 16; ++i)
-                  if ((i / 4) % kPieces == p) acc[m][t][i] += from[i * 64];
+                for (int i = p; i < 4; i += kPieces) {
+                  struct Quad { elem_t e[4]; };
+                  const Quad q = __builtin_bit_cast(Quad, from[i * 64]);
+#pragma unroll
+                  for (int e = 0; e < 4; ++e) acc[m][t][4 * i + e] += q.e[e];
+                }
               }
   }
 
   // ---- epilogue: a lane holds output channel `row` of each channel tile and, per accumulator quad k, pixels
   // 8 k + 4 half + 0 .. 3 of a pixel tile. The results meet in LDS as [channel][pixel] and leave from there in runs: a tile of
   // whole rows is one run of a channel's plane (per image), else every row is one ----
-  if (KS > 1 || !box) __syncthreads();  // the window, the partial sums or the block before are read
+  if (KS > 1 || !box) __syncthreads();  // the window, the partial sums or the block before are read, the window sums complete
 #pragma unroll
   for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -523,7 +549,7 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
           int v[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = acc[m][t][4 * k + e] + bias[t];
-          if (c.zws) {
+          if (SUMS) {
             const v4i z = *reinterpret_cast<const v4i*>(lds + c.off_zt + q0 * 4);
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] += z[e];
@@ -624,11 +650,13 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
 typedef void (*TileFn)(TileArgs);
 
 // The ways a workgroup's wavefronts share a tile.
-struct Shape { int pixels, channels, ks, waves; double length; TileFn fn[3][2]; };  // length: of its chain, fitted (Cost)
-#define TVX_TILE_DT(DT, WM, WN, KS, MT, NT, R, EU) { ConvTileKernel<DT, WM, WN, KS, MT, NT, R, EU, false>, ConvTileKernel<DT, WM, WN, KS, MT, NT, R, 2, true> }
+// fn: int8, float16, float32, int8 with sums in the loop and with sums box-filtered; one chunk of the channels or several
+struct Shape { int pixels, channels, ks, waves; double length; TileFn fn[5][2]; };  // length: of its chain, fitted (Cost)
+#define TVX_TILE_DT(DT, SUMS, WM, WN, KS, MT, NT, R, EU) { ConvTileKernel<DT, SUMS, WM, WN, KS, MT, NT, R, EU, false>, ConvTileKernel<DT, SUMS, WM, WN, KS, MT, NT, R, EU, true> }
 #define TVX_TILE(WM, WN, KS, MT, NT, R, EU, LENGTH)                                                               \
-  { WM * MT * 32, WN * NT * 32, KS, WM * WN * KS, LENGTH, { TVX_TILE_DT(kI8, WM, WN, KS, MT, NT, R, EU), TVX_TILE_DT(kF16, WM, WN, KS, MT, NT, R, EU), \
-                                                    TVX_TILE_DT(kF32, WM, WN, KS, MT, NT, R, EU) } }
+  { WM * MT * 32, WN * NT * 32, KS, WM * WN * KS, LENGTH, { TVX_TILE_DT(kI8, kNoSums, WM, WN, KS, MT, NT, R, EU), TVX_TILE_DT(kF16, kNoSums, WM, WN, KS, MT, NT, R, EU), \
+                                                    TVX_TILE_DT(kF32, kNoSums, WM, WN, KS, MT, NT, R, EU), TVX_TILE_DT(kI8, kSumsInLoop, WM, WN, KS, MT, NT, R, EU), \
+                                                    TVX_TILE_DT(kI8, (MT * NT > 1 ? kSumsBox : kSumsInLoop), WM, WN, KS, MT, NT, R, EU) } }
 const Shape kShapes[] = {
     TVX_TILE(4, 2, 1, 2, 1, 4, 4, 1.0),   // 0: 256 x 64, eight wavefronts
     TVX_TILE(2, 2, 2, 2, 1, 4, 4, 1.27),  // 1: 128 x 64, eight
@@ -657,7 +685,7 @@ int64_t WindowBytes(const Shape& sp, int64_t staged, int E, int loop) {
 
 struct Geometry {
   int shape, TW, TH, G, gpc, chunks, loop;
-  int IW, IH, pitch, lds_bytes;
+  int IW, IH, pitch, lds_bytes, sums;
   int64_t wgs;
   double cost;
 };
@@ -688,6 +716,14 @@ double Cost(const Shape& sp, const Geometry& g, int dt, int taps, int group_px, 
   const double alone = sp.ks == 1 && sp.waves == 8 && waves_cu == 12 ? 1.12 : 1.0;
   const double by_chain = chain * sp.length * alone * (1.0 + 0.48 * (resident - 1.0) * sp.waves / 8);
   return 3.1 + by_chain * (per_cu <= resident ? 1.0 : per_cu / resident + 0.35) + per_cu * shared;
+}
+
+// How the window sums are made: in the loop up to 80 multiplications of a wavefront, and always where each of them waits for a weight
+// fragment of its own (316 drawn layers, captured: 0.92 of the box filter's time below the line, as low as 0.69; beyond it the dot
+// products cost the matrix cores' issue slots, 1.03 on the average and up to 1.17).
+int SumsBy(const Shape& sp, int steps) {
+  const int tiles = sp.pixels * sp.channels / 1024 * sp.ks / sp.waves;
+  return tiles == 1 || steps * tiles / sp.ks <= 80 ? kSumsInLoop : kSumsBox;
 }
 
 struct Plan {
@@ -832,7 +868,8 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
         const int steps = (taps * g.gpc + 1) / 2;
         int64_t bytes = WindowBytes(sp, npx * g.pitch, E, loop);
         bytes += 2 * RoundUp(steps + kMostAhead + 4, 4) * 4;
-        if (zws) bytes += npx * 4 + sp.pixels * 4;
+        g.sums = zws ? SumsBy(sp, steps * g.chunks * loop) : kNoSums;
+        if (zws) bytes += sp.pixels * 4 + (g.sums == kSumsBox ? npx * 4 : 0);
         if (loop > 1) bytes = RoundUp(bytes, 16) + OutBytes(sp, E);
         g.lds_bytes = static_cast<int>(std::min<int64_t>(bytes, 1 << 30));
         if (g.lds_bytes <= 78 * 1024) break;
@@ -879,7 +916,7 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   const int64_t npx = static_cast<int64_t>(g.G) * g.IH * g.IW;
   a.off_tab = static_cast<int>(WindowBytes(sp, npx * g.pitch, E, g.loop));
   a.off_sum = a.off_tab + 2 * a.steps_pad * 4;
-  a.off_zt = a.off_sum + (zws ? static_cast<int>(npx) * 4 : 0);
+  a.off_zt = a.off_sum + (g.sums == kSumsBox ? static_cast<int>(npx) * 4 : 0);
   a.off_out = g.loop > 1 ? g.lds_bytes - static_cast<int>(OutBytes(sp, E)) : 0;
   const bool whole = g.TW == OW;
   a.runs = whole ? g.G : g.TH;
@@ -985,7 +1022,7 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
 
   Plan plan{};
   plan.a = a;
-  plan.fn = sp.fn[dt][a.chunks > 1];
+  plan.fn = sp.fn[g.sums == kNoSums ? dt : g.sums == kSumsInLoop ? 3 : 4][a.chunks > 1];
   plan.lds_bytes = static_cast<unsigned>(g.lds_bytes);
   plan.grid = static_cast<unsigned>(a.per_xcd) * 8;
   plan.threads = 64u * sp.waves;
