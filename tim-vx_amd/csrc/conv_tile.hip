@@ -291,7 +291,10 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
     for (int t = 0; t < NT; ++t) f[t] = w.wp[t * w.tile_stride + at];
   };
   // ---- stage a chunk's window. `a`: what the first loads need; `late()`: the rest ----
+  // (lanes without an item stay out: reading some valid address instead kept the L1 busy as long as an item does, 0.97 of the time without on 400
+  // drawn layers, int8 32 -> 16, 5x5 on 65 x 65, batch 24, 12.3 -> 9.8 us)
   auto load = [&](const TileArgs& a, const uint8_t* xg, bool all_full, item_t& item, const Where& w) {
+    if (!w.inside) return;
     if (all_full) item.template Load<true>(xg, w.at, a.plane_bytes, 16 / E);
     else if (a.icg < 16 / E) item.LoadFew(xg, w.at, a.plane_bytes, a.icg);
     else item.template Load<false>(xg, w.at, a.plane_bytes, max(w.valid, 1));
