@@ -39,6 +39,25 @@ def test_transpose_forms(oracle, in_dims, perm, form, dt):
         assert (y[:off * e] == 0xA5).all() and (y[(off + n) * e:] == 0xA5).all(), off
 
 
+# up to eight channels sorted in registers: around a thread's pixels (8 bytes, 4 halves, 2 words), a workgroup's, and with two batch dimensions; more
+# through LDS in blocks or one by one: around a workgroup's pixels and a block's
+FEW = [((a, b, 3), (1, 0, 2), "interleaved") for a in range(2, 9) for b in (2, 7, 8, 9, 511, 2051)] + \
+      [((a, 11, 3, 2), (1, 0, 3, 2), "interleaved") for a in (2, 3, 8, 12)] + [((3, 2048, 2), (1, 0, 2), "interleaved")] + \
+      [((a, b, 2), (1, 0, 2), "interleaved") for a in (9, 10, 12, 16) for b in (2, 3, 255, 509, 681, 683)]
+
+
+@pytest.mark.parametrize("dt", [np.uint8, np.float16, np.int32])
+@pytest.mark.parametrize("in_dims,perm,form", FEW)
+def test_transpose_of_few_channels(oracle, in_dims, perm, form, dt):
+    test_transpose_forms(oracle, in_dims, perm, form, dt)
+
+
+@pytest.mark.parametrize("channels,dt", [(20, np.uint8), (32, np.uint8), (60, np.uint8), (64, np.uint8), (20, np.float16), (32, np.float16), (18, np.float16)])
+@pytest.mark.parametrize("pixels", [3, 126, 128, 129, 410])
+def test_transpose_of_wide_pixels(oracle, pixels, channels, dt):
+    test_transpose_forms(oracle, (channels, pixels, 3), (1, 0, 2), "interleaved", dt)
+
+
 @pytest.mark.parametrize("out_dt", [0, 1, 2, 3])
 @pytest.mark.parametrize("in_dt", [0, 1, 2, 3])
 @pytest.mark.parametrize("count", [1, 3, 4, 1021, 4099])

@@ -4,11 +4,14 @@
 // The permutation is reduced first: dimensions of one element go, input dimensions that stay neighbours become one. What is
 // left either keeps its fastest dimension (rows move whole: a gather of the widest units the rows, their strides and the
 // pointers allow) or is a batch of matrices whose rows become columns, read along one and written along the other through LDS:
-//  - the layout change of images: a few interleaved channels to planes. A run of pixels is one contiguous piece of the
-//    input, read in 16-byte units; a thread picks one channel of four neighbouring bytes' worth of pixels out of LDS.
+//  - the layout change of images: a few interleaved channels to planes. A run of pixels is one contiguous piece of the input. Up to eight
+//    channels: a thread reads its pixels as they lie and sorts them in registers. More, up to 64 bytes a pixel: the run goes through LDS, from
+//    where a thread takes blocks of channels and pixels that it sorts (multiples of four channels of up to two bytes) or single elements.
 //  - anything else: tiles of 64 x 64 elements, 4 bytes per thread on either side.
 // 32 x 224 x 224 x 3 bytes (9.6 MB read + written) 19.1 -> 4.1 us, 27 x 91 x 91 x 134 bytes (60 MB) 134 -> 26 us against one thread
-// per element with 64-bit divisions; the first is bound by the launch, the second by rows that cross cache lines.
+// per element with 64-bit divisions; the second is bound by rows that cross cache lines. The first spent its time on a byte a lane out of LDS:
+// captured 3.6 us, 2.7 in registers (an empty launch: 2.0), 64 x 61 x 61 x 3 2.9 -> 2.1, 8 x 113 x 113 x 8 3.8 -> 2.3, halves 32 x 224 x 224 x 3 5.5
+// -> 4.2. Wide pixels met in a bank of LDS: 4 x 224 x 224 x 32 bytes 16.6 -> 3.9, 8 x 113 x 113 x 12 3.8 -> 3.0, halves x 16 4.2 -> 3.8.
 #include <algorithm>
 #include <cstring>
 
@@ -21,6 +24,7 @@ constexpr int kThreads = 256;
 constexpr int kMaxDims = 6;
 constexpr int kChunkBytes = 8192;   // interleaved form: input bytes of a workgroup
 constexpr int kTile = 64;
+constexpr int kOwn = 2, kMostOwn = 8;  // interleaved form in registers: dwords of a channel a thread moves, most channels
 
 // Everything a kernel is given stays under 112 bytes: from there on a launch took the host 3.6 us instead of 2.8.
 struct MatrixArgs {
@@ -31,6 +35,7 @@ struct MatrixArgs {
   uint32_t tiles_a, tiles_b, m_tiles_a, m_tiles_b;
   uint32_t chunk;           // interleaved form: pixels of a workgroup (a multiple of 4)
   uint32_t m_groups;        // ... reciprocal of chunk / V
+  uint32_t m_quads;         // ... of A / 4
 };
 struct Batch {  // the dimensions beside the matrix's two; the first of up to three has its own extent in the grid only
   uint32_t in_stride[3], out_stride[3];  // elements
@@ -112,6 +117,96 @@ __global__ void __launch_bounds__(kThreads) InterleavedKernel(MatrixArgs a, BATC
   }
 }
 
+// ... of a multiple of four channels of one or two bytes: a thread sorts V channels of V pixels, read as dwords, in registers. The run lies in LDS
+// with a dword behind every V pixels, a stride of A + 1 dwords: neighbouring lanes, V pixels apart, would meet in a bank otherwise. (Elements of
+// four bytes, with nothing to sort, are 5 % slower for the padding at 12 channels and as much faster at 16: they stay with the kernel above.)
+template <typename T, typename BATCH>
+__global__ void __launch_bounds__(kThreads) InterleavedBlockKernel(MatrixArgs a, BATCH batch) {
+  __shared__ uint32_t lds[kChunkBytes / 4 + kChunkBytes / 32];
+  constexpr uint32_t V = 4 / sizeof(T);
+  static_assert(V > 1);
+  const uint32_t bt = DivM(blockIdx.x, a.m_tiles_b), tb = blockIdx.x - bt * a.tiles_b;
+  uint32_t in_off, out_off;
+  BatchOffsets(batch, bt, &in_off, &out_off);
+  const uint32_t b0 = tb * a.chunk, n = min(a.chunk, a.B - b0);
+  const uint32_t bytes = n * a.A * sizeof(T);
+  const uint8_t* src = a.x + static_cast<uint64_t>(in_off + b0 * a.A) * sizeof(T);
+  for (uint32_t i = threadIdx.x * 16; i < bytes; i += kThreads * 16) {
+    uint32_t v[4] = {0, 0, 0, 0};
+    if (i + 16 <= bytes) __builtin_memcpy(v, src + i, 16);
+    else  // (whole dwords: four channels)
+      for (uint32_t j = 0; j < 3; ++j)
+        if (i + 4 * j < bytes) __builtin_memcpy(&v[j], src + i + 4 * j, 4);
+    uint32_t* to = lds + i / 4 + DivM(i / 16, a.m_quads);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) to[j] = v[j];
+  }
+  __syncthreads();
+  T* y = reinterpret_cast<T*>(a.y) + out_off + b0;
+  const uint32_t groups = a.chunk / V;
+  for (uint32_t i = threadIdx.x; i < groups * (a.A / V); i += kThreads) {
+    const uint32_t c = DivM(i, a.m_groups), g = i - c * groups, p = g * V;
+    if (p >= n) continue;
+    uint32_t w[V], o[V];
+#pragma unroll
+    for (uint32_t k = 0; k < V; ++k) w[k] = lds[g * (a.A + 1) + k * (a.A / V) + c];  // (past the run's end: inside the array, not stored)
+    if constexpr (V == 4) {
+      Transpose4x4(w, o);
+    } else {
+      o[0] = __builtin_amdgcn_perm(w[1], w[0], 0x05040100);
+      o[1] = __builtin_amdgcn_perm(w[1], w[0], 0x07060302);
+    }
+    T* to = y + c * V * a.out_a + p;
+#pragma unroll
+    for (uint32_t k = 0; k < V; ++k) {
+      T* at = to + k * a.out_a;
+      if (p + V <= n) {
+        __builtin_memcpy(at, &o[k], 4);
+      } else {
+#pragma unroll 1
+        for (uint32_t e = 0; p + e < n; ++e) at[e] = static_cast<T>(o[k] >> (8 * sizeof(T) * e & 31));
+      }
+    }
+  }
+}
+
+// Two to eight channels interleaved: a thread takes V * G neighbouring pixels, A * G dwords as they lie, and puts the channels' elements together
+// with byte permutes. The last threads of a matrix begin at B - V * G and move some pixels a second time. Two dwords of a channel a thread:
+// one and four are level for bytes, one is 5 % behind for halves.
+template <typename T, int A, typename BATCH>
+__global__ void __launch_bounds__(kThreads) InterleavedRegKernel(MatrixArgs a, BATCH batch) {
+  constexpr int V = 4 / sizeof(T), G = kOwn;
+  const uint32_t bt = DivM(blockIdx.x, a.m_tiles_b), tb = blockIdx.x - bt * a.tiles_b;
+  uint32_t in_off, out_off;
+  BatchOffsets(batch, bt, &in_off, &out_off);
+  uint32_t p = (tb * kThreads + threadIdx.x) * (V * G);
+  if (p >= a.B) return;
+  p = min(p, a.B - V * G);
+  uint32_t d[A * G];
+  __builtin_memcpy(d, a.x + static_cast<uint64_t>(in_off + p * A) * sizeof(T), sizeof(d));
+  T* y = reinterpret_cast<T*>(a.y) + out_off + p;
+#pragma unroll
+  for (int c = 0; c < A; ++c) {
+    uint32_t o[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      [[maybe_unused]] const uint32_t* w = d + g * A;
+      if constexpr (sizeof(T) == 1) {
+        const auto pair = [&](int e) {  // elements e and e + 1 of the channel as the low half of a dword
+          const int i = e * A + c, j = i + A;
+          return __builtin_amdgcn_perm(w[j / 4], w[i / 4], 0x0c0c0400u + (static_cast<uint32_t>(j % 4) << 8) + i % 4);
+        };
+        o[g] = __builtin_amdgcn_perm(pair(2), pair(0), 0x05040100);
+      } else if constexpr (sizeof(T) == 2) {
+        o[g] = __builtin_amdgcn_perm(w[(c + A) / 2], w[c / 2], ((c + A) % 2 ? 0x07060000u : 0x05040000u) + (c % 2 ? 0x0302u : 0x0100u));
+      } else {
+        o[g] = w[c];
+      }
+    }
+    __builtin_memcpy(y + c * a.out_a, o, sizeof(o));
+  }
+}
+
 // 64 x 64 tiles of a matrix with rows of A elements in_b apart.
 template <typename T, typename BATCH>
 __global__ void __launch_bounds__(kThreads) TileKernel(MatrixArgs a, BATCH batch) {
@@ -181,7 +276,7 @@ __global__ void __launch_bounds__(kThreads) GatherLargeKernel(GatherLargeArgs a)
   reinterpret_cast<T*>(a.y)[i] = reinterpret_cast<const T*>(a.x)[in];
 }
 
-enum Form { kGather, kGatherLarge, kInterleaved, kTiles };
+enum Form { kGather, kGatherLarge, kInterleaved, kInterleavedBlock, kInterleavedReg, kTiles };
 struct Plan {
   Form form;
   MatrixArgs m;
@@ -217,11 +312,33 @@ void LaunchGather(const Plan& p, uint32_t elem, const void* in0, void* out, hipS
   }
 }
 
+template <typename T, int A>
+void LaunchInterleavedReg(const Plan& p, const MatrixArgs& a, hipStream_t st) {
+  const dim3 grid(p.grid), block(kThreads);
+  if (p.batched) hipLaunchKernelGGL((InterleavedRegKernel<T, A, Batch>), grid, block, 0, st, a, p.batch);
+  else hipLaunchKernelGGL((InterleavedRegKernel<T, A, NoBatch>), grid, block, 0, st, a, NoBatch{p.batch.in_stride[0], p.batch.out_stride[0]});
+}
+
 template <typename T>
 void LaunchMatrix(const Plan& p, const MatrixArgs& a, hipStream_t st) {
   const dim3 grid(p.grid), block(kThreads);
   const NoBatch one{p.batch.in_stride[0], p.batch.out_stride[0]};
-  if (p.form == kInterleaved) {
+  if (p.form == kInterleavedReg) {
+    switch (a.A) {
+      case 2: LaunchInterleavedReg<T, 2>(p, a, st); break;
+      case 3: LaunchInterleavedReg<T, 3>(p, a, st); break;
+      case 4: LaunchInterleavedReg<T, 4>(p, a, st); break;
+      case 5: LaunchInterleavedReg<T, 5>(p, a, st); break;
+      case 6: LaunchInterleavedReg<T, 6>(p, a, st); break;
+      case 7: LaunchInterleavedReg<T, 7>(p, a, st); break;
+      default: LaunchInterleavedReg<T, kMostOwn>(p, a, st);
+    }
+  } else if (p.form == kInterleavedBlock) {
+    if constexpr (sizeof(T) <= 2) {
+      if (p.batched) hipLaunchKernelGGL((InterleavedBlockKernel<T, Batch>), grid, block, 0, st, a, p.batch);
+      else hipLaunchKernelGGL((InterleavedBlockKernel<T, NoBatch>), grid, block, 0, st, a, one);
+    }
+  } else if (p.form == kInterleaved) {
     if (p.batched) hipLaunchKernelGGL((InterleavedKernel<T, Batch>), grid, block, 0, st, a, p.batch);
     else hipLaunchKernelGGL((InterleavedKernel<T, NoBatch>), grid, block, 0, st, a, one);
   } else {
@@ -336,8 +453,15 @@ int TransposeSetup(tvx_op* op) {
     if (others.size() == 2) plan.batch.dims[1] = 1;
     const uint64_t pixel = static_cast<uint64_t>(a.A) * d.elem_bytes;
     uint64_t grid;
-    if (a.in_b == a.A && pixel <= 64) {
-      plan.form = kInterleaved;
+    const uint32_t own = 4 / d.elem_bytes * kOwn;  // pixels of a thread, where they stay in registers
+    if (a.in_b == a.A && a.A <= kMostOwn && a.B >= own) {
+      plan.form = kInterleavedReg;
+      a.tiles_b = (a.B + kThreads * own - 1) / (kThreads * own);
+      a.m_tiles_b = Magic(a.tiles_b);
+      grid = batches * a.tiles_b;
+    } else if (a.in_b == a.A && pixel <= 64) {
+      plan.form = a.A % 4 || d.elem_bytes > 2 ? kInterleaved : kInterleavedBlock;
+      a.m_quads = Magic(a.A / 4);
       a.chunk = static_cast<uint32_t>(std::min<uint64_t>(kChunkBytes / pixel, 1024) & ~uint64_t{3});
       a.m_groups = Magic(a.chunk * d.elem_bytes / 4);
       a.tiles_b = (a.B + a.chunk - 1) / a.chunk;
@@ -367,7 +491,7 @@ int TransposeSetup(tvx_op* op) {
   }
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
   op->run = TransposeRun;
-  op->kernel_name = plan.form == kInterleaved ? "transpose_interleaved" : plan.form == kTiles ? "transpose_tiles" : "transpose_gather";
+  op->kernel_name = plan.form == kInterleaved || plan.form == kInterleavedBlock || plan.form == kInterleavedReg ? "transpose_interleaved" : plan.form == kTiles ? "transpose_tiles" : "transpose_gather";
   return TVX_OK;
 }
 
