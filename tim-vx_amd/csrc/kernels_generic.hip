@@ -1087,28 +1087,31 @@ __device__ __forceinline__ void ConvertFour(const float (&f)[4], const ConvertAr
   }
 }
 
-// One such unit a thread: two, four and eight took 13 to 40 % longer (more wavefronts hide more than longer ones).
+// One such unit a thread (two and four are level, eight a fifth behind). The elements behind the last whole unit have code of their own: with
+// loads of both kinds in front of one conversion the compiler took the unit in four single loads, sixteen bytes apart between lanes, and float32 ->
+// uint8 over 32 x 224 x 224 x 3 elements 7.35 us captured for 5.8, -> float16 8.7 for 6.0.
 template <typename TI, typename TO>
 __global__ void __launch_bounds__(kBlock)
 ConvertKernel(ConvertArgs a, const TI* __restrict__ x, TO* __restrict__ y, uint64_t total) {
   const uint64_t at = (static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x) * 4;
   if (at >= total) return;
-  TI v[4];
-  TO o[4];
-  const int n = total - at < 4 ? static_cast<int>(total - at) : 4;
-  if (n == 4) __builtin_memcpy(v, x + at, 4 * sizeof(TI));
-  else
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = x[at + min(e, n - 1)];
   float f[4];
+  TO o[4];
+  if (total - at >= 4) {
+    TI v[4];
+    __builtin_memcpy(v, x + at, 4 * sizeof(TI));
 #pragma unroll
-  for (int e = 0; e < 4; ++e) f[e] = ConvertLoad(v[e], a);
-  ConvertFour<TO>(f, a, o);
-  if (n == 4) __builtin_memcpy(y + at, o, 4 * sizeof(TO));
-  else
-#pragma unroll
-    for (int e = 0; e < 3; ++e)  // (indexed at compile time: an indexed array would live in scratch, 15 us a launch)
-      if (e < n) y[at + e] = o[e];
+    for (int e = 0; e < 4; ++e) f[e] = ConvertLoad(v[e], a);
+    ConvertFour<TO>(f, a, o);
+    __builtin_memcpy(y + at, o, 4 * sizeof(TO));
+    return;
+  }
+#pragma unroll 1
+  for (uint64_t i = at; i < total; ++i) {
+    f[0] = f[1] = f[2] = f[3] = ConvertLoad(x[i], a);
+    ConvertFour<TO>(f, a, o);
+    y[i] = o[0];
+  }
 }
 
 template <typename TI, typename TO>
