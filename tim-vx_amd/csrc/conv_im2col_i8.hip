@@ -617,7 +617,7 @@ int RoundUp(int v, int m) { return (v + m - 1) / m * m; }
 
 // Claims dense quantized convolutions with constant weights whose whole window is at most 64
 // bytes and whose channel count the implicit-GEMM kernel would have to pad (C % 16 != 0).
-int ConvIm2colSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const void* bias_host) {
+static int Im2colSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const void* bias_host, bool rest) {
   if (!op->quantized || !w_host || d->multiplier != 0 || d->groups > 1) return TVX_E_UNSUPPORTED;
   const int taps = static_cast<int>(d->k_w * d->k_h);
   const uint64_t k_real = static_cast<uint64_t>(d->in_c) * taps;
@@ -638,6 +638,12 @@ int ConvIm2colSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, co
   if ((d->k_h - 1) * d->dilation_h > 31 || (d->k_w - 1) * d->dilation_w > 31) return TVX_E_UNSUPPORTED;  // window offsets index 32-bit masks
   const int reg = RegSetup(op, d, w_host, bias_host, zxs, zws);
   if (reg != TVX_E_UNSUPPORTED) return reg;
+  // What does not fit registers is asked for twice, in front of the tiles (conv_tile.hip) and behind them, which take what lies between a handful of
+  // pixels (windows of several taps: a few thousand) and eighty thousand: 0.64 of the time on 80 drawn layers (int8 12 -> 115, 1x1 / 2 on 13 x 13, batch 2, 11.9 -> 5.1 us; uint8 43 -> 80,
+  // 1x1 / 2 on 17 x 17, batch 10, 15.9 -> 5.5). With more pixels a pass of this kernel is the shorter one (8 -> 64, 1x1 / 2 on 126 x 160, batch 64,
+  // 16.6 against 26.8; 1 -> 80 on 79 x 153, batch 33, 13.0 against 15.9; 1 -> 128, 7x7 on 120 x 120, batch 30, 47.6 against 67.3).
+  const uint64_t pixels = static_cast<uint64_t>(d->batch) * d->out_h * d->out_w;
+  if (!rest && !op->fused_pool && pixels < 80000 && pixels > (taps == 1 ? 128u : 4096u)) return TVX_E_UNSUPPORTED;
   a.xor_mask = x_u8 ? 0x80 : 0;
   a.pad_fill = zxs & 0xff;
   a.zws = zws;
@@ -698,5 +704,8 @@ int ConvIm2colSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, co
   op->kernel_name = op->fused_pool ? "conv2d_im2col_maxpool_i8" : "conv2d_im2col_i8";
   return TVX_OK;
 }
+
+int ConvIm2colSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const void* bias_host) { return Im2colSetup(op, d, w_host, bias_host, false); }
+int ConvIm2colRestSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const void* bias_host) { return Im2colSetup(op, d, w_host, bias_host, true); }
 
 }  // namespace tvx

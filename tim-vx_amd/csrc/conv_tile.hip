@@ -755,41 +755,47 @@ int ConvTileRun(tvx_op* op, const void* in0, const void*, void* out, hipStream_t
 static bool IsBetterChoice(const tvx_conv2d_desc* d, int dt, bool sums) {
   const int groups = d->groups > 1 ? d->groups : 1, ocg = d->out_c / groups;
   const uint64_t reduction = static_cast<uint64_t>(d->in_c / groups) * d->k_w * d->k_h;
-  const uint64_t macs = reduction * d->out_c * d->out_w * d->out_h * d->batch;
+  const uint64_t outputs = static_cast<uint64_t>(d->out_c) * d->out_w * d->out_h * d->batch, macs = reduction * outputs;
   const bool pointwise = d->k_w == 1 && d->k_h == 1;
   // a group of three output channels and fewer fills less than a tenth of a tile's 32 channels: only where each has little to add up
   // (float16 432 -> 12 in four groups, 7x7 on 42 x 42, batch 28: 2495 us with one thread per output, 140 here)
   if (groups > 1 && ocg < 4 && reduction <= 128) return false;
-  // a handful of products per output: one thread per output is quicker than staging a window (4.3 against 5.7 us; int8 in groups, which
-  // has no other kernel for so few: 4 -> 64 in two, 1x1 on 25 x 25, 3.9 against 6.5, but 64 -> 240 in eight on 22 x 22 7.7 against 6.0)
-  if (dt != kI8 && reduction <= 9 && macs <= 4000000) return false;
+  // a handful of products per output: one thread per output is quicker than staging a window, up to so many outputs (float32 1 -> 304, 1x1 / 2 on
+  // 31 x 31, batch 2: 3.9 against 5.0 us; 1 -> 16 on 39 x 39, batch 41, however 14.2 against 5.9; on 60 drawn layers of a line at 4 M products
+  // .82 of the time)
+  if (dt != kI8 && groups == 1 && outputs <= (reduction == 1 ? 300000u : reduction <= 3 ? 200000u : reduction <= 9 && !pointwise ? 30000u : 0u)) return false;
+  // (in groups: 4.3 against 5.7; int8, which has no other kernel for so few: 4 -> 64 in two, 1x1 on 25 x 25, 3.9 against 6.5, but 64 -> 240 in
+  // eight on 22 x 22 7.7 against 6.0)
+  if (dt != kI8 && groups > 1 && reduction <= 9 && macs <= 4000000) return false;
   if (dt == kI8 && groups > 1 && reduction <= 8 && macs <= (reduction <= 4 ? 4000000 : 1000000)) return false;
   // int8 1 x 1 in groups that fill less than a tile's channels: conv2d_gemm_i8 (188 -> 60 in four groups on 108 x 108, batch 6: 9.9 against
   // 17.4 us, 240 -> 96 on 74 x 74, batch 49: 36.8 against 52.3); with more than 32 channels in a group the tiles (144 -> 128 in two on
   // 29889 pixels: 9.5 against 16.8)
   if (dt == kI8 && groups > 1 && pointwise && reduction >= 32 && reduction <= 128 && ocg >= 8 && ocg <= 32) return false;
-  // float16 1 x 1: conv2d_gemm_f16 gathers four pixels a load where planes are whole quads and has less to set up. Few channels (4.2
-  // against 6.9 us at 24 -> 16 on 50 x 50, batch 4; 7.4 against 9.5 at 40 -> 384 on 28 x 28, batch 12), few results (10.2 against 13.4 at
-  // 32 -> 8 on 105 x 105, batch 18). Its rows are cache lines where a plane is a multiple of sixteen pixels: there also few results of
-  // many pixels (22.0 against 28.6 at 480 -> 16 on 146 x 160, batch 4) and many pixels of deep inputs (38.5 against 53.7 at 240 -> 240 on
-  // 60 x 60, batch 19; 74.3 against 100.5 at 465 -> 224 on 44 x 44, batch 48); on other planes the tiles (117 against 61.5 at 496 -> 160 on
-  // 58 x 58, batch 22).
+  // float16 1 x 1: conv2d_gemm_f16 has less to set up, and gathers four pixels a load where planes are whole quads. Few channels and few results
+  // (16 -> 24 on 46 x 46: 4.6 against 5.1 us), in quads also many pixels (24 -> 56 on 44 x 44, batch 18, 5.6 against 6.4; with fewer the tiles: 48 -> 40
+  // on 14 x 14, batch 22, 7.7 against 5.2). Its rows are cache lines where a plane is a multiple of sixteen pixels: there also up to 64 channels and
+  // 50 M products (56 -> 48 on 20 x 20, batch 31, 5.1 against 5.5) and deep inputs to few results of many pixels (352 -> 32 on 156 x 156, batch 10, 48.4
+  // against 49.9; to more results the tiles: 400 -> 66 on 84 x 84, batch 5, 21.9 against 17.1). 69 drawn layers .93 of the time under lines by
+  // products alone, .90 with the better kernel for each.
   if (dt == kF16 && groups == 1 && pointwise && d->in_c >= 16) {
     const uint64_t plane = static_cast<uint64_t>(d->in_w) * d->in_h, pixels = plane * d->batch;
-    if (d->in_c <= 32 && (macs <= 20000000 || d->out_c <= 8)) return false;
-    if (d->stride_w == 1 && d->stride_h == 1) {
-      if (plane % 4 == 0 && d->in_c <= 64 && d->out_c <= 512 && macs <= 200000000) return false;
-      if (plane % 16 == 0 && ((d->out_c <= 16 && pixels >= 32768) || (d->in_c >= 144 && pixels >= 16384))) return false;
+    if (macs <= 4000000 && ((d->in_c <= 24 && d->out_c <= 24) || (d->in_c <= 32 && d->out_c <= 8))) return false;
+    if (d->stride_w == 1 && d->stride_h == 1 && plane % 4 == 0) {
+      if (d->in_c <= 32 && (macs <= 4000000 || d->out_c <= 24 || pixels >= 30000)) return false;
+      if (d->in_c <= 64 && ((d->out_c <= 24 && pixels >= 16384) || (plane % 16 == 0 && macs <= 50000000) || (d->out_c <= 512 && pixels <= 256))) return false;
+      if (plane % 16 == 0 && d->in_c >= 144 && d->out_c <= 64 && pixels >= 16384) return false;
     }
   }
   if (dt == kI8 && groups == 1) {
     if (ConvIgemmPersists(d)) return false;
-    // a granule of channels under weights with a zero point: conv2d_igemm_i8 takes the window sums from a second multiplication instead of a
-    // pass over the window, stages rows of whole dwords in one aligned pass, and its chain is short on planes of at most 16 x 16 (16 ->
-    // 16, 3x3 on 7 x 7, batch 20, 5.4 against 6.6 us; even on the average). With more work than this its tiles queue up
-    // (8 -> 416 on 40 x 40, batch 24, 43 against 28); without the sums, and from two granules on, the tiles are ahead by a sixth.
-    const bool aligned = d->stride_w == 1 && d->stride_h == 1 && d->in_w % 4 == 0 && macs <= 400000000;
-    if (sums && d->in_c <= 16 && reduction <= 512 && (aligned || (d->in_w * d->in_h <= 256 && macs <= 250000000))) return false;
+    // a granule of channels under weights with a zero point: up to two million products conv2d_igemm_i8, whose chain is short on small planes and on
+    // rows of whole dwords, is within a tenth of the tiles at 5 to 6 us; beyond them its tiles queue up (60 drawn layers .55 of its time, 16 -> 192
+    // on 140 x 140, batch 3, 129 us against 15.7). What conv2d_im2col_i8 has left (its short windows) it does not get.
+    const bool aligned = d->stride_w == 1 && d->stride_h == 1 && d->in_w % 4 == 0;
+    const bool short_window = reduction <= 64 && d->in_c % 16 != 0 && d->out_c <= 128;
+    if (sums && d->in_c <= 16 && reduction <= 512 && macs <= 2000000 && !short_window && (aligned || d->in_w * d->in_h <= 256)) return false;
+    if (short_window && static_cast<uint64_t>(d->batch) * d->out_h * d->out_w >= 80000) return false;  // (conv2d_im2col_i8, see there)
   }
   return true;
 }

@@ -36,6 +36,7 @@ int ConvTileSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 int ConvBandSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 // Dense quantized conv whose whole window (C * Kh * Kw) is at most 64 bytes: im2col rows in registers or LDS + MFMA.
 int ConvIm2colSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
+int ConvIm2colRestSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 
 // with a 2 x 2 MAX pooling behind it, planes that fit LDS (conv_pool_i8.hip)
 int ConvPoolSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
