@@ -1,0 +1,59 @@
+"""Float16 1x1 convolutions with their pixels in registers: ends of pixel groups, images, channel steps and output tiles, both ways of sharing a
+reduction, against the oracle and, where infinities are among the inputs, against each product by itself."""
+import numpy as np
+import pytest
+
+import tvx_case as TC
+from test_gpu_parity import conv_case
+
+pytestmark = pytest.mark.gpu
+
+# batch, channels, height, width, output channels
+LAYERS = [(1, 1, 2, 4, 1), (3, 8, 3, 3, 17), (2, 31, 5, 5, 16), (1, 32, 16, 8, 33), (5, 33, 7, 9, 40), (2, 64, 11, 13, 15), (1, 97, 9, 31, 65), (2, 128, 12, 12, 48),
+          (3, 40, 1, 41, 130), (2, 129, 6, 7, 20), (1, 200, 8, 8, 96), (2, 260, 5, 7, 31), (1, 515, 4, 5, 64), (2, 777, 3, 4, 18), (1, 1024, 3, 3, 16)]
+
+
+@pytest.mark.parametrize("act", [0, 1, 2])
+@pytest.mark.parametrize("ks", [1, 4])
+@pytest.mark.parametrize("layer", LAYERS)
+def test_pointwise_f16_in_registers(oracle, layer, ks, act, monkeypatch):
+    n, c, h, w, oc = layer
+    if ks == 1 and c > 128:
+        pytest.skip("a wavefront holds 128 channels")
+    rng = np.random.default_rng(8800 + c + oc)
+    x, wt, b, kws = conv_case(rng, mult=0, mode="f16", n=n, c=c, h=h, w=w, oc=oc, kh=1, kw=1, stride=[1, 1], dil=[1, 1], pad=[0] * 4)
+    monkeypatch.setenv("TVX_PWCONV_F16", str(ks))
+    want = oracle.conv2d(x, wt, b, act=act, **kws)
+    for waves in (1, 1 << 20):   # all output tiles after one another, each by itself
+        monkeypatch.setenv("TVX_PWCONV_F16_WAVES", str(waves))
+        got = TC.gpu_conv2d(x, wt, b, act=act, want_kernel="pwconv_reg_f16", **kws)
+        # a float32 sum's rounding (c 2^-24 of the products' magnitudes) far below that of the result, 2^-11
+        magnitude = np.abs(x.astype(np.float64)).max() * np.abs(wt.astype(np.float64)).max() * c
+        assert np.abs(got.astype(np.float64) - want.astype(np.float64)).max() <= 2.0 ** -10 * max(np.abs(want.astype(np.float64)).max(), 2.0 ** -14) + c * 2.0 ** -23 * magnitude
+
+
+@pytest.mark.parametrize("ks,c", [(1, 13), (1, 100), (4, 133)])
+def test_an_infinity_stays_with_its_pixel(ks, c, monkeypatch):
+    n, h, w, oc = 2, 5, 7, 20
+    rng = np.random.default_rng(8900 + c)
+    x, wt, b, kws = conv_case(rng, mult=0, mode="f16", n=n, c=c, h=h, w=w, oc=oc, kh=1, kw=1, stride=[1, 1], dil=[1, 1], pad=[0] * 4)
+    wt = np.abs(wt) + np.float16(0.125)
+    x = np.clip(x, -4, 4)
+    x.reshape(n, c, h * w)[1, c - 1, 3] = np.inf
+    x.reshape(n, c, h * w)[0, 0, h * w - 1] = -np.inf
+    monkeypatch.setenv("TVX_PWCONV_F16", str(ks))
+    got = TC.gpu_conv2d(x, wt, b, act=0, want_kernel="pwconv_reg_f16", **kws).reshape(n, oc, h * w)
+    odd = np.zeros((n, h * w), bool)
+    odd[1, 3] = odd[0, -1] = True
+    assert (got[1, :, 3] == np.inf).all() and (got[0, :, -1] == -np.inf).all()
+    assert np.isfinite(got.transpose(0, 2, 1)[~odd]).all()
+
+
+@pytest.mark.parametrize("n,c,h,w,oc,mine", [(1, 64, 1, 577, 17, True), (1, 64, 24, 24, 17, False), (4, 64, 16, 16, 16, False), (4, 65, 16, 16, 16, True), (3, 64, 15, 17, 16, True),
+                                               (4, 64, 16, 16, 17, True), (2, 300, 31, 37, 40, True), (1, 1025, 25, 25, 20, False)])
+def test_which_layers(oracle, n, c, h, w, oc, mine):
+    """More than 576 pixels; of whole cache lines to at most 16 results from at most 64 channels none; at most 1024 channels."""
+    x, wt, b, kws = conv_case(np.random.default_rng(8990), mult=0, mode="f16", n=n, c=c, h=h, w=w, oc=oc, kh=1, kw=1, stride=[1, 1], dil=[1, 1], pad=[0] * 4)
+    want = oracle.conv2d(x, wt, b, act=1, **kws)
+    got = TC.gpu_conv2d(x, wt, b, act=1, want_kernel="pwconv_reg_f16" if mine else ("conv2d_tile_f16", "conv2d_gemm_f16", "conv2d_igemm_f16"), **kws)
+    assert np.allclose(got.astype(np.float32), want.astype(np.float32), rtol=5e-3, atol=2e-2)

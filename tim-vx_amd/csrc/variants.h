@@ -45,6 +45,7 @@ int PwConvSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 
 // ... with a wavefront's pixels in registers (pwconv_reg_i8.hip)
 int PwRegSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
+int PwRegF16Setup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 
 // depthwise 3x3 stencil (dwconv3x3_i8.hip)
 int DwConv3x3Setup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
