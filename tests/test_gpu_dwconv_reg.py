@@ -77,3 +77,19 @@ def test_tensors_at_any_address(oracle, c, h, w, k, stride, mode, offset):
     want = oracle.conv2d(x, wt, b, act=2, **kws)
     got = TC.gpu_conv2d(x, wt, b, act=2, want_kernel="dwconv_planes_i8", want_variant="dwconv_reg_i8", misalign=offset, **kws)
     assert np.array_equal(got, want), int((got != want).sum())
+
+
+@pytest.mark.parametrize("zw", [0, 1, 64, 127, 129, 255])
+@pytest.mark.parametrize("k,stride", [(3, 1), (3, 2), (5, 1), (5, 2)])
+def test_weight_zero_points_over_their_range(oracle, k, stride, zw, monkeypatch):
+    """Every sign and size of the zero point, 0 too (128 in the signed domain, whose negative no byte holds), on codes at both ends."""
+    rng = np.random.default_rng(7400 + zw)
+    x, wt, b, kws = conv_case(rng, n=2, c=3, h=22, w=33, oc=0, kh=k, kw=k, stride=[stride, stride], dil=[1, 1], pad=[k // 2] * 4, mult=1, mode="u8")
+    x, wt = rng.choice([0, 255], x.shape).astype(np.uint8), rng.choice([0, 1, 254, 255], wt.shape).astype(np.uint8)
+    kws.update(w_q=(0.01, zw, None), out_q=(0.15 * k, 3))  # (two standard deviations of the sums fill the codes)
+    monkeypatch.setenv("TVX_DWCONV_REG", "1")
+    want = oracle.conv2d(x, wt, b, act=0, **kws)
+    for rows in ("1", "4"):
+        monkeypatch.setenv("TVX_DWCONV_REG_ROWS", rows)
+        got = TC.gpu_conv2d(x, wt, b, act=0, want_kernel=NAME["u8"], want_variant="dwconv_reg_i8", **kws)
+        assert np.array_equal(got, want), (rows, int((got != want).sum()))

@@ -29,7 +29,8 @@ struct DwrArgs : PlaneArgs {
   int C;
   uint32_t m_c;
   int act;
-  int zws, lo, hi, narrow, out_xor, pre_ties;
+  int nzws4, nzws1, sum_shift;  // minus the weights' zero point (its half, where that is 128) in the bytes of a row's two windows; twice the sum then
+  int lo, hi, narrow, out_xor, pre_ties;
 };
 
 // DT: TVX_I8 (uint8 too), TVX_F16 or TVX_F32
@@ -126,8 +127,12 @@ __device__ __forceinline__ int Cut(const uint32_t (&d)[N], int o) {
   return static_cast<int>(o % 4 ? __builtin_amdgcn_alignbyte(hi, lo, o % 4) : lo);
 }
 
-// Accumulators start from the folded bias. A row's window is two dot products (weights 0 .. 3, and the fifth alone); under a weight
-// zero point (SUMS) the rows' window sums are made once per input row and added to the output rows they belong to.
+// Accumulators start from the folded bias. A row's window is two dot products (weights 0 .. 3, and the fifth alone); under a weight zero point (SUMS)
+// the rows' window sums are made once per input row, times minus that (times minus its half, and doubled, where that is 128), and added up per
+// output row. The first dot product of a sum is the form that saturates, which none does (the bound of BuildTieRecords): it has a destination of its
+// own, where the other adds in place and what it starts from is copied in front of it. Bound by vector instructions (93 % of the busy cycles).
+// Layer and pointwise one behind it against a sum of plain windows times the zero point at the end, with choices in place of plane_rows.h's masks:
+// uint8 3x3 on 72 of 138 x 138, batch 10, 25.3 -> 24.6 us, 5x5 on 64 of 74 x 74, batch 14, 14.6 -> 14.3; int8 3x3 on 336 of 54 x 54, batch 17, 20.2 -> 19.7.
 template <int K, int S, int R, bool UNIFORM, bool SUMS>
 __global__ void __launch_bounds__(256) DwRegI8Kernel(DwrArgs a) {
   using T = Tile<TVX_I8, K, S, R>;
@@ -146,14 +151,14 @@ __global__ void __launch_bounds__(256) DwRegI8Kernel(DwrArgs a) {
       const int w0 = Cut(rows.d[i], q * S), w1 = K > 4 ? Cut(rows.d[i], q * S + 4) : 0;
       int box = 0;
       if (SUMS) {
-        box = __builtin_amdgcn_sdot4(w0, K > 3 ? 0x01010101 : 0x00010101, 0, false);
-        if (K > 4) box = __builtin_amdgcn_sdot4(w1, 0x00000001, box, false);
+        box = __builtin_amdgcn_sdot4(w0, a.nzws4, 0, true);
+        if (K > 4) box = __builtin_amdgcn_sdot4(w1, a.nzws1, box, true);
       }
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const int ky = i - r * S;
         if (ky < 0 || ky >= K) continue;
-        acc[r][q] = __builtin_amdgcn_sdot4(w0, w[2 * ky], ky == 0 ? bias : acc[r][q], false);
+        acc[r][q] = ky == 0 ? __builtin_amdgcn_sdot4(w0, w[2 * ky], bias, true) : __builtin_amdgcn_sdot4(w0, w[2 * ky], acc[r][q], false);
         if (K > 4) acc[r][q] = __builtin_amdgcn_sdot4(w1, w[2 * ky + 1], acc[r][q], false);
         if (SUMS) sum[r][q] = ky == 0 ? box : sum[r][q] + box;
       }
@@ -171,7 +176,7 @@ __global__ void __launch_bounds__(256) DwRegI8Kernel(DwrArgs a) {
     for (int h = 0; h < PX / 4; ++h) {
       int v[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = SUMS ? __mul24(-a.zws, sum[r][4 * h + e]) + acc[r][4 * h + e] : acc[r][4 * h + e];
+      for (int e = 0; e < 4; ++e) v[e] = SUMS ? (sum[r][4 * h + e] << a.sum_shift) + acc[r][4 * h + e] : acc[r][4 * h + e];
       if (a.pre_ties) {  // (uniform)
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] <<= a.pre_ties >> 1;
@@ -288,6 +293,7 @@ int DwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   a.m_c = Reciprocal(a.C);
 
   int s = TVX_OK;
+  bool sums = false;  // window sums are needed
   if (q) {
     const bool w_u8 = d->w_dtype == TVX_U8, x_u8 = d->in_dtype == TVX_U8;
     const int zxs = d->in_zp - (x_u8 ? 128 : 0), zws = op->w_zp - (w_u8 ? 128 : 0);
@@ -315,7 +321,11 @@ int DwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
     a.pre_ties = up * 2 + ties;
     a.fill = static_cast<int>(static_cast<uint32_t>(zxs & 0xff) * 0x01010101u);
     a.xor_in = x_u8 ? static_cast<int>(0x80808080u) : 0;
-    a.zws = zws;
+    a.sum_shift = zws == -128;
+    const uint32_t nzws = static_cast<uint32_t>(zws == -128 ? 64 : -zws) & 0xff;
+    a.nzws4 = static_cast<int>(nzws * (K > 3 ? 0x01010101u : 0x00010101u));
+    a.nzws1 = static_cast<int>(nzws);
+    sums = zws != 0;
     a.lo = op->act_lo - out_flip; a.hi = op->act_hi - out_flip; a.narrow = a.lo > -128 || a.hi < 127;
     a.out_xor = out_flip ? static_cast<int>(0x80808080u) : 0;
     s = op->packed.Upload(tab.data(), tab.size() * 4);
@@ -339,7 +349,7 @@ int DwRegSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const v
   }
   if (s != TVX_OK) return s;
   Plan plan{a, nullptr, dim3(1), block};
-  plan.fn = dt == TVX_I8 ? PickKernel<TVX_I8>(K, S, R, uniform, a.zws != 0) : dt == TVX_F16 ? PickKernel<TVX_F16>(K, S, R, uniform, false) : PickKernel<TVX_F32>(K, S, R, uniform, false);
+  plan.fn = dt == TVX_I8 ? PickKernel<TVX_I8>(K, S, R, uniform, sums) : dt == TVX_F16 ? PickKernel<TVX_F16>(K, S, R, uniform, false) : PickKernel<TVX_F32>(K, S, R, uniform, false);
   plan.grid = uniform ? dim3(a.C, parts, d->batch) : dim3(static_cast<unsigned>((planes * a.tpp + 255) / 256));
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
   op->run = DwRegRun;

@@ -86,6 +86,25 @@ struct PlaneRows {
     }
   }
 
+  // the columns of dword j of a row that begins in column ix: ones where the image has them
+  static __device__ __forceinline__ uint32_t Columns(const PlaneArgs& a, int ix, int j) {
+    constexpr int N = 4 / E;  // elements
+    const int c = ix + j * N;
+    uint32_t keep;
+    if constexpr (N == 1) {
+      keep = ~static_cast<uint32_t>((c | (a.W - 1 - c)) >> 31);
+    } else if constexpr (N == 2) {
+      keep = (static_cast<unsigned>(c) < static_cast<unsigned>(a.W) ? 0xffffu : 0u) | (static_cast<unsigned>(c + 1) < static_cast<unsigned>(a.W) ? 0xffff0000u : 0u);
+    } else {  // (by half as many bits twice: a shift by 32 is one by 0)
+      const int in_front = 4 * min(max(-c, 0), 4), behind = 4 * min(max(c + 4 - a.W, 0), 4);
+      keep = (~0u << in_front << in_front) & (~0u >> behind >> behind);
+    }
+    // (a mask and a bit operation per dword, not a condition and a choice: chains of choices by VCC take 16 to 23 cycles each, these 4. float32 3x3
+    // maximum on 213 of 28 x 28, batch 17: 7.20 -> 6.91 us; float32 5x5 stencil at stride 2 and pointwise layer on 8 of 22 x 22, batch 10: 9.8 -> 9.3)
+    asm("" : "+v"(keep));
+    return keep;
+  }
+
   __device__ __forceinline__ void Load(const PlaneArgs& a, int plane, int iy, int ix) {
     const int first = plane * (a.H * a.W);
     int moved[NR];  // elements by which a run was moved to lie inside the tensor
@@ -113,20 +132,19 @@ struct PlaneRows {
     if (__ballot(ix < 0 || ix + L > a.W)) {
 #pragma unroll
       for (int j = 0; j < LD; ++j) {
-        uint32_t keep = 0;
+        const uint32_t keep = Columns(a, ix, j);
 #pragma unroll
-        for (int e = 0; e < 4 / E; ++e)
-          if (static_cast<unsigned>(ix + j * (4 / E) + e) < static_cast<unsigned>(a.W)) keep |= (E == 4 ? ~0u : (1u << (8 * E & 31)) - 1u) << (8 * E * e);
-#pragma unroll
-        for (int i = 0; i < NR; ++i) d[i][j] = (d[i][j] & keep) | (fill & ~keep);
+        for (int i = 0; i < NR; ++i) d[i][j] = static_cast<uint32_t>(__builtin_amdgcn_bitop3_b32(static_cast<int>(d[i][j]), static_cast<int>(keep), static_cast<int>(fill), 0xe2));  // keep ? d : fill
       }
     }
     if (__ballot(iy < 0 || iy + NR > a.H)) {
 #pragma unroll
       for (int i = 0; i < NR; ++i) {
-        const bool in = static_cast<unsigned>(iy + i) < static_cast<unsigned>(a.H);
+        const int y = iy + i;
+        int outside = (y | (a.H - 1 - y)) >> 31;
+        asm("" : "+v"(outside));
 #pragma unroll
-        for (int j = 0; j < LD; ++j) d[i][j] = in ? d[i][j] : fill;
+        for (int j = 0; j < LD; ++j) d[i][j] = static_cast<uint32_t>(__builtin_amdgcn_bitop3_b32(static_cast<int>(fill), outside, static_cast<int>(d[i][j]), 0xe2));  // outside ? fill : d
       }
     }
   }
