@@ -45,6 +45,23 @@ def test_tiles_through_lds(oracle, m, k, n, mode, offset, monkeypatch):
             assert np.array_equal(got, want), (shape, int((got != want).sum()))
 
 
+@pytest.mark.parametrize("mode", ["u8", "i8pc", "f16"])
+@pytest.mark.parametrize("m,n", [(1, 1), (65, 70), (130, 129), (300, 257)])
+@pytest.mark.parametrize("k", [64, 128, 129, 300, 512, 577, 1153])
+def test_stages_on_groups(oracle, m, n, k, mode, monkeypatch):
+    """Reductions cut over groups of wavefronts: fewer stages than groups, as many, one more, a last round that is not full."""
+    x, w, b, kws = _case(m, k, n, mode)
+    monkeypatch.setenv("TVX_FC_ROWS", "1")
+    want = oracle.fully_connected(x, w, b, act=1, **kws)
+    TC.expect_variant(monkeypatch, "fc_tile_f16" if mode == "f16" else "fc_tile_i8")
+    monkeypatch.setenv("TVX_FC_ROWS_SHAPE", "8")
+    got = TC.gpu_fully_connected(x, w, b, act=1, want_kernel="fc_rows_f16" if mode == "f16" else "fc_rows_i8", **kws)
+    if mode == "f16":   # (results of a few units, off by up to one unit of float16's last place: 2^-9 at 1 to 2)
+        assert np.allclose(got.astype(np.float64), want.astype(np.float64), rtol=2e-3, atol=2e-3)
+    else:
+        assert np.array_equal(got, want), int((got != want).sum())
+
+
 @pytest.mark.parametrize("shape", [3, 5, 7])
 def test_rows_keep_an_infinity_apart(monkeypatch, shape):
     """What lies behind a row that ends inside a stage is not multiplied."""

@@ -319,15 +319,21 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
 // outputs leave eight bytes at a time. Here four wavefronts share a tile of 64 MT x 64 NT outputs: 128 bytes of each row and the weights
 // behind them, in fragment order, are brought to LDS once for all of them - rows through registers (they begin anywhere), weights by
 // DMA - while the stage before is multiplied. Weights are packed so that a lane ends up with sixteen consecutive features of a row.
-template <int DT, int MT, int NT, int kStage>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) FcTileKernel(RowsArgs a) {
+// Where the tiles are about as many as the CUs, a stage is a chain - load, store, barrier, fragments, products - that the four wavefronts, one a
+// SIMD, wait through (0.6 us): KS such groups of a workgroup take every KS-th stage each, with buffers of their own, and add up at the end.
+// Four groups fill the SIMDs' issue (1.0 us for four stages). u8 5008 x 2944 -> 115: 19.0 us on 32 x 32 tiles, 11.5; f16 456 x 1920 -> 1203 18.9,
+// 12.8; u8 7621 x 1312 -> 107 11.4 on one group, 9.1. Two groups, and two of 64 x 128 or 128 x 128 tiles, lay between one and four in all but a few.
+template <int DT, int MT, int NT, int kStage, int KS>
+__global__ void __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(KS > 2 ? KS : 2))) FcTileKernel(RowsArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   using mfma = Mfma<DT, 32>;
+  using quad = typename Mfma<DT, 16>::acc;
   constexpr int E = DT == kI8 ? 1 : DT == kF16 ? 2 : 4;
   constexpr int kRows = 64 * MT, kPitch = kStage + 16, kSteps = kStage / 32, kPer = kStage / 16;
   constexpr int kX = kRows * kPitch, kBuffer = kX + 2 * NT * kSteps * 1024;  // bytes of one of two buffers: rows, weights
   constexpr int kChunks = kRows * (kStage / 16) / 256;                       // sixteen-byte chunks of rows a thread brings
-  const int tid = threadIdx.x, lane = tid & 63, row = lane & 31, part = lane >> 5;
+  const int tid = threadIdx.x & 255, lane = tid & 63, row = lane & 31, part = lane >> 5;
+  const int group = KS > 1 ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 8)) : 0;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
   const int id = static_cast<int>(blockIdx.x & 7) * a.per_xcd + static_cast<int>(blockIdx.x >> 3);
   if (id >= a.total) return;
@@ -389,26 +395,31 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) F
   int rs[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) rs[t] = 0;
-  fetch_x(0);
-  fetch_w(0, lds);
+  uint8_t* const own = lds + group * 2 * kBuffer;
+  if (KS == 1 || group < stages) {
+    fetch_x(group);
+    fetch_w(group, own);
+  }
   // the features' tables, behind the buffers
-  uint8_t* const tables = lds + 2 * kBuffer;
+  uint8_t* const tables = lds + KS * 2 * kBuffer;
   constexpr int kFeatures = 64 * NT;
-  for (int i = tid; i < kFeatures; i += 256) {
+  for (int i = threadIdx.x; i < kFeatures; i += 256 * KS) {
     if (DT == kI8) reinterpret_cast<tvx_v4i*>(tables)[i] = a.rq[tn * kFeatures + i];
     reinterpret_cast<int*>(tables + kFeatures * 16)[i] = a.bias[tn * kFeatures + i];
   }
-  store_x(0, lds);
+  if (KS == 1 || group < stages) store_x(group, own);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the weights' DMA)
   __syncthreads();
-  for (int stage = 0; stage < stages; ++stage) {
-    const uint8_t* const now = lds + (stage & 1) * kBuffer;
-    uint8_t* const then = lds + (~stage & 1) * kBuffer;
-    const bool more = stage + 1 < stages;
+  for (int first = 0, turn = 0; first < stages; first += KS, turn ^= 1) {
+    const int stage = first + group;
+    const uint8_t* const now = own + turn * kBuffer;
+    uint8_t* const then = own + (turn ^ 1) * kBuffer;
+    const bool more = stage + KS < stages;
     if (more) {
-      fetch_x(stage + 1);
-      fetch_w(stage + 1, then);
+      fetch_x(stage + KS);
+      fetch_w(stage + KS, then);
     }
+    if (KS == 1 || stage < stages)  // (uniform)
 #pragma unroll
     for (int s = 0; s < kSteps; ++s) {
       v4i fx[MT], fw[NT];
@@ -427,9 +438,40 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) F
         for (int n = 0; n < NT; ++n) mfma::Step(acc[t][n], fw[n], fx[t]);
     }
     if (more) {
-      store_x(stage + 1, then);
+      store_x(stage + KS, then);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
+    }
+    if (first + KS < stages) __syncthreads();
+  }
+  if constexpr (KS > 1) {  // the groups' sums: the others' into the buffers, the first group adds
+    constexpr int kQuads = MT * NT * 4, kSums = kQuads * 4096 + MT * 1024;
+    static_assert((KS - 1) * kSums <= KS * 2 * kBuffer);
+    __syncthreads();
+    if (group) {
+      uint8_t* const to = lds + (group - 1) * kSums;
+#pragma unroll
+      for (int q = 0; q < kQuads; ++q) {
+        const auto& c = acc[q / 4 / NT][q / 4 % NT];
+        reinterpret_cast<quad*>(to + q * 4096)[tid] = quad{c[4 * (q % 4)], c[4 * (q % 4) + 1], c[4 * (q % 4) + 2], c[4 * (q % 4) + 3]};
+      }
+      if (DT == kI8)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) reinterpret_cast<int*>(to + kQuads * 4096 + t * 1024)[tid] = rs[t];
+    }
+    __syncthreads();
+    if (group) return;
+#pragma unroll
+    for (int g = 0; g < KS - 1; ++g) {
+      const uint8_t* const from = lds + g * kSums;
+#pragma unroll
+      for (int q = 0; q < kQuads; ++q) {
+        const quad v = reinterpret_cast<const quad*>(from + q * 4096)[tid];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[q / 4 / NT][q / 4 % NT][4 * (q % 4) + e] += v[e];
+      }
+      if (DT == kI8)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) rs[t] += reinterpret_cast<const int*>(from + kQuads * 4096 + t * 1024)[tid];
     }
   }
 
@@ -508,19 +550,20 @@ struct Shape { int ts, rows, features, waves, ks, lds, stage; RowsFn fn[3][2]; }
     { { FcRowsKernel<kI8, TS, WM, WN, KS, MT, NT, R, false>, FcRowsKernel<kI8, TS, WM, WN, KS, MT, NT, R, true> },                        \
       { FcRowsKernel<kF16, TS, WM, WN, KS, MT, NT, R, false>, FcRowsKernel<kF16, TS, WM, WN, KS, MT, NT, R, true> },                      \
       { FcRowsKernel<kF32, TS, WM, WN, KS, MT, NT, R, false>, nullptr } } }
-#define TVX_FC_TILE(MT, NT, STAGE)                                                                                                         \
-  { 32, 64 * MT, 64 * NT, 4, 1, 2 * (64 * MT * (STAGE + 16) + 2 * NT * STAGE * 32) + 64 * NT * 20, STAGE / 32,                                               \
-    { { FcTileKernel<kI8, MT, NT, STAGE>, FcTileKernel<kI8, MT, NT, STAGE> }, { FcTileKernel<kF16, MT, NT, STAGE>, FcTileKernel<kF16, MT, NT, STAGE> },            \
+#define TVX_FC_TILE(MT, NT, STAGE, KS)                                                                                                         \
+  { 32, 64 * MT, 64 * NT, 4 * KS, KS, KS * 2 * (64 * MT * (STAGE + 16) + 2 * NT * STAGE * 32) + 64 * NT * 20, STAGE / 32,                                           \
+    { { FcTileKernel<kI8, MT, NT, STAGE, KS>, FcTileKernel<kI8, MT, NT, STAGE, KS> }, { FcTileKernel<kF16, MT, NT, STAGE, KS>, FcTileKernel<kF16, MT, NT, STAGE, KS> }, \
       { nullptr, nullptr } } }
 const Shape kShapes[] = {
     TVX_ROWS(16, 1, 1, 4, 1, 1, 8),  // 0: 16 x 16, reduction on four wavefronts
     TVX_ROWS(32, 1, 1, 4, 1, 1, 7),  // 1: 32 x 32, on four
     TVX_ROWS(32, 2, 2, 1, 1, 1, 8),  // 2: 64 x 64, not split
-    TVX_FC_TILE(1, 1, 128),          // 3: 64 x 64 through LDS, 128 bytes of a row at a time
-    TVX_FC_TILE(1, 2, 128),          // 4: 64 rows x 128
-    TVX_FC_TILE(2, 2, 128),          // 5: 128 x 128
-    TVX_FC_TILE(1, 1, 256),          // 6: 64 x 64, 256 bytes
-    TVX_FC_TILE(2, 2, 64),           // 7: 128 x 128, 64 bytes
+    TVX_FC_TILE(1, 1, 128, 1),          // 3: 64 x 64 through LDS, 128 bytes of a row at a time
+    TVX_FC_TILE(1, 2, 128, 1),          // 4: 64 rows x 128
+    TVX_FC_TILE(2, 2, 128, 1),          // 5: 128 x 128
+    TVX_FC_TILE(1, 1, 256, 1),          // 6: 64 x 64, 256 bytes
+    TVX_FC_TILE(2, 2, 64, 1),           // 7: 128 x 128, 64 bytes
+    TVX_FC_TILE(1, 1, 128, 4),          // 8: 64 x 64, every fourth stage on each of four groups
 };
 #undef TVX_ROWS
 #undef TVX_FC_TILE
@@ -538,27 +581,31 @@ uint32_t Magic(int d) { return d <= 1 ? 0u : static_cast<uint32_t>(((uint64_t{1}
 struct Fit { int resident; double base, latency, share, end, unaligned; };  // workgroups of a CU; us, and by how much more at any byte
 const Fit kFits[2][kShapeCount] = {
     {{}, {4, 1.15, 0.48, 0.80, 0.10, 0.49}, {4, 2.25, 0.11, 0.16, 1.12, 1.33}, {4, 1.53, 0.62, 0.37, 0.55, 0.17}, {2, 2.09, 0.72, 0.56, 1.02, 0.14},
-     {2, 3.69, 0.92, 0.97, 2.01, 0.20}, {2, 1.83, 0.95, 0.80, 0.99, 0.19}, {3, 3.21, 0.60, 0.48, 1.61, 0.14}},
+     {2, 3.69, 0.92, 0.97, 2.01, 0.20}, {2, 1.83, 0.95, 0.80, 0.99, 0.19}, {3, 3.21, 0.60, 0.48, 1.61, 0.14},
+     {1, 1.21, 1.10, 0.37, 2.51, 0.38}},
     {{}, {4, 1.07, 0.43, 0.76, 0.00, 0.66}, {4, 1.97, 0.11, 0.16, 0.29, 0.79}, {4, 0.96, 0.57, 0.32, 0.89, 0.24}, {2, 1.61, 0.64, 0.55, 1.22, 0.18},
-     {2, 3.10, 0.84, 0.94, 3.26, 0.20}, {2, 1.50, 0.80, 0.74, 0.90, 0.22}, {3, 2.40, 0.56, 0.55, 1.93, 0.22}}};
+     {2, 3.10, 0.84, 0.94, 3.26, 0.20}, {2, 1.50, 0.80, 0.74, 0.90, 0.22}, {3, 2.40, 0.56, 0.55, 1.93, 0.22},
+     {1, 0.98, 1.02, 0.41, 2.30, 0.22}}};
 double Cost(const tvx_fc_desc& d, int dt, int shape) {
   const Shape& sp = kShapes[shape];
   const Fit& f = kFits[dt][shape];
   const double row = static_cast<double>(d.k) * (dt == kI8 ? 1 : 2);
-  const int stage = sp.stage ? 32 * sp.stage : 32 * sp.ks * (sp.ks > 1 ? 4 : 1);
+  const int stage = sp.stage ? 32 * sp.stage : 32 * sp.ks * (sp.ks > 1 ? 4 : 1), groups = sp.stage ? sp.ks : 1;
   const double per_cu = static_cast<double>((d.m + sp.rows - 1) / sp.rows) * ((d.n + sp.features - 1) / sp.features) / ComputeUnits();
   double stages = std::ceil(row / stage);
   // (a reduction cut over wavefronts may end early in its last stage, which saves half of what is missing; behind one stage alone, nothing)
-  if (sp.ks > 1 && stages > 1) stages = 0.5 * (stages + 0.25 * std::ceil(std::ceil(row / 32) / sp.ks));
-  if (static_cast<uint64_t>(row) % 4) stages *= 1 + f.unaligned;
-  const double latency = std::max(per_cu / f.resident, 1.0) * stages * f.latency, share = per_cu * (f.end + stages * f.share);
+  if (!sp.stage && sp.ks > 1 && stages > 1) stages = 0.5 * (stages + 0.25 * std::ceil(std::ceil(row / 32) / sp.ks));
+  const double each = static_cast<uint64_t>(row) % 4 ? 1 + f.unaligned : 1.0, chain = groups > 1 ? std::ceil(stages / groups) : stages;
+  // (tiles on groups leave a CU no room for a second: 259 of them take two rounds - f16 2332 x 2544 -> 401 34.5 us, 24.3 on 32 x 32)
+  const double rounds = groups > 1 ? std::ceil(per_cu / f.resident) : std::max(per_cu / f.resident, 1.0);
+  const double latency = rounds * chain * each * f.latency, share = per_cu * (f.end + stages * each * f.share);
   return 2.2 + f.base + std::sqrt(std::sqrt(std::pow(latency, 4) + std::pow(share, 4)));
 }
 
 // 16 x 16 tiles until there is one for each CU (f16 16 x 4096 -> 4096: 7.5 us against 9.1 on 32 x 32 tiles), 32 x 32 from there on (f32
 // 256 x 1024 -> 1024: 8.8 against 11.9), and 64 x 64 - fragments used twice, no exchange at the end - where there are more than one
 // of those per CU, or half as many with a reduction too short to split; int8 and float16 otherwise where Cost sees more than it may be
-// off by. float32, whose products take the longest, gains nothing by rows through LDS (882 x 3984 -> 1070: 95 us, 101 with).
+// off by. Stages on four groups are a fit to 260 layers (7 and 10 % off each); of 420 others eleven take them, 0.82 of the time, one of these 1.02. float32, whose products take the longest, gains nothing by rows through LDS (882 x 3984 -> 1070: 95 us, 101 with).
 int ChooseShape(const tvx_fc_desc& d, int dt) {
   const uint64_t t16 = static_cast<uint64_t>((d.m + 15) / 16) * ((d.n + 15) / 16), t64 = static_cast<uint64_t>((d.m + 63) / 64) * ((d.n + 63) / 64);
   const uint64_t cus = ComputeUnits();
@@ -568,6 +615,8 @@ int ChooseShape(const tvx_fc_desc& d, int dt) {
   int best = direct;
   double least = 0.94 * Cost(d, dt, direct);  // (what the fit is off by; then the shorter program)
   for (int shape = 1; shape < kShapeCount; ++shape) {
+    const Shape& sp = kShapes[shape];
+    if (sp.stage && sp.ks > 1 && static_cast<uint64_t>(d.k) * (dt == kI8 ? 1 : 2) <= 64ull * sp.stage * sp.ks) continue;  // (two stages a group at least)
     const double cost = Cost(d, dt, shape);
     if (cost < least) { best = shape; least = cost; }
   }
