@@ -85,6 +85,8 @@ struct TileArgs {
   int OC, OH, OW, ocg;     // ocg: output channels of a group
   int taps_w, taps_h, dil_col, dil_row;  // for the box sum: LDS pixels between taps
   int runs, run_px, run_out, out_pitch;  // copy-out: runs of consecutive outputs of a channel, their pixels and distance; LDS bytes of a channel
+  int stack;               // output rows that a tile's row stands for (STACK), the channels of each behind one another
+  uint32_t m_ocg, m_th;
   uint32_t m_run4;         // reciprocal of a run's groups of four pixels
   int runs_shift;          // log2 of the threads that a channel's runs take
   uint32_t m_run_wide;     // the same with sixteen bytes a thread
@@ -194,7 +196,12 @@ template <int DT> struct Item {
 
 // WM x WN wavefronts share the tile's pixels and channels (MT x NT MFMA tiles each), KS wavefronts a tile's reduction.
 // R: steps whose weights are on their way to a wavefront at a time.
-template <int DT, int SUMS, int WM, int WN, int KS, int MT, int NT, int R, int EU, bool MULTI>
+// STACK: up to 16 output channels of quantized tensors would leave half of a tile's 32 and more empty. The channels of several output rows
+// stand behind one another there instead: a tile's row is `stack` rows of the image, its window as much taller, and each row's weights lie at its
+// own taps among the weights' zero point (which drops out with the window sums; a zero of floating point would not under an infinity).
+// Three rows of 3x3 take 5 / 9 of the multiplications, LDS reads and weights, two rows of 5x5 3 / 5: int8 144 -> 16 in four groups, 3x3 on 125 x 125, batch 29: 87.7 -> 41.1 us; uint8 160 -> 16, 7x7 on 134 x 134, batch 14, 116.9 -> 87.7.
+// (Kernels of their own: the rows' places cost the others .1 to .2 us a launch.)
+template <int DT, int SUMS, int WM, int WN, int KS, int MT, int NT, int R, int EU, bool MULTI, bool STACK>
 __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves_per_eu(EU))) ConvTileKernel(TileArgs a) {
   constexpr int kThreads = 64 * WM * WN * KS;
   static_assert(R % 2 == 0 && R <= kMostAhead, "the activations' two buffers alternate with the steps");
@@ -585,11 +592,12 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
         }
       }
   __syncthreads();
-  const int ohw = c.OH * c.OW, whole = c.TW == c.OW;  // (uniform)
+  const int stack = STACK ? c.stack : 1;  // (uniform)
+  const int ohw = c.OH * c.OW, whole = !STACK && c.TW == c.OW;  // (uniform)
   const int rows_live = min(c.TH, c.OH - y0);
-  const int runs_live = whole ? min(c.G, c.batch - n0) : rows_live, run_live = whole ? rows_live * c.OW : min(c.TW, c.OW - x0);
-  const int ocb0 = ocl * (WN * NT * 32), channels = min(WN * NT * 32, c.ocg - ocb0);
-  uint8_t* yb = c.y + ((static_cast<size_t>(n0) * c.OC + static_cast<size_t>(group) * c.ocg + ocb0) * ohw + y0 * c.OW + x0) * E;
+  const int runs_live = whole ? min(c.G, c.batch - n0) : STACK ? c.runs : rows_live, run_live = whole ? rows_live * c.OW : min(c.TW, c.OW - x0);
+  const int ocb0 = ocl * (WN * NT * 32), channels = STACK ? stack * c.ocg : min(WN * NT * 32, c.ocg - ocb0);
+  uint8_t* yb = c.y + ((static_cast<size_t>(n0) * c.OC + static_cast<size_t>(group) * c.ocg + ocb0) * ohw + y0 * stack * c.OW + x0) * E;
   // a thread keeps its place in the channels' runs and walks the channels: sixteen bytes of one at a time (a run's last begin sixteen
   // bytes before its end), four pixels where runs are shorter. Against four pixels everywhere: f16 44 -> 192, 3x3 on 44 x 44, batch 18,
   // 21.5 -> 18.1 us, 19 -> 432 on 114 x 114, batch 2, 21.4 -> 19.1; int8 1 % on 40 drawn layers, at most 6.
@@ -604,10 +612,18 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
   const uint8_t* from = lds + c.off_out + ch0 * c.out_pitch + (run * c.run_px + px) * E;
   uint8_t* to = yb + (static_cast<size_t>(ch0) * ohw + static_cast<size_t>(run) * c.run_out + px) * E;
   const size_t to_step = static_cast<size_t>(ch_step) * ohw * E;
+  // stacked rows: where a slot's channel and row begin; false where there is no such row
+  const int image = STACK ? DivM(run, c.m_th) : 0, first = (run - image * c.TH) * stack;
+  auto find_row = [&](int ch) {
+    const int j = DivM(ch, c.m_ocg), r = first + j;
+    to = yb + (static_cast<size_t>(image) * c.OC + (ch - j * c.ocg)) * ohw + r * c.OW + px;
+    return y0 * stack + r < c.OH && n0 + image < c.batch;
+  };
   if (left > 0 && wide) {
     if constexpr (E < 4) {
       const uint32_t by = static_cast<uint32_t>(run * c.run_px + px) * E & 3;
       for (int ch = ch0; ch < channels; ch += ch_step, from += ch_step * c.out_pitch, to += to_step) {
+        if (STACK && !find_row(ch)) continue;
         const uint32_t* const w = reinterpret_cast<const uint32_t*>(from - by);  // (the dwords behind a run that begins at any byte)
         uint32_t d[5], out[4];
 #pragma unroll
@@ -619,6 +635,7 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
     }
   } else if (left > 0)
   for (int ch = ch0; ch < channels; ch += ch_step, from += ch_step * c.out_pitch, to += to_step) {
+    if (STACK && !find_row(ch)) continue;
     uint32_t four[E];
     if (left >= 4) {
       if constexpr (E == 1) {  // (a run begins at any byte: the dword out of two)
@@ -653,24 +670,30 @@ __global__ void __launch_bounds__(64 * WM * WN * KS) __attribute__((amdgpu_waves
 typedef void (*TileFn)(TileArgs);
 
 // The ways a workgroup's wavefronts share a tile.
-// fn: int8, float16, float32, int8 with sums in the loop and with sums box-filtered; one chunk of the channels or several
-struct Shape { int pixels, channels, ks, waves; double length; TileFn fn[5][2]; };  // length: of its chain, fitted (Cost)
-#define TVX_TILE_DT(DT, SUMS, WM, WN, KS, MT, NT, R, EU) { ConvTileKernel<DT, SUMS, WM, WN, KS, MT, NT, R, EU, false>, ConvTileKernel<DT, SUMS, WM, WN, KS, MT, NT, R, EU, true> }
-#define TVX_TILE(WM, WN, KS, MT, NT, R, EU, LENGTH)                                                               \
-  { WM * MT * 32, WN * NT * 32, KS, WM * WN * KS, LENGTH, { TVX_TILE_DT(kI8, kNoSums, WM, WN, KS, MT, NT, R, EU), TVX_TILE_DT(kF16, kNoSums, WM, WN, KS, MT, NT, R, EU), \
-                                                    TVX_TILE_DT(kF32, kNoSums, WM, WN, KS, MT, NT, R, EU), TVX_TILE_DT(kI8, kSumsInLoop, WM, WN, KS, MT, NT, R, EU), \
-                                                    TVX_TILE_DT(kI8, (MT * NT > 1 ? kSumsBox : kSumsInLoop), WM, WN, KS, MT, NT, R, EU) } }
+// fn: int8, float16, float32, int8 with sums in the loop and with sums box-filtered, int8 in stacked rows without and with sums; one chunk of the channels or several
+struct Shape { int pixels, channels, ks, waves; double length; TileFn fn[7][2]; };  // length: of its chain, fitted (Cost)
+#define TVX_TILE_DT(DT, SUMS, WM, WN, KS, MT, NT, R, EU, STACK) { ConvTileKernel<DT, SUMS, WM, WN, KS, MT, NT, R, EU, false, STACK>, ConvTileKernel<DT, SUMS, WM, WN, KS, MT, NT, R, EU, true, STACK> }
+#define TVX_TILE_FNS(WM, WN, KS, MT, NT, R, EU)                                                                   \
+  TVX_TILE_DT(kI8, kNoSums, WM, WN, KS, MT, NT, R, EU, false), TVX_TILE_DT(kF16, kNoSums, WM, WN, KS, MT, NT, R, EU, false), \
+  TVX_TILE_DT(kF32, kNoSums, WM, WN, KS, MT, NT, R, EU, false), TVX_TILE_DT(kI8, kSumsInLoop, WM, WN, KS, MT, NT, R, EU, false), \
+  TVX_TILE_DT(kI8, (MT * NT > 1 ? kSumsBox : kSumsInLoop), WM, WN, KS, MT, NT, R, EU, false)
+#define TVX_TILE(WM, WN, KS, MT, NT, R, EU, LENGTH) \
+  { WM * MT * 32, WN * NT * 32, KS, WM * WN * KS, LENGTH, { TVX_TILE_FNS(WM, WN, KS, MT, NT, R, EU), { nullptr, nullptr }, { nullptr, nullptr } } }
+#define TVX_TILE_32(WM, KS, R, EU, LENGTH) \
+  { WM * 32, 32, KS, WM * KS, LENGTH, { TVX_TILE_FNS(WM, 1, KS, 1, 1, R, EU), TVX_TILE_DT(kI8, kNoSums, WM, 1, KS, 1, 1, R, EU, true), TVX_TILE_DT(kI8, kSumsInLoop, WM, 1, KS, 1, 1, R, EU, true) } }
 const Shape kShapes[] = {
     TVX_TILE(4, 2, 1, 2, 1, 4, 4, 1.0),   // 0: 256 x 64, eight wavefronts
     TVX_TILE(2, 2, 2, 2, 1, 4, 4, 1.27),  // 1: 128 x 64, eight
     TVX_TILE(2, 2, 1, 2, 1, 4, 4, 0.8),   // 2: 128 x 64, four
-    TVX_TILE(4, 1, 2, 1, 1, 6, 4, 1.43),  // 3: 128 x 32, eight
-    TVX_TILE(4, 1, 1, 1, 1, 6, 4, 1.0),   // 4: 128 x 32, four
+    TVX_TILE_32(4, 2, 6, 4, 1.43),        // 3: 128 x 32, eight
+    TVX_TILE_32(4, 1, 6, 4, 1.0),         // 4: 128 x 32, four
     TVX_TILE(2, 2, 2, 1, 1, 6, 4, 1.4),   // 5: 64 x 64, eight
-    TVX_TILE(2, 1, 4, 1, 1, 4, 4, 1.7),   // 6: 64 x 32, eight
-    TVX_TILE(1, 1, 8, 1, 1, 6, 4, 1.75),  // 7: 32 x 32, eight
+    TVX_TILE_32(2, 4, 4, 4, 1.7),         // 6: 64 x 32, eight
+    TVX_TILE_32(1, 8, 6, 4, 1.75),        // 7: 32 x 32, eight
 };
+#undef TVX_TILE_32
 #undef TVX_TILE
+#undef TVX_TILE_FNS
 #undef TVX_TILE_DT
 constexpr int kShapeCount = sizeof(kShapes) / sizeof(kShapes[0]);
 
@@ -688,7 +711,7 @@ int64_t WindowBytes(const Shape& sp, int64_t staged, int E, int loop) {
 
 struct Geometry {
   int shape, TW, TH, G, gpc, chunks, loop;
-  int IW, IH, pitch, lds_bytes, sums;
+  int IW, IH, pitch, lds_bytes, sums, stack;
   int64_t wgs;
   double cost;
 };
@@ -728,6 +751,14 @@ int SumsBy(const Shape& sp, int steps) {
   const int tiles = sp.pixels * sp.channels / 1024 * sp.ks / sp.waves;
   return tiles == 1 || steps * tiles / sp.ks <= 80 ? kSumsInLoop : kSumsBox;
 }
+
+// By how much less a tile of stacked rows has to promise, and the products of an output that two rows need up to so many outputs: what the results'
+// shorter runs take.
+// Without these lines the choice was 1.04 to 1.17 of the time of unstacked tiles on four of 132 layers, of 16 channels and few products each (int8
+// 8 -> 16, 3x3 / 2 on 50 x 69, batch 37, 7.2 us for 6.1; uint8 3 -> 16, 5x5 on 99 x 99, batch 7, 7.5 for 6.9;
+// but int8 20 -> 64 in four groups, 3x3 on 69 x 121, batch 46, 33.0 for 55.3).
+constexpr double kStackedMore = 1.06;
+constexpr int kStackedProducts = 128, kStackedOutputs = 2000000;
 
 struct Plan {
   TileArgs a;
@@ -819,7 +850,8 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
 
   TileArgs a{};
   int W = d->in_w, H = d->in_h, OW = d->out_w, OH = d->out_h;
-  const int kh = d->k_h, kw = d->k_w, dh = d->dilation_h, dw = d->dilation_w;
+  int kh = d->k_h;
+  const int kw = d->k_w, dh = d->dilation_h, dw = d->dilation_w;
   const bool flat = kh == 1 && kw == 1 && d->stride_w == 1 && d->stride_h == 1 && d->pad_left == 0 && d->pad_top == 0 && OW == W && OH == H;
   if (flat) { W = OW = W * H; H = OH = 1; }  // a 1 x 1 window needs no rows: an image is one
   const int group_px = dt == kF32 ? 4 : 8;
@@ -829,7 +861,8 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   a.H = H; a.W = W; a.OC = d->out_c; a.OH = OH; a.OW = OW; a.batch = d->batch;
   a.sh = d->stride_h; a.sw = d->stride_w; a.pad_t = d->pad_top; a.pad_l = d->pad_left;
   a.icg = C / groups; a.ocg = a.OC / groups;
-  const int granules = (a.icg * E + 15) / 16, taps = kh * kw;
+  const int granules = (a.icg * E + 15) / 16, real_taps = kh * kw;
+  int taps = real_taps;
   if (taps > 1024) return TVX_E_UNSUPPORTED;
   const uint64_t image = static_cast<uint64_t>(C) * H * W * E, out_image = static_cast<uint64_t>(a.OC) * OH * OW;
   a.row_step = kh == 1 ? a.sh : 1;
@@ -845,17 +878,35 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   if (const char* f = getenv("TVX_CONV_TILE_SHAPE")) want = atoi(f);  // test lever
   if (const char* f = getenv("TVX_CONV_TILE_COLS")) want_tw = atoi(f);  // test lever
   if (const char* f = getenv("TVX_CONV_TILE_LOOP")) want_loop = atoi(f);  // test lever
+  int want_stack = 0;
+  if (const char* f = getenv("TVX_CONV_TILE_STACK")) want_stack = atoi(f);  // test lever
+  const int rows = OH;
+  auto stacked = [&](int stack) {
+    OH = (rows + stack - 1) / stack;
+    kh = d->k_h + (stack - 1) * d->stride_h;
+    taps = kh * kw;
+    a.sh = stack * d->stride_h;
+    if (d->k_h > 1) a.row_stride = a.sh;
+  };
   Geometry best{};
   best.shape = -1;
+  for (int stack = 1; stack <= 4; ++stack) {
+  if (want_stack && stack != want_stack) continue;
+  if (stack > 1 && (dt != kI8 || d->k_h == 1 || dh != 1 || stack * a.ocg > 32 || stack > rows)) break;
+  if (!want_stack && stack == 2 && real_taps * a.icg < kStackedProducts && out_image * d->batch < kStackedOutputs) continue;
+  stacked(stack);
+  if (taps > 1024) break;
   for (int sidx = 0; sidx < kShapeCount; ++sidx) {
     if (want >= 0 && sidx != want) continue;
     const Shape& sp = kShapes[sidx];
+    if (stack > 1 && !sp.fn[5][0]) continue;
     const int cand[] = {OW, (OW + 1) / 2, (OW + 2) / 3, 8, 16, 32, 64, 128};
     for (int tw : cand) {
       if (want_tw) tw = want_tw;
       if (tw < 1 || tw > OW || tw > sp.pixels) continue;
       Geometry g{};
       g.shape = sidx;
+      g.stack = stack;
       g.TW = tw;
       g.TH = std::min(OH, sp.pixels / tw);
       // rows spread evenly over the tiles of a column
@@ -888,13 +939,16 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
       g.wgs = tiles * ((blocks + loop - 1) / loop) * groups;
       if (g.wgs > 0x3fffffff) continue;
       g.cost = Cost(sp, g, dt, taps, group_px, zws != 0, (a.pad_l || a.pad_t) && taps > 1, OW, cus);
+      if (stack > 1) g.cost *= kStackedMore;
       if (best.shape < 0 || g.cost < best.cost) best = g;
       }
     }
   }
+  }
   if (best.shape < 0) return TVX_E_UNSUPPORTED;
   const Geometry& g = best;
   const Shape& sp = kShapes[g.shape];
+  stacked(g.stack);
   if (image * g.G >= (1ull << 32) || out_image * g.G >= (1ull << 31)) return TVX_E_UNSUPPORTED;
 
   a.TW = g.TW; a.TH = g.TH; a.G = g.G; a.NQ = g.TW * g.TH * g.G;
@@ -927,8 +981,11 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   a.off_sum = a.off_tab + 2 * a.steps_pad * 4;
   a.off_zt = a.off_sum + (g.sums == kSumsBox ? static_cast<int>(npx) * 4 : 0);
   a.off_out = g.loop > 1 ? g.lds_bytes - static_cast<int>(OutBytes(sp, E)) : 0;
-  const bool whole = g.TW == OW;
-  a.runs = whole ? g.G : g.TH;
+  const bool whole = g.stack == 1 && g.TW == OW;
+  a.stack = g.stack;
+  a.m_ocg = Magic(a.ocg);
+  a.m_th = Magic(g.TH);
+  a.runs = whole ? g.G : g.G * g.TH;
   a.run_px = whole ? g.TH * OW : g.TW;
   a.run_out = whole ? a.OC * OH * OW : OW;
   a.out_pitch = OutPitch(sp, E);
@@ -978,26 +1035,34 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   const int32_t* bi = static_cast<const int32_t*>(bias_host);
   const uint8_t flip = w_u8 ? 0x80 : 0;
   const int epg = 16 / E;  // elements of a granule
-  for (int oc = 0; oc < a.OC; ++oc) {
-    const int grp = oc / a.ocg, ol = oc % a.ocg;
+  for (int oc = 0; oc < a.OC; ++oc)
+  for (int up = 0; up < g.stack; ++up) {
+    const int grp = oc / a.ocg, ol = up * a.ocg + oc % a.ocg;
     const size_t slot = static_cast<size_t>(grp) * a.tiles_per_group * sp.channels + ol;
     uint8_t* tile = packed.data() + slot / 32 * tile_bytes + (slot % 32) * 16;
-    const uint8_t* ws = src + static_cast<size_t>(oc) * a.icg * taps * E;
+    const uint8_t* ws = src + static_cast<size_t>(oc) * a.icg * real_taps * E;
     int64_t sw = 0;
     // (copies: a byte stored may be any of the fields')
     const int icg = a.icg, gpc = a.gpc;
     const size_t chunk_bytes = static_cast<size_t>(a.steps) * 1024;
+    // taps in front of the row's own and behind them: the weights' zero point
+    const int before = up * d->stride_h * kw, behind = taps - before - real_taps;
+    const uint8_t none = static_cast<uint8_t>(zws & 0xff);
     for (int c = 0; c < icg; ++c) {
-      const int gg = c / epg, chunk = gg / gpc, gr = gg % gpc;
+      const int gg = c / epg, chunk = gg / gpc;
       uint8_t* cp = tile + static_cast<size_t>(chunk) * chunk_bytes + (c % epg) * E;
+      int q = gg % gpc;
       if (E == 1) {
-        for (int t = 0, q = gr; t < taps; ++t, q += gpc) {
-          const uint8_t v = *ws++ ^ flip;
+        auto put = [&](uint8_t v) {
           cp[static_cast<size_t>(q >> 1) * 1024 + (q & 1) * 512] = v;
           sw += static_cast<int8_t>(v);
-        }
+          q += gpc;
+        };
+        for (int t = 0; t < before; ++t) put(none);
+        for (int t = 0; t < real_taps; ++t) put(*ws++ ^ flip);
+        for (int t = 0; t < behind; ++t) put(none);
       } else {
-        for (int t = 0, q = gr; t < taps; ++t, q += gpc, ws += E) std::memcpy(cp + static_cast<size_t>(q >> 1) * 1024 + (q & 1) * 512, ws, E);
+        for (int t = 0; t < taps; ++t, q += gpc, ws += E) std::memcpy(cp + static_cast<size_t>(q >> 1) * 1024 + (q & 1) * 512, ws, E);
       }
     }
     if (dt == kI8) {
@@ -1011,7 +1076,7 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   if (s == TVX_OK) s = op->aux3.Upload(tab.data(), tab.size() * 4);
   if (s == TVX_OK && dt == kI8) {
     std::vector<int32_t> rqt;
-    const int64_t bound = AccumulatorBound(static_cast<uint64_t>(taps) * a.icg, bias_host, d->out_c);
+    const int64_t bound = AccumulatorBound(static_cast<uint64_t>(real_taps) * a.icg, bias_host, d->out_c);
     const int slots = static_cast<int>(alloc_oc);
     int up;
     bool ties;
@@ -1031,7 +1096,7 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
 
   Plan plan{};
   plan.a = a;
-  plan.fn = sp.fn[g.sums == kNoSums ? dt : g.sums == kSumsInLoop ? 3 : 4][a.chunks > 1];
+  plan.fn = sp.fn[g.stack > 1 ? (g.sums == kNoSums ? 5 : 6) : g.sums == kNoSums ? dt : g.sums == kSumsInLoop ? 3 : 4][a.chunks > 1];
   plan.lds_bytes = static_cast<unsigned>(g.lds_bytes);
   plan.grid = static_cast<unsigned>(a.per_xcd) * 8;
   plan.threads = 64u * sp.waves;
