@@ -1,5 +1,5 @@
 // pwconv_dwconv3x3_pwconv_i8: an inverted-residual block - 1x1 expansion, depthwise 3x3, 1x1 projection and the
-// residual Add behind it - as one kernel, for the small feature maps (28, 14 and 7 columns) where three or four
+// residual Add behind it - as one kernel, for the small feature maps and batches where three or four
 // launches of a few microseconds of work each cost more than the arithmetic. The closed driver fuses such
 // chains when it verifies the graph (reference: src/tim/vx/internal/src/vsi_nn_graph.c:1591-1603); the
 // operators it fuses are the Conv2d nodes of src/tim/vx/internal/src/ops/vsi_nn_op_conv2d.c:35-118.
@@ -857,7 +857,8 @@ int MbConvSetup(tvx_op* op, const MbStage& ex, const MbStage& dw, const tvx_conv
   const int Cin = e->in_c, Cexp = e->out_c, Cout = pr->out_c;
   const int cin_steps = (Cin + 31) / 32, chunks = (Cexp + 31) / 32, nt = (Cout + 31) / 32;
   if (cin_steps > kMaxCinSteps) return TVX_E_UNSUPPORTED;
-  if (S == 1 ? (W != 7 && W != 14 && W != 28) || nt > (W == 28 ? 5 : 10) : (W != 14 && W != 28) || nt > 10) return TVX_E_UNSUPPORTED;
+  const bool two_forms = W == 7 || W == 14;
+  if (S == 1 ? W < 3 || Cin * H * W < 4 || nt > (two_forms ? 10 : 5) : (W != 14 && W != 28) || nt > 10) return TVX_E_UNSUPPORTED;
   Plan plan{};
   MbTileArgs& a = plan.a;
   a.nt = nt;
@@ -887,10 +888,15 @@ int MbConvSetup(tvx_op* op, const MbStage& ex, const MbStage& dw, const tvx_conv
     // Taken: up to 160 results; of 28 columns only while workgroups are few (batch 13, here and as two or three launches: 32 to 192 to 32 9.2 and 9.9,
     // 64 to 384 to 64 13.1 and 14.2, 96 to 576 to 96 20.9 and 22.8; batch 14 10.1 and 10.2, 14.7 and 14.8; 160 to 160 to 160 batch 5 8.2 and 10.1, 6
     // 13.0 and 10.1; 128 to 768 to 128 14.5 and 16.6, 21.3 and 18.2). Narrow as long as each of its workgroups finds a CU of its own.
+    // The narrow form cares for no width, and what counts is the workgroups: 3 to 56 columns, batch 1 to 64, 480 blocks of the sizes above in front of
+    // the same line take .28 to 1.11 of the time apart, .62 on the average (24 to 144 to 24 on 56 columns, batch 1, 5.5 and 9.1; 64 to 384 to 64 on 12, batch 16, 7.2
+    // and 9.8; 96 to 576 to 96 on 5, batch 8, 7.1 and 10.4; 160 to 160 on 10, batch 1, 9.9 and 9.4, batch 16 11.2 and 15.4); behind it .78 to 1.41. Fewer
+    // chunks than the four wavefronts that walk them leave wavefronts idle: those stay apart but on the widths above.
     const uint64_t narrow_wgs = static_cast<uint64_t>(e->batch) * ((H + 1) / 2) * ((W + 3) / 4), cus = ComputeUnits();
-    wide = W != 28 && nt <= 5 && narrow_wgs > cus;
-    if (const char* f = getenv("TVX_MBCONV_WIDE")) wide = W != 28 && nt <= 5 && atoi(f);  // test lever
-    if (!all && (nt > 5 || (W == 28 && narrow_wgs > (std::max(cin_steps, nt) <= 3 ? 5 : 2) * cus))) return TVX_E_UNSUPPORTED;
+    wide = two_forms && nt <= 5 && narrow_wgs > cus;
+    if (const char* f = getenv("TVX_MBCONV_WIDE")) wide = two_forms && nt <= 5 && atoi(f);  // test lever
+    if (!all && W != 28 && !two_forms && chunks < kMinWaves) return TVX_E_UNSUPPORTED;
+    if (!all && (nt > 5 || (!two_forms && narrow_wgs > (std::max(cin_steps, nt) <= 3 ? 5 : 2) * cus))) return TVX_E_UNSUPPORTED;
     a.W = W; a.batch = e->batch;
     a.half_rows = wide && W == 7 ? 2 : 0;
     a.half_cols = wide && W == 14 ? 7 : 0;
