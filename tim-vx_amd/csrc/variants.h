@@ -48,6 +48,7 @@ int PwRegSetup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 int PwRegF16Setup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 
 // depthwise 3x3 stencil (dwconv3x3_i8.hip)
+int DwManyPlanesSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const void* bias_host);
 int DwConv3x3Setup(tvx_op*, const tvx_conv2d_desc*, const void*, const void*);
 
 // convolutions, whole-plane average pooling and the layout change on channel-blocked tensors (blocked_i8.hip)

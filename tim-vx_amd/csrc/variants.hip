@@ -4,7 +4,7 @@
 namespace tvx {
 
 const std::vector<ConvSetupFn>& ConvVariants() {
-  static const std::vector<ConvSetupFn> v = {DwRegSetup, DwConv3x3Setup, DwPlanesSetup, PwRegSetup, PwRegF16Setup, PwConvSetup, ConvIm2colSetup, ConvBandSetup, ConvIgemmF16Setup, ConvTileSetup, ConvIm2colRestSetup, ConvIgemmSetup, ConvGemmSetup, ConvGenericSetup};
+  static const std::vector<ConvSetupFn> v = {DwRegSetup, DwManyPlanesSetup, DwConv3x3Setup, DwPlanesSetup, PwRegSetup, PwRegF16Setup, PwConvSetup, ConvIm2colSetup, ConvBandSetup, ConvIgemmF16Setup, ConvTileSetup, ConvIm2colRestSetup, ConvIgemmSetup, ConvGemmSetup, ConvGenericSetup};
   return v;
 }
 
