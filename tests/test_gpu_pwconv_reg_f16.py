@@ -50,7 +50,8 @@ def test_an_infinity_stays_with_its_pixel(ks, c, monkeypatch):
 
 
 @pytest.mark.parametrize("n,c,h,w,oc,mine", [(1, 64, 1, 577, 17, True), (1, 64, 24, 24, 17, False), (4, 64, 16, 16, 16, False), (4, 65, 16, 16, 16, True), (3, 64, 15, 17, 16, True),
-                                               (4, 64, 16, 16, 17, True), (2, 300, 31, 37, 40, True), (1, 1025, 25, 25, 20, False)])
+                                               (4, 64, 16, 16, 17, True), (2, 300, 31, 37, 40, True), (1, 1025, 25, 25, 20, False),
+                                               (1, 40, 512, 256, 50, True), (1, 40, 512, 257, 50, True), (1, 70, 363, 362, 49, True)])
 def test_which_layers(oracle, n, c, h, w, oc, mine):
     """More than 576 pixels; of whole cache lines to at most 16 results from at most 64 channels none; at most 1024 channels."""
     x, wt, b, kws = conv_case(np.random.default_rng(8990), mult=0, mode="f16", n=n, c=c, h=h, w=w, oc=oc, kh=1, kw=1, stride=[1, 1], dil=[1, 1], pad=[0] * 4)

@@ -230,9 +230,13 @@ int PwRegF16Setup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   a.tiles = tiles;
   a.act = d->activation;
   // pixel tiles fill the chip, or the output tiles of each are spread over wavefronts: two a SIMD, four where that reads at most 32 channels again
-  // (16 -> 160 on 57 x 85, batch 36: 18.1 us and 14.5; 64 -> 96 on 29 x 29, batch 61: 7.6 and 8.5)
+  // (16 -> 160 on 57 x 85, batch 36: 18.1 us and 14.5; 64 -> 96 on 29 x 29, batch 61: 7.6 and 8.5). Four as well of up to 96 channels
+  // where two would leave the SIMDs with one, if there are four output tiles to spread: 16 drawn layers of 1050 to 1841 pixel tiles .88 of the time, none
+  // slower (64 -> 344 on 139 x 139, batch 8, 33.4 us and 25.5; 92 -> 64 on 105 x 160, batch 8, 12.4 and 11.3); of 512 to 1024 pixel tiles .91 to 1.16
+  // (64 -> 160 on 147 x 147, batch 6, 13.5 and 15.7), of fewer output tiles to 1.2 (80 -> 48 on 99 x 99, batch 14, 9.8 and 11.7).
   const uint64_t pix_tiles = (groups + 15) / 16;
-  uint64_t want = cus * (ks > 1 ? (kr > 4 ? 1 : kr > 2 ? 2 : 4) : kr == 1 ? 16 : 8);
+  const bool four = kr == 1 || (kr <= 3 && tiles >= 4 && pix_tiles > 4 * cus);
+  uint64_t want = cus * (ks > 1 ? (kr > 4 ? 1 : kr > 2 ? 2 : 4) : four ? 16 : 8);
   if (const char* f = getenv("TVX_PWCONV_F16_WAVES")) want = std::max(1, atoi(f));  // test lever
   const uint64_t split = std::min<uint64_t>(tiles, std::max<uint64_t>(1, want / pix_tiles));
   a.tiles_per_wave = static_cast<int>((tiles + split - 1) / split);
