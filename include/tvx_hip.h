@@ -240,8 +240,8 @@ int tvx_conv2d_dw_pw_create(const tvx_conv2d_desc* dw, const void* dw_weights_ho
  * tvx_conv2d_add_create, its other operand going in as in1 of tvx_op_run. Returns TVX_E_UNSUPPORTED when no
  * kernel fuses this block (the kernel covers feature maps of three columns and more, SAME depthwise padding,
  * at most 160 input and 160 output channels (320 on 7 and 14 columns), and by default claims only the blocks where
- * it is faster than the two or three launches: stride 1, up to 160 output channels, and of those the ones of other
- * than 7 and 14 columns on small feature maps or in small batches; the caller then creates the operators one by one). */
+ * it is faster than the two or three launches: stride 1, up to 160 output channels, and of other widths than 7 and 14
+ * columns only small feature maps and small batches; the caller then creates the operators one by one). */
 int tvx_mbconv_create(const tvx_conv2d_desc* expand, const void* expand_weights_host, const void* expand_bias_host,
                       const tvx_conv2d_desc* dw, const void* dw_weights_host, const void* dw_bias_host,
                       const tvx_conv2d_desc* project, const void* project_weights_host, const void* project_bias_host,
