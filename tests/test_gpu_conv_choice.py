@@ -1,5 +1,5 @@
 """Convolutions on both sides of the lines between the tiles and the kernels for few products, short windows and pointwise layers: the kernel that
-takes them, and its results against the oracle, over odd sizes, strides and uneven padding."""
+takes them without a lever, and its results against the oracle, over odd sizes, strides and uneven padding."""
 import numpy as np
 import pytest
 
@@ -25,23 +25,22 @@ LAYERS = [
     # floating point, a handful of products an output
     ("f32", dict(n=2, c=1, h=50, w=60, oc=50, kh=1, kw=1, pad=P0), "conv2d_generic"),                          # 300000 outputs
     ("f32", dict(n=2, c=1, h=50, w=60, oc=51, kh=1, kw=1, pad=P0), "conv2d_tile_f32"),
-    ("f16", dict(n=2, c=3, h=50, w=50, oc=41, kh=1, kw=1, pad=P0), "conv2d_tile_f16"),
+    ("f16", dict(n=2, c=3, h=50, w=50, oc=41, kh=1, kw=1, pad=P0), "pwconv_reg_f16"),                          # (unit stride)
+    ("f16", dict(n=2, c=3, h=99, w=99, oc=41, kh=1, kw=1, stride=[2, 2], pad=P0), "conv2d_tile_f16"),          # 205000
     ("f32", dict(n=1, c=1, h=30, w=41, oc=25, kh=3, kw=3, pad=P1), "conv2d_tile_f32"),                         # 30750 outputs
     ("f16", dict(n=1, c=1, h=29, w=41, oc=25, kh=3, kw=3, pad=P1), "conv2d_generic"),
     ("f32", dict(n=1, c=8, h=9, w=11, oc=12, kh=1, kw=1, pad=P0), "conv2d_tile_f32"),
-    # float16, pointwise
-    ("f16", dict(n=2, c=24, h=13, w=13, oc=24, kh=1, kw=1, pad=P0), "conv2d_gemm_f16"),
-    ("f16", dict(n=2, c=24, h=13, w=13, oc=25, kh=1, kw=1, pad=P0), "conv2d_tile_f16"),
-    ("f16", dict(n=3, c=48, h=14, w=14, oc=40, kh=1, kw=1, pad=P0), "conv2d_tile_f16"),
-    ("f16", dict(n=1, c=144, h=128, w=128, oc=65, kh=1, kw=1, pad=P0), "conv2d_tile_f16"),
+    # float16, pointwise: at unit stride pixels in registers, whatever their number and that of the results
+    ("f16", dict(n=2, c=24, h=13, w=13, oc=24, kh=1, kw=1, pad=P0), "pwconv_reg_f16"),
+    ("f16", dict(n=2, c=24, h=13, w=13, oc=25, kh=1, kw=1, pad=P0), "pwconv_reg_f16"),
+    ("f16", dict(n=3, c=48, h=14, w=14, oc=40, kh=1, kw=1, pad=P0), "pwconv_reg_f16"),
+    ("f16", dict(n=1, c=144, h=128, w=128, oc=65, kh=1, kw=1, pad=P0), "pwconv_reg_f16"),
     ("f16", dict(n=2, c=40, h=15, w=17, oc=33, kh=1, kw=1, stride=[2, 2], pad=P0), "conv2d_tile_f16"),
 ]
 
 
 @pytest.mark.parametrize("mode,layer,kernel", LAYERS)
-def test_conv_choice(oracle, mode, layer, kernel, monkeypatch):
-    if mode == "f16":
-        monkeypatch.setenv("TVX_NO_CONV_IGEMM_F16", "1")   # (asked before both)
+def test_conv_choice(oracle, mode, layer, kernel):
     x, wt, b, kws = conv_case(np.random.default_rng(740), mult=0, mode=mode, **{"stride": [1, 1], "dil": [1, 1], **layer})
     want = oracle.conv2d(x, wt, b, act=1, **kws)
     got = TC.gpu_conv2d(x, wt, b, act=1, want_kernel=kernel, **kws)

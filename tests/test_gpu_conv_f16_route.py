@@ -1,5 +1,5 @@
-"""Which float16 convolutions stay with conv2d_igemm_f16 (pointwise, few results of not too many pixels; 3x3 on many
-rows of 56 pixels or more), and that the kernels on both sides of the line agree with the oracle."""
+"""Which float16 convolutions stay with conv2d_igemm_f16 (3x3 on many rows of 56 pixels or more), which take their pixels in registers (1x1 at unit
+stride), and that the kernels on both sides of the line agree with the oracle."""
 import numpy as np
 import pytest
 
@@ -10,11 +10,11 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("layer,kernel", [
-    (dict(n=2, c=48, h=10, w=10, oc=16, kh=1, kw=1, pad=[0] * 4), "conv2d_igemm_f16"),
-    (dict(n=2, c=48, h=10, w=10, oc=17, kh=1, kw=1, pad=[0] * 4), "conv2d_gemm_f16"),
-    (dict(n=2, c=80, h=9, w=10, oc=17, kh=1, kw=1, pad=[0] * 4), "conv2d_tile_f16"),
+    (dict(n=2, c=48, h=10, w=10, oc=16, kh=1, kw=1, pad=[0] * 4), "pwconv_reg_f16"),
+    (dict(n=2, c=48, h=10, w=10, oc=17, kh=1, kw=1, pad=[0] * 4), "pwconv_reg_f16"),
+    (dict(n=2, c=80, h=9, w=10, oc=17, kh=1, kw=1, pad=[0] * 4), "pwconv_reg_f16"),
     (dict(n=2, c=48, h=10, w=10, oc=16, kh=3, kw=3, pad=[1] * 4), "conv2d_tile_f16"),
-    (dict(n=2, c=48, h=128, w=128, oc=16, kh=1, kw=1, pad=[0] * 4), "conv2d_gemm_f16"),   # 32768 pixels
+    (dict(n=2, c=48, h=128, w=128, oc=16, kh=1, kw=1, pad=[0] * 4), "pwconv_reg_f16"),    # 32768 pixels
     (dict(n=21, c=32, h=56, w=56, oc=8, kh=3, kw=3, pad=[1] * 4), "conv2d_igemm_f16"),
     (dict(n=20, c=32, h=56, w=56, oc=8, kh=3, kw=3, pad=[1] * 4), "conv2d_tile_f16"),     # 62720 pixels
 ])

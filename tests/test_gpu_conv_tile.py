@@ -43,6 +43,7 @@ def test_conv2d_tile(oracle, name, mode, monkeypatch):
     rng = np.random.default_rng(list(CASES).index(name) + 400)
     x, wt, b, kws = conv_case(rng, mult=0, mode=mode, **CASES[name])
     monkeypatch.setenv("TVX_CONV_TILE", "1")
+    monkeypatch.setenv("TVX_PWCONV_F16", "0")   # (asked before the tiles)
     want = oracle.conv2d(x, wt, b, act=1, **kws)
     assert len(np.unique(want)) > 4
     kernel = EARLIER.get(name, KERNEL[mode]) if mode in ("u8", "i8pc") else KERNEL[mode]
@@ -155,7 +156,7 @@ def test_conv2d_pads_wider_than_the_window_by_default(oracle, mode, case):
 
 
 ROUTES = [
-    # mode, layer, kernel: both sides of the lines between the tiles and the kernels asked behind them
+    # mode, layer, kernel: both sides of the lines between the tiles and the kernels asked behind them, as a caller gets them
     ("u8", dict(c=16, h=8, w=8, oc=16, kh=3, kw=3, pad=[1, 1, 1, 1]), "conv2d_igemm_i8"),            # one granule, weights with a zero point
     ("u8", dict(c=17, h=8, w=8, oc=16, kh=3, kw=3, pad=[1, 1, 1, 1]), "conv2d_tile_i8"),
     ("i8pc", dict(c=16, h=8, w=8, oc=16, kh=3, kw=3, pad=[1, 1, 1, 1]), "conv2d_tile_i8"),           # without one
@@ -165,18 +166,16 @@ ROUTES = [
     ("i8pc", dict(c=80, h=9, w=9, oc=66, kh=1, kw=1, pad=[0] * 4, groups=2), "conv2d_tile_i8"),
     ("i8pc", dict(c=8, h=9, w=9, oc=64, kh=1, kw=1, pad=[0] * 4, groups=2), "conv2d_generic"),       # four products a result
     ("i8pc", dict(c=18, h=9, w=9, oc=64, kh=1, kw=1, pad=[0] * 4, groups=2), "conv2d_tile_i8"),
-    ("f16", dict(c=64, h=10, w=10, oc=512, kh=1, kw=1, pad=[0] * 4), "conv2d_gemm_f16"),
-    ("f16", dict(c=64, h=10, w=10, oc=513, kh=1, kw=1, pad=[0] * 4), "conv2d_tile_f16"),
-    ("f16", dict(c=32, h=9, w=9, oc=8, kh=1, kw=1, pad=[0] * 4), "conv2d_gemm_f16"),
-    ("f16", dict(c=144, h=64, w=128, oc=24, kh=1, kw=1, pad=[0] * 4), "conv2d_gemm_f16"),            # 16384 pixels of whole cache lines
-    ("f16", dict(c=144, h=63, w=127, oc=24, kh=1, kw=1, pad=[0] * 4), "conv2d_tile_f16"),
+    ("f16", dict(c=64, h=10, w=10, oc=512, kh=1, kw=1, pad=[0] * 4), "pwconv_reg_f16"),              # (1x1 at unit stride: asked before both)
+    ("f16", dict(c=64, h=10, w=10, oc=513, kh=1, kw=1, pad=[0] * 4), "pwconv_reg_f16"),
+    ("f16", dict(c=32, h=9, w=9, oc=8, kh=1, kw=1, pad=[0] * 4), "pwconv_reg_f16"),
+    ("f16", dict(c=144, h=64, w=128, oc=24, kh=1, kw=1, pad=[0] * 4), "pwconv_reg_f16"),
+    ("f16", dict(c=144, h=63, w=127, oc=24, kh=1, kw=1, pad=[0] * 4), "pwconv_reg_f16"),
 ]
 
 
 @pytest.mark.parametrize("mode,layer,kernel", ROUTES)
-def test_conv2d_tile_or_an_older_kernel(oracle, mode, layer, kernel, monkeypatch):
-    if mode == "f16":
-        monkeypatch.setenv("TVX_NO_CONV_IGEMM_F16", "1")   # (asked before both)
+def test_conv2d_tile_or_an_older_kernel(oracle, mode, layer, kernel):
     x, wt, b, kws = conv_case(np.random.default_rng(720), mult=0, mode=mode, n=2, stride=[1, 1], dil=[1, 1], **layer)
     got = TC.gpu_conv2d(x, wt, b, act=1, want_kernel=kernel, **kws)
     _check(got, oracle.conv2d(x, wt, b, act=1, **kws), mode, kernel)

@@ -827,6 +827,7 @@ def test_conv2d_gemm(oracle, gi, mode, monkeypatch):
     x, wt, b, kws = conv_case(rng, n=n, c=c, h=h, w=w, oc=oc, kh=kh, kw=kw, stride=stride, dil=dil,
                               pad=pad, mult=0, mode=mode, groups=groups if groups > 1 else 0)
     quant = mode != "f16"
+    monkeypatch.setenv("TVX_PWCONV_F16", "0")   # (takes the float16 1x1 case before both)
     if quant and groups == 1 and kh == 1 and kw == 1:
         pytest.skip("the pointwise kernel takes the quantized 1x1 case")
     for act in (0, 2):
@@ -891,6 +892,7 @@ def test_conv2d_igemm_f16(oracle, gi, pixel_tiles, monkeypatch):
     n, c, oc, h, w, kh, kw, stride, pad = IGEMM_F16_GRID[gi]
     monkeypatch.setenv("TVX_CONV_F16_PIXEL_TILES", str(pixel_tiles))   # 128- and 256-pixel workgroups
     monkeypatch.setenv("TVX_CONV_TILE", "0")   # (asked between the two kernels compared)
+    monkeypatch.setenv("TVX_PWCONV_F16", "0")  # (asked before both)
     rng = np.random.default_rng(7600 + gi)
     x, wt, b, kws = conv_case(rng, n=n, c=c, h=h, w=w, oc=oc, kh=kh, kw=kw, stride=[stride, stride], dil=[1, 1],
                               pad=pad, mult=0, mode="f16")

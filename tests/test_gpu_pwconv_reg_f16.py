@@ -49,12 +49,17 @@ def test_an_infinity_stays_with_its_pixel(ks, c, monkeypatch):
     assert np.isfinite(got.transpose(0, 2, 1)[~odd]).all()
 
 
-@pytest.mark.parametrize("n,c,h,w,oc,mine", [(1, 64, 1, 577, 17, True), (1, 64, 24, 24, 17, False), (4, 64, 16, 16, 16, False), (4, 65, 16, 16, 16, True), (3, 64, 15, 17, 16, True),
-                                               (4, 64, 16, 16, 17, True), (2, 300, 31, 37, 40, True), (1, 1025, 25, 25, 20, False),
-                                               (1, 40, 512, 256, 50, True), (1, 40, 512, 257, 50, True), (1, 70, 363, 362, 49, True)])
-def test_which_layers(oracle, n, c, h, w, oc, mine):
-    """More than 576 pixels; of whole cache lines to at most 16 results from at most 64 channels none; at most 1024 channels."""
+@pytest.mark.parametrize("n,c,h,w,oc,mine", [
+    (1, 64, 1, 577, 17, True), (1, 64, 24, 24, 17, True), (4, 64, 16, 16, 16, True), (4, 65, 16, 16, 16, True), (3, 64, 15, 17, 16, True), (4, 64, 16, 16, 17, True),
+    (2, 300, 31, 37, 40, True), (1, 1025, 25, 25, 20, False), (1, 40, 512, 256, 50, True), (1, 40, 512, 257, 50, True), (1, 70, 363, 362, 49, True),
+    # a group of eight pixels, one less; a single result of a handful of pixels and of many; 1024 channels of few
+    (1, 24, 2, 4, 9, True), (9, 24, 1, 7, 9, False), (5, 16, 3, 3, 1, True), (2, 64, 120, 128, 6, True), (3, 1024, 4, 4, 24, True)])
+@pytest.mark.parametrize("levers", [{}, {"TVX_CONV_TILE": "0"}, {"TVX_CONV_TILE": "1"}, {"TVX_NO_CONV_IGEMM_F16": "1", "TVX_NO_CONV_GEMM": "1"}])
+def test_which_layers(oracle, n, c, h, w, oc, mine, levers, monkeypatch):
+    """Planes of eight pixels and more, up to 1024 channels; the levers of the kernels asked behind it are theirs alone."""
+    for k, v in levers.items():
+        monkeypatch.setenv(k, v)
     x, wt, b, kws = conv_case(np.random.default_rng(8990), mult=0, mode="f16", n=n, c=c, h=h, w=w, oc=oc, kh=1, kw=1, stride=[1, 1], dil=[1, 1], pad=[0] * 4)
     want = oracle.conv2d(x, wt, b, act=1, **kws)
-    got = TC.gpu_conv2d(x, wt, b, act=1, want_kernel="pwconv_reg_f16" if mine else ("conv2d_tile_f16", "conv2d_gemm_f16", "conv2d_igemm_f16"), **kws)
+    got = TC.gpu_conv2d(x, wt, b, act=1, want_kernel="pwconv_reg_f16" if mine else ("conv2d_tile_f16", "conv2d_gemm_f16", "conv2d_igemm_f16", "conv2d_generic"), **kws)
     assert np.allclose(got.astype(np.float32), want.astype(np.float32), rtol=5e-3, atol=2e-2)

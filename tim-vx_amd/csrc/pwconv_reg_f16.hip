@@ -10,7 +10,9 @@
 //  - Channels that do not exist are zero (their weights are too, but a channel read in their place may hold an infinity).
 // Bound by memory where results are many, by the chain load - pair - multiply - store where few. Against the window in LDS (conv_tile.hip) and the
 // gathered windows (conv_gemm.hip): 70 drawn layers .63 of the time, none slower: 20 -> 144 on 9344 pixels, batch 40, 56.7 -> 21.7 us (122 MB, floor
-// 24.5 at a copy's rate), 464 -> 156 on 77 x 110, batch 15, 88 -> 52, 416 -> 48 on 39 x 39, batch 24, 15.9 -> 11.1, 40 -> 24 on 15 x 15 5.2 -> 3.0.
+// 24.5 at a copy's rate), 464 -> 156 on 77 x 110, batch 15, 88 -> 52, 416 -> 48 on 39 x 39, batch 24, 15.9 -> 11.1. 191 layers of at most 576 pixels .59 (56 ->
+// 382 on 6 x 6 7.2 -> 2.5; the slowest 848 -> 8 on 12 pixels, batch 13, 5.7 -> 5.8), 110 of at most 16 results from at most 64 channels on planes of
+// whole 16 pixels .42 (16 -> 8 on 88 x 88, batch 8, 3.9 -> 3.1; 64 -> 6 on 15200 pixels, batch 20, 162 by a thread per output, 8.4).
 // Reference: src/tim/vx/ops/conv2d.cc (1x1 kernels).
 #include <algorithm>
 #include <cstdlib>
@@ -186,7 +188,7 @@ uint32_t Magic(uint64_t d) { return d <= 1 ? 0u : static_cast<uint32_t>(((uint64
 
 }  // namespace
 
-// Claims dense float16 1x1 convolutions with unit stride, no padding and constant weights of up to 1024 channels.
+// Claims dense float16 1x1 convolutions with unit stride, no padding and constant weights of up to 1024 channels on planes of eight pixels and more.
 int PwRegF16Setup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const void* bias_host) {
   if (op->kind != OP_CONV2D || !w_host || d->multiplier != 0 || d->groups > 1 || op->fused_add || op->fused_pool) return TVX_E_UNSUPPORTED;
   if (d->in_dtype != TVX_F16 || d->w_dtype != TVX_F16 || d->out_dtype != TVX_F16) return TVX_E_UNSUPPORTED;
@@ -202,14 +204,9 @@ int PwRegF16Setup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   // and 8.6; 64 -> 96 on 29 x 29, batch 61, 4800, 8.9 and 7.8.
   const uint64_t cus = ComputeUnits(), pieces = (pixels + 63) / 64 * tiles;
   int ks = ksteps <= 4 && 2 * pieces > 7 * cus * ksteps ? 1 : 4;
-  const char* lever = getenv("TVX_PWCONV_F16");  // test lever: wavefronts that share a reduction; 0 declines
-  if (lever) {
-    ks = atoi(lever);
+  if (const char* f = getenv("TVX_PWCONV_F16")) {  // test lever: wavefronts that share a reduction; 0 declines
+    ks = atoi(f);
     if ((ks != 1 && ks != 4) || (ks == 1 && ksteps > 4)) return TVX_E_UNSUPPORTED;
-  } else if (getenv("TVX_CONV_TILE") || getenv("TVX_NO_CONV_IGEMM_F16") || getenv("TVX_NO_CONV_GEMM")) {
-    return TVX_E_UNSUPPORTED;  // (levers of the kernels asked behind this one)
-  } else if (pixels <= 576 || (OC <= 16 && C <= 64 && hw % 16 == 0)) {
-    return TVX_E_UNSUPPORTED;  // (these are asked for by the names of the kernels behind this one)
   }
   const int pw = ks == 1 ? 8 : 4;
   int kr = (ksteps + ks - 1) / ks;
