@@ -36,6 +36,12 @@ LAYERS = [
     ("f16", dict(n=3, c=48, h=14, w=14, oc=40, kh=1, kw=1, pad=P0), "pwconv_reg_f16"),
     ("f16", dict(n=1, c=144, h=128, w=128, oc=65, kh=1, kw=1, pad=P0), "pwconv_reg_f16"),
     ("f16", dict(n=2, c=40, h=15, w=17, oc=33, kh=1, kw=1, stride=[2, 2], pad=P0), "conv2d_tile_f16"),
+    # ... strided: few channels and results, results too few for a matrix tile, few results of more channels
+    ("f16", dict(n=7, c=24, h=16, w=16, oc=16, kh=1, kw=1, stride=[2, 2], pad=P0), "conv2d_gemm_f16"),
+    ("f16", dict(n=7, c=24, h=16, w=16, oc=7, kh=1, kw=1, stride=[2, 2], pad=P0), "conv2d_tile_f16"),
+    ("f16", dict(n=2, c=32, h=19, w=17, oc=8, kh=1, kw=1, stride=[2, 2], pad=P0), "conv2d_gemm_f16"),
+    ("f16", dict(n=2, c=32, h=19, w=17, oc=9, kh=1, kw=1, stride=[2, 2], pad=P0), "conv2d_tile_f16"),
+    ("f16", dict(n=1, c=48, h=62, w=62, oc=11, kh=1, kw=1, stride=[2, 2], pad=P0), "conv2d_tile_f16"),
 ]
 
 

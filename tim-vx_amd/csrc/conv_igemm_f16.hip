@@ -255,18 +255,16 @@ int ConvIgemmF16Setup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, 
   if (d->in_c % 16 || d->in_c > 16 * kMaxSteps || (d->in_w & 1) || d->k_w > 11 || d->k_h > 11) return TVX_E_UNSUPPORTED;
   if (const char* f = getenv("TVX_NO_CONV_IGEMM_F16"))  // tuning aid: leaves float16 convolutions to conv2d_gemm_f16
     if (atoi(f)) return TVX_E_UNSUPPORTED;
-  // The tiles and conv2d_gemm_f16, asked behind this one, are ahead nearly everywhere: on 123 drawn layers that this kernel could take they
-  // needed 0.75 of its time (median; 80 -> 112, 7x7 on 23 x 18, batch 3, 38.0 -> 8.9 us, 96 -> 256, 1x1 on 68 x 68, batch 11, 28.2 -> 17.0), but for
-  // pointwise layers with few results and not too many pixels (64 -> 8 on 54 x 54, batch 10, 4.8 against 6.8; 96 -> 16 on 84 x 84, batch 38, 25.7
-  // against 16.1) and many rows of at least 56 pixels under 3x3 taps and 32 to 64 channels with few results (batch 32, 56 x 56: 32 -> 16 10.6 against
+  // The kernels asked beside this one are ahead nearly everywhere: on 123 drawn layers that this kernel could take they needed 0.75 of its time
+  // (median; 80 -> 112, 7x7 on 23 x 18, batch 3, 38.0 -> 8.9 us; strided 1x1, 64 -> 13 on 64 x 64, batch 13, 6.2 -> 4.8), but for many rows of at least 56
+  // pixels under 3x3 taps and 32 to 64 channels with few results (batch 32, 56 x 56: 32 -> 16 10.6 against
   // 12.9, 64 -> 32 16.5 against 21.1, 64 -> 64 22.8 against 24.3; on the other side of that line 16 -> 16 at batch 64 13.6 against 12.9, 96 -> 16
   // 46.8 against 41.7, 64 -> 128 at batch 32 38.9 against 38.5, 64 -> 64 at batch 22 21.3 against 19.2, 64 -> 16 on 28 x 28, batch 96, 14.9 against 14.6).
   const uint64_t pixels = static_cast<uint64_t>(d->batch) * d->out_w * d->out_h, cu = ComputeUnits();  // (the lines were drawn on 256 of them)
-  const bool few = d->k_w == 1 && d->k_h == 1 && d->in_c >= 48 && d->out_c <= 16 && pixels < 128 * cu;
   const bool rows = d->k_w == 3 && d->k_h == 3 && d->stride_w == 1 && d->in_c >= 32 && d->in_c <= 64 && d->out_w >= 56 && d->out_c <= 64 &&
                     pixels >= (d->out_c <= 32 ? 256 : 384) * cu;
   const char* const tiles = getenv("TVX_CONV_TILE");  // (its lever 0 leaves the tiles' layers to the kernels before them)
-  if (!few && !rows && !(tiles && atoi(tiles) == 0)) return TVX_E_UNSUPPORTED;
+  if (!rows && !(tiles && atoi(tiles) == 0)) return TVX_E_UNSUPPORTED;
   Plan plan{};
   FcvArgs& a = plan.a;
   a.C = d->in_c; a.H = d->in_h; a.W = d->in_w; a.OC = d->out_c; a.OH = d->out_h; a.OW = d->out_w;

@@ -787,6 +787,7 @@ static bool IsBetterChoice(const tvx_conv2d_desc* d, int dt, bool sums) {
   const int groups = d->groups > 1 ? d->groups : 1, ocg = d->out_c / groups;
   const uint64_t reduction = static_cast<uint64_t>(d->in_c / groups) * d->k_w * d->k_h;
   const uint64_t outputs = static_cast<uint64_t>(d->out_c) * d->out_w * d->out_h * d->batch, macs = reduction * outputs;
+  const uint64_t cus = ComputeUnits();
   const bool pointwise = d->k_w == 1 && d->k_h == 1;
   // a group of three output channels and fewer fills less than a tenth of a tile's 32 channels: only where each has little to add up
   // (float16 432 -> 12 in four groups, 7x7 on 42 x 42, batch 28: 2495 us with one thread per output, 140 here)
@@ -803,21 +804,12 @@ static bool IsBetterChoice(const tvx_conv2d_desc* d, int dt, bool sums) {
   // 17.4 us, 240 -> 96 on 74 x 74, batch 49: 36.8 against 52.3); with more than 32 channels in a group the tiles (144 -> 128 in two on
   // 29889 pixels: 9.5 against 16.8)
   if (dt == kI8 && groups > 1 && pointwise && reduction >= 32 && reduction <= 128 && ocg >= 8 && ocg <= 32) return false;
-  // float16 1 x 1: conv2d_gemm_f16 has less to set up, and gathers four pixels a load where planes are whole quads. Few channels and few results
-  // (16 -> 24 on 46 x 46: 4.6 against 5.1 us), in quads also many pixels (24 -> 56 on 44 x 44, batch 18, 5.6 against 6.4; with fewer the tiles: 48 -> 40
-  // on 14 x 14, batch 22, 7.7 against 5.2). Its rows are cache lines where a plane is a multiple of sixteen pixels: there also up to 64 channels and
-  // 50 M products (56 -> 48 on 20 x 20, batch 31, 5.1 against 5.5) and deep inputs to few results of many pixels (352 -> 32 on 156 x 156, batch 10, 48.4
-  // against 49.9; to more results the tiles: 400 -> 66 on 84 x 84, batch 5, 21.9 against 17.1). 69 drawn layers .93 of the time under lines by
-  // products alone, .90 with the better kernel for each.
-  if (dt == kF16 && groups == 1 && pointwise && d->in_c >= 16) {
-    const uint64_t plane = static_cast<uint64_t>(d->in_w) * d->in_h, pixels = plane * d->batch;
-    if (macs <= 4000000 && ((d->in_c <= 24 && d->out_c <= 24) || (d->in_c <= 32 && d->out_c <= 8))) return false;
-    if (d->stride_w == 1 && d->stride_h == 1 && plane % 4 == 0) {
-      if (d->in_c <= 32 && (macs <= 4000000 || d->out_c <= 24 || pixels >= 30000)) return false;
-      if (d->in_c <= 64 && ((d->out_c <= 24 && pixels >= 16384) || (plane % 16 == 0 && macs <= 50000000) || (d->out_c <= 512 && pixels <= 256))) return false;
-      if (plane % 16 == 0 && d->in_c >= 144 && d->out_c <= 64 && pixels >= 16384) return false;
-    }
-  }
+  // float16 1 x 1 that pwconv_reg_f16, asked in front, leaves (strided ones, mostly): conv2d_gemm_f16 has less to set up where channels and results are
+  // few (24 -> 16 on 16 x 16 at stride 2, batch 7, 4.1 against 4.8 us; 32 -> 8 on 144 x 144 at stride 2, batch 2, 4.2 against 4.5). It takes eight
+  // results and more; fewer would go to a thread per output (32 -> 5 on 9 x 9 at stride 2, batch 3, 14.7 against 4.8). 260 drawn strided layers 1.005 of the
+  // time with the better kernel for each, 160 of more than 1024 channels 1.000.
+  if (dt == kF16 && groups == 1 && pointwise && d->in_c >= 16 && d->out_c >= 8 && macs <= 16000 * cus && ((d->in_c <= 24 && d->out_c <= 24) || (d->in_c <= 32 && d->out_c <= 8)))
+    return false;
   if (dt == kI8 && groups == 1) {
     if (ConvIgemmPersists(d)) return false;
     // a granule of channels under weights with a zero point: up to two million products conv2d_igemm_i8, whose chain is short on small planes and on
