@@ -13,6 +13,19 @@ LAYERS = [(1, 1, 2, 4, 1), (3, 8, 3, 3, 17), (2, 31, 5, 5, 16), (1, 32, 16, 8, 3
           (3, 40, 1, 41, 130), (2, 129, 6, 7, 20), (1, 200, 8, 8, 96), (2, 260, 5, 7, 31), (1, 515, 4, 5, 64), (2, 777, 3, 4, 18), (1, 1024, 3, 3, 16)]
 
 
+def _exact(x, wt, b, act):
+    """The convolution in 64 bits; by how much a result may be off: c + 1 additions of float32, each by at most a unit of its last place of what the
+    magnitudes add up to, and half a unit of float16's last place; and the convolution without its last channel."""
+    x, wt, b = x.astype(np.float64), wt.astype(np.float64), b.astype(np.float64)[:, None]
+    c = wt.shape[1]
+
+    def activated(v):
+        return v if act == 0 else np.clip(v, 0, None if act == 1 else 6)
+    exact, lost = wt @ x + b, wt[:, :-1] @ x[:, :-1] + b
+    bound = (c + 1) * 2.0 ** -23 * (np.abs(wt) @ np.abs(x) + np.abs(b))
+    return activated(exact), bound + 2.0 ** -11 * (np.abs(exact) + bound) + 2.0 ** -25, activated(lost)
+
+
 @pytest.mark.parametrize("act", [0, 1, 2])
 @pytest.mark.parametrize("ks", [1, 4])
 @pytest.mark.parametrize("layer", LAYERS)
@@ -23,13 +36,14 @@ def test_pointwise_f16_in_registers(oracle, layer, ks, act, monkeypatch):
     rng = np.random.default_rng(8800 + c + oc)
     x, wt, b, kws = conv_case(rng, mult=0, mode="f16", n=n, c=c, h=h, w=w, oc=oc, kh=1, kw=1, stride=[1, 1], dil=[1, 1], pad=[0] * 4)
     monkeypatch.setenv("TVX_PWCONV_F16", str(ks))
-    want = oracle.conv2d(x, wt, b, act=act, **kws)
+    want = oracle.conv2d(x, wt, b, act=act, **kws).astype(np.float64).reshape(n, oc, h * w)
+    exact, bound, lost = _exact(x.reshape(n, c, h * w), wt.reshape(oc, c), b, act)
+    assert (np.abs(want - exact) <= bound).all()
     for waves in (1, 1 << 20):   # all output tiles after one another, each by itself
         monkeypatch.setenv("TVX_PWCONV_F16_WAVES", str(waves))
-        got = TC.gpu_conv2d(x, wt, b, act=act, want_kernel="pwconv_reg_f16", **kws)
-        # a float32 sum's rounding (c 2^-24 of the products' magnitudes) far below that of the result, 2^-11
-        magnitude = np.abs(x.astype(np.float64)).max() * np.abs(wt.astype(np.float64)).max() * c
-        assert np.abs(got.astype(np.float64) - want.astype(np.float64)).max() <= 2.0 ** -10 * max(np.abs(want.astype(np.float64)).max(), 2.0 ** -14) + c * 2.0 ** -23 * magnitude
+        got = TC.gpu_conv2d(x, wt, b, act=act, want_kernel="pwconv_reg_f16", **kws).astype(np.float64).reshape(n, oc, h * w)
+        assert (np.abs(got - exact) <= bound).all(), np.max(np.abs(got - exact) / bound)
+        assert c == 1 or act or (np.abs(got - lost) > bound).mean() > 0.5   # (the bound tells the sum from one without its last channel)
 
 
 @pytest.mark.parametrize("ks,c", [(1, 13), (1, 100), (4, 133)])
