@@ -1,5 +1,5 @@
 """Which kernel takes a quantized depthwise 3x3 layer of rows that are whole dwords, on both sides of the lines by planes, and the four- and
-eight-column forms on either side of theirs. Exact against the oracle."""
+eight-column forms on either side of theirs (at 256 compute units). Exact against the oracle."""
 import numpy as np
 import pytest
 
@@ -14,7 +14,11 @@ pytestmark = pytest.mark.gpu
     (6, 1000, 16, 16, 1, "dwconv_rows_i8"), (6, 999, 16, 16, 1, "dwconv3x3_i8"),
     (12, 1000, 20, 20, 1, "dwconv_rows_i8"), (12, 1000, 21, 20, 1, "dwconv3x3_i8"),
     (4, 1000, 16, 16, 2, "dwconv_rows_i8"), (6, 1000, 32, 32, 2, "dwconv_rows_i8"), (6, 999, 32, 32, 2, "dwconv3x3_i8"),
-    (2, 3, 9, 56, 1, "dwconv3x3_i8"), (16, 192, 53, 56, 1, "dwconv3x3_i8"), (1, 5, 9, 88, 1, "dwconv3x3_i8"), (1, 5, 9, 96, 1, "dwconv3x3_i8")])
+    (2, 3, 9, 56, 1, "dwconv3x3_i8"), (1, 5, 9, 88, 1, "dwconv3x3_i8"), (1, 5, 9, 96, 1, "dwconv3x3_i8"),
+    # tall planes; many results, without window sums (even batches) and with them
+    (2, 3, 95, 16, 1, "dwconv3x3_i8"), (1, 3, 96, 16, 1, "dwconv3x3_i8_eight"), (1, 2, 130, 224, 1, "dwconv3x3_i8_eight"), (2, 3, 97, 20, 1, "dwconv3x3_i8"),
+    (2, 1000, 53, 56, 1, "dwconv3x3_i8"), (16, 128, 53, 56, 1, "dwconv3x3_i8_eight"), (15, 128, 53, 56, 1, "dwconv3x3_i8"), (53, 128, 53, 56, 1, "dwconv3x3_i8_eight"),
+    (2, 3, 192, 16, 2, "dwconv3x3_i8")])
 def test_depthwise_choice(oracle, n, c, h, w, stride, kernel):
     pad = [1, 1, 1, 1] if stride == 1 else [0, 1, 0, 1]
     rng = np.random.default_rng(9500 + h * w + n)

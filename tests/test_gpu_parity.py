@@ -719,43 +719,48 @@ DW_GRID = [
 
 
 @pytest.mark.parametrize("mode", ["u8", "i8pc", "u8pc"])
-@pytest.mark.parametrize("gi", range(len(DW_GRID)))
-def test_depthwise3x3_shapes(oracle, gi, mode):
+@pytest.mark.parametrize("gi,cols", [(gi, None) for gi in range(len(DW_GRID))] + [(gi, "8") for gi in (0, 5, 6, 7, 8)])
+def test_depthwise3x3_shapes(oracle, gi, cols, mode, monkeypatch):
+    """Every shape as it is planned, and rows of whole 8-byte units with eight columns per thread too (small layers of low planes are planned
+    with four)."""
     n, c, h, w, s, pad = DW_GRID[gi]
+    if cols:
+        monkeypatch.setenv("TVX_DWCONV_COLS", cols)
     rng = np.random.default_rng(3000 + gi)
     x, wt, b, kws = conv_case(rng, n=n, c=c, h=h, w=w, oc=0, kh=3, kw=3, stride=[s, s], dil=[1, 1],
                               pad=pad, mult=1, mode=mode)
     fast = kws["out_shape"][0] % 4 == 0
     for act in (0, 2):
         want = oracle.conv2d(x, wt, b, act=act, **kws)
-        got = TC.gpu_conv2d(x, wt, b, act=act, want_kernel="dwconv3x3_i8" if fast else "dwconv_planes_i8", **kws)
+        got = TC.gpu_conv2d(x, wt, b, act=act, want_kernel="dwconv3x3_i8" if fast else "dwconv_planes_i8",
+                            want_variant="dwconv3x3_i8_eight" if cols or gi == 7 else None, **kws)
         assert np.array_equal(got, want)
 
 
 @pytest.mark.parametrize("gi", [0, 6, 7, 8])
 def test_depthwise3x3_four_columns_per_thread_on_wide_rows(oracle, gi, monkeypatch):
-    """The four-column form on shapes that would take the eight-column one (it is what runs there when a tensor
-    is not 8-byte aligned)."""
+    """The four-column form on rows of whole 8-byte units, one of them (a tall plane) of its own accord on eight columns."""
     n, c, h, w, s, pad = DW_GRID[gi]
     monkeypatch.setenv("TVX_DWCONV_COLS", "4")
     rng = np.random.default_rng(3100 + gi)
     x, wt, b, kws = conv_case(rng, n=n, c=c, h=h, w=w, oc=0, kh=3, kw=3, stride=[s, s], dil=[1, 1],
                               pad=pad, mult=1, mode="u8")
     want = oracle.conv2d(x, wt, b, act=2, **kws)
-    got = TC.gpu_conv2d(x, wt, b, act=2, want_kernel="dwconv3x3_i8", **kws)
+    got = TC.gpu_conv2d(x, wt, b, act=2, want_kernel="dwconv3x3_i8", want_variant="dwconv3x3_i8", **kws)
     assert np.array_equal(got, want)
 
 
-@pytest.mark.parametrize("gi", [0, 6, 8])
-def test_depthwise3x3_tensors_off_the_eight_byte_grid(oracle, gi):
+@pytest.mark.parametrize("gi", [0, 6, 7, 8])
+def test_depthwise3x3_tensors_off_the_eight_byte_grid(oracle, gi, monkeypatch):
     """Tensors that start four bytes into their allocations: the operator planned for 64-bit row loads has to
     take its four-column form at run time."""
     n, c, h, w, s, pad = DW_GRID[gi]
+    monkeypatch.setenv("TVX_DWCONV_COLS", "8")
     rng = np.random.default_rng(3200 + gi)
     x, wt, b, kws = conv_case(rng, n=n, c=c, h=h, w=w, oc=0, kh=3, kw=3, stride=[s, s], dil=[1, 1],
                               pad=pad, mult=1, mode="u8")
     want = oracle.conv2d(x, wt, b, act=0, **kws)
-    got = TC.gpu_conv2d(x, wt, b, act=0, want_kernel="dwconv3x3_i8", misalign=4, **kws)
+    got = TC.gpu_conv2d(x, wt, b, act=0, want_kernel="dwconv3x3_i8", want_variant="dwconv3x3_i8_eight", misalign=4, **kws)
     assert np.array_equal(got, want)
     assert len(np.unique(want)) > 4
 

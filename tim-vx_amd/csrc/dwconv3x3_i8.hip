@@ -390,20 +390,20 @@ int DwConv3x3Setup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, con
   a.rq = op->aux2.as<tvx_v4i>();
   a.C = C; a.H = d->in_h; a.W = d->in_w; a.OH = d->out_h; a.OW = d->out_w;
   a.pad_t = d->pad_top; a.pad_l = d->pad_left;
-  // Eight columns per thread (stride 1, rows that are whole 8-byte units): one 64-bit load per input row and lane. On long rows, and on many of
-  // middle length; a wavefront of short rows has half as many lanes with eight, and a longer chain. Captured, four over eight, by planes:
-  //                32    192    576   1536   3072   6144  15360
-  //   16 x 16     .78    .79    .59    .68    .59    .61    .60    (15360: 16.3 -> 9.8 us)
-  //   32 x 32     .72    .73    .83    .79    .76    .72    .67
-  //   48 x 48     .85    .83    .86    .79    .88    .84    .89    (15360: 27.4 -> 24.5)
-  //   64 x 64     .82    .83    .86    .88    .98    .97
-  //   80 x 80     .83    .89    .98    .98   1.02   1.08
-  //  112 x 112   1.06   1.04   1.00   1.06   1.04
-  const uint64_t pixels = static_cast<uint64_t>(d->batch) * C * d->out_w * d->out_h;
-  int cols = S == 1 && (d->in_w & 7) == 0 && (d->out_w & 7) == 0 && (d->out_w >= 96 || (d->out_w >= 56 && pixels >= 9000000)) ? 8 : 4;
+  // Eight columns per thread (stride 1, rows that are whole 8-byte units): one 64-bit load per input row and lane. A wavefront of short rows has half as
+  // many lanes with eight, and a longer chain. Captured, four over eight, 770 layers:
+  //   planes of 96 rows and more (below: eight rows of four columns a thread, or four of eight), 16 to 224 columns, 32 to 3072 planes: 1.00 to 1.11, mean 1.05;
+  //   lower planes of up to 55 columns: .59 to .97 (15360 of 16 x 16 9.8 and 16.3 us);
+  //   lower planes of wider rows, by results in millions, means:   to 1    4    6     9    13    20    26    40  above
+  //                                               no window sums    .93  .96  .96  1.03  1.04  1.02  1.06  1.08  1.10
+  //                                               window sums       .84  .88  .88   .94   .98   .96  1.01  1.03  1.06
+  // The line is drawn at 6 and at 20 million on 256 compute units: 1.004 of the time with the better form for each, and 1.002.
+  const uint64_t results = static_cast<uint64_t>(d->batch) * C * d->out_w * d->out_h, cus = ComputeUnits();
+  const bool wide_rows = S == 1 && (d->in_w & 7) == 0 && (d->out_w & 7) == 0;
+  int cols = wide_rows && (d->out_h >= 96 || (d->out_w >= 56 && results >= (any_box ? 78000 : 23500) * cus)) ? 8 : 4;
   if (const char* f = getenv("TVX_DWCONV_COLS")) {  // tuning aid: output columns per thread
     if (atoi(f) == 4) cols = 4;
-    if (atoi(f) == 8 && S == 1 && (d->in_w & 7) == 0 && (d->out_w & 7) == 0) cols = 8;
+    if (atoi(f) == 8 && wide_rows) cols = 8;
   }
   auto shape_for = [&](int cw) {
     Shape sh{};
@@ -440,6 +440,7 @@ int DwConv3x3Setup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, con
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&p), reinterpret_cast<const uint8_t*>(&p) + sizeof(p));
   op->run = DwRun;
   op->kernel_name = "dwconv3x3_i8";
+  if (cols == 8) op->variant = "dwconv3x3_i8_eight";  // (of tensors at multiples of eight bytes)
   return TVX_OK;
 }
 
