@@ -1,5 +1,5 @@
 """Convolutions on both sides of the lines between the tiles and the kernels for few products, short windows and pointwise layers: the kernel that
-takes them without a lever, and its results against the oracle, over odd sizes, strides and uneven padding."""
+takes them without a lever (at 256 compute units), and its results against the oracle, over odd sizes, strides and uneven padding."""
 import numpy as np
 import pytest
 
@@ -27,8 +27,10 @@ LAYERS = [
     ("f32", dict(n=2, c=1, h=50, w=60, oc=51, kh=1, kw=1, pad=P0), "conv2d_tile_f32"),
     ("f16", dict(n=2, c=3, h=50, w=50, oc=41, kh=1, kw=1, pad=P0), "pwconv_reg_f16"),                          # (unit stride)
     ("f16", dict(n=2, c=3, h=99, w=99, oc=41, kh=1, kw=1, stride=[2, 2], pad=P0), "conv2d_tile_f16"),          # 205000
-    ("f32", dict(n=1, c=1, h=30, w=41, oc=25, kh=3, kw=3, pad=P1), "conv2d_tile_f32"),                         # 30750 outputs
+    ("f32", dict(n=1, c=1, h=30, w=41, oc=25, kh=3, kw=3, pad=P1), "conv2d_generic"),                          # 30750 outputs
     ("f16", dict(n=1, c=1, h=29, w=41, oc=25, kh=3, kw=3, pad=P1), "conv2d_generic"),
+    ("f32", dict(n=4, c=1, h=30, w=46, oc=25, kh=3, kw=3, pad=P1), "conv2d_generic"),                          # 138000
+    ("f16", dict(n=4, c=1, h=30, w=47, oc=25, kh=3, kw=3, pad=P1), "conv2d_tile_f16"),                         # 141000
     ("f32", dict(n=1, c=8, h=9, w=11, oc=12, kh=1, kw=1, pad=P0), "conv2d_tile_f32"),
     # float16, pointwise: at unit stride pixels in registers, whatever their number and that of the results
     ("f16", dict(n=2, c=24, h=13, w=13, oc=24, kh=1, kw=1, pad=P0), "pwconv_reg_f16"),
