@@ -31,7 +31,13 @@ def test_widths(oracle, monkeypatch, ci, mode):
 
 @pytest.mark.parametrize("n,cin,cexp,cout,h,w,taken", [
     (1, 24, 128, 24, 12, 12, True), (1, 24, 96, 24, 12, 12, False), (1, 24, 128, 24, 12, 2, False), (1, 64, 128, 161, 12, 12, False),
-    (40, 24, 128, 24, 16, 16, True), (41, 24, 128, 24, 16, 16, False), (16, 128, 128, 32, 16, 16, True), (17, 128, 128, 32, 16, 16, False)])
+    (40, 24, 128, 24, 16, 16, True), (41, 24, 128, 24, 16, 16, False), (16, 128, 128, 32, 16, 16, True), (17, 128, 128, 32, 16, 16, False),
+    # many chunks of more than three steps: a second workgroup of a CU just begun, one small image whose planes are whole dwords and whose rows are not
+    (33, 160, 960, 160, 8, 8, False), (32, 160, 960, 160, 8, 8, True), (40, 160, 960, 160, 8, 8, True), (33, 160, 768, 160, 8, 8, True), (15, 160, 960, 160, 12, 12, True),
+    (4, 128, 768, 128, 24, 24, False), (5, 128, 768, 128, 24, 24, True), (5, 160, 960, 160, 24, 24, False), (7, 160, 960, 160, 24, 24, True),
+    (4, 96, 960, 96, 24, 24, True),
+    (1, 160, 960, 160, 10, 10, False), (2, 160, 960, 160, 10, 10, True), (1, 160, 800, 160, 10, 10, True), (1, 160, 960, 160, 7, 6, True), (1, 160, 960, 160, 9, 12, True),
+    (1, 160, 960, 160, 12, 9, False), (1, 160, 960, 160, 18, 18, True), (1, 160, 960, 160, 14, 14, True), (1, 160, 960, 160, 7, 7, True)])
 def test_blocks_taken_by_workgroups(n, cin, cexp, cout, h, w, taken):
     """Both sides of the rule's lines, at 256 compute units."""
     import torch

@@ -858,7 +858,7 @@ int MbConvSetup(tvx_op* op, const MbStage& ex, const MbStage& dw, const tvx_conv
   const int cin_steps = (Cin + 31) / 32, chunks = (Cexp + 31) / 32, nt = (Cout + 31) / 32;
   if (cin_steps > kMaxCinSteps) return TVX_E_UNSUPPORTED;
   const bool two_forms = W == 7 || W == 14;
-  if (S == 1 ? W < 3 || Cin * H * W < 4 || nt > (two_forms ? 10 : 5) : (W != 14 && W != 28) || nt > 10) return TVX_E_UNSUPPORTED;
+  if (S == 1 ? W < 3 || static_cast<uint64_t>(Cin) * H * W < 4 || nt > (two_forms ? 10 : 5) : (W != 14 && W != 28) || nt > 10) return TVX_E_UNSUPPORTED;
   Plan plan{};
   MbTileArgs& a = plan.a;
   a.nt = nt;
@@ -889,13 +889,24 @@ int MbConvSetup(tvx_op* op, const MbStage& ex, const MbStage& dw, const tvx_conv
     // 64 to 384 to 64 13.1 and 14.2, 96 to 576 to 96 20.9 and 22.8; batch 14 10.1 and 10.2, 14.7 and 14.8; 160 to 160 to 160 batch 5 8.2 and 10.1, 6
     // 13.0 and 10.1; 128 to 768 to 128 14.5 and 16.6, 21.3 and 18.2). Narrow as long as each of its workgroups finds a CU of its own.
     // The narrow form cares for no width, and what counts is the workgroups: 3 to 56 columns, batch 1 to 64, 480 blocks of the sizes above in front of
-    // the same line take .28 to 1.11 of the time apart, .62 on the average (24 to 144 to 24 on 56 columns, batch 1, 5.5 and 9.1; 64 to 384 to 64 on 12, batch 16, 7.2
-    // and 9.8; 96 to 576 to 96 on 5, batch 8, 7.1 and 10.4; 160 to 160 on 10, batch 1, 9.9 and 9.4, batch 16 11.2 and 15.4); behind it .78 to 1.41. Fewer
+    // the same line take .62 of the time apart on the average (24 to 144 to 24 on 56 columns, batch 1, 5.5 and 9.1; 64 to 384 to 64 on 12, batch 16, 7.2
+    // and 9.8; 96 to 576 to 96 on 5, batch 8, 7.1 and 10.4; 160 to 160 on 10, batch 16, 11.2 and 15.4); behind it .78 to 1.41. Fewer
     // chunks than the four wavefronts that walk them leave wavefronts idle: those stay apart but on the widths above.
+    // In front of the line the parts are ahead in blocks of more than three steps (96 channels) and many chunks only, measured on 1600 of them:
+    //  - a second workgroup of a CU has just begun, and the rows are those that dwconv3x3_i8 is best at: 160 to 960 to 160 on 8 columns, 264 to 288 workgroups,
+    //    1.06 to 1.10 of the time apart (320 and more below 1), on 24 to 56 (wholes of eight), 288 to 400, 1.03 to 1.18 (448 and more below .95);
+    //    of 20 to 24 chunks on 24 and 48 columns, 288, 1.00 to 1.13. Rows of 12, 20, 36: .82 to .99.
+    //  - one small image whose rows are no whole dwords but whose planes are: 6 x 6 1.08 to 1.11, 10 x 10 1.05 to 1.07, 12 x 9 1.04 to 1.06 with 30 chunks
+    //    (25 .95 to 1.01; 7 x 6, planes of no whole dwords, .95 to .99; 18 x 18 .95).
     const uint64_t narrow_wgs = static_cast<uint64_t>(e->batch) * ((H + 1) / 2) * ((W + 3) / 4), cus = ComputeUnits();
     wide = two_forms && nt <= 5 && narrow_wgs > cus;
     if (const char* f = getenv("TVX_MBCONV_WIDE")) wide = two_forms && nt <= 5 && atoi(f);  // test lever
     if (!all && W != 28 && !two_forms && chunks < kMinWaves) return TVX_E_UNSUPPORTED;
+    const bool deep = std::max(cin_steps, nt) > 3, eights = W % 8 == 0;
+    if (!all && deep && !two_forms && eights && narrow_wgs > cus &&
+        ((5 * narrow_wgs <= 6 * cus && (chunks > 24 || (chunks >= 20 && W >= 24))) || (5 * narrow_wgs <= 8 * cus && chunks > 24 && W >= 24)))
+      return TVX_E_UNSUPPORTED;
+    if (!all && deep && !two_forms && chunks > 25 && e->batch == 1 && W % 4 && H * W % 4 == 0 && H * W <= 128) return TVX_E_UNSUPPORTED;
     if (!all && (nt > 5 || (!two_forms && narrow_wgs > (std::max(cin_steps, nt) <= 3 ? 5 : 2) * cus))) return TVX_E_UNSUPPORTED;
     a.W = W; a.batch = e->batch;
     a.half_rows = wide && W == 7 ? 2 : 0;
