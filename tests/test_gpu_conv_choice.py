@@ -18,6 +18,7 @@ LAYERS = [
     ("i8pc", dict(n=2, c=7, h=45, w=45, oc=5, kh=3, kw=3, stride=[1, 1], pad=P1, dil=[2, 1]), "conv2d_im2col_i8"),  # 43 x 45 pixels and dilated rows
     ("u8", dict(n=5, c=8, h=252, w=256, oc=6, kh=1, kw=1, stride=[2, 2], pad=P0), "conv2d_im2col_i8"),        # 80640
     ("u8", dict(n=5, c=8, h=248, w=255, oc=6, kh=1, kw=1, stride=[2, 2], pad=P0), "conv2d_tile_i8"),          # 79360
+    ("u8", dict(n=1, c=3, h=300, w=301, oc=20, kh=3, kw=3, pad=[16] * 4, dil=[16, 16]), "conv2d_tile_i8"),    # 90300, taps further apart than conv2d_im2col_i8 reaches
     # a granule of channels under weights with a zero point: two million products
     ("u8", dict(n=3, c=16, h=14, w=16, oc=20, kh=3, kw=3, pad=P1), "conv2d_igemm_i8"),
     ("u8", dict(n=3, c=16, h=14, w=16, oc=21, kh=3, kw=3, pad=P1), "conv2d_tile_i8"),

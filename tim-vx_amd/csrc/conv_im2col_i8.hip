@@ -636,8 +636,10 @@ static int Im2colSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host,
   const int zws = op->w_zp - (w_u8 ? 128 : 0);
   if (zxs < -128 || zxs > 127) return TVX_E_UNSUPPORTED;  // zero point outside the tensor's range
   if ((d->k_h - 1) * d->dilation_h > 31 || (d->k_w - 1) * d->dilation_w > 31) return TVX_E_UNSUPPORTED;  // window offsets index 32-bit masks
-  const int reg = RegSetup(op, d, w_host, bias_host, zxs, zws);
-  if (reg != TVX_E_UNSUPPORTED) return reg;
+  if (!rest) {
+    const int reg = RegSetup(op, d, w_host, bias_host, zxs, zws);
+    if (reg != TVX_E_UNSUPPORTED) return reg;
+  }
   // What does not fit registers is asked for twice, in front of the tiles (conv_tile.hip) and behind them, which take what lies between a handful of
   // pixels (windows of several taps: a few thousand) and eighty thousand: 0.64 of the time on 80 drawn layers (int8 12 -> 115, 1x1 / 2 on 13 x 13, batch 2, 11.9 -> 5.1 us; uint8 43 -> 80,
   // 1x1 / 2 on 17 x 17, batch 10, 15.9 -> 5.5). With more pixels a pass of this kernel is the shorter one (8 -> 64, 1x1 / 2 on 126 x 160, batch 64,

@@ -820,7 +820,6 @@ static bool IsBetterChoice(const tvx_conv2d_desc* d, int dt, bool sums) {
     const bool aligned = d->stride_w == 1 && d->stride_h == 1 && d->in_w % 4 == 0;
     const bool short_window = reduction <= 64 && d->in_c % 16 != 0 && d->out_c <= 128;
     if (sums && d->in_c <= 16 && reduction <= 512 && macs <= 2000000 && !short_window && (aligned || d->in_w * d->in_h <= 256)) return false;
-    if (short_window && static_cast<uint64_t>(d->batch) * d->out_h * d->out_w >= 80000) return false;  // (conv2d_im2col_i8, see there)
   }
   return true;
 }
