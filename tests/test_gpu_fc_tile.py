@@ -62,7 +62,7 @@ def test_stages_on_groups(oracle, m, n, k, mode, monkeypatch):
         assert np.array_equal(got, want), int((got != want).sum())
 
 
-@pytest.mark.parametrize("shape", [3, 5, 7])
+@pytest.mark.parametrize("shape", [3, 5, 7, 8])
 def test_rows_keep_an_infinity_apart(monkeypatch, shape):
     """What lies behind a row that ends inside a stage is not multiplied."""
     monkeypatch.setenv("TVX_FC_ROWS", "1")
@@ -76,7 +76,10 @@ def test_rows_keep_an_infinity_apart(monkeypatch, shape):
 
 @pytest.mark.parametrize("m,k,n,mode,kernel", [
     (332, 672, 1965, "i8pc", "fc_rows_i8"), (578, 685, 832, "i8pc", "fc_rows_i8"), (617, 358, 921, "f16", "fc_rows_f16"),   # reductions that end early in their last stage
-    (393, 704, 1908, "u8", "fc_tile_i8"), (900, 512, 1100, "f16", "fc_tile_f16"), (3521, 560, 1238, "i8pc", "fc_tile_i8")])
+    (393, 704, 1908, "u8", "fc_tile_i8"), (900, 512, 1100, "f16", "fc_tile_f16"), (3521, 560, 1238, "i8pc", "fc_tile_i8"),
+    # up to two 32 x 32 tiles a compute unit (of 256): rows that fit an L2 and are no whole cache lines apart, whole ones, more than fit, rows at odd bytes
+    (263, 1168, 1639, "f16", "fc_rows_f16"), (361, 2576, 1124, "i8pc", "fc_rows_i8"), (192, 2752, 2517, "f16", "fc_tile_f16"), (2195, 1888, 163, "f16", "fc_tile_f16"),
+    (383, 1098, 1136, "u8", "fc_tile_i8")])
 def test_which_tiles_a_layer_gets(oracle, m, k, n, mode, kernel, monkeypatch):
     x, w, b, kws = _case(m, k, n, mode)
     TC.expect_variant(monkeypatch, kernel)

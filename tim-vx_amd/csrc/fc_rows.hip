@@ -605,18 +605,23 @@ double Cost(const tvx_fc_desc& d, int dt, int shape) {
 // 16 x 16 tiles until there is one for each CU (f16 16 x 4096 -> 4096: 7.5 us against 9.1 on 32 x 32 tiles), 32 x 32 from there on (f32
 // 256 x 1024 -> 1024: 8.8 against 11.9), and 64 x 64 - fragments used twice, no exchange at the end - where there are more than one
 // of those per CU, or half as many with a reduction too short to split; int8 and float16 otherwise where Cost sees more than it may be
-// off by. Stages on four groups are a fit to 260 layers (7 and 10 % off each); of 420 others eleven take them, 0.82 of the time, one of these 1.02. float32, whose products take the longest, gains nothing by rows through LDS (882 x 3984 -> 1070: 95 us, 101 with).
+// off by. Stages on four groups are a fit to 260 layers (7 and 10 % off each), which knows nothing of where rows lie: up to two 32 x 32 tiles a CU are ahead of
+// them by .96 to 1.28, 1.12 on the average of 29 layers (f16 263 x 1168 -> 1639 7.0 us and 8.7), where all rows fit an XCD's L2 and are no whole cache lines
+// apart. Elsewhere the groups, chosen for 380 of 1500 drawn layers, take .81 of the time, 1.04 at most. float32, whose products take the longest, gains
+// nothing by rows through LDS (882 x 3984 -> 1070: 95 us, 101 with).
 int ChooseShape(const tvx_fc_desc& d, int dt) {
-  const uint64_t t16 = static_cast<uint64_t>((d.m + 15) / 16) * ((d.n + 15) / 16), t64 = static_cast<uint64_t>((d.m + 63) / 64) * ((d.n + 63) / 64);
+  const auto tiles = [&](uint32_t side) { return static_cast<uint64_t>((d.m + side - 1) / side) * ((d.n + side - 1) / side); };
+  const uint64_t t16 = tiles(16), t64 = tiles(64), row = static_cast<uint64_t>(d.k) * (dt == kI8 ? 1 : 2);
   const uint64_t cus = ComputeUnits();
   if (t16 <= cus) return 0;
   const int direct = 2 * t64 >= 3 * cus || (2 * t64 >= cus && static_cast<uint64_t>(d.k) * (dt == kI8 ? 1 : dt == kF16 ? 2 : 4) <= 384) ? 2 : 1;
   if (dt == kF32) return direct;
   int best = direct;
   double least = 0.94 * Cost(d, dt, direct);  // (what the fit is off by; then the shorter program)
+  const bool near_rows = direct == 1 && tiles(32) <= 2 * cus && row % 4 == 0 && row % 128 && d.m * row <= (4u << 20);
   for (int shape = 1; shape < kShapeCount; ++shape) {
     const Shape& sp = kShapes[shape];
-    if (sp.stage && sp.ks > 1 && static_cast<uint64_t>(d.k) * (dt == kI8 ? 1 : 2) <= 64ull * sp.stage * sp.ks) continue;  // (two stages a group at least)
+    if (sp.stage && sp.ks > 1 && (row <= 64ull * sp.stage * sp.ks || near_rows)) continue;  // (two stages a group at least)
     const double cost = Cost(d, dt, shape);
     if (cost < least) { best = shape; least = cost; }
   }
