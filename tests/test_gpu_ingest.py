@@ -15,7 +15,7 @@ MOVES = [((3, 2731, 2), (1, 0, 2), "interleaved"), ((1, 3, 5), (1, 2, 0), "gathe
 
 @pytest.mark.parametrize("dt", [np.uint8, np.float16, np.int32])
 @pytest.mark.parametrize("in_dims,perm,form", MOVES)
-def test_transpose_forms(oracle, in_dims, perm, form, dt):
+def test_transpose_forms(oracle, in_dims, perm, form, dt, variant=None):
     import torch
     T, n = TC.tvx(), int(np.prod(in_dims))
     if dt == np.int32 and in_dims[0] in (16,) and form == "interleaved":
@@ -28,6 +28,7 @@ def test_transpose_forms(oracle, in_dims, perm, form, dt):
         d.in_dims[i], d.perm[i] = e, p
     op = T.transpose_create(d)
     assert op.kernel_name == "transpose_" + form
+    assert variant is None or op.variant == op.kernel_name + variant, op.variant
     e = x.dtype.itemsize
     for off in (0, 1, 2):   # elements
         xd, yd = torch.zeros((n + 8) * e, dtype=torch.uint8, device="cuda"), torch.full(((n + 8) * e,), 0xA5, dtype=torch.uint8, device="cuda")
@@ -49,13 +50,15 @@ FEW = [((a, b, 3), (1, 0, 2), "interleaved") for a in range(2, 9) for b in (2, 7
 @pytest.mark.parametrize("dt", [np.uint8, np.float16, np.int32])
 @pytest.mark.parametrize("in_dims,perm,form", FEW)
 def test_transpose_of_few_channels(oracle, in_dims, perm, form, dt):
-    test_transpose_forms(oracle, in_dims, perm, form, dt)
+    e, (channels, pixels) = np.dtype(dt).itemsize, in_dims[:2]
+    blocks = channels % 4 == 0 and e <= 2 and pixels >= 4 // e
+    test_transpose_forms(oracle, in_dims, perm, form, dt, "_reg" if channels <= 8 and pixels >= 8 // e else "_block" if blocks else "")
 
 
 @pytest.mark.parametrize("channels,dt", [(20, np.uint8), (32, np.uint8), (60, np.uint8), (64, np.uint8), (20, np.float16), (32, np.float16), (18, np.float16)])
-@pytest.mark.parametrize("pixels", [3, 126, 128, 129, 410])
+@pytest.mark.parametrize("pixels", [3, 4, 5, 126, 128, 129, 130, 131, 410])
 def test_transpose_of_wide_pixels(oracle, pixels, channels, dt):
-    test_transpose_forms(oracle, (channels, pixels, 3), (1, 0, 2), "interleaved", dt)
+    test_transpose_forms(oracle, (channels, pixels, 3), (1, 0, 2), "interleaved", dt, "" if channels == 18 or (pixels == 3 and dt == np.uint8) else "_block")
 
 
 @pytest.mark.parametrize("out_dt", [0, 1, 2, 3])
