@@ -33,6 +33,11 @@ LAYERS = [
     ("f32", dict(n=4, c=1, h=30, w=46, oc=25, kh=3, kw=3, pad=P1), "conv2d_generic"),                          # 138000
     ("f16", dict(n=4, c=1, h=30, w=47, oc=25, kh=3, kw=3, pad=P1), "conv2d_tile_f16"),                         # 141000
     ("f32", dict(n=1, c=8, h=9, w=11, oc=12, kh=1, kw=1, pad=P0), "conv2d_tile_f32"),
+    ("f32", dict(n=2, c=4, h=41, w=42, oc=40, kh=1, kw=1, pad=P0), "conv2d_generic"),                          # 137760 of four products
+    ("f32", dict(n=2, c=4, h=41, w=43, oc=40, kh=1, kw=1, pad=P0), "conv2d_tile_f32"),                         # 141040
+    ("f16", dict(n=2, c=5, h=39, w=63, oc=79, kh=1, kw=1, stride=[2, 2], pad=P0), "conv2d_generic"),           # 101120 of five
+    ("f16", dict(n=2, c=5, h=39, w=63, oc=81, kh=1, kw=1, stride=[2, 2], pad=P0), "conv2d_tile_f16"),          # 103680
+    ("f32", dict(n=2, c=5, h=9, w=11, oc=12, kh=1, kw=1, pad=P0), "conv2d_tile_f32"),
     # float16, pointwise: at unit stride pixels in registers, whatever their number and that of the results
     ("f16", dict(n=2, c=24, h=13, w=13, oc=24, kh=1, kw=1, pad=P0), "pwconv_reg_f16"),
     ("f16", dict(n=2, c=24, h=13, w=13, oc=25, kh=1, kw=1, pad=P0), "pwconv_reg_f16"),
