@@ -641,11 +641,11 @@ static int Im2colSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host,
     if (reg != TVX_E_UNSUPPORTED) return reg;
   }
   // What does not fit registers is asked for twice, in front of the tiles (conv_tile.hip) and behind them, which take what lies between a handful of
-  // pixels (windows of several taps: a few thousand) and eighty thousand: 0.64 of the time on 80 drawn layers (int8 12 -> 115, 1x1 / 2 on 13 x 13, batch 2, 11.9 -> 5.1 us; uint8 43 -> 80,
+  // pixels (windows of several taps: a few thousand) and eighty thousand on 256 compute units: 0.64 of the time on 80 drawn layers (int8 12 -> 115, 1x1 / 2 on 13 x 13, batch 2, 11.9 -> 5.1 us; uint8 43 -> 80,
   // 1x1 / 2 on 17 x 17, batch 10, 15.9 -> 5.5). With more pixels a pass of this kernel is the shorter one (8 -> 64, 1x1 / 2 on 126 x 160, batch 64,
   // 16.6 against 26.8; 1 -> 80 on 79 x 153, batch 33, 13.0 against 15.9; 1 -> 128, 7x7 on 120 x 120, batch 30, 47.6 against 67.3).
-  const uint64_t pixels = static_cast<uint64_t>(d->batch) * d->out_h * d->out_w;
-  if (!rest && !op->fused_pool && pixels < 80000 && pixels > (taps == 1 ? 128u : 4096u)) return TVX_E_UNSUPPORTED;
+  const uint64_t pixels = static_cast<uint64_t>(d->batch) * d->out_h * d->out_w, cus = ComputeUnits();
+  if (!rest && !op->fused_pool && 2 * pixels < 625 * cus && 2 * pixels > (taps == 1 ? 1 : 32) * cus) return TVX_E_UNSUPPORTED;
   a.xor_mask = x_u8 ? 0x80 : 0;
   a.pad_fill = zxs & 0xff;
   a.zws = zws;

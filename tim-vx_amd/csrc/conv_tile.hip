@@ -758,7 +758,7 @@ int SumsBy(const Shape& sp, int steps) {
 // 8 -> 16, 3x3 / 2 on 50 x 69, batch 37, 7.2 us for 6.1; uint8 3 -> 16, 5x5 on 99 x 99, batch 7, 7.5 for 6.9;
 // but int8 20 -> 64 in four groups, 3x3 on 69 x 121, batch 46, 33.0 for 55.3).
 constexpr double kStackedMore = 1.06;
-constexpr int kStackedProducts = 128, kStackedOutputs = 2000000;
+constexpr int kStackedProducts = 128, kStackedOutputs = 7812;  // (a compute unit: two million on 256)
 
 struct Plan {
   TileArgs a;
@@ -803,10 +803,10 @@ static bool IsBetterChoice(const tvx_conv2d_desc* d, int dt, bool sums) {
   //                                                                larger windows, up to nine        1.11  1.04   .94   .86   .66
   const uint64_t few = reduction == 1 ? 1172 : reduction <= 3 ? 800 : reduction == 4 || (reduction <= 9 && !pointwise) ? 550 : reduction == 5 && dt == kF16 ? 400 : 0;
   if (dt != kI8 && groups == 1 && outputs <= few * cus) return false;
-  // (in groups: 4.3 against 5.7; int8, which has no other kernel for so few: 4 -> 64 in two, 1x1 on 25 x 25, 3.9 against 6.5, but 64 -> 240 in
-  // eight on 22 x 22 7.7 against 6.0)
-  if (dt != kI8 && groups > 1 && reduction <= 9 && macs <= 4000000) return false;
-  if (dt == kI8 && groups > 1 && reduction <= 8 && macs <= (reduction <= 4 ? 4000000 : 1000000)) return false;
+  // (in groups, by products, four millions and one on 256 compute units: 4.3 against 5.7; int8, which has no other kernel for so few: 4 -> 64 in two, 1x1 on
+  // 25 x 25, 3.9 against 6.5, but 64 -> 240 in eight on 22 x 22 7.7 against 6.0)
+  if (dt != kI8 && groups > 1 && reduction <= 9 && macs <= 15625 * cus) return false;
+  if (dt == kI8 && groups > 1 && reduction <= 8 && macs <= (reduction <= 4 ? 15625 : 3906) * cus) return false;
   // int8 1 x 1 in groups that fill less than a tile's channels: conv2d_gemm_i8 (188 -> 60 in four groups on 108 x 108, batch 6: 9.9 against
   // 17.4 us, 240 -> 96 on 74 x 74, batch 49: 36.8 against 52.3); with more than 32 channels in a group the tiles (144 -> 128 in two on
   // 29889 pixels: 9.5 against 16.8)
@@ -819,12 +819,12 @@ static bool IsBetterChoice(const tvx_conv2d_desc* d, int dt, bool sums) {
     return false;
   if (dt == kI8 && groups == 1) {
     if (ConvIgemmPersists(d)) return false;
-    // a granule of channels under weights with a zero point: up to two million products conv2d_igemm_i8, whose chain is short on small planes and on
+    // a granule of channels under weights with a zero point: up to two million products (on 256 compute units) conv2d_igemm_i8, whose chain is short on small planes and on
     // rows of whole dwords, is within a tenth of the tiles at 5 to 6 us; beyond them its tiles queue up (60 drawn layers .55 of its time, 16 -> 192
     // on 140 x 140, batch 3, 129 us against 15.7). What conv2d_im2col_i8 has left (its short windows) it does not get.
     const bool aligned = d->stride_w == 1 && d->stride_h == 1 && d->in_w % 4 == 0;
     const bool short_window = reduction <= 64 && d->in_c % 16 != 0 && d->out_c <= 128;
-    if (sums && d->in_c <= 16 && reduction <= 512 && macs <= 2000000 && !short_window && (aligned || d->in_w * d->in_h <= 256)) return false;
+    if (sums && d->in_c <= 16 && reduction <= 512 && 2 * macs <= 15625 * cus && !short_window && (aligned || d->in_w * d->in_h <= 256)) return false;
   }
   return true;
 }
@@ -891,7 +891,7 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   for (int stack = 1; stack <= 4; ++stack) {
   if (want_stack && stack != want_stack) continue;
   if (stack > 1 && (dt != kI8 || d->k_h == 1 || dh != 1 || stack * a.ocg > 32 || stack > rows)) break;
-  if (!want_stack && stack == 2 && real_taps * a.icg < kStackedProducts && out_image * d->batch < kStackedOutputs) continue;
+  if (!want_stack && stack == 2 && real_taps * a.icg < kStackedProducts && out_image * d->batch < static_cast<uint64_t>(kStackedOutputs) * cus) continue;
   stacked(stack);
   if (taps > 1024) break;
   for (int sidx = 0; sidx < kShapeCount; ++sidx) {

@@ -497,14 +497,15 @@ int DwRowsSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const 
 
 }  // namespace
 
-// Asked in front of DwConv3x3Setup, whose workgroup is a plane: many small planes, several to a workgroup here. Captured, us there (four columns a
+// Asked in front of DwConv3x3Setup, whose workgroup is a plane: many small planes, several to a workgroup here. The lines are in sixteenths of a plane a
+// compute unit, from layers on 256 of these. Captured, us there (four columns a
 // thread) and here, by planes: stride 1, 4 x 4: 1536 3.8 and 4.3, 6144 6.1 and 3.9, 36864 19.3 and 5.0; 8 x 8: 1536 3.8 and 4.3, 3072 4.4 and 3.8, 15360 10.1 and
 // 5.0; 16 x 16: 3072 4.0 and 5.0, 6144 5.7 and 5.3, 15360 9.8 and 7.2; 20 x 20: 6144 5.8 and 6.4, 15360 10.1 and 8.9; 24 x 24: 15360 10.3 and 12.4. Stride 2, 16 x 16:
 // 1536 4.2 and 4.8, 4608 5.7 and 5.0, 36864 22.0 and 7.1; 32 x 32: 4608 5.9 and 5.7, 15360 12.7 and 9.7; 40 x 40: 15360 12.1 and 13.9.
 int DwManyPlanesSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, const void* bias_host) {
   if (!op->quantized || !w_host || d->multiplier != 1 || op->out_blocked) return TVX_E_UNSUPPORTED;
-  const uint64_t plane = static_cast<uint64_t>(d->in_w) * d->in_h, planes = static_cast<uint64_t>(d->batch) * d->in_c;
-  if (d->stride_w == 1 ? plane > 400 || planes < (plane <= 64 ? 3072 : plane <= 256 ? 6000 : 12000) : plane > 1024 || planes < (plane <= 256 ? 4000 : 6000))
+  const uint64_t plane = static_cast<uint64_t>(d->in_w) * d->in_h, planes = 16 * static_cast<uint64_t>(d->batch) * d->in_c, cus = ComputeUnits();
+  if (d->stride_w == 1 ? plane > 400 || planes < (plane <= 64 ? 192 : plane <= 256 ? 375 : 750) * cus : plane > 1024 || planes < (plane <= 256 ? 250 : 375) * cus)
     return TVX_E_UNSUPPORTED;
   return DwRowsSetup(op, d, w_host, bias_host);
 }
