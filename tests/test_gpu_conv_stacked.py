@@ -35,7 +35,7 @@ def test_stacked_rows(oracle, monkeypatch, name, mode):
         monkeypatch.setenv("TVX_CONV_TILE_STACK", str(stack))
         for shape in (3, 4, 6, 7):   # (those of 32 channels)
             monkeypatch.setenv("TVX_CONV_TILE_SHAPE", str(shape))
-            got = TC.gpu_conv2d(x, wt, b, act=1, want_kernel="conv2d_tile_i8", **kws)
+            got = TC.gpu_conv2d(x, wt, b, act=1, want_kernel="conv2d_tile_i8", want_variant="conv2d_tile_i8_stacked" + ("_sums" if mode == "u8" else ""), **kws)
             assert np.array_equal(got, want), (stack, shape, int((got != want).sum()))
             ran += 1
     assert ran >= 4

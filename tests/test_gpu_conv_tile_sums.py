@@ -24,5 +24,8 @@ def test_window_sums(oracle, monkeypatch, c, k, loop):
         monkeypatch.setenv("TVX_CONV_TILE_SHAPE", str(shape))
         if loop:
             monkeypatch.setenv("TVX_CONV_TILE_LOOP", str(loop))
-        got = TC.gpu_conv2d(x, wt, b, act=1, want_kernel="conv2d_tile_i8", **kws)
+        # steps of sixteen bytes of a wavefront, for each of its tiles (two in the first three shapes), shared by those that split them (shape 1)
+        steps = (k * k * -(-c // 16) + 1) // 2 * (loop or 1)
+        variant = "conv2d_tile_i8_box" if shape < 3 and steps * 2 // (2 if shape == 1 else 1) > 80 else "conv2d_tile_i8_sums"
+        got = TC.gpu_conv2d(x, wt, b, act=1, want_kernel="conv2d_tile_i8", want_variant=variant, **kws)
         assert np.array_equal(got, want), (shape, int((got != want).sum()))

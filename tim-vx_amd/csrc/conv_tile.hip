@@ -1094,7 +1094,8 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
 
   Plan plan{};
   plan.a = a;
-  plan.fn = sp.fn[g.stack > 1 ? (g.sums == kNoSums ? 5 : 6) : g.sums == kNoSums ? dt : g.sums == kSumsInLoop ? 3 : 4][a.chunks > 1];
+  const int flavour = g.stack > 1 ? (g.sums == kNoSums ? 5 : 6) : g.sums == kNoSums ? dt : g.sums == kSumsInLoop ? 3 : 4;
+  plan.fn = sp.fn[flavour][a.chunks > 1];
   plan.lds_bytes = static_cast<unsigned>(g.lds_bytes);
   plan.grid = static_cast<unsigned>(a.per_xcd) * 8;
   plan.threads = 64u * sp.waves;
@@ -1106,6 +1107,8 @@ int ConvTileSetup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, cons
   op->host_blob.assign(reinterpret_cast<const uint8_t*>(&plan), reinterpret_cast<const uint8_t*>(&plan) + sizeof(plan));
   op->run = ConvTileRun;
   op->kernel_name = dt == kF32 ? "conv2d_tile_f32" : dt == kF16 ? "conv2d_tile_f16" : "conv2d_tile_i8";
+  static const char* const kVariants[7] = {nullptr, nullptr, nullptr, "conv2d_tile_i8_sums", "conv2d_tile_i8_box", "conv2d_tile_i8_stacked", "conv2d_tile_i8_stacked_sums"};
+  op->variant = kVariants[flavour];
   return TVX_OK;
 }
 
