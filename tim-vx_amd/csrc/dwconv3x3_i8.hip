@@ -390,17 +390,28 @@ int DwConv3x3Setup(tvx_op* op, const tvx_conv2d_desc* d, const void* w_host, con
   a.rq = op->aux2.as<tvx_v4i>();
   a.C = C; a.H = d->in_h; a.W = d->in_w; a.OH = d->out_h; a.OW = d->out_w;
   a.pad_t = d->pad_top; a.pad_l = d->pad_left;
-  // Eight columns per thread (stride 1, rows that are whole 8-byte units): one 64-bit load per input row and lane. A wavefront of short rows has half as
-  // many lanes with eight, and a longer chain. Captured, four over eight, 770 layers:
-  //   planes of 96 rows and more (below: eight rows of four columns a thread, or four of eight), 16 to 224 columns, 32 to 3072 planes: 1.00 to 1.11, mean 1.05;
-  //   lower planes of up to 55 columns: .59 to .97 (15360 of 16 x 16 9.8 and 16.3 us);
-  //   lower planes of wider rows, by results in millions, means:   to 1    4    6     9    13    20    26    40  above
-  //                                               no window sums    .93  .96  .96  1.03  1.04  1.02  1.06  1.08  1.10
-  //                                               window sums       .84  .88  .88   .94   .98   .96  1.01  1.03  1.06
-  // The line is drawn at 6 and at 20 million on 256 compute units: 1.004 of the time with the better form for each, and 1.002.
-  const uint64_t results = static_cast<uint64_t>(d->batch) * C * d->out_w * d->out_h, cus = ComputeUnits();
+  // Eight columns per thread (stride 1, rows that are whole 8-byte units): one 64-bit load per input row and lane, and a longer chain. Planes of 96 rows and
+  // more, whose threads take eight rows of four columns (below) or four of eight: ahead on 354 layers, four columns 1.00 to 1.11 of the time, mean 1.05.
+  // On lower ones it is ahead where it halves a plane's wavefronts (short rows leave lanes idle with it) and there are enough of them. Four over eight,
+  // captured, means of 702 layers, by wavefronts with four columns, of a plane and a compute unit:
+  //                                             to 1.5    5    10    18    36    72   150  above
+  //   no window sums   2 to 1                     .93   .97  1.02  1.05  1.06  1.10
+  //                    4 to 2                     .92   .92   .94   .96   .95  1.05  1.05  1.11
+  //                    6, 7, 8 to 3, 4            .92   .99  1.00   .98  1.00  1.10  1.11  1.12
+  //                    more, to half as many      .92   .93   .93   .95   .96  1.03  1.04  1.10
+  //                    not to half as many        .89   .92   .92   .89   .90   .98   .94   .91
+  //   window sums      2 to 1                     .83   .88   .90   .97  1.00  1.02
+  //                    4 to 2                     .83   .84   .86   .87   .88  1.00  1.01  1.07
+  //                    6, 7, 8 to 3, 4            .83   .90   .91   .91   .93  1.02  1.05  1.06
+  //                    more, to half as many      .83   .84   .85   .88   .88   .96   .99  1.06
+  //                    not to half as many        .80   .85   .84   .80   .82   .89   .88   .88
+  // By these lines all 1056 take 1.001 of the time with the better form for each, 1.06 at most.
+  const uint64_t planes = static_cast<uint64_t>(d->batch) * C, cus = ComputeUnits();
   const bool wide_rows = S == 1 && (d->in_w & 7) == 0 && (d->out_w & 7) == 0;
-  int cols = wide_rows && (d->out_h >= 96 || (d->out_w >= 56 && results >= (any_box ? 78000 : 23500) * cus)) ? 8 : 4;
+  const auto wavefronts = [&](int cw) { return (((d->out_h + 3) / 4 << lanes_shift(cw)) + 63) / 64; };  // of a plane
+  const uint32_t by4 = wavefronts(4), by8 = wide_rows ? wavefronts(8) : by4;
+  const uint64_t enough = by4 == 2 ? (any_box ? 24 : 4) : by4 <= 8 || !any_box ? 36 : 100;
+  int cols = wide_rows && (d->out_h >= 96 || (2 * by8 <= by4 + (by4 >= 7) && planes * by4 >= enough * cus)) ? 8 : 4;
   if (const char* f = getenv("TVX_DWCONV_COLS")) {  // tuning aid: output columns per thread
     if (atoi(f) == 4) cols = 4;
     if (atoi(f) == 8 && wide_rows) cols = 8;
