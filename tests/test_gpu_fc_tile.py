@@ -79,7 +79,7 @@ def test_rows_keep_an_infinity_apart(monkeypatch, shape):
     (393, 704, 1908, "u8", "fc_tile_i8"), (900, 512, 1100, "f16", "fc_tile_f16"), (3521, 560, 1238, "i8pc", "fc_tile_i8"),
     # up to two 32 x 32 tiles a compute unit (of 256): rows that fit an L2 and are no whole cache lines apart, whole ones, more than fit, rows at odd bytes
     (263, 1168, 1639, "f16", "fc_rows_f16"), (361, 2576, 1124, "i8pc", "fc_rows_i8"), (192, 2752, 2517, "f16", "fc_tile_f16"), (2195, 1888, 163, "f16", "fc_tile_f16"),
-    (383, 1098, 1136, "u8", "fc_tile_i8")])
+    (383, 1098, 1136, "u8", "fc_tile_i8"), (3532, 1696, 127, "i8pc", "fc_rows_i8"), (3468, 1952, 108, "f16", "fc_tile_f16")])
 def test_which_tiles_a_layer_gets(oracle, m, k, n, mode, kernel, monkeypatch):
     x, w, b, kws = _case(m, k, n, mode)
     TC.expect_variant(monkeypatch, kernel)

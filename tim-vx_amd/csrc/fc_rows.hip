@@ -607,7 +607,8 @@ double Cost(const tvx_fc_desc& d, int dt, int shape) {
 // of those per CU, or half as many with a reduction too short to split; int8 and float16 otherwise where Cost sees more than it may be
 // off by. Stages on four groups are a fit to 260 layers (7 and 10 % off each), which knows nothing of where rows lie: up to two 32 x 32 tiles a CU are ahead of
 // them by .96 to 1.28, 1.12 on the average of 29 layers (f16 263 x 1168 -> 1639 7.0 us and 8.7), where all rows fit an XCD's L2 and are no whole cache lines
-// apart. Elsewhere the groups, chosen for 380 of 1500 drawn layers, take .81 of the time, 1.04 at most. float32, whose products take the longest, gains
+// apart, and by .90 to 1.33, 1.14 on the average of eight, where more rows than that have up to 2000 bytes (int8 8000 x 1584 -> 41 6.1 us and 7.4). Elsewhere the
+// groups, chosen for 380 of 1500 drawn layers, take .81 of the time, 1.04 at most; .88 of it for 144 more of up to two 32 x 32 tiles a CU. float32, whose products take the longest, gains
 // nothing by rows through LDS (882 x 3984 -> 1070: 95 us, 101 with).
 int ChooseShape(const tvx_fc_desc& d, int dt) {
   const auto tiles = [&](uint32_t side) { return static_cast<uint64_t>((d.m + side - 1) / side) * ((d.n + side - 1) / side); };
@@ -618,7 +619,7 @@ int ChooseShape(const tvx_fc_desc& d, int dt) {
   if (dt == kF32) return direct;
   int best = direct;
   double least = 0.94 * Cost(d, dt, direct);  // (what the fit is off by; then the shorter program)
-  const bool near_rows = direct == 1 && tiles(32) <= 2 * cus && row % 4 == 0 && row % 128 && d.m * row <= (4u << 20);
+  const bool near_rows = direct == 1 && tiles(32) <= 2 * cus && row % 4 == 0 && row % 128 && (row <= 2000 || d.m * row <= (4u << 20));
   for (int shape = 1; shape < kShapeCount; ++shape) {
     const Shape& sp = kShapes[shape];
     if (sp.stage && sp.ks > 1 && (row <= 64ull * sp.stage * sp.ks || near_rows)) continue;  // (two stages a group at least)
