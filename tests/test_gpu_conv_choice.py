@@ -30,8 +30,15 @@ LAYERS = [
     ("f16", dict(n=2, c=3, h=99, w=99, oc=41, kh=1, kw=1, stride=[2, 2], pad=P0), "conv2d_tile_f16"),          # 205000
     ("f32", dict(n=1, c=1, h=30, w=41, oc=25, kh=3, kw=3, pad=P1), "conv2d_generic"),                          # 30750 outputs
     ("f16", dict(n=1, c=1, h=29, w=41, oc=25, kh=3, kw=3, pad=P1), "conv2d_generic"),
-    ("f32", dict(n=4, c=1, h=30, w=46, oc=25, kh=3, kw=3, pad=P1), "conv2d_generic"),                          # 138000
-    ("f16", dict(n=4, c=1, h=30, w=47, oc=25, kh=3, kw=3, pad=P1), "conv2d_tile_f16"),                         # 141000
+    ("f32", dict(n=4, c=1, h=30, w=34, oc=25, kh=3, kw=3, pad=P1), "conv2d_generic"),                          # 102000
+    ("f16", dict(n=4, c=1, h=30, w=35, oc=25, kh=3, kw=3, pad=P1), "conv2d_tile_f16"),                         # 105000
+    ("f32", dict(n=19, c=1, h=144, w=144, oc=1, kh=3, kw=3, pad=[2] * 4, dil=[2, 2]), "conv2d_generic"),       # few channels: of one, three and six
+    ("f16", dict(n=4, c=1, h=256, w=257, oc=3, kh=3, kw=3, pad=P1), "conv2d_generic"),
+    ("f16", dict(n=4, c=1, h=267, w=257, oc=3, kh=3, kw=3, pad=P1), "conv2d_tile_f16"),
+    ("f32", dict(n=3, c=1, h=118, w=119, oc=6, kh=3, kw=3, pad=P1), "conv2d_generic"),
+    ("f32", dict(n=3, c=1, h=118, w=122, oc=6, kh=3, kw=3, pad=P1), "conv2d_tile_f32"),
+    ("f32", dict(n=3, c=1, h=60, w=62, oc=18, kh=1, kw=5, pad=[2, 2, 0, 0]), "conv2d_generic"),                # 200880 of five products
+    ("f32", dict(n=3, c=4, h=60, w=62, oc=18, kh=1, kw=2, pad=[1, 0, 0, 0]), "conv2d_tile_f32"),               # 200880 of eight
     ("f32", dict(n=1, c=8, h=9, w=11, oc=12, kh=1, kw=1, pad=P0), "conv2d_tile_f32"),
     ("f32", dict(n=2, c=4, h=41, w=42, oc=40, kh=1, kw=1, pad=P0), "conv2d_generic"),                          # 137760 of four products
     ("f32", dict(n=2, c=4, h=41, w=43, oc=40, kh=1, kw=1, pad=P0), "conv2d_tile_f32"),                         # 141040

@@ -793,17 +793,22 @@ static bool IsBetterChoice(const tvx_conv2d_desc* d, int dt, bool sums) {
   // a group of three output channels and fewer fills less than a tenth of a tile's 32 channels: only where each has little to add up
   // (float16 432 -> 12 in four groups, 7x7 on 42 x 42, batch 28: 2495 us with one thread per output, 140 here)
   if (groups > 1 && ocg < 4 && reduction <= 128) return false;
-  // a handful of products per output: one thread per output is quicker than staging a window, up to so many outputs. 597 layers over its time, by
-  // outputs in thousands (captured, means; the lines at 300, 205, 141 and 102 on 256 compute units):   to 60   140   220   350  above
-  //                                                                1x1 of one channel                1.50  1.45  1.30  1.17   .74
-  //                                                                of two or three                   1.29  1.24  1.09   .94   .78
-  //                                                                of four                           1.12  1.07  1.06   .81   .58
-  //                                                                of five, float16                  1.10  1.04               .51
-  //                                                                of five, float32                   .99   .93   .85   .74   .46
-  //                                                                of six to nine                     .86   .82   .79   .67   .47
-  //                                                                larger windows, up to nine        1.11  1.04   .94   .86   .66
-  const uint64_t few = reduction == 1 ? 1172 : reduction <= 3 ? 800 : reduction == 4 || (reduction <= 9 && !pointwise) ? 550 : reduction == 5 && dt == kF16 ? 400 : 0;
-  if (dt != kI8 && groups == 1 && outputs <= few * cus) return false;
+  // a handful of products per output: one thread per output is quicker than staging a window, up to so many outputs. Tiles over it, captured, 1400 layers
+  // of seven channels and more, means by outputs in thousands (on 256 compute units):   to 60   140   220   350   600  above
+  //                                                     1x1 of one channel                1.49  1.46  1.30  1.14   .90   .61
+  //                                                         of two or three               1.29  1.23  1.10   .96   .80   .57
+  //                                                         of four                       1.12  1.07  1.01   .82   .65   .49
+  //                                                         of five, float16              1.08  1.04   .97   .86   .60   .40
+  //                                                         of five, float32               .99  1.02   .85   .75   .60   .42
+  //                                                         of six to nine                 .85   .83   .77   .64   .53   .32
+  //                                                     larger windows, to five products  1.31  1.25  1.14  1.01   .83   .50
+  //                                                         six to eight                  1.10  1.07   .98   .89   .74   .43
+  //                                                         nine                          1.06  1.01   .94   .85   .71   .39
+  // Fewer channels leave most of a tile's 32 empty: of one the tiles take 1.3 to 2.9 of the time at 20 thousand to 1.8 million outputs, of two or three 1.1 to
+  // 1.5, of four to six 1.15 to .87. By these lines all 2097 layers take 1.006 of the time with the better kernel for each.
+  const uint64_t few = !pointwise ? (reduction <= 5 ? 1000 : reduction <= 8 ? 700 : reduction == 9 ? 400 : 0)
+                                  : reduction == 1 ? 1172 : reduction <= 3 ? 800 : reduction == 4 ? 550 : reduction == 5 && dt == kF16 ? 400 : 0;
+  if (dt != kI8 && groups == 1 && 2 * outputs <= few * cus * (d->out_c == 1 ? 64 : d->out_c <= 3 ? 16 : d->out_c <= 6 ? 5 : 2)) return false;
   // (in groups, by products, four millions and one on 256 compute units: 4.3 against 5.7; int8, which has no other kernel for so few: 4 -> 64 in two, 1x1 on
   // 25 x 25, 3.9 against 6.5, but 64 -> 240 in eight on 22 x 22 7.7 against 6.0)
   if (dt != kI8 && groups > 1 && reduction <= 9 && macs <= 15625 * cus) return false;
