@@ -241,7 +241,8 @@ int tvx_conv2d_dw_pw_create(const tvx_conv2d_desc* dw, const void* dw_weights_ho
  * kernel fuses this block (the kernel covers feature maps of three columns and more, SAME depthwise padding,
  * at most 160 input and 160 output channels (320 on 7 and 14 columns), and by default claims only the blocks where
  * it is faster than the two or three launches: stride 1, up to 160 output channels, and of other widths than 7 and 14
- * columns only small feature maps and small batches; the caller then creates the operators one by one). */
+ * columns only small feature maps and small batches, fewer of them with many channels; the caller then creates the
+ * operators one by one). */
 int tvx_mbconv_create(const tvx_conv2d_desc* expand, const void* expand_weights_host, const void* expand_bias_host,
                       const tvx_conv2d_desc* dw, const void* dw_weights_host, const void* dw_bias_host,
                       const tvx_conv2d_desc* project, const void* project_weights_host, const void* project_bias_host,
@@ -352,8 +353,8 @@ int tvx_op_run(tvx_op* op, const void* in0, const void* in1, void* out, void* st
 int tvx_op_run3(tvx_op* op, const void* in0, const void* in1, const void* in2, void* out, void* stream);
 /* Name of the kernel variant chosen at creation, e.g. "conv2d_generic". */
 const char* tvx_op_kernel_name(const tvx_op* op);
-/* Several kernels report one name, where a newer one took over some of a name's layers. This tells them apart, e.g.
- * "dwconv_reg_i8" for an operator named "dwconv_planes_i8"; the name itself where it says enough. */
+/* Several kernels report one name, where a newer one took over some of a name's layers or one has forms. This tells them
+ * apart, e.g. "dwconv_reg_i8" for an operator named "dwconv_planes_i8"; the name itself where it says enough. */
 const char* tvx_op_variant(const tvx_op* op);
 void tvx_op_destroy(tvx_op* op);
 
