@@ -9,8 +9,8 @@
 //  - KS = 4: inputs of more than 128 channels share the reduction between the four wavefronts of a workgroup, which exchange partial sums through LDS.
 //  - Channels that do not exist are zero (their weights are too, but a channel read in their place may hold an infinity).
 // Bound by memory where results are many, by the chain load - pair - multiply - store where few. Against the window in LDS (conv_tile.hip) and the
-// gathered windows (conv_gemm.hip): 70 drawn layers .63 of the time, none slower: 20 -> 144 on 9344 pixels, batch 40, 56.7 -> 21.7 us (122 MB, floor
-// 24.5 at a copy's rate), 464 -> 156 on 77 x 110, batch 15, 88 -> 52, 416 -> 48 on 39 x 39, batch 24, 15.9 -> 11.1. 191 layers of at most 576 pixels .59 (56 ->
+// gathered windows (conv_gemm.hip): 70 drawn layers .63 of the time, none slower: 20 -> 144 on 73 x 128, batch 40, 39.0 -> 21.4 us (122 MB, floor
+// 24.5 at a copy's rate), 464 -> 156 on 77 x 110, batch 15, 84 -> 40, 416 -> 48 on 39 x 39, batch 24, 17.6 -> 9.8. 191 layers of at most 576 pixels .59 (56 ->
 // 382 on 6 x 6 7.2 -> 2.5; the slowest 848 -> 8 on 12 pixels, batch 13, 5.7 -> 5.8), 110 of at most 16 results from at most 64 channels on planes of
 // whole 16 pixels .42 (16 -> 8 on 88 x 88, batch 8, 3.9 -> 3.1; 64 -> 6 on 15200 pixels, batch 20, 162 by a thread per output, 8.4).
 // Reference: src/tim/vx/ops/conv2d.cc (1x1 kernels).
